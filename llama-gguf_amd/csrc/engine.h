@@ -47,6 +47,16 @@ struct PfScratch {
   uint8_t *xh_gather = nullptr, *xh_act_e = nullptr;   // per expert: gathered inputs [E][xh_bytes(H)], activations [E][xh_bytes(EI)]
 };
 
+// long prompts (prefill_wide.hip): buffers for blocks of up to `cap` tokens
+struct PfwScratch {
+  uint32_t cap = 0;                    // 0: not allocated
+  uint8_t *x = nullptr, *attn = nullptr, *act = nullptr;   // row-major f16: [cap][hidden], [cap][QD], [rows][ffn]
+  float *hidden = nullptr, *q = nullptr, *part = nullptr, *inv_rms = nullptr, *moe_w = nullptr, *moe_roww = nullptr;
+  size_t part_bytes = 0;
+  int *tokens = nullptr, *moe_sel = nullptr, *moe_seg = nullptr, *moe_tile = nullptr, *moe_slot = nullptr, *moe_src = nullptr;
+  uint32_t moe_tiles = 0;
+};
+
 struct ProfRec { int cls; int sym; uint64_t bytes; hipEvent_t a, b; };
 
 // multi-sequence decode (engine_batch.hip): `max_batch` slots, each one sequence's KV caches and position, and the vectors of
@@ -117,6 +127,7 @@ struct lgh_ctx {
   std::vector<void*> allocs;  // everything hipMalloc'ed by this context
   std::vector<lgh::XqBuf> xqs;
   lgh::PfScratch pf;
+  lgh::PfwScratch pfw;
   lgh::BatchScratch batch;
   float* tq_signs = nullptr;                   // TurboQuant KV cache: [owned layer][kv head][k, v][head_dim] rotation signs (device)
   std::vector<float> tq_signs_host;

@@ -15,6 +15,7 @@
 //                                                            arg-max back on device
 //   reset() zero-fills every cache over PCIe (808-843)       O(1): position rewind
 #include "engine.h"
+#include "layered.h"
 #include "prefill.h"
 #include "xq.h"
 
@@ -840,6 +841,31 @@ static int pf_ensure(lgh_ctx* c) {
   return LGH_OK;
 }
 
+// token ids of a block at positions pos .. pos + m - 1 -> dst (device)
+static int pf_stage_tokens(lgh_ctx* c, const uint32_t* tokens, uint32_t m, int* dst) {
+  PfScratch& P = c->pf;
+  const lgh_model_desc& d = c->d;
+  const uint32_t pos0 = (uint32_t)c->pos;
+  // The caller's `tokens` may be freed as soon as this returns (lgh_stage_prefill_batch does not synchronise), so the ids
+  // go through a context-owned PINNED buffer, one slot per position; a slot is only rewritten after the copy that last
+  // read it has completed (reset + a second prompt before the first one has run).
+  if (!P.tok_pinned) {
+    HIP_TRY(c, LGH_ALLOCATION_FAILED, hipHostMalloc((void**)&P.tok_pinned, (size_t)d.max_seq_len * 4, hipHostMallocDefault));
+    HIP_TRY(c, LGH_OPERATION_FAILED, hipEventCreateWithFlags(&P.tok_copied, hipEventDisableTiming));
+  } else if (pos0 < P.tok_hi && pos0 + m > P.tok_lo) {
+    // only when a slot about to be rewritten may still be read: a reset / shift / truncate followed by a new prompt.  The blocks
+    // of ONE prompt use ascending slots and never wait here (lgh_stage_prefill_batch stays asynchronous).
+    HIP_TRY(c, LGH_OPERATION_FAILED, hipEventSynchronize(P.tok_copied));
+    P.tok_lo = P.tok_hi = 0;
+  }
+  if (P.tok_hi == P.tok_lo) { P.tok_lo = pos0; P.tok_hi = pos0 + m; }
+  else { P.tok_lo = std::min(P.tok_lo, pos0); P.tok_hi = std::max(P.tok_hi, pos0 + m); }
+  std::memcpy(P.tok_pinned + pos0, tokens, (size_t)m * 4);
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipMemcpyAsync(dst, P.tok_pinned + pos0, (size_t)m * 4, hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipEventRecord(P.tok_copied, c->stream));
+  return LGH_OK;
+}
+
 // m <= 128 prompt tokens at positions pos .. pos+m-1: fills every owned layer's K/V rows.  The first stage starts from the
 // tokens' embedding rows, any other stage from the block of hidden vectors its predecessor left in pf.hidden; a stage that
 // is not the last leaves its output block there (the last one stops after its final layer's K/V rows: nothing else of a
@@ -856,23 +882,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
     return e == hipSuccess ? LGH_OK : fail(c, LGH_OPERATION_FAILED, std::string("batched prefill, ") + what + ": " + hipGetErrorString(e));
   };
   if (c->first) {
-    // The caller's `tokens` may be freed as soon as this returns (lgh_stage_prefill_batch does not synchronise), so the ids
-    // go through a context-owned PINNED buffer, one slot per position; a slot is only rewritten after the copy that last
-    // read it has completed (reset + a second prompt before the first one has run).
-    if (!P.tok_pinned) {
-      HIP_TRY(c, LGH_ALLOCATION_FAILED, hipHostMalloc((void**)&P.tok_pinned, (size_t)d.max_seq_len * 4, hipHostMallocDefault));
-      HIP_TRY(c, LGH_OPERATION_FAILED, hipEventCreateWithFlags(&P.tok_copied, hipEventDisableTiming));
-    } else if (pos0 < P.tok_hi && pos0 + m > P.tok_lo) {
-      // only when a slot about to be rewritten may still be read: a reset / shift / truncate followed by a new prompt.  The blocks
-      // of ONE prompt use ascending slots and never wait here (lgh_stage_prefill_batch stays asynchronous).
-      HIP_TRY(c, LGH_OPERATION_FAILED, hipEventSynchronize(P.tok_copied));
-      P.tok_lo = P.tok_hi = 0;
-    }
-    if (P.tok_hi == P.tok_lo) { P.tok_lo = pos0; P.tok_hi = pos0 + m; }
-    else { P.tok_lo = std::min(P.tok_lo, pos0); P.tok_hi = std::max(P.tok_hi, pos0 + m); }
-    std::memcpy(P.tok_pinned + pos0, tokens, (size_t)m * 4);
-    HIP_TRY(c, LGH_OPERATION_FAILED, hipMemcpyAsync(P.tokens, P.tok_pinned + pos0, (size_t)m * 4, hipMemcpyHostToDevice, st));
-    HIP_TRY(c, LGH_OPERATION_FAILED, hipEventRecord(P.tok_copied, st));
+    if ((rc = pf_stage_tokens(c, tokens, m, P.tokens))) return rc;
     if ((rc = K(embed_batch_launch(c->embd_type, c->embd_raw, P.tokens, P.hidden, H, m, st), "embedding"))) return rc;
   }
   if ((rc = K(pf_row_epi_launch(nullptr, 0, 0, 0, nullptr, P.hidden, H, c->layers[c->l0].attn_norm, P.xh_h, P.ssq, m, st), "attn_norm"))) return rc;
@@ -933,6 +943,164 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
   c->pos += m;
   c->stats.tokens_processed += m;
   HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
+  return LGH_OK;
+}
+
+// ---- long prompts: blocks of up to kPfwTokens tokens (prefill_wide.hip) ----
+// From this many tokens on a prompt takes the wide path.  A dense model's products fill a workgroup's 256 tokens there: at Llama-3-8B widths, 8 layers,
+// 255 tokens take 2.12 ms as two blocks and 2.08 ms wide, 192 tokens 1.86 and 1.93, 257 tokens 2.75 and 2.21, 512 tokens 4.33 and 2.67.  A mixture's
+// tokens spread over its experts, so its rows fill no tile either way (Mixtral widths, 2 layers: 160 tokens 1.00 and 0.70 ms, 600 tokens 2.67 and 1.07).
+// Shorter ones keep the blocks that pipeline stages hand over, with their bits.
+static size_t pfw_min_tokens(const lgh_ctx* c) { return c->d.num_experts ? 160 : 256; }
+
+static bool pfw_eligible(const lgh_ctx* c) {
+  if (!c->first || !c->last || !pf_eligible(c)) return false;   // (stages hand blocks of 128 tokens over)
+  for (uint32_t i = c->l0; i < c->l1; i++) {
+    const LayerW& L = c->layers[i];
+    if (L.moe() ? !pfw_pairs(&L.gate_exps, &L.up_exps) || L.gate_exps.n % 16 : !pfw_pairs(&L.gate, &L.up)) return false;
+  }
+  return true;
+}
+
+static int pfw_ensure(lgh_ctx* c) {
+  PfwScratch& P = c->pfw;
+  if (P.cap) return LGH_OK;
+  const lgh_model_desc& d = c->d;
+  const uint32_t H = d.hidden_size, QD = d.num_heads * d.head_dim, KD = d.num_kv_heads * d.head_dim;
+  const uint32_t cap = std::min<uint32_t>(kPfwTokens, (d.max_seq_len + kPfwTile - 1) / kPfwTile * kPfwTile);
+  bool any_moe = false;
+  size_t act = 0;
+  for (uint32_t i = c->l0; i < c->l1; i++) {
+    const LayerW& L = c->layers[i];
+    any_moe |= L.moe();
+    act = std::max(act, L.moe() ? (size_t)cap * d.num_experts_per_token * L.gate_exps.n : (size_t)cap * L.gate.n);
+  }
+  const uint32_t top = any_moe ? d.num_experts_per_token : 1, pairs = any_moe ? cap * top : 0;
+  const uint32_t tiles = any_moe ? moe_max_tiles(pairs, d.num_experts, kPfwTile) : 0;
+  const size_t pb = std::max(pfw_part_bytes(cap, QD + 2 * KD), pfw_part_bytes(cap * top, H));
+  struct { void** p; size_t n; } bufs[] = {
+      {(void**)&P.x, (size_t)cap * H * 2},      {(void**)&P.attn, (size_t)cap * QD * 2},   {(void**)&P.act, act * 2},
+      {(void**)&P.hidden, (size_t)cap * H * 4}, {(void**)&P.q, (size_t)cap * QD * 4},      {(void**)&P.part, pb},
+      {(void**)&P.inv_rms, (size_t)cap * 4},    {(void**)&P.tokens, (size_t)cap * 4},
+      {(void**)&P.moe_sel, (size_t)pairs * 4},  {(void**)&P.moe_w, (size_t)pairs * 4},     {(void**)&P.moe_roww, (size_t)pairs * 4},
+      {(void**)&P.moe_slot, (size_t)pairs * 4}, {(void**)&P.moe_src, (size_t)pairs * 4},   {(void**)&P.moe_tile, (size_t)tiles * 8},
+      {(void**)&P.moe_seg, any_moe ? (size_t)(d.num_experts + 1) * 4 : 0},
+  };
+  for (auto& b : bufs) {
+    if (!b.n) continue;
+    if (int rc = dev_alloc(c, b.p, b.n)) return rc;
+    c->stats.scratch_bytes += b.n;
+  }
+  P.part_bytes = pb;
+  P.moe_tiles = tiles;
+  P.cap = cap;
+  return LGH_OK;
+}
+
+// m prompt tokens at positions pos .. pos + m - 1 through every layer of a single-stage context: its K / V rows
+static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
+  PfwScratch& P = c->pfw;
+  const lgh_model_desc& d = c->d;
+  const uint32_t H = d.hidden_size, QD = d.num_heads * d.head_dim, KD = d.num_kv_heads * d.head_dim, pos0 = (uint32_t)c->pos;
+  hipStream_t st = c->stream;
+  int rc;
+  auto K = [&](hipError_t e, const char* what) -> int {
+    return e == hipSuccess ? LGH_OK : fail(c, LGH_OPERATION_FAILED, std::string("long prompt, ") + what + ": " + hipGetErrorString(e));
+  };
+  if ((rc = pf_stage_tokens(c, tokens, m, P.tokens))) return rc;
+  if ((rc = K(embed_batch_launch(c->embd_type, c->embd_raw, P.tokens, P.hidden, H, m, st), "embedding"))) return rc;
+  auto resid = [&](const float* part, const PfWide& G, const float* bias, const float* nw, const int* row_of) -> int {
+    PfwResid r{};
+    r.part = part;
+    r.S = G.S;
+    r.part_rows = G.part_rows;
+    r.row_of = row_of;
+    r.weight = P.moe_w;
+    r.top = d.num_experts_per_token;
+    r.bias = bias;
+    r.hidden = P.hidden;
+    r.H = H;
+    r.nw = nw;
+    r.x = nw ? P.x : nullptr;
+    r.inv_rms = nw ? P.inv_rms : nullptr;
+    r.eps = d.norm_eps;
+    return K(pfw_resid_launch(r, m, st), "residual");
+  };
+  if ((rc = resid(nullptr, PfWide{}, nullptr, c->layers[c->l0].attn_norm, nullptr))) return rc;
+  const float scale = 1.0f / std::sqrt((float)d.head_dim);  // layers.rs:374
+  for (uint32_t li = c->l0; li < c->l1; li++) {
+    LayerW& L = c->layers[li];
+    auto product = [&](std::initializer_list<const DevWeight*> W, const uint8_t* x, PfWide& G, int epi, uint32_t rows, const PfwGroups* grp, const char* what) -> int {
+      G.x = x;
+      if (epi == PW_PART) { G.part = P.part; G.part_bytes = P.part_bytes; }
+      else { G.act = P.act; G.act_cols = (*W.begin())->n; G.inv_rms = P.inv_rms; }
+      return K(pfw_gemm_launch(W.begin(), (int)W.size(), G, epi, rows, grp, st), what);
+    };
+    PfWide G{};
+    if ((rc = product({&L.wq, &L.wk, &L.wv}, P.x, G, PW_PART, m, nullptr, "qkv product"))) return rc;
+    const PfwQkv e{P.part, G.S, G.part_rows, QD, KD, d.head_dim, L.bq, L.bk, L.bv, c->rope_cs, P.inv_rms, pos0, d.max_seq_len, P.q, L.kcache, L.vcache, (int)d.use_neox_rope};
+    if ((rc = K(pfw_qkv_launch(e, m, st), "qkv"))) return rc;
+    if (li + 1 == c->l1) break;   // the last layer: its K / V rows are written, its output would be discarded
+    if ((rc = K(attn_prefill_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.attn, st, true), "attention"))) return rc;
+    G = PfWide{};
+    if ((rc = product({&L.wo}, P.attn, G, PW_PART, m, nullptr, "output product"))) return rc;
+    if ((rc = resid(P.part, G, L.bo, L.ffn_norm, nullptr))) return rc;
+    const float* next_nw = c->layers[li + 1].attn_norm;
+    if (!L.moe()) {
+      G = PfWide{};
+      if ((rc = product({&L.gate, &L.up}, P.x, G, PW_SWIGLU, m, nullptr, "gate | up product"))) return rc;
+      G = PfWide{};
+      if ((rc = product({&L.down}, P.act, G, PW_PART, m, nullptr, "down product"))) return rc;
+      if ((rc = resid(P.part, G, nullptr, next_nw, nullptr))) return rc;
+      continue;
+    }
+    // mixtures (moe.rs:321-413): the decode router for every token, the (token, slot) pairs grouped by expert, one row per pair
+    const uint32_t top = d.num_experts_per_token, pairs = m * top;
+    if ((rc = K(moe_router_launch(P.hidden, L.ffn_norm, d.norm_eps, L.router, H, d.num_experts, top, P.moe_sel, P.moe_w, st, m), "router"))) return rc;
+    MoeRoute R{};
+    R.M = m;
+    R.experts = d.num_experts;
+    R.top = top;
+    R.bm = kPfwTile;
+    R.sel = P.moe_sel;
+    R.w = P.moe_w;
+    R.seg = P.moe_seg;
+    R.tile_e = P.moe_tile;
+    R.tiles = moe_max_tiles(pairs, d.num_experts, kPfwTile);
+    R.tile_row = P.moe_tile + R.tiles;
+    R.slot = P.moe_slot;
+    R.src = P.moe_src;
+    R.roww = P.moe_roww;
+    if ((rc = K(moe_group_launch(R, st), "expert grouping"))) return rc;
+    PfwGroups grp{P.moe_seg, R.tile_e, R.tile_row, P.moe_src, d.num_experts, R.tiles, std::max<uint32_t>(d.num_experts, (pairs + kPfwTile - 1) / kPfwTile)};
+    G = PfWide{};
+    if ((rc = product({&L.gate_exps, &L.up_exps}, P.x, G, PW_SWIGLU, pairs, &grp, "experts' gate | up product"))) return rc;
+    grp.src = nullptr;   // the activations are rows already
+    G = PfWide{};
+    if ((rc = product({&L.down_exps}, P.act, G, PW_PART, pairs, &grp, "experts' down product"))) return rc;
+    if ((rc = resid(P.part, G, nullptr, next_nw, P.moe_slot))) return rc;
+  }
+  c->pos += m;
+  c->stats.tokens_processed += m;
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
+  return LGH_OK;
+}
+
+// n prompt tokens on the batched path
+static int prefill_tokens(lgh_ctx* c, const uint32_t* tokens, size_t n) {
+  int rc;
+  size_t i = 0;
+  const size_t least = pfw_min_tokens(c);
+  if (n >= least && pfw_eligible(c)) {
+    if ((rc = pfw_ensure(c))) return rc;
+    while (n - i >= least) {
+      const uint32_t m = (uint32_t)std::min<size_t>(c->pfw.cap, n - i);
+      if ((rc = prefill_wide(c, tokens + i, m))) return rc;
+      i += m;
+    }
+  }
+  for (; i < n; i += kPfTokens)
+    if ((rc = prefill_block(c, tokens + i, (uint32_t)std::min<size_t>(kPfTokens, n - i)))) return rc;
   return LGH_OK;
 }
 
@@ -1415,8 +1583,7 @@ int lgh_prefill_batch(lgh_ctx* c, const uint32_t* tokens, size_t n) {
       return fail(c, LGH_INVALID_ARGUMENT, "prompt of " + std::to_string(n) + " tokens at position " + std::to_string(c->pos) + " exceeds max_seq_len");
     for (size_t i = 0; i < n; i++)
       if (tokens[i] >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");
-    for (size_t i = 0; i < n; i += kPfTokens)
-      if ((rc = prefill_block(c, tokens + i, (uint32_t)std::min<size_t>(kPfTokens, n - i)))) return rc;
+    if ((rc = prefill_tokens(c, tokens, n))) return rc;
     HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
     return LGH_OK;
   }
@@ -1476,7 +1643,7 @@ int lgh_batch_prefill(lgh_ctx* c, uint32_t slot, const uint32_t* tokens, size_t 
     c->layers[i].vcache = Bs.vcache[i] + (size_t)slot * Bs.cache_stride;
   }
   c->pos = Bs.pos[slot];
-  for (size_t i = 0; i < n && !rc; i += kPfTokens) rc = prefill_block(c, tokens + i, (uint32_t)std::min<size_t>(kPfTokens, n - i));
+  rc = prefill_tokens(c, tokens, n);
   if (!rc) Bs.pos[slot] = c->pos;
   c->pos = keep;
   for (uint32_t i = c->l0; i < c->l1; i++) { c->layers[i].kcache = saved[i - c->l0].first; c->layers[i].vcache = saved[i - c->l0].second; }

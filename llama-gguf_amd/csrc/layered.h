@@ -232,6 +232,7 @@ struct MoeRoute {
 };
 uint32_t moe_max_tiles(uint32_t rows, uint32_t experts, uint32_t bm);
 hipError_t moe_route_launch(const MoeRoute& a, bool f32, hipStream_t st);   // router product, scores, groups
+hipError_t moe_group_launch(const MoeRoute& a, hipStream_t st);            // groups of pairs that are already routed (sel, w)
 
 // ---- tied_attention.hip: grouped heads, values = keys before their norm ----
 struct TiedShape {

@@ -132,6 +132,14 @@ __global__ void __launch_bounds__(1024) moe_group_rows_kernel(const MoeRoute a) 
   }
 }
 
+hipError_t moe_group_launch(const MoeRoute& a, hipStream_t st) {
+  if (!a.sel || !a.w || !a.slot || !a.src || !a.roww || !a.seg || !a.tile_e || !a.tile_row || a.M == 0 || a.top == 0 || a.experts == 0 || a.experts > kMaxExperts || a.bm == 0 ||
+      a.tiles < moe_max_tiles(a.M * a.top, a.experts, a.bm))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(moe_group_rows_kernel, dim3(1), dim3(1024), 0, st, a);
+  return hipGetLastError();
+}
+
 uint32_t moe_max_tiles(uint32_t rows, uint32_t experts, uint32_t bm) { return rows / bm + (rows < experts ? rows : experts); }
 
 hipError_t moe_route_launch(const MoeRoute& a, bool f32, hipStream_t st) {

@@ -66,13 +66,69 @@ hipError_t pf_moe_swiglu_launch(const float* part, uint32_t S, uint32_t F, uint8
 hipError_t pf_moe_combine_launch(const float* part, uint32_t S, const int* tokmap, const float* moe_w, uint32_t top_k, float* hidden, uint32_t H,
                                  const float* nw, uint8_t* xh, float* ssq, uint32_t m_tokens, hipStream_t st);
 hipError_t pf_to_xh_launch(const float* x, uint32_t K, uint8_t* xh, uint32_t m_tokens, hipStream_t st);
+// ---- long prompts (prefill_wide.hip): blocks of up to kPfwTokens tokens, row-major f16 activations [token][K] (16-byte chunks in XH's element order) ----
+constexpr uint32_t kPfwTile = 256;                // tokens of a workgroup
+constexpr uint32_t kPfwTokens = 2048;             // tokens of a block
+constexpr uint32_t kPfwMaxRows = kPfwTokens * kPfMaxTopK;   // rows of a product: tokens, or the (token, expert) pairs of a mixture
+constexpr uint32_t kPfwPartRows = 4096;           // k-splits x rows whose partial sums the buffer holds beyond one split
+constexpr int PW_PART = 0, PW_SWIGLU = 1;         // what becomes of a product: partial sums | silu(gate) * up as f16 rows
+
+struct PfwSeg {
+  const uint8_t* w;      // tile16 weights
+  uint64_t expert_stride;
+  uint32_t ntiles, col0, rg_begin;
+  int fmt;
+};
+struct PfWide {
+  PfwSeg seg[3];
+  int nseg;
+  uint32_t nblk, S, ncols, m;                      // 256-element blocks of k, k-splits, floats per row of partial sums, rows
+  const uint8_t* x;      // [row][k] f16
+  float* part;           // PW_PART: [S][part_rows][ncols]
+  size_t part_bytes;
+  uint32_t part_rows;
+  uint8_t* act;          // PW_SWIGLU: [row][act_cols] f16
+  uint32_t act_cols;
+  const float* inv_rms;  // PW_SWIGLU: per token
+  const int *src, *tile_e, *tile_row, *row_seg;    // mixtures: token of a row (null: the row itself), expert and first row of a tile, first row of an expert
+};
+// rows grouped by expert: at most `tiles` tiles of kPfwTile rows, about `likely` of them used
+struct PfwGroups { const int *seg, *tile_e, *tile_row, *src; uint32_t experts, tiles, likely; };
+struct PfwResid {
+  const float* part;     // null: the hidden rows as they are
+  uint32_t S, part_rows;
+  const int* row_of;     // mixtures: row of (token, slot)
+  const float* weight;
+  uint32_t top;
+  const float* bias;
+  float* hidden;
+  uint32_t H;
+  const float* nw;       // norm weight of the next product's input
+  uint8_t* x;            // that input, or null
+  float* inv_rms;
+  float eps;
+};
+struct PfwQkv {
+  const float* part;
+  uint32_t S, part_rows, QD, KD, head_dim;
+  const float *bq, *bk, *bv, *rope_cs, *inv_rms;
+  uint32_t pos0, max_seq;
+  float *q, *kcache, *vcache;
+  int neox;
+};
+bool pfw_pairs(const DevWeight* gate, const DevWeight* up);      // the two can run as one PW_SWIGLU product
+size_t pfw_part_bytes(uint32_t max_rows, uint32_t cols);
+// up to 3 matrices on the same input; G: x, and part / part_bytes or act / act_cols / inv_rms; S and ncols come back in it
+hipError_t pfw_gemm_launch(const DevWeight* const* W, int nw, PfWide& G, int epi, uint32_t rows, const PfwGroups* grp, hipStream_t st);
+hipError_t pfw_resid_launch(const PfwResid& a, uint32_t m_tokens, hipStream_t st);
+hipError_t pfw_qkv_launch(const PfwQkv& a, uint32_t m_tokens, hipStream_t st);
 // dequant.hip: rows tokens[0..m) of the embedding table -> dst[m][hidden]
 hipError_t embed_batch_launch(int src_type, const uint8_t* table, const int* tokens, float* dst, uint32_t hidden, uint32_t m_tokens,
                               hipStream_t st);
 // attention.hip: causal attention of a block of m tokens at positions pos0 .. pos0+m-1 (their K/V rows already cached)
 hipError_t attn_prefill_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv,
                                uint32_t head_dim, uint32_t max_seq, float scale, uint32_t pos0, uint32_t m_tokens, uint8_t* xh_out,
-                               hipStream_t st);
+                               hipStream_t st, bool rows = false);   // rows: xh_out is row-major (prefill_wide.hip)
 // byte offset of element k of token t in an XH matrix
 __host__ __device__ inline size_t xh_offset(uint32_t t, uint32_t k) {
   const uint32_t ch = k >> 3, j = k & 7, pj = (j == 1 || j == 5) ? j + 1 : (j == 2 || j == 6) ? j - 1 : j;

@@ -31,26 +31,12 @@
 // read from LDS feeds 4 MFMAs (LDS at 50 % of its bandwidth), 128 f32 accumulators per lane.  K is split over
 // gridDim.y workgroups to fill the chip; the f32 partial sums [split][token][column] are added up by the row-wise
 // kernel that consumes them (together with bias, RoPE, residual, RMSNorm, SwiGLU).
-// Weights are dequantized as w * 2^8 (kPfScale) to keep small block scales out of the f16 subnormals; |w| < 256 is
-// assumed (f16 overflow otherwise) — GGUF weights are O(1).
 #include "device_utils.h"
 #include "mv_epilogue.h"
 #include "prefill.h"
+#include "prefill_dequant.h"
 
 namespace lgh {
-
-typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
-
-// formats as in matvec_mfma.hip (same tile16 layouts)
-enum : int { PF_Q4K = 0, PF_Q6K = 1, PF_Q5K = 2, PF_Q80 = 3, PF_Q40 = 4 };
-__host__ __device__ constexpr uint32_t pf_tile_bytes(int f) {
-  return f == PF_Q4K ? 2304u : f == PF_Q6K ? 3392u : f == PF_Q5K ? 2816u : f == PF_Q80 ? 4352u : 2304u;
-}
-static int pf_fmt_of(int dev_type) {
-  return dev_type == kDevQ4K_T16 ? PF_Q4K : dev_type == kDevQ6K_T16 ? PF_Q6K : dev_type == kDevQ5K_T16 ? PF_Q5K
-         : dev_type == kDevQ80_T16 ? PF_Q80 : dev_type == kDevQ40_T16 ? PF_Q40 : -1;
-}
 
 // waves per workgroup: 4 (one per SIMD, 4 row tiles each).  8 waves of 2 tiles (-DPF_WAVES=8: two per SIMD, twice the LDS
 // reads per MFMA) measured the same 4.68 ms per 128-token Llama-3-8B prompt: the loop is not latency-bound.
@@ -66,7 +52,6 @@ static int pf_fmt_of(int dev_type) {
 constexpr int kPfWaves = PF_WAVES;
 constexpr int kPfRT = 16 / kPfWaves;     // row tiles per wave (a workgroup covers 256 rows)
 constexpr int kPfMT = kPfTokens / 16;    // token tiles of a full block
-constexpr float kPfScale = 256.0f;
 
 #ifdef LGH_STAMPS
 // diagnostic build: per-workgroup phase stamps (100 MHz s_memrealtime) of the GEMM launches whose output is LGH_PF_STAMP_COLS wide
@@ -87,120 +72,6 @@ hipError_t pf_read_stamps(unsigned long long* host, size_t n) {
 #else
 #define LGH_PF_STAMP(i)
 #endif
-
-struct PfRaw { u32x4 hd; u32x4 q[4]; };
-
-template <int F>
-__device__ __forceinline__ void pf_load(PfRaw& r, const uint8_t* tile, uint32_t lane, uint32_t n) {
-  if (F == PF_Q6K) {
-    r.hd = ldg_nt128(tile + 3072 + n * 16);
-#pragma unroll
-    for (int i = 0; i < 3; i++) r.q[i] = ldg_nt128(tile + i * 1024 + lane * 16);
-    r.q[3].x = ldg_nt32(tile + 3328 + (n >> 1) * 4);
-  } else if (F == PF_Q80) {
-    r.hd = ldg_nt128(tile + 4096 + n * 16);
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.q[i] = ldg_nt128(tile + i * 1024 + lane * 16);
-  } else {
-    r.hd = ldg_nt128(tile + 2048 + n * 16);
-    r.q[0] = ldg_nt128(tile + lane * 16);
-    r.q[1] = ldg_nt128(tile + 1024 + lane * 16);
-    if (F == PF_Q5K) {
-      const u32x2 h = ldg_nt64(tile + 2304 + lane * 8);
-      r.q[2].x = h.x;
-      r.q[2].y = h.y;
-    }
-  }
-}
-
-__device__ __forceinline__ h16x2 pf_bcast(float v) {
-  const _Float16 h = (_Float16)v;
-  h16x2 r = {h, h};
-  return r;
-}
-
-// scale S and offset O (both times kPfScale, as f16 pairs) of MFMA step pp of the lane's row n and k-chunk c:
-// weight = S * u + O with u the unsigned stored quant
-template <int F>
-__device__ __forceinline__ void pf_scale(const PfRaw& r, int pp, uint32_t n, uint32_t c, h16x2& S, h16x2& O) {
-  if (F == PF_Q6K) {   // y = d * sc * (q' - 32), one int8 scale per 16 elements (dequant.rs:321-356)
-    const uint32_t hdw = pp == 0 ? r.hd.x : pp == 1 ? r.hd.y : pp == 2 ? r.hd.z : r.hd.w;
-    const float scf = (float)(int)__builtin_amdgcn_sbfe((int)hdw, c * 8, 8);
-    const uint32_t dh = (n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu;
-    S = pf_bcast(h2f(dh) * scf * kPfScale);
-    O = S * pf_bcast(-32.0f);
-  } else if (F == PF_Q80 || F == PF_Q40) {   // y = d * q (Q8_0, stored q + 128 after the sign flip) / d * (q - 8) (Q4_0)
-    const uint32_t hdw = pp == 0 ? r.hd.x : pp == 1 ? r.hd.y : pp == 2 ? r.hd.z : r.hd.w;
-    const float dd = h2f((c >> 1) ? hdw >> 16 : hdw & 0xFFFFu);
-    S = pf_bcast(dd * kPfScale);
-    O = S * pf_bcast(F == PF_Q80 ? -128.0f : -8.0f);
-  } else {   // Q4_K / Q5_K: y = d * sc * q - dmin * m, 6-bit (sc, m) per 32 elements (dequant.rs:210-255)
-    const uint32_t s8 = (c >> 1) * 8;
-    const uint32_t a = (r.hd.y >> s8) & 0x00FF00FFu, bq = (r.hd.z >> s8) & 0x00FF00FFu, cq = (r.hd.w >> s8) & 0x00FF00FFu;
-    uint32_t sc, mn;
-    if (pp < 2) {
-      const uint32_t sc01 = a & 0x003F003Fu, mn01 = bq & 0x003F003Fu;
-      sc = pp == 0 ? sc01 & 0xFFu : sc01 >> 16;
-      mn = pp == 0 ? mn01 & 0xFFu : mn01 >> 16;
-    } else {
-      const uint32_t sc23 = (cq & 0x000F000Fu) | ((a >> 2) & 0x00300030u);
-      const uint32_t mn23 = ((cq >> 4) & 0x000F000Fu) | ((bq >> 2) & 0x00300030u);
-      sc = pp == 2 ? sc23 & 0xFFu : sc23 >> 16;
-      mn = pp == 2 ? mn23 & 0xFFu : mn23 >> 16;
-    }
-    const float dd = h2f(r.hd.x & 0xFFFFu), dmin = h2f(r.hd.x >> 16);
-    S = pf_bcast(dd * (float)sc * kPfScale);
-    O = pf_bcast(-(dmin * (float)mn) * kPfScale);
-  }
-}
-
-// four words of two f16 (0x6400 | u == 1024 + u exactly) -> S * u + O.  Stage by stage over the four words (not word by
-// word): a packed-f16 op that consumes the previous instruction's result costs an extra s_nop on gfx950.
-__device__ __forceinline__ h16x8 pf_fin4(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3, h16x2 S, h16x2 O) {
-  const h16x2 k = {(_Float16)1024.0f, (_Float16)1024.0f};
-  const h16x2 u0 = __builtin_bit_cast(h16x2, b0) - k, u1 = __builtin_bit_cast(h16x2, b1) - k;
-  const h16x2 u2 = __builtin_bit_cast(h16x2, b2) - k, u3 = __builtin_bit_cast(h16x2, b3) - k;
-  const h16x2 w0 = __builtin_elementwise_fma(u0, S, O), w1 = __builtin_elementwise_fma(u1, S, O);
-  const h16x2 w2 = __builtin_elementwise_fma(u2, S, O), w3 = __builtin_elementwise_fma(u3, S, O);
-  h16x8 r = {w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
-  return r;
-}
-
-// eight nibbles (word byte t = w[t] | w[t+4] << 4) -> f16 in the order w0 w2 w1 w3 w4 w6 w5 w7
-__device__ __forceinline__ h16x8 pf_frag_nib(uint32_t N, h16x2 S, h16x2 O) {
-  const uint32_t m = opaque(0x000F000Fu), e = 0x64006400u;   // mask in a VGPR: (x & m) | e is then one v_and_or_b32
-  return pf_fin4((N & m) | e, ((N >> 8) & m) | e, ((N >> 4) & m) | e, ((N >> 12) & m) | e, S, O);
-}
-// eight bytes (B0 = w0..w3, B1 = w4..w7) -> f16 in the same order
-__device__ __forceinline__ h16x8 pf_frag_bytes(uint32_t B0, uint32_t B1, h16x2 S, h16x2 O) {
-  const uint32_t e = 0x64646464u;
-  return pf_fin4(__builtin_amdgcn_perm(e, B0, 0x04020400u), __builtin_amdgcn_perm(e, B0, 0x04030401u),
-                 __builtin_amdgcn_perm(e, B1, 0x04020400u), __builtin_amdgcn_perm(e, B1, 0x04030401u), S, O);
-}
-
-// the A operand of MFMA (pp, h): elements 64pp + 16c + 8h .. +7 of row n, dequantized
-template <int F>
-__device__ __forceinline__ h16x8 pf_frag(const PfRaw& r, int pp, int h, h16x2 S, h16x2 O) {
-  if (F == PF_Q80) {
-    const u32x4 b = r.q[pp];
-    const uint32_t B0 = (h ? b.z : b.x) ^ 0x80808080u, B1 = (h ? b.w : b.y) ^ 0x80808080u;
-    return pf_frag_bytes(B0, B1, S, O);
-  }
-  const uint32_t N0 = (pp & 1) ? r.q[pp >> 1].z : r.q[pp >> 1].x, N1 = (pp & 1) ? r.q[pp >> 1].w : r.q[pp >> 1].y;
-  const uint32_t N = h ? N1 : N0;
-  if (F == PF_Q4K || F == PF_Q40) return pf_frag_nib(N, S, O);
-  uint32_t B0 = N & 0x0F0F0F0Fu, B1 = (N >> 4) & 0x0F0F0F0Fu;
-  if (F == PF_Q6K) {   // H byte t = f[t] | f[t+4] << 2 | f[t+8] << 4 | f[t+12] << 6 (the two high bits of the chunk's 16 weights)
-    const uint32_t H = pp == 0 ? r.q[2].x : pp == 1 ? r.q[2].y : pp == 2 ? r.q[2].z : r.q[2].w;
-    B0 |= ((H >> (4 * h)) & 0x03030303u) << 4;
-    B1 |= ((H >> (4 * h + 2)) & 0x03030303u) << 4;
-  } else {             // Q5_K: fifth bits, dword of the step pair, low nibbles = even step, high nibbles = odd step
-    const uint32_t H = ((pp >> 1) ? r.q[2].y : r.q[2].x) >> (4 * (pp & 1));
-    B0 |= ((H >> (2 * h)) & 0x01010101u) << 4;
-    B1 |= ((H >> (2 * h + 1)) & 0x01010101u) << 4;
-  }
-  return pf_frag_bytes(B0, B1, S, O);
-}
 
 // MT = token tiles computed: 8 for a full block, 4 / 2 when at most 64 / 32 rows are real (short prompts, and the rows routed
 // to one MoE expert — about 32 of 128 with 2-of-8 routing): the MFMAs, the LDS reads and the activation DMA shrink with it.

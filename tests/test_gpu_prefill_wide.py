@@ -1,0 +1,64 @@
+"""Prompts of 256 tokens (mixtures 160) and more (prefill_wide.hip): the cache they leave, seen through the logits of the tokens that follow, against the exact
+engine (f32 throughout, token by token).
+
+Tolerance: that of the 128-token blocks, 1e-2 * max|logit| + 1e-2: the operands of every product are rounded to f16 (2^-12 each) in both paths, and
+the rounding of a layer's output is carried on by the next ones; measured 1e-3 to 3e-3 of the largest logit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _engines(pkg, name, mix, max_seq, **over):
+    cfg = pkg.make_config(name, max_seq_len=max_seq, **over)
+    model = pkg.SynthModel(cfg, mix=mix, with_bias=bool(over.get("use_neox_rope")))
+    return cfg, pkg.HipGpuInference.from_model(model, max_seq, flags=pkg.hip_backend.FLAG_EXACT_PREFILL), pkg.HipGpuInference.from_model(model, max_seq)
+
+
+def _follow(a, b, toks):
+    for t in toks:
+        want, got = a.forward(t), b.forward(t)
+        assert np.abs(got - want).max() <= 1e-2 * float(np.abs(want).max()) + 1e-2
+
+
+@pytest.mark.parametrize("name,mix,n,over", [
+    ("test-dense", "Q4_K_M", 256, {}), ("test-dense", "Q4_K_M", 257, {}), ("test-dense", "Q5_K_M", 384, {}), ("test-dense", "Q8_0", 511, {}),
+    ("test-dense", "Q4_0", 513, {}), ("test-dense", "Q6_K", 641, {}),                       # edges of the 256- and 128-token tiles, every format
+    ("test-dense-d128", "Q4_K_M", 300, {}), ("test-dense-d128", "Q5_K_M", 700, dict(use_neox_rope=1)),     # 11 k-blocks; biases and halves
+    ("test-dense-d128", "Q4_K_M", 2304, {}),                                                # a full block and a remainder of its own
+    ("test-moe", "Q5_K_M", 160, {}), ("test-moe", "Q5_K_M", 259, {}), ("test-moe", "Q4_K_M", 600, {}), ("test-moe", "Q8_0", 400, {})])
+def test_long_prompts_match_the_exact_engine(pkg, name, mix, n, over):
+    cfg, exact, wide = _engines(pkg, name, mix, n + 16, **over)
+    prompt = [(7 * i + 3) % cfg.vocab_size for i in range(n)]
+    for eng in (exact, wide):
+        eng.forward_batch(prompt)
+        assert eng.position() == n
+    _follow(exact, wide, (5, 77, 9))
+    wide.reset()                                             # the same prompt again: bit for bit
+    wide.forward_batch(prompt)
+    first = wide.forward(5)
+    wide.reset()
+    wide.forward_batch(prompt)
+    assert np.array_equal(wide.forward(5), first)
+    exact.close()
+    wide.close()
+
+
+def test_long_prompts_continue_a_sequence_and_fill_slots(pkg):
+    cfg, exact, wide = _engines(pkg, "test-dense", "Q4_K_M", 700)
+    a, b = [(5 * i + 1) % cfg.vocab_size for i in range(37)], [(11 * i + 2) % cfg.vocab_size for i in range(419)]
+    for eng in (exact, wide):
+        eng.forward_batch(a)
+        eng.forward(77)
+        eng.forward_batch(b)
+        assert eng.position() == 457
+    _follow(exact, wide, (3, 4))
+    wide.batch_create(3)
+    wide.batch_prefill(2, b)
+    exact.reset()
+    exact.forward_batch(b)
+    want, got = exact.forward(8), wide.forward_multi([2], [8])[0][0]
+    assert np.abs(got - want).max() <= 1e-2 * float(np.abs(want).max()) + 1e-2
+    assert wide.position() == 459    # the context's own sequence is where it was
+    exact.close()
+    wide.close()
