@@ -572,7 +572,7 @@ hipError_t attn_direct_launch(const float* q, const float* kcache, const float* 
 template <int D, int NW>
 __global__ void __launch_bounds__(NW * 64) attn_pf_mfma_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
                                                                uint32_t n_heads, uint32_t g_per_kv, uint32_t max_seq, float scale, uint32_t pos0,
-                                                               uint32_t m_tokens, uint8_t* __restrict__ xh_out, int rows) {
+                                                               uint32_t m_tokens, uint8_t* __restrict__ xh_out) {
   constexpr int DJ = D / 4;    // contraction steps of S^T (dims per lane group)
   constexpr int DQ = D / 16;   // output dims per M index
   constexpr int DP = D + 4;    // padded row of the merge buffer
@@ -682,20 +682,19 @@ __global__ void __launch_bounds__(NW * 64) attn_pf_mfma_kernel(const float* __re
       a += s_o[w][t][dim] * f;
     }
     const _Float16 o = (_Float16)(a * (1.0f / lsum));   // simd.rs:718-720: multiply by 1/sum
-    const uint32_t k = head * D + dim;   // row-major: the chunk's element order is XH's, its place is not
-    *reinterpret_cast<_Float16*>(xh_out + (rows ? ((size_t)(tt * 16 + t) * n_heads * D + (k & ~7u)) * 2 + (xh_offset(0, k) & 15) : xh_offset(tt * 16 + t, k))) = o;
+    *reinterpret_cast<_Float16*>(xh_out + xh_offset(tt * 16 + t, head * D + dim)) = o;
   }
 }
 
 template <int D>
 static hipError_t attn_pf_mfma_go(const float* q, const float* kc, const float* vc, uint32_t n_heads, uint32_t g, uint32_t max_seq, float scale,
-                                  uint32_t pos0, uint32_t m_tokens, uint8_t* xh_out, hipStream_t st, bool rows) {
+                                  uint32_t pos0, uint32_t m_tokens, uint8_t* xh_out, hipStream_t st) {
   constexpr int NW = 8;   // (4 waves: 11.7 us per layer of a 128-token Llama-3-8B prompt, the last token tile's waves take two kv tiles each)
   constexpr size_t lds = (size_t)(NW * 16 * (D + 4) + 2 * NW * 16) * 4;
   static bool attr_set[64] = {};
   if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&attn_pf_mfma_kernel<D, NW>), (int)lds, attr_set); e != hipSuccess) return e;
   hipLaunchKernelGGL((attn_pf_mfma_kernel<D, NW>), dim3(n_heads, (m_tokens + 15) / 16), dim3(NW * 64), lds, st, q, kc, vc, n_heads, g, max_seq, scale,
-                     pos0, m_tokens, xh_out, (int)rows);
+                     pos0, m_tokens, xh_out);
   return hipGetLastError();
 }
 
@@ -711,13 +710,13 @@ static hipError_t attn_pf_go(const float* q, const float* kc, const float* vc, u
 
 hipError_t attn_prefill_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv,
                                uint32_t head_dim, uint32_t max_seq, float scale, uint32_t pos0, uint32_t m_tokens, uint8_t* xh_out,
-                               hipStream_t st, bool rows) {
+                               hipStream_t st) {
   if (n_kv == 0 || n_heads % n_kv || m_tokens == 0) return hipErrorInvalidValue;
   const uint32_t g = n_heads / n_kv;
   static const bool valu = [] { const char* e = std::getenv("LGH_PF_ATTN_VALU"); return e && std::atoi(e) != 0; }();   // (A/B switch: the VALU kernel)
-  if ((!valu || rows) && (head_dim == 128 || head_dim == 64)) {
-    return head_dim == 128 ? attn_pf_mfma_go<128>(q, kcache, vcache, n_heads, g, max_seq, scale, pos0, m_tokens, xh_out, st, rows)
-                           : attn_pf_mfma_go<64>(q, kcache, vcache, n_heads, g, max_seq, scale, pos0, m_tokens, xh_out, st, rows);
+  if (!valu && (head_dim == 128 || head_dim == 64)) {
+    return head_dim == 128 ? attn_pf_mfma_go<128>(q, kcache, vcache, n_heads, g, max_seq, scale, pos0, m_tokens, xh_out, st)
+                           : attn_pf_mfma_go<64>(q, kcache, vcache, n_heads, g, max_seq, scale, pos0, m_tokens, xh_out, st);
   }
 #define LGH_ATTN_CASE(DD, GG) \
   if (head_dim == DD && g == GG) return attn_pf_go<DD, GG>(q, kcache, vcache, n_kv, max_seq, scale, pos0, m_tokens, xh_out, st);

@@ -51,6 +51,7 @@ struct PfScratch {
 struct PfwScratch {
   uint32_t cap = 0;                    // 0: not allocated
   uint8_t *x = nullptr, *attn = nullptr, *act = nullptr;   // row-major f16: [cap][hidden], [cap][QD], [rows][ffn]
+  uint8_t* kv_split = nullptr;         // a layer's cache rows for attention_wide.hip
   float *hidden = nullptr, *q = nullptr, *part = nullptr, *inv_rms = nullptr, *moe_w = nullptr, *moe_roww = nullptr;
   size_t part_bytes = 0;
   int *tokens = nullptr, *moe_sel = nullptr, *moe_seg = nullptr, *moe_tile = nullptr, *moe_slot = nullptr, *moe_src = nullptr;

@@ -982,6 +982,7 @@ static int pfw_ensure(lgh_ctx* c) {
       {(void**)&P.x, (size_t)cap * H * 2},      {(void**)&P.attn, (size_t)cap * QD * 2},   {(void**)&P.act, act * 2},
       {(void**)&P.hidden, (size_t)cap * H * 4}, {(void**)&P.q, (size_t)cap * QD * 4},      {(void**)&P.part, pb},
       {(void**)&P.inv_rms, (size_t)cap * 4},    {(void**)&P.tokens, (size_t)cap * 4},
+      {(void**)&P.kv_split, attn_wide_bytes(d.num_kv_heads, d.head_dim, d.max_seq_len)},
       {(void**)&P.moe_sel, (size_t)pairs * 4},  {(void**)&P.moe_w, (size_t)pairs * 4},     {(void**)&P.moe_roww, (size_t)pairs * 4},
       {(void**)&P.moe_slot, (size_t)pairs * 4}, {(void**)&P.moe_src, (size_t)pairs * 4},   {(void**)&P.moe_tile, (size_t)tiles * 8},
       {(void**)&P.moe_seg, any_moe ? (size_t)(d.num_experts + 1) * 4 : 0},
@@ -1041,7 +1042,7 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
     const PfwQkv e{P.part, G.S, G.part_rows, QD, KD, d.head_dim, L.bq, L.bk, L.bv, c->rope_cs, P.inv_rms, pos0, d.max_seq_len, P.q, L.kcache, L.vcache, (int)d.use_neox_rope};
     if ((rc = K(pfw_qkv_launch(e, m, st), "qkv"))) return rc;
     if (li + 1 == c->l1) break;   // the last layer: its K / V rows are written, its output would be discarded
-    if ((rc = K(attn_prefill_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.attn, st, true), "attention"))) return rc;
+    if ((rc = K(attn_wide_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.kv_split, P.attn, st), "attention"))) return rc;
     G = PfWide{};
     if ((rc = product({&L.wo}, P.attn, G, PW_PART, m, nullptr, "output product"))) return rc;
     if ((rc = resid(P.part, G, L.bo, L.ffn_norm, nullptr))) return rc;
