@@ -1,5 +1,5 @@
 // prefill_wide.hip — long prompts: products of quantized weights with up to kPfwTokens prompt tokens at once on the f16 matrix cores
-// (v_mfma_f32_16x16x32_f16), and the row kernels around them.
+// (v_mfma_f32_32x32x16_f16), and the row kernels around them.
 //
 // prefill.hip takes 128 tokens per weight read; its loop is bound by the vector issue port, because every weight is dequantized for 128
 // tokens only, and a product of 128 tokens must be split over k to fill the chip, which costs partial sums and a row kernel to fold them.
@@ -9,8 +9,10 @@
 // Activations: row-major f16, [token][K], the eight elements of a 16-byte chunk in the order 0,2,1,3,4,6,5,7 (the order in which two masks pull
 // nibbles out of a tile16 word, as in prefill.h's XH).  Same operands, same rounding points and f32 accumulation as prefill.hip.
 //
-// Measured: 2047 tokens of Llama-3-8B Q4_K_M widths, 16 layers, 42.1 -> 23.8 ms (gate | up 0.52 ms a layer, 0.93 PFLOP/s); 600 tokens of Mixtral
-// widths, 2 layers, 2.95 -> 1.48 ms.
+// Measured: 2047 tokens of Llama-3-8B Q4_K_M widths, 16 layers: 42.1 ms in blocks of 128, 16.4 ms here with attention_wide.hip (gate | up 0.44 ms a layer =
+// 1.09 PFLOP/s; torch's f16 product of 8192^3 reaches 1.14); 600 tokens of Mixtral widths, 2 layers: 2.95 and 1.21 ms.  What bounds it: the chip's power
+// before any single unit (the same loop without the dequantization takes 26 % less time, without the activations' DMA 22 %, without the stores 11 %).
+// Eight waves of half the tokens each (two per SIMD, weights dequantized twice) took the same time.
 #include "mv_epilogue.h"
 #include "prefill_dequant.h"
 
@@ -18,6 +20,7 @@ namespace lgh {
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWWaves = 4, kWRT = 4;                      // waves of a workgroup, 16-row weight tiles of a wave
 constexpr uint32_t kWStepBytes = kPfwTile * 128;          // 64 elements of 256 tokens
@@ -37,49 +40,49 @@ constexpr uint32_t pw_lds(int f) {
                        : pw_bufs<PF_Q40>() * kWStepBytes + kWWaves * pw_raw_bytes<PF_Q40>();
 }
 
-// 16 bytes per lane from global memory into LDS at lds + 16 * lane.  Inline assembly: the compiler's wait-count pass does not see these loads
-// (it would wait for all of them before any LDS read); the loop below waits by hand.
+// 16 bytes per lane from global memory into LDS at lds + 16 * lane.  Inline assembly: the compiler's wait-count pass does not see these loads (it would wait
+// for all of them before any LDS read); the loop below waits by hand.
 __device__ __forceinline__ void pw_dma(const uint8_t* base, uint32_t off, uint32_t lds) {
-  uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
 // all but the last N vector-memory operations of this wave have completed
 template <uint32_t N> __device__ __forceinline__ void pw_wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
 
-// acc += a b.  Inline assembly for its register class: 256 accumulators fill the accumulation registers, and with the builtin the allocator moves them
-// about inside the loop (1 284 copies beside 512 MFMAs).  The compiler knows no wait states for it: operands written by a vector instruction are
-// at least two instructions old here (a half step, one region), and the epilogue waits before it reads the sums.
-__device__ __forceinline__ void pw_mma(f32x4& acc, h16x8 a, h16x8 b) { asm("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b)); }
-// keeps reads of these sums behind the wait in front of the epilogue, and one token tile's behind the stores of the one before
-__device__ __forceinline__ void pw_settle(f32x4& a, f32x4& b, f32x4& c, f32x4& d) { asm volatile("" : "+a"(a), "+a"(b), "+a"(c), "+a"(d) : : "memory"); }
+// The 32 x 32 shape: with one wave per SIMD the 16 x 16 x 32 one sustains 1.25 PFLOP/s on this chip, this one 1.66 (random operands, nothing but MFMAs).
+__device__ __forceinline__ void pw_mma(f32x16& acc, h16x8 a, h16x8 b) { acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc, 0, 0, 0); }
+// keeps a token tile's sums in their accumulation registers until the stores of the one before are under way (read all at once they spill)
+__device__ __forceinline__ void pw_settle(f32x16& a, f32x16& b) { asm volatile("" : "+a"(a), "+a"(b) : : "memory"); }
 
-template <int F> __device__ __forceinline__ void pw_raw_read(PfRaw& w, const uint8_t* raw, int r, uint32_t lane, uint32_t n) {
+// raw weights of row n of tile r as lane `l16` of the 16-row scheme holds them (chunk l16 >> 4 of every 64 elements)
+template <int F> __device__ __forceinline__ void pw_raw_read(PfRaw& w, const uint8_t* raw, uint32_t r, uint32_t l16, uint32_t n) {
   constexpr uint32_t nf = pw_full<F>();
-  const uint8_t* full = raw + r * nf * 1024 + lane * 16;
-  const uint8_t* tail = raw + kWRT * nf * 1024 + r * pw_tail<F>() * 16;
+  const uint8_t* full = raw + r * (nf * 1024) + l16 * 16;
+  const uint8_t* tail = raw + kWRT * nf * 1024 + r * (pw_tail<F>() * 16);
   w.hd = *reinterpret_cast<const u32x4*>(tail + n * 16);
 #pragma unroll
   for (int i = 0; i < (int)nf; i++) w.q[i] = *reinterpret_cast<const u32x4*>(full + i * 1024);
   if (F == PF_Q6K) w.q[3].x = *reinterpret_cast<const uint32_t*>(tail + 256 + (n >> 1) * 4);
   if (F == PF_Q5K) {
-    const u32x2 h = *reinterpret_cast<const u32x2*>(tail + 256 + lane * 8);
+    const u32x2 h = *reinterpret_cast<const u32x2*>(tail + 256 + l16 * 8);
     w.q[2].x = h.x;
     w.q[2].y = h.y;
   }
 }
 
-// One workgroup: 16 row tiles x up to MT token tiles over the k-blocks [b0, b1).  Per step of 64 elements a wave runs 2 * 4 * MT MFMAs on its own
-// 64 rows; their A operands are dequantized in registers one half step ahead, the B operands (all tokens) are read from LDS three ahead.
+// One workgroup: 16 row tiles x up to TT token tiles of 32 over the k-blocks [b0, b1).  A wave's four 16-row tiles are two of 32 rows: lane 32g + 16s + n
+// holds row n of tile 2v + s, and of every 64 elements the two 16-element chunks 2g + j that the tile16 layout keeps for lanes 16(2g + j) + n.  A step of
+// 64 elements has four phases (j, h), each the contraction of elements 16(2g + j) + 8h .. + 7 of both g, 2 * TT MFMAs.  A operands are dequantized in
+// registers one phase ahead, B operands (all tokens) are read from LDS three units ahead.
 // What arrives by DMA: the activations of the step after next (256 tokens x 128 bytes, shared by the waves), and per 256 elements the wave's own raw
 // weights.  The barrier stands three units before a step's end, where every read of the step's buffer has returned, so that the next step's first
 // operands are under way when its first MFMA issues.
-template <int F, int MT, bool GRP, int EPI>
+template <int F, int TT, bool GRP, int EPI>
 __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint32_t rg, uint32_t ks, uint32_t m0, uint32_t m_end, uint32_t expert, uint8_t* smem) {
-  constexpr uint32_t tb = pf_tile_bytes(F), NB = pw_bufs<F>(), DIST = NB - 1, NX = MT / 2;   // NX: activation DMA operations per wave and step
-  constexpr int UN = 2 * MT, AHEAD = 3;                                                       // units (half, token tile) of a step
+  constexpr uint32_t tb = pf_tile_bytes(F), NB = pw_bufs<F>(), DIST = NB - 1;
+  constexpr int NX = TT;   // NX: activation DMA operations per wave and step
+  constexpr int UN = 4 * TT, AHEAD = 3;                                                     // units (phase, token tile) of a step
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t n = lane & 15, c = lane >> 4;
+  const uint32_t n = lane & 15, g = lane >> 5, tk = lane & 31, sub = lane >> 4 & 1;
   const uint32_t per = (G.nblk + G.S - 1) / G.S, b0 = ks * per, b1 = b0 + per < G.nblk ? b0 + per : G.nblk;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   const uint32_t raw_at = NB * kWStepBytes + wave * pw_raw_bytes<F>();
@@ -108,65 +111,74 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
     const uint8_t* w = r == 0 ? wbase[0] : r == 1 ? wbase[1] : r == 2 ? wbase[2] : wbase[3];
     tail_src[i] = (uint64_t)(uintptr_t)(w + pw_full<F>() * 1024 + j * 16);
   }
-  auto raw_dma = [&](uint32_t b) {
-    const uint32_t at = lds0 + raw_at;
+  constexpr int R = (int)pw_raw_ops<F>(), NF = (int)pw_full<F>();
+  auto raw_dma = [&](int k, uint32_t b) {   // operation k of a block's raw weights
+    const uint32_t at = lds0 + raw_at + k * 1024;
     const size_t bo = (size_t)b * tb;
-#pragma unroll
-    for (int r = 0; r < kWRT; r++)
-#pragma unroll
-      for (int i = 0; i < (int)pw_full<F>(); i++) pw_dma(wbase[r] + bo, lane * 16 + i * 1024, at + (r * pw_full<F>() + i) * 1024);
-#pragma unroll
-    for (int i = 0; i < (int)pw_tail_ops<F>(); i++) {
-      const uint8_t* src = reinterpret_cast<const uint8_t*>(tail_src[i]) + bo;
-      uint32_t keep;
-      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                   : "=&s"(keep) : "v"(src), "s"(at + (kWRT * pw_full<F>() + i) * 1024) : "memory");
+    if (k < kWRT * NF) {
+      pw_dma(wbase[k / NF] + bo + k % NF * 1024, lane * 16, at);
+    } else {
+      const uint8_t* src = reinterpret_cast<const uint8_t*>(tail_src[k - kWRT * NF]) + bo;
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(at) : "memory", "m0");
     }
   };
   // activations: an operation covers 8 tokens x 128 bytes; chunk q of token t lies at position q ^ (t & 7)
   uint32_t xoff[NX];
 #pragma unroll
   for (int i = 0; i < (int)NX; i++) {
-    const uint32_t row = (i * kWWaves + wave) * 8 + (lane >> 3);
+    const uint32_t row = (wave * NX + i) * 8 + (lane >> 3);
     uint32_t m = m0 + row < m_end ? m0 + row : m_end - 1;
     if (GRP && G.src) m = (uint32_t)G.src[m];
     xoff[i] = m * (G.nblk * 512u) + (((lane & 7) ^ (row & 7)) << 4);
   }
   const uint32_t s0 = b0 * 4, s1 = b1 * 4;   // steps of 64 elements
-  auto x_dma = [&](uint32_t s, uint32_t buf) {
+  // regions of a step; raw operations per region, spread over a block's first two steps, and how many of them each of the two makes
+  constexpr int RS = UN / 4, RP = (R + 2 * RS - 1) / (2 * RS), R0 = R < RS * RP ? R : RS * RP, R1 = R - R0;
+  static_assert((int)NX == RS, "one activation operation per region");
+  auto x_dma = [&](int i, uint32_t s, uint32_t buf) {   // operation i of a step's activations
     const uint8_t* base = G.x + (size_t)(s < s1 ? s : s1 - 1) * 128;   // past the end: requested again, never read
-#pragma unroll
-    for (int i = 0; i < (int)NX; i++) pw_dma(base, xoff[i], lds0 + buf * kWStepBytes + (i * kWWaves + wave) * 1024);
+    pw_dma(base, xoff[i], lds0 + buf * kWStepBytes + (wave * NX + i) * 1024);
   };
 
-  f32x4 acc[kWRT][MT];
+  f32x16 acc[2][TT];
 #pragma unroll
-  for (int r = 0; r < kWRT; r++)
+  for (int v = 0; v < 2; v++)
 #pragma unroll
-    for (int t = 0; t < MT; t++) acc[r][t] = (f32x4)(0.0f);
+    for (int t = 0; t < TT; t++) acc[v][t] = (f32x16)(0.0f);
 
-  raw_dma(b0);
-  x_dma(s0, 0);
-  if (NB == 3) x_dma(s0 + 1, 1);
+#pragma unroll
+  for (int k = 0; k < R; k++) raw_dma(k, b0);
+#pragma unroll
+  for (int i = 0; i < NX; i++) x_dma(i, s0, 0);
+  if (NB == 3) {
+#pragma unroll
+    for (int i = 0; i < NX; i++) x_dma(i, s0 + 1, 1);
+  }
   pw_wait_vm<NB == 3 ? NX : 0>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
-  const uint32_t bo0 = n * 128 + (((2 * c) ^ (n & 7)) << 4), bo1 = n * 128 + (((2 * c + 1) ^ (n & 7)) << 4);
-  PfRaw w[kWRT];
-  h16x2 S[kWRT], O[kWRT];
-  h16x8 af[2][kWRT], bf[4];
+  uint32_t bo[4];   // this lane's place in a token tile, per phase
 #pragma unroll
-  for (int r = 0; r < kWRT; r++) pw_raw_read<F>(w[r], raw, r, lane, n);
+  for (int p = 0; p < 4; p++) bo[p] = tk * 128 + (((4 * g + p) ^ (tk & 7)) << 4);
+  PfRaw w[2][2];    // [v][j]
+  h16x2 S[2], O[2];
+  h16x8 af[2][2], bf[4];
+  auto raw_read = [&]() {
 #pragma unroll
-  for (int r = 0; r < kWRT; r++) {
-    pf_scale<F>(w[r], 0, n, c, S[r], O[r]);
-    af[0][r] = pf_frag<F>(w[r], 0, 0, S[r], O[r]);
-  }
-  uint32_t cur = 0, nxt = 1, far = NB - 1;   // buffers of this step, the next one, and the one to request
-  auto rd = [&](uint32_t buf, int u) {
-    return *reinterpret_cast<const h16x8*>(smem + buf * kWStepBytes + (u >= MT ? bo1 : bo0) + (u % MT) * 2048);
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) pw_raw_read<F>(w[v][j], raw, 2 * v + sub, 16 * (2 * g + j) + n, n);
   };
+  auto operand = [&](int v, int pp, int p, h16x8& out) {   // phase p = (j, h)
+    if (p == 0 || (F == PF_Q6K && p == 2)) pf_scale<F>(w[v][p >> 1], pp, n, 2 * g + (p >> 1), S[v], O[v]);
+    out = pf_frag<F>(w[v][p >> 1], pp, p & 1, S[v], O[v]);
+  };
+  raw_read();
+#pragma unroll
+  for (int v = 0; v < 2; v++) operand(v, 0, 0, af[0][v]);
+  uint32_t cur = 0, nxt = 1, far = NB - 1;   // buffers of this step, the next one, and the one to request
+  auto rd = [&](uint32_t buf, int u) { return *reinterpret_cast<const h16x8*>(smem + buf * kWStepBytes + bo[u / TT] + (u % TT) * 4096); };
 #pragma unroll
   for (int u = 0; u < AHEAD; u++) bf[u] = rd(0, u);
 
@@ -174,23 +186,27 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
 #pragma unroll
     for (int pp = 0; pp < 4; pp++) {
       const uint32_t s = b * 4 + pp;
-      if (pp == 0) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the raw weights of this block are in registers
-        if (NB == 2) { x_dma(s + DIST, far); raw_dma(b + 1 < b1 ? b + 1 : b); }
-        else { raw_dma(b + 1 < b1 ? b + 1 : b); x_dma(s + DIST, far); }
-      } else {
-        x_dma(s + DIST, far);
+      if (pp == 0) __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the raw weights of this block are in registers
+      if (NB == 2) {
+#pragma unroll
+        for (int i = 0; i < NX; i++) x_dma(i, s + DIST, far);
       }
 #pragma unroll
-      for (int g = 0; g < UN / 4; g++) {   // regions of 4 units: 16 MFMAs, 4 operand reads and a quarter (or half) of a dequantization
-        const int h = g / (MT / 4);
+      for (int r = 0; r < RS; r++) {   // regions of 4 units: 8 MFMAs, 4 operand reads, one or both of the next phase's A operands, and the DMA piece by piece
+        if (NB == 3) x_dma(r, s + DIST, far);
+        if (pp < 2) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int u = g * 4 + v;
+          for (int k = (pp * RS + r) * RP; k < (pp * RS + r + 1) * RP; k++)
+            if (k < R) raw_dma(k, b + 1 < b1 ? b + 1 : b);
+        }
+        const int p = r / (TT / 4);
+#pragma unroll
+        for (int v4 = 0; v4 < 4; v4++) {
+          const int u = r * 4 + v4;
           if (u == UN - AHEAD) {   // the last reads of this buffer were issued by the unit before
             __builtin_amdgcn_sched_barrier(0);
-            if (NB == 3) { if (pp == 0) pw_wait_vm<NX + pw_raw_ops<F>()>(); else pw_wait_vm<NX>(); }
-            else { if (pp == 0) pw_wait_vm<pw_raw_ops<F>()>(); else pw_wait_vm<0>(); }
+            constexpr uint32_t XW = NB == 3 ? NX : 0;   // what this step has requested for later ones may be under way
+            if (pp == 0) pw_wait_vm<XW + R0>(); else if (pp == 1) pw_wait_vm<XW + R1>(); else pw_wait_vm<XW>();
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -198,23 +214,22 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
           }
           bf[(u + AHEAD) & 3] = u + AHEAD < UN ? rd(cur, u + AHEAD) : rd(nxt, u + AHEAD - UN);
 #pragma unroll
-          for (int r = 0; r < kWRT; r++) pw_mma(acc[r][u % MT], af[h][r], bf[u & 3]);
+          for (int v = 0; v < 2; v++) pw_mma(acc[v][u % TT], af[p & 1][v], bf[u & 3]);
         }
-        // the next half step's operands, spread over this half's regions
-        constexpr int PER = kWRT / (MT / 4) > 0 ? kWRT / (MT / 4) : 1;   // row tiles per region
-        const int gi = g % (MT / 4);
-        if (gi * PER < kWRT) {
-          const int pp2 = h == 0 ? pp : (pp + 1) & 3, h2 = h ^ 1;
-          if (gi == 0 && pp == 3 && h == 1) {
+        const int p2 = (p + 1) & 3, pp2 = p == 3 ? (pp + 1) & 3 : pp, ri = r % (TT / 4);
+        if (TT == 8) {
+          operand(ri, pp2, p2, af[p2 & 1][ri]);
+        } else {
+          operand(0, pp2, p2, af[p2 & 1][0]);
+          operand(1, pp2, p2, af[p2 & 1][1]);
+        }
+        if (pp == 3 && p == 2 && ri == TT / 4 - 1) raw_read();   // the block's last operands are made: the next block's weights
+        // one MFMA keeps the matrix pipe busy for 32 cycles, in which this wave can issue a few other instructions: a quarter of the region's between any two
 #pragma unroll
-            for (int r = 0; r < kWRT; r++) pw_raw_read<F>(w[r], raw, r, lane, n);
-          }
-#pragma unroll
-          for (int q = 0; q < PER; q++) {
-            const int r = gi * PER + q;
-            if (h2 == 0) pf_scale<F>(w[r], pp2, n, c, S[r], O[r]);
-            af[h2][r] = pf_frag<F>(w[r], pp2, h2, S[r], O[r]);
-          }
+        for (int i = 0; i < 8; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // MFMA
+          if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // LDS read
+          __builtin_amdgcn_sched_group_barrier(0x002, TT == 8 ? 3 : 6, 0);      // vector
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -223,39 +238,48 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
       far = far + 1 == NB ? 0 : far + 1;
     }
   }
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs' results
-  __builtin_amdgcn_sched_barrier(0);
   pw_wait_vm<0>();   // what was requested past the end has landed before the LDS is given back
 
-  // a lane holds, per (row tile, token tile), rows 4c .. 4c + 3 of token n
-  if constexpr (EPI == PW_SWIGLU) {
+  // A lane holds, per (32 rows, 32 tokens), rows 8i + 4g .. + 3 (i = 0 .. 3) of token tk.  A wave turns each token tile round in LDS (the activation buffers
+  // are free), so that a token's 64 sums (32 activations) leave in one piece: stored as they lie, every token's 32 bytes of an instruction are a piece
+  // of their own, and this phase took a seventh of the kernel.
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  uint8_t* turn = smem + wave * (32 * 68 * 4);
 #pragma unroll
-    for (int t = 0; t < MT; t++) {
-      pw_settle(acc[0][t], acc[1][t], acc[2][t], acc[3][t]);
-      const uint32_t m = m0 + t * 16 + n;
-      if (m >= m_end) continue;
+  for (int t = 0; t < TT; t++) {
+    pw_settle(acc[0][t], acc[1][t]);
+    if constexpr (EPI == PW_SWIGLU) {
+      const uint32_t m = min(m0 + t * 32 + tk, m_end - 1);
       const float inv = G.inv_rms[GRP ? (uint32_t)G.src[m] : m] * (1.0f / kPfScale);
 #pragma unroll
-      for (int r = 0; r < 2; r++) {
-        const uint32_t tile = (rg * kWWaves + wave) * 2 + r;
-        if (tile >= sg.ntiles) continue;
-        const f32x4 gt = acc[r][t] * inv, up = acc[r + 2][t] * inv;
-        const h16x4 o = {(_Float16)(silu_f(gt.x) * up.x), (_Float16)(silu_f(gt.z) * up.z), (_Float16)(silu_f(gt.y) * up.y), (_Float16)(silu_f(gt.w) * up.w)};
-        *reinterpret_cast<h16x4*>(G.act + ((size_t)m * G.act_cols + tile * 16 + c * 4) * 2) = o;
+      for (int i = 0; i < 4; i++) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = silu_f(acc[0][t][4 * i + e] * inv) * (acc[1][t][4 * i + e] * inv);
+        const h16x4 o = {(_Float16)v[0], (_Float16)v[2], (_Float16)v[1], (_Float16)v[3]};
+        *reinterpret_cast<h16x4*>(turn + tk * 80 + i * 16 + g * 8) = o;
       }
-    }
-  } else {
-    float* part = G.part + (size_t)ks * G.part_rows * G.ncols;
 #pragma unroll
-    for (int t = 0; t < MT; t++) {
-      pw_settle(acc[0][t], acc[1][t], acc[2][t], acc[3][t]);
-      const uint32_t m = m0 + t * 16 + n;
-      if (m >= m_end) continue;
+      for (int j = 0; j < 2; j++) {
+        const uint32_t tok = j * 16 + (lane >> 2), q = lane & 3, mo = m0 + t * 32 + tok, tile = (rg * kWWaves + wave) * 2 + (q >> 1);
+        const h16x8 o = *reinterpret_cast<const h16x8*>(turn + tok * 80 + q * 16);
+        if (mo < m_end && tile < sg.ntiles) *reinterpret_cast<h16x8*>(G.act + ((size_t)mo * G.act_cols + tile * 16 + (q & 1) * 8) * 2) = o;
+      }
+    } else {
 #pragma unroll
-      for (int r = 0; r < kWRT; r++) {
-        const uint32_t tile = (rg * kWWaves + wave) * kWRT + r;
-        if (tile >= sg.ntiles) continue;
-        *reinterpret_cast<f32x4*>(part + (size_t)m * G.ncols + sg.col0 + tile * 16 + c * 4) = acc[r][t] * (1.0f / kPfScale);
+      for (int v = 0; v < 2; v++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const f32x4 o = {acc[v][t][4 * i], acc[v][t][4 * i + 1], acc[v][t][4 * i + 2], acc[v][t][4 * i + 3]};
+          *reinterpret_cast<f32x4*>(turn + tk * 272 + (32 * v + 8 * i + 4 * g) * 4) = o * (1.0f / kPfScale);
+        }
+      float* part = G.part + (size_t)ks * G.part_rows * G.ncols + sg.col0;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const uint32_t tok = j * 4 + (lane >> 4), mo = m0 + t * 32 + tok, row = (rg * kWWaves + wave) * (kWRT * 16) + n * 4;
+        const f32x4 o = *reinterpret_cast<const f32x4*>(turn + tok * 272 + n * 16);
+        if (mo < m_end && row < sg.ntiles * 16) *reinterpret_cast<f32x4*>(part + (size_t)mo * G.ncols + row) = o;
       }
     }
   }
@@ -264,13 +288,21 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
 template <uint32_t MASK, bool GRP, int EPI>
 __global__ void __launch_bounds__(kWWaves * 64) pw_gemm_kernel(const PfWide G, uint32_t n_rg, uint32_t tiles_m) {
   extern __shared__ __attribute__((aligned(16))) uint8_t pw_smem[];
-  // token tiles of one weight panel side by side on one XCD (workgroups go round-robin over the 8 XCDs): the panel comes from HBM once per XCD
-  uint32_t t = blockIdx.x;
+  // token tiles of one weight panel side by side on one XCD (workgroups go round-robin over the 8 XCDs): the panel comes from HBM once per XCD.  A last
+  // token tile that is at most half full takes half the time: its workgroups are the last ones, to fill up the last round.
+  uint32_t t = blockIdx.x, total = gridDim.x, wide = tiles_m, tm0 = 0;
+  if (!GRP && tiles_m > 1 && (G.m - 1) % kPfwTile < kPfwTile / 2) {
+    const uint32_t first = n_rg * G.S * (tiles_m - 1);
+    wide = t < first ? tiles_m - 1 : 1;
+    tm0 = t < first ? 0 : tiles_m - 1;
+    total = t < first ? first : total - first;
+    t -= t < first ? 0 : first;
+  }
   {
-    const uint32_t q = gridDim.x / 8, r = gridDim.x % 8, xcd = t % 8, i = t / 8;
+    const uint32_t q = total / 8, r = total % 8, xcd = t % 8, i = t / 8;
     t = xcd * q + (xcd < r ? xcd : r) + i;
   }
-  const uint32_t tm = t % tiles_m, ks = t / tiles_m % G.S, rgid = t / (tiles_m * G.S);
+  const uint32_t tm = tm0 + t % wide, ks = t / wide % G.S, rgid = t / (wide * G.S);
   uint32_t m0 = tm * kPfwTile, m_end = G.m, expert = 0;
   if (GRP) {
     const int e = G.tile_e[tm];
@@ -290,8 +322,8 @@ __global__ void __launch_bounds__(kWWaves * 64) pw_gemm_kernel(const PfWide G, u
   auto is = [&](int f) { return (MASK & (1u << f)) && (MASK == (1u << f) || sg.fmt == f); };
 #define LGH_PW_RUN(F)                                                                                       \
   do {                                                                                                      \
-    if (m_end - m0 > (uint32_t)kPfwTile / 2) pw_body<F, 16, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); \
-    else pw_body<F, 8, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);                                      \
+    if (m_end - m0 > (uint32_t)kPfwTile / 2) pw_body<F, 8, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); \
+    else pw_body<F, 4, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);                                      \
   } while (0)
   if (is(PF_Q4K)) LGH_PW_RUN(PF_Q4K);
   else if (is(PF_Q6K)) LGH_PW_RUN(PF_Q6K);
@@ -360,7 +392,7 @@ bool pfw_pairs(const DevWeight* gate, const DevWeight* up) { return gate->type =
 hipError_t pfw_gemm_launch(const DevWeight* const* W, int nw, PfWide& G, int epi, uint32_t rows, const PfwGroups* grp, hipStream_t st) {
   if (nw < 1 || nw > 3 || rows == 0 || rows > (uint32_t)kPfwMaxRows || !G.x) return hipErrorInvalidValue;
   const uint32_t k = W[0]->k;
-  if (k % 256 || (size_t)rows * k * 2 > 0xFFFFFFFFull) return hipErrorInvalidValue;   // (32-bit row offsets)
+  if (k % 256 || (size_t)rows * k * 2 > 0xFFFFF000ull) return hipErrorInvalidValue;   // (32-bit row offsets)
   G.nseg = nw;
   G.nblk = k / 256;
   uint32_t rg = 0, col = 0, mask = 0;
