@@ -121,7 +121,7 @@ enum {
   LGH_FLAG_REMOVED_MASK = (1u << 1) | (1u << 3) | (1u << 5) | (1u << 6) | (1u << 7) | (0xFFu << 24),
   LGH_FLAG_ATTN_SPLITS_SHIFT = 8,    /* bits 8..15: KV splits per kv-head in decode attention (0 = auto) */
   LGH_FLAG_ATTN_DIRECT_SHIFT = 16    /* bits 16..23: contexts of up to 64 * n rows use the single-launch decode attention (one workgroup
-                                        per kv head, no split + combine pair); 0 = the tuned default, 255 = never */
+                                        per query head, no split + combine pair); 0 = the tuned default, 255 = never */
 };
 
 typedef struct lgh_ctx lgh_ctx;

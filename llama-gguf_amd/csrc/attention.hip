@@ -35,13 +35,10 @@ constexpr float kNegBig = -1e30f;
 // PF (prefill.hip): blockIdx.y = token t of a block of prompt tokens; it sees kv_len_fixed + t cache rows (causal), its
 // query is q + t * n_heads * D, there is one split, and the normalised output goes, as f16, into the XH matrix at
 // `part_acc` (prefill.h: the wo GEMM's input).
-// DIRECT: one workgroup of NW = 16 waves per kv head and no second kernel: the workgroup merges its waves and writes the
-// normalised output (f32 at part_acc, XQ records at part_ml when not null) itself.  It saves one launch floor per layer
-// but pulls a kv head's whole K/V through one CU, so it only pays below ~100 rows (engine.hip: kDirectAttnDefaultKv).
 // MULTI (multi-sequence decode, engine_batch.hip): blockIdx.y = sequence s of the step; its query is q + s * n_heads * D, its
 // position pos_ptr[s], its K / V the cache slot slot[s] (slot_stride floats apart), its partials the s-th block of
 // part_ml / part_acc.  Per sequence the arithmetic is the single-sequence kernel's.
-template <int D, int G, int NW, bool PF = false, bool DIRECT = false, bool MULTI = false>
+template <int D, int G, int NW, bool PF = false, bool MULTI = false>
 __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __restrict__ q, const float* __restrict__ kc,
                                                            const float* __restrict__ vc, uint32_t max_seq, float scale,
                                                            const int* pos_ptr, int kv_len_fixed, uint32_t n_splits,
@@ -118,7 +115,7 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
   // Batches of kAhead iterations: all their K/V rows are requested before the first one is used (clamped when past the
   // end, so the loads are unconditional).  At decode lengths a workgroup has 1-3 iterations and everything is in flight
   // at once; at 4K context it has ~30, and with a single iteration ahead the kernel ran at 1 TB/s (latency-bound).
-  constexpr int kAhead = G >= 8 && NW >= 16 ? 3 : 4;   // (16 waves leave 128 registers per lane: 3 for 8 heads; 8 measured slower: 604 / 518 vs 614 / 528 tokens/s at kv 272 / 4000)
+  constexpr int kAhead = 4;   // (8 measured slower: 604 / 518 vs 614 / 528 tokens/s at kv 272 / 4000)
   for (uint32_t base = (sp * NW + wave) * RPW; base < kv_len; base += kAhead * stride) {
     f32x4 kk[kAhead], vv[kAhead];
 #pragma unroll
@@ -170,11 +167,7 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
       lsum += s_ml[w][g][1] * f;
       a += s_acc[w][g][dim] * f;
     }
-    if (DIRECT) {
-      const float o = a * (1.0f / lsum);   // simd.rs:718-720: multiply by 1/sum
-      part_acc[(pbase + g) * D + dim] = o;
-      if (part_ml) xq_store_chunk(reinterpret_cast<uint8_t*>(part_ml), (uint32_t)((pbase + g) * D + dim) >> 4, o);   // wo's input as XQ records
-    } else if (PF) {
+    if (PF) {
       const _Float16 o = (_Float16)(a * (1.0f / lsum));   // simd.rs:718-720: multiply by 1/sum
       *reinterpret_cast<_Float16*>(reinterpret_cast<uint8_t*>(part_acc) + xh_offset(blockIdx.y, (uint32_t)(pbase + g) * D + dim)) = o;
     } else {
@@ -534,12 +527,124 @@ hipError_t attn_launch(const float* q, const float* kcache, const float* vcache,
   return hipErrorInvalidValue;
 }
 
-template <int D, int G>
-static hipError_t attn_direct_go(const float* q, const float* kc, const float* vc, uint32_t n_kv, uint32_t max_seq, float scale, const int* pos,
-                                 float* out, uint8_t* xq_out, hipStream_t st) {
-  hipLaunchKernelGGL((attn_partial_kernel<D, G, 16, false, true>), dim3(n_kv), dim3(1024), 0, st, q, kc, vc, max_seq, scale, pos, 0, 1u,
-                     reinterpret_cast<float*>(xq_out), out);
-  return hipGetLastError();
+// Decode attention of short contexts in one launch: a workgroup of 16 waves per QUERY head.  It is latency: launch, position, rows from memory, scores,
+// softmax, weighted sum, merge.  The rows of the first batch are requested before the position is known (rows past it are masked, scores and values both:
+// what lies there may be anything), all rows of a batch before the first is used, and a wave's rows share one maximum, so that nothing but additions is
+// exchanged inside a wave.  The query heads of a kv head lie on one XCD (workgroups go round-robin over the 8) and share its rows in that L2.
+// (One workgroup per kv head, each wave with all its query heads, took 10.0 us at 8 heads of 64 and 6.5 at 4 of 128 and 40 rows, split and merge 10.1 at
+// 128 rows of the latter; this 3.8 and 4.8.  A token of TinyLlama-1.1B Q4_K_M at 40 rows 766 -> 626 us, of Llama-3-8B Q4_K_M at 130 1695 -> 1582 us, both with
+// the logits to the host.)
+__device__ __forceinline__ float swap16_add(float v) {   // sum of rows 2i and 2i + 1 of 16 lanes, in both
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap32_add(float v) {   // sum of lanes l and l + 32, in both
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap16_max(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float swap32_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int D>
+__global__ void __launch_bounds__(1024) attn_direct_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, uint32_t n_kv,
+                                                           uint32_t g_per_kv, uint32_t max_seq, float scale, const int* pos_ptr, float* __restrict__ out,
+                                                           uint8_t* __restrict__ xq_out) {
+  constexpr int NW = 16, LPR = D / 4, RPW = 64 / LPR, B = 4;   // lanes of a row, rows of a wave's load, loads of a batch
+  __shared__ __attribute__((aligned(16))) float s_m[NW], s_l[NW];
+  __shared__ __attribute__((aligned(16))) float s_acc[NW][D];
+  LGH_TL_BEGIN(attn, lgh::TL_ATTN, 1);
+  const uint32_t kvh = blockIdx.x % n_kv, head = kvh * g_per_kv + blockIdx.x / n_kv;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane / LPR, li = lane % LPR;
+  const float* kb = kc + (size_t)kvh * max_seq * D + li * 4;
+  const float* vb = vc + (size_t)kvh * max_seq * D + li * 4;
+  constexpr uint32_t STEP = B * NW * RPW;
+  f32x4 kn[B], vn[B];                                   // the next batch
+  auto request = [&](uint32_t base, uint32_t rows) {   // this lane's rows base + (j * NW + wave) * RPW + sub
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+      const uint32_t r = base + (j * NW + wave) * RPW + sub, rc = r < rows ? r : rows - 1;
+      kn[j] = *reinterpret_cast<const f32x4*>(kb + (size_t)rc * D);
+    }
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+      const uint32_t r = base + (j * NW + wave) * RPW + sub, rc = r < rows ? r : rows - 1;
+      vn[j] = *reinterpret_cast<const f32x4*>(vb + (size_t)rc * D);
+    }
+  };
+  request(0, max_seq);
+  f32x4 qv = *reinterpret_cast<const f32x4*>(q + (size_t)head * D + li * 4);
+  uint32_t pw;
+  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pw) : "s"(pos_ptr) : "memory");
+  const uint32_t kv_len = pw + 1;
+  qv *= scale * 1.44269504088896f;                      // scores in units of log2
+  float m = kNegBig, l = 0.0f;
+  f32x4 acc = (f32x4)(0.0f);
+  for (uint32_t base = 0; base < kv_len; base += STEP) {
+    f32x4 kk[B], vv[B];
+#pragma unroll
+    for (int j = 0; j < B; j++) { kk[j] = kn[j]; vv[j] = vn[j]; }
+    if (base + STEP < kv_len) request(base + STEP, kv_len);
+    float s[B], mx = m;
+    bool ok[B];
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+      ok[j] = base + (j * NW + wave) * RPW + sub < kv_len;
+      float t = qv.x * kk[j].x;
+      t = __builtin_fmaf(qv.y, kk[j].y, t);
+      t = __builtin_fmaf(qv.z, kk[j].z, t);
+      t = __builtin_fmaf(qv.w, kk[j].w, t);
+      t += dpp_f<0xB1>(t);
+      t += dpp_f<0x4E>(t);
+      t += dpp_f<0x141>(t);
+      t += dpp_f<0x140>(t);
+      if (LPR == 32) t = swap16_add(t);
+      s[j] = ok[j] ? t : kNegBig;
+      mx = fmaxf(mx, s[j]);
+    }
+    if (LPR == 16) mx = swap16_max(mx);
+    mx = swap32_max(mx);
+    const float a = __builtin_amdgcn_exp2f(m - mx);
+    m = mx;
+    l *= a;
+    acc = acc * a;
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+      const float p = ok[j] ? __builtin_amdgcn_exp2f(s[j] - mx) : 0.0f;
+      l += p;
+      acc.x = __builtin_fmaf(ok[j] ? vv[j].x : 0.0f, p, acc.x);
+      acc.y = __builtin_fmaf(ok[j] ? vv[j].y : 0.0f, p, acc.y);
+      acc.z = __builtin_fmaf(ok[j] ? vv[j].z : 0.0f, p, acc.z);
+      acc.w = __builtin_fmaf(ok[j] ? vv[j].w : 0.0f, p, acc.w);
+    }
+  }
+  auto rows_sum = [&](float v) { return swap32_add(LPR == 16 ? swap16_add(v) : v); };   // over the wave's row slots
+  l = rows_sum(l);
+  acc.x = rows_sum(acc.x); acc.y = rows_sum(acc.y); acc.z = rows_sum(acc.z); acc.w = rows_sum(acc.w);
+  if (lane == 0) { s_m[wave] = m; s_l[wave] = l; }
+  if (sub == 0) *reinterpret_cast<f32x4*>(&s_acc[wave][li * 4]) = acc;
+  __syncthreads();
+  const uint32_t dim = threadIdx.x;
+  if (dim < (uint32_t)D) {
+    float mm[NW], mn = kNegBig, ls = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) { mm[w] = s_m[w]; mn = fmaxf(mn, mm[w]); }
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = __builtin_amdgcn_exp2f(mm[w] - mn);
+      ls = __builtin_fmaf(s_l[w], f, ls);
+      o = __builtin_fmaf(s_acc[w][dim], f, o);
+    }
+    o *= 1.0f / ls;                                     // simd.rs:718-720: multiply by 1/sum
+    out[(size_t)head * D + dim] = o;
+    if (xq_out) xq_store_chunk(xq_out, (head * D + dim) >> 4, o);   // wo's input as XQ records
+  }
+  LGH_TL_END();
 }
 
 // single-launch decode attention for short contexts (engine.hip picks it by the host-side position)
@@ -547,12 +652,10 @@ hipError_t attn_direct_launch(const float* q, const float* kcache, const float* 
                               uint32_t max_seq, float scale, const int* pos, float* out, uint8_t* xq_out, hipStream_t st) {
   if (n_kv == 0 || n_heads % n_kv || !pos) return hipErrorInvalidValue;
   const uint32_t g = n_heads / n_kv;
-#define LGH_ATTN_CASE(DD, GG) \
-  if (head_dim == DD && g == GG) return attn_direct_go<DD, GG>(q, kcache, vcache, n_kv, max_seq, scale, pos, out, xq_out, st);
-  LGH_ATTN_CASE(128, 1) LGH_ATTN_CASE(128, 2) LGH_ATTN_CASE(128, 4) LGH_ATTN_CASE(128, 8)
-  LGH_ATTN_CASE(64, 1) LGH_ATTN_CASE(64, 2) LGH_ATTN_CASE(64, 4) LGH_ATTN_CASE(64, 8)
-#undef LGH_ATTN_CASE
-  return hipErrorInvalidValue;
+  if (!attn_shape_has_fast_kernel(head_dim, g) || max_seq == 0) return hipErrorInvalidValue;
+  if (head_dim == 128) hipLaunchKernelGGL(attn_direct_kernel<128>, dim3(n_heads), dim3(1024), 0, st, q, kcache, vcache, n_kv, g, max_seq, scale, pos, out, xq_out);
+  else hipLaunchKernelGGL(attn_direct_kernel<64>, dim3(n_heads), dim3(1024), 0, st, q, kcache, vcache, n_kv, g, max_seq, scale, pos, out, xq_out);
+  return hipGetLastError();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -848,10 +951,10 @@ static hipError_t attn_multi_go(const float* q, const float* kc, const float* vc
                                 const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* part_ml, float* part_acc,
                                 hipStream_t st) {
   if (max_seq >= 2048)
-    hipLaunchKernelGGL((attn_partial_kernel<D, G, 8, false, false, true>), dim3(n_kv * n_splits, n_seq), dim3(512), 0, st, q, kc, vc, max_seq, scale,
+    hipLaunchKernelGGL((attn_partial_kernel<D, G, 8, false, true>), dim3(n_kv * n_splits, n_seq), dim3(512), 0, st, q, kc, vc, max_seq, scale,
                        pos, 0, n_splits, part_ml, part_acc, slot, slot_stride);
   else
-    hipLaunchKernelGGL((attn_partial_kernel<D, G, 4, false, false, true>), dim3(n_kv * n_splits, n_seq), dim3(256), 0, st, q, kc, vc, max_seq, scale,
+    hipLaunchKernelGGL((attn_partial_kernel<D, G, 4, false, true>), dim3(n_kv * n_splits, n_seq), dim3(256), 0, st, q, kc, vc, max_seq, scale,
                        pos, 0, n_splits, part_ml, part_acc, slot, slot_stride);
   return hipGetLastError();
 }

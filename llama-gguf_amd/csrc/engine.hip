@@ -61,10 +61,10 @@ void dev_free_tracked(lgh_ctx* c, void* p) {
   (void)hipFree(p);
 }
 
-// Contexts up to this many rows run the single-launch decode attention (attention.hip, DIRECT) unless the flags say
-// otherwise.  Measured on Llama-3-8B Q4_K_M: 640 vs 618 tokens/s at kv <= 64, equal at kv 69..128, 581 vs 614 at kv
-// 137..272 — one workgroup per kv head fetches that head's whole K/V (1 KB per row) through ONE CU's memory path.
-constexpr uint32_t kDirectAttnDefaultKv = 64;
+// Contexts up to this many rows run the single-launch decode attention (attention.hip, attn_direct_kernel) unless the flags say otherwise.  Measured against
+// the split kernel with its merge, us per layer gained: 8 kv heads of 128 with 4 query heads each 4.8 / 5.1 / 3.8 / 2.4 / 1.6 / 0.2 / -0.4 at 40 / 144 / 256 /
+// 512 / 1000 / 1500 / 3000 rows (a query head's rows all pass through one CU), 4 of 64 with 8 each 6.9 / 7.2 / 7.4 / 6.3 / 5.6 / 5.6 / 4.3 at the same, 4.3 at 4000.
+static uint32_t direct_attn_default_kv(uint32_t head_dim) { return head_dim == 64 ? 4096 : 1024; }
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ------------------------------------------------------------------------------------------------
@@ -1193,7 +1193,7 @@ int lgh_create(const lgh_model_desc* desc, lgh_ctx** out) {
   if (splits > 32) splits = 32;   // the split merge keeps one partial per split in registers
   c->n_splits = splits;
   const uint32_t dsel = (d.flags >> LGH_FLAG_ATTN_DIRECT_SHIFT) & 0xFFu;
-  c->direct_attn_max_kv = dsel == 255 ? 0 : dsel ? dsel * 64 : kDirectAttnDefaultKv;
+  c->direct_attn_max_kv = dsel == 255 ? 0 : dsel ? dsel * 64 : direct_attn_default_kv(d.head_dim);
   if (d.flags & LGH_FLAG_KV_INT8) c->direct_attn_max_kv = 0;   // the byte caches have one attention structure: splits + combine
   *out = c;
   return LGH_OK;

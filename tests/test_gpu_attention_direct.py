@@ -1,0 +1,31 @@
+"""The single-launch decode attention (attention.hip, attn_direct_kernel) against the split kernel and its merge, on the same cache: lengths around the
+edges of a batch (128 rows of 128 values, 256 of 64) and behind stale rows, every number of query heads per kv head.
+
+Tolerance: both sum at most 600 products of a softmax in f32 in another order, 600 * 2^-24 = 4e-5 of the largest at worst; logits of two layers, 2e-4."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROWS = (1, 2, 33, 127, 128, 129, 255, 256, 257, 384, 513, 600)
+
+
+@pytest.mark.parametrize("head_dim,heads,kv_heads", [(64, 8, 8), (64, 8, 4), (64, 8, 2), (64, 8, 1), (128, 4, 4), (128, 4, 2), (128, 4, 1), (128, 8, 1)])
+def test_direct_attention_matches_the_split_kernel(pkg, head_dim, heads, kv_heads):
+    cfg = pkg.make_config("test-dense", max_seq_len=640, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim)
+    model = pkg.SynthModel(cfg, mix="Q8_0")
+    direct, split = (pkg.HipGpuInference.from_model(model, 640, attn_direct=d) for d in (16, 255))
+    prompt = [(7 * i + 5) % cfg.vocab_size for i in range(620)]
+    for eng in (direct, split):
+        eng.forward_batch(prompt)
+    for rows in ROWS:
+        got = []
+        for eng in (direct, split):
+            eng.kv_truncate(rows - 1)
+            got.append(eng.forward(rows % cfg.vocab_size))
+        assert np.abs(got[0] - got[1]).max() <= 2e-4 * np.abs(got[1]).max(), rows
+        for eng in (direct, split):                       # the row that the step overwrote, and the stale ones behind it
+            eng.kv_truncate(rows - 1)
+            eng.forward_batch(prompt[rows - 1:])
+    direct.close()
+    split.close()
