@@ -423,6 +423,203 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_kernel(const Mvqb2Geom Gm,
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// From three sequences on: the sequences four at a time.  mvqb2 gives every MFMA one sequence: its A operand, the four digits of four chunks, is three
+// quarters zeros, and every lane reads 16 bytes for it all the same: six LDS reads of 1 KB per (tile, sequence) and wave, 96 % of what LDS can deliver in the time of
+// the vector work.  Here the A operand is the four digits of FOUR sequences, all lanes full, and the weights are masked instead: B operand c keeps chunk c of
+// every 64 elements and zeros for the other lane groups (masked once per tile).  A lane then has, per MFMA, the four digit sums of one sequence (4 * group + its lane
+// group) for chunk c of weight row n: three LDS reads per (tile, sequence).  Per (row, sequence, chunk class) the floating-point operations and their order are
+// mvqb2's (mvq_mac_finish); the classes, there in four lanes, lie in one: (class 0 + 1) + (2 + 3) is what the two exchanges add up.
+// Records lie 1296 bytes apart in LDS, so that the four sequences' digits of a read fall into different banks.
+// gate | up of an 8B model (28672 rows of 4096, Q4_K), 16 sequences: 72 us with mvqb2, 58 here, of which about 42 are vector instructions (8 a product of 16 elements).
+// ------------------------------------------------------------------------------------------------
+constexpr uint32_t kXLdsRecord = kXqRecord + 16;
+__host__ __device__ constexpr uint32_t mvqb4_buf_bytes(uint32_t records) { return (records * kXLdsRecord + 1023u) & ~1023u; }
+
+// scales of row n for all four chunk classes: f[pp][class], class pairs (a 32-element sub-block) sharing one where the format has it so
+struct TileScales { float f[4][4], g[4][2], dd, dmin; };
+template <uint32_t MASK>
+__device__ __forceinline__ void mvq_row_scales(int fmt, const RawT16& r, uint32_t lane, TileScales& t) {
+  const uint32_t n = lane & 15;
+  auto is = [&](int f) { return mvq_is<MASK>(fmt, f); };
+  const uint32_t hdw[4] = {r.hd.x, r.hd.y, r.hd.z, r.hd.w};
+  if (is(F_Q6K)) {
+#pragma unroll
+    for (int pp = 0; pp < 4; pp++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) t.f[pp][c] = (float)(int)__builtin_amdgcn_sbfe((int)hdw[pp], c * 8, 8);
+    t.dd = h2f((n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu);
+    t.dmin = 0.0f;
+  } else if (is(F_Q80) || is(F_Q40)) {
+#pragma unroll
+    for (int pp = 0; pp < 4; pp++) {
+      t.f[pp][0] = t.f[pp][1] = h2f(hdw[pp] & 0xFFFFu);
+      t.f[pp][2] = t.f[pp][3] = h2f(hdw[pp] >> 16);
+    }
+    t.dd = t.dmin = 0.0f;
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {   // sub-blocks h, h + 2, h + 4, h + 6 (as mvq_unpack_tile)
+      const uint32_t a = (r.hd.y >> (h * 8)) & 0x00FF00FFu, bq = (r.hd.z >> (h * 8)) & 0x00FF00FFu, cq = (r.hd.w >> (h * 8)) & 0x00FF00FFu;
+      const uint32_t sc01 = a & 0x003F003Fu, mn01 = bq & 0x003F003Fu;
+      const uint32_t sc23 = (cq & 0x000F000Fu) | ((a >> 2) & 0x00300030u);
+      const uint32_t mn23 = ((cq >> 4) & 0x000F000Fu) | ((bq >> 2) & 0x00300030u);
+      const float f[4] = {ub0(sc01), ub2(sc01), ub0(sc23), ub2(sc23)}, g[4] = {ub0(mn01), ub2(mn01), ub0(mn23), ub2(mn23)};
+#pragma unroll
+      for (int pp = 0; pp < 4; pp++) { t.f[pp][2 * h] = t.f[pp][2 * h + 1] = f[pp]; t.g[pp][h] = g[pp]; }
+    }
+    t.dd = h2f(r.hd.x & 0xFFFFu);
+    t.dmin = h2f(r.hd.x >> 16);
+  }
+}
+
+template <uint32_t MASK, int NB, bool SEQ>
+__global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  constexpr int NG = NB / 4;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
+  const bool active = u < Gm.n_units;
+  const int sg = (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  const MvSeg& S = L.seg[active ? sg : 0];
+  constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
+  const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
+  auto is = [&](int f) { return ((MASK >> f) & 1u) != 0 && (kSingle || fmt == f); };
+  const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q6K) ? fmt_tile_bytes(F_Q6K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K)
+                      : is(F_Q80) ? fmt_tile_bytes(F_Q80) : fmt_tile_bytes(F_Q40);
+  const uint32_t ntiles = (S.n_rows + 15) >> 4;
+  const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
+  const uint32_t pass = active ? ul / ntiles : 0, tl = active ? ul - pass * ntiles : 0;
+  const uint8_t* wbase = (pass == 0 ? S.pass[0].plane[0] : S.pass[1].plane[0]) + (size_t)tl * Gm.nblk * tb;
+  const uint8_t* xg = L.seg[0].pass[0].xq;                        // sequence 0's records (all segments and passes share the input)
+  const uint32_t n = lane & 15, mq = lane >> 4;
+  const uint32_t ks0 = SEQ ? 0u : blockIdx.y, ks1 = SEQ ? Gm.T : blockIdx.y + 1;   // this workgroup's slices
+  float acc[NG][4], tot[NG];                                      // per group: the lane's sequence, chunk classes
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    tot[g] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[g][c] = 0.0f;
+  }
+  const uint32_t a_off = (mq >> 1) * 128 + (n & 3) * 32 + (mq & 1) * 16;
+
+  RawT16 nxt;
+  {
+    const uint32_t bfirst = ks0 * Gm.nbw;
+    if (active && bfirst < Gm.nblk) mvq_issue_tile<MASK>(fmt, wbase + (size_t)bfirst * tb, lane, nxt);
+  }
+  // chunks of records through a two-deep LDS buffer, as mvqb2, but by DMA: no staging registers
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem8;
+  const uint32_t buf_bytes = mvqb4_buf_bytes(Gm.cb * n_seq);
+  auto chunk_len = [&](uint32_t ks, uint32_t b0) { return min(Gm.cb, min(ks * Gm.nbw + Gm.nbw, Gm.nblk) - b0); };
+  auto fetch = [&](uint32_t b0, uint32_t cn, uint32_t buf) {
+    constexpr uint32_t kP = kXLdsRecord / 16;
+    const uint32_t recs = cn * n_seq, kb = (recs * kP + 63) / 64;
+    for (uint32_t k = wave; k < kb; k += kBWaves) {
+      const uint32_t i = k * 64 + lane, rec = min(i / kP, recs - 1), off = min(i - rec * kP, kP - 2);   // a record's pad and the tail: any of its bytes
+      const uint32_t bi = rec / n_seq, s = rec - bi * n_seq;
+      const uint8_t* src = xg + (size_t)s * B.xq_stride + (size_t)(b0 + bi) * kXqRecord + off * 16;
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds0 + buf * buf_bytes + k * 1024) : "memory", "m0");
+    }
+  };
+  uint32_t ks = ks0, b0 = ks0 * Gm.nbw;
+  while (ks < ks1 && b0 >= min(ks * Gm.nbw + Gm.nbw, Gm.nblk)) { ks++; b0 = ks * Gm.nbw; }
+  uint32_t buf = 0;
+  if (ks < ks1) fetch(b0, chunk_len(ks, b0), 0);
+  while (ks < ks1) {
+    const uint32_t sb1 = min(ks * Gm.nbw + Gm.nbw, Gm.nblk);
+    const uint32_t cn = chunk_len(ks, b0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    uint32_t nks = ks, nb0 = b0 + cn;   // the chunk after this one
+    if (nb0 >= sb1) {
+      nks = ks + 1; nb0 = nks * Gm.nbw;
+      while (nks < ks1 && nb0 >= min(nks * Gm.nbw + Gm.nbw, Gm.nblk)) { nks++; nb0 = nks * Gm.nbw; }
+    }
+    if (nks < ks1) fetch(nb0, chunk_len(nks, nb0), buf ^ 1u);
+    if (active) {
+      for (uint32_t bi = 0; bi < cn; bi++) {
+        const uint32_t b = b0 + bi;
+        TileScales ts;
+        i32x4 bm[4][4];   // [class][step]
+        {
+          TileOps t;
+          mvq_unpack_tile<MASK>(fmt, nxt, lane, t);
+          mvq_row_scales<MASK>(fmt, nxt, lane, ts);
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++)
+#pragma unroll
+              for (int e = 0; e < 4; e++) bm[c][pp][e] = mq == (uint32_t)c ? t.bw[pp][e] : 0;
+        }
+        {   // the unit's next tile (its next block — of this slice, or of the next one this workgroup walks)
+          uint32_t bn = b + 1;
+          if (bn == sb1) bn = nks < ks1 ? nb0 : Gm.nblk;
+          if (bn < Gm.nblk) mvq_issue_tile<MASK>(fmt, wbase + (size_t)bn * tb, lane, nxt);
+        }
+        const uint32_t xb = buf * buf_bytes + bi * n_seq * kXLdsRecord;
+        // sequences past the last one repeat it: computed, never stored
+        i32x4 a[4];
+        auto load_a = [&](uint32_t g) {
+          const uint8_t* p = smem8 + xb + min(4 * g + (n >> 2), n_seq - 1) * kXLdsRecord + a_off;
+#pragma unroll
+          for (int pp = 0; pp < 4; pp++) a[pp] = *reinterpret_cast<const i32x4*>(p + pp * 256);
+        };
+        f32x4 xs[2], sx[2];   // by step (group, class) parity
+        auto load_x = [&](uint32_t step) {
+          const uint8_t* p = smem8 + xb + min((step & ~3u) + mq, n_seq - 1) * kXLdsRecord + kXqXs16 + (step & 3) * 16;
+          xs[step & 1] = *reinterpret_cast<const f32x4*>(p);
+          sx[step & 1] = *reinterpret_cast<const f32x4*>(p + (kXqSx16 - kXqXs16));
+        };
+        MacD m[2];
+        const i32x4 zero = {0, 0, 0, 0};
+        auto mfma = [&](uint32_t step) {
+#pragma unroll
+          for (int pp = 0; pp < 4; pp++) m[step & 1].d[pp] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[pp], bm[step & 3][pp], zero, 0, 0, 0);
+        };
+        load_a(0);
+        load_x(0);
+        mfma(0);
+#pragma unroll
+        for (int step = 0; step < 4 * NG; step++) {   // a step's products and factors ahead of the vector work of the one before
+          if ((step & 3) == 0 && (uint32_t)step >= n_seq) break;
+          if ((step & 3) == 3 && step + 1 < 4 * NG) load_a(step / 4 + 1);
+          if (step + 1 < 4 * NG) { load_x(step + 1); mfma(step + 1); }
+          const int c = step & 3;
+          TileOps t;
+#pragma unroll
+          for (int pp = 0; pp < 4; pp++) { t.f[pp] = ts.f[pp][c]; t.g[pp] = ts.g[pp][c >> 1]; }
+          t.dd = ts.dd;
+          t.dmin = ts.dmin;
+          mvq_mac_finish<MASK>(fmt, t, m[c & 1], xs[c & 1], sx[c & 1], acc[step / 4][c]);
+          asm volatile("" : "+v"(acc[step / 4][c]));   // here, not sunk past the later groups' products
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if (b0 + cn >= sb1) {   // end of the k-slice: the slice's partial sum, in the single-sequence kernel's order
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+          const float t = (acc[g][0] + acc[g][1]) + (acc[g][2] + acc[g][3]);
+          if (SEQ) tot[g] += t;
+          else tot[g] = t;
+#pragma unroll
+          for (int c = 0; c < 4; c++) acc[g][c] = 0.0f;
+        }
+      }
+    }
+    ks = nks; b0 = nb0; buf ^= 1u;
+  }
+  if (active) {
+    const uint32_t slot = SEQ ? 0u : blockIdx.y;
+    const size_t rows16 = (size_t)Gm.n_units * 16;
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+      if (4 * g + mq < n_seq) part[((size_t)slot * n_seq + 4 * g + mq) * rows16 + (size_t)u * 16 + n] = tot[g];
+  }
+}
+
 // grid / block = the single-sequence geometry of `L` (segments' wg_begin, rows_per_wg).  dynamic LDS: mvqb_lds_bytes(n_seq, L.red_floats)
 __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_floats,
                                                                       const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B,
@@ -479,12 +676,33 @@ static hipError_t mvqb_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, 
   return hipGetLastError();
 }
 
+// Sequences from which the groups of four are the faster ones (a step, 4 layers of an 8B model in Q4_K_M / Q8_0, us: 2 sequences 366 / 411 with mvqb2,
+// 388 / 398 in groups; 3: 416 / 439 against 390 / 419; 5: 495 / 494 against 504 / 488; 8: 579 / 567 against 529 / 520; 16: 905 / 867 against 786 / 751).
+// Indirect launches (a mixture's experts) have one or two sequences per expert: they stay with mvqb2.
+constexpr uint32_t kMvqb4MinSeq = 3;
+
+template <uint32_t MASK, int NB>
+static hipError_t mvqb4_go(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, bool seq, uint32_t groups, hipStream_t st) {
+  static bool attr_set[2][64] = {};
+  const size_t lds = (size_t)2 * mvqb4_buf_bytes(Gm.cb * B.n_seq);
+  if (seq) {
+    if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb4_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
+    hipLaunchKernelGGL((mvqb4_kernel<MASK, NB, true>), dim3(groups), dim3(kBWaves * 64), lds, st, Gm, L, B, B.part);
+  } else {
+    if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb4_kernel<MASK, NB, false>), 160 * 1024, attr_set[1]); e != hipSuccess) return e;
+    hipLaunchKernelGGL((mvqb4_kernel<MASK, NB, false>), dim3(groups, Gm.T), dim3(kBWaves * 64), lds, st, Gm, L, B, B.part);
+  }
+  return hipGetLastError();
+}
+
 template <uint32_t MASK, int NB>
 static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, const Mvqb2Geom& Gm, bool seq, uint32_t groups, size_t lds_x,
                            size_t lds_e, uint32_t threads, hipStream_t st) {
   static bool attr_set[3][64] = {};
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
-  if (seq) {
+  if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
+    if (hipError_t e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st); e != hipSuccess) return e;
+  } else if (seq) {
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb2_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
     hipLaunchKernelGGL((mvqb2_kernel<MASK, NB, true>), dim3(groups, 1, nz), dim3(kBWaves * 64), lds_x, st, Gm, L, B, B.part);
   } else {

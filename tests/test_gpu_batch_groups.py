@@ -1,0 +1,40 @@
+"""The batched step's mat-vec from three sequences on takes them in groups (matvec_batch.hip): group sizes around full ones, every
+weight format, plans with whole rows per workgroup and plans with k-slices.
+
+Per (row, sequence) the kernel does the single-sequence kernel's floating-point operations in its order, on sums that are exact, so the
+bound is equality of all bits with a single-sequence engine that runs the split attention too (attn_direct=255)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("name,mix,sizes,kw", [
+    ("test-dense-d128", "Q4_K_M", (3, 4, 5, 7, 8, 9, 12, 13, 16), {}),
+    ("test-dense-d128", "Q5_K_M", (3, 6, 11, 15), {}),
+    ("test-dense-d128", "Q6_K", (3, 5, 10, 14), {}),
+    ("test-dense-d128", "Q8_0", (3, 5, 9, 16), {}),
+    ("test-dense-d128", "Q4_0", (3, 5, 9, 16), {}),
+    ("llama-3-8b", "Q4_K_M", (3, 8, 13), dict(num_layers=1, vocab_size=4096)),     # gate | up: whole rows per workgroup
+    ("llama-3-8b", "Q5_K_M", (5, 16), dict(num_layers=1, vocab_size=4096)),
+])
+def test_groups_of_sequences_are_bitwise_the_single_sequence(pkg, name, mix, sizes, kw):
+    cfg = pkg.make_config(name, max_seq_len=32, **kw)
+    model = pkg.SynthModel(cfg, mix=mix)
+    multi = pkg.HipGpuInference.from_model(model, 32)
+    single = pkg.HipGpuInference.from_model(model, 32, attn_direct=255)
+    multi.batch_create(16)
+    tok = np.random.default_rng(5).integers(0, cfg.vocab_size, (16, 2))
+    want = []
+    for s in range(16):
+        single.reset()
+        want.append([single.forward(int(t)).copy() for t in tok[s]])
+    for n in sizes:
+        for s in range(16):
+            multi.batch_reset(s)
+        for step in range(2):
+            got, _ = multi.forward_multi(list(range(n)), tok[:n, step])
+            for s in range(n):
+                assert np.array_equal(got[s].view(np.uint32), want[s][step].view(np.uint32)), (n, s, step)
+    multi.close()
+    single.close()
