@@ -11,7 +11,8 @@
 // Two structures.  mvqb2 (below, the default from 2 sequences on): a workgroup = 8 (row tile, pass) units x one range of blocks,
 // the sequences' records staged ONCE per workgroup in LDS and shared by its 8 waves, sequences two at a time (the pair's 8 MFMAs,
 // then the vector work while the next pair's operands load), the epilogue as a second small launch — what bounded the first
-// structure and what each change bought: profiles/r03e_batched_decode.md.  mvqb (first): the single-sequence decomposition (a
+// structure and what each change bought: profiles/r03e_batched_decode.md.  From three sequences on its products take the sequences in
+// groups of four (mvqb4) or, from five on and for weights below 8 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
 // workgroup = the 8 k-slices of a few row tiles) with a loop over the sequences inside it and their records from L2 into a
 // register ring; kept for one sequence and for launches whose segments do not share their input vector.
 // Epilogues: store, +residual, SwiGLU pair, RoPE (every sequence at its own position) and the K / V rows into the sequence's
@@ -437,7 +438,7 @@ constexpr uint32_t kXLdsRecord = kXqRecord + 16;
 __host__ __device__ constexpr uint32_t mvqb4_buf_bytes(uint32_t records) { return (records * kXLdsRecord + 1023u) & ~1023u; }
 
 // scales of row n for all four chunk classes: f[pp][class], class pairs (a 32-element sub-block) sharing one where the format has it so
-struct TileScales { float f[4][4], g[4][2], dd, dmin; };
+struct TileScales { float f[4][4], g[4][2], gq[2], dd, dmin; };   // gq: g[lane group]
 template <uint32_t MASK>
 __device__ __forceinline__ void mvq_row_scales(int fmt, const RawT16& r, uint32_t lane, TileScales& t) {
   const uint32_t n = lane & 15;
@@ -467,6 +468,7 @@ __device__ __forceinline__ void mvq_row_scales(int fmt, const RawT16& r, uint32_
       const float f[4] = {ub0(sc01), ub2(sc01), ub0(sc23), ub2(sc23)}, g[4] = {ub0(mn01), ub2(mn01), ub0(mn23), ub2(mn23)};
 #pragma unroll
       for (int pp = 0; pp < 4; pp++) { t.f[pp][2 * h] = t.f[pp][2 * h + 1] = f[pp]; t.g[pp][h] = g[pp]; }
+      t.gq[h] = ub0(((lane & 32) ? mn23 : mn01) >> (lane & 16));
     }
     t.dd = h2f(r.hd.x & 0xFFFFu);
     t.dmin = h2f(r.hd.x >> 16);
@@ -620,6 +622,245 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The same for formats whose weights are whole numbers below 64 (all but Q8_0), on the bf16 matrix cores: what a digit needs beside its product moves into the
+// operands.  mvqb4 spends eight vector instructions per (row, sequence, 16 elements): two shifts and additions of digit sums, two conversions, a fused
+// multiply-add, and the scales.  Here a digit is a bf16 number, the digit times its power of 256 times the chunk's scale, itself a power of two (both exact),
+// and the high two and the low two digits of 16 elements lie along one K of 32: the product IS the scaled high or low half, in f32.  Every partial sum is a whole
+// multiple of the scale below 2^24 of it (high digits |I| >> 16 <= 2^14, weights <= 63, 16 elements: 63 * 2^18 < 2^24), so nothing rounds in it.  What is left is one
+// addition (the halves: the rounding that the fused multiply-add of the other kernels does, shifted by a power of two) and the fused multiply-add with the weights' scale: the same
+// bits.  The sum over the minima, a chain of four fused multiply-adds, is a 16x16x4 f32 matrix instruction, which rounds as that chain does.
+//   A: row 4 m + 2 q + half of sequence m + 4 q of eight (a lane of group m gets both halves of sequences m and m + 4), K = lane group's four elements of the half's first digit, then of its second
+//   B: the lane group's four weights twice; a lane unpacks one chunk of 64 elements, so the chunks' words are exchanged between the lane groups (4 x 4, four swaps)
+// (Inputs beyond 2^117 in magnitude may overflow a half where a zero scale would have hidden it.)
+// The records are rewritten to this form as they are staged: 80 instructions per 32 digits (without them 2 % less time: not worth a second form of the
+// records in memory).  gate | up of an 8B model (28672 rows of 4096, Q4_K), 16 sequences: 58 us with mvqb4, 44 here, vector instructions three quarters of it.
+// ------------------------------------------------------------------------------------------------
+constexpr uint32_t kX8Group = 512;                   // a lane group's part of a record: [chunk 16][half 2][digit 2][element 4] bf16
+constexpr uint32_t kX8Record = 4 * kX8Group + 32;    // an odd multiple of 32: the halves of eight sequences fall into different banks, whichever lane groups read at once
+constexpr uint32_t kX8Sums = 80;                     // a record's 16 sums ([class][step]), behind all records; 16 sequences' in different banks
+constexpr uint32_t kX8Records = 32;                  // a chunk's records: two per 32 threads
+typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
+
+template <uint32_t MASK, int NB, bool SEQ>
+__global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  static_assert((MASK & (1u << F_Q80)) == 0, "weights of 8 bits do not fit the exact range");
+  constexpr int NG = (NB + 7) / 8;
+  auto nq = [](int g) { return NB - 8 * g > 4 ? 2 : 1; };          // a last group of up to four sequences: one per lane
+  const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
+  const bool active = u < Gm.n_units;
+  const int sg = (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  const MvSeg& S = L.seg[active ? sg : 0];
+  constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
+  const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
+  auto is = [&](int f) { return ((MASK >> f) & 1u) != 0 && (kSingle || fmt == f); };
+  const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q6K) ? fmt_tile_bytes(F_Q6K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K) : fmt_tile_bytes(F_Q40);
+  const uint32_t ntiles = (S.n_rows + 15) >> 4;
+  const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
+  const uint32_t pass = active ? ul / ntiles : 0, tl = active ? ul - pass * ntiles : 0;
+  const uint8_t* wbase = (pass == 0 ? S.pass[0].plane[0] : S.pass[1].plane[0]) + (size_t)tl * Gm.nblk * tb;
+  const uint32_t n = lane & 15, mq = lane >> 4;
+  const uint32_t ks0 = SEQ ? 0u : blockIdx.y, ks1 = SEQ ? Gm.T : blockIdx.y + 1;   // this workgroup's slices
+  float acc[NG][4][2], tot[NG][2];                                // per group: chunk classes, the lane's sequences 8 g + mq + 4 q
+#pragma unroll
+  for (int g = 0; g < NG; g++)
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      tot[g][q] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc[g][c][q] = 0.0f;
+    }
+
+  RawT16 nxt;
+  {
+    const uint32_t bfirst = ks0 * Gm.nbw;
+    if (active && bfirst < Gm.nblk) mvq_issue_tile<MASK>(fmt, wbase + (size_t)bfirst * tb, lane, nxt);
+  }
+  // a chunk of records (cb blocks x sequences): a thread has a chunk of 16 and a half of two records, fetched a chunk ahead and rewritten into a two-deep LDS buffer
+  const uint32_t sj = (tid >> 1) & 15, sh = tid & 1;
+  const uint32_t s_dig = (sj >> 1) * 128 + sh * 64 + (sj & 1) * 16, s_sum = kXqXs16 + (sj & 3) * 16 + (sj >> 2) * 4;
+  const uint32_t buf_recs = Gm.cb * n_seq, buf_bytes = buf_recs * (kX8Record + kX8Sums);
+  struct { u32x4 d[2]; float sx, xs; } stg[2];
+  auto chunk_len = [&](uint32_t ks, uint32_t b0) { return min(Gm.cb, min(ks * Gm.nbw + Gm.nbw, Gm.nblk) - b0); };
+  auto fetch = [&](uint32_t b0, uint32_t cn) {
+#pragma unroll
+    for (uint32_t k = 0; k < 2; k++) {
+      const uint32_t rec = (tid >> 5) + k * 16;
+      if (rec < cn * n_seq) {
+        const uint32_t bi = rec / n_seq, s = rec - bi * n_seq;
+        const uint8_t* p = L.seg[0].pass[0].xq + (size_t)s * B.xq_stride + (size_t)(b0 + bi) * kXqRecord;   // (all segments and passes share the input)
+        stg[k].d[0] = *reinterpret_cast<const u32x4*>(p + s_dig);
+        stg[k].d[1] = *reinterpret_cast<const u32x4*>(p + s_dig + 32);
+        stg[k].xs = *reinterpret_cast<const float*>(p + s_sum);
+        stg[k].sx = *reinterpret_cast<const float*>(p + s_sum + (kXqSx16 - kXqXs16));
+      }
+    }
+  };
+  auto stash = [&](uint32_t cn, uint32_t buf) {
+    auto pack = [](uint32_t w, float s) {
+      const float a = (float)(int)(int8_t)w * s, b = (float)(int)(int8_t)(w >> 8) * s, c = (float)(int)(int8_t)(w >> 16) * s, d = (float)((int)w >> 24) * s;
+      return make_uint2(__builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u), __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x07060302u));
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < 2; k++) {
+      const uint32_t rec = (tid >> 5) + k * 16;
+      if (rec < cn * n_seq) {
+        uint8_t* to = smem8 + buf * buf_bytes;
+        const float s0 = stg[k].sx * (sh ? 256.0f : 16777216.0f), s1 = stg[k].sx * (sh ? 1.0f : 65536.0f);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint2 a = pack(stg[k].d[0][e], s0), b = pack(stg[k].d[1][e], s1);
+          *reinterpret_cast<u32x4*>(to + rec * kX8Record + e * kX8Group + sj * 32 + sh * 16) = u32x4{a.x, a.y, b.x, b.y};
+        }
+        if (sh == 0) *reinterpret_cast<float*>(to + buf_recs * kX8Record + rec * kX8Sums + (sj & 3) * 16 + (sj >> 2) * 4) = stg[k].xs;
+      }
+    }
+  };
+  uint32_t ks = ks0, b0 = ks0 * Gm.nbw;
+  while (ks < ks1 && b0 >= min(ks * Gm.nbw + Gm.nbw, Gm.nblk)) { ks++; b0 = ks * Gm.nbw; }
+  uint32_t buf = 0;
+  if (ks < ks1) fetch(b0, chunk_len(ks, b0));
+  while (ks < ks1) {
+    const uint32_t sb1 = min(ks * Gm.nbw + Gm.nbw, Gm.nblk);
+    const uint32_t cn = chunk_len(ks, b0);
+    stash(cn, buf);
+    __syncthreads();
+    uint32_t nks = ks, nb0 = b0 + cn;   // the chunk after this one
+    if (nb0 >= sb1) {
+      nks = ks + 1; nb0 = nks * Gm.nbw;
+      while (nks < ks1 && nb0 >= min(nks * Gm.nbw + Gm.nbw, Gm.nblk)) { nks++; nb0 = nks * Gm.nbw; }
+    }
+    if (nks < ks1) fetch(nb0, chunk_len(nks, nb0));
+    if (active) {
+      for (uint32_t bi = 0; bi < cn; bi++) {
+        const uint32_t b = b0 + bi;
+        // sequences past the last one repeat it: computed, never stored
+        const uint8_t* rec0 = smem8 + buf * buf_bytes + bi * n_seq * kX8Record;
+        const uint8_t* sum0 = smem8 + buf * buf_bytes + buf_recs * kX8Record + bi * n_seq * kX8Sums;
+        const uint8_t *pa[NG], *px[NG][2];
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+          pa[g] = rec0 + min(8 * g + (n >> 2) + (n & 2) * 2, n_seq - 1) * kX8Record + mq * kX8Group + (n & 1) * 16;
+#pragma unroll
+          for (int q = 0; q < 2; q++) px[g][q] = sum0 + min(8 * g + mq + 4 * q, n_seq - 1) * kX8Sums;
+        }
+        const bool mins = is(F_Q4K) || is(F_Q5K);
+        float xm[4];   // the minima's operand: row 4 m + 2 g + q = sequence 8 g + m + 4 q, K = step
+        if (mins) {
+          const uint8_t* p = sum0 + min((n & 2) * 4 + (n >> 2) + (n & 1) * 4, n_seq - 1) * kX8Sums + mq * 4;
+#pragma unroll
+          for (int c = 0; c < 4; c++) xm[c] = *reinterpret_cast<const float*>(p + c * 16);
+        }
+        // steps (class, group), a step's products ahead of the vector work of the one before, its operands a step ahead of those
+        constexpr int kSteps = 4 * NG;
+        b16x8 a[2][4], w[4];
+        f32x4 d[2][4], xs[2][2], s2[2];
+        auto load_a = [&](int st) {
+#pragma unroll
+          for (int pp = 0; pp < 4; pp++) a[st & 1][pp] = *reinterpret_cast<const b16x8*>(pa[st % NG] + (pp * 4 + st / NG) * 32);
+        };
+        load_a(0);
+        load_a(1);
+        TileScales ts;
+        uint32_t tw[4][4];   // [step pp][class c]: the lane group's four weights of chunk 4 pp + c
+        {
+          TileOps t;
+          mvq_unpack_tile<MASK>(fmt, nxt, lane, t);
+          mvq_row_scales<MASK>(fmt, nxt, lane, ts);
+#pragma unroll
+          for (int pp = 0; pp < 4; pp++) {
+            const auto r01 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][0], (uint32_t)t.bw[pp][1], false, false);
+            const auto r23 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][2], (uint32_t)t.bw[pp][3], false, false);
+            const auto r02 = __builtin_amdgcn_permlane32_swap(r01[0], r23[0], false, false);
+            const auto r13 = __builtin_amdgcn_permlane32_swap(r01[1], r23[1], false, false);
+            tw[pp][0] = r02[0]; tw[pp][1] = r13[0]; tw[pp][2] = r02[1]; tw[pp][3] = r13[1];
+          }
+        }
+        {   // the unit's next tile (its next block — of this slice, or of the next one this workgroup walks)
+          uint32_t bn = b + 1;
+          if (bn == sb1) bn = nks < ks1 ? nb0 : Gm.nblk;
+          if (bn < Gm.nblk) mvq_issue_tile<MASK>(fmt, wbase + (size_t)bn * tb, lane, nxt);
+        }
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto products = [&](int st) {
+          const int c = st / NG, g = st % NG;
+          if (g == 0) {
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) {
+              const uint32_t v = tw[pp][c];
+              const uint32_t lo = __builtin_amdgcn_perm(__float_as_uint(ub1(v)), __float_as_uint(ub0(v)), 0x07060302u);
+              const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(ub3(v)), __float_as_uint(ub2(v)), 0x07060302u);
+              w[pp] = __builtin_bit_cast(b16x8, u32x4{lo, hi, lo, hi});
+            }
+            if (mins) s2[c & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xm[c], ts.gq[c >> 1], zero, 0, 0, 0);
+          }
+#pragma unroll
+          for (int pp = 0; pp < 4; pp++) d[st & 1][pp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[st & 1][pp], w[pp], zero, 0, 0, 0);
+          if (!mins) {
+#pragma unroll
+            for (int q = 0; q < nq(g); q++) xs[st & 1][q] = *reinterpret_cast<const f32x4*>(px[g][q] + c * 16);
+          }
+        };
+        products(0);
+#pragma unroll
+        for (int st = 0; st < kSteps; st++) {
+          const int c = st / NG, g = st % NG;
+          if (st + 1 < kSteps) {   // (ahead of the other wave's vector work)
+            __builtin_amdgcn_s_setprio(1);
+            products(st + 1);
+            __builtin_amdgcn_s_setprio(0);
+          }
+          if (st + 2 < kSteps) load_a(st + 2);
+#pragma unroll
+          for (int q = 0; q < nq(g); q++) {
+            float s1 = 0.0f, V[4];
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) V[pp] = d[st & 1][pp][2 * q] + d[st & 1][pp][2 * q + 1];
+            if (mins) {
+#pragma unroll
+              for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], V[pp], s1);
+              acc[g][c][q] += ts.dd * s1 - ts.dmin * s2[c & 1][2 * g + q];
+            } else {
+#pragma unroll
+              for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], __builtin_fmaf(is(F_Q40) ? -8.0f : -32.0f, xs[st & 1][q][pp], V[pp]), s1);
+              acc[g][c][q] = is(F_Q40) ? acc[g][c][q] + s1 : __builtin_fmaf(ts.dd, s1, acc[g][c][q]);
+            }
+            asm volatile("" : "+v"(acc[g][c][q]));   // here, not sunk past the later steps' products
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if (b0 + cn >= sb1) {   // end of the k-slice: the slice's partial sum, in the single-sequence kernel's order
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+#pragma unroll
+          for (int q = 0; q < 2; q++) {
+            const float t = (acc[g][0][q] + acc[g][1][q]) + (acc[g][2][q] + acc[g][3][q]);
+            if (SEQ) tot[g][q] += t;
+            else tot[g][q] = t;
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[g][c][q] = 0.0f;
+          }
+      }
+    }
+    ks = nks; b0 = nb0; buf ^= 1u;
+  }
+  if (active) {
+    const uint32_t slot = SEQ ? 0u : blockIdx.y;
+    const size_t rows16 = (size_t)Gm.n_units * 16;
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const uint32_t s = 8 * g + mq + 4 * q;
+        if (q < nq(g) && s < n_seq) part[((size_t)slot * n_seq + s) * rows16 + (size_t)u * 16 + n] = tot[g][q];
+      }
+  }
+}
+
 // grid / block = the single-sequence geometry of `L` (segments' wg_begin, rows_per_wg).  dynamic LDS: mvqb_lds_bytes(n_seq, L.red_floats)
 __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_floats,
                                                                       const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B,
@@ -681,6 +922,26 @@ static hipError_t mvqb_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, 
 // Indirect launches (a mixture's experts) have one or two sequences per expert: they stay with mvqb2.
 constexpr uint32_t kMvqb4MinSeq = 3;
 
+// Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers of an 8B model in Q4_K_M / Q4_0, us, groups of four against
+// groups of eight: 3 sequences 391 / 378 against 440 / 414, 4: 406 / 381 against 447 / 423; 5: 503 / 484 against 479 / 455, 8: 531 / 512 against 502 / 480,
+// 9: 648 / 624 against 581 / 564, 16: 786 / 761 against 683 / 679)
+constexpr uint32_t kMvqb8MinSeq = 5;
+
+template <uint32_t MASK, int NB>
+static hipError_t mvqb8_go(const MvLaunch& L, const MvBatch& B, Mvqb2Geom Gm, bool seq, uint32_t groups, hipStream_t st) {
+  static bool attr_set[2][64] = {};
+  Gm.cb = std::max(1u, std::min(Gm.nbw, kX8Records / B.n_seq));
+  const size_t lds = (size_t)2 * Gm.cb * B.n_seq * (kX8Record + kX8Sums);
+  if (seq) {
+    if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb8_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
+    hipLaunchKernelGGL((mvqb8_kernel<MASK, NB, true>), dim3(groups), dim3(kBWaves * 64), lds, st, Gm, L, B, B.part);
+  } else {
+    if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb8_kernel<MASK, NB, false>), 160 * 1024, attr_set[1]); e != hipSuccess) return e;
+    hipLaunchKernelGGL((mvqb8_kernel<MASK, NB, false>), dim3(groups, Gm.T), dim3(kBWaves * 64), lds, st, Gm, L, B, B.part);
+  }
+  return hipGetLastError();
+}
+
 template <uint32_t MASK, int NB>
 static hipError_t mvqb4_go(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, bool seq, uint32_t groups, hipStream_t st) {
   static bool attr_set[2][64] = {};
@@ -701,7 +962,13 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   static bool attr_set[3][64] = {};
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
-    if (hipError_t e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st); e != hipSuccess) return e;
+    hipError_t e;
+    if constexpr ((MASK & (1u << F_Q80)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
+    else if (B.n_seq < kMvqb8MinSeq) e = mvqb4_go<MASK, 4>(L, B, Gm, seq, groups, st);
+    else if (B.n_seq <= 8) e = mvqb8_go<MASK, 8>(L, B, Gm, seq, groups, st);
+    else if (B.n_seq <= 12) e = mvqb8_go<MASK, 12>(L, B, Gm, seq, groups, st);
+    else e = mvqb8_go<MASK, 16>(L, B, Gm, seq, groups, st);
+    if (e != hipSuccess) return e;
   } else if (seq) {
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb2_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
     hipLaunchKernelGGL((mvqb2_kernel<MASK, NB, true>), dim3(groups, 1, nz), dim3(kBWaves * 64), lds_x, st, Gm, L, B, B.part);

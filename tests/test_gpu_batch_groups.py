@@ -1,5 +1,6 @@
-"""The batched step's mat-vec from three sequences on takes them in groups (matvec_batch.hip): group sizes around full ones, every
-weight format, plans with whole rows per workgroup and plans with k-slices.
+"""The batched step's mat-vec from three sequences on takes them in groups (matvec_batch.hip: of four on the integer matrix cores, from five
+sequences on of eight on the bf16 ones, 8-bit weights apart): group sizes around full ones, every weight format, plans with whole rows per
+workgroup and plans with k-slices.
 
 Per (row, sequence) the kernel does the single-sequence kernel's floating-point operations in its order, on sums that are exact, so the
 bound is equality of all bits with a single-sequence engine that runs the split attention too (attn_direct=255)."""
