@@ -534,23 +534,6 @@ hipError_t attn_launch(const float* q, const float* kcache, const float* vcache,
 // (One workgroup per kv head, each wave with all its query heads, took 10.0 us at 8 heads of 64 and 6.5 at 4 of 128 and 40 rows, split and merge 10.1 at
 // 128 rows of the latter; this 3.8 and 4.8.  A token of TinyLlama-1.1B Q4_K_M at 40 rows 766 -> 626 us, of Llama-3-8B Q4_K_M at 130 1695 -> 1582 us, both with
 // the logits to the host.)
-__device__ __forceinline__ float swap16_add(float v) {   // sum of rows 2i and 2i + 1 of 16 lanes, in both
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float swap32_add(float v) {   // sum of lanes l and l + 32, in both
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float swap16_max(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float swap32_max(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 template <int D>
 __global__ void __launch_bounds__(1024) attn_direct_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, uint32_t n_kv,
                                                            uint32_t g_per_kv, uint32_t max_seq, float scale, const int* pos_ptr, float* __restrict__ out,

@@ -22,7 +22,7 @@
 // (R^-1 is linear; rotation.rs:80-96) — the same terms in another order, equal to f32 rounding; like the f32 attention it does not
 // apply the reference's `weight < 1e-8` skip (each skipped term is < 1e-8 of the output scale).
 //
-// Launch structure = the f32 / int8 caches': (kv head x split) workgroups leave (m, l, acc) partials, a merge kernel per query
+// Launch structure of long contexts and of the caches with sign bits = the f32 / int8 caches': (kv head x split) workgroups leave (m, l, acc) partials, a merge kernel per query
 // head combines them — plus, here, the inverse rotation and the XQ image for the output projection.  The QKV launch leaves the
 // current token's rotated-by-RoPE K row and V row as f32 in a staging vector; every workgroup of a kv head compresses them
 // itself (identical bits everywhere), split 0 stores the codes at row `pos`, and the row takes part through its codes.
@@ -104,23 +104,23 @@ __device__ __forceinline__ void tq_fwht_wave(float& x0, float& x1, uint32_t lane
   }
 }
 
-// codes of the D floats at `y` (already rotated) -> row bytes, by the first D / 4 (2 bits) or D / 8 (3 bits) threads
+// codes of the D floats at `y` (already rotated) -> row bytes, by the first D / 4 (2 bits) or D / 8 (3 bits) threads (`t`: which one this is)
 template <int D, int BITS>
-__device__ __forceinline__ void tq_pack_row(const TqTables& T, const float* y, uint8_t* out) {
+__device__ __forceinline__ void tq_pack_row(const TqTables& T, const float* y, uint8_t* out, uint32_t t = threadIdx.x) {
   if (BITS == 2) {
-    if (threadIdx.x < D / 4) {
+    if (t < D / 4) {
       uint32_t byte = 0;
 #pragma unroll
-      for (int i = 0; i < 4; i++) byte |= tq_quantize<2>(T, y[threadIdx.x * 4 + i]) << (i * 2);
-      out[threadIdx.x] = (uint8_t)byte;
+      for (int i = 0; i < 4; i++) byte |= tq_quantize<2>(T, y[t * 4 + i]) << (i * 2);
+      out[t] = (uint8_t)byte;
     }
-  } else if (threadIdx.x < D / 8) {
+  } else if (t < D / 8) {
     uint32_t acc = 0;
 #pragma unroll
-    for (int i = 0; i < 8; i++) acc |= tq_quantize<3>(T, y[threadIdx.x * 8 + i]) << (i * 3);
-    out[threadIdx.x * 3] = (uint8_t)(acc & 0xFF);
-    out[threadIdx.x * 3 + 1] = (uint8_t)((acc >> 8) & 0xFF);
-    out[threadIdx.x * 3 + 2] = (uint8_t)((acc >> 16) & 0xFF);
+    for (int i = 0; i < 8; i++) acc |= tq_quantize<3>(T, y[t * 8 + i]) << (i * 3);
+    out[t * 3] = (uint8_t)(acc & 0xFF);
+    out[t * 3 + 1] = (uint8_t)((acc >> 8) & 0xFF);
+    out[t * 3 + 2] = (uint8_t)((acc >> 16) & 0xFF);
   }
 }
 
@@ -465,6 +465,162 @@ __global__ void __launch_bounds__(D) attn_tq_combine_kernel(const float* __restr
   if (xq_out) xq_store_chunk(xq_out, (h * D + dim) >> 4, o);
 }
 
+// ------------------------------------------------------------------------------------------------
+// Short contexts: one launch, a workgroup of 16 waves per QUERY head (as the f32 cache's attn_direct_kernel).  The split kernel and its merge are two launches of
+// which neither has much to do: at 500 rows of an 8B model (3 bits) 11.6 + 4.9 us, the rotations, the merge of four heads' accumulators across the lanes and the
+// launches, not the 400 KB of codes.  Here a wave rotates one vector (the head's query, the new K row, the new V row, each packed by the wave that rotated it),
+// 16 waves take 16 * 1024 / D rows a round, one head's accumulators meet in registers, and the first wave merges the waves, inverts the rotation and writes the
+// projection's input: 7.8 us.  Every head of a kv head packs the new row itself (identical bits); the first one stores it.
+// ------------------------------------------------------------------------------------------------
+template <int D, int BITS, bool MULTI>
+__global__ void __launch_bounds__(1024) attn_tq_direct_kernel(const float* __restrict__ q, uint8_t* __restrict__ kq, uint8_t* __restrict__ vq,
+                                                              const float* __restrict__ k_new, const float* __restrict__ v_new,
+                                                              const float* __restrict__ signs, const TqTables T, uint32_t g_per_kv, uint32_t max_seq, float scale,
+                                                              const int* pos_ptr, float* __restrict__ out, uint8_t* __restrict__ xq_out, const TqMulti ms, uint32_t xq_stride) {
+  constexpr uint32_t RB = tq_row_bytes<BITS>(D);
+  constexpr int LPR = D / 16, RPW = 64 / LPR, NW = 16;               // lanes per row, rows per wave and round, waves
+  __shared__ float rot[3][D];
+  __shared__ __attribute__((aligned(16))) uint8_t newrow[2][64];
+  __shared__ float s_m[NW], s_l[NW];
+  __shared__ float s_acc[NW][D];
+  __shared__ float s_cen[8];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t h = blockIdx.x, kvh = h / g_per_kv;
+  uint32_t pos;
+  if (MULTI) {   // blockIdx.y = the sequence: its position and its slot's rows
+    const uint32_t sq = blockIdx.y;
+    uint32_t sl;
+    asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(pos), "=&s"(sl) : "s"(pos_ptr + sq), "s"(ms.slot + sq) : "memory");
+    q += (size_t)sq * gridDim.x * D;
+    k_new += (size_t)sq * ms.kv_stride;
+    v_new += (size_t)sq * ms.kv_stride;
+    kq += (size_t)sl * ms.code_stride;
+    vq += (size_t)sl * ms.code_stride;
+    out += (size_t)sq * gridDim.x * D;
+    if (xq_out) xq_out += (size_t)sq * xq_stride;
+  }
+  const float* sk = signs + (size_t)(kvh * 2) * D;
+  const float* sv = sk + D;
+  uint8_t* krow0 = kq + (size_t)kvh * max_seq * RB;
+  uint8_t* vrow0 = vq + (size_t)kvh * max_seq * RB;
+  const uint32_t sub = lane / LPR, li = lane % LPR;
+  auto load_codes = [&](const uint8_t* row) -> unsigned long long {   // this lane's 16 codes of a row, as in the split kernel
+    if (BITS == 2) return *reinterpret_cast<const uint32_t*>(row + li * 4);
+    const uint32_t off = li * 6, al = off & ~3u;
+    const unsigned long long w = (unsigned long long)*reinterpret_cast<const uint32_t*>(row + al) |
+                                 (unsigned long long)*reinterpret_cast<const uint32_t*>(row + (al + 4 < RB ? al + 4 : al)) << 32;
+    return w >> ((off & 3u) * 8);
+  };
+  constexpr int kAhead = 2;
+  constexpr uint32_t kRound = NW * RPW;
+  unsigned long long kk[kAhead], vv[kAhead];
+  const uint32_t first = wave * RPW + sub;
+#pragma unroll
+  for (int j = 0; j < kAhead; j++) {                                  // requested before the position is known: rows inside the cache, masked below
+    const uint32_t p = min(first + j * kRound, max_seq - 1);
+    kk[j] = load_codes(krow0 + (size_t)p * RB);
+    vv[j] = load_codes(vrow0 + (size_t)p * RB);
+  }
+  if (!MULTI) asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pos) : "s"(pos_ptr) : "memory");
+  if (wave == NW - 1 && lane < 8) s_cen[lane] = T.cen[lane & ((1u << BITS) - 1u)];
+  if (wave < 3) {
+    const float* src = wave == 0 ? q + (size_t)h * D : wave == 1 ? k_new + (size_t)kvh * D : v_new + (size_t)kvh * D;
+    const float* sg = wave < 2 ? sk : sv;
+    float x0 = src[lane] * sg[lane], x1 = 0.0f;
+    if (D == 128) x1 = src[lane + 64] * sg[lane + 64];
+    tq_fwht_wave<D>(x0, x1, lane);
+    rot[wave][lane] = x0 * T.norm;
+    if (D == 128) rot[wave][lane + 64] = x1 * T.norm;
+    __builtin_amdgcn_wave_barrier();
+    if (wave > 0) tq_pack_row<D, BITS>(T, rot[wave], newrow[wave - 1], lane);
+  }
+  __syncthreads();
+  if (h == kvh * g_per_kv && tid < RB) { krow0[(size_t)pos * RB + tid] = newrow[0][tid]; vrow0[(size_t)pos * RB + tid] = newrow[1][tid]; }
+  float rq[16], acc[16], m = -1e30f, l = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 16; c++) { rq[c] = rot[0][li * 16 + c]; acc[c] = 0.0f; }
+  // centroid of code c: from LDS (8 addresses, no bank conflicts), two instructions for its offset; picking it by selects takes eleven and was three quarters of a row
+  auto centroid = [&](unsigned long long codes, int c) {
+    const uint32_t w = c == 0 ? (uint32_t)codes << 2 : (uint32_t)(codes >> (c * BITS >= 2 ? c * BITS - 2 : 0));
+    return *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(s_cen) + (w & (((1u << BITS) - 1u) << 2)));
+  };
+  auto step = [&](uint32_t p, unsigned long long kc, unsigned long long vc) {
+    const bool valid = p <= pos;
+    if (p == pos) { kc = load_codes(newrow[0]); vc = load_codes(newrow[1]); }
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 16; c++) s = __builtin_fmaf(rq[c], centroid(kc, c), s);
+    s += dpp_f<0xB1>(s);
+    s += dpp_f<0x4E>(s);
+    if (LPR >= 8) s += dpp_f<0x141>(s);
+    s *= scale;
+    const float mn = valid ? fmaxf(m, s) : m, a = __expf(m - mn), pe = valid ? __expf(s - mn) : 0.0f;
+    l = __builtin_fmaf(l, a, pe);
+    m = mn;
+#pragma unroll
+    for (int c = 0; c < 16; c++) acc[c] = __builtin_fmaf(acc[c], a, centroid(vc, c) * pe);
+  };
+  for (uint32_t base = wave * RPW; base <= pos; base += kAhead * kRound) {   // wave-uniform
+    unsigned long long k2[kAhead], v2[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) {
+      k2[j] = kk[j]; v2[j] = vv[j];
+      const uint32_t nx = base + (kAhead + j) * kRound;
+      if (nx <= pos) {                                                // the round after this one
+        const uint32_t p = min(nx + sub, pos);
+        kk[j] = load_codes(krow0 + (size_t)p * RB);
+        vv[j] = load_codes(vrow0 + (size_t)p * RB);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; j++)
+      if (base + j * kRound <= pos) step(base + j * kRound + sub, k2[j], v2[j]);
+  }
+  // the wave's row slots: lanes with equal li hold the same coordinates (sums over the row of 16 lanes by rotations, then over the rows)
+  auto sum_slots = [&](float v) {
+    v += dpp_f<0x128>(v);
+    if (LPR < 8) v += dpp_f<0x124>(v);
+    return swap32_add(swap16_add(v));
+  };
+  float wm = fmaxf(m, dpp_f<0x128>(m));
+  if (LPR < 8) wm = fmaxf(wm, dpp_f<0x124>(wm));
+  wm = swap32_max(swap16_max(wm));
+  const float f = expf(m - wm);
+  const float wl = sum_slots(l * f);
+#pragma unroll
+  for (int c = 0; c < 16; c++) acc[c] = sum_slots(acc[c] * f);
+  if (sub == 0) {
+    if (li == 0) { s_m[wave] = wm; s_l[wave] = wl; }
+#pragma unroll
+    for (int c = 0; c < 16; c++) s_acc[wave][li * 16 + c] = acc[c];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  // the first wave: the waves' parts, then out = signs * (1 / d) * H (sqrt(d) * o), as attn_tq_combine_kernel
+  float mn = s_m[0];
+#pragma unroll
+  for (int w = 1; w < NW; w++) mn = fmaxf(mn, s_m[w]);
+  float lsum = 0.0f, a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+  for (int w = 0; w < NW; w++) {
+    const float fw = expf(s_m[w] - mn);
+    lsum += s_l[w] * fw;
+    a0 += s_acc[w][lane] * fw;
+    if (D == 128) a1 += s_acc[w][lane + (D == 128 ? 64 : 0)] * fw;
+  }
+  const float linv = 1.0f / lsum;
+  a0 = (a0 * linv) * T.inv_scale;
+  a1 = (a1 * linv) * T.inv_scale;
+  tq_fwht_wave<D>(a0, a1, lane);
+#pragma unroll
+  for (int e = 0; e < D / 64; e++) {
+    const uint32_t dim = lane + e * 64;
+    const float o = (e ? a1 : a0) * T.inv_d * sv[dim];
+    out[(size_t)h * D + dim] = o;
+    if (xq_out) xq_store_chunk(xq_out, (h * D + dim) >> 4, o);
+  }
+}
+
 // one row through the compressor (the code path of attn_tq_partial_kernel's new-row handling, stand-alone): lgh_op_tq_compress
 template <int D, int BITS>
 __global__ void __launch_bounds__(256) tq_compress_kernel(const float* __restrict__ x, const float* __restrict__ signs, const TqTables T,
@@ -555,6 +711,28 @@ hipError_t attn_tq_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, co
     return hipErrorInvalidValue;
   const TqArgs a{q, kq, vq, k_new, v_new, signs, n_kv, max_seq, scale, pos, n_splits, part_ml, part_acc, qjl_s, kx, st, 0, TqMulti{}};
   return attn_tq_dispatch(bits, head_dim, n_heads / n_kv, a);
+}
+
+// one launch instead of attn_tq_launch + attn_tq_combine_launch (caches without the residual's sign bits).  n_seq 0: a single sequence; otherwise grid y =
+// sequences as in attn_tq_multi_launch
+hipError_t attn_tq_direct_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, const float* k_new, const float* v_new, const float* signs,
+                                 uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos, float* out, uint8_t* xq_out,
+                                 hipStream_t st, uint32_t n_seq, const int* slot, uint64_t code_stride, uint32_t kv_stride, uint32_t xq_stride) {
+  if (n_kv == 0 || n_heads % n_kv || !pos || max_seq == 0 || (n_seq && !slot)) return hipErrorInvalidValue;
+  const TqMulti ms{slot, code_stride, 0, kv_stride};
+#define LGH_TQ_GO(DD, BB, MU)                                                                                                                               \
+  hipLaunchKernelGGL((attn_tq_direct_kernel<DD, BB, MU>), dim3(n_heads, MU ? n_seq : 1), dim3(1024), 0, st, q, kq, vq, k_new, v_new, signs, tq_tables(DD, BB), \
+                     n_heads / n_kv, max_seq, scale, pos, out, xq_out, ms, xq_stride)
+#define LGH_TQ_CASE(DD, BB)                   \
+  if (head_dim == DD && bits == BB) {         \
+    if (n_seq) LGH_TQ_GO(DD, BB, true);       \
+    else LGH_TQ_GO(DD, BB, false);            \
+    return hipGetLastError();                 \
+  }
+  LGH_TQ_CASE(128, 2) LGH_TQ_CASE(128, 3) LGH_TQ_CASE(64, 2) LGH_TQ_CASE(64, 3)
+#undef LGH_TQ_CASE
+#undef LGH_TQ_GO
+  return hipErrorInvalidValue;
 }
 
 // the same for n_seq sequences (grid y): positions pos[s], cache slots slot[s] (code_stride bytes / x_stride words between slots),

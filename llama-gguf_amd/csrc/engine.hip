@@ -64,7 +64,9 @@ void dev_free_tracked(lgh_ctx* c, void* p) {
 // Contexts up to this many rows run the single-launch decode attention (attention.hip, attn_direct_kernel) unless the flags say otherwise.  Measured against
 // the split kernel with its merge, us per layer gained: 8 kv heads of 128 with 4 query heads each 4.8 / 5.1 / 3.8 / 2.4 / 1.6 / 0.2 / -0.4 at 40 / 144 / 256 /
 // 512 / 1000 / 1500 / 3000 rows (a query head's rows all pass through one CU), 4 of 64 with 8 each 6.9 / 7.2 / 7.4 / 6.3 / 5.6 / 5.6 / 4.3 at the same, 4.3 at 4000.
-static uint32_t direct_attn_default_kv(uint32_t head_dim) { return head_dim == 64 ? 4096 : 1024; }
+// TurboQuant caches (attn_tq_direct_kernel), the same two models, 3 / 2 bits: 10.8 / 9.1 and 20.3 / 20.0 us gained at 512 rows, 9.7 / 7.6 and 19.9 / 19.3 at 8000: a row is
+// a tenth of the bytes (measured no further).
+static uint32_t direct_attn_default_kv(uint32_t head_dim, bool tq) { return tq ? 8192 : head_dim == 64 ? 4096 : 1024; }
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ------------------------------------------------------------------------------------------------
@@ -565,17 +567,25 @@ static int layer_forward(lgh_ctx* c, uint32_t li, const float* next_nw, bool nex
     const float* qjl_s = qjl ? c->tq_qjl + (size_t)(li - c->l0) * d.num_kv_heads * d.head_dim * d.head_dim : nullptr;
     const uint64_t tq_bytes = (uint64_t)d.num_kv_heads * (c->pos + 1) * (2 * tq_row_bytes_host(bits, d.head_dim) + (qjl ? d.head_dim / 8 + 4 : 0)) +
                               (qjl ? (uint64_t)d.num_kv_heads * d.head_dim * d.head_dim * 4 : 0);
-    if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, tq_bytes, [&] {
-           return attn_tq_launch(bits, c->q, (uint8_t*)Lw.k8, (uint8_t*)Lw.v8, k_new, v_new, signs, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len,
-                                 scale, c->state + ST_POS, c->n_splits, c->part_ml, c->part_acc, c->stream, qjl_s, qjl ? Lw.kx : nullptr);
-         })))
-      return rc;
     XqBuf* qa = mfma_type(Lw.wo.type) ? xq_get(c, c->attn_out, d.num_heads * d.head_dim) : nullptr;
-    if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
-           return attn_tq_combine_launch(bits, c->part_ml, c->part_acc, signs, d.num_heads, d.num_kv_heads, d.head_dim, c->n_splits, c->attn_out,
-                                         qa ? qa->xq : nullptr, c->stream);
-         })))
-      return rc;
+    if (c->attn_direct && !qjl) {
+      if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, tq_bytes, [&] {
+             return attn_tq_direct_launch(bits, c->q, (uint8_t*)Lw.k8, (uint8_t*)Lw.v8, k_new, v_new, signs, d.num_heads, d.num_kv_heads, d.head_dim,
+                                          d.max_seq_len, scale, c->state + ST_POS, c->attn_out, qa ? qa->xq : nullptr, c->stream);
+           })))
+        return rc;
+    } else {
+      if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, tq_bytes, [&] {
+             return attn_tq_launch(bits, c->q, (uint8_t*)Lw.k8, (uint8_t*)Lw.v8, k_new, v_new, signs, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len,
+                                   scale, c->state + ST_POS, c->n_splits, c->part_ml, c->part_acc, c->stream, qjl_s, qjl ? Lw.kx : nullptr);
+           })))
+        return rc;
+      if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
+             return attn_tq_combine_launch(bits, c->part_ml, c->part_acc, signs, d.num_heads, d.num_kv_heads, d.head_dim, c->n_splits, c->attn_out,
+                                           qa ? qa->xq : nullptr, c->stream);
+           })))
+        return rc;
+    }
     if (qa) { qa->fresh = true; qa->tag = nullptr; }
     else xq_stale(c, c->attn_out);
   } else if (kv8) {
@@ -1193,8 +1203,9 @@ int lgh_create(const lgh_model_desc* desc, lgh_ctx** out) {
   if (splits > 32) splits = 32;   // the split merge keeps one partial per split in registers
   c->n_splits = splits;
   const uint32_t dsel = (d.flags >> LGH_FLAG_ATTN_DIRECT_SHIFT) & 0xFFu;
-  c->direct_attn_max_kv = dsel == 255 ? 0 : dsel ? dsel * 64 : direct_attn_default_kv(d.head_dim);
-  if (d.flags & LGH_FLAG_KV_INT8) c->direct_attn_max_kv = 0;   // the byte caches have one attention structure: splits + combine
+  const bool tq_direct = kv_is_tq(d.kv_cache_type) && !kv_is_qjl(d.kv_cache_type);
+  c->direct_attn_max_kv = dsel == 255 ? 0 : dsel ? dsel * 64 : direct_attn_default_kv(d.head_dim, tq_direct);
+  if ((d.flags & LGH_FLAG_KV_INT8) && !tq_direct) c->direct_attn_max_kv = 0;   // the other byte caches have one attention structure: splits + combine
   *out = c;
   return LGH_OK;
 }

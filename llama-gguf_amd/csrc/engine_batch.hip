@@ -209,18 +209,27 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       const uint32_t KD = d.num_kv_heads * d.head_dim;
       const float* signs = c->tq_signs + (size_t)(li - c->l0) * d.num_kv_heads * 2 * d.head_dim;
       const float* qjl_s = qjl ? c->tq_qjl + (size_t)(li - c->l0) * d.num_kv_heads * d.head_dim * d.head_dim : nullptr;
-      if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
-             return attn_tq_multi_launch(bits, Bs.q, Bs.kq[li], Bs.vq[li], Bs.kv_tmp, Bs.kv_tmp + KD, signs, d.num_heads, d.num_kv_heads, d.head_dim,
-                                         d.max_seq_len, scale, Bs.d_pos, Bs.d_slot, Bs.code_stride, Bs.x_stride, 2 * KD, n_seq, c->n_splits, Bs.part_ml,
-                                         Bs.part_acc, c->stream, qjl_s, qjl ? Bs.kx[li] : nullptr);
-           })))
-        return rc;
       XqBuf* qa = view_of(c, Bs.attn_out);
-      if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
-             return attn_tq_combine_launch(bits, Bs.part_ml, Bs.part_acc, signs, d.num_heads, d.num_kv_heads, d.head_dim, c->n_splits, Bs.attn_out, qa->xq,
-                                           c->stream, n_seq, (uint32_t)xq_stride_of(QD));
-           })))
-        return rc;
+      if (!qjl && d.max_seq_len <= c->direct_attn_max_kv) {   // every context takes the single-launch form, as the single-sequence engine's do (the same bits)
+        if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
+               return attn_tq_direct_launch(bits, Bs.q, Bs.kq[li], Bs.vq[li], Bs.kv_tmp, Bs.kv_tmp + KD, signs, d.num_heads, d.num_kv_heads, d.head_dim,
+                                            d.max_seq_len, scale, Bs.d_pos, Bs.attn_out, qa->xq, c->stream, n_seq, Bs.d_slot, Bs.code_stride, 2 * KD,
+                                            (uint32_t)xq_stride_of(QD));
+             })))
+          return rc;
+      } else {
+        if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
+               return attn_tq_multi_launch(bits, Bs.q, Bs.kq[li], Bs.vq[li], Bs.kv_tmp, Bs.kv_tmp + KD, signs, d.num_heads, d.num_kv_heads, d.head_dim,
+                                           d.max_seq_len, scale, Bs.d_pos, Bs.d_slot, Bs.code_stride, Bs.x_stride, 2 * KD, n_seq, c->n_splits, Bs.part_ml,
+                                           Bs.part_acc, c->stream, qjl_s, qjl ? Bs.kx[li] : nullptr);
+             })))
+          return rc;
+        if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
+               return attn_tq_combine_launch(bits, Bs.part_ml, Bs.part_acc, signs, d.num_heads, d.num_kv_heads, d.head_dim, c->n_splits, Bs.attn_out, qa->xq,
+                                             c->stream, n_seq, (uint32_t)xq_stride_of(QD));
+             })))
+          return rc;
+      }
       for (uint32_t s = 0; s < n_seq; s++)
         if (XqBuf* q = view_of(c, Bs.attn_out + (size_t)s * QD)) { q->fresh = true; q->tag = nullptr; }
     } else {

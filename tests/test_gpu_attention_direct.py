@@ -29,3 +29,27 @@ def test_direct_attention_matches_the_split_kernel(pkg, head_dim, heads, kv_head
             eng.forward_batch(prompt[rows - 1:])
     direct.close()
     split.close()
+
+
+@pytest.mark.parametrize("bits", [2, 3])
+@pytest.mark.parametrize("head_dim,heads,kv_heads", [(64, 8, 8), (64, 8, 1), (128, 4, 2), (128, 8, 1)])
+def test_direct_attention_over_codes_matches_the_split_kernel(pkg, head_dim, heads, kv_heads, bits):
+    """The same over a TurboQuant cache (attn_tq_direct_kernel): rounds of 128 rows of 128 values, 256 of 64, two ahead.  One layer, so that both
+    engines store the same codes (behind a second one a value at a cell's border could fall to either side)."""
+    cfg = pkg.make_config("test-dense", max_seq_len=640, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, num_layers=1)
+    model = pkg.SynthModel(cfg, mix="Q8_0")
+    signs = np.where(np.random.default_rng(3).random(kv_heads * 2 * head_dim) < 0.5, -1.0, 1.0).astype(np.float32)
+    kv = {2: pkg.hip_backend.KV_TQ2, 3: pkg.hip_backend.KV_TQ3}[bits]
+    direct, split = (pkg.HipGpuInference.from_model(model, 640, attn_direct=d, kv_cache_type=kv, kv_rotation_signs=signs) for d in (16, 255))
+    prompt = [(7 * i + 5) % cfg.vocab_size for i in range(620)]
+    for eng in (direct, split):
+        for t in prompt:
+            eng.prefill_token(t)
+    for rows in ROWS:
+        got = []
+        for eng in (direct, split):
+            eng.kv_truncate(rows - 1)
+            got.append(eng.forward(prompt[rows - 1]))       # (the row that was there)
+        assert np.abs(got[0] - got[1]).max() <= 2e-4 * np.abs(got[1]).max(), rows
+    direct.close()
+    split.close()
