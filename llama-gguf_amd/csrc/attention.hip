@@ -17,6 +17,7 @@
 //     a tiny combine kernel across splits.
 // The reference CPU path skips softmax weights <= 1e-8 (ops.rs:1529); like the reference's own GPU
 // kernel this one does not (each skipped term is < 1e-8 of the output scale).
+#include <algorithm>
 #include <cstdlib>
 
 #include "device_utils.h"
@@ -43,14 +44,16 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
                                                            const float* __restrict__ vc, uint32_t max_seq, float scale,
                                                            const int* pos_ptr, int kv_len_fixed, uint32_t n_splits,
                                                            float* __restrict__ part_ml, float* __restrict__ part_acc,
-                                                           const int* __restrict__ slot = nullptr, uint64_t slot_stride = 0) {
+                                                           const int* __restrict__ slot = nullptr, uint64_t slot_stride = 0, uint32_t grid_splits = 0) {
   constexpr int LPR = D / 4;       // lanes per row
   constexpr int RPW = 64 / LPR;    // rows per wave-instruction
   __shared__ float s_ml[NW][G][2];
   __shared__ float s_acc[NW][G][D];
   LGH_TL_BEGIN(attn, lgh::TL_ATTN, n_splits);
 
-  const uint32_t kvh = blockIdx.x / n_splits, sp = blockIdx.x % n_splits;
+  const uint32_t gs = MULTI ? grid_splits : n_splits;
+  const uint32_t kvh = blockIdx.x / gs;
+  uint32_t sp = blockIdx.x % gs;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t sub = lane / LPR, li = lane % LPR;
   // the position word by SCALAR load: the loop bounds depend on it, and a vector load here would be a full memory round
@@ -64,11 +67,11 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
     uint32_t pw, sl;
     asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(pw), "=&s"(sl) : "s"(pos_ptr + sq), "s"(slot + sq) : "memory");
     kv_len = pw + 1;
-    q += (size_t)sq * (gridDim.x / n_splits) * G * D;
+    q += (size_t)sq * (gridDim.x / gs) * G * D;
     kc += (size_t)sl * slot_stride;
     vc += (size_t)sl * slot_stride;
-    part_ml += (size_t)sq * gridDim.x * G * 2;
-    part_acc += (size_t)sq * gridDim.x * G * D;
+    part_ml += (size_t)sq * (gridDim.x / gs) * n_splits * G * 2;
+    part_acc += (size_t)sq * (gridDim.x / gs) * n_splits * G * D;
   } else if (pos_ptr) {
     uint32_t pw;
     asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pw) : "s"(pos_ptr) : "memory");
@@ -81,9 +84,6 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
 
   float m[G], l[G];
   f32x4 acc[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) { m[g] = kNegBig; l[g] = 0.0f; acc[g] = (f32x4)(0.0f); }
-
   const float* kbase = kc + (size_t)kvh * max_seq * D + li * 4;
   const float* vbase = vc + (size_t)kvh * max_seq * D + li * 4;
   const uint32_t stride = n_splits * NW * RPW;
@@ -112,6 +112,21 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
       m[g] = mn;
     }
   };
+  for (bool first = true;; first = false) {   // MULTI: a workgroup's splits one after the other; otherwise one
+  if (MULTI) {
+    if (!first && (sp += gs) >= n_splits) break;
+    if (sp * (NW * RPW) >= kv_len) {   // a split without rows (the grid is made for every position): the merge reads no more than this of it
+      if (threadIdx.x < (uint32_t)G) {
+        float* ml = part_ml + (((size_t)kvh * n_splits + sp) * G + threadIdx.x) * 2;
+        ml[0] = kNegBig;
+        ml[1] = 0.0f;
+      }
+      continue;
+    }
+    if (!first) __syncthreads();   // the split before this one has been merged
+  }
+#pragma unroll
+  for (int g = 0; g < G; g++) { m[g] = kNegBig; l[g] = 0.0f; acc[g] = (f32x4)(0.0f); }
   // Batches of kAhead iterations: all their K/V rows are requested before the first one is used (clamped when past the
   // end, so the loads are unconditional).  At decode lengths a workgroup has 1-3 iterations and everything is in flight
   // at once; at 4K context it has ~30, and with a single iteration ahead the kernel ran at 1 TB/s (latency-bound).
@@ -174,6 +189,8 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
       part_acc[(pbase + g) * D + dim] = a;
       if (dim == 0) { part_ml[(pbase + g) * 2] = mn; part_ml[(pbase + g) * 2 + 1] = lsum; }
     }
+  }
+  if (!MULTI) break;
   }
   LGH_TL_END();
 }
@@ -456,16 +473,20 @@ hipError_t kv_roundtrip_launch(int fmt, const float* x, uint32_t n, uint8_t* byt
 template <bool MULTI>
 __global__ void __launch_bounds__(128) attn_combine_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_acc,
                                                            uint32_t g_per_kv, uint32_t head_dim, uint32_t n_splits,
-                                                           float* __restrict__ out, uint8_t* __restrict__ xq_out) {
+                                                           float* __restrict__ out, uint8_t* __restrict__ xq_out, const int* pos_ptr, uint32_t split_rows) {
   __shared__ float s_f[64];
   __shared__ float s_linv;
   LGH_TL_BEGIN(attn, lgh::TL_COMBINE, n_splits);
+  uint32_t used = n_splits;   // splits that have rows
   if (MULTI) {   // blockIdx.y = sequence: its partials, its output vector and XQ image
     const uint32_t sq = blockIdx.y, n_heads = gridDim.x;
     part_ml += (size_t)sq * n_heads * n_splits * 2;
     part_acc += (size_t)sq * n_heads * n_splits * head_dim;
     out += (size_t)sq * n_heads * head_dim;
     if (xq_out) xq_out += (size_t)sq * xq_bytes((size_t)n_heads * head_dim);
+    uint32_t pw;
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pw) : "s"(pos_ptr + sq) : "memory");
+    used = min(n_splits, pw / split_rows + 1);
   }
   const uint32_t h = blockIdx.x, kvh = h / g_per_kv, g = h % g_per_kv;
   const size_t p0 = (size_t)kvh * n_splits * g_per_kv + g;   // split s lives at p0 + s * g_per_kv
@@ -475,7 +496,7 @@ __global__ void __launch_bounds__(128) attn_combine_kernel(const float* __restri
   float pa[32];
 #pragma unroll
   for (uint32_t sidx = 0; sidx < 32; sidx++)
-    pa[sidx] = (sidx < n_splits && dim < head_dim) ? part_acc[(p0 + (size_t)sidx * g_per_kv) * head_dim + dim] : 0.0f;
+    pa[sidx] = (sidx < used && dim < head_dim) ? part_acc[(p0 + (size_t)sidx * g_per_kv) * head_dim + dim] : 0.0f;
   if (threadIdx.x < 64) {
     const uint32_t sidx = threadIdx.x;
     const bool ok = sidx < n_splits;
@@ -491,7 +512,7 @@ __global__ void __launch_bounds__(128) attn_combine_kernel(const float* __restri
   if (dim < head_dim) {
     float a = 0.0f;
 #pragma unroll
-    for (uint32_t sidx = 0; sidx < 32; sidx++) a += pa[sidx] * s_f[sidx];   // s_f of absent splits is exp(-1e30 - m) = 0
+    for (uint32_t sidx = 0; sidx < 32; sidx++) a += pa[sidx] * s_f[sidx];   // s_f of absent and empty splits is exp(-1e30 - m) = 0
     const float o = a * s_linv;
     out[(size_t)h * head_dim + dim] = o;
     if (xq_out) xq_store_chunk(xq_out, (h * head_dim + dim) >> 4, o);   // wo's input as XQ records (head_dim % 16 == 0)
@@ -924,21 +945,28 @@ hipError_t attn_combine_launch(const float* part_ml, const float* part_acc, uint
                                uint32_t head_dim, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st) {
   if (n_kv == 0 || n_heads % n_kv || head_dim % 16 || head_dim > 128 || n_splits > 32) return hipErrorInvalidValue;
   hipLaunchKernelGGL(attn_combine_kernel<false>, dim3(n_heads), dim3(head_dim > 64 ? 128 : 64), 0, st, part_ml, part_acc,
-                     n_heads / n_kv, head_dim, n_splits, out, xq_out);
+                     n_heads / n_kv, head_dim, n_splits, out, xq_out, (const int*)nullptr, 0u);
   return hipGetLastError();
 }
 
 // ---- multi-sequence decode (engine_batch.hip): the split attention and its merge for n_seq sequences in one launch each
+static uint32_t attn_multi_waves(uint32_t max_seq) { return max_seq >= 2048 ? 8 : 4; }
+// Workgroups of the launch, each walking its share of the splits.  A workgroup costs the dispatcher 4 ns whether its split has rows or not, and of 32 splits a
+// context of 60 rows fills eight: attention of 16 sequences of up to 124 rows (8B model) took 21 us with 4096 workgroups.  Long contexts want the waves, so the
+// line goes by what the cache holds (a step of 16 sequences with 512 / 1024 / 4096 workgroups: 4 layers, 20 rows 620 / 627 / 671 us; 2 layers, 1800 rows
+// 443 / 416 / 413; 4000 rows 522 / 524 / 510).
+static uint32_t attn_multi_groups(uint32_t max_seq) { return max_seq < 512 ? 512 : max_seq < 2048 ? 1024 : 2048; }
 template <int D, int G>
 static hipError_t attn_multi_go(const float* q, const float* kc, const float* vc, uint32_t n_kv, uint32_t max_seq, float scale, const int* pos,
                                 const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* part_ml, float* part_acc,
                                 hipStream_t st) {
-  if (max_seq >= 2048)
-    hipLaunchKernelGGL((attn_partial_kernel<D, G, 8, false, true>), dim3(n_kv * n_splits, n_seq), dim3(512), 0, st, q, kc, vc, max_seq, scale,
-                       pos, 0, n_splits, part_ml, part_acc, slot, slot_stride);
+  const uint32_t gs = std::min(n_splits, std::max(1u, attn_multi_groups(max_seq) / (n_kv * n_seq)));
+  if (attn_multi_waves(max_seq) == 8)
+    hipLaunchKernelGGL((attn_partial_kernel<D, G, 8, false, true>), dim3(n_kv * gs, n_seq), dim3(512), 0, st, q, kc, vc, max_seq, scale,
+                       pos, 0, n_splits, part_ml, part_acc, slot, slot_stride, gs);
   else
-    hipLaunchKernelGGL((attn_partial_kernel<D, G, 4, false, true>), dim3(n_kv * n_splits, n_seq), dim3(256), 0, st, q, kc, vc, max_seq, scale,
-                       pos, 0, n_splits, part_ml, part_acc, slot, slot_stride);
+    hipLaunchKernelGGL((attn_partial_kernel<D, G, 4, false, true>), dim3(n_kv * gs, n_seq), dim3(256), 0, st, q, kc, vc, max_seq, scale,
+                       pos, 0, n_splits, part_ml, part_acc, slot, slot_stride, gs);
   return hipGetLastError();
 }
 
@@ -956,11 +984,11 @@ hipError_t attn_multi_launch(const float* q, const float* kcache, const float* v
   return hipErrorInvalidValue;
 }
 
-hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
-                                     uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st) {
-  if (n_kv == 0 || n_heads % n_kv || head_dim % 16 || head_dim > 128 || n_splits > 32 || n_seq == 0) return hipErrorInvalidValue;
+hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq,
+                                     const int* pos, uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st) {
+  if (n_kv == 0 || n_heads % n_kv || head_dim % 16 || head_dim > 128 || n_splits > 32 || n_seq == 0 || !pos) return hipErrorInvalidValue;
   hipLaunchKernelGGL(attn_combine_kernel<true>, dim3(n_heads, n_seq), dim3(head_dim > 64 ? 128 : 64), 0, st, part_ml, part_acc,
-                     n_heads / n_kv, head_dim, n_splits, out, xq_out);
+                     n_heads / n_kv, head_dim, n_splits, out, xq_out, pos, attn_multi_waves(max_seq) * (256 / head_dim));   // (rows a split takes first)
   return hipGetLastError();
 }
 

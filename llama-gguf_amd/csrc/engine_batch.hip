@@ -241,7 +241,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
     {
       XqBuf* qa = view_of(c, Bs.attn_out);
       if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
-             return attn_combine_multi_launch(Bs.part_ml, Bs.part_acc, d.num_heads, d.num_kv_heads, d.head_dim, c->n_splits, n_seq, Bs.attn_out, qa->xq,
+             return attn_combine_multi_launch(Bs.part_ml, Bs.part_acc, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, Bs.d_pos, c->n_splits, n_seq, Bs.attn_out, qa->xq,
                                               c->stream);
            })))
         return rc;

@@ -39,3 +39,26 @@ def test_groups_of_sequences_are_bitwise_the_single_sequence(pkg, name, mix, siz
                 assert np.array_equal(got[s].view(np.uint32), want[s][step].view(np.uint32)), (n, s, step)
     multi.close()
     single.close()
+
+
+@pytest.mark.parametrize("name,max_seq", [("test-dense-d128", 640), ("test-dense-d128", 2100), ("test-dense", 500)])
+def test_splits_walked_by_one_workgroup_are_bitwise_the_single_sequence(pkg, name, max_seq):
+    """The batched attention gives a workgroup several splits, with and without rows: contexts around the rows a split takes at a time."""
+    cfg = pkg.make_config(name, max_seq_len=max_seq)
+    model = pkg.SynthModel(cfg, mix="Q4_K_M")
+    multi = pkg.HipGpuInference.from_model(model, max_seq)
+    single = pkg.HipGpuInference.from_model(model, max_seq, attn_direct=255)
+    lens = (2, 3, 7, 8, 9, 16, 17, 63, 64, 65, 127, 256, 257, 300, 449, 480)
+    multi.batch_create(16)
+    tok = np.random.default_rng(8).integers(0, cfg.vocab_size, (16, max(lens) + 2))
+    for s, n in enumerate(lens):
+        multi.batch_prefill(s, tok[s, :n])
+    got = [multi.forward_multi(list(range(16)), [int(tok[s, n + k]) for s, n in enumerate(lens)])[0] for k in range(2)]
+    for s, n in enumerate(lens):
+        single.reset()
+        single.forward_batch(tok[s, :n])
+        for k in range(2):
+            want = single.forward(int(tok[s, n + k]))
+            assert np.array_equal(got[k][s].view(np.uint32), want.view(np.uint32)), (s, k)
+    multi.close()
+    single.close()
