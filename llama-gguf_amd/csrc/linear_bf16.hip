@@ -504,17 +504,29 @@ hipError_t lin_mv_launch(int pro, const LinMv& a, hipStream_t st, int src) {
 
 // ------------------------------------------------------------------------------------------------
 // block product.  A workgroup of 4 waves computes BN weight rows x BM tokens, k in steps of 64; both operands go global -> LDS by
-// DMA (two buffers), 16-byte chunks of a row stored at chunk ^ (row & mask) so that the 16 rows of a fragment read different banks.
+// DMA (two to four buffers), 16-byte chunks of a row stored at chunk ^ (row & mask) so that the 16 rows of a fragment read different banks.
 // The weights are the A operand: a lane ends up with 4 consecutive output columns of one token.
 // ------------------------------------------------------------------------------------------------
 template <class T> constexpr uint32_t act_chunks() { return 64 * sizeof(T) / 16; }   // 16-byte chunks of a row's 64 columns
+
+// Buffers of a k-step: as many as leave two workgroups a CU, two to four.  A step's loads take about 0.9 us to arrive, its products 0.1 to 0.2, so with one step
+// requested ahead the loop was a chain of arrivals; the wait is for the step at hand only.  1501 tokens in bf16: 64 x 128 tiles (three buffers) 5632 -> 2048 columns
+// 78 -> 53 us, 2048 -> 2048 33 -> 22; 128 x 128 tiles have room for two and gain the barrier that is gone: 2048 -> 5632 61 -> 57.  One workgroup a CU with four buffers is slower
+// (128 x 128, 192 tiles, 5632 -> 2048: 59 us), and so are three and four buffers of the larger tile (the whole prompt 2650, 2970 us against 2520).
+template <class T, int BM, int BN> constexpr uint32_t lin_step_bytes() { return BN * 128 + BM * act_chunks<T>() * 16; }
+template <class T, int BM, int BN> constexpr int lin_stages() {
+  constexpr uint32_t n = 80u * 1024 / lin_step_bytes<T, BM, BN>();
+  return n < 2 ? 2 : n > 4 ? 4 : (int)n;
+}
 
 template <class T, int BM, int BN, int WN, int EPI, bool GRP>
 __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t tiles_n, uint32_t tiles_m) {
   constexpr int WM = 4 / WN, NT = BN / WN / 16, MT = BM / WM / 16;
   constexpr uint32_t XC = act_chunks<T>();
   constexpr uint32_t kWBytes = BN * 128, kXBytes = BM * XC * 16, kBuf = kWBytes + kXBytes;
+  constexpr uint32_t NS = lin_stages<T, BM, BN>();
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const uint32_t lds0 = lds_addr_of(smem);
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   // consecutive tiles of one weight panel on one XCD (workgroups go round-robin over the 8 XCDs)
   uint32_t t = blockIdx.x;
@@ -549,12 +561,12 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
     }
   }
   auto stage = [&](uint32_t k0, uint32_t buf) {
-    uint8_t* base = smem + buf * kBuf;
+    const uint32_t base = lds0 + buf * kBuf;
 #pragma unroll
     for (int i = 0; i < (int)(kWBytes / 4096); i++) {       // weights: 8 chunks a row, a wave instruction covers 8 rows
       const uint32_t row = (i * 4 + wave) * 8 + (lane >> 3), ch = (lane & 7) ^ (row & 7);
       const uint32_t n = n0 + row < a.np ? n0 + row : a.np - 1;
-      lds_dma16(W + (size_t)n * a.kp + k0 + ch * 8, base + (i * 4 + wave) * 1024);
+      lds_dma16_untracked(W + (size_t)n * a.kp + k0 + ch * 8, base + (i * 4 + wave) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NX; i++) {
@@ -562,7 +574,7 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
       if (kXBytes / 1024 % 4 == 0 || blk < kXBytes / 1024) {
         const uint32_t row = blk * RPI + lane / XC, ch = (lane % XC) ^ (row & (XC - 1));
         const uint32_t m = GRP ? xrow[GRP ? i : 0] : m0 + row < a.M ? m0 + row : a.M - 1;
-        lds_dma16(X + (size_t)m * a.ldx + k0 + ch * (16 / sizeof(T)), base + kWBytes + blk * 1024);
+        lds_dma16_untracked(X + (size_t)m * a.ldx + k0 + ch * (16 / sizeof(T)), base + kWBytes + blk * 1024);
       }
     }
   };
@@ -573,13 +585,16 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
 #pragma unroll
     for (int j = 0; j < MT; j++) acc[i][j] = (f32x4)(0.0f);
 
-  stage(0, 0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-  __syncthreads();
+  // a wave issues at least kDma loads a step; all but those of the NS - 2 steps after this one have to be there (a wave that issues one more waits for more than that)
+  constexpr uint32_t kDma = kWBytes / 4096 + kXBytes / 4096;
   const uint32_t steps = a.kp / 64;
+  for (uint32_t s = 0; s + 1 < NS && s < steps; s++) stage(s * 64, s);
+  uint32_t cur = 0, fill = NS - 1;                           // buffer of this step, and of the step NS - 1 after it
   for (uint32_t s = 0; s < steps; s++) {
-    const uint32_t cur = s & 1;
-    if (s + 1 < steps) stage((s + 1) * 64, cur ^ 1);
+    if (s + NS - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NS - 2) * kDma) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // past the barrier every wave has read the step before this one: its buffer is free
+    if (s + NS - 1 < steps) stage((s + NS - 1) * 64, fill);
     const uint8_t* wb = smem + cur * kBuf;
     const uint8_t* xb = wb + kWBytes;
     constexpr int U = 64 / Frag<T>::KU;
@@ -608,8 +623,8 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
 #pragma unroll
         for (int j = 0; j < MT; j++) acc[i][j] = Frag<T>::mma(wf[i], xf[j], acc[i][j]);
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
+    cur = cur + 1 < NS ? cur + 1 : 0;
+    fill = fill + 1 < NS ? fill + 1 : 0;
   }
   // lane: token r16 of a token tile, columns 4g .. 4g + 3 of a weight tile
 #pragma unroll
@@ -686,7 +701,7 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
 template <class T, int BM, int BN, int WN, int EPI, bool GRP = false>
 static hipError_t lin_gemm_go(const LinGemm& a, hipStream_t st) {
   static bool opted[64] = {};
-  constexpr size_t lds = 2 * (BN * 128 + (size_t)BM * act_chunks<T>() * 16);
+  constexpr size_t lds = lin_stages<T, BM, BN>() * (size_t)lin_step_bytes<T, BM, BN>();
   if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&lin_gemm_kernel<T, BM, BN, WN, EPI, GRP>), (int)lds, opted); e != hipSuccess) return e;
   const uint32_t tn = (a.n + BN - 1) / BN, tm = GRP ? a.grp.tiles : (a.M + BM - 1) / BM;
   hipLaunchKernelGGL((lin_gemm_kernel<T, BM, BN, WN, EPI, GRP>), dim3(tn * tm), dim3(256), lds, st, a, tn, tm);

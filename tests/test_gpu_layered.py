@@ -357,3 +357,18 @@ def test_trace_run_program(pkg, gpu, tmp_path):
         check(rows(0), A[[0, 5, 19]], dtype)
         check(rows(2), A[[22]], dtype)
         check(rows(3), B, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [60, 120, 190, 250, 310])
+def test_products_of_one_to_five_steps(pkg, gpu, width, dtype):
+    """The block product keeps up to three k-steps of 64 columns under way: inner sizes of one step to five, outputs on tiles of 16 to 128 tokens (a
+    vocabulary wide enough to fill the chip with the larger ones)."""
+    cfg = lc.config([lc.mem(ff=width)], width=width, vocab=15000)
+    eng, W = make(pkg, cfg, dtype)
+    toks = lc.tokens(150, cfg["vocab"])
+    want = lo.forward(cfg, W, toks)
+    for n in (9, 20, 100, 150):
+        eng.reset()
+        check(eng.eval(toks[:n], range(n)), want[:n], dtype, f"{n} tokens")
+    eng.close()
