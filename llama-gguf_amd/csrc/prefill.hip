@@ -31,6 +31,8 @@
 // read from LDS feeds 4 MFMAs (LDS at 50 % of its bandwidth), 128 f32 accumulators per lane.  K is split over
 // gridDim.y workgroups to fill the chip; the f32 partial sums [split][token][column] are added up by the row-wise
 // kernel that consumes them (together with bias, RoPE, residual, RMSNorm, SwiGLU).
+#include <type_traits>
+
 #include "device_utils.h"
 #include "mv_epilogue.h"
 #include "prefill.h"
@@ -123,21 +125,20 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
   __syncthreads();
   LGH_PF_STAMP(1);
-  for (uint32_t b = b0; b < b1; b++) {
+  auto block = [&](auto more, uint32_t b) {   // more: another block comes.  (The last one has a body without requests: re-requesting its own weights, for one body, cost 1 to 3 % of a prompt)
     const uint32_t cur = (b - b0) & 1;
     PfRaw w[kPfRT];
 #pragma unroll
     for (int r = 0; r < kPfRT; r++) w[r] = nxt[r];
+    if constexpr (more.value) {
 #if PF_EXP != 4 && PF_EXP != 6   /* experiment 4 / 6: no activation slabs after the first */
-    if (b + 1 < b1) x_dma(b + 1, cur ^ 1);
+      x_dma(b + 1, cur ^ 1);
 #endif
 #if PF_EXP != 5 && PF_EXP != 6   /* experiment 5 / 6: no weight loads after the first block's */
-    {
-      const uint32_t bn = b + 1 < b1 ? b + 1 : b;   // the last iteration re-requests its own block (unconditional loads)
 #pragma unroll
-      for (int r = 0; r < kPfRT; r++) pf_load<F>(nxt[r], wt[r] + (size_t)bn * tb, lane, n);
-    }
+      for (int r = 0; r < kPfRT; r++) pf_load<F>(nxt[r], wt[r] + (size_t)(b + 1) * tb, lane, n);
 #endif
+    }
     // The block's 32 units (MFMA step pp, half h, row tile r) as a software pipeline, one scheduling region per unit:
     // the unit's 8 MFMAs, the dequantization of the NEXT unit's A fragment, and — in the first unit of a (pp, h) phase —
     // the LDS reads of the next phase's activation fragments.  Measured on Llama-3-8B Q4_K_M (128 tokens, 4.9 ms): with
@@ -188,10 +189,15 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
       __builtin_amdgcn_sched_barrier(0);
     }
     LGH_PF_STAMP(2 + 2 * (b - b0 < 5 ? b - b0 : 5));
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-    __syncthreads();
+    if constexpr (more.value) {
+      __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+      __syncthreads();
+    }
     LGH_PF_STAMP(3 + 2 * (b - b0 < 5 ? b - b0 : 5));
-  }
+  };
+  uint32_t b = b0;
+  for (; b + 1 < b1; b++) block(std::true_type{}, b);
+  if (b < b1) block(std::false_type{}, b);
   // partial sums: lane holds, per (row tile, token tile), rows 4c .. 4c+3 of token n
   uint32_t row0 = 0;
   if (G.row_base) asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(row0) : "s"(G.row_base) : "memory");
