@@ -19,6 +19,7 @@
 // kernel this one does not (each skipped term is < 1e-8 of the output scale).
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "device_utils.h"
 #include "xq.h"
@@ -102,7 +103,7 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
       s += dpp_f<0x4E>(s);
       s += dpp_f<0x141>(s);
       s += dpp_f<0x140>(s);
-      if (LPR == 32) s += __shfl_xor(s, 16, 64);
+      if (LPR == 32) s = swap16_add(s);
       s *= scale;
       const float mn = valid ? fmaxf(m[g], s) : m[g];
       const float a = __expf(m[g] - mn);            // v_exp_f32: ~2 ulp, far inside the attention tolerance
@@ -144,22 +145,32 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
       if (base + j * stride < kv_len) step(base + j * stride, kk[j], vv[j]);   // wave-uniform
   }
 
-  // merge the RPW row slots of the wave (lanes with equal li hold the same output dims)
-#pragma unroll
-  for (int off = LPR; off < 64; off <<= 1) {
+  // merge the RPW row slots of the wave (lanes with equal li hold the same output dims): rows of 16 lanes first, then the halves
+  auto merge = [&](auto half) {
+    auto both = [&](float v, float& lo, float& hi) {
+      const auto r = half.value == 16 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)
+                                      : __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+      lo = __uint_as_float(r[0]);
+      hi = __uint_as_float(r[1]);
+    };
 #pragma unroll
     for (int g = 0; g < G; g++) {
-      const float om = __shfl_xor(m[g], off, 64), ol = __shfl_xor(l[g], off, 64);
-      f32x4 oa;
-      oa.x = __shfl_xor(acc[g].x, off, 64); oa.y = __shfl_xor(acc[g].y, off, 64);
-      oa.z = __shfl_xor(acc[g].z, off, 64); oa.w = __shfl_xor(acc[g].w, off, 64);
-      const float mn = fmaxf(m[g], om);
-      const float a = expf(m[g] - mn), b = expf(om - mn);
-      l[g] = l[g] * a + ol * b;
-      acc[g] = acc[g] * a + oa * b;
+      float m0, m1, l0, l1, a0, a1;
+      both(m[g], m0, m1);
+      both(l[g], l0, l1);
+      const float mn = fmaxf(m0, m1);
+      const float a = expf(m0 - mn), b = expf(m1 - mn);
+      l[g] = l0 * a + l1 * b;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        both(acc[g][e], a0, a1);
+        acc[g][e] = a0 * a + a1 * b;
+      }
       m[g] = mn;
     }
-  }
+  };
+  if (LPR == 16) merge(std::integral_constant<int, 16>{});
+  merge(std::integral_constant<int, 32>{});
   if (sub == 0) {
 #pragma unroll
     for (int g = 0; g < G; g++) {
