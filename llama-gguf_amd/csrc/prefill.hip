@@ -223,8 +223,7 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
 // LDS of the largest and is scheduled as one: 8 layers of an 8B model, 33 / 64 / 100 / 128 tokens 756 / 825 / 1059 / 1126 us, a kernel each 738 / 800 / 1022 / 1085.
 // (Up to 32 tokens no difference; more k-splits with two workgroups a CU there: 625 -> 684 us, the partial sums.)
 template <uint32_t MASK, int MT>
-__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+__device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem) {
   const uint32_t rgid = blockIdx.x;
   int si = 0;
   if (G.nseg > 1 && rgid >= G.seg[1].rg_begin) si = 1;
@@ -253,21 +252,31 @@ __global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) 
   else if (is(PF_Q40)) LGH_PF_RUN(PF_Q40);
 #undef LGH_PF_RUN
 }
-
+template <uint32_t MASK>
+__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) {   // blocks of more than 64 tokens
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+  pf_gemm_device<MASK, kPfMT>(G, pf_smem);
+}
 template <uint32_t MASK, int MT>
+__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_few_kernel(const PfGemm G) {   // of up to 32 / 64, and a mixture's experts
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+  pf_gemm_device<MASK, MT>(G, pf_smem);
+}
+
+template <auto* Kernel, int MT>
 static hipError_t pf_gemm_run(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
   static bool attr_set[64] = {};
   constexpr size_t lds = MT ? 2 * (size_t)MT * 16 * 512 : 2 * kPfSlabBytes;
-  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&pf_gemm_kernel<MASK, MT>), (int)lds, attr_set); e != hipSuccess) return e;
-  hipLaunchKernelGGL((pf_gemm_kernel<MASK, MT>), dim3(n_rg, G.S), dim3(kPfWaves * 64), lds, st, G);
+  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(Kernel), (int)lds, attr_set); e != hipSuccess) return e;
+  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S), dim3(kPfWaves * 64), lds, st, G);
   return hipGetLastError();
 }
 template <uint32_t MASK>
 static hipError_t pf_gemm_go(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
-  if (G.m_count) return pf_gemm_run<MASK, 0>(G, n_rg, st);
-  if (G.m_tiles <= 2) return pf_gemm_run<MASK, 2>(G, n_rg, st);
-  if (G.m_tiles <= 4) return pf_gemm_run<MASK, 4>(G, n_rg, st);
-  return pf_gemm_run<MASK, kPfMT>(G, n_rg, st);
+  if (G.m_count) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 0>, 0>(G, n_rg, st);
+  if (G.m_tiles <= 2) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 2>, 2>(G, n_rg, st);
+  if (G.m_tiles <= 4) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 4>, 4>(G, n_rg, st);
+  return pf_gemm_run<&pf_gemm_kernel<MASK>, kPfMT>(G, n_rg, st);
 }
 
 bool pf_supported_type(int dev_type) { return pf_fmt_of(dev_type) >= 0; }
