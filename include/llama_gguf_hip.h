@@ -121,7 +121,8 @@ enum {
   LGH_FLAG_REMOVED_MASK = (1u << 1) | (1u << 3) | (1u << 5) | (1u << 6) | (1u << 7) | (0xFFu << 24),
   LGH_FLAG_ATTN_SPLITS_SHIFT = 8,    /* bits 8..15: KV splits per kv-head in decode attention (0 = auto) */
   LGH_FLAG_ATTN_DIRECT_SHIFT = 16    /* bits 16..23: contexts of up to 64 * n rows use the single-launch decode attention (one workgroup
-                                        per query head, no split + combine pair); 0 = the tuned default, 255 = never */
+                                        per query head, no split + combine pair); 0 = the tuned default, 255 = never.  A TurboQuant
+                                        cache's batched steps take it where max_seq_len lies within the limit */
 };
 
 typedef struct lgh_ctx lgh_ctx;
@@ -226,8 +227,8 @@ int lgh_forward(lgh_ctx* ctx, uint32_t token_id, float* logits_out);
 int lgh_prefill_token(lgh_ctx* ctx, uint32_t token_id);
 /* GpuOnlyInference::forward_batch minus the last token (gpu_only.rs:776-790: n prefill_tokens).  Single-stage models
  * (dense or MoE) whose 2-D weights are all in matrix-core tile layouts (Q4_K, Q5_K, Q6_K, Q8_0, Q4_0 with k % 256 == 0)
- * take the batched path: blocks of up to 128 tokens, one f16-MFMA GEMM per weight (MoE: per expert, over
- * the tokens routed to it), causal attention over the block; the KV cache it leaves equals the token-by-token one within
+ * take the batched path: blocks of up to 128 tokens, of up to 2048 for prompts of 256 tokens and more
+ * (160 with experts), one f16-MFMA GEMM per weight (MoE: over the tokens routed to an expert), causal attention over the block; the KV cache it leaves equals the token-by-token one within
  * 1e-2 relative (f16 operands, f32 accumulation).  Everything else (pipeline stages, other formats), and any
  * context created with LGH_FLAG_EXACT_PREFILL, runs n exact prefill_tokens. */
 int lgh_prefill_batch(lgh_ctx* ctx, const uint32_t* tokens, size_t n);

@@ -61,12 +61,13 @@ void dev_free_tracked(lgh_ctx* c, void* p) {
   (void)hipFree(p);
 }
 
-// Contexts up to this many rows run the single-launch decode attention (attention.hip, attn_direct_kernel) unless the flags say otherwise.  Measured against
-// the split kernel with its merge, us per layer gained: 8 kv heads of 128 with 4 query heads each 4.8 / 5.1 / 3.8 / 2.4 / 1.6 / 0.2 / -0.4 at 40 / 144 / 256 /
-// 512 / 1000 / 1500 / 3000 rows (a query head's rows all pass through one CU), 4 of 64 with 8 each 6.9 / 7.2 / 7.4 / 6.3 / 5.6 / 5.6 / 4.3 at the same, 4.3 at 4000.
-// TurboQuant caches (attn_tq_direct_kernel), the same two models, 3 / 2 bits: 10.8 / 9.1 and 20.3 / 20.0 us gained at 512 rows, 9.7 / 7.6 and 19.9 / 19.3 at 8000: a row is
-// a tenth of the bytes (measured no further).
-static uint32_t direct_attn_default_kv(uint32_t head_dim, bool tq) { return tq ? 8192 : head_dim == 64 ? 4096 : 1024; }
+// Contexts up to this many rows run the single-launch decode attention (attention.hip, attn_direct_kernel; attention_tq.hip, attn_tq_direct_kernel) unless the flags say
+// otherwise: a query head's rows all pass through one CU, which pays until they take longer than the split kernel's merge and second launch.  Measured against the split kernel with
+// its merge, us per layer gained, 8 kv heads of 128 with 4 query heads each: f32 4.8 / 5.0 / 3.6 / 1.0 / -0.1 / -5.1 at 40 / 128 / 256 / 400 / 512 / 1000 rows, TurboQuant 3 bits
+// 9.7 / 8.9 / 6.8 / 3.3 / 2.8 / 0.5 / -3.5 at 40 / 256 / 512 / 1000 / 1200 / 1500 / 2000, 2 bits 8.8 / 7.6 / 5.5 / 0.9 / 0.1 / -2.8 at 40 / 256 / 512 / 1000 / 1200 / 1500;
+// 4 kv heads of 64 with 8 each: f32 7.7 / 7.9 / 6.5 / 2.8 / 1.6 / -0.9 at 40 / 256 / 512 / 1000 / 1500 / 2000, 3 bits 19.8 / 17.9 / 13.7 / 8.1 / 3.7 / -1.0 at 40 / 1000 / 2000 / 4000 /
+// 6000 / 8000, 2 bits 11.5 at 2000.
+static uint32_t direct_attn_default_kv(uint32_t head_dim, bool tq) { return tq ? (head_dim == 64 ? 4096 : 1152) : (head_dim == 64 ? 1536 : 448); }
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ------------------------------------------------------------------------------------------------
