@@ -368,6 +368,10 @@ __device__ __forceinline__ float pf_inv_rms(const float* ssq, uint32_t n_ssq, ui
   return 1.0f / __builtin_sqrtf(tot / (float)H + eps);
 }
 
+// The residual's partial sums are requested eight splits at a time and added in order: 16 tokens and 16 splits 6.5 -> 4.8 us (128 tokens 7.2 -> 7.1).  QKV's eight splits of two values
+// a thread are no faster that way (4.4 -> 4.9).
+constexpr uint32_t kPfAtOnce = 8;
+
 // Row epilogue, (2048-column chunks) x (tokens) workgroups:
 //   v[i] = sum_s part[s][t][col0 + i] (+ bias[i]) + hidden[t][i]  (the residual, layers.rs:1201-1208, 1235-1241);
 //   hidden[t][i] = v[i];  XH[t][i] = f16(v[i] * nw[i]);  ssq[t][chunk] = sum of v^2 over the chunk.
@@ -384,15 +388,25 @@ __global__ void __launch_bounds__(256) pf_resid_kernel(const float* __restrict__
     f32x4 v0 = *reinterpret_cast<const f32x4*>(hidden + (size_t)t * H + i), v1 = *reinterpret_cast<const f32x4*>(hidden + (size_t)t * H + i + 4);
     if (S) {
       f32x4 a0 = (f32x4)(0.0f), a1 = (f32x4)(0.0f);
-      for (uint32_t s = 0; s < S; s++) {
-        const float* row = part + ((size_t)s * kPfTokens + t) * ncols + col0 + i;
-        if (moe_w) {   // MoeLayer::forward (moe.rs:363-368): zero-initialised, += routing weight * expert output in selection order
-          const float w = moe_w[t * S + s];
-          a0 += *reinterpret_cast<const f32x4*>(row) * w;
-          a1 += *reinterpret_cast<const f32x4*>(row + 4) * w;
-        } else {
-          a0 += *reinterpret_cast<const f32x4*>(row);
-          a1 += *reinterpret_cast<const f32x4*>(row + 4);
+      for (uint32_t s0 = 0; s0 < S; s0 += kPfAtOnce) {
+        f32x4 r0[kPfAtOnce], r1[kPfAtOnce];
+#pragma unroll
+        for (uint32_t k = 0; k < kPfAtOnce; k++) {
+          const float* row = part + ((size_t)(s0 + k < S ? s0 + k : s0) * kPfTokens + t) * ncols + col0 + i;
+          r0[k] = *reinterpret_cast<const f32x4*>(row);
+          r1[k] = *reinterpret_cast<const f32x4*>(row + 4);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPfAtOnce; k++) {
+          if (s0 + k >= S) break;
+          if (moe_w) {   // MoeLayer::forward (moe.rs:363-368): zero-initialised, += routing weight * expert output in selection order
+            const float w = moe_w[t * S + s0 + k];
+            a0 += r0[k] * w;
+            a1 += r1[k] * w;
+          } else {
+            a0 += r0[k];
+            a1 += r1[k];
+          }
         }
       }
       if (bias) { a0 += *reinterpret_cast<const f32x4*>(bias + i); a1 += *reinterpret_cast<const f32x4*>(bias + i + 4); }
