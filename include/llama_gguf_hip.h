@@ -499,6 +499,10 @@ int lgh_op_matvec(int device, const float* a, const float* x, float* out, size_t
 int lgh_op_matvec_q(int device, uint32_t ggml_type, const void* a, const float* x, float* out, size_t m, size_t k);
 int lgh_op_attention(int device, const float* q, const float* k, const float* v, float* out, size_t n_heads, size_t n_kv_heads,
                      size_t seq_len, size_t kv_len, size_t head_dim, float scale);
+/* The attention of long prompt blocks by itself, its sums in f32 where the prompt path rounds them to f16: q / out [n_tokens][n_heads][head_dim] at positions
+ * pos0 .. pos0 + n_tokens - 1, caches [n_kv_heads][max_seq][head_dim] with their rows already in place; head_dim 64 / 128, 1 / 2 / 4 / 8 heads per kv head. */
+int lgh_op_attention_prompt(int device, const float* q, const float* k_cache, const float* v_cache, float* out, size_t n_heads, size_t n_kv_heads,
+                            size_t head_dim, size_t max_seq, float scale, size_t pos0, size_t n_tokens);
 /* Device-resident weights by tensor name for the per-op surface: `CudaBackend::load_model_weights` and the `b.name()`
  * lookups in its vec_mat / vec_mat_q (src/backend/cuda/mod.rs:121-146, 436-470, 511-575).  A weight is uploaded once
  * (native GGUF bytes; the library re-lays it out as lgh_upload_tensor does) and later calls name it. */

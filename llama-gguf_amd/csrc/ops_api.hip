@@ -377,6 +377,22 @@ int lgh_op_attention(int device, const float* q, const float* k, const float* v,
   return t.down(out, dout, n_heads * seq_len * d);
 }
 
+int lgh_op_attention_prompt(int device, const float* q, const float* kc, const float* vc, float* out, size_t n_heads, size_t n_kv, size_t d,
+                            size_t max_seq, float scale, size_t pos0, size_t n_tokens) {
+  Tmp t(device);
+  if (t.rc) return t.rc;
+  if (!q || !kc || !vc || !out || n_kv == 0 || n_heads % n_kv || n_tokens == 0 || n_tokens > kPfwTokens || pos0 + n_tokens > max_seq || max_seq > (1u << 20)) return LGH_INVALID_ARGUMENT;
+  const size_t g = n_heads / n_kv, cache = n_kv * max_seq * d;
+  if ((d != 64 && d != 128) || (g != 1 && g != 2 && g != 4 && g != 8)) return LGH_UNSUPPORTED;
+  float *dq = t.up(q, n_tokens * n_heads * d), *dk = t.up(kc, cache), *dv = t.up(vc, cache), *dout = t.up(nullptr, n_tokens * n_heads * d);
+  uint8_t* scratch = nullptr;
+  if (!dq || !dk || !dv || !dout || dev_alloc(t.c, (void**)&scratch, attn_wide_bytes((uint32_t)n_kv, (uint32_t)d, (uint32_t)(pos0 + n_tokens)))) return LGH_ALLOCATION_FAILED;
+  if (attn_wide_launch(dq, dk, dv, (uint32_t)n_heads, (uint32_t)n_kv, (uint32_t)d, (uint32_t)max_seq, scale, (uint32_t)pos0, (uint32_t)n_tokens, scratch, nullptr,
+                       t.c->stream, dout) != hipSuccess)
+    return LGH_OPERATION_FAILED;
+  return t.down(out, dout, n_tokens * n_heads * d);
+}
+
 // ---- device-resident weights by tensor name: CudaBackend::load_model_weights + the `b.name()` lookups of its vec_mat /
 // vec_mat_q (src/backend/cuda/mod.rs:121-146, 436-470, 511-575; store: cuda/dequant_weights.rs) ----
 }  // extern "C"

@@ -129,11 +129,11 @@ hipError_t embed_batch_launch(int src_type, const uint8_t* table, const int* tok
 hipError_t attn_prefill_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv,
                                uint32_t head_dim, uint32_t max_seq, float scale, uint32_t pos0, uint32_t m_tokens, uint8_t* xh_out,
                                hipStream_t st);
-// attention_wide.hip: the same for long blocks; scratch holds the layer's rows as the kernel wants them, out is row-major f16
+// attention_wide.hip: the same for long blocks; scratch holds the layer's rows as the kernel wants them, out is row-major f16 (or out32, f32)
 uint32_t attn_wide_tiles(uint32_t rows);
 size_t attn_wide_bytes(uint32_t n_kv, uint32_t head_dim, uint32_t rows);
 hipError_t attn_wide_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale,
-                            uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, uint8_t* out, hipStream_t st);
+                            uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, uint8_t* out, hipStream_t st, float* out32 = nullptr);
 // byte offset of element k of token t in an XH matrix
 __host__ __device__ inline size_t xh_offset(uint32_t t, uint32_t k) {
   const uint32_t ch = k >> 3, j = k & 7, pj = (j == 1 || j == 5) ? j + 1 : (j == 2 || j == 6) ? j - 1 : j;
