@@ -12,7 +12,7 @@
 // the sequences' records staged ONCE per workgroup in LDS and shared by its 8 waves, sequences two at a time (the pair's 8 MFMAs,
 // then the vector work while the next pair's operands load), the epilogue as a second small launch — what bounded the first
 // structure and what each change bought: profiles/r03e_batched_decode.md.  From three sequences on its products take the sequences in
-// groups of four (mvqb4) or, from five on and for weights below 8 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
+// groups of four (mvqb4) or, from five on and for weights below 6 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
 // workgroup = the 8 k-slices of a few row tiles) with a loop over the sequences inside it and their records from L2 into a
 // register ring; kept for one sequence and for launches whose segments do not share their input vector.
 // Epilogues: store, +residual, SwiGLU pair, RoPE (every sequence at its own position) and the K / V rows into the sequence's
@@ -626,11 +626,12 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
 }
 
 // ------------------------------------------------------------------------------------------------
-// The same for formats whose weights are whole numbers below 64 (all but Q8_0), on the bf16 matrix cores: what a digit needs beside its product moves into the
+// The same for formats whose weights are whole numbers below 32 (all but Q6_K and Q8_0), on the bf16 matrix cores: what a digit needs beside its product moves into the
 // operands.  mvqb4 spends eight vector instructions per (row, sequence, 16 elements): two shifts and additions of digit sums, two conversions, a fused
 // multiply-add, and the scales.  Here a digit is a bf16 number, the digit times its power of 256 times the chunk's scale, itself a power of two (both exact),
 // and the high two and the low two digits of 16 elements lie along one K of 32: the product IS the scaled high or low half, in f32.  Every partial sum is a whole
-// multiple of the scale below 2^24 of it (high digits |I| >> 16 <= 2^14, weights <= 63, 16 elements: 63 * 2^18 < 2^24), so nothing rounds in it.  What is left is one
+// multiple of the scale below 2^24 of it (16 elements, weights <= 31; high half |I| >> 16 <= 2^14: 31 * 2^18; low half, two balanced digits, up to 128 * 256 + 128: 16 * 31 * 32896 = 16 316 416),
+// so nothing rounds in it.  (Weights of six bits would reach 33 158 336 in the low half, and beyond 2^24 the matrix instruction rounds where the integer sum does not.)  What is left is one
 // addition (the halves: the rounding that the fused multiply-add of the other kernels does, shifted by a power of two) and the fused multiply-add with the weights' scale: the same
 // bits.  The sum over the minima, a chain of four fused multiply-adds, is a 16x16x4 f32 matrix instruction, which rounds as that chain does.
 //   A: row 4 m + 2 q + half of sequence m + 4 q of eight (a lane of group m gets both halves of sequences m and m + 4), K = lane group's four elements of the half's first digit, then of its second
@@ -648,7 +649,7 @@ typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
 template <uint32_t MASK, int NB, bool SEQ>
 __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
-  static_assert((MASK & (1u << F_Q80)) == 0, "weights of 8 bits do not fit the exact range");
+  static_assert((MASK & (1u << F_Q80 | 1u << F_Q6K)) == 0, "weights of more than 5 bits do not fit the exact range");
   constexpr int NG = (NB + 7) / 8;
   auto nq = [](int g) { return NB - 8 * g > 4 ? 2 : 1; };          // a last group of up to four sequences: one per lane
   const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
@@ -660,7 +661,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
   constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
   const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
   auto is = [&](int f) { return ((MASK >> f) & 1u) != 0 && (kSingle || fmt == f); };
-  const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q6K) ? fmt_tile_bytes(F_Q6K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K) : fmt_tile_bytes(F_Q40);
+  const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K) : fmt_tile_bytes(F_Q40);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
   const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
   const uint32_t pass = active ? ul / ntiles : 0, tl = active ? ul - pass * ntiles : 0;
@@ -828,8 +829,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
               acc[g][c][q] += ts.dd * s1 - ts.dmin * s2[c & 1][2 * g + q];
             } else {
 #pragma unroll
-              for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], __builtin_fmaf(is(F_Q40) ? -8.0f : -32.0f, xs[st & 1][q][pp], V[pp]), s1);
-              acc[g][c][q] = is(F_Q40) ? acc[g][c][q] + s1 : __builtin_fmaf(ts.dd, s1, acc[g][c][q]);
+              for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], __builtin_fmaf(-8.0f, xs[st & 1][q][pp], V[pp]), s1);
+              acc[g][c][q] += s1;
             }
             asm volatile("" : "+v"(acc[g][c][q]));   // here, not sunk past the later steps' products
           }
@@ -954,7 +955,8 @@ constexpr uint32_t kMvqb4MinSeq = 3;
 
 // Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers of an 8B model in Q4_K_M / Q4_0, us, groups of four against
 // groups of eight: 3 sequences 391 / 378 against 440 / 414, 4: 406 / 381 against 447 / 423; 5: 503 / 484 against 479 / 455, 8: 531 / 512 against 502 / 480,
-// 9: 648 / 624 against 581 / 564, 16: 786 / 761 against 683 / 679)
+// 9: 648 / 624 against 581 / 564, 16: 786 / 761 against 683 / 679; measured with the Q6_K matrices of Q4_K_M in groups of eight as well: in groups of four, as they are for the
+// sake of exact sums, they take a step of 16 sequences from 548 to 565)
 constexpr uint32_t kMvqb8MinSeq = 5;
 
 template <uint32_t MASK, int NB>
@@ -993,7 +995,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
-    if constexpr ((MASK & (1u << F_Q80)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
+    if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
     else if (B.n_seq < kMvqb8MinSeq) e = mvqb4_go<MASK, 4>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 8) e = mvqb8_go<MASK, 8>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 12) e = mvqb8_go<MASK, 12>(L, B, Gm, seq, groups, st);

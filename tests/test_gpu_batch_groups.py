@@ -62,3 +62,49 @@ def test_splits_walked_by_one_workgroup_are_bitwise_the_single_sequence(pkg, nam
             assert np.array_equal(got[k][s].view(np.uint32), want.view(np.uint32)), (s, k)
     multi.close()
     single.close()
+
+
+def test_sums_at_the_edge_of_their_range_are_bitwise_the_single_sequence(pkg):
+    """Six-bit weights near 63 on chunks whose low 16 bits are near their extremes and all of one sign: the sum over a chunk's low halves (16 * 63 * 32896) needs 25 bits,
+    and the large value that sets the chunk's scale meets a weight of zero, so that the sum is all there is of the product."""
+    syn = pkg.synth
+
+    class Model(pkg.SynthModel):
+        def specs(self, layers=None):
+            for s in super().specs(layers):
+                yield syn.TensorSpec(s.name, syn.F32, s.ne) if s.name == "token_embd.weight" else s
+
+    cfg = pkg.make_config("test-dense-d128", max_seq_len=8, num_layers=1)
+    model, rng = Model(cfg, mix="Q6_K"), np.random.default_rng(4)
+    k, vocab = cfg.hidden_size, cfg.vocab_size
+    x = rng.integers(32640, 32768, (vocab, k // 16, 16))
+    x[::2] = -rng.integers(32769, 32897, x[::2].shape)                 # digits -128, < 0
+    x = x.astype(np.float32) * np.float32(2.0 ** -29)
+    x[..., 3] = 1.0
+    model._cache["token_embd.weight"] = x.reshape(-1).view(np.uint8)
+    model._cache["blk.0.attn_norm.weight"] = np.ones(k, dtype=np.float32).view(np.uint8)
+    for name, n in (("attn_q", cfg.num_heads * cfg.head_dim), ("attn_k", cfg.num_kv_heads * cfg.head_dim), ("attn_v", cfg.num_kv_heads * cfg.head_dim)):
+        q = rng.integers(56, 64, (n * k // 256, 256))
+        q[:, 3::16] = 0
+        ql, qh = np.zeros((len(q), 128), np.uint8), np.zeros((len(q), 64), np.uint8)
+        for half in range(2):                                          # block_q6_K: 128 values a half, four stripes of 32
+            for stripe in range(4):
+                v = q[:, half * 128 + stripe * 32:half * 128 + stripe * 32 + 32]
+                ql[:, half * 64 + stripe % 2 * 32:half * 64 + stripe % 2 * 32 + 32] |= ((v & 15) << (4 * (stripe // 2))).astype(np.uint8)
+                qh[:, half * 32:half * 32 + 32] |= ((v >> 4) << (2 * stripe)).astype(np.uint8)
+        sc = rng.integers(1, 64, (len(q), 16)).astype(np.int8).view(np.uint8)
+        d = np.full((len(q), 1), 0.01, np.float16).view(np.uint8)
+        model._cache[f"blk.0.{name}.weight"] = np.concatenate([ql, qh, sc, d], axis=1).reshape(-1)
+    multi = pkg.HipGpuInference.from_model(model, 8)
+    single = pkg.HipGpuInference.from_model(model, 8, attn_direct=255)
+    multi.batch_create(16)
+    for n in (2, 4, 5, 9, 16):
+        for s in range(16):
+            multi.batch_reset(s)
+        tok = rng.integers(0, vocab, 16)
+        got, _ = multi.forward_multi(list(range(n)), tok[:n])
+        for s in range(n):
+            single.reset()
+            assert np.array_equal(got[s].view(np.uint32), single.forward(int(tok[s])).view(np.uint32)), (n, s)
+    multi.close()
+    single.close()
