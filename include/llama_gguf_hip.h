@@ -401,6 +401,8 @@ int lgh_synchronize(lgh_ctx* ctx);
 
 /* debug tap: copy the hidden state (f32[hidden_size]) of the last processed token to host */
 int lgh_read_hidden(lgh_ctx* ctx, float* out);
+/* debug: the nth device allocation of this context from now on fails as if the memory were gone, the ones after it succeed (0: none fails) */
+int lgh_debug_fail_alloc(lgh_ctx* ctx, uint32_t nth);
 
 /* ---- pipeline stages over xGMI (replaces ShardServer::forward, src/distributed/shard.rs:377-445) ----
  * The hop between stages is one f32[hidden_size] vector; the host side moves it with RCCL

@@ -51,7 +51,8 @@ struct PfScratch {
 struct PfwScratch {
   uint32_t cap = 0;                    // 0: not allocated
   uint8_t *x = nullptr, *attn = nullptr, *act = nullptr;   // row-major f16: [cap][hidden], [cap][QD], [rows][ffn]
-  uint8_t* kv_split = nullptr;         // a layer's cache rows for attention_wide.hip
+  uint8_t* kv_split = nullptr;         // a layer's cache rows for attention_wide.hip: kv_bytes, enough for the longest position so far
+  size_t kv_bytes = 0;
   float *hidden = nullptr, *q = nullptr, *part = nullptr, *inv_rms = nullptr, *moe_w = nullptr, *moe_roww = nullptr;
   size_t part_bytes = 0;
   int *tokens = nullptr, *moe_sel = nullptr, *moe_seg = nullptr, *moe_tile = nullptr, *moe_slot = nullptr, *moe_src = nullptr;
@@ -118,6 +119,7 @@ struct lgh_ctx {
   bool finalized = false;
   bool profiling = false;
   std::string err;
+  uint32_t fail_alloc = 0;                         // lgh_debug_fail_alloc
   hipGraphExec_t graph[lgh::MODE_COUNT][2] = {};   // [mode][attention variant: 0 split + combine, 1 single launch (short context)]
   bool attn_direct = false;                        // variant of the token being enqueued (chosen by the host-side position)
   uint32_t direct_attn_max_kv = 0;                 // contexts up to this many rows take the single-launch attention

@@ -49,6 +49,7 @@ int fail(lgh_ctx* c, int status, const std::string& msg) {
 
 int dev_alloc(lgh_ctx* c, void** p, size_t bytes) {
   if (bytes == 0) bytes = 4;
+  if (c->fail_alloc && --c->fail_alloc == 0) return fail(c, LGH_ALLOCATION_FAILED, "device allocation (lgh_debug_fail_alloc)");
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipSuccess) return fail(c, LGH_ALLOCATION_FAILED, std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
   c->allocs.push_back(*p);
@@ -973,40 +974,63 @@ static bool pfw_eligible(const lgh_ctx* c) {
   return true;
 }
 
-static int pfw_ensure(lgh_ctx* c) {
+// The long path's buffers, for `rows` cached rows in sight.  False: the memory is not there, and no part of a set is held (the blocks of 128 do without it)
+static bool pfw_ensure(lgh_ctx* c, size_t rows) {
   PfwScratch& P = c->pfw;
-  if (P.cap) return LGH_OK;
   const lgh_model_desc& d = c->d;
-  const uint32_t H = d.hidden_size, QD = d.num_heads * d.head_dim, KD = d.num_kv_heads * d.head_dim;
-  const uint32_t cap = std::min<uint32_t>(kPfwTokens, (d.max_seq_len + kPfwTile - 1) / kPfwTile * kPfwTile);
-  bool any_moe = false;
-  size_t act = 0;
-  for (uint32_t i = c->l0; i < c->l1; i++) {
-    const LayerW& L = c->layers[i];
-    any_moe |= L.moe();
-    act = std::max(act, L.moe() ? (size_t)cap * d.num_experts_per_token * L.gate_exps.n : (size_t)cap * L.gate.n);
-  }
-  const uint32_t top = any_moe ? d.num_experts_per_token : 1, pairs = any_moe ? cap * top : 0;
-  const uint32_t tiles = any_moe ? moe_max_tiles(pairs, d.num_experts, kPfwTile) : 0;
-  const size_t pb = std::max(pfw_part_bytes(cap, QD + 2 * KD), pfw_part_bytes(cap * top, H));
-  struct { void** p; size_t n; } bufs[] = {
-      {(void**)&P.x, (size_t)cap * H * 2},      {(void**)&P.attn, (size_t)cap * QD * 2},   {(void**)&P.act, act * 2},
-      {(void**)&P.hidden, (size_t)cap * H * 4}, {(void**)&P.q, (size_t)cap * QD * 4},      {(void**)&P.part, pb},
-      {(void**)&P.inv_rms, (size_t)cap * 4},    {(void**)&P.tokens, (size_t)cap * 4},
-      {(void**)&P.kv_split, attn_wide_bytes(d.num_kv_heads, d.head_dim, d.max_seq_len)},
-      {(void**)&P.moe_sel, (size_t)pairs * 4},  {(void**)&P.moe_w, (size_t)pairs * 4},     {(void**)&P.moe_roww, (size_t)pairs * 4},
-      {(void**)&P.moe_slot, (size_t)pairs * 4}, {(void**)&P.moe_src, (size_t)pairs * 4},   {(void**)&P.moe_tile, (size_t)tiles * 8},
-      {(void**)&P.moe_seg, any_moe ? (size_t)(d.num_experts + 1) * 4 : 0},
+  const std::string err = c->err;
+  auto alloc = [&](void** p, size_t n) {
+    if (dev_alloc(c, p, n) == LGH_OK) { c->stats.scratch_bytes += n; return true; }
+    *p = nullptr;
+    (void)hipGetLastError();   // (the next launch's check would find it)
+    c->err = err;              // the call goes on without
+    return false;
   };
-  for (auto& b : bufs) {
-    if (!b.n) continue;
-    if (int rc = dev_alloc(c, b.p, b.n)) return rc;
-    c->stats.scratch_bytes += b.n;
+  if (!P.cap) {
+    const uint32_t H = d.hidden_size, QD = d.num_heads * d.head_dim, KD = d.num_kv_heads * d.head_dim;
+    const uint32_t cap = std::min<uint32_t>(kPfwTokens, (d.max_seq_len + kPfwTile - 1) / kPfwTile * kPfwTile);
+    bool any_moe = false;
+    size_t act = 0;
+    for (uint32_t i = c->l0; i < c->l1; i++) {
+      const LayerW& L = c->layers[i];
+      any_moe |= L.moe();
+      act = std::max(act, L.moe() ? (size_t)cap * d.num_experts_per_token * L.gate_exps.n : (size_t)cap * L.gate.n);
+    }
+    const uint32_t top = any_moe ? d.num_experts_per_token : 1, pairs = any_moe ? cap * top : 0;
+    const uint32_t tiles = any_moe ? moe_max_tiles(pairs, d.num_experts, kPfwTile) : 0;
+    const size_t pb = std::max(pfw_part_bytes(cap, QD + 2 * KD), pfw_part_bytes(cap * top, H));
+    struct { void** p; size_t n; } bufs[] = {
+        {(void**)&P.x, (size_t)cap * H * 2},      {(void**)&P.attn, (size_t)cap * QD * 2},   {(void**)&P.act, act * 2},
+        {(void**)&P.hidden, (size_t)cap * H * 4}, {(void**)&P.q, (size_t)cap * QD * 4},      {(void**)&P.part, pb},
+        {(void**)&P.inv_rms, (size_t)cap * 4},    {(void**)&P.tokens, (size_t)cap * 4},
+        {(void**)&P.moe_sel, (size_t)pairs * 4},  {(void**)&P.moe_w, (size_t)pairs * 4},     {(void**)&P.moe_roww, (size_t)pairs * 4},
+        {(void**)&P.moe_slot, (size_t)pairs * 4}, {(void**)&P.moe_src, (size_t)pairs * 4},   {(void**)&P.moe_tile, (size_t)tiles * 8},
+        {(void**)&P.moe_seg, any_moe ? (size_t)(d.num_experts + 1) * 4 : 0},
+    };
+    for (auto& b : bufs) {
+      if (!b.n || alloc(b.p, b.n)) continue;
+      for (auto* f = bufs; f != &b; f++)
+        if (f->n) {
+          dev_free_tracked(c, *f->p);
+          *f->p = nullptr;
+          c->stats.scratch_bytes -= f->n;
+        }
+      return false;
+    }
+    P.part_bytes = pb;
+    P.moe_tiles = tiles;
+    P.cap = cap;
   }
-  P.part_bytes = pb;
-  P.moe_tiles = tiles;
-  P.cap = cap;
-  return LGH_OK;
+  // (a layer's cache once more and half as much: for the rows in use, in steps of 4096)
+  const size_t need = attn_wide_bytes(d.num_kv_heads, d.head_dim, (uint32_t)std::min<size_t>((rows + 4095) / 4096 * 4096, d.max_seq_len));
+  if (P.kv_bytes < need) {
+    if (P.kv_split) dev_free_tracked(c, P.kv_split);   // (waits for what still reads it)
+    c->stats.scratch_bytes -= P.kv_bytes;
+    P.kv_bytes = 0;
+    if (!alloc((void**)&P.kv_split, need)) return false;
+    P.kv_bytes = need;
+  }
+  return true;
 }
 
 // m prompt tokens at positions pos .. pos + m - 1 through every layer of a single-stage context: its K / V rows
@@ -1103,8 +1127,7 @@ static int prefill_tokens(lgh_ctx* c, const uint32_t* tokens, size_t n) {
   int rc;
   size_t i = 0;
   const size_t least = pfw_min_tokens(c);
-  if (n >= least && pfw_eligible(c)) {
-    if ((rc = pfw_ensure(c))) return rc;
+  if (n >= least && pfw_eligible(c) && pfw_ensure(c, c->pos + n)) {
     while (n - i >= least) {
       const uint32_t m = (uint32_t)std::min<size_t>(c->pfw.cap, n - i);
       if ((rc = prefill_wide(c, tokens + i, m))) return rc;
@@ -1836,6 +1859,12 @@ int lgh_synchronize(lgh_ctx* c) {
   if (!c) return LGH_INVALID_ARGUMENT;
   if (bind(c)) return LGH_NOT_AVAILABLE;
   HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
+  return LGH_OK;
+}
+
+int lgh_debug_fail_alloc(lgh_ctx* c, uint32_t nth) {
+  if (!c) return LGH_INVALID_ARGUMENT;
+  c->fail_alloc = nth;
   return LGH_OK;
 }
 

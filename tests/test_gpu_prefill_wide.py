@@ -62,3 +62,50 @@ def test_long_prompts_continue_a_sequence_and_fill_slots(pkg):
     assert wide.position() == 459    # the context's own sequence is where it was
     exact.close()
     wide.close()
+
+
+def test_long_prompts_without_their_own_memory_take_the_short_blocks(pkg):
+    """An allocation that fails, whichever it is, is not left half made and costs speed alone; with the memory back the long path is taken.  Its copy of a layer's cache
+    follows the positions in use, not the context's capacity."""
+    cfg = pkg.make_config("test-dense", max_seq_len=65536)
+    model = pkg.SynthModel(cfg, mix="Q4_K_M")
+    eng, whole, short = (pkg.HipGpuInference.from_model(model, 65536) for _ in range(3))
+    prompt = [(7 * i + 3) % cfg.vocab_size for i in range(300)]
+    for at in range(0, 300, 100):
+        short.forward_batch(prompt[at:at + 100])             # blocks of 100 tokens
+    want = short.forward(9)
+    for e in (eng, whole):
+        e.forward_batch(prompt[:100])
+    before = eng.stats()["scratch_bytes"]
+    whole.forward_batch(prompt)
+    full = whole.stats()["scratch_bytes"]
+    copy = cfg.num_kv_heads * 4096 * cfg.head_dim * 2 * 6     # K and V of 4096 rows in three numbers of two bytes
+    assert before + copy < full
+    for nth in range(1, 40):
+        eng.reset()
+        eng.debug_fail_alloc(nth)
+        eng.forward_batch(prompt)
+        assert eng.position() == 300
+        got = eng.forward(9)
+        assert np.abs(got - want).max() <= 1e-2 * float(np.abs(want).max()) + 1e-2, nth
+        held = eng.stats()["scratch_bytes"]
+        if held == full:
+            break
+        assert held in (before, full - copy), nth              # (the copy comes last; the others wait for it)
+    assert nth > 3 and held == full
+    eng.debug_fail_alloc(0)
+    eng.forward_batch(prompt)                                 # 301 .. 600: grows nothing
+    assert eng.stats()["scratch_bytes"] == full
+    tail = [(5 * i) % cfg.vocab_size for i in range(4000)]
+    eng.debug_fail_alloc(1)
+    eng.forward_batch(tail)                                   # behind position 4096: no room
+    assert eng.stats()["scratch_bytes"] == full - copy
+    eng.forward_batch(tail)                                   # 4601 .. 8600: rows of 12288
+    assert eng.stats()["scratch_bytes"] == full + 2 * copy and eng.position() == 301 + 300 + 8000
+    exact = pkg.HipGpuInference.from_model(model, 65536, flags=pkg.hip_backend.FLAG_EXACT_PREFILL)
+    exact.forward_batch(prompt)
+    eng.reset()
+    eng.forward_batch(prompt)
+    _follow(exact, eng, (5, 77))
+    for e in (eng, whole, short, exact):
+        e.close()
