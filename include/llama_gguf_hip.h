@@ -121,8 +121,9 @@ enum {
   LGH_FLAG_REMOVED_MASK = (1u << 1) | (1u << 3) | (1u << 5) | (1u << 6) | (1u << 7) | (0xFFu << 24),
   LGH_FLAG_ATTN_SPLITS_SHIFT = 8,    /* bits 8..15: KV splits per kv-head in decode attention (0 = auto) */
   LGH_FLAG_ATTN_DIRECT_SHIFT = 16    /* bits 16..23: contexts of up to 64 * n rows use the single-launch decode attention (one workgroup
-                                        per query head, no split + combine pair); 0 = the tuned default, 255 = never.  A TurboQuant
-                                        cache's batched steps take it where max_seq_len lies within the limit */
+                                        per query head, no split + combine pair); 0 = the tuned default, 255 = never.  A context with slots
+                                        (lgh_batch_create) takes it where max_seq_len lies within the limit of a TurboQuant cache, and
+                                        never over an f32 cache */
 };
 
 typedef struct lgh_ctx lgh_ctx;
@@ -368,7 +369,9 @@ int lgh_read_layers(lgh_ctx* ctx, float* out, size_t n_floats);
  * iteration of its loop calls model.forward for each active sequence in turn (236-290 -> step_sequence 355-400): B sequences read
  * the weights B times.  Here a finalized single-stage context owns `max_batch` <= 16 SLOTS (a slot = one sequence's f32 KV caches
  * + position), and one step feeds one token to each listed slot while reading every weight tile ONCE.  Every sequence's
- * logits are bit-identical to what lgh_forward returns for the same token history (same arithmetic, same summation orders).
+ * logits are bit-identical to what lgh_forward of the same context returns for the same token history (same arithmetic, same summation
+ * orders); a context without slots equals them bit for bit where LGH_FLAG_ATTN_DIRECT_SHIFT keeps it from the single-launch attention
+ * (255; over a TurboQuant cache also where max_seq_len lies within the limit), to f32 rounding otherwise.
  * Dense and MoE models whose matrices are in the matrix-core tile layouts (Q4_K / Q5_K / Q6_K / Q8_0 / Q4_0, k % 256 == 0);
  * anything else answers LGH_UNSUPPORTED.  The slots' caches have the context's kv_cache_type: f32, or the TurboQuant formats
  * (LGH_KV_TQ2 / TQ3 / TQ2_QJL / TQ3_QJL: per slot the packed code rows (+ QJL rows); the reference's BatchedEngine itself only

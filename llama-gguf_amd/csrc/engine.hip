@@ -748,12 +748,19 @@ static int ensure_graph(lgh_ctx* c, int mode) {
   return LGH_OK;
 }
 
+// Rows up to which this token's attention is the single-launch one.  A context with slots takes the batched step's form for its own sequence too, so that a request has
+// the same bits served alone and in a batch: split and merge over an f32 cache, over codes what the context's capacity says (engine_batch.hip).
+static uint32_t direct_attn_rows(const lgh_ctx* c) {
+  if (!c->batch.ready) return c->direct_attn_max_kv;
+  return kv_is_tq(c->d.kv_cache_type) && c->d.max_seq_len <= c->direct_attn_max_kv ? c->direct_attn_max_kv : 0;
+}
+
 // run one token in `mode` (token id already in the device state)
 static int step(lgh_ctx* c, int mode) {
   if (c->pos >= c->d.max_seq_len)  // the reference has no such check: OOB write past the KV capacity
     return fail(c, LGH_INVALID_ARGUMENT, "position " + std::to_string(c->pos) + " >= max_seq_len " + std::to_string(c->d.max_seq_len));
   int rc;
-  c->attn_direct = c->pos + 1 <= c->direct_attn_max_kv;   // the token at position pos attends to pos + 1 rows
+  c->attn_direct = c->pos + 1 <= direct_attn_rows(c);   // the token at position pos attends to pos + 1 rows
   if (c->profiling || (c->d.flags & LGH_FLAG_NO_GRAPH)) {
     if ((rc = enqueue_token(c, mode))) return rc;
     if (c->profiling && (rc = drain_prof(c))) return rc;

@@ -9,8 +9,8 @@
 // TurboQuant slots); MoE layers route every sequence to its own experts: from 3 sequences on (moe_group_min) the step's (sequence,
 // slot) pairs are grouped by expert and each selected expert is read once — all experts of a layer in one gate | up and one down
 // launch, the expert as the grid's third dimension — below that the FFN runs sequence by sequence.  Every sequence's logits are
-// bit-identical to what the single-sequence engine computes for the same tokens (tests/test_gpu_batch.py): same kernels'
-// arithmetic, same summation orders.
+// bit-identical to what lgh_forward of the same context computes for the same tokens (tests/test_gpu_batch.py, test_gpu_batch_same_context.py): same
+// kernels' arithmetic, same summation orders.  (A context without slots may take the single-launch attention, another order of sums.)
 //
 // A step is a constant hipGraph per n_seq: tokens, positions and slot numbers live in device words (d_tokens / d_pos /
 // d_slot), the arg-max feeds the next token back on the device and `batch_advance` moves the positions, so
@@ -210,7 +210,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       const float* signs = c->tq_signs + (size_t)(li - c->l0) * d.num_kv_heads * 2 * d.head_dim;
       const float* qjl_s = qjl ? c->tq_qjl + (size_t)(li - c->l0) * d.num_kv_heads * d.head_dim * d.head_dim : nullptr;
       XqBuf* qa = view_of(c, Bs.attn_out);
-      if (!qjl && d.max_seq_len <= c->direct_attn_max_kv) {   // every context takes the single-launch form, as the single-sequence engine's do (the same bits)
+      if (!qjl && d.max_seq_len <= c->direct_attn_max_kv) {   // by capacity: one graph for every position (engine.hip, direct_attn_rows: the context's own sequence goes by it too)
         if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
                return attn_tq_direct_launch(bits, Bs.q, Bs.kq[li], Bs.vq[li], Bs.kv_tmp, Bs.kv_tmp + KD, signs, d.num_heads, d.num_kv_heads, d.head_dim,
                                             d.max_seq_len, scale, Bs.d_pos, Bs.attn_out, qa->xq, c->stream, n_seq, Bs.d_slot, Bs.code_stride, 2 * KD,
