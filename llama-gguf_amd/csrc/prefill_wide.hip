@@ -303,13 +303,16 @@ __global__ void __launch_bounds__(kWWaves * 64) pw_gemm_kernel(const PfWide G, u
     t = xcd * q + (xcd < r ? xcd : r) + i;
   }
   const uint32_t tm = tm0 + t % wide, ks = t / wide % G.S, rgid = t / (wide * G.S);
-  uint32_t m0 = tm * kPfwTile, m_end = G.m, expert = 0;
-  if (GRP) {
+  uint32_t m0, m_end, expert = 0;
+  if constexpr (GRP) {
     const int e = G.tile_e[tm];
     if (e < 0) return;
     expert = (uint32_t)e;
     m0 = (uint32_t)G.tile_row[tm];
     m_end = (uint32_t)G.row_seg[e + 1];
+  } else {   // (G.m as a value the branch above replaces ended up in scratch, to be read through a flat address)
+    m0 = tm * kPfwTile;
+    m_end = G.m;
   }
   if (m_end - m0 > (uint32_t)kPfwTile) m_end = m0 + kPfwTile;
   int si = 0;

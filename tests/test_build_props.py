@@ -3,6 +3,7 @@
 A kernel that touches scratch memory pays for the scratch setup at every launch: measured -3.5 % end to end when a
 struct was passed to the epilogue by pointer, and again when a per-pass array was indexed by the pass number.  The
 compiler reports it; this keeps it at zero for every kernel on the decode path."""
+import functools
 import os
 import re
 import subprocess
@@ -15,6 +16,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
          "-Rpass-analysis=kernel-resource-usage", "--cuda-device-only", "-c"]
 
 
+@functools.cache
 def _usage(src):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     out = subprocess.run([hipcc, *FLAGS, os.path.join(CSRC, src), "-o", os.devnull], capture_output=True, text=True, check=True).stderr
@@ -54,5 +56,26 @@ def test_prefill_gemm_keeps_its_accumulators_in_registers():
     usage = _usage("prefill.hip")
     gemm = {fn: u for fn, u in usage.items() if "pf_gemm_kernel" in fn}
     assert len(gemm) == 8   # five formats, the Q4_K/Q6_K and Q5_K/Q6_K mixes, and the any-mix instantiation
+    for fn, u in gemm.items():
+        assert u.get("AGPRs", 0) >= 128 and u["VGPRs"] <= 256, (fn, u)
+
+
+def test_long_prompt_kernels_use_no_scratch_and_keep_their_sums_in_registers():
+    """prefill_wide.hip: 256 f32 accumulators per lane, one wave per SIMD; attention_wide.hip: two waves per SIMD."""
+    for src in ("prefill_wide.hip", "attention_wide.hip"):
+        usage = _usage(src)
+        assert usage, f"no kernels found in {src}"
+        for fn, u in usage.items():
+            assert u.get("ScratchSize", 0) == 0 and u.get("VGPRs Spill", 0) == 0, f"{src}: {fn}: {u}"
+            if "pw_gemm_kernel" in fn:
+                assert u.get("AGPRs", 0) >= 256 and u["VGPRs"] <= 256, (fn, u)
+            if "attn_wide_kernel" in fn:
+                assert u["VGPRs"] + u.get("AGPRs", 0) <= 256 and u.get("Occupancy", 2) >= 2, (fn, u)
+
+
+def test_prefill_gemm_of_a_mixtures_experts_keeps_its_accumulators_in_registers():
+    """The experts' kernels (pf_gemm_few_kernel<..., 0>) choose the number of token tiles on the device: up to the 128 accumulators of a full block."""
+    gemm = {fn: u for fn, u in _usage("prefill.hip").items() if "pf_gemm_few_kernel" in fn and "ELi0E" in fn}
+    assert len(gemm) == 8
     for fn, u in gemm.items():
         assert u.get("AGPRs", 0) >= 128 and u["VGPRs"] <= 256, (fn, u)
