@@ -10,6 +10,8 @@
 // Measured: 2047 tokens, 32 query heads on 8 of 128 dims: 523 us a layer with the f32 kernel, 209 + 11 us for the rows here, bound by the matrix products.  (Two f16 limbs
 // under an exponent per tile take 139 + 8: they lose what lies far below its tile's largest value, whole weights where a tile's values do.)  Error against 64 bits, 2-norm, random
 // inputs of 129 to 1000 rows: 2.3e-7 to 4.8e-7; an emulation of the f32 kernel's order of sums 4.5e-7 to 7.2e-7 on the same inputs.
+#include <algorithm>
+
 #include "device_utils.h"
 #include "prefill.h"
 
@@ -90,11 +92,13 @@ __global__ void __launch_bounds__(256) attn_wide_split_kernel(const float* __res
 // A workgroup: one kv head, up to four of its query heads, 128 (token, head) rows: a wave has two tiles of 16 tokens of one head.  S^T = K Q^T leaves a
 // lane with the scores of one token and eight of a tile's rows, which is the operand of O^T += V^T P^T: weights never leave their registers.  K and V of a tile of
 // 32 rows arrive by DMA in turn, through a ring of three buffers, each requested while the one two before it is used up.  Two workgroups share a CU (72 KB of LDS each at 128 dims).
-// F32: sums to out32, unrounded.
-template <int D, bool F32>
+// Few tokens behind many rows leave the chip idle: grid y = splits of the tiles, each leaving its sums, maximum and weight of every (token, head) to attn_wide_merge_kernel.
+// OUT: f16 rows to out, f32 rows to part (unrounded sums), or a split's parts to part and ml.
+enum : int { AW_F16 = 0, AW_F32 = 1, AW_PART = 2 };
+template <int D, int OUT>
 __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restrict__ q, const uint8_t* __restrict__ kv, uint32_t n_heads, uint32_t g, uint32_t tiles,
                                                            float scale, uint32_t pos0, uint32_t m_tokens, uint32_t n_blk, uint32_t paired, uint8_t* __restrict__ out,
-                                                           float* __restrict__ out32) {
+                                                           float* __restrict__ part, float* __restrict__ ml) {
   constexpr int KK = D / 32, DT = D / 16;
   constexpr uint32_t LIMB = aw_limb<D>(), HALF = aw_half<D>(), OPS = HALF / 4096;   // DMA operations of a wave per half tile
   extern __shared__ __attribute__((aligned(16))) uint8_t aw_lds[];
@@ -105,7 +109,8 @@ __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restri
   const uint32_t blk = paired && idx >= n_blk / 2 ? idx - n_blk / 2 : n_blk - 1 - idx;
   const uint32_t head = hw * gw + wave % gw, kvh = head / g;
   const uint32_t tok0 = blk * (128 / gw) + wave / gw * 32;                // the wave's first token
-  const uint32_t last_blk = min(blk * (128 / gw) + 128 / gw, m_tokens) - 1, n_half = ((pos0 + last_blk) / kAwRows + 1) * 2;
+  const uint32_t last_blk = min(blk * (128 / gw) + 128 / gw, m_tokens) - 1, n_tiles = (pos0 + last_blk) / kAwRows + 1;
+  const uint32_t sp = blockIdx.y, first = n_tiles * sp / gridDim.y * 2, last = n_tiles * (sp + 1) / gridDim.y * 2;   // its half tiles (no split is empty: attn_wide_splits)
   const uint32_t last_wave = min(tok0 + 31, m_tokens - 1);
   const uint8_t* src = kv + (size_t)kvh * tiles * aw_tile<D>() + lane * 16;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)aw_lds;
@@ -130,8 +135,8 @@ __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restri
       ql[t][k] = aw_split8(v);
     }
   }
-  dma(0, 0);
-  dma(1, 1);
+  dma(first, 0);
+  dma(first + 1, 1);
   const float f = scale * 1.44269504088896f;                              // scores in units of log2
   f32x4 acc[DT][2];
   float m_run[2] = {kAwNeg, kAwNeg}, l_run[2] = {0.0f, 0.0f};
@@ -140,15 +145,15 @@ __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restri
 
   // half tile h is there (its wave's operations; only those of the next one may be under way), every wave is done with the one before: its buffer takes the one after the next
   auto arrive = [&](uint32_t h, uint32_t free_buf) {
-    if (h + 1 < n_half) __builtin_amdgcn_s_waitcnt(0x0070 | OPS);         // vmcnt(OPS) lgkmcnt(0)
+    if (h + 1 < last) __builtin_amdgcn_s_waitcnt(0x0070 | OPS);         // vmcnt(OPS) lgkmcnt(0)
     else __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (h + 2 < n_half) dma(h + 2, free_buf);
+    if (h + 2 < last) dma(h + 2, free_buf);
   };
   const uint32_t k_off = n * D * 2, v_off = n * 64 + ((c ^ (n >> 1 & 3)) << 4);
   uint32_t kb = 0, vb = 1, fb = 2;                                        // buffers of this tile's K and V, and the third
-  for (uint32_t h = 0; h < n_half; h += 2) {
+  for (uint32_t h = first; h < last; h += 2) {
     const uint32_t kv0 = h / 2 * kAwRows;
     const bool seen = kv0 <= pos0 + last_wave;                            // something of the tile is visible to this wave
     arrive(h, fb);
@@ -223,15 +228,16 @@ __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restri
     float l = l_run[t];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    const float inv = 1.0f / l;
     const uint32_t tok = tok0 + t * 16 + n;
     if (tok >= m_tokens) continue;
-    const size_t at = ((size_t)tok * n_heads + head) * D + c * 4;
+    const size_t row = ((size_t)(OUT == AW_PART ? sp * m_tokens : 0) + tok) * n_heads + head, at = row * D + c * 4;
+    const float inv = OUT == AW_PART ? 1.0f : 1.0f / l;
+    if (OUT == AW_PART && c == 0) { ml[row * 2] = m_run[t]; ml[row * 2 + 1] = l; }
 #pragma unroll
     for (int x = 0; x < DT; x++) {                                         // dims 16 x + 4c .. + 3; f16: in the chunk's element order
       const f32x4 v = acc[x][t] * inv;
-      if constexpr (F32) {
-        *reinterpret_cast<f32x4*>(out32 + at + x * 16) = v;
+      if constexpr (OUT != AW_F16) {
+        *reinterpret_cast<f32x4*>(part + at + x * 16) = v;
       } else {
         const h16x4 w = {(_Float16)v.x, (_Float16)v.z, (_Float16)v.y, (_Float16)v.w};
         *reinterpret_cast<h16x4*>(out + (at + x * 16) * 2) = w;
@@ -240,35 +246,81 @@ __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restri
   }
 }
 
+// splits of a (token, head) -> its row.  A split that the token sees nothing of has the maximum kAwNeg: its parts count for nothing.
+template <int D>
+__global__ void __launch_bounds__(256) attn_wide_merge_kernel(const float* __restrict__ part, const float* __restrict__ ml, uint32_t n_rows, uint32_t n_splits,
+                                                              uint8_t* __restrict__ out, float* __restrict__ out32) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x, row = i / (D / 4), q = i % (D / 4);
+  if (row >= n_rows) return;
+  float mn = kAwNeg, l = 0.0f;
+  for (uint32_t s = 0; s < n_splits; s++) mn = fmaxf(mn, ml[((size_t)s * n_rows + row) * 2]);
+  f32x4 v = (f32x4)(0.0f);
+  for (uint32_t s = 0; s < n_splits; s++) {
+    const size_t r = (size_t)s * n_rows + row;
+    const float f = __builtin_amdgcn_exp2f(ml[r * 2] - mn);
+    l += ml[r * 2 + 1] * f;
+    v += *reinterpret_cast<const f32x4*>(part + r * D + q * 4) * f;
+  }
+  v *= 1.0f / l;
+  if (out32) {
+    *reinterpret_cast<f32x4*>(out32 + (size_t)row * D + q * 4) = v;
+  } else {
+    const h16x4 w = {(_Float16)v.x, (_Float16)v.z, (_Float16)v.y, (_Float16)v.w};
+    *reinterpret_cast<h16x4*>(out + ((size_t)row * D + q * 4) * 2) = w;
+  }
+}
+
 uint32_t attn_wide_tiles(uint32_t rows) { return (rows + kAwRows - 1) / kAwRows; }
 size_t attn_wide_bytes(uint32_t n_kv, uint32_t head_dim, uint32_t rows) {
   return (size_t)n_kv * attn_wide_tiles(rows) * (head_dim == 128 ? aw_tile<128>() : aw_tile<64>());
 }
 
-template <int D, bool F32>
-static hipError_t attn_wide_go(const float* q, const float* kc, const float* vc, uint32_t n_heads, uint32_t n_kv, uint32_t max_seq, float scale, uint32_t pos0,
-                               uint32_t m_tokens, uint8_t* scratch, uint8_t* out, hipStream_t st, float* out32) {
+// Splits of a launch of `wgs` workgroups: until two a CU are there, none of fewer than 8 tiles nor without one (the first token block's tiles end behind pos0).  256 tokens of an 8B
+// model are 64 workgroups, and behind many rows each walked them all: 256 tokens behind 1000 / 4000 / 16000 rows, 4 layers, 1059 / 1805 / 4741 us, with splits 948 / 1140 / 1911
+// (blocks of 128 with the f32 kernel 1120 / 1497 / 3142); of 16 tiles or more each 1109 behind 1000.
+static uint32_t attn_wide_splits(uint32_t wgs, uint32_t pos0, uint32_t m_tokens, uint32_t n_heads, uint32_t head_dim, size_t part_floats) {
+  const size_t room = part_floats / ((size_t)m_tokens * n_heads * (head_dim + 2));
+  const uint32_t s = std::min({2u * kNumCU / wgs, pos0 / kAwRows / 8, (uint32_t)std::min<size_t>(room, 16)});
+  return s > 1 ? s : 1;
+}
+
+template <int D, int OUT>
+static hipError_t attn_wide_run(const float* q, const uint8_t* kv, uint32_t n_heads, uint32_t g, uint32_t tiles, float scale, uint32_t pos0, uint32_t m_tokens, uint32_t n_blk,
+                                uint32_t wgs, uint32_t splits, uint8_t* out, float* part, float* ml, hipStream_t st) {
   static bool attr_set[64] = {};
   constexpr uint32_t lds = 3 * aw_half<D>();
-  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&attn_wide_kernel<D, F32>), (int)lds, attr_set); e != hipSuccess) return e;
-  const uint32_t kv_len = pos0 + m_tokens, tiles = attn_wide_tiles(kv_len), g = n_heads / n_kv, gw = g < 4 ? g : 4;
-  hipLaunchKernelGGL((attn_wide_split_kernel<D>), dim3(tiles, n_kv), dim3(256), 0, st, kc, vc, max_seq, kv_len, tiles, scratch);
-  const uint32_t n_blk = (m_tokens + 128 / gw - 1) / (128 / gw), wgs = n_blk * (n_heads / gw);
-  hipLaunchKernelGGL((attn_wide_kernel<D, F32>), dim3(wgs), dim3(256), lds, st, q, scratch, n_heads, g, tiles, scale, pos0, m_tokens, n_blk,
-                     (uint32_t)(wgs <= 2u * kNumCU), out, out32);
+  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&attn_wide_kernel<D, OUT>), (int)lds, attr_set); e != hipSuccess) return e;
+  hipLaunchKernelGGL((attn_wide_kernel<D, OUT>), dim3(wgs, splits), dim3(256), lds, st, q, kv, n_heads, g, tiles, scale, pos0, m_tokens, n_blk,
+                     (uint32_t)(wgs <= 2u * kNumCU), out, part, ml);
   return hipGetLastError();
 }
 
-// scratch: attn_wide_bytes(n_kv, head_dim, pos0 + m_tokens).  out: row-major f16 [token][head][dim] in XH's element order; or out32, f32 in plain order
+template <int D>
+static hipError_t attn_wide_go(const float* q, const float* kc, const float* vc, uint32_t n_heads, uint32_t n_kv, uint32_t max_seq, float scale, uint32_t pos0,
+                               uint32_t m_tokens, uint8_t* scratch, float* part, size_t part_floats, uint8_t* out, hipStream_t st, float* out32) {
+  const uint32_t kv_len = pos0 + m_tokens, tiles = attn_wide_tiles(kv_len), g = n_heads / n_kv, gw = g < 4 ? g : 4;
+  hipLaunchKernelGGL((attn_wide_split_kernel<D>), dim3(tiles, n_kv), dim3(256), 0, st, kc, vc, max_seq, kv_len, tiles, scratch);
+  const uint32_t n_blk = (m_tokens + 128 / gw - 1) / (128 / gw), wgs = n_blk * (n_heads / gw);
+  const uint32_t splits = attn_wide_splits(wgs, pos0, m_tokens, n_heads, D, part_floats), rows = m_tokens * n_heads;
+  if (splits == 1)
+    return out32 ? attn_wide_run<D, AW_F32>(q, scratch, n_heads, g, tiles, scale, pos0, m_tokens, n_blk, wgs, 1, nullptr, out32, nullptr, st)
+                 : attn_wide_run<D, AW_F16>(q, scratch, n_heads, g, tiles, scale, pos0, m_tokens, n_blk, wgs, 1, out, nullptr, nullptr, st);
+  float* ml = part + (size_t)splits * rows * D;
+  if (hipError_t e = attn_wide_run<D, AW_PART>(q, scratch, n_heads, g, tiles, scale, pos0, m_tokens, n_blk, wgs, splits, nullptr, part, ml, st); e != hipSuccess) return e;
+  hipLaunchKernelGGL((attn_wide_merge_kernel<D>), dim3((rows * (D / 4) + 255) / 256), dim3(256), 0, st, part, ml, rows, splits, out, out32);
+  return hipGetLastError();
+}
+
+// scratch: attn_wide_bytes(n_kv, head_dim, pos0 + m_tokens); part: memory for splits (a launch without it has one).  out: row-major f16 [token][head][dim] in XH's element
+// order; or out32, f32 in plain order
 hipError_t attn_wide_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale,
-                            uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, uint8_t* out, hipStream_t st, float* out32) {
+                            uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, float* part, size_t part_bytes, uint8_t* out, hipStream_t st, float* out32) {
   if (n_kv == 0 || n_heads % n_kv || m_tokens == 0 || (head_dim != 64 && head_dim != 128) || pos0 + m_tokens > max_seq || n_kv > 65535 || (!out && !out32)) return hipErrorInvalidValue;
   const uint32_t g = n_heads / n_kv;
   if (g != 1 && g != 2 && g != 4 && g != 8) return hipErrorInvalidValue;
-#define LGH_AW_GO(DD, FF) attn_wide_go<DD, FF>(q, kcache, vcache, n_heads, n_kv, max_seq, scale, pos0, m_tokens, scratch, out, st, out32)
-  if (out32) return head_dim == 128 ? LGH_AW_GO(128, true) : LGH_AW_GO(64, true);
-  return head_dim == 128 ? LGH_AW_GO(128, false) : LGH_AW_GO(64, false);
-#undef LGH_AW_GO
+  if ((size_t)m_tokens * n_heads * 32 > 0xFFFFFFFFull) return hipErrorInvalidValue;   // (the merge's threads)
+  return head_dim == 128 ? attn_wide_go<128>(q, kcache, vcache, n_heads, n_kv, max_seq, scale, pos0, m_tokens, scratch, part, part ? part_bytes / 4 : 0, out, st, out32)
+                         : attn_wide_go<64>(q, kcache, vcache, n_heads, n_kv, max_seq, scale, pos0, m_tokens, scratch, part, part ? part_bytes / 4 : 0, out, st, out32);
 }
 
 }  // namespace lgh

@@ -1084,7 +1084,7 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
     const PfwQkv e{P.part, G.S, G.part_rows, QD, KD, d.head_dim, L.bq, L.bk, L.bv, c->rope_cs, P.inv_rms, pos0, d.max_seq_len, P.q, L.kcache, L.vcache, (int)d.use_neox_rope};
     if ((rc = K(pfw_qkv_launch(e, m, st), "qkv"))) return rc;
     if (li + 1 == c->l1) break;   // the last layer: its K / V rows are written, its output would be discarded
-    if ((rc = K(attn_wide_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.kv_split, P.attn, st), "attention"))) return rc;
+    if ((rc = K(attn_wide_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.kv_split, P.part, P.part_bytes, P.attn, st), "attention"))) return rc;
     G = PfWide{};
     if ((rc = product({&L.wo}, P.attn, G, PW_PART, m, nullptr, "output product"))) return rc;
     if ((rc = resid(P.part, G, L.bo, L.ffn_norm, nullptr))) return rc;

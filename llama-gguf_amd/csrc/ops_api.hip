@@ -386,8 +386,12 @@ int lgh_op_attention_prompt(int device, const float* q, const float* kc, const f
   if ((d != 64 && d != 128) || (g != 1 && g != 2 && g != 4 && g != 8)) return LGH_UNSUPPORTED;
   float *dq = t.up(q, n_tokens * n_heads * d), *dk = t.up(kc, cache), *dv = t.up(vc, cache), *dout = t.up(nullptr, n_tokens * n_heads * d);
   uint8_t* scratch = nullptr;
-  if (!dq || !dk || !dv || !dout || dev_alloc(t.c, (void**)&scratch, attn_wide_bytes((uint32_t)n_kv, (uint32_t)d, (uint32_t)(pos0 + n_tokens)))) return LGH_ALLOCATION_FAILED;
-  if (attn_wide_launch(dq, dk, dv, (uint32_t)n_heads, (uint32_t)n_kv, (uint32_t)d, (uint32_t)max_seq, scale, (uint32_t)pos0, (uint32_t)n_tokens, scratch, nullptr,
+  float* part = nullptr;
+  const size_t part_bytes = (size_t)kPfwPartRows * n_heads * (d + 2) * 4;   // splits x tokens, as in the engine
+  if (!dq || !dk || !dv || !dout || dev_alloc(t.c, (void**)&scratch, attn_wide_bytes((uint32_t)n_kv, (uint32_t)d, (uint32_t)(pos0 + n_tokens))) ||
+      dev_alloc(t.c, (void**)&part, part_bytes))
+    return LGH_ALLOCATION_FAILED;
+  if (attn_wide_launch(dq, dk, dv, (uint32_t)n_heads, (uint32_t)n_kv, (uint32_t)d, (uint32_t)max_seq, scale, (uint32_t)pos0, (uint32_t)n_tokens, scratch, part, part_bytes, nullptr,
                        t.c->stream, dout) != hipSuccess)
     return LGH_OPERATION_FAILED;
   return t.down(out, dout, n_tokens * n_heads * d);

@@ -133,7 +133,7 @@ hipError_t attn_prefill_launch(const float* q, const float* kcache, const float*
 uint32_t attn_wide_tiles(uint32_t rows);
 size_t attn_wide_bytes(uint32_t n_kv, uint32_t head_dim, uint32_t rows);
 hipError_t attn_wide_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale,
-                            uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, uint8_t* out, hipStream_t st, float* out32 = nullptr);
+                            uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, float* part, size_t part_bytes, uint8_t* out, hipStream_t st, float* out32 = nullptr);
 // byte offset of element k of token t in an XH matrix
 __host__ __device__ inline size_t xh_offset(uint32_t t, uint32_t k) {
   const uint32_t ch = k >> 3, j = k & 7, pj = (j == 1 || j == 5) ? j + 1 : (j == 2 || j == 6) ? j - 1 : j;

@@ -59,7 +59,8 @@ def _inputs(d, heads, n_kv, pos0, m, seed):
 @pytest.mark.parametrize("d,heads,n_kv,pos0,m", [
     (64, 4, 4, 0, 1), (64, 8, 1, 0, 31), (128, 4, 2, 0, 33), (128, 8, 2, 5, 127), (128, 4, 4, 31, 128), (64, 8, 4, 33, 129), (128, 8, 1, 64, 257),
     (64, 16, 2, 700, 300), (128, 16, 4, 0, 511), (128, 3, 3, 1, 1025),
-    (64, 40, 40, 0, 2047)])                                   # more than two workgroups a CU
+    (64, 40, 40, 0, 2047),                                    # more than two workgroups a CU
+    (128, 4, 1, 1100, 40), (64, 8, 8, 9000, 70), (128, 8, 1, 3001, 129), (64, 8, 2, 1050, 511)])   # few tokens behind many rows: splits, 2 to 16 of them
 def test_ordinary_inputs(pkg, d, heads, n_kv, pos0, m):
     q, kc, vc = _inputs(d, heads, n_kv, pos0, m, 7 * m + d)
     print("relative error", _check(q, kc, vc, pos0, _run(pkg, q, kc, vc, pos0), ordinary=True))
