@@ -63,12 +63,26 @@ void dev_free_tracked(lgh_ctx* c, void* p) {
 }
 
 // Contexts up to this many rows run the single-launch decode attention (attention.hip, attn_direct_kernel; attention_tq.hip, attn_tq_direct_kernel) unless the flags say
-// otherwise: a query head's rows all pass through one CU, which pays until they take longer than the split kernel's merge and second launch.  Measured against the split kernel with
-// its merge, us per layer gained, 8 kv heads of 128 with 4 query heads each: f32 4.8 / 5.0 / 3.6 / 1.0 / -0.1 / -5.1 at 40 / 128 / 256 / 400 / 512 / 1000 rows, TurboQuant 3 bits
-// 9.7 / 8.9 / 6.8 / 3.3 / 2.8 / 0.5 / -3.5 at 40 / 256 / 512 / 1000 / 1200 / 1500 / 2000, 2 bits 8.8 / 7.6 / 5.5 / 0.9 / 0.1 / -2.8 at 40 / 256 / 512 / 1000 / 1200 / 1500;
-// 4 kv heads of 64 with 8 each: f32 7.7 / 7.9 / 6.5 / 2.8 / 1.6 / -0.9 at 40 / 256 / 512 / 1000 / 1500 / 2000, 3 bits 19.8 / 17.9 / 13.7 / 8.1 / 3.7 / -1.0 at 40 / 1000 / 2000 / 4000 /
-// 6000 / 8000, 2 bits 11.5 at 2000.
-static uint32_t direct_attn_default_kv(uint32_t head_dim, bool tq) { return tq ? (head_dim == 64 ? 4096 : 1152) : (head_dim == 64 ? 1536 : 448); }
+// otherwise: a query head's rows all pass through one CU, which pays until they take longer than the split kernel's merge and second launch.  The query heads of a kv head
+// share its rows in an L2, and the split kernel's workgroup grows with their number (over codes by far), so the line depends on it.  us per layer gained against split and
+// merge (4 layers of 2048; heads / kv heads: 16/16 and 32/32, 16/8, 32/8, 64/8 and 8/1; the least of a column's shapes):
+//   heads per kv head       1                            2                            4                            8
+//   f32   128 dims   1.0 at 384, -0.6 at 448      0.9 at 448, 0.9 at 512       1.2 at 448, -0.2 at 640      3.6 at 448, 1.8 at 640
+//          64        1.1 at 768, -1.6 at 1024     1.4 at 1024, -0.1 at 1280    0.7 at 1280, -1.3 at 1536    1.2 at 1536, -1.4 at 1800
+//   codes of 3 bits
+//         128        0.1 at 900, -0.3 at 1024     0.7 at 900, 0.0 at 1024      3.9 at 1152, 2.6 at 1300     11.4 at 1152, 10.3 at 1300
+//          64        0.2 at 2048, -0.4 at 2560    0.7 at 2048, 0.2 at 2560     0.9 at 3584, -1.4 at 4096    7.3 at 4096, 6.8 at 5000
+//   codes of 2 bits
+//         128        0.2 at 512, -1.4 at 768      1.9 at 512, -0.2 at 768      1.0 at 1152, -0.1 at 1300    9.8 at 1152, 8.5 at 1300
+//          64        -1.0 at 1536                 0.4 at 1536, -1.6 at 2048    1.3 at 2560, -0.7 at 3072    5.0 at 3584, 2.1 at 4096
+// Over codes the line is a context's capacity too, up to which its batched steps take the single launch (engine_batch.hip).  A full cache of 1152 rows, 32/8 heads of 128, gained by
+// 2 / 4 / 16 sequences: 1.2 / 12.5 / 66 (2 bits), 2.5 / 17.7 / 81 (3 bits); 3584 rows, 32/4 of 64: 1.9 / 23 / 136 and 5.8 / 32 / 157 (2 bits and 2 sequences lose 1.9 at 4096).
+static uint32_t direct_attn_default_kv(uint32_t head_dim, uint32_t group, uint32_t bits) {   // bits: of codes, 0 over f32
+  static constexpr uint32_t rows[3][2][4] = {{{384, 448, 448, 448}, {768, 1152, 1280, 1536}},
+                                             {{512, 640, 1152, 1152}, {1280, 1536, 2560, 3584}},
+                                             {{896, 1024, 1152, 1152}, {2048, 2304, 3584, 4096}}};
+  return rows[bits == 0 ? 0 : bits == 2 ? 1 : 2][head_dim == 64][group >= 8 ? 3 : group >= 4 ? 2 : group >= 2 ? 1 : 0];
+}
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ------------------------------------------------------------------------------------------------
@@ -1235,7 +1249,7 @@ int lgh_create(const lgh_model_desc* desc, lgh_ctx** out) {
   c->n_splits = splits;
   const uint32_t dsel = (d.flags >> LGH_FLAG_ATTN_DIRECT_SHIFT) & 0xFFu;
   const bool tq_direct = kv_is_tq(d.kv_cache_type) && !kv_is_qjl(d.kv_cache_type);
-  c->direct_attn_max_kv = dsel == 255 ? 0 : dsel ? dsel * 64 : direct_attn_default_kv(d.head_dim, tq_direct);
+  c->direct_attn_max_kv = dsel == 255 ? 0 : dsel ? dsel * 64 : direct_attn_default_kv(d.head_dim, d.num_heads / d.num_kv_heads, tq_direct ? kv_tq_bits(d.kv_cache_type) : 0);
   if ((d.flags & LGH_FLAG_KV_INT8) && !tq_direct) c->direct_attn_max_kv = 0;   // the other byte caches have one attention structure: splits + combine
   *out = c;
   return LGH_OK;

@@ -53,3 +53,19 @@ def test_direct_attention_over_codes_matches_the_split_kernel(pkg, head_dim, hea
         assert np.abs(got[0] - got[1]).max() <= 2e-4 * np.abs(got[1]).max(), rows
     direct.close()
     split.close()
+
+
+@pytest.mark.parametrize("head_dim,heads,kv_heads,limit", [(128, 4, 4, 384), (128, 4, 2, 448), (128, 8, 1, 448), (64, 4, 4, 768), (64, 4, 2, 1152), (64, 8, 2, 1280), (64, 8, 1, 1536)])
+def test_the_default_limit_goes_by_the_query_heads_of_a_kv_head(pkg, head_dim, heads, kv_heads, limit):
+    """Up to the limit a default engine has the bits of the single launch, behind it those of split and merge."""
+    cfg = pkg.make_config("test-dense", max_seq_len=limit + 64, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, num_layers=1)
+    model = pkg.SynthModel(cfg, mix="Q8_0")
+    engs = [pkg.HipGpuInference.from_model(model, limit + 64, attn_direct=d) for d in (0, 32, 255)]
+    prompt = [(7 * i + 5) % cfg.vocab_size for i in range(limit - 1)]
+    got = []
+    for eng in engs:
+        eng.forward_batch(prompt)
+        got.append([eng.forward(t) for t in (3, 4)])          # limit and limit + 1 rows
+        eng.close()
+    assert not np.array_equal(got[1][0], got[2][0]) and not np.array_equal(got[1][1], got[2][1])
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[2][1])
