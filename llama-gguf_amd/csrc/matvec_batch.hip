@@ -866,6 +866,9 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
 }
 
 // grid / block = the single-sequence geometry of `L` (segments' wg_begin, rows_per_wg).  dynamic LDS: mvqb_lds_bytes(n_seq, L.red_floats)
+// FEW: up to four sequences whose rows in a workgroup are one a thread at most (mvqb2_epilogue_few): loaded as they are, divided into quads they take longer than they save
+// (a step, 32 layers of an 8B model, 2 / 4 sequences: 2.545 / 2.850 ms in quads, 2.486 / 2.822 here)
+template <bool FEW>
 __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_floats,
                                                                       const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B,
                                                                       const float* __restrict__ part) {
@@ -895,42 +898,51 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t w
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
   const uint32_t ub = sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2;
   const size_t rows16 = (size_t)Gm.n_units * 16;
-  // four rows a load, four loads of a thread under way at once, the norms' behind the first of them: 6.0 us at 16 sequences of an 8B model (one row a load, each awaited: 7.2)
-  const uint32_t quads = S_rpw / 4, items = n_seq * npass * nslots * quads;
-  constexpr uint32_t kAtOnce = 4;
-  f32x4 v[kAtOnce];
-  auto place = [&](uint32_t i, uint32_t& s, uint32_t& ps, uint32_t& rl) {   // item -> sequence, p * nslots + slot, first row
-    const uint32_t j = i / quads;
-    rl = (i - j * quads) * 4;
-    s = j / (npass * nslots);
-    ps = j - s * npass * nslots;
-  };
-  auto load = [&](uint32_t i0) {
+  if constexpr (FEW) {
+    const uint32_t per_seq = npass * nslots * S_rpw, s = threadIdx.x / per_seq, j = threadIdx.x - s * per_seq;
+    const uint32_t ps = j / S_rpw, p = ps / nslots, row = wg * S_rpw + j - ps * S_rpw;                 // ps = p * nslots + slot
+    float v = 0.0f;
+    if (s < n_seq && row < ntiles * 16) v = part[((size_t)(ps - p * nslots) * B.n_seq + s) * rows16 + (size_t)(ub + p * ntiles) * 16 + row];
+    if (nrm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
+    if (s < n_seq) red[(size_t)s * red_floats + j] = v;
+  } else {
+    // four rows a load, four loads of a thread under way at once, the norms' behind the first of them: 6.0 us at 16 sequences of an 8B model (one row a load, each awaited: 7.2)
+    const uint32_t quads = S_rpw / 4, items = n_seq * npass * nslots * quads;
+    constexpr uint32_t kAtOnce = 4;
+    f32x4 v[kAtOnce];
+    auto place = [&](uint32_t i, uint32_t& s, uint32_t& ps, uint32_t& rl) {   // item -> sequence, p * nslots + slot, first row
+      const uint32_t j = i / quads;
+      rl = (i - j * quads) * 4;
+      s = j / (npass * nslots);
+      ps = j - s * npass * nslots;
+    };
+    auto load = [&](uint32_t i0) {
 #pragma unroll
-    for (uint32_t k = 0; k < kAtOnce; k++) {
-      const uint32_t i = i0 + k * (kBWaves * 64);
-      uint32_t s, ps, rl;
-      place(i < items ? i : 0, s, ps, rl);
-      const uint32_t p = ps / nslots, slot = ps - p * nslots, row = wg * S_rpw + rl;
-      v[k] = (f32x4)(0.0f);
-      if (i < items && row < ntiles * 16)
-        v[k] = *reinterpret_cast<const f32x4*>(part + ((size_t)slot * B.n_seq + s) * rows16 + (size_t)(ub + p * ntiles) * 16 + row);
-    }
-  };
-  load(threadIdx.x);
-  if (nrm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
-  for (uint32_t i0 = threadIdx.x; i0 < items; i0 += kAtOnce * kBWaves * 64) {
-#pragma unroll
-    for (uint32_t k = 0; k < kAtOnce; k++) {
-      const uint32_t i = i0 + k * (kBWaves * 64);
-      if (i < items) {
+      for (uint32_t k = 0; k < kAtOnce; k++) {
+        const uint32_t i = i0 + k * (kBWaves * 64);
         uint32_t s, ps, rl;
-        place(i, s, ps, rl);
-#pragma unroll
-        for (int e = 0; e < 4; e++) red[(size_t)s * red_floats + ps * S_rpw + rl + e] = v[k][e];
+        place(i < items ? i : 0, s, ps, rl);
+        const uint32_t p = ps / nslots, slot = ps - p * nslots, row = wg * S_rpw + rl;
+        v[k] = (f32x4)(0.0f);
+        if (i < items && row < ntiles * 16)
+          v[k] = *reinterpret_cast<const f32x4*>(part + ((size_t)slot * B.n_seq + s) * rows16 + (size_t)(ub + p * ntiles) * 16 + row);
       }
+    };
+    load(threadIdx.x);
+    if (nrm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
+    for (uint32_t i0 = threadIdx.x; i0 < items; i0 += kAtOnce * kBWaves * 64) {
+#pragma unroll
+      for (uint32_t k = 0; k < kAtOnce; k++) {
+        const uint32_t i = i0 + k * (kBWaves * 64);
+        if (i < items) {
+          uint32_t s, ps, rl;
+          place(i, s, ps, rl);
+#pragma unroll
+          for (int e = 0; e < 4; e++) red[(size_t)s * red_floats + ps * S_rpw + rl + e] = v[k][e];
+        }
+      }
+      if (i0 + kAtOnce * kBWaves * 64 < items) load(i0 + kAtOnce * kBWaves * 64);
     }
-    if (i0 + kAtOnce * kBWaves * 64 < items) load(i0 + kAtOnce * kBWaves * 64);
   }
   mvqb_tail(L, S, B, sg, wg, n_seq, red_floats, red, ssq, nslots, ind_idx);
 }
@@ -988,10 +1000,17 @@ static hipError_t mvqb4_go(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom&
   return hipGetLastError();
 }
 
+static bool mvqb2_epilogue_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm) {
+  if (B.ind_cnt || B.n_seq > 4) return false;
+  for (int i = 0; i < L.nseg; i++)
+    if (B.n_seq * (uint32_t)L.seg[i].npass * Gm.nslots * L.seg[i].rows_per_wg > (uint32_t)kBWaves * 64) return false;
+  return true;
+}
+
 template <uint32_t MASK, int NB>
 static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, const Mvqb2Geom& Gm, bool seq, uint32_t groups, size_t lds_x,
                            size_t lds_e, uint32_t threads, hipStream_t st) {
-  static bool attr_set[3][64] = {};
+  static bool attr_set[4][64] = {};
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
@@ -1009,10 +1028,12 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
     hipLaunchKernelGGL((mvqb2_kernel<MASK, NB, false>), dim3(groups, Gm.T, nz), dim3(kBWaves * 64), lds_x, st, Gm, L, B, B.part);
   }
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb2_epilogue_kernel), 160 * 1024, attr_set[2]); e != hipSuccess) return e;
-  hipLaunchKernelGGL(mvqb2_epilogue_kernel, dim3(g.n_wg, 1, nz), dim3(threads), lds_e, st, g.wbpack, g.geom, g.geom2, L.red_floats, Gm, L, B,
-                     (const float*)B.part);
-  return hipGetLastError();
+  auto epilogue = [&](auto* kernel, bool (&opted)[64]) -> hipError_t {
+    if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(kernel), 160 * 1024, opted); e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3(g.n_wg, 1, nz), dim3(threads), lds_e, st, g.wbpack, g.geom, g.geom2, L.red_floats, Gm, L, B, (const float*)B.part);
+    return hipGetLastError();
+  };
+  return mvqb2_epilogue_few(L, B, Gm) ? epilogue(&mvqb2_epilogue_kernel<true>, attr_set[2]) : epilogue(&mvqb2_epilogue_kernel<false>, attr_set[3]);
 }
 
 // 0: the records-through-LDS structure (mvqb2) from LGH_MVQB2_MIN sequences on (default: measured crossover), 1: never, 2: always
