@@ -982,7 +982,9 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
 // ---- long prompts: blocks of up to kPfwTokens tokens (prefill_wide.hip) ----
 // From this many tokens on a prompt takes the wide path.  A dense model's products fill a workgroup's 256 tokens there: at Llama-3-8B widths, 8 layers,
 // 255 tokens take 2.12 ms as two blocks and 2.08 ms wide, 192 tokens 1.86 and 1.93, 257 tokens 2.75 and 2.21, 512 tokens 4.33 and 2.67.  A mixture's
-// tokens spread over its experts, so its rows fill no tile either way (Mixtral widths, 2 layers: 160 tokens 1.00 and 0.70 ms, 600 tokens 2.67 and 1.07).
+// tokens spread over its experts, so its rows fill no tile either way (Mixtral widths, 2 layers: 160 tokens 1.05 and 0.59 ms, 600 tokens 2.65 and 1.01).
+// The lines hold for narrow models too, whose products leave CUs idle either way: 256 / 257 / 600 tokens in blocks and wide, TinyLlama 4.19 and 3.58, 5.41 and 3.57, 10.5 and
+// 4.18 ms; hidden 512 x 1024, 8 layers, 0.98 and 0.80, 1.28 and 0.79, 2.50 and 0.96; four experts of 768, 160 tokens 1.67 and 0.75.
 // Shorter ones keep the blocks that pipeline stages hand over, with their bits.
 static size_t pfw_min_tokens(const lgh_ctx* c) { return c->d.num_experts ? 160 : 256; }
 

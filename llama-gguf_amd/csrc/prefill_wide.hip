@@ -9,8 +9,8 @@
 // Activations: row-major f16, [token][K], the eight elements of a 16-byte chunk in the order 0,2,1,3,4,6,5,7 (the order in which two masks pull
 // nibbles out of a tile16 word, as in prefill.h's XH).  Same operands, same rounding points and f32 accumulation as prefill.hip.
 //
-// Measured: 2047 tokens of Llama-3-8B Q4_K_M widths, 16 layers: 42.1 ms in blocks of 128, 16.4 ms here with attention_wide.hip (gate | up 0.44 ms a layer =
-// 1.09 PFLOP/s; torch's f16 product of 8192^3 reaches 1.14); 600 tokens of Mixtral widths, 2 layers: 2.95 and 1.21 ms.  What bounds it: the chip's power
+// Measured: 2047 tokens of Llama-3-8B Q4_K_M widths, 16 layers: 44.4 ms in blocks of 128, 18.4 ms here with attention_wide.hip (gate | up 0.44 to 0.47 ms a layer from box
+// to box = 1.02 to 1.09 PFLOP/s; torch's f16 product of 8192^3 reaches 1.14); 600 tokens of Mixtral widths, 2 layers: 2.99 and 1.31 ms.  What bounds it: the chip's power
 // before any single unit (the same loop without the dequantization takes 26 % less time, without the activations' DMA 22 %, without the stores 11 %).
 // Eight waves of half the tokens each (two per SIMD, weights dequantized twice) took the same time.
 #include "mv_epilogue.h"
