@@ -3,6 +3,8 @@ engine (f32 throughout, token by token).
 
 Tolerance: that of the 128-token blocks, 1e-2 * max|logit| + 1e-2: the operands of every product are rounded to f16 (2^-12 each) in both paths, and
 the rounding of a layer's output is carried on by the next ones; measured 1e-3 to 3e-3 of the largest logit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -108,4 +110,35 @@ def test_long_prompts_without_their_own_memory_take_the_short_blocks(pkg):
     eng.forward_batch(prompt)
     _follow(exact, eng, (5, 77))
     for e in (eng, whole, short, exact):
+        e.close()
+
+
+@pytest.mark.parametrize("n", [200, 300])
+def test_stages_against_one_context(pkg, n):
+    """Stages hand blocks of 128 tokens over: below 256 tokens the bits of a single context, which takes the long path from there on, behind it its rounding."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+
+    def hop(dst, src, rows):
+        s0.synchronize()
+        assert hip.hipMemcpy(dst, src, rows * cfg.hidden_size * 4, 3) == 0 and hip.hipDeviceSynchronize() == 0
+
+    cfg = pkg.make_config("test-dense-d128", max_seq_len=400)
+    model = pkg.SynthModel(cfg, mix="Q4_K_M")
+    one, s0, s1 = (pkg.HipGpuInference.from_model(model, 400, layer_range=r) for r in (None, (0, 1), (1, cfg.num_layers)))
+    prompt = [(7 * i + 3) % cfg.vocab_size for i in range(n)]
+    one.forward_batch(prompt)
+    for at in range(0, n, 128):
+        block = prompt[at:at + 128]
+        s0.stage_prefill_batch(block, len(block))
+        hop(s1.stage_hidden_block_ptr(), s0.stage_hidden_block_ptr(), len(block))
+        s1.stage_prefill_batch(None, len(block))
+        s1.synchronize()
+    want = one.forward(5)
+    s0.stage_forward(5)
+    hop(s1.stage_hidden_ptr(), s0.stage_hidden_ptr(), 1)
+    got = s1.stage_forward(0, want_logits=True)
+    assert n >= 256 or np.array_equal(want, got)
+    assert np.abs(got - want).max() <= 1e-2 * float(np.abs(want).max()) + 1e-2
+    for e in (one, s0, s1):
         e.close()
