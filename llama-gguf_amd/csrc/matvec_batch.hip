@@ -795,8 +795,14 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
 #pragma unroll
             for (int pp = 0; pp < 4; pp++) {
               const uint32_t v = tw[pp][c];
-              const uint32_t lo = __builtin_amdgcn_perm(__float_as_uint(ub1(v)), __float_as_uint(ub0(v)), 0x07060302u);
-              const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(ub3(v)), __float_as_uint(ub2(v)), 0x07060302u);
+              uint32_t lo, hi;
+              if (is(F_Q5K)) {
+                lo = __builtin_amdgcn_perm(__float_as_uint(ub1(v)), __float_as_uint(ub0(v)), 0x07060302u);
+                hi = __builtin_amdgcn_perm(__float_as_uint(ub3(v)), __float_as_uint(ub2(v)), 0x07060302u);
+              } else {   // a byte up to 16 is, as an 8-bit float, 2^-9 of itself: two a conversion (gate | up as above 42.7 -> 40.3 us)
+                lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, false));
+                hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, true));
+              }
               w[pp] = __builtin_bit_cast(b16x8, u32x4{lo, hi, lo, hi});
             }
             if (mins) s2[c & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xm[c], ts.gq[c >> 1], zero, 0, 0, 0);
