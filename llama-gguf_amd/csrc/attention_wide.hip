@@ -234,12 +234,12 @@ __global__ void __launch_bounds__(256, 2) attn_wide_kernel(const float* __restri
     const float inv = OUT == AW_PART ? 1.0f : 1.0f / l;
     if (OUT == AW_PART && c == 0) { ml[row * 2] = m_run[t]; ml[row * 2 + 1] = l; }
 #pragma unroll
-    for (int x = 0; x < DT; x++) {                                         // dims 16 x + 4c .. + 3; f16: in the chunk's element order
+    for (int x = 0; x < DT; x++) {                                         // dims 16 x + 4c .. + 3
       const f32x4 v = acc[x][t] * inv;
       if constexpr (OUT != AW_F16) {
         *reinterpret_cast<f32x4*>(part + at + x * 16) = v;
       } else {
-        const h16x4 w = {(_Float16)v.x, (_Float16)v.z, (_Float16)v.y, (_Float16)v.w};
+        const h16x4 w = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
         *reinterpret_cast<h16x4*>(out + (at + x * 16) * 2) = w;
       }
     }
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256) attn_wide_merge_kernel(const float* __res
   if (out32) {
     *reinterpret_cast<f32x4*>(out32 + (size_t)row * D + q * 4) = v;
   } else {
-    const h16x4 w = {(_Float16)v.x, (_Float16)v.z, (_Float16)v.y, (_Float16)v.w};
+    const h16x4 w = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
     *reinterpret_cast<h16x4*>(out + ((size_t)row * D + q * 4) * 2) = w;
   }
 }

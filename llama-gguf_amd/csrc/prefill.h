@@ -66,7 +66,7 @@ hipError_t pf_moe_swiglu_launch(const float* part, uint32_t S, uint32_t F, uint8
 hipError_t pf_moe_combine_launch(const float* part, uint32_t S, const int* tokmap, const float* moe_w, uint32_t top_k, float* hidden, uint32_t H,
                                  const float* nw, uint8_t* xh, float* ssq, uint32_t m_tokens, hipStream_t st);
 hipError_t pf_to_xh_launch(const float* x, uint32_t K, uint8_t* xh, uint32_t m_tokens, hipStream_t st);
-// ---- long prompts (prefill_wide.hip): blocks of up to kPfwTokens tokens, row-major f16 activations [token][K] (16-byte chunks in XH's element order) ----
+// ---- long prompts (prefill_wide.hip): blocks of up to kPfwTokens tokens, row-major f16 activations [token][K] ----
 constexpr uint32_t kPfwTile = 256;                // tokens of a workgroup
 constexpr uint32_t kPfwTokens = 2048;             // tokens of a block
 constexpr uint32_t kPfwMaxRows = kPfwTokens * kPfMaxTopK;   // rows of a product: tokens, or the (token, expert) pairs of a mixture
@@ -136,8 +136,8 @@ hipError_t attn_wide_launch(const float* q, const float* kcache, const float* vc
                             uint32_t pos0, uint32_t m_tokens, uint8_t* scratch, float* part, size_t part_bytes, uint8_t* out, hipStream_t st, float* out32 = nullptr);
 // byte offset of element k of token t in an XH matrix
 __host__ __device__ inline size_t xh_offset(uint32_t t, uint32_t k) {
-  const uint32_t ch = k >> 3, j = k & 7, pj = (j == 1 || j == 5) ? j + 1 : (j == 2 || j == 6) ? j - 1 : j;
-  return (size_t)(ch >> 5) * kPfSlabBytes + t * 512 + (((ch & 31) ^ (t & 15)) << 4) + pj * 2;
+  const uint32_t ch = k >> 3;
+  return (size_t)(ch >> 5) * kPfSlabBytes + t * 512 + (((ch & 31) ^ (t & 15)) << 4) + (k & 7) * 2;
 }
 
 }  // namespace lgh

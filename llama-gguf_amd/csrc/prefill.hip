@@ -23,8 +23,7 @@
 //
 // "XH": an activation matrix [128 tokens][K] in f16, laid out for the GEMM's B operand: one 64 KB slab per 256
 // elements of K (copied verbatim into LDS by LDS-DMA), inside a slab token t owns 512 B = 32 chunks of 8 elements, chunk
-// q stored at position q ^ (t & 15) (so that the 16 tokens of an MFMA operand read 16 different LDS banks groups), inside
-// a chunk the elements are in the order 0,2,1,3,4,6,5,7 (the order in which two masks pull nibbles out of a tile16 word).
+// q stored at position q ^ (t & 15) (so that the 16 tokens of an MFMA operand read 16 different LDS banks groups).
 //
 // GEMM: a workgroup = 4 waves = 256 weight rows x one k-range x all 128 tokens; a wave = 4 row tiles (64 rows): weights
 // go HBM -> registers -> f16 (never through LDS: the dequantized lane layout IS the A operand), an activation fragment
@@ -356,7 +355,7 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
 // chunk `ch` (8 consecutive elements starting at 8*ch) of token t
 __device__ __forceinline__ void xh_store_chunk(uint8_t* xh, uint32_t t, uint32_t ch, const float v[8]) {
   const uint32_t b = ch >> 5, q = ch & 31;
-  h16x8 o = {(_Float16)v[0], (_Float16)v[2], (_Float16)v[1], (_Float16)v[3], (_Float16)v[4], (_Float16)v[6], (_Float16)v[5], (_Float16)v[7]};
+  h16x8 o = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3], (_Float16)v[4], (_Float16)v[5], (_Float16)v[6], (_Float16)v[7]};
   *reinterpret_cast<h16x8*>(xh + (size_t)b * kPfSlabBytes + t * 512 + ((q ^ (t & 15)) << 4)) = o;
 }
 

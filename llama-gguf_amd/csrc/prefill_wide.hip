@@ -6,8 +6,7 @@
 // Here a workgroup keeps 256 weight rows x 256 tokens (256 f32 accumulators per lane): a dequantized weight feeds twice as many products, the loop is
 // bound by the matrix pipe, and from about 512 tokens on the widest matrices need no split at all, so that SwiGLU runs in the epilogue.
 //
-// Activations: row-major f16, [token][K], the eight elements of a 16-byte chunk in the order 0,2,1,3,4,6,5,7 (the order in which two masks pull
-// nibbles out of a tile16 word, as in prefill.h's XH).  Same operands, same rounding points and f32 accumulation as prefill.hip.
+// Activations: row-major f16, [token][K].  Same operands, same rounding points and f32 accumulation as prefill.hip.
 //
 // Measured: 2047 tokens of Llama-3-8B Q4_K_M widths, 16 layers: 44.4 ms in blocks of 128, 18.4 ms here with attention_wide.hip (gate | up 0.44 to 0.47 ms a layer from box
 // to box = 1.02 to 1.09 PFLOP/s; torch's f16 product of 8192^3 reaches 1.14); 600 tokens of Mixtral widths, 2 layers: 2.99 and 1.31 ms.  What bounds it: the chip's power
@@ -257,7 +256,7 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = silu_f(acc[0][t][4 * i + e] * inv) * (acc[1][t][4 * i + e] * inv);
-        const h16x4 o = {(_Float16)v[0], (_Float16)v[2], (_Float16)v[1], (_Float16)v[3]};
+        const h16x4 o = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
         *reinterpret_cast<h16x4*>(turn + tk * 80 + i * 16 + g * 8) = o;
       }
 #pragma unroll
@@ -436,7 +435,7 @@ size_t pfw_part_bytes(uint32_t max_rows, uint32_t cols) { return (size_t)std::ma
 // row kernels
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void pw_store_chunk(uint8_t* x, uint32_t K, uint32_t t, uint32_t ch, const float v[8]) {
-  const h16x8 o = {(_Float16)v[0], (_Float16)v[2], (_Float16)v[1], (_Float16)v[3], (_Float16)v[4], (_Float16)v[6], (_Float16)v[5], (_Float16)v[7]};
+  const h16x8 o = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3], (_Float16)v[4], (_Float16)v[5], (_Float16)v[6], (_Float16)v[7]};
   *reinterpret_cast<h16x8*>(x + (size_t)t * K * 2 + ch * 16) = o;
 }
 
