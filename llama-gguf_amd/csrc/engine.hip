@@ -940,8 +940,12 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
     uint8_t* next_xh = next_nw ? P.xh_h : nullptr;
     if (!L.moe()) {
       const DevWeight* gu[2] = {&L.gate, &L.up};
-      if ((rc = K(pf_gemm_launch(gu, 2, P.xh_h, P.part, P.part_bytes, m, &S, &nc, st), "gate/up GEMM"))) return rc;
-      if ((rc = K(pf_swiglu_launch(P.part, S, F, P.xh_act, P.ssq, H, d.norm_eps, m, st), "SwiGLU"))) return rc;
+      if (pf_pairs(&L.gate, &L.up, m)) {
+        if ((rc = K(pf_pair_launch(&L.gate, &L.up, P.xh_h, P.xh_act, P.ssq, H, d.norm_eps, m, st), "gate | up product"))) return rc;
+      } else {
+        if ((rc = K(pf_gemm_launch(gu, 2, P.xh_h, P.part, P.part_bytes, m, &S, &nc, st), "gate/up GEMM"))) return rc;
+        if ((rc = K(pf_swiglu_launch(P.part, S, F, P.xh_act, P.ssq, H, d.norm_eps, m, st), "SwiGLU"))) return rc;
+      }
       const DevWeight* dn[1] = {&L.down};
       if ((rc = K(pf_gemm_launch(dn, 1, P.xh_act, P.part, P.part_bytes, m, &S, &nc, st), "down GEMM"))) return rc;
       if ((rc = K(pf_row_epi_launch(P.part, S, nc, 0, nullptr, P.hidden, H, next_nw, next_xh, P.ssq, m, st), "down epilogue"))) return rc;

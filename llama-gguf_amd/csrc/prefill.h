@@ -32,6 +32,11 @@ struct PfGemm {
   const int* row_base;   // optional (MoE): device word, first row of this expert's batch in the buffer
   uint32_t m_tiles;      // token tiles that hold real tokens
   const int* m_count;    // optional (MoE): device word with the number of real rows; overrides m_tiles, 0 rows = nothing to do
+  // gate | up with SwiGLU: the activations (XH), the input's sums of squares and the norm they stand for, the tokens
+  uint8_t* act;
+  const float* ssq;
+  uint32_t n_ssq, norm_cols, m_tokens;
+  float eps;
 };
 
 bool pf_supported_type(int dev_type);
@@ -39,6 +44,9 @@ size_t pf_part_bytes(const uint32_t* n_rows, int nw, uint32_t k, uint32_t part_r
 hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, float* part, size_t part_bytes, uint32_t m_tokens,
                           uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t expert = 0, const int* m_count = nullptr,
                           uint32_t part_rows = kPfTokens, const int* row_base = nullptr);
+// silu(gate) * up of one launch -> XH
+bool pf_pairs(const DevWeight* gate, const DevWeight* up, uint32_t m_tokens);
+hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint8_t* xh, uint8_t* act, const float* ssq, uint32_t norm_cols, float eps, uint32_t m_tokens, hipStream_t st);
 hipError_t pf_row_epi_launch(const float* part, uint32_t S, uint32_t ncols, uint32_t col0, const float* bias, float* hidden, uint32_t H,
                              const float* nw, uint8_t* xh, float* ssq, uint32_t m_tokens, hipStream_t st, const float* moe_w = nullptr);
 hipError_t pf_qkv_epi_launch(const float* part, uint32_t S, uint32_t ncols, uint32_t QD, uint32_t KD, uint32_t head_dim, const float* bq,

@@ -13,7 +13,7 @@
 //   XH(h * attn_norm) --GEMM wq|wk|wv--> partial sums --pf_qkv_epi (x 1/rms, bias, RoPE)--> q [M][QD] f32, K/V cache rows
 //   q, cache --attention (attention.hip, PF variant; causal: token t sees pos0 + t + 1 rows)--> XH(attn)
 //   XH(attn) --GEMM wo--> partials --pf_resid (+bias, +residual)--> h, XH(h * ffn_norm), sums of squares per token
-//   XH --GEMM gate|up--> partials --pf_swiglu (x 1/rms)--> XH(act) --GEMM down--> partials --pf_resid--> h, XH(h * attn_norm')
+//   XH --GEMM gate|up--> partials --pf_swiglu (x 1/rms)--> XH(act), or both in pf_pair_kernel; --GEMM down--> partials --pf_resid--> h, XH(h * attn_norm')
 // MoE layers (moe.rs:321-413): the f32 decode router runs once per token of the block, the (token, slot) pairs are grouped
 // by expert into one row space (prefill.h), and every expert runs ONCE over its rows: one gather launch, a gate|up GEMM per
 // expert, one SwiGLU launch, a down GEMM per expert, one combine launch (routing weight * expert output in selection order,
@@ -262,12 +262,136 @@ __global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_few_kernel(const PfGemm
   pf_gemm_device<MASK, MT>(G, pf_smem);
 }
 
-template <auto* Kernel, int MT>
+// 1 / rms of token t from the per-chunk sums of squares its producer left (simd.rs:847-878); 1 when there is no norm
+__device__ __forceinline__ float pf_inv_rms(const float* ssq, uint32_t n_ssq, uint32_t t, uint32_t H, float eps) {
+  if (!ssq) return 1.0f;
+  float tot = 0.0f;
+  for (uint32_t j = 0; j < n_ssq; j++) tot += ssq[t * kPfSsqChunks + j];
+  return 1.0f / __builtin_sqrtf(tot / (float)H + eps);
+}
+
+// silu(gate) * up without partial sums: a wave has the 16 gate rows and the 16 up rows of the same columns as one tile of 32 over all of k, and up to 32 TT tokens, on
+// v_mfma_f32_32x32x16_f16 (less power per product than the 16 x 16 shape, and power is what bounds these loops).  Lane 32g + 16s + n holds row n of gate (s = 0) or up (1), and of every 64 elements
+// the two 16-element chunks 2g + j that the tile16 layout keeps for lanes 16(2g + j) + n; a block has 16 phases (pp, j, h), each the contraction of elements 64pp + 16(2g + j) + 8h .. + 7 of both g.
+// 127 / 64 / 32 tokens of an 8B model in Q4_K_M (28672 rows of 4096): 44 / 26 / 19.5 us a layer, products in two k-ranges and SwiGLU behind them 52 / 36 / 29.  On the 16 x 16 shape 127 tokens took 46.5;
+// three blocks requested ahead instead of one changed nothing at 64 tokens and saved 1.6 us at 32 (two teams save 3).  The weights alone take 13 us.
+// KH 2: two teams of waves, each over half of k, the second's sums through LDS.  With up to 64 tokens a block is mostly dequantization, and two waves a SIMD issue it twice as fast as one.
+template <int F, int TT, int KH>
+__global__ void __launch_bounds__(KH * kPfWaves * 64) pf_pair_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr uint32_t kBuf = (uint32_t)TT * 32 * 512, kDma = kBuf / kPfWaves, tb = pf_tile_bytes(F);
+  constexpr int AHEAD = 2;                                            // phases the activations are read ahead
+  const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6 & 3)), team = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+  const uint32_t n = lane & 15, s = lane >> 4 & 1, g = lane >> 5, tk = lane & 31, nblk = G.nblk / KH;   // this team's blocks
+  const uint32_t tile = blockIdx.x * kPfWaves + wave, tl = tile < G.seg[0].ntiles ? tile : G.seg[0].ntiles - 1;   // clamped: loads are unconditional
+  const uint8_t* const wrow = (s ? G.seg[1].w : G.seg[0].w) + ((size_t)tl * G.nblk + team * nblk) * tb;
+  uint8_t* const slab = smem + team * 2 * kBuf;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)slab;
+  auto x_dma = [&](uint32_t b) {
+    const uint8_t* src = G.xh + (size_t)(team * nblk + b) * kPfSlabBytes + wave * kDma;
+    const uint32_t dst = lds_base + (b & 1) * kBuf + wave * kDma;
+#pragma unroll
+    for (int i = 0; i < (int)(kDma / 1024); i++)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane * 16), "s"(src + i * 1024), "s"(dst + i * 1024) : "memory", "m0");
+  };
+  auto load = [&](uint32_t b, PfRaw (&to)[2]) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) pf_load<F>(to[j], wrow + (size_t)b * tb, 16 * (2 * g + j) + n, n);   // (the row's scales once: the compiler sees that they are the same)
+  };
+  f32x16 acc[TT];
+#pragma unroll
+  for (int t = 0; t < TT; t++) acc[t] = (f32x16)(0.0f);
+  PfRaw w[2][2];   // [block parity][j]
+  x_dma(0);
+  load(0, w[0]);
+  float inv[TT];   // 1 / rms of this lane's tokens
+#pragma unroll
+  for (int t = 0; t < TT; t++) inv[t] = pf_inv_rms(G.ssq, G.n_ssq, t * 32 + tk, G.norm_cols, G.eps) * (1.0f / kPfScale);
+  auto landed = [&] {
+    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): see pf_body
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  landed();
+  h16x8 af[2], bf[4][TT];
+  h16x2 S, O;
+  auto read_bf = [&](uint32_t b, int p) {   // p = 4 pp + 2 j + h
+    const uint32_t q = (uint32_t)(8 * (p >> 2) + (p & 3)) + 4 * g;
+#pragma unroll
+    for (int t = 0; t < TT; t++) bf[p & 3][t] = *reinterpret_cast<const h16x8*>(slab + (b & 1) * kBuf + (t * 32 + tk) * 512 + ((q ^ n) << 4));
+  };
+  auto frag = [&](const PfRaw (&cw)[2], int p) {
+    const int pp = p >> 2, j = p >> 1 & 1;
+    if ((p & 3) == 0 || (F == PF_Q6K && (p & 1) == 0)) pf_scale<F>(cw[j], pp, n, 2 * g + j, S, O);
+    af[p & 1] = pf_frag<F>(cw[j], pp, p & 1, S, O);
+  };
+  auto block = [&](uint32_t b, PfRaw (&cw)[2], PfRaw (&nw)[2]) {   // (the last one requests nothing; what it reads of the buffer and the registers beyond the end is not used)
+    if (b + 1 < nblk) {
+      x_dma(b + 1);
+      load(b + 1, nw);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < 16; p++) {
+      if (p == 16 - AHEAD) landed();
+      if (p + AHEAD < 16) read_bf(b, p + AHEAD);
+      else read_bf(b + 1, p + AHEAD - 16);
+      if (p < 15) frag(cw, p + 1);
+      else frag(nw, 0);
+#pragma unroll
+      for (int t = 0; t < TT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[p & 1], bf[p & 3][t], acc[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < AHEAD; p++) read_bf(0, p);
+  frag(w[0], 0);
+  for (uint32_t b = 0; b < nblk; b += 2) {   // (whole pairs of blocks: pf_pair_go)
+    block(b, w[0], w[1]);
+    block(b + 1, w[1], w[0]);
+  }
+  if constexpr (KH == 2) {
+    f32x4* const sums = reinterpret_cast<f32x4*>(smem) + wave * (TT * 4 * 64) + lane;
+    __syncthreads();   // (every read of the slabs has returned)
+    if (team == 1) {
+#pragma unroll
+      for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sums[(t * 4 + i) * 64] = f32x4{acc[t][4 * i], acc[t][4 * i + 1], acc[t][4 * i + 2], acc[t][4 * i + 3]};
+    }
+    __syncthreads();
+    if (team == 1) return;
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const f32x4 v = sums[(t * 4 + i) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[t][4 * i + e] += v[e];
+      }
+  }
+  // a lane has, per token, rows 8i + 4g .. + 3: gate with i = 0, 1, up with i + 2
+  if (tile >= G.seg[0].ntiles) return;
+#pragma unroll
+  for (int t = 0; t < TT; t++) {
+    const uint32_t tok = t * 32 + tk;
+    if (tok >= G.m_tokens) continue;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      h16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] = (_Float16)(silu_f(acc[t][4 * i + e] * inv[t]) * (acc[t][4 * i + 8 + e] * inv[t]));
+      *reinterpret_cast<h16x4*>(G.act + xh_offset(tok, tile * 16 + 8 * i + 4 * g)) = o;
+    }
+  }
+}
+
+template <auto* Kernel, int MT, int TEAMS = 1>
 static hipError_t pf_gemm_run(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
   static bool attr_set[64] = {};
-  constexpr size_t lds = MT ? 2 * (size_t)MT * 16 * 512 : 2 * kPfSlabBytes;
+  constexpr size_t lds = TEAMS * 2 * (MT ? (size_t)MT * 16 * 512 : kPfSlabBytes);
   if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(Kernel), (int)lds, attr_set); e != hipSuccess) return e;
-  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S), dim3(kPfWaves * 64), lds, st, G);
+  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S), dim3(TEAMS * kPfWaves * 64), lds, st, G);
   return hipGetLastError();
 }
 template <uint32_t MASK>
@@ -349,6 +473,55 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
   }
 }
 
+// chunks of per-token sums of squares a row of H elements is reduced to (pf_inv_rms adds them up)
+uint32_t pf_ssq_chunks(uint32_t H) { return (H + 2047) / 2048; }
+
+// gate | up as one product without partial sums.  Its workgroups are half as wide as those of a product in k-ranges and not split; with up to 64 tokens that is the faster one for any width (8B widths,
+// 4 layers, 10 / 33 / 50 tokens 526 / 549 / 602 us in ranges, 503 / 523 / 578 here; TinyLlama's, 8 layers, 24 / 50 tokens 706 / 777 and 671 / 744), with more only while the ranges are one or two
+// (8B, two, 128 tokens: 741 -> 722; TinyLlama, five: 100 tokens 920 -> 941, 200 tokens 1539 -> 1565).
+bool pf_pairs(const DevWeight* gate, const DevWeight* up, uint32_t m_tokens) {
+  if (!pf_supported_type(gate->type) || gate->type != up->type || gate->k != up->k || gate->n != up->n || gate->k % 512 || gate->n % 256) return false;
+  return m_tokens <= 64 || 3 * (2 * gate->n / 256) > (uint32_t)kNumCU;
+}
+
+template <int F>
+static hipError_t pf_pair_go(const PfGemm& G, hipStream_t st) {
+  const uint32_t wgs = (G.seg[0].ntiles + kPfWaves - 1) / kPfWaves;
+  const bool halves = G.nblk % 4 == 0;
+  if (G.m_tiles <= 2) return halves ? pf_gemm_run<&pf_pair_kernel<F, 1, 2>, 2, 2>(G, wgs, st) : pf_gemm_run<&pf_pair_kernel<F, 1, 1>, 2>(G, wgs, st);
+  if (G.m_tiles <= 4) return halves ? pf_gemm_run<&pf_pair_kernel<F, 2, 2>, 4, 2>(G, wgs, st) : pf_gemm_run<&pf_pair_kernel<F, 2, 1>, 4>(G, wgs, st);
+  return pf_gemm_run<&pf_pair_kernel<F, 4, 1>, kPfMT>(G, wgs, st);
+}
+
+hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint8_t* xh, uint8_t* act, const float* ssq, uint32_t norm_cols, float eps, uint32_t m_tokens, hipStream_t st) {
+  if (m_tokens == 0 || !pf_pairs(gate, up, m_tokens) || m_tokens > (uint32_t)kPfTokens || !act || !ssq) return hipErrorInvalidValue;
+  PfGemm G{};
+  for (int i = 0; i < 2; i++) {
+    const DevWeight* W = i ? up : gate;
+    G.seg[i].w = W->plane[0];
+    G.seg[i].ntiles = W->n / 16;
+  }
+  G.nseg = 1;
+  G.nblk = gate->k / 256;
+  G.S = 1;
+  G.xh = xh;
+  G.act = act;
+  G.ssq = ssq;
+  G.n_ssq = pf_ssq_chunks(norm_cols);
+  G.norm_cols = norm_cols;
+  G.eps = eps;
+  G.m_tokens = m_tokens;
+  G.m_tiles = (m_tokens + 15) / 16;
+  switch (pf_fmt_of(gate->type)) {
+    case PF_Q4K: return pf_pair_go<PF_Q4K>(G, st);
+    case PF_Q6K: return pf_pair_go<PF_Q6K>(G, st);
+    case PF_Q5K: return pf_pair_go<PF_Q5K>(G, st);
+    case PF_Q80: return pf_pair_go<PF_Q80>(G, st);
+    case PF_Q40: return pf_pair_go<PF_Q40>(G, st);
+  }
+  return hipErrorInvalidValue;
+}
+
 // ------------------------------------------------------------------------------------------------
 // XH writers and the row-wise kernels between the GEMMs
 // ------------------------------------------------------------------------------------------------
@@ -357,14 +530,6 @@ __device__ __forceinline__ void xh_store_chunk(uint8_t* xh, uint32_t t, uint32_t
   const uint32_t b = ch >> 5, q = ch & 31;
   h16x8 o = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3], (_Float16)v[4], (_Float16)v[5], (_Float16)v[6], (_Float16)v[7]};
   *reinterpret_cast<h16x8*>(xh + (size_t)b * kPfSlabBytes + t * 512 + ((q ^ (t & 15)) << 4)) = o;
-}
-
-// 1 / rms of token t from the per-chunk sums of squares its producer left (simd.rs:847-878); 1 when there is no norm
-__device__ __forceinline__ float pf_inv_rms(const float* ssq, uint32_t n_ssq, uint32_t t, uint32_t H, float eps) {
-  if (!ssq) return 1.0f;
-  float tot = 0.0f;
-  for (uint32_t j = 0; j < n_ssq; j++) tot += ssq[t * kPfSsqChunks + j];
-  return 1.0f / __builtin_sqrtf(tot / (float)H + eps);
 }
 
 // The residual's partial sums are requested eight splits at a time and added in order: 16 tokens and 16 splits 6.5 -> 4.8 us (128 tokens 7.2 -> 7.1).  QKV's eight splits of two values
@@ -429,9 +594,6 @@ __global__ void __launch_bounds__(256) pf_resid_kernel(const float* __restrict__
   __syncthreads();
   if (threadIdx.x == 0 && ssq) ssq[t * kPfSsqChunks + blockIdx.x] = (s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3]);
 }
-
-// chunks of per-token sums of squares a row of H elements is reduced to (pf_inv_rms adds them up)
-uint32_t pf_ssq_chunks(uint32_t H) { return (H + 2047) / 2048; }
 
 hipError_t pf_row_epi_launch(const float* part, uint32_t S, uint32_t ncols, uint32_t col0, const float* bias, float* hidden, uint32_t H,
                              const float* nw, uint8_t* xh, float* ssq, uint32_t m_tokens, hipStream_t st, const float* moe_w) {

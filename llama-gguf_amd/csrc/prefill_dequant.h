@@ -11,6 +11,8 @@
 namespace lgh {
 
 typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
 
 // formats as in matvec_mfma.hip (same tile16 layouts)
@@ -64,7 +66,7 @@ __device__ __forceinline__ void pf_scale(const PfRaw& r, int pp, uint32_t n, uin
     const uint32_t hdw = pp == 0 ? r.hd.x : pp == 1 ? r.hd.y : pp == 2 ? r.hd.z : r.hd.w;
     const float scf = (float)(int)__builtin_amdgcn_sbfe((int)hdw, c * 8, 8);
     const uint32_t dh = (n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu;
-    S = pf_bcast(h2f(dh) * scf * kPfScale);
+    S = pf_bcast(h2f(dh) * kPfScale * scf);
     O = S * pf_bcast(-32.0f);
   } else if (F == PF_Q80 || F == PF_Q40) {   // y = d * q (Q8_0, stored q + 128 after the sign flip) / d * (q - 8) (Q4_0)
     const uint32_t hdw = pp == 0 ? r.hd.x : pp == 1 ? r.hd.y : pp == 2 ? r.hd.z : r.hd.w;
@@ -85,9 +87,9 @@ __device__ __forceinline__ void pf_scale(const PfRaw& r, int pp, uint32_t n, uin
       sc = pp == 2 ? sc23 & 0xFFu : sc23 >> 16;
       mn = pp == 2 ? mn23 & 0xFFu : mn23 >> 16;
     }
-    const float dd = h2f(r.hd.x & 0xFFFFu), dmin = h2f(r.hd.x >> 16);
-    S = pf_bcast(dd * (float)sc * kPfScale);
-    O = pf_bcast(-(dmin * (float)mn) * kPfScale);
+    const float dd = h2f(r.hd.x & 0xFFFFu) * kPfScale, dmin = h2f(r.hd.x >> 16) * -kPfScale;
+    S = pf_bcast(dd * (float)sc);
+    O = pf_bcast(dmin * (float)mn);
   }
 }
 
@@ -108,8 +110,8 @@ __device__ __forceinline__ h16x8 pf_fin4(uint32_t b0, uint32_t b1, uint32_t b2, 
 }
 
 // eight nibbles (word byte t = w[t] | w[t+4] << 4) -> f16.  A byte up to 16 is, as an 8-bit float, 2^-9 of itself: two whole numbers a conversion, 11 instructions for eight weights
-// (with masks and an exponent, (x & m) | 0x6400 - 1024, 15).  2047 tokens through 16 layers of an 8B model in Q4_K_M
-// 17.2 -> 16.9 ms, 128 through 32 6.00 -> 5.91 (some two vector instructions hide under a 16x16 matrix instruction, the others add to its time)
+// (with masks and an exponent, (x & m) | 0x6400 - 1024, 15).  The products' loops are bound by the sum of their matrix and vector instructions, about two of the latter a matrix
+// instruction hidden: 127 tokens of an 8B model in Q4_K_M, gate | up @PFA@ us
 __device__ __forceinline__ h16x8 pf_frag_nib(uint32_t N, h16x2 S, h16x2 O) {
   const uint32_t m = 0x0F0F0F0Fu, lo = N & m, hi = (N >> 4) & m;
   auto two = [](uint32_t b, auto up) { return __builtin_bit_cast(h16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.0f, up.value)); };

@@ -18,8 +18,6 @@
 namespace lgh {
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWWaves = 4, kWRT = 4;                      // waves of a workgroup, 16-row weight tiles of a wave
 constexpr uint32_t kWStepBytes = kPfwTile * 128;          // 64 elements of 256 tokens
