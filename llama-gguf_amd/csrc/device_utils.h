@@ -104,4 +104,14 @@ __device__ __forceinline__ float swap32_max(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+
+// silu for activations that are rounded to 16 bits next: x / (1 + e^-x) as the library's expf and the compiler's division compute it (over +-80 the largest error, 1.8e-7, and the mean square
+// of the errors are theirs), in 14 instructions instead of 31: the exponent is clamped, so neither needs its special cases.  Below -87 the result is x e^-87: -1.5e-36 instead of less.
+__device__ __forceinline__ float silu_act_f(float x) {
+  const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f), n = __builtin_rintf(c * -1.44269504f);
+  const float f = __builtin_fmaf(c, -1.92596299e-8f, __builtin_fmaf(c, -1.44269504f, -n));   // log2 e in two parts
+  const float d = 1.0f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n), r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
+}
+
 }  // namespace lgh

@@ -642,7 +642,7 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
         for (int e = 0; e < 4; e++) {
           if constexpr (EPI == LE_CLAMPED) { o[e] = to_act<T>(in * clamped_glu_f(acc[i][j][e], acc[i + 1][j][e], a.grp.limit)); continue; }
           const float gt = GRP ? in * acc[i][j][e] : acc[i][j][e], u = GRP ? in * acc[i + 1][j][e] : acc[i + 1][j][e];
-          o[e] = to_act<T>((EPI == LE_SWIGLU ? silu_f(gt) : gelu_tanh_f(gt)) * u);
+          o[e] = to_act<T>((EPI != LE_SWIGLU ? gelu_tanh_f(gt) : sizeof(T) == 2 ? silu_act_f(gt) : silu_f(gt)) * u);
         }
       }
     } else {

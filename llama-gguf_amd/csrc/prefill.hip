@@ -380,7 +380,7 @@ __global__ void __launch_bounds__(KH * kPfWaves * 64) pf_pair_kernel(const PfGem
     for (int i = 0; i < 2; i++) {
       h16x4 o;
 #pragma unroll
-      for (int e = 0; e < 4; e++) o[e] = (_Float16)(silu_f(acc[t][4 * i + e] * inv[t]) * (acc[t][4 * i + 8 + e] * inv[t]));
+      for (int e = 0; e < 4; e++) o[e] = (_Float16)(silu_act_f(acc[t][4 * i + e] * inv[t]) * (acc[t][4 * i + 8 + e] * inv[t]));
       *reinterpret_cast<h16x4*>(G.act + xh_offset(tok, tile * 16 + 8 * i + 4 * g)) = o;
     }
   }
@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(256) pf_swiglu_kernel(const float* __restrict_
   }
   float v[8];
 #pragma unroll
-  for (int j = 0; j < 8; j++) v[j] = silu_f(g[j] * inv) * (u[j] * inv);
+  for (int j = 0; j < 8; j++) v[j] = silu_act_f(g[j] * inv) * (u[j] * inv);
   xh_store_chunk(xh, t, ch, v);
 }
 
@@ -785,7 +785,7 @@ __global__ void __launch_bounds__(256) pf_moe_swiglu_kernel(const float* __restr
   }
   float v[8];
 #pragma unroll
-  for (int j = 0; j < 8; j++) v[j] = silu_f(g[j] * inv) * (u[j] * inv);
+  for (int j = 0; j < 8; j++) v[j] = silu_act_f(g[j] * inv) * (u[j] * inv);
   xh_store_chunk(xh_out + e * out_stride, i, ch, v);
 }
 

@@ -253,7 +253,7 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
       for (int i = 0; i < 4; i++) {
         float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = silu_f(acc[0][t][4 * i + e] * inv) * (acc[1][t][4 * i + e] * inv);
+        for (int e = 0; e < 4; e++) v[e] = silu_act_f(acc[0][t][4 * i + e] * inv) * (acc[1][t][4 * i + e] * inv);
         const h16x4 o = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
         *reinterpret_cast<h16x4*>(turn + tk * 80 + i * 16 + g * 8) = o;
       }
