@@ -51,13 +51,13 @@ __device__ __forceinline__ void mvqb_norms(const MvLaunch& L, const MvBatch& B, 
   }
 }
 
-__device__ __forceinline__ void mvqb_tail(const MvLaunch& L, const MvSeg& S, const MvBatch& B, int sg, uint32_t wg, uint32_t n_seq,
+__device__ __forceinline__ void mvqb_tail(const MvLaunch& L, const MvSeg& S, const MvBatch& B, int sg, uint32_t wg, uint32_t rows_per_wg, uint32_t n_seq,
                                           uint32_t red_floats, float* red, float* ssq, uint32_t nslots, const int* ind_idx = nullptr) {
   const uint32_t tid = threadIdx.x;
   __syncthreads();
   // the sequences side by side: a sequence's epilogue needs one thread per row (pair) — groups of `tpr` threads take sequences
   // s, s + n_par, ...; each runs the single-sequence epilogue
-  const uint32_t tpr = (S.rows_per_wg + 15u) & ~15u;   // (16-lane rows: what the XQ image's cross-lane steps work on)
+  const uint32_t tpr = (rows_per_wg + 15u) & ~15u;   // (16-lane rows: what the XQ image's cross-lane steps work on)
   const uint32_t n_par = max(1u, blockDim.x / tpr);
   const uint32_t grp = tid / tpr, tl = tid - grp * tpr;
   if (grp >= n_par) return;
@@ -70,7 +70,7 @@ __device__ __forceinline__ void mvqb_tail(const MvLaunch& L, const MvSeg& S, con
     V.xq_out = S.xq_out ? S.xq_out + (size_t)so * B.xq_out_stride[sg] : nullptr;
     V.xq_ssq = S.xq_ssq ? S.xq_ssq + (size_t)so * B.ssq_out_stride[sg] : nullptr;
     V.pos = B.pos + s;
-    mv_epilogue_view(L, S, V, wg, red + (size_t)s * red_floats, ssq + s * 8, nslots, MvEpiPre{0.0f, 0.0f, false}, tl);
+    mv_epilogue_view(L, S, V, wg, rows_per_wg, red + (size_t)s * red_floats, ssq + s * 8, nslots, MvEpiPre{0.0f, 0.0f, false}, tl);
   }
 }
 
@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb_kernel(uint32_t wbpack, uin
   }
 
   if (nrm) mvqb_norms(L, B, n_seq, ssq, nullptr);
-  mvqb_tail(L, S, B, sg, wg, n_seq, red_floats, red, ssq, S_T);
+  mvqb_tail(L, S, B, sg, wg, S.rows_per_wg, n_seq, red_floats, red, ssq, S_T);
 }
 
 // ================================================================================================
@@ -225,10 +225,11 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb_kernel(uint32_t wbpack, uin
 // single-sequence kernel (blocks [ks * nbw, (ks + 1) * nbw)) the four lane groups are folded with the same two shuffles, giving
 // the slice's partial sum p_ks.  The single-sequence epilogue adds the slices up as ((0 + p_0) + p_1) + ...:
 //   SEQ  = true   a workgroup walks ALL slices of its units and keeps that running sum in registers (same additions, same order);
-//                 one value per (sequence, row) goes to the partial buffer (nslots = 1: the epilogue computes 0 + sum = sum);
+//                 one value per (sequence, row) goes to the epilogue (nslots = 1: it computes 0 + sum = sum), in the same launch where the launch has one segment
+//                 (Mvqb2Geom::fuse), else through the partial buffer;
 //   SEQ  = false  (matrices with too few units to fill the chip that way: wo, down, QKV) blockIdx.y = the slice; p_ks goes to
 //                 the partial buffer (nslots = T) and the epilogue adds them in slice order.
-// Either way a second, small launch (mvqb2_epilogue_kernel) loads the partial sums into LDS in the layout the single-sequence
+// Otherwise a second, small launch (mvqb2_epilogue_kernel) loads the partial sums into LDS in the layout the single-sequence
 // epilogue reads and runs exactly that epilogue per sequence — every sequence's result is bit-identical to matvec_mfma.hip's.
 // ================================================================================================
 struct Mvqb2Geom {
@@ -237,7 +238,28 @@ struct Mvqb2Geom {
   uint32_t ub1, ub2;          // first unit of segment 1 / 2 (n_units when absent)
   uint32_t cb;                // blocks staged per chunk
   uint32_t nslots;            // partial sums per (sequence, row) in the buffer: 1 (SEQ) or T
+  // SEQ, one segment (gate | up, the output head): a workgroup has all there is of its rows and runs the epilogue itself, its eight units being 8 tiles, or 4 tiles of both passes.  fuse = passes, 0: no.
+  // 16 sequences, 8 layers of an 8B model: gate | up 40.3 -> 43.3 us and the head 58 -> 63, their epilogue launches (7.3 and 7.5 us and a gap each) gone; a batch with its prompts 43.2 -> 42.4 ms
+  uint32_t fuse;
+  uint32_t ssq_at;            // fuse: LDS byte of the sequences' sums of squares, behind all else
 };
+
+// unit of wave w of workgroup wg
+__device__ __forceinline__ void mvqb_unit(const Mvqb2Geom& Gm, uint32_t wg, uint32_t w, uint32_t ntiles, uint32_t ul, bool& active, uint32_t& pass, uint32_t& tl) {
+  if (Gm.fuse) {
+    pass = Gm.fuse == 2 ? w & 1 : 0;
+    tl = Gm.fuse == 2 ? wg * (kBWaves / 2) + (w >> 1) : wg * kBWaves + w;
+    active = tl < ntiles;
+    if (!active) pass = tl = 0;
+  } else {
+    pass = active ? ul / ntiles : 0;
+    tl = active ? ul - pass * ntiles : 0;
+  }
+}
+constexpr uint32_t kFuseRed = kBWaves * 16;   // floats a sequence: [pass][row of the workgroup]
+// place of row n of this wave's unit
+__device__ __forceinline__ uint32_t mvqb_red_at(const Mvqb2Geom& Gm, uint32_t w, uint32_t n) { return Gm.fuse == 2 ? ((w & 1) * 4 + (w >> 1)) * 16 + n : w * 16 + n; }
+__host__ __device__ constexpr uint32_t mvqb_fuse_lds(uint32_t n_seq) { return n_seq * 8 * 4; }
 
 #ifndef LGH_XSTAGE_KB
 #define LGH_XSTAGE_KB 40   /* (experiment builds vary it: the cost of a chunk boundary, profiles/r03e_batched_decode.md) */
@@ -265,8 +287,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_kernel(const Mvqb2Geom Gm,
     part += (size_t)ez * B.part_z_floats;
   }
   const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
-  const bool active = u < Gm.n_units;
-  const int sg = (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  bool active = u < Gm.n_units;
+  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
   const MvSeg& S = L.seg[active ? sg : 0];
   constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
   const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
@@ -275,7 +297,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_kernel(const Mvqb2Geom Gm,
                       : is(F_Q80) ? fmt_tile_bytes(F_Q80) : fmt_tile_bytes(F_Q40);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
   const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
-  const uint32_t pass = active ? ul / ntiles : 0, tl = active ? ul - pass * ntiles : 0;
+  uint32_t pass, tl;
+  mvqb_unit(Gm, blockIdx.x, wave, ntiles, ul, active, pass, tl);
   const uint8_t* wbase = (pass == 0 ? S.pass[0].plane[0] + (uint64_t)ez * S.pass[0].sel_stride[0] : S.pass[1].plane[0] + (uint64_t)ez * S.pass[1].sel_stride[0]) +
                          (size_t)tl * Gm.nblk * tb;
   const uint8_t* xg = L.seg[0].pass[0].xq;                        // sequence 0's records (all segments and passes share the input)
@@ -293,6 +316,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_kernel(const Mvqb2Geom Gm,
   for (uint32_t i = tid; i < kXZeroBytes / 16; i += kBWaves * 64) *reinterpret_cast<u32x4*>(smem8 + zero_off + i * 16) = u32x4{0u, 0u, 0u, 0u};
   uint32_t* xsel = reinterpret_cast<uint32_t*>(smem8 + zero_off + kXZeroBytes);
   if (tid < n_seq) xsel[tid] = ind_idx ? (uint32_t)ind_idx[tid] / B.ind_div : tid;
+  float* const ssq = reinterpret_cast<float*>(smem8 + Gm.ssq_at);
+  if (SEQ && Gm.fuse && L.do_norm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
   __syncthreads();
   const bool a_valid = (n >> 2) == mq;
   const uint32_t a_off = (mq >> 1) * 128 + (n & 3) * 32 + (mq & 1) * 16;
@@ -418,6 +443,17 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_kernel(const Mvqb2Geom Gm,
     }
     ks = nks; b0 = nb0; buf ^= 1u;
   }
+  if (SEQ && Gm.fuse) {
+    float* red = reinterpret_cast<float*>(smem8);
+    __syncthreads();   // every record has been read
+    if (mq == 0) {
+#pragma unroll
+      for (int s = 0; s < NB; s++)
+        if ((uint32_t)s < n_seq) red[s * kFuseRed + mvqb_red_at(Gm, wave, n)] = tot[s];
+    }
+    mvqb_tail(L, S, B, 0, blockIdx.x, Gm.fuse == 2 ? kFuseRed / 2 : kFuseRed, n_seq, kFuseRed, red, ssq, 1, ind_idx);
+    return;
+  }
   if (active && mq == 0) {
     const uint32_t slot = SEQ ? 0u : blockIdx.y;
     const size_t rows16 = (size_t)Gm.n_units * 16;
@@ -485,8 +521,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
   const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
-  const bool active = u < Gm.n_units;
-  const int sg = (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  bool active = u < Gm.n_units;
+  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
   const MvSeg& S = L.seg[active ? sg : 0];
   constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
   const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
@@ -495,7 +531,10 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
                       : is(F_Q80) ? fmt_tile_bytes(F_Q80) : fmt_tile_bytes(F_Q40);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
   const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
-  const uint32_t pass = active ? ul / ntiles : 0, tl = active ? ul - pass * ntiles : 0;
+  uint32_t pass, tl;
+  mvqb_unit(Gm, blockIdx.x, wave, ntiles, ul, active, pass, tl);
+  float* const ssq = reinterpret_cast<float*>(smem8 + Gm.ssq_at);
+  if (SEQ && Gm.fuse && L.do_norm) mvqb_norms(L, B, n_seq, ssq, nullptr);
   const uint8_t* wbase = (pass == 0 ? S.pass[0].plane[0] : S.pass[1].plane[0]) + (size_t)tl * Gm.nblk * tb;
   const uint8_t* xg = L.seg[0].pass[0].xq;                        // sequence 0's records (all segments and passes share the input)
   const uint32_t n = lane & 15, mq = lane >> 4;
@@ -616,6 +655,16 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
     }
     ks = nks; b0 = nb0; buf ^= 1u;
   }
+  if (SEQ && Gm.fuse) {
+    float* red = reinterpret_cast<float*>(smem8);
+    const uint32_t at = mvqb_red_at(Gm, wave, n);
+    __syncthreads();   // every record has been read
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+      if (4 * g + mq < n_seq) red[(4 * g + mq) * kFuseRed + at] = tot[g];
+    mvqb_tail(L, S, B, 0, blockIdx.x, Gm.fuse == 2 ? kFuseRed / 2 : kFuseRed, n_seq, kFuseRed, red, ssq, 1);
+    return;
+  }
   if (active) {
     const uint32_t slot = SEQ ? 0u : blockIdx.y;
     const size_t rows16 = (size_t)Gm.n_units * 16;
@@ -655,8 +704,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
   const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
-  const bool active = u < Gm.n_units;
-  const int sg = (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  bool active = u < Gm.n_units;
+  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
   const MvSeg& S = L.seg[active ? sg : 0];
   constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
   const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
@@ -664,7 +713,10 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
   const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K) : fmt_tile_bytes(F_Q40);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
   const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
-  const uint32_t pass = active ? ul / ntiles : 0, tl = active ? ul - pass * ntiles : 0;
+  uint32_t pass, tl;
+  mvqb_unit(Gm, blockIdx.x, wave, ntiles, ul, active, pass, tl);
+  float* const ssq = reinterpret_cast<float*>(smem8 + Gm.ssq_at);
+  if (SEQ && Gm.fuse && L.do_norm) mvqb_norms(L, B, n_seq, ssq, nullptr);
   const uint8_t* wbase = (pass == 0 ? S.pass[0].plane[0] : S.pass[1].plane[0]) + (size_t)tl * Gm.nblk * tb;
   const uint32_t n = lane & 15, mq = lane >> 4;
   const uint32_t ks0 = SEQ ? 0u : blockIdx.y, ks1 = SEQ ? Gm.T : blockIdx.y + 1;   // this workgroup's slices
@@ -858,6 +910,20 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
     }
     ks = nks; b0 = nb0; buf ^= 1u;
   }
+  if (SEQ && Gm.fuse) {
+    float* red = reinterpret_cast<float*>(smem8);
+    const uint32_t at = mvqb_red_at(Gm, wave, n);
+    __syncthreads();   // every record has been read
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const uint32_t s = 8 * g + mq + 4 * q;
+        if (q < nq(g) && s < n_seq) red[s * kFuseRed + at] = tot[g][q];
+      }
+    mvqb_tail(L, S, B, 0, blockIdx.x, Gm.fuse == 2 ? kFuseRed / 2 : kFuseRed, n_seq, kFuseRed, red, ssq, 1);
+    return;
+  }
   if (active) {
     const uint32_t slot = SEQ ? 0u : blockIdx.y;
     const size_t rows16 = (size_t)Gm.n_units * 16;
@@ -950,7 +1016,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t w
       if (i0 + kAtOnce * kBWaves * 64 < items) load(i0 + kAtOnce * kBWaves * 64);
     }
   }
-  mvqb_tail(L, S, B, sg, wg, n_seq, red_floats, red, ssq, nslots, ind_idx);
+  mvqb_tail(L, S, B, sg, wg, S.rows_per_wg, n_seq, red_floats, red, ssq, nslots, ind_idx);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -981,7 +1047,8 @@ template <uint32_t MASK, int NB>
 static hipError_t mvqb8_go(const MvLaunch& L, const MvBatch& B, Mvqb2Geom Gm, bool seq, uint32_t groups, hipStream_t st) {
   static bool attr_set[2][64] = {};
   Gm.cb = std::max(1u, std::min(Gm.nbw, kX8Records / B.n_seq));
-  const size_t lds = (size_t)2 * Gm.cb * B.n_seq * (kX8Record + kX8Sums);
+  Gm.ssq_at = 2 * Gm.cb * B.n_seq * (kX8Record + kX8Sums);
+  const size_t lds = Gm.ssq_at + mvqb_fuse_lds(B.n_seq);
   if (seq) {
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb8_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
     hipLaunchKernelGGL((mvqb8_kernel<MASK, NB, true>), dim3(groups), dim3(kBWaves * 64), lds, st, Gm, L, B, B.part);
@@ -993,9 +1060,10 @@ static hipError_t mvqb8_go(const MvLaunch& L, const MvBatch& B, Mvqb2Geom Gm, bo
 }
 
 template <uint32_t MASK, int NB>
-static hipError_t mvqb4_go(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, bool seq, uint32_t groups, hipStream_t st) {
+static hipError_t mvqb4_go(const MvLaunch& L, const MvBatch& B, Mvqb2Geom Gm, bool seq, uint32_t groups, hipStream_t st) {
   static bool attr_set[2][64] = {};
-  const size_t lds = (size_t)2 * mvqb4_buf_bytes(Gm.cb * B.n_seq);
+  Gm.ssq_at = 2 * mvqb4_buf_bytes(Gm.cb * B.n_seq);
+  const size_t lds = Gm.ssq_at + mvqb_fuse_lds(B.n_seq);
   if (seq) {
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb4_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
     hipLaunchKernelGGL((mvqb4_kernel<MASK, NB, true>), dim3(groups), dim3(kBWaves * 64), lds, st, Gm, L, B, B.part);
@@ -1014,10 +1082,12 @@ static bool mvqb2_epilogue_few(const MvLaunch& L, const MvBatch& B, const Mvqb2G
 }
 
 template <uint32_t MASK, int NB>
-static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, const Mvqb2Geom& Gm, bool seq, uint32_t groups, size_t lds_x,
+static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, Mvqb2Geom Gm, bool seq, uint32_t groups, size_t lds_x,
                            size_t lds_e, uint32_t threads, hipStream_t st) {
   static bool attr_set[4][64] = {};
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
+  Gm.ssq_at = (uint32_t)lds_x;
+  lds_x += mvqb_fuse_lds(B.n_seq);
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
     if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
@@ -1033,7 +1103,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb2_kernel<MASK, NB, false>), 160 * 1024, attr_set[1]); e != hipSuccess) return e;
     hipLaunchKernelGGL((mvqb2_kernel<MASK, NB, false>), dim3(groups, Gm.T, nz), dim3(kBWaves * 64), lds_x, st, Gm, L, B, B.part);
   }
-  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || Gm.fuse) return e;
   auto epilogue = [&](auto* kernel, bool (&opted)[64]) -> hipError_t {
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(kernel), 160 * 1024, opted); e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(g.n_wg, 1, nz), dim3(threads), lds_e, st, g.wbpack, g.geom, g.geom2, L.red_floats, Gm, L, B, (const float*)B.part);
@@ -1076,10 +1146,15 @@ hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uin
     Gm.n_units = ub[L.nseg];
     Gm.ub1 = L.nseg > 1 ? ub[1] : Gm.n_units;
     Gm.ub2 = L.nseg > 2 ? ub[2] : Gm.n_units;
-    const uint32_t groups = (Gm.n_units + kBWaves - 1) / kBWaves;
+    uint32_t groups = (Gm.n_units + kBWaves - 1) / kBWaves;
     static const uint32_t seq_min_groups = [] { const char* e = std::getenv("LGH_MVQB2_SEQ_GROUPS"); return e ? (uint32_t)std::atoi(e) : 160u; }();
     const bool seq = groups >= seq_min_groups || Gm.T == 1;  // enough units to fill the chip with whole rows per workgroup
     Gm.nslots = seq ? 1 : Gm.T;
+    if (seq && L.nseg == 1 && (S0.epi == EPI_STORE || S0.epi == EPI_RESID || S0.epi == EPI_SWIGLU)) {
+      Gm.fuse = S0.npass == 2 ? 2 : 1;
+      const uint32_t a_wg = kBWaves / (uint32_t)S0.npass;
+      groups = ((S0.n_rows + 15) / 16 + a_wg - 1) / a_wg;
+    }
     const int nb_inst = B.n_seq <= 4 ? 4 : B.n_seq <= 8 ? 8 : 16;
     Gm.cb = std::max(1u, std::min(Gm.nbw, mvqb2_stage_bytes((mask & (mask - 1)) == 0, nb_inst) / (B.n_seq * (uint32_t)kXqRecord)));
     const size_t lds_x = (size_t)2 * Gm.cb * B.n_seq * kXqRecord + kXZeroBytes + kXSelBytes;

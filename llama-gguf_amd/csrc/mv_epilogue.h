@@ -49,11 +49,11 @@ struct MvEpiView { float* out; const float* resid; uint8_t* xq_out; float* xq_ss
 
 // Per-row epilogue, one thread per row (or per row pair for RoPE)
 // `nslots` = partial sums per (pass, row) in `red`, laid out red[(p * nslots + slot) * rows_per_wg + row]
-__device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg& S, const MvEpiView V, uint32_t wg, const float* red,
+__device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg& S, const MvEpiView V, uint32_t wg, uint32_t rows_per_wg, const float* red,
                                                  const float* ssq, uint32_t nslots, const MvEpiPre pre = MvEpiPre{0.0f, 0.0f, false},
                                                  uint32_t tid = threadIdx.x) {
   const uint32_t t = tid;
-  const uint32_t rbase = wg * S.rows_per_wg;
+  const uint32_t rbase = wg * rows_per_wg;
   float inv = 1.0f;
   if (L.do_norm) {  // simd.rs:853-855: rms = sqrt(ss/n + eps); inv = 1/rms
     float tot = 0.0f;
@@ -62,12 +62,12 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
   }
   auto rowval = [&](int p, uint32_t rl) {
     float v = 0.0f;
-    for (uint32_t ks = 0; ks < nslots; ks++) v += red[(size_t)(p * nslots + ks) * S.rows_per_wg + rl];
+    for (uint32_t ks = 0; ks < nslots; ks++) v += red[(size_t)(p * nslots + ks) * rows_per_wg + rl];
     return v * inv;
   };
   if (S.epi == EPI_ROPE_Q || S.epi == EPI_ROPE_K) {
     uint32_t rl = 2 * t, row = rbase + rl;
-    if (rl >= S.rows_per_wg || row >= S.n_rows) return;
+    if (rl >= rows_per_wg || row >= S.n_rows) return;
     float x0 = rowval(0, rl), x1 = rowval(0, rl + 1);
     if (S.bias) { x0 += S.bias[row]; x1 += S.bias[row + 1]; }
     const uint32_t pos = (uint32_t)*V.pos, d = S.head_dim, half = d / 2;
@@ -85,7 +85,7 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
     }
     return;
   }
-  if (t >= S.rows_per_wg) return;
+  if (t >= rows_per_wg) return;
   const uint32_t row = rbase + t;
   if (row >= S.n_rows) return;
   float v0 = rowval(0, t);
@@ -144,7 +144,7 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
 
 __device__ __forceinline__ void mv_epilogue(const MvLaunch& L, const MvSeg& S, uint32_t wg, const float* red, const float* ssq,
                                             uint32_t nslots, const MvEpiPre pre = MvEpiPre{0.0f, 0.0f, false}, uint32_t tid = threadIdx.x) {
-  mv_epilogue_view(L, S, MvEpiView{S.out, S.resid, S.xq_out, S.xq_ssq, L.pos}, wg, red, ssq, nslots, pre, tid);
+  mv_epilogue_view(L, S, MvEpiView{S.out, S.resid, S.xq_out, S.xq_ssq, L.pos}, wg, S.rows_per_wg, red, ssq, nslots, pre, tid);
 }
 
 }  // namespace lgh
