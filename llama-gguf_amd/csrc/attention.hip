@@ -1003,4 +1003,148 @@ hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc
   return hipGetLastError();
 }
 
+
+// ---- the same in one launch, bit for bit: a workgroup of 16 waves per (query head, sequence) works through the head's splits, 16 / NW at a time with NW waves each, every split's rows, waves
+// and merges exactly as in attn_partial_kernel, and then merges the splits as attn_combine_kernel does.  Rows are requested four steps ahead, across splits.
+// What the two launches cost is the dispatch of their workgroups, the partial sums' way through memory and the splits that a workgroup walks one after the other; what this costs is that a query head's rows pass
+// through one CU and are read once per query head (from the L2 that the heads of a kv head share: attn_direct_kernel).
+template <int D, int NW>
+__global__ void __launch_bounds__(1024, 8) attn_multi_direct_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, uint32_t n_kv, uint32_t g_per_kv,
+                                                                 uint32_t max_seq, float scale, const int* pos_ptr, const int* slot, uint64_t slot_stride, uint32_t n_splits,
+                                                                 float* __restrict__ out, uint8_t* __restrict__ xq_out) {
+  constexpr int LPR = D / 4, RPW = 64 / LPR, QS = 16 / NW, B = NW == 4 ? 3 : 2;   // lanes of a row, rows of a load, splits of a round, steps requested ahead
+  __shared__ float s_ml[2][16][2];
+  __shared__ __attribute__((aligned(16))) float s_acc[2][16][D];
+  __shared__ float p_ml[32][2], p_acc[32][D], s_f[64];
+  __shared__ float s_linv;
+  const uint32_t n_heads = n_kv * g_per_kv, kvh = blockIdx.x % n_kv, head = kvh * g_per_kv + blockIdx.x / n_kv, sq = blockIdx.y;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), sub = lane / LPR, li = lane % LPR;
+  uint32_t pw, sl;
+  asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(pw), "=&s"(sl) : "s"(pos_ptr + sq), "s"(slot + sq) : "memory");
+  const uint32_t kv_len = pw + 1;
+  const float* kb = kc + (size_t)sl * slot_stride + (size_t)kvh * max_seq * D + li * 4;
+  const float* vb = vc + (size_t)sl * slot_stride + (size_t)kvh * max_seq * D + li * 4;
+  const uint32_t stride = n_splits * NW * RPW, used = min(n_splits, pw / (NW * RPW) + 1);
+  const uint32_t per = (kv_len + stride - 1) / stride, rounds = (used + QS - 1) / QS, items = rounds * per;   // steps of a split, rounds, steps of a wave
+  f32x4 kk[B], vv[B];
+  uint32_t rr = 0, rj = 0;   // the next step to request: round, step of the split
+  auto request = [&](int u) {
+    const uint32_t r = (rr * 16 + wave) * RPW + sub + rj * stride, rc = r < kv_len ? r : kv_len - 1;   // clamped: loads are unconditional
+    kk[u] = *reinterpret_cast<const f32x4*>(kb + (size_t)rc * D);
+    vv[u] = *reinterpret_cast<const f32x4*>(vb + (size_t)rc * D);
+    if (++rj == per) { rj = 0; rr++; }
+  };
+#pragma unroll
+  for (int u = 0; u < B; u++) request(u);
+  const f32x4 qv = *reinterpret_cast<const f32x4*>(q + ((size_t)sq * n_heads + head) * D + li * 4);
+  float m = kNegBig, l = 0.0f;
+  f32x4 acc = (f32x4)(0.0f);
+  uint32_t r = 0, j = 0;
+  for (uint32_t i0 = 0; i0 < items; i0 += B) {
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      if (i0 + u >= items) break;
+      const uint32_t base = (r * 16 + wave) * RPW + j * stride;
+      if (base < kv_len && r * QS + wave / NW < n_splits) {   // wave-uniform
+        const f32x4 k4 = kk[u], v4 = vv[u];
+        const bool valid = base + sub < kv_len;
+        float s = qv.x * k4.x;
+        s = __builtin_fmaf(qv.y, k4.y, s);
+        s = __builtin_fmaf(qv.z, k4.z, s);
+        s = __builtin_fmaf(qv.w, k4.w, s);
+        s += dpp_f<0xB1>(s);
+        s += dpp_f<0x4E>(s);
+        s += dpp_f<0x141>(s);
+        s += dpp_f<0x140>(s);
+        if (LPR == 32) s = swap16_add(s);
+        s *= scale;
+        const float mn = valid ? fmaxf(m, s) : m;
+        const float a = __expf(m - mn);
+        const float pe = valid ? __expf(s - mn) : 0.0f;
+        l = __builtin_fmaf(l, a, pe);
+        acc = acc * a + v4 * pe;
+        m = mn;
+      }
+      request(u);
+      if (++j < per) continue;
+      j = 0;
+      // the split's end: the row slots of the wave, then its waves
+      auto merge = [&](auto half) {
+        auto both = [&](float v, float& lo, float& hi) {
+          const auto w = half.value == 16 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)
+                                          : __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+          lo = __uint_as_float(w[0]);
+          hi = __uint_as_float(w[1]);
+        };
+        float m0, m1, l0, l1, a0, a1;
+        both(m, m0, m1);
+        both(l, l0, l1);
+        const float mn = fmaxf(m0, m1), a = expf(m0 - mn), b = expf(m1 - mn);
+        l = l0 * a + l1 * b;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          both(acc[e], a0, a1);
+          acc[e] = a0 * a + a1 * b;
+        }
+        m = mn;
+      };
+      if (LPR == 16) merge(std::integral_constant<int, 16>{});
+      merge(std::integral_constant<int, 32>{});
+      if (sub == 0) {
+        if (li == 0) { s_ml[r & 1][wave][0] = m; s_ml[r & 1][wave][1] = l; }
+        *reinterpret_cast<f32x4*>(&s_acc[r & 1][wave][li * 4]) = acc;
+      }
+      m = kNegBig; l = 0.0f; acc = (f32x4)(0.0f);
+      __syncthreads();   // (two sets: the next round's waves may write while this one is merged)
+      const uint32_t qs = tid / D, dim = tid % D, sp = r * QS + qs;
+      if (tid < (uint32_t)(QS * D) && sp < used) {
+        const float(*ml)[2] = &s_ml[r & 1][qs * NW];
+        const float(*ac)[D] = &s_acc[r & 1][qs * NW];
+        float mn = ml[0][0];
+#pragma unroll
+        for (int w = 1; w < NW; w++) mn = fmaxf(mn, ml[w][0]);
+        float lsum = 0.0f, a = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+          const float f = expf(ml[w][0] - mn);
+          lsum += ml[w][1] * f;
+          a += ac[w][dim] * f;
+        }
+        p_acc[sp][dim] = a;
+        if (dim == 0) { p_ml[sp][0] = mn; p_ml[sp][1] = lsum; }
+      }
+      r++;
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const float mm = tid < used ? p_ml[tid][0] : kNegBig, ll = tid < used ? p_ml[tid][1] : 0.0f;
+    const float mn = wave_max(mm), f = expf(mm - mn), lsum = wave_sum(ll * f);
+    s_f[tid] = f;
+    if (tid == 0) s_linv = 1.0f / lsum;
+  }
+  __syncthreads();
+  if (tid < (uint32_t)D) {
+    float a = 0.0f;
+    for (uint32_t sp = 0; sp < used; sp++) a += p_acc[sp][tid] * s_f[sp];
+    const float o = a * s_linv;
+    out[((size_t)sq * n_heads + head) * D + tid] = o;
+    if (xq_out) xq_store_chunk(xq_out + (size_t)sq * xq_bytes((size_t)n_heads * D), (head * D + tid) >> 4, o);
+  }
+}
+
+hipError_t attn_multi_direct_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos,
+                                    const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st) {
+  if (n_kv == 0 || n_heads % n_kv || !pos || !slot || n_seq == 0 || n_splits == 0 || n_splits > 32 || !attn_shape_has_fast_kernel(head_dim, n_heads / n_kv)) return hipErrorInvalidValue;
+#define LGH_AMD(DD, WW)                                                                                                                                                          \
+  if (head_dim == DD && attn_multi_waves(max_seq) == WW) {                                                                                                                       \
+    hipLaunchKernelGGL((attn_multi_direct_kernel<DD, WW>), dim3(n_heads, n_seq), dim3(1024), 0, st, q, kcache, vcache, n_kv, n_heads / n_kv, max_seq, scale, pos, slot, slot_stride, \
+                       n_splits, out, xq_out);                                                                                                                                   \
+    return hipGetLastError();                                                                                                                                                    \
+  }
+  LGH_AMD(128, 4) LGH_AMD(128, 8) LGH_AMD(64, 4) LGH_AMD(64, 8)
+#undef LGH_AMD
+  return hipErrorInvalidValue;
+}
+
 }  // namespace lgh

@@ -226,6 +226,8 @@ hipError_t argmax_multi_launch(const float* logits, uint32_t n, uint32_t n_seq, 
 hipError_t attn_multi_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                              uint32_t max_seq, float scale, const int* pos, const int* slot, uint64_t slot_stride, uint32_t n_seq,
                              uint32_t n_splits, float* part_ml, float* part_acc, hipStream_t st);
+hipError_t attn_multi_direct_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos,
+                                    const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st);
 hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq,
                                      const int* pos, uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st);
 // the rest of the per-op Backend surface (misc.hip): op = 0 add, 1 mul, 2 scale, 3 silu, 4 gelu

@@ -86,7 +86,8 @@ struct BatchScratch {
   float *moe_act = nullptr, *moe_tmp = nullptr;
   int *moe_cnt = nullptr, *moe_idx = nullptr;
   std::vector<size_t> pos;                            // per slot: tokens in its cache
-  hipGraphExec_t graph[kMaxBatch + 1][2] = {};        // [n_seq][0 logits only, 1 + arg-max fed back]
+  bool attn_short = false;                            // attention of the step being enqueued: one launch (chosen by the longest sequence's position), or split and merge; the same bits
+  hipGraphExec_t graph[kMaxBatch + 1][2][2] = {};     // [n_seq][0 logits only, 1 + arg-max fed back][attn_short]
 };
 
 struct LayeredModel;   // layered.hip: models described layer by layer

@@ -792,8 +792,9 @@ static void drop_graphs(lgh_ctx* c) {
     for (int v = 0; v < 2; v++)
       if (c->graph[m][v]) { (void)hipGraphExecDestroy(c->graph[m][v]); c->graph[m][v] = nullptr; }
   for (auto& gg : c->batch.graph)
-    for (auto& ge : gg)
-      if (ge) { (void)hipGraphExecDestroy(ge); ge = nullptr; }
+    for (auto& gs : gg)
+      for (auto& ge : gs)
+        if (ge) { (void)hipGraphExecDestroy(ge); ge = nullptr; }
 }
 
 static int bind(const lgh_ctx* c) { return hipSetDevice(c->device) == hipSuccess ? LGH_OK : LGH_NOT_AVAILABLE; }
@@ -1574,8 +1575,9 @@ void lgh_destroy(lgh_ctx* c) {
   for (auto& r : c->prof) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
   for (void* p : c->allocs) (void)hipFree(p);
   for (auto& gg : c->batch.graph)
-    for (auto& ge : gg)
-      if (ge) (void)hipGraphExecDestroy(ge);
+    for (auto& gs : gg)
+      for (auto& ge : gs)
+        if (ge) (void)hipGraphExecDestroy(ge);
   if (c->batch.h_ctl) (void)hipHostFree(c->batch.h_ctl);
   if (c->pf.tok_pinned) (void)hipHostFree(c->pf.tok_pinned);
   if (c->pf.tok_copied) (void)hipEventDestroy(c->pf.tok_copied);

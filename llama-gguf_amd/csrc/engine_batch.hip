@@ -232,6 +232,15 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       }
       for (uint32_t s = 0; s < n_seq; s++)
         if (XqBuf* q = view_of(c, Bs.attn_out + (size_t)s * QD)) { q->fresh = true; q->tag = nullptr; }
+    } else if (Bs.attn_short) {
+      XqBuf* qa = view_of(c, Bs.attn_out);
+      if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
+             return attn_multi_direct_launch(Bs.q, Bs.kcache[li], Bs.vcache[li], d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, Bs.d_pos, Bs.d_slot, Bs.cache_stride, n_seq,
+                                             c->n_splits, Bs.attn_out, qa->xq, c->stream);
+           })))
+        return rc;
+      for (uint32_t s = 0; s < n_seq; s++)
+        if (XqBuf* q = view_of(c, Bs.attn_out + (size_t)s * QD)) { q->fresh = true; q->tag = nullptr; }
     } else {
     if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
            return attn_multi_launch(Bs.q, Bs.kcache[li], Bs.vcache[li], d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, Bs.d_pos, Bs.d_slot,
@@ -378,14 +387,33 @@ int stage_control(lgh_ctx* c, const uint32_t* slots, const uint32_t* tokens, uin
   return LGH_OK;
 }
 
-int run_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
+// Rows of the longest sequence up to which a step's attention over f32 slots is one launch (attn_multi_direct_kernel: a workgroup per query head and sequence, 4096 values of rows a step of its waves).  The line
+// goes by how many of them there are: few leave the chip to one head's rows each.  us a step of 4 layers, split and merge against one launch, 32/8 heads of 128:
+//   sequences        1              2              4              8              16
+//   30 rows      256  245      305  289      343  322      407  384      537  516
+//   120          256  252      306  300      347  337      413  395      559  535
+//   250          259  268      312  324      356  355      435  411      593  559
+//   500          262  283      316  342      363  367      451  421      627  592
+//   1000         263  314      321  364      372  388      464  461      653  678
+// (32/4 heads of 64, 8 layers, 2 / 8 / 16 sequences: 30 rows 448 406, 568 478, 677 592; 500 rows 461 504, 587 561, 779 713; 1000 rows 466 519, 600 567, 806 769.  Capacities from 2048 rows on, whose splits
+// have eight waves, 4 layers of 32/8 heads of 128, 2 / 8 / 16 sequences: 30 rows 311 290, 457 386, 585 516; 500 rows 322 366, 467 449, 667 628; 1000 rows 328 381, 486 467, 714 676.)
+size_t short_attn_rows(const lgh_ctx* c, uint32_t n_seq) {
+  const lgh_model_desc& d = c->d;
+  if (kv_is_tq(d.kv_cache_type)) return 0;
+  const uint32_t wgs = d.num_heads * n_seq, steps = wgs >= (uint32_t)kNumCU ? 24 : wgs >= (uint32_t)kNumCU / 2 ? 8 : 4;
+  return (size_t)steps * 4096 / d.head_dim;
+}
+
+// one step; `longest`: the largest position among its sequences
+int run_multi(lgh_ctx* c, uint32_t n_seq, bool greedy, size_t longest) {
   BatchScratch& Bs = c->batch;
+  Bs.attn_short = longest + 1 <= short_attn_rows(c, n_seq);
   if (c->profiling || (c->d.flags & LGH_FLAG_NO_GRAPH)) {
     int rc = enqueue_multi(c, n_seq, greedy);
     if (rc) return rc;
     return c->profiling ? drain_prof(c) : LGH_OK;
   }
-  hipGraphExec_t& ge = Bs.graph[n_seq][greedy ? 1 : 0];
+  hipGraphExec_t& ge = Bs.graph[n_seq][greedy ? 1 : 0][Bs.attn_short ? 1 : 0];
   if (!ge) {
     hipGraph_t g = nullptr;
     HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -399,6 +427,12 @@ int run_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
   }
   HIP_TRYB(c, LGH_OPERATION_FAILED, hipGraphLaunch(ge, c->stream));
   return LGH_OK;
+}
+
+size_t longest_of(const lgh_ctx* c, const uint32_t* slots, uint32_t n_seq) {
+  size_t p = 0;
+  for (uint32_t i = 0; i < n_seq; i++) p = std::max(p, c->batch.pos[slots[i]]);
+  return p;
 }
 
 int check_batch(lgh_ctx* c) {
@@ -517,7 +551,12 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
   for (uint32_t i = 0; i < (uint32_t)kMaxBatch; i++) slots0[i] = i;
   for (uint32_t n : {1u, 2u, 3u, 4u, 5u, 9u, 13u}) {
     if (n > max_batch) break;
+    Bs.attn_short = false;
     if ((rc = stage_control(c, slots0, toks0, n)) || (rc = enqueue_multi(c, n, true))) return rc;
+    if (n == 1 && short_attn_rows(c, 1))   // (the single-launch attention's kernel is the same for every size; attn_out is scratch here)
+      HIP_TRYB(c, LGH_OPERATION_FAILED,
+               attn_multi_direct_launch(Bs.q, Bs.kcache[c->l0], Bs.vcache[c->l0], d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, 1.0f, Bs.d_pos, Bs.d_slot, Bs.cache_stride, 1, c->n_splits,
+                                        Bs.attn_out, nullptr, c->stream));
     HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
   }
   return LGH_OK;
@@ -541,7 +580,7 @@ int lgh_forward_multi(lgh_ctx* c, const uint32_t* slots, const uint32_t* tokens,
   if (rc) return rc;
   if (!slots || !tokens) return fail(c, LGH_INVALID_ARGUMENT, "slots / tokens is NULL");
   if ((rc = stage_control(c, slots, tokens, n_seq))) return rc;
-  if ((rc = run_multi(c, n_seq, next_tokens != nullptr))) return rc;
+  if ((rc = run_multi(c, n_seq, next_tokens != nullptr, longest_of(c, slots, n_seq)))) return rc;
   BatchScratch& Bs = c->batch;
   if (logits_out)
     HIP_TRYB(c, LGH_OPERATION_FAILED, hipMemcpyAsync(logits_out, Bs.logits, (size_t)n_seq * c->d.vocab_size * 4, hipMemcpyDeviceToHost, c->stream));
@@ -563,7 +602,7 @@ int lgh_decode_greedy_multi(lgh_ctx* c, const uint32_t* slots, const uint32_t* f
   if (n_steps > c->d.max_seq_len) return fail(c, LGH_INVALID_ARGUMENT, "too many steps");
   if ((rc = stage_control(c, slots, first_tokens, n_seq))) return rc;
   for (size_t st = 0; st < n_steps; st++) {
-    if ((rc = run_multi(c, n_seq, true))) return rc;
+    if ((rc = run_multi(c, n_seq, true, longest_of(c, slots, n_seq) + st))) return rc;
     if (tokens_out)
       HIP_TRYB(c, LGH_OPERATION_FAILED, hipMemcpyAsync(Bs.d_log + st * kMaxBatch, Bs.d_tokens, (size_t)n_seq * 4, hipMemcpyDeviceToDevice, c->stream));
   }
