@@ -59,6 +59,14 @@ struct PfwScratch {
   uint32_t moe_tiles = 0;
 };
 
+// pinned memory through which results reach the caller (engine.hip: floats_to_host)
+constexpr int kOutSlots = 4;
+struct HostOut {
+  float *pin = nullptr, *dev = nullptr;   // the same memory, as the host and as the device sees it
+  hipEvent_t ready[kOutSlots] = {};
+  bool refused = false;                   // there is none: the runtime's own copies
+};
+
 struct ProfRec { int cls; int sym; uint64_t bytes; hipEvent_t a, b; };
 
 // multi-sequence decode (engine_batch.hip): `max_batch` slots, each one sequence's KV caches and position, and the vectors of
@@ -133,6 +141,7 @@ struct lgh_ctx {
   lgh::PfScratch pf;
   lgh::PfwScratch pfw;
   lgh::BatchScratch batch;
+  lgh::HostOut out;
   float* tq_signs = nullptr;                   // TurboQuant KV cache: [owned layer][kv head][k, v][head_dim] rotation signs (device)
   std::vector<float> tq_signs_host;
   float* tq_qjl = nullptr;                     // TurboQuantProd: [owned layer][kv head][head_dim][head_dim] QJL projection matrices (device)
@@ -191,6 +200,7 @@ void xq_stale(lgh_ctx* c, const float* f32);
 int linear_any(lgh_ctx* c, int cls, const lgh::DevWeight& W, const float* x, float* out, const float* norm_w,
                const float* resid, const float* bias, int xq_next = 0, const float* xq_next_nw = nullptr);
 int drain_prof(lgh_ctx* c);
+int floats_to_host(lgh_ctx* c, float* dst, const float* src, size_t cols, size_t ld, size_t rows);
 // layered.hip, behind the entry points of engine.hip when c->lm is set
 int layered_upload(lgh_ctx* c, const char* name, uint32_t type, const uint64_t ne[4], const void* host, size_t nbytes);
 int layered_finalize(lgh_ctx* c);

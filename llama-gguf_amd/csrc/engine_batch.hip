@@ -582,8 +582,7 @@ int lgh_forward_multi(lgh_ctx* c, const uint32_t* slots, const uint32_t* tokens,
   if ((rc = stage_control(c, slots, tokens, n_seq))) return rc;
   if ((rc = run_multi(c, n_seq, next_tokens != nullptr, longest_of(c, slots, n_seq)))) return rc;
   BatchScratch& Bs = c->batch;
-  if (logits_out)
-    HIP_TRYB(c, LGH_OPERATION_FAILED, hipMemcpyAsync(logits_out, Bs.logits, (size_t)n_seq * c->d.vocab_size * 4, hipMemcpyDeviceToHost, c->stream));
+  if (logits_out && (rc = floats_to_host(c, logits_out, Bs.logits, (size_t)n_seq * c->d.vocab_size, (size_t)n_seq * c->d.vocab_size, 1))) return rc;
   if (next_tokens) HIP_TRYB(c, LGH_OPERATION_FAILED, hipMemcpyAsync(next_tokens, Bs.d_tokens, (size_t)n_seq * 4, hipMemcpyDeviceToHost, c->stream));
   HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
   for (uint32_t i = 0; i < n_seq; i++) Bs.pos[slots[i]] += 1;

@@ -1333,9 +1333,7 @@ static int block_pass(lgh_ctx* c, const uint32_t* tokens, uint32_t M, const uint
          })))
       return rc;
     if ((rc = block_gemm(c, LGH_K_OUTPUT, m.head, LE_F32, m.bla, ldx, m.blogits, ldl, n, nullptr, (float)d.logit_cap))) return rc;
-    L_TRY(c, LGH_OPERATION_FAILED, hipMemcpy2DAsync(logits_out + (size_t)w * d.vocab_size, (size_t)d.vocab_size * 4, m.blogits, (size_t)ldl * 4,
-                                                    (size_t)d.vocab_size * 4, n, hipMemcpyDeviceToHost, st));
-    L_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(st));
+    if ((rc = floats_to_host(c, logits_out + (size_t)w * d.vocab_size, m.blogits, d.vocab_size, ldl, n))) return rc;
   }
   c->pos += M;
   c->stats.tokens_processed += M;

@@ -338,7 +338,8 @@ hipError_t moe_combine_launch(const float* tmp, const float* moe_w, uint32_t top
   return hipGetLastError();
 }
 
-// same-device pipeline hop (hidden vector / token word) as a graph node of the producing stage
+// same-device pipeline hop (hidden vector / token word) as a graph node of the producing stage; results on their way to pinned host memory.  (One word a lane: a wave's store is
+// 256 bytes either way, and neither side need be aligned to more.)
 __global__ void copy_words_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
