@@ -108,6 +108,8 @@ struct lgh_ctx {
   uint32_t l0 = 0, l1 = 0;
   bool first = true, last = true;
   hipStream_t own_stream = nullptr, stream = nullptr;
+  hipStream_t side_stream = nullptr;                  // the token behind a prompt block (engine.hip: tail_layer)
+  hipEvent_t side_go = nullptr, side_done = nullptr;
   std::vector<lgh::LayerW> layers;
   // embedding table in native GGUF layout (row-dequantized per token) and the output projection
   uint8_t* embd_raw = nullptr;

@@ -662,9 +662,8 @@ static int layer_forward(lgh_ctx* c, uint32_t li, const float* next_nw, bool nex
   return ffn_forward(c, Lw, FfnView{c->hidden, c->act, c->act2, c->xnorm, c->moe_sel, c->moe_w}, next_nw, next_mfma);
 }
 
-// Everything one token needs, in stream order.  Used eagerly and under graph capture.
-static int enqueue_token(lgh_ctx* c, int mode) {
-  if (c->lm) return layered_enqueue_token(c, mode);
+// the token's embedding row (or the hidden vector that the stage before left) and its position
+static int token_begin(lgh_ctx* c) {
   const lgh_model_desc& d = c->d;
   int rc;
   for (auto& q : c->xqs) q.fresh = false;   // the residual stream is (re)written in f32 now (embedding / previous stage)
@@ -685,20 +684,28 @@ static int enqueue_token(lgh_ctx* c, int mode) {
   } else {
     if ((rc = run_k(c, LGH_K_MISC, LGH_SYM_OTHER, 0, [&] { return advance_launch(c->state, c->stream); }))) return rc;
   }
-  for (uint32_t li = c->l0; li < c->l1; li++) {
-    // who consumes this layer's output: the next layer's QKV (attn_norm), the output projection (output_norm), or — at a
-    // pipeline-stage boundary and at the end of a prefill step — nobody on this device
-    const float* next_nw = nullptr;
-    bool next_mfma = false;
-    if (li + 1 < c->l1) {
-      next_nw = c->layers[li + 1].attn_norm;
-      next_mfma = mfma_type(c->layers[li + 1].wq.type);
-    } else if (c->last && mode != MODE_PREFILL) {
-      next_nw = c->output_norm;
-      next_mfma = mfma_type(c->output.type);
-    }
-    if ((rc = layer_forward(c, li, next_nw, next_mfma, mode))) return rc;
+  return LGH_OK;
+}
+
+static int token_layer(lgh_ctx* c, uint32_t li, int mode) {
+  // who consumes this layer's output: the next layer's QKV (attn_norm), the output projection (output_norm), or — at a
+  // pipeline-stage boundary and at the end of a prefill step — nobody on this device
+  const float* next_nw = nullptr;
+  bool next_mfma = false;
+  if (li + 1 < c->l1) {
+    next_nw = c->layers[li + 1].attn_norm;
+    next_mfma = mfma_type(c->layers[li + 1].wq.type);
+  } else if (c->last && mode != MODE_PREFILL) {
+    next_nw = c->output_norm;
+    next_mfma = mfma_type(c->output.type);
   }
+  return layer_forward(c, li, next_nw, next_mfma, mode);
+}
+
+// the logits, the greedy token and the in-graph hops
+static int token_end(lgh_ctx* c, int mode) {
+  const lgh_model_desc& d = c->d;
+  int rc;
   if (c->last && mode != MODE_PREFILL) {
     // compute_logits (llama.rs:247-266): final RMSNorm fused into the output projection
     if ((rc = linear_any(c, LGH_K_OUTPUT, c->output, c->hidden, c->logits, c->output_norm, nullptr, nullptr))) return rc;
@@ -717,6 +724,16 @@ static int enqueue_token(lgh_ctx* c, int mode) {
       (rc = run_k(c, LGH_K_MISC, LGH_SYM_OTHER, 8, [&] { return copy_words_launch(c->fwd_token, c->state + ST_ARGMAX, 1, c->stream); })))
     return rc;
   return LGH_OK;
+}
+
+// Everything one token needs, in stream order.  Used eagerly and under graph capture.
+static int enqueue_token(lgh_ctx* c, int mode) {
+  if (c->lm) return layered_enqueue_token(c, mode);
+  int rc;
+  if ((rc = token_begin(c))) return rc;
+  for (uint32_t li = c->l0; li < c->l1; li++)
+    if ((rc = token_layer(c, li, mode))) return rc;
+  return token_end(c, mode);
 }
 
 // One token through the context's kernels, launched eagerly, before any of them is first launched inside a stream
@@ -960,11 +977,82 @@ static int pf_stage_tokens(lgh_ctx* c, const uint32_t* tokens, uint32_t m, int* 
   return LGH_OK;
 }
 
+// ---- the token behind a block, beside it ----
+// The token whose logits a prompt is for takes the decode step.  Of the block before it, its layer li needs nothing but the K / V rows of layer li: the step's layers follow
+// the block's on a stream of their own, each behind an event that says that the block has written that layer's rows.  The two share no scratch, and neither reads a cache row that the
+// other writes while it runs (the block its own rows and those before them, the step its one row behind them besides).  The same kernels on the same values: the same bits.
+struct PfTail { uint32_t token; size_t pos; bool taken = false; };   // at position pos; taken: its step is under way
+
+// A process's streams share a few hardware queues, and two streams in one queue run one after the other: then the events between them cost a layer some 8 us and nothing is gained (8 layers of an 8B
+// model, 300 tokens: 2.43 -> 2.50 ms).  Which queue a stream gets is the runtime's affair, so it is tried: a kernel on the context's stream waits, some 200 us at most, for what one on the other says.
+__global__ void side_wait_kernel(int* w) {
+  for (int i = 0; i < 150; i++) {
+    if (__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) { w[1] = 1; return; }
+    __builtin_amdgcn_s_sleep(8);
+  }
+  w[1] = 0;
+}
+__global__ void side_say_kernel(int* w, int v) { __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// c->side_stream beside c->stream, if there is one to be had; without it a prompt's last token follows its block
+static void side_make(lgh_ctx* c) {
+  hipStream_t tried[4] = {};
+  int n = 0, *w = nullptr, seen = 0;
+  bool ok = hipEventCreateWithFlags(&c->side_go, hipEventDisableTiming) == hipSuccess && hipEventCreateWithFlags(&c->side_done, hipEventDisableTiming) == hipSuccess &&
+            hipMalloc((void**)&w, 8) == hipSuccess;
+  while (ok && !seen && n < 4) {
+    ok = hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) == hipSuccess;
+    if (!ok) break;
+    hipStream_t s = tried[n++];
+    for (int pass = 0; pass < 2 && ok; pass++) {   // (the first launches on a stream take longer)
+      hipLaunchKernelGGL(side_say_kernel, dim3(1), dim3(1), 0, s, w, 0);
+      ok = hipStreamSynchronize(s) == hipSuccess;
+      hipLaunchKernelGGL(side_wait_kernel, dim3(1), dim3(1), 0, c->stream, w);
+      hipLaunchKernelGGL(side_say_kernel, dim3(1), dim3(1), 0, s, w, 1);
+      ok = ok && hipStreamSynchronize(s) == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess;
+    }
+    ok = ok && hipMemcpy(&seen, w + 1, 4, hipMemcpyDeviceToHost) == hipSuccess;
+  }
+  if (ok && seen) c->side_stream = tried[--n];
+  while (n > 0) (void)hipStreamDestroy(tried[--n]);
+  if (w) (void)hipFree(w);
+  if (!ok) (void)hipGetLastError();   // (the next launch's check would find it)
+}
+
+// (no stream of the caller's, no recording of launch times, no context that wants its launches one after the other, no model whose steps are not built layer by layer here)
+static bool tail_eligible(const lgh_ctx* c) { return c->side_stream && c->stream == c->own_stream && !c->lm && c->first && c->last && !c->profiling && !(c->d.flags & LGH_FLAG_NO_GRAPH) && pf_eligible(c); }
+
+// the block's rows of layer li are under way on c->stream: the token's layer li behind them
+static int tail_layer(lgh_ctx* c, const PfTail& t, uint32_t li) {
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipEventRecord(c->side_go, c->stream));
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamWaitEvent(c->side_stream, c->side_go, 0));
+  hipStream_t main = c->stream;
+  c->stream = c->side_stream;
+  int rc = LGH_OK;
+  if (li == c->l0) {
+    if (hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)t.pos, 1, c->stream) != hipSuccess) rc = fail(c, LGH_OPERATION_FAILED, "token behind a block: position");
+    if (!rc && !(rc = set_token(c, t.token))) rc = token_begin(c);
+  }
+  if (!rc) rc = token_layer(c, li, MODE_FORWARD);
+  if (!rc && li + 1 == c->l1) rc = token_end(c, MODE_FORWARD);
+  c->stream = main;
+  return rc;
+}
+
+static int tail_end(lgh_ctx* c, PfTail& t) {
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipEventRecord(c->side_done, c->side_stream));
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamWaitEvent(c->stream, c->side_done, 0));
+  c->pos += 1;
+  c->stats.tokens_processed += 1;
+  t.taken = true;
+  return LGH_OK;
+}
+
 // m <= 128 prompt tokens at positions pos .. pos+m-1: fills every owned layer's K/V rows.  The first stage starts from the
 // tokens' embedding rows, any other stage from the block of hidden vectors its predecessor left in pf.hidden; a stage that
 // is not the last leaves its output block there (the last one stops after its final layer's K/V rows: nothing else of a
 // prefill survives).
-static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
+static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail* tail = nullptr) {
   int rc = pf_ensure(c);
   if (rc) return rc;
   PfScratch& P = c->pf;
@@ -990,6 +1078,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
                                   d.norm_eps, (int)d.use_neox_rope, m, st),
                 "qkv epilogue")))
       return rc;
+    if (tail && (rc = tail_layer(c, *tail, li))) return rc;
     if (li + 1 == c->l1 && c->last) break;   // the model's last layer: its K/V rows are written, its output would be discarded
     if ((rc = K(attn_prefill_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.xh_attn, st),
                 "attention")))
@@ -1040,6 +1129,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
   }
   c->pos += m;
   c->stats.tokens_processed += m;
+  if (tail) return tail_end(c, *tail);
   HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
   return LGH_OK;
 }
@@ -1122,7 +1212,7 @@ static bool pfw_ensure(lgh_ctx* c, size_t rows) {
 }
 
 // m prompt tokens at positions pos .. pos + m - 1 through every layer of a single-stage context: its K / V rows
-static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
+static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail* tail = nullptr) {
   PfwScratch& P = c->pfw;
   const lgh_model_desc& d = c->d;
   const uint32_t H = d.hidden_size, QD = d.num_heads * d.head_dim, KD = d.num_kv_heads * d.head_dim, pos0 = (uint32_t)c->pos;
@@ -1164,6 +1254,7 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
     if ((rc = product({&L.wq, &L.wk, &L.wv}, P.x, G, PW_PART, m, nullptr, "qkv product"))) return rc;
     const PfwQkv e{P.part, G.S, G.part_rows, QD, KD, d.head_dim, L.bq, L.bk, L.bv, c->rope_cs, P.inv_rms, pos0, d.max_seq_len, P.q, L.kcache, L.vcache, (int)d.use_neox_rope};
     if ((rc = K(pfw_qkv_launch(e, m, st), "qkv"))) return rc;
+    if (tail && (rc = tail_layer(c, *tail, li))) return rc;
     if (li + 1 == c->l1) break;   // the last layer: its K / V rows are written, its output would be discarded
     if ((rc = K(attn_wide_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.kv_split, P.part, P.part_bytes, P.attn, st), "attention"))) return rc;
     G = PfWide{};
@@ -1206,24 +1297,31 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m) {
   }
   c->pos += m;
   c->stats.tokens_processed += m;
+  if (tail) return tail_end(c, *tail);
   HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
   return LGH_OK;
 }
 
-// n prompt tokens on the batched path
-static int prefill_tokens(lgh_ctx* c, const uint32_t* tokens, size_t n) {
+// The token behind a block goes beside it up to this much of one: the larger the products, the less of the chip they leave, and the less a step is of the whole.  The block and then the step against
+// both side by side, ms: 8B widths, 8 layers in Q4_K_M, 170 tokens 2.25 and 2.06, 600: 3.58 and 3.34, 1300: 6.49 and 6.27, 2047: 8.43 and 8.50; 4 layers in Q8_0, 600: 1.75 and 1.65, 2047: 3.92 and 3.91;
+// TinyLlama, 600: 4.79 and 4.35, 2047: 10.0 and 9.5; Mixtral widths, 2 layers, 600: 1.22 and 1.17, 2047: 2.58 and 2.53.  In blocks of 128, 8B widths, 10 tokens 0.99 and 0.83, 65: 1.18 and 1.06,
+// 129: 1.44 and 1.34.
+static bool tail_pays(const lgh_ctx* c, uint32_t m) { return (uint64_t)m * c->d.hidden_size <= 1536u * 4096u; }
+
+// n prompt tokens on the batched path; `tail`: the token behind them, beside the last of their blocks
+static int prefill_tokens(lgh_ctx* c, const uint32_t* tokens, size_t n, PfTail* tail = nullptr) {
   int rc;
   size_t i = 0;
   const size_t least = pfw_min_tokens(c);
   if (n >= least && pfw_eligible(c) && pfw_ensure(c, c->pos + n)) {
     while (n - i >= least) {
       const uint32_t m = (uint32_t)std::min<size_t>(c->pfw.cap, n - i);
-      if ((rc = prefill_wide(c, tokens + i, m))) return rc;
+      if ((rc = prefill_wide(c, tokens + i, m, i + m == n && tail_pays(c, m) ? tail : nullptr))) return rc;
       i += m;
     }
   }
   for (; i < n; i += kPfTokens)
-    if ((rc = prefill_block(c, tokens + i, (uint32_t)std::min<size_t>(kPfTokens, n - i)))) return rc;
+    if ((rc = prefill_block(c, tokens + i, (uint32_t)std::min<size_t>(kPfTokens, n - i), i + kPfTokens >= n ? tail : nullptr))) return rc;
   return LGH_OK;
 }
 
@@ -1622,7 +1720,9 @@ int lgh_finalize(lgh_ctx* c) {
   HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
   c->finalized = true;
   c->pos = 0;
-  return warm_kernels(c);
+  if ((rc = warm_kernels(c))) return rc;
+  if (c->first && c->last && !(d.flags & LGH_FLAG_NO_GRAPH) && pf_eligible(c)) side_make(c);
+  return LGH_OK;
 }
 
 void lgh_destroy(lgh_ctx* c) {
@@ -1644,6 +1744,9 @@ void lgh_destroy(lgh_ctx* c) {
   if (c->out.pin) (void)hipHostFree(c->out.pin);
   for (auto& e : c->out.ready)
     if (e) (void)hipEventDestroy(e);
+  if (c->side_go) (void)hipEventDestroy(c->side_go);
+  if (c->side_done) (void)hipEventDestroy(c->side_done);
+  if (c->side_stream) (void)hipStreamDestroy(c->side_stream);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   layered_destroy(c);
   delete c;
@@ -1719,6 +1822,21 @@ int lgh_prefill_batch(lgh_ctx* c, const uint32_t* tokens, size_t n) {
   return LGH_OK;
 }
 
+// n tokens as blocks and the token behind them, whose logits are wanted
+static int eval_stretch(lgh_ctx* c, const uint32_t* tokens, size_t n, uint32_t token, float* logits_out) {
+  PfTail t{token, c->pos + n};
+  c->attn_direct = t.pos + 1 <= direct_attn_rows(c);
+  int rc = prefill_tokens(c, tokens, n, &t);
+  if (!rc && !t.taken && !(rc = set_token(c, token))) rc = step(c, MODE_FORWARD);
+  if (rc) {
+    (void)hipStreamSynchronize(c->side_stream);   // nothing of the call goes on behind its error, and the next token's position is the one behind what is there
+    (void)hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, c->stream);
+    (void)hipStreamSynchronize(c->stream);
+    return rc;
+  }
+  return floats_to_host(c, logits_out, c->logits, c->d.vocab_size, c->d.vocab_size, 1);
+}
+
 int lgh_eval(lgh_ctx* c, const uint32_t* tokens, size_t n, const uint32_t* want, size_t n_want, float* logits_out) {
   int rc = check_ready(c);
   if (rc) return rc;
@@ -1735,8 +1853,13 @@ int lgh_eval(lgh_ctx* c, const uint32_t* tokens, size_t n, const uint32_t* want,
   size_t at = 0;
   for (size_t i = 0; i < n_want; i++) {
     const size_t len = want[i] - at;
-    if (len && (rc = lgh_prefill_batch(c, tokens + at, len))) return rc;
-    if ((rc = lgh_forward(c, tokens[want[i]], logits_out + i * (size_t)c->d.vocab_size))) return rc;
+    float* out = logits_out + i * (size_t)c->d.vocab_size;
+    if (len >= 2 && tail_eligible(c)) {
+      if ((rc = eval_stretch(c, tokens + at, len, tokens[want[i]], out))) return rc;
+    } else {
+      if (len && (rc = lgh_prefill_batch(c, tokens + at, len))) return rc;
+      if ((rc = lgh_forward(c, tokens[want[i]], out))) return rc;
+    }
     at = want[i] + 1;
   }
   if (at < n) return lgh_prefill_batch(c, tokens + at, n - at);

@@ -1,0 +1,43 @@
+"""The token behind a prompt block, whose step runs beside the block (engine.hip, tail_layer), against the block and then the step: all bits equal, its own logits and those of the tokens after it.  Portions
+around one block (128 tokens) and a remainder of one token, from nothing and behind earlier tokens, several wanted places, short and long contexts (the two forms of attention), mixtures, a context with slots."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("model,mix,max_seq,slots", [
+    ("test-dense", "Q4_K_M", 700, 0),
+    ("test-dense-d128", "Q8_0", 700, 0),
+    ("test-dense-d128", "Q5_K_M", 5000, 2),
+    ("test-moe", "Q5_K_M", 700, 0),
+])
+def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
+    cfg = pkg.make_config(model, max_seq_len=max_seq)
+    m = pkg.SynthModel(cfg, mix=mix)
+    beside, behind = (pkg.HipGpuInference.from_model(m, max_seq) for _ in range(2))
+    assert beside.prefill_is_batched()
+    if slots:
+        beside.batch_create(slots)
+        behind.batch_create(slots)
+    tok = np.random.default_rng(5).integers(0, cfg.vocab_size, 700).astype(np.uint32)
+    for before, portion in ((0, (3,)), (0, (17,)), (0, (129,)), (0, (130,)), (5, (64, 3, 1, 130)), (0, (258,)), (0, (300, 40)), (160, (150,))):
+        beside.reset()
+        behind.reset()
+        if before:
+            beside.forward_batch(tok[:before])
+            behind.forward_batch(tok[:before])
+        n = sum(portion)
+        got = beside.eval(tok[before:before + n], [int(v) - 1 for v in np.cumsum(portion)])
+        at = before
+        for i, length in enumerate(portion):
+            if length > 1:
+                behind.forward_batch(tok[at:at + length - 1])
+            want = behind.forward(int(tok[at + length - 1]))
+            at += length
+            assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), (before, portion, i)
+        assert beside.position() == behind.position() == at
+        for t in (4, 9):
+            assert np.array_equal(beside.forward(t).view(np.uint32), behind.forward(t).view(np.uint32)), (before, portion)
+    beside.close()
+    behind.close()
