@@ -514,20 +514,24 @@ template <class T> constexpr uint32_t act_chunks() { return 64 * sizeof(T) / 16;
 // 78 -> 53 us, 2048 -> 2048 33 -> 22; 128 x 128 tiles have room for two and gain the barrier that is gone: 2048 -> 5632 61 -> 57.  One workgroup a CU with four buffers is slower
 // (128 x 128, 192 tiles, 5632 -> 2048: 59 us), and so are three and four buffers of the larger tile (the whole prompt 2650, 2970 us against 2520).
 template <class T, int BM, int BN> constexpr uint32_t lin_step_bytes() { return BN * 128 + BM * act_chunks<T>() * 16; }
-template <class T, int BM, int BN> constexpr int lin_stages() {
-  constexpr uint32_t n = 80u * 1024 / lin_step_bytes<T, BM, BN>();
-  return n < 2 ? 2 : n > 4 ? 4 : (int)n;
+template <class T, int BM, int BN, int TEAMS> constexpr int lin_stages() {
+  constexpr uint32_t n = (TEAMS == 1 ? 80u : 160u) * 1024 / lin_step_bytes<T, BM, BN>();
+  return n < 2 ? 2 : n > (TEAMS == 1 ? 4 : 6) ? (TEAMS == 1 ? 4 : 6) : (int)n;
 }
 
-template <class T, int BM, int BN, int WN, int EPI, bool GRP>
-__global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t tiles_n, uint32_t tiles_m) {
-  constexpr int WM = 4 / WN, NT = BN / WN / 16, MT = BM / WM / 16;
+// TEAMS 2: a CU's only workgroup, eight waves; two teams of four share every k-step's columns and add their sums through LDS at the end.  What bounds it is the loads' way from L2 (28 KB a step of a tile
+// of 96, 0.5 us, four steps under way): a larger tile moves fewer bytes for its products, all LDS keeps more of them in flight, and 256 tiles of one size end together, where 384 smaller ones leave half of the
+// CUs with one and half with two.
+template <class T, int BM, int BN, int WN, int EPI, bool GRP, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS) lin_gemm_kernel(const LinGemm a, uint32_t tiles_n, uint32_t tiles_m) {
+  constexpr int WM = 4 / WN, NT = BN / WN / 16, MT = BM / WM / 16, NWV = 4 * TEAMS;
   constexpr uint32_t XC = act_chunks<T>();
   constexpr uint32_t kWBytes = BN * 128, kXBytes = BM * XC * 16, kBuf = kWBytes + kXBytes;
-  constexpr uint32_t NS = lin_stages<T, BM, BN>();
+  constexpr uint32_t NS = lin_stages<T, BM, BN, TEAMS>();
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t lds0 = lds_addr_of(smem);
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t team = TEAMS == 1 ? 0 : wave >> 2;
   // consecutive tiles of one weight panel on one XCD (workgroups go round-robin over the 8 XCDs)
   uint32_t t = blockIdx.x;
   const uint32_t total = tiles_n * tiles_m;
@@ -546,32 +550,32 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
     m_end = (uint32_t)a.grp.seg[e + 1];
     W += (size_t)e * a.grp.stride;
   }
-  const uint32_t wn = wave % WN, wm = wave / WN;
+  const uint32_t wn = wave % 4 % WN, wm = wave % 4 / WN;
   const uint32_t r16 = lane & 15, g = lane >> 4;
   const T* X = reinterpret_cast<const T*>(a.x);
 
   constexpr uint32_t RPI = 64 / XC;                          // rows of x per wave instruction
-  constexpr int NX = (int)((kXBytes / 1024 + 3) / 4);
+  constexpr int NX = (int)((kXBytes / 1024 + NWV - 1) / NWV);
   uint32_t xrow[GRP ? NX : 1];                               // grouped: where this lane's rows lie
   if constexpr (GRP) {
 #pragma unroll
     for (int i = 0; i < NX; i++) {
-      const uint32_t r = m0 + (i * 4 + wave) * RPI + lane / XC, m = r < m_end ? r : m_end - 1;
+      const uint32_t r = m0 + (i * NWV + wave) * RPI + lane / XC, m = r < m_end ? r : m_end - 1;
       xrow[i] = a.grp.src ? (uint32_t)a.grp.src[m] : m;
     }
   }
   auto stage = [&](uint32_t k0, uint32_t buf) {
     const uint32_t base = lds0 + buf * kBuf;
 #pragma unroll
-    for (int i = 0; i < (int)(kWBytes / 4096); i++) {       // weights: 8 chunks a row, a wave instruction covers 8 rows
-      const uint32_t row = (i * 4 + wave) * 8 + (lane >> 3), ch = (lane & 7) ^ (row & 7);
+    for (int i = 0; i < (int)(kWBytes / (NWV * 1024)); i++) {       // weights: 8 chunks a row, a wave instruction covers 8 rows
+      const uint32_t row = (i * NWV + wave) * 8 + (lane >> 3), ch = (lane & 7) ^ (row & 7);
       const uint32_t n = n0 + row < a.np ? n0 + row : a.np - 1;
-      lds_dma16_untracked(W + (size_t)n * a.kp + k0 + ch * 8, base + (i * 4 + wave) * 1024);
+      lds_dma16_untracked(W + (size_t)n * a.kp + k0 + ch * 8, base + (i * NWV + wave) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NX; i++) {
-      const uint32_t blk = i * 4 + wave;
-      if (kXBytes / 1024 % 4 == 0 || blk < kXBytes / 1024) {
+      const uint32_t blk = i * NWV + wave;
+      if (kXBytes / 1024 % NWV == 0 || blk < kXBytes / 1024) {
         const uint32_t row = blk * RPI + lane / XC, ch = (lane % XC) ^ (row & (XC - 1));
         const uint32_t m = GRP ? xrow[GRP ? i : 0] : m0 + row < a.M ? m0 + row : a.M - 1;
         lds_dma16_untracked(X + (size_t)m * a.ldx + k0 + ch * (16 / sizeof(T)), base + kWBytes + blk * 1024);
@@ -586,7 +590,7 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
     for (int j = 0; j < MT; j++) acc[i][j] = (f32x4)(0.0f);
 
   // a wave issues at least kDma loads a step; all but those of the NS - 2 steps after this one have to be there (a wave that issues one more waits for more than that)
-  constexpr uint32_t kDma = kWBytes / 4096 + kXBytes / 4096;
+  constexpr uint32_t kDma = kWBytes / (NWV * 1024) + kXBytes / (NWV * 1024);
   const uint32_t steps = a.kp / 64;
   for (uint32_t s = 0; s + 1 < NS && s < steps; s++) stage(s * 64, s);
   uint32_t cur = 0, fill = NS - 1;                           // buffer of this step, and of the step NS - 1 after it
@@ -597,17 +601,18 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
     if (s + NS - 1 < steps) stage((s + NS - 1) * 64, fill);
     const uint8_t* wb = smem + cur * kBuf;
     const uint8_t* xb = wb + kWBytes;
-    constexpr int U = 64 / Frag<T>::KU;
+    constexpr int U = 64 / Frag<T>::KU / TEAMS;
 #pragma unroll
-    for (int u = 0; u < U; u++) {
+    for (int ul = 0; ul < U; ul++) {
+      const uint32_t u = team * U + ul;
       typename Frag<T>::V wf[NT], xf[MT];
 #pragma unroll
       for (int i = 0; i < NT; i++) {
         const uint32_t row = (wn * NT + i) * 16 + r16;
         if constexpr (sizeof(T) == 2) {
-          wf[i] = *reinterpret_cast<const bf16x8*>(wb + row * 128 + (((uint32_t)(u * 4) + g) ^ (row & 7)) * 16);
+          wf[i] = *reinterpret_cast<const bf16x8*>(wb + row * 128 + ((u * 4 + g) ^ (row & 7)) * 16);
         } else {   // 4 bf16 values of the 16-column unit: half a chunk
-          const u32x2 h = *reinterpret_cast<const u32x2*>(wb + row * 128 + (((uint32_t)(u * 2) + (g >> 1)) ^ (row & 7)) * 16 + (g & 1) * 8);
+          const u32x2 h = *reinterpret_cast<const u32x2*>(wb + row * 128 + ((u * 2 + (g >> 1)) ^ (row & 7)) * 16 + (g & 1) * 8);
           f32x4 v;
           v.x = bf_lo(h.x); v.y = bf_hi(h.x); v.z = bf_lo(h.y); v.w = bf_hi(h.y);
           wf[i] = v;
@@ -616,7 +621,7 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
 #pragma unroll
       for (int j = 0; j < MT; j++) {
         const uint32_t row = (wm * MT + j) * 16 + r16;
-        xf[j] = Frag<T>::load(reinterpret_cast<const T*>(xb + row * (XC * 16) + (((uint32_t)(u * 4) + g) ^ (row & (XC - 1))) * 16));
+        xf[j] = Frag<T>::load(reinterpret_cast<const T*>(xb + row * (XC * 16) + ((u * 4 + g) ^ (row & (XC - 1))) * 16));
       }
 #pragma unroll
       for (int i = 0; i < NT; i++)
@@ -625,6 +630,22 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
     }
     cur = cur + 1 < NS ? cur + 1 : 0;
     fill = fill + 1 < NS ? fill + 1 : 0;
+  }
+  if constexpr (TEAMS == 2) {   // the second team's sums; the first one's follow in every place
+    __syncthreads();            // every buffer has been read
+    f32x4* red = reinterpret_cast<f32x4*>(smem) + (wave & 3) * (NT * MT * 64) + lane;
+    if (team == 1) {
+#pragma unroll
+      for (int i = 0; i < NT; i++)
+#pragma unroll
+        for (int j = 0; j < MT; j++) red[(i * MT + j) * 64] = acc[i][j];
+    }
+    __syncthreads();
+    if (team == 1) return;
+#pragma unroll
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+      for (int j = 0; j < MT; j++) acc[i][j] += red[(i * MT + j) * 64];
   }
   // lane: token r16 of a token tile, columns 4g .. 4g + 3 of a weight tile
 #pragma unroll
@@ -698,19 +719,31 @@ __global__ void __launch_bounds__(256) lin_gemm_kernel(const LinGemm a, uint32_t
   }
 }
 
-template <class T, int BM, int BN, int WN, int EPI, bool GRP = false>
+template <class T, int BM, int BN, int WN, int EPI, bool GRP = false, int TEAMS = 1>
 static hipError_t lin_gemm_go(const LinGemm& a, hipStream_t st) {
   static bool opted[64] = {};
-  constexpr size_t lds = lin_stages<T, BM, BN>() * (size_t)lin_step_bytes<T, BM, BN>();
-  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&lin_gemm_kernel<T, BM, BN, WN, EPI, GRP>), (int)lds, opted); e != hipSuccess) return e;
+  constexpr size_t lds = lin_stages<T, BM, BN, TEAMS>() * (size_t)lin_step_bytes<T, BM, BN>();
+  static_assert(lds <= 160 * 1024 && (TEAMS == 1 || (size_t)BM * BN * 4 <= lds), "LDS");
+  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&lin_gemm_kernel<T, BM, BN, WN, EPI, GRP, TEAMS>), (int)lds, opted); e != hipSuccess) return e;
   const uint32_t tn = (a.n + BN - 1) / BN, tm = GRP ? a.grp.tiles : (a.M + BM - 1) / BM;
-  hipLaunchKernelGGL((lin_gemm_kernel<T, BM, BN, WN, EPI, GRP>), dim3(tn * tm), dim3(256), lds, st, a, tn, tm);
+  hipLaunchKernelGGL((lin_gemm_kernel<T, BM, BN, WN, EPI, GRP, TEAMS>), dim3(tn * tm), dim3(256 * TEAMS), lds, st, a, tn, tm);
   return hipGetLastError();
 }
 
 template <class T, int EPI>
 static hipError_t lin_gemm_pick(const LinGemm& a, hipStream_t st) {
   const uint32_t tn = (a.n + 127) / 128;
+  // More tiles of 32 rows than CUs, and tiles of 64 to 128 that give every CU one at most: two teams, with all of the CU's LDS for steps under way (tiles of 128 only where few CUs go without).
+  // Two small workgroups a CU against these, us, bf16: 5632 -> 2048 columns, 768 tokens 37.0 and 33.4, 1501: 54.8 and 44.8; 2048 -> 2048, 1501: 22.3 and 21.1; 4096 -> 4096, 300: 28.3 and 25.7,
+  // 1000: 46.2 and 44.0; 14336 -> 4096, 300: 104.6 and 95.9, 768: 168 and 120, 1000: 191 and 139.  With 192 tiles of 128 23.0 and 23.7 (2048 -> 3072, 1000), with up to 256 of 32 26.7 and 26.1 (5632 -> 2048, 300).
+  if constexpr (EPI == LE_F32 && sizeof(T) == 2) {
+    auto tiles = [&](uint32_t bm) { return tn * ((a.M + bm - 1) / bm); };
+    if (a.kp >= 1024 && tiles(32) > kNumCU) {
+      if (tiles(64) <= kNumCU) return lin_gemm_go<T, 64, 128, 2, EPI, false, 2>(a, st);
+      if (tiles(96) <= kNumCU) return lin_gemm_go<T, 96, 128, 2, EPI, false, 2>(a, st);
+      if (tiles(128) <= kNumCU && tiles(128) >= 224) return lin_gemm_go<T, 128, 128, 2, EPI, false, 2>(a, st);
+    }
+  }
   if (a.M > 64 && tn * ((a.M + 127) / 128) >= 224) return lin_gemm_go<T, 128, 128, 2, EPI>(a, st);
   if (a.M > 32 && tn * ((a.M + 63) / 64) >= 160) return lin_gemm_go<T, 64, 128, 4, EPI>(a, st);
   if (a.M > 16) return lin_gemm_go<T, 32, 128, 4, EPI>(a, st);
