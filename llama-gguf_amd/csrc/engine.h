@@ -80,7 +80,6 @@ struct BatchScratch {
   uint64_t mv_part_floats = 0;
   int *amax_i = nullptr, *moe_sel = nullptr;
   int *d_tokens = nullptr, *d_pos = nullptr, *d_slot = nullptr, *d_log = nullptr;   // the step's control words (device), the greedy token log
-  int* h_ctl = nullptr;                               // pinned staging of the control words
   std::vector<float*> kcache, vcache;                 // per layer: [slot][kv_head][max_seq][head_dim]
   // TurboQuant caches (kv_cache_type LGH_KV_TQ*): per layer the slots' code rows [slot][kv_head][max_seq][row bytes] (K, V) and, with
   // QJL, the K rows' sign bits + norms [slot][kv_head][max_seq][head_dim / 32 + 1]; kv_tmp = the step's rotated K / V rows, f32,

@@ -1738,7 +1738,6 @@ void lgh_destroy(lgh_ctx* c) {
     for (auto& gs : gg)
       for (auto& ge : gs)
         if (ge) (void)hipGraphExecDestroy(ge);
-  if (c->batch.h_ctl) (void)hipHostFree(c->batch.h_ctl);
   if (c->pf.tok_pinned) (void)hipHostFree(c->pf.tok_pinned);
   if (c->pf.tok_copied) (void)hipEventDestroy(c->pf.tok_copied);
   if (c->out.pin) (void)hipHostFree(c->out.pin);
