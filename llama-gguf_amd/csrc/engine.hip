@@ -870,6 +870,9 @@ int floats_to_host(lgh_ctx* c, float* dst, const float* src, size_t cols, size_t
   int rc;
   for (size_t i = 0; i < std::min<size_t>(n, kOutSlots); i++)
     if ((rc = request(i))) return rc;
+  // the caller's pages, while the device works: a caller that keeps its results has the next one on fresh pages, whose faults would come between the pieces (steps of 16 sequences, 4 layers of an 8B model,
+  // all 40 results kept: 1008 us a step without this, 683 with it, 634 on used pages)
+  for (size_t at_byte = 0; at_byte < cols * rows * 4; at_byte += 4096) reinterpret_cast<volatile uint8_t*>(dst)[at_byte] = 0;
   for (size_t i = 0; i < n; i++) {
     size_t from, to, len;
     piece(i, from, to, len);
