@@ -220,6 +220,23 @@ hipError_t embed_batch_launch(int src_type, const uint8_t* table, const int* tok
   return hipGetLastError();
 }
 
+// a block of up to 128 prompt tokens: their ids in the launch itself.  (A copy out of pinned memory in front of it, and two fills of a position word behind a slot's prompt: 10 tokens into a slot, 8 layers
+// of an 8B model, 542 us with them and 531 without; 100 tokens 996 and 978.)
+struct BlockTokens { uint32_t id[kPfTokens]; };
+__global__ void __launch_bounds__(256) embed_block_kernel(int type, const uint8_t* __restrict__ table, float* __restrict__ dst, uint32_t hidden, const BlockTokens t) {
+  const uint64_t row = t.id[blockIdx.y];
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < hidden) dst[(size_t)blockIdx.y * hidden + i] = deq_any(type, table, row * hidden + i);
+}
+
+hipError_t embed_block_launch(int src_type, const uint8_t* table, const uint32_t* tokens, float* dst, uint32_t hidden, uint32_t m_tokens, hipStream_t st) {
+  if (!blk_elems(src_type) || m_tokens == 0 || m_tokens > (uint32_t)kPfTokens) return hipErrorInvalidValue;
+  BlockTokens t{};
+  for (uint32_t i = 0; i < m_tokens; i++) t.id[i] = tokens[i];
+  hipLaunchKernelGGL(embed_block_kernel, dim3((hidden + 255) / 256, m_tokens), dim3(256), 0, st, src_type, table, dst, hidden, t);
+  return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------------------------
 // Upload-time re-layout of formats whose blocks are not 16-byte multiples into aligned planes
 // (see DevWeight in common.h).  One thread per block, 2-byte moves (all block sizes are even).

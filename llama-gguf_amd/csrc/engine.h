@@ -37,7 +37,6 @@ struct PfScratch {
   uint8_t *xh_h = nullptr, *xh_attn = nullptr, *xh_act = nullptr;   // XH activations: [128][hidden], [128][QD], [128][ffn]
   float *hidden = nullptr, *q = nullptr, *part = nullptr, *ssq = nullptr;
   size_t part_bytes = 0;
-  int* tokens = nullptr;
   uint32_t* tok_pinned = nullptr;      // pinned host staging of the prompt's token ids, one slot per position
   hipEvent_t tok_copied = nullptr;     // recorded behind the last copy out of it
   uint32_t tok_lo = 0, tok_hi = 0;     // slots [tok_lo, tok_hi) may still be read by a copy enqueued since the last wait for tok_copied
@@ -126,6 +125,7 @@ struct lgh_ctx {
   uint32_t n_splits = 8;
   // host mirrors
   size_t pos = 0;
+  bool slot_prompt = false;                        // pos is a slot's for the moment (lgh_batch_prefill)
   bool finalized = false;
   bool profiling = false;
   std::string err;

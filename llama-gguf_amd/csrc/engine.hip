@@ -934,7 +934,7 @@ static int pf_ensure(lgh_ctx* c) {
       {(void**)&P.xh_h, xh_bytes(H)},           {(void**)&P.xh_attn, xh_bytes(QD)},
       {(void**)&P.xh_act, xh_bytes(std::max(F, EI))}, {(void**)&P.hidden, (size_t)kPfTokens * H * 4},
       {(void**)&P.q, (size_t)kPfTokens * QD * 4},
-      {(void**)&P.part, pb},                    {(void**)&P.tokens, (size_t)kPfTokens * 4},
+      {(void**)&P.part, pb},
       {(void**)&P.ssq, (size_t)kPfTokens * kPfSsqChunks * 4},
       {(void**)&P.moe_sel, any_moe ? (size_t)kPfTokens * topk * 4 : 0},  {(void**)&P.moe_w, any_moe ? (size_t)kPfTokens * topk * 4 : 0},
       {(void**)&P.moe_cnt, any_moe ? (size_t)kPfMaxExperts * 4 : 0},    {(void**)&P.moe_list, any_moe ? (size_t)kPfMaxExperts * kPfTokens * 4 : 0},
@@ -960,7 +960,7 @@ static int pf_stage_tokens(lgh_ctx* c, const uint32_t* tokens, uint32_t m, int* 
   PfScratch& P = c->pf;
   const lgh_model_desc& d = c->d;
   const uint32_t pos0 = (uint32_t)c->pos;
-  // The caller's `tokens` may be freed as soon as this returns (lgh_stage_prefill_batch does not synchronise), so the ids
+  // (Blocks of 128 carry theirs in the launch: embed_block_launch.)  The caller's `tokens` may be freed as soon as this returns, so the ids
   // go through a context-owned PINNED buffer, one slot per position; a slot is only rewritten after the copy that last
   // read it has completed (reset + a second prompt before the first one has run).
   if (!P.tok_pinned) {
@@ -968,7 +968,7 @@ static int pf_stage_tokens(lgh_ctx* c, const uint32_t* tokens, uint32_t m, int* 
     HIP_TRY(c, LGH_OPERATION_FAILED, hipEventCreateWithFlags(&P.tok_copied, hipEventDisableTiming));
   } else if (pos0 < P.tok_hi && pos0 + m > P.tok_lo) {
     // only when a slot about to be rewritten may still be read: a reset / shift / truncate followed by a new prompt.  The blocks
-    // of ONE prompt use ascending slots and never wait here (lgh_stage_prefill_batch stays asynchronous).
+    // of ONE prompt use ascending slots and never wait here.
     HIP_TRY(c, LGH_OPERATION_FAILED, hipEventSynchronize(P.tok_copied));
     P.tok_lo = P.tok_hi = 0;
   }
@@ -1066,10 +1066,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail*
   auto K = [&](hipError_t e, const char* what) -> int {
     return e == hipSuccess ? LGH_OK : fail(c, LGH_OPERATION_FAILED, std::string("batched prefill, ") + what + ": " + hipGetErrorString(e));
   };
-  if (c->first) {
-    if ((rc = pf_stage_tokens(c, tokens, m, P.tokens))) return rc;
-    if ((rc = K(embed_batch_launch(c->embd_type, c->embd_raw, P.tokens, P.hidden, H, m, st), "embedding"))) return rc;
-  }
+  if (c->first && (rc = K(embed_block_launch(c->embd_type, c->embd_raw, tokens, P.hidden, H, m, st), "embedding"))) return rc;
   if ((rc = K(pf_row_epi_launch(nullptr, 0, 0, 0, nullptr, P.hidden, H, c->layers[c->l0].attn_norm, P.xh_h, P.ssq, m, st), "attn_norm"))) return rc;
   const float scale = 1.0f / std::sqrt((float)d.head_dim);  // layers.rs:374
   for (uint32_t li = c->l0; li < c->l1; li++) {
@@ -1133,7 +1130,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail*
   c->pos += m;
   c->stats.tokens_processed += m;
   if (tail) return tail_end(c, *tail);
-  HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
+  if (!c->slot_prompt) HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
   return LGH_OK;
 }
 
@@ -1301,7 +1298,7 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail* 
   c->pos += m;
   c->stats.tokens_processed += m;
   if (tail) return tail_end(c, *tail);
-  HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
+  if (!c->slot_prompt) HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, st));
   return LGH_OK;
 }
 
@@ -1894,11 +1891,12 @@ int lgh_batch_prefill(lgh_ctx* c, uint32_t slot, const uint32_t* tokens, size_t 
     c->layers[i].vcache = Bs.vcache[i] + (size_t)slot * Bs.cache_stride;
   }
   c->pos = Bs.pos[slot];
+  c->slot_prompt = true;   // (the device's word for the context's own next position stays as it is)
   rc = prefill_tokens(c, tokens, n);
+  c->slot_prompt = false;
   if (!rc) Bs.pos[slot] = c->pos;
   c->pos = keep;
   for (uint32_t i = c->l0; i < c->l1; i++) { c->layers[i].kcache = saved[i - c->l0].first; c->layers[i].vcache = saved[i - c->l0].second; }
-  if (hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)keep, 1, c->stream) != hipSuccess && !rc) rc = fail(c, LGH_OPERATION_FAILED, "state reset");
   if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = fail(c, LGH_OPERATION_FAILED, "hipStreamSynchronize");
   return rc;
 }

@@ -133,6 +133,8 @@ hipError_t pfw_qkv_launch(const PfwQkv& a, uint32_t m_tokens, hipStream_t st);
 // dequant.hip: rows tokens[0..m) of the embedding table -> dst[m][hidden]
 hipError_t embed_batch_launch(int src_type, const uint8_t* table, const int* tokens, float* dst, uint32_t hidden, uint32_t m_tokens,
                               hipStream_t st);
+// the same for a block of up to kPfTokens tokens, ids in host memory that is free again when this returns
+hipError_t embed_block_launch(int src_type, const uint8_t* table, const uint32_t* tokens, float* dst, uint32_t hidden, uint32_t m_tokens, hipStream_t st);
 // attention.hip: causal attention of a block of m tokens at positions pos0 .. pos0+m-1 (their K/V rows already cached)
 hipError_t attn_prefill_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv,
                                uint32_t head_dim, uint32_t max_seq, float scale, uint32_t pos0, uint32_t m_tokens, uint8_t* xh_out,
