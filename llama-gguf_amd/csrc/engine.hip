@@ -1563,6 +1563,7 @@ int lgh_finalize(lgh_ctx* c) {
     if ((rc = layered_finalize(c))) return rc;
     c->finalized = true;
     c->pos = 0;
+    (void)out_ensure(c);
     return warm_kernels(c);
   }
   if (c->first && !c->embd_raw) return fail(c, LGH_INITIALIZATION_FAILED, "missing token_embd.weight");
@@ -1721,6 +1722,7 @@ int lgh_finalize(lgh_ctx* c) {
   c->finalized = true;
   c->pos = 0;
   if ((rc = warm_kernels(c))) return rc;
+  if (c->last) (void)out_ensure(c);   // (0.4 ms that the first result would wait for)
   if (c->first && c->last && !(d.flags & LGH_FLAG_NO_GRAPH) && pf_eligible(c)) side_make(c);
   return LGH_OK;
 }
