@@ -749,9 +749,10 @@ static int warm_kernels(lgh_ctx* c) {
   for (int v = 0; v < 2 && !rc; v++) {
     if (v == 1 && c->direct_attn_max_kv == 0) continue;
     c->attn_direct = v == 1;
-    HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetAsync(c->state, 0, ST_WORDS * 4, c->stream));
-    for (int mode : {c->last ? MODE_GREEDY : MODE_PREFILL, MODE_PREFILL})   // the last stage: with and without the output head
+    for (int mode : {c->last ? MODE_GREEDY : MODE_PREFILL, MODE_PREFILL}) {   // the last stage: with and without the output head
+      HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetAsync(c->state, 0, ST_WORDS * 4, c->stream));   // (each at position 0: a context may hold no other)
       if (!rc) rc = enqueue_token(c, mode);
+    }
   }
   c->attn_direct = keep_direct;
   for (auto& q : c->xqs) q.fresh = false;
