@@ -561,11 +561,12 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
   for (uint32_t n : {1u, 2u, 3u, 4u, 5u, 9u, 13u}) {
     if (n > max_batch) break;
     Bs.attn_short = false;
-    if ((rc = stage_control(c, slots0, toks0, n)) || (rc = enqueue_multi(c, n, true))) return rc;
-    if (n == 1 && short_attn_rows(c, 1))   // (the single-launch attention's kernel is the same for every size; attn_out is scratch here)
+    if ((rc = stage_control(c, slots0, toks0, n))) return rc;
+    if (n == 1 && short_attn_rows(c, 1))   // (the single-launch attention's kernel is the same for every size; attn_out is scratch here.  In front of the step, which moves the positions on: a context may hold one row)
       HIP_TRYB(c, LGH_OPERATION_FAILED,
                attn_multi_direct_launch(Bs.q, Bs.kcache[c->l0], Bs.vcache[c->l0], d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, 1.0f, Bs.d_pos, Bs.d_slot, Bs.cache_stride, 1, c->n_splits,
                                         Bs.attn_out, nullptr, c->stream));
+    if ((rc = enqueue_multi(c, n, true))) return rc;
     HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
   }
   return LGH_OK;

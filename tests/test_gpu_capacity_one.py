@@ -17,3 +17,17 @@ def test_one_token(pkg, model, mix):
             one.forward(token)
     one.close()
     more.close()
+
+
+@pytest.mark.parametrize("slots", [1, 3])
+def test_one_token_a_slot(pkg, slots):
+    cfg = pkg.make_config("test-dense-d128", max_seq_len=1, num_layers=2)
+    eng = pkg.HipGpuInference.from_model(pkg.SynthModel(cfg, mix="Q4_K_M"), 1)
+    eng.batch_create(slots)
+    got, _ = eng.forward_multi(list(range(slots)), [7 + s for s in range(slots)])
+    for s in range(slots):
+        eng.reset()
+        assert np.array_equal(got[s].view(np.uint32), eng.forward(7 + s).view(np.uint32))
+    with pytest.raises(pkg.hip_backend.BackendError):
+        eng.forward_multi([0], [1])
+    eng.close()
