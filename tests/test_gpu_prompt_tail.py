@@ -41,3 +41,16 @@ def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
             assert np.array_equal(beside.forward(t).view(np.uint32), behind.forward(t).view(np.uint32)), (before, portion)
     beside.close()
     behind.close()
+
+
+def test_the_step_behind_a_first_prompt_is_there(pkg):
+    """A prompt's last token is launched kernel by kernel where it runs beside its block; the graph that the tokens after it take is captured in the same call, not in theirs."""
+    m = pkg.SynthModel(pkg.make_config("test-dense", max_seq_len=300), mix="Q4_K_M")
+    eng = pkg.HipGpuInference.from_model(m, 300)
+    assert eng.stats()["graph_nodes"] == 0
+    eng.eval(np.arange(40) % m.config.vocab_size, [39])
+    nodes = eng.stats()["graph_nodes"]
+    assert nodes > 0
+    eng.forward(3)
+    assert eng.stats()["graph_nodes"] == nodes
+    eng.close()
