@@ -108,6 +108,7 @@ struct lgh_ctx {
   hipStream_t own_stream = nullptr, stream = nullptr;
   hipStream_t side_stream = nullptr;                  // the token behind a prompt block (engine.hip: tail_layer)
   hipEvent_t side_go = nullptr, side_done = nullptr;
+  uint64_t beside_blocks = 0;                         // tokens that ran beside their block
   std::vector<lgh::LayerW> layers;
   // embedding table in native GGUF layout (row-dequantized per token) and the output projection
   uint8_t* embd_raw = nullptr;

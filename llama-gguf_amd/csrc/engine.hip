@@ -1050,6 +1050,7 @@ static int tail_end(lgh_ctx* c, PfTail& t) {
   HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamWaitEvent(c->stream, c->side_done, 0));
   c->pos += 1;
   c->stats.tokens_processed += 1;
+  c->beside_blocks += 1;
   t.taken = true;
   return LGH_OK;
 }
@@ -1842,6 +1843,14 @@ static int eval_stretch(lgh_ctx* c, const uint32_t* tokens, size_t n, uint32_t t
     return rc;
   }
   return floats_to_host(c, logits_out, c->logits, c->d.vocab_size, c->d.vocab_size, 1);
+}
+
+int lgh_beside_blocks(lgh_ctx* c, int* possible, uint64_t* count) {
+  int rc = check_ready(c);
+  if (rc) return rc;
+  if (possible) *possible = tail_eligible(c) ? 1 : 0;
+  if (count) *count = c->beside_blocks;
+  return LGH_OK;
 }
 
 int lgh_eval(lgh_ctx* c, const uint32_t* tokens, size_t n, const uint32_t* want, size_t n_want, float* logits_out) {

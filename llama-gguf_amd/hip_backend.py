@@ -13,7 +13,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 import threading
-from typing import Iterable, Optional, Sequence
+from typing import Iterable, Optional, Sequence, Tuple
 
 import numpy as np
 
@@ -28,7 +28,7 @@ ABI_SYMBOLS = (
     "lgh_op_kv_roundtrip", "lgh_op_add", "lgh_op_mul", "lgh_op_scale", "lgh_op_silu", "lgh_op_gelu", "lgh_op_softmax", "lgh_op_matmul", "lgh_op_matvec",
     "lgh_op_matvec_q", "lgh_op_attention", "lgh_op_attention_prompt", "lgh_backend_create", "lgh_backend_destroy", "lgh_backend_load_weight",
     "lgh_backend_has_weight", "lgh_backend_vec_mat_q", "lgh_backend_last_error", "lgh_reset", "lgh_position", "lgh_kv_truncate", "lgh_kv_shift_left", "lgh_stage_prefill_batch", "lgh_stage_hidden_block_buffer", "lgh_forward_argmax", "lgh_decode_greedy",
-    "lgh_last_error", "lgh_get_stats", "lgh_set_profiling", "lgh_set_stream", "lgh_get_stream", "lgh_synchronize",
+    "lgh_last_error", "lgh_get_stats", "lgh_beside_blocks", "lgh_set_profiling", "lgh_set_stream", "lgh_get_stream", "lgh_synchronize",
     "lgh_read_hidden", "lgh_debug_fail_alloc", "lgh_stage_hidden_buffer", "lgh_stage_forward", "lgh_op_dequantize", "lgh_op_vec_mat",
     "lgh_op_rms_norm", "lgh_op_rope", "lgh_op_attention_cached", "lgh_op_silu_mul", "lgh_op_norm_vec_mat",
     "lgh_op_swiglu_vec_mat", "lgh_bench_vec_mat", "lgh_bench_hbm_read", "lgh_gguf_inspect", "lgh_load_gguf",
@@ -156,6 +156,7 @@ def load_library() -> C.CDLL:
         "lgh_forward_argmax": (C.c_int, [vp, u32, C.POINTER(u32)]),
         "lgh_decode_greedy": (C.c_int, [vp, u32, sz, vp]),
         "lgh_last_error": (C.c_char_p, [vp]), "lgh_get_stats": (C.c_int, [vp, C.POINTER(Stats)]),
+        "lgh_beside_blocks": (C.c_int, [vp, C.POINTER(C.c_int), C.POINTER(C.c_uint64)]),
         "lgh_set_profiling": (C.c_int, [vp, C.c_int]), "lgh_set_stream": (C.c_int, [vp, vp]),
         "lgh_get_stream": (vp, [vp]), "lgh_synchronize": (C.c_int, [vp]), "lgh_read_hidden": (C.c_int, [vp, vp]),
         "lgh_debug_fail_alloc": (C.c_int, [vp, u32]),
@@ -531,6 +532,12 @@ class HipGpuInference:
                                          "alg_bytes": s.sym_alg_bytes[i]}
                           for i in range(len(SYM_NAMES)) if s.sym_launches[i]}
         return out
+
+    def beside_blocks(self) -> Tuple[bool, int]:
+        """Whether a prompt's last token can run beside its block in this context, and how many did."""
+        possible, count = C.c_int(), C.c_uint64()
+        self._call(load_library().lgh_beside_blocks(self._h, C.byref(possible), C.byref(count)))
+        return bool(possible.value), count.value
 
     def close(self) -> None:
         if self._h:

@@ -17,6 +17,9 @@ def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
     m = pkg.SynthModel(cfg, mix=mix)
     beside, behind = (pkg.HipGpuInference.from_model(m, max_seq) for _ in range(2))
     assert beside.prefill_is_batched()
+    if not beside.beside_blocks()[0]:
+        pytest.skip("no stream here runs beside the context's own")
+    ran = 0
     if slots:
         beside.batch_create(slots)
         behind.batch_create(slots)
@@ -29,6 +32,8 @@ def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
             behind.forward_batch(tok[:before])
         n = sum(portion)
         got = beside.eval(tok[before:before + n], [int(v) - 1 for v in np.cumsum(portion)])
+        ran += sum(length > 2 for length in portion)   # two tokens in front and more: a block
+        assert beside.beside_blocks() == (True, ran), (before, portion)
         at = before
         for i, length in enumerate(portion):
             if length > 1:
@@ -39,6 +44,27 @@ def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
         assert beside.position() == behind.position() == at
         for t in (4, 9):
             assert np.array_equal(beside.forward(t).view(np.uint32), behind.forward(t).view(np.uint32)), (before, portion)
+    assert behind.beside_blocks()[1] == 0
+    beside.close()
+    behind.close()
+
+
+def test_large_blocks_go_first(pkg):
+    """1536 tokens of width 4096 and fewer have the step beside them, larger blocks in front of it."""
+    cfg = pkg.make_config("test-dense-d128", max_seq_len=1700, hidden_size=4096, intermediate_size=512, num_heads=32, num_kv_heads=8, num_layers=2, vocab_size=512)
+    m = pkg.SynthModel(cfg, mix="Q8_0")
+    beside, behind = (pkg.HipGpuInference.from_model(m, 1700) for _ in range(2))
+    if not beside.beside_blocks()[0]:
+        pytest.skip("no stream here runs beside the context's own")
+    tok = np.random.default_rng(6).integers(0, cfg.vocab_size, 1700).astype(np.uint32)
+    for block, ran in ((1536, 1), (1537, 1), (1600, 1), (700, 2)):
+        beside.reset()
+        behind.reset()
+        got = beside.eval(tok[:block + 1], [block])[0]
+        assert beside.beside_blocks()[1] == ran, block
+        behind.forward_batch(tok[:block])
+        assert np.array_equal(got.view(np.uint32), behind.forward(int(tok[block])).view(np.uint32)), block
+        assert np.array_equal(beside.forward(4).view(np.uint32), behind.forward(4).view(np.uint32)), block
     beside.close()
     behind.close()
 
