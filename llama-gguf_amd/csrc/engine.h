@@ -1,6 +1,7 @@
 // engine.h — the GPU-resident decode engine behind the lgh_* C ABI (internal).
 #pragma once
 
+#include <atomic>
 #include <string>
 #include <vector>
 
@@ -106,7 +107,7 @@ struct lgh_ctx {
   uint32_t l0 = 0, l1 = 0;
   bool first = true, last = true;
   hipStream_t own_stream = nullptr, stream = nullptr;
-  hipStream_t side_stream = nullptr;                  // the token behind a prompt block (engine.hip: tail_layer)
+  hipStream_t side_stream = nullptr;                  // the token behind a prompt block (engine.hip: tail_layer); the device's, not this context's own
   hipEvent_t side_go = nullptr, side_done = nullptr;
   uint64_t beside_blocks = 0;                         // tokens that ran beside their block
   std::vector<lgh::LayerW> layers;
@@ -202,6 +203,15 @@ void xq_stale(lgh_ctx* c, const float* f32);
 int linear_any(lgh_ctx* c, int cls, const lgh::DevWeight& W, const float* x, float* out, const float* norm_w,
                const float* resid, const float* bias, int xq_next = 0, const float* xq_next_nw = nullptr);
 int drain_prof(lgh_ctx* c);
+// a call at work on the context's device, until everything it launched has ended (engine.hip: the side stream); alone: no other was when it began
+struct AtWork {
+  std::atomic<int>* const calls;
+  const bool alone;
+  explicit AtWork(const lgh_ctx* c);
+  ~AtWork();
+  AtWork(const AtWork&) = delete;
+  AtWork& operator=(const AtWork&) = delete;
+};
 int floats_to_host(lgh_ctx* c, float* dst, const float* src, size_t cols, size_t ld, size_t rows);
 // layered.hip, behind the entry points of engine.hip when c->lm is set
 int layered_upload(lgh_ctx* c, const char* name, uint32_t type, const uint64_t ne[4], const void* host, size_t nbytes);

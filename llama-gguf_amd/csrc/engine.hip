@@ -20,10 +20,13 @@
 #include "xq.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
+#include <thread>
 
 using namespace lgh;
 
@@ -989,8 +992,8 @@ static int pf_stage_tokens(lgh_ctx* c, const uint32_t* tokens, uint32_t m, int* 
 // other writes while it runs (the block its own rows and those before them, the step its one row behind them besides).  The same kernels on the same values: the same bits.
 struct PfTail { uint32_t token; size_t pos; bool taken = false; };   // at position pos; taken: its step is under way
 
-// A process's streams share a few hardware queues, and two streams in one queue run one after the other: then the events between them cost a layer some 8 us and nothing is gained (8 layers of an 8B
-// model, 300 tokens: 2.43 -> 2.50 ms).  Which queue a stream gets is the runtime's affair, so it is tried: a kernel on the context's stream waits, some 200 us at most, for what one on the other says.
+// Two streams in one hardware queue run one after the other: then the events between them cost a layer some 8 us and nothing is gained (8 layers of an 8B model, 300 tokens: 2.43 -> 2.50 ms).  Which queue
+// a stream gets is the runtime's affair, so it is tried: a kernel on one stream waits, some 200 us at most, for what one on the other says.
 __global__ void side_wait_kernel(int* w) {
   for (int i = 0; i < 150; i++) {
     if (__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) { w[1] = 1; return; }
@@ -1000,33 +1003,103 @@ __global__ void side_wait_kernel(int* w) {
 }
 __global__ void side_say_kernel(int* w, int v) { __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// c->side_stream beside c->stream, if there is one to be had; without it a prompt's last token follows its block
-static void side_make(lgh_ctx* c) {
-  hipStream_t tried[4] = {};
-  int n = 0, *w = nullptr, seen = 0;
-  bool ok = hipEventCreateWithFlags(&c->side_go, hipEventDisableTiming) == hipSuccess && hipEventCreateWithFlags(&c->side_done, hipEventDisableTiming) == hipSuccess &&
-            hipMalloc((void**)&w, 8) == hipSuccess;
-  while (ok && !seen && n < 4) {
-    ok = hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) == hipSuccess;
-    if (!ok) break;
-    hipStream_t s = tried[n++];
-    for (int pass = 0; pass < 2 && ok; pass++) {   // (the first launches on a stream take longer)
-      hipLaunchKernelGGL(side_say_kernel, dim3(1), dim3(1), 0, s, w, 0);
-      ok = hipStreamSynchronize(s) == hipSuccess;
-      hipLaunchKernelGGL(side_wait_kernel, dim3(1), dim3(1), 0, c->stream, w);
-      hipLaunchKernelGGL(side_say_kernel, dim3(1), dim3(1), 0, s, w, 1);
-      ok = ok && hipStreamSynchronize(s) == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess;
-    }
-    ok = ok && hipMemcpy(&seen, w + 1, 4, hipMemcpyDeviceToHost) == hipSuccess;
+// The side stream, one a device for all of its contexts.  Streams share four hardware queues, handed out in turn: with a stream of its own beside each context's, contexts at work in threads met in one queue
+// (11 layers of TinyLlama, six contexts decoding 100 tokens each: 114 ms, 87 without; three with one more stream in a queue of its own: 70 and 46).  This one shares the null stream's
+// queue, so contexts' streams lie as if it were not there, and is left alone while that queue has work (side_idle).
+// One call at a time has it, and only while no other is at work on the device: beside others' launches a step finds no idle part of the chip and takes theirs (20 prompts of 100 tokens each from two / three / six
+// contexts in threads: 34.0 / 40.8 / 88 ms with a step beside every block, 31.1 / 36.5 / 73 without).
+struct SideStream {
+  std::mutex mu;                   // stream, users
+  hipStream_t stream = nullptr;
+  int users = 0;                   // contexts that hold it
+  std::atomic<int> calls{0};       // calls at work
+};
+static SideStream side_streams[64];
+static SideStream* side_of(const lgh_ctx* c) { return c->device >= 0 && c->device < 64 ? &side_streams[c->device] : nullptr; }
+
+AtWork::AtWork(const lgh_ctx* c) : calls(side_of(c) ? &side_of(c)->calls : nullptr), alone(calls && calls->fetch_add(1) == 0) {}
+AtWork::~AtWork() { if (calls) calls->fetch_sub(1); }
+
+// do the streams run side by side?  w: two words on the device
+static bool side_by_side(hipStream_t a, hipStream_t b, int* w, bool& ok) {
+  int seen = 0;
+  for (int pass = 0; pass < 2 && ok; pass++) {   // (the first launches on a stream take longer)
+    hipLaunchKernelGGL(side_say_kernel, dim3(1), dim3(1), 0, b, w, 0);
+    ok = hipStreamSynchronize(b) == hipSuccess;
+    hipLaunchKernelGGL(side_wait_kernel, dim3(1), dim3(1), 0, a, w);
+    hipLaunchKernelGGL(side_say_kernel, dim3(1), dim3(1), 0, b, w, 1);
+    ok = ok && hipStreamSynchronize(b) == hipSuccess && hipStreamSynchronize(a) == hipSuccess;
   }
-  if (ok && seen) c->side_stream = tried[--n];
-  while (n > 0) (void)hipStreamDestroy(tried[--n]);
+  ok = ok && hipMemcpy(&seen, w + 1, 4, hipMemcpyDeviceToHost) == hipSuccess;
+  return ok && seen;
+}
+
+// c->side_stream: the device's side stream, if it runs beside the context's; the first context to ask makes it (1 ms: six streams or so are tried).  Without it a prompt's last token follows its block
+static void side_make(lgh_ctx* c) {
+  SideStream* S = side_of(c);
+  int* w = nullptr;
+  bool ok = S && hipEventCreateWithFlags(&c->side_go, hipEventDisableTiming) == hipSuccess && hipEventCreateWithFlags(&c->side_done, hipEventDisableTiming) == hipSuccess &&
+            hipMalloc((void**)&w, 8) == hipSuccess;
+  if (ok) {
+    std::lock_guard<std::mutex> lock(S->mu);
+    if (!S->stream) {
+      hipStream_t tried[8] = {};
+      int n = 0;
+      while (ok && !S->stream && n < 8) {
+        ok = hipStreamCreateWithFlags(&tried[n], hipStreamNonBlocking) == hipSuccess;
+        if (ok && !side_by_side(nullptr, tried[n++], w, ok) && ok) S->stream = tried[--n];
+      }
+      while (n > 0) (void)hipStreamDestroy(tried[--n]);
+    }
+    for (int i = 0; i < 50 && ok && S->stream; i++) {   // (between the others' calls)
+      const AtWork call(c);
+      if (call.alone) {
+        if (side_by_side(c->own_stream, S->stream, w, ok)) c->side_stream = S->stream;
+        break;
+      }
+      std::this_thread::sleep_for(std::chrono::milliseconds(1));
+    }
+    if (c->side_stream) S->users++;
+    if (S->stream && S->users == 0) {
+      (void)hipStreamDestroy(S->stream);
+      S->stream = nullptr;
+    }
+  }
   if (w) (void)hipFree(w);
   if (!ok) (void)hipGetLastError();   // (the next launch's check would find it)
 }
 
+static void side_leave(lgh_ctx* c) {
+  if (c->side_stream) {
+    SideStream* S = side_of(c);
+    std::lock_guard<std::mutex> lock(S->mu);
+    if (--S->users == 0) {
+      (void)hipStreamDestroy(S->stream);
+      S->stream = nullptr;
+    }
+  }
+  if (c->side_go) (void)hipEventDestroy(c->side_go);
+  if (c->side_done) (void)hipEventDestroy(c->side_done);
+}
+
 // (no stream of the caller's, no recording of launch times, no context that wants its launches one after the other, no model whose steps are not built layer by layer here)
 static bool tail_eligible(const lgh_ctx* c) { return c->side_stream && c->stream == c->own_stream && !c->lm && c->first && c->last && !c->profiling && !(c->d.flags & LGH_FLAG_NO_GRAPH) && pf_eligible(c); }
+
+// Has the side stream's queue nothing else to do?  Work on the null stream, which need not be this library's, would hold every layer of the step up.  An event is recorded when the prompt begins and has to be
+// there when the first layer's rows are under way, or some microseconds later, which the device does not notice: it has those launches in front of it
+static hipError_t side_ask(lgh_ctx* c) {
+  const hipError_t e = hipEventRecord(c->side_done, c->side_stream);
+  if (e == hipSuccess && hipEventQuery(c->side_done) != hipSuccess) (void)hipGetLastError();   // (the runtime sends the event on its way with the first question)
+  return e;
+}
+static bool side_idle(lgh_ctx* c) {
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(30);
+  for (;;) {
+    const bool idle = hipEventQuery(c->side_done) == hipSuccess;
+    if (!idle) (void)hipGetLastError();   // (the next launch's check would find it)
+    if (idle || std::chrono::steady_clock::now() >= until) return idle;
+  }
+}
 
 // the block's rows of layer li are under way on c->stream: the token's layer li behind them
 static int tail_layer(lgh_ctx* c, const PfTail& t, uint32_t li) {
@@ -1082,6 +1155,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail*
                                   d.norm_eps, (int)d.use_neox_rope, m, st),
                 "qkv epilogue")))
       return rc;
+    if (li == c->l0 && tail && !side_idle(c)) tail = nullptr;
     if (tail && (rc = tail_layer(c, *tail, li))) return rc;
     if (li + 1 == c->l1 && c->last) break;   // the model's last layer: its K/V rows are written, its output would be discarded
     if ((rc = K(attn_prefill_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.xh_attn, st),
@@ -1258,6 +1332,7 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail* 
     if ((rc = product({&L.wq, &L.wk, &L.wv}, P.x, G, PW_PART, m, nullptr, "qkv product"))) return rc;
     const PfwQkv e{P.part, G.S, G.part_rows, QD, KD, d.head_dim, L.bq, L.bk, L.bv, c->rope_cs, P.inv_rms, pos0, d.max_seq_len, P.q, L.kcache, L.vcache, (int)d.use_neox_rope};
     if ((rc = K(pfw_qkv_launch(e, m, st), "qkv"))) return rc;
+    if (li == c->l0 && tail && !side_idle(c)) tail = nullptr;
     if (tail && (rc = tail_layer(c, *tail, li))) return rc;
     if (li + 1 == c->l1) break;   // the last layer: its K / V rows are written, its output would be discarded
     if ((rc = K(attn_wide_launch(P.q, L.kcache, L.vcache, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, pos0, m, P.kv_split, P.part, P.part_bytes, P.attn, st), "attention"))) return rc;
@@ -1749,9 +1824,7 @@ void lgh_destroy(lgh_ctx* c) {
   if (c->out.pin) (void)hipHostFree(c->out.pin);
   for (auto& e : c->out.ready)
     if (e) (void)hipEventDestroy(e);
-  if (c->side_go) (void)hipEventDestroy(c->side_go);
-  if (c->side_done) (void)hipEventDestroy(c->side_done);
-  if (c->side_stream) (void)hipStreamDestroy(c->side_stream);
+  side_leave(c);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   layered_destroy(c);
   delete c;
@@ -1769,6 +1842,7 @@ int lgh_forward(lgh_ctx* c, uint32_t token, float* logits_out) {
   if (rc) return rc;
   if (!logits_out) return fail(c, LGH_INVALID_ARGUMENT, "logits_out is NULL");
   if (!c->first || !c->last) return fail(c, LGH_INVALID_ARGUMENT, "lgh_forward needs a single-stage context; use lgh_stage_forward");
+  const AtWork call(c);
   if ((rc = set_token(c, token))) return rc;
   if ((rc = step(c, MODE_FORWARD))) return rc;
   return floats_to_host(c, logits_out, c->logits, c->d.vocab_size, c->d.vocab_size, 1);
@@ -1817,6 +1891,7 @@ int lgh_prefill_batch(lgh_ctx* c, const uint32_t* tokens, size_t n) {
       return fail(c, LGH_INVALID_ARGUMENT, "prompt of " + std::to_string(n) + " tokens at position " + std::to_string(c->pos) + " exceeds max_seq_len");
     for (size_t i = 0; i < n; i++)
       if (tokens[i] >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");
+    const AtWork call(c);
     if ((rc = prefill_tokens(c, tokens, n))) return rc;
     HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
     return LGH_OK;
@@ -1829,15 +1904,17 @@ int lgh_prefill_batch(lgh_ctx* c, const uint32_t* tokens, size_t n) {
 
 // n tokens as blocks and the token behind them, whose logits are wanted
 static int eval_stretch(lgh_ctx* c, const uint32_t* tokens, size_t n, uint32_t token, float* logits_out) {
+  const AtWork call(c);
   PfTail t{token, c->pos + n};
   c->attn_direct = t.pos + 1 <= direct_attn_rows(c);
-  int rc = prefill_tokens(c, tokens, n, &t);
+  if (call.alone) HIP_TRY(c, LGH_OPERATION_FAILED, side_ask(c));
+  int rc = prefill_tokens(c, tokens, n, call.alone ? &t : nullptr);
   if (!rc && !t.taken && !(rc = set_token(c, token))) rc = step(c, MODE_FORWARD);
   // the step that the next token takes, captured while the device works where it is not there yet: a first token behind a first prompt would wait for it (8B model 2.6 ms
   // instead of 1.57, its prompt of 128 tokens 6.0 either way)
   if (!rc) rc = ensure_graph(c, MODE_FORWARD);
   if (rc) {
-    (void)hipStreamSynchronize(c->side_stream);   // nothing of the call goes on behind its error, and the next token's position is the one behind what is there
+    if (call.alone) (void)hipStreamSynchronize(c->side_stream);   // nothing of the call goes on behind its error, and the next token's position is the one behind what is there
     (void)hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, c->stream);
     (void)hipStreamSynchronize(c->stream);
     return rc;
@@ -1864,7 +1941,10 @@ int lgh_eval(lgh_ctx* c, const uint32_t* tokens, size_t n, const uint32_t* want,
     if (tokens[i] >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");
   for (size_t i = 0; i < n_want; i++)
     if (want[i] >= n || (i && want[i] <= want[i - 1])) return fail(c, LGH_INVALID_ARGUMENT, "wanted places must ascend within the portion");
-  if (c->lm && n >= 2 && layered_has_blocks(c)) return layered_block(c, tokens, n, want, n_want, logits_out);
+  if (c->lm && n >= 2 && layered_has_blocks(c)) {
+    const AtWork call(c);
+    return layered_block(c, tokens, n, want, n_want, logits_out);
+  }
   // stretches without a wanted place as prompt blocks, wanted places as steps
   size_t at = 0;
   for (size_t i = 0; i < n_want; i++) {
@@ -1900,6 +1980,7 @@ int lgh_batch_prefill(lgh_ctx* c, uint32_t slot, const uint32_t* tokens, size_t 
       if ((rc = lgh_forward_multi(c, &slot, tokens + i, 1, nullptr, nullptr))) return rc;
     return LGH_OK;
   }
+  const AtWork call(c);
   const size_t keep = c->pos;
   std::vector<std::pair<float*, float*>> saved;
   for (uint32_t i = c->l0; i < c->l1; i++) {
@@ -1984,6 +2065,7 @@ int lgh_forward_argmax(lgh_ctx* c, uint32_t token, uint32_t* next_token) {
   if (rc) return rc;
   if (!next_token) return fail(c, LGH_INVALID_ARGUMENT, "next_token is NULL");
   if (!c->first || !c->last) return fail(c, LGH_INVALID_ARGUMENT, "needs a single-stage context");
+  const AtWork call(c);
   if ((rc = set_token(c, token))) return rc;
   if ((rc = step(c, MODE_GREEDY))) return rc;
   int tok = 0;
@@ -1999,6 +2081,7 @@ int lgh_decode_greedy(lgh_ctx* c, uint32_t first_token, size_t n_steps, uint32_t
   if (n_steps && !tokens_out) return fail(c, LGH_INVALID_ARGUMENT, "tokens_out is NULL");
   if (!c->first || !c->last) return fail(c, LGH_INVALID_ARGUMENT, "needs a single-stage context");
   if (c->pos + n_steps > c->d.max_seq_len) return fail(c, LGH_INVALID_ARGUMENT, "decode would exceed max_seq_len");
+  const AtWork call(c);
   if ((rc = set_token(c, first_token))) return rc;
   // argmax_stage2 writes each token into state[TOKEN] (the feedback) and into tok_log[position]
   const size_t pos0 = c->pos;

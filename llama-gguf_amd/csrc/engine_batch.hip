@@ -589,6 +589,7 @@ int lgh_forward_multi(lgh_ctx* c, const uint32_t* slots, const uint32_t* tokens,
   int rc = check_batch(c);
   if (rc) return rc;
   if (!slots || !tokens) return fail(c, LGH_INVALID_ARGUMENT, "slots / tokens is NULL");
+  const AtWork call(c);
   if ((rc = stage_control(c, slots, tokens, n_seq))) return rc;
   if ((rc = run_multi(c, n_seq, next_tokens != nullptr, longest_of(c, slots, n_seq)))) return rc;
   BatchScratch& Bs = c->batch;
@@ -609,6 +610,7 @@ int lgh_decode_greedy_multi(lgh_ctx* c, const uint32_t* slots, const uint32_t* f
     for (uint32_t i = 0; i < n_seq && i < (uint32_t)kMaxBatch; i++)
       if (slots[i] < Bs.max_batch && Bs.pos[slots[i]] + n_steps > c->d.max_seq_len) return fail(c, LGH_INVALID_ARGUMENT, "the steps would run past max_seq_len");
   if (n_steps > c->d.max_seq_len) return fail(c, LGH_INVALID_ARGUMENT, "too many steps");
+  const AtWork call(c);
   if ((rc = stage_control(c, slots, first_tokens, n_seq))) return rc;
   for (size_t st = 0; st < n_steps; st++) {
     if ((rc = run_multi(c, n_seq, true, longest_of(c, slots, n_seq) + st))) return rc;

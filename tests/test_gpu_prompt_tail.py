@@ -1,5 +1,7 @@
 """The token behind a prompt block, whose step runs beside the block (engine.hip, tail_layer), against the block and then the step: all bits equal, its own logits and those of the tokens after it.  Portions
 around one block (128 tokens) and a remainder of one token, from nothing and behind earlier tokens, several wanted places, short and long contexts (the two forms of attention), mixtures, a context with slots."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -33,7 +35,6 @@ def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
         n = sum(portion)
         got = beside.eval(tok[before:before + n], [int(v) - 1 for v in np.cumsum(portion)])
         ran += sum(length > 2 for length in portion)   # two tokens in front and more: a block
-        assert beside.beside_blocks() == (True, ran), (before, portion)
         at = before
         for i, length in enumerate(portion):
             if length > 1:
@@ -44,6 +45,7 @@ def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
         assert beside.position() == behind.position() == at
         for t in (4, 9):
             assert np.array_equal(beside.forward(t).view(np.uint32), behind.forward(t).view(np.uint32)), (before, portion)
+    assert ran // 2 < beside.beside_blocks()[1] <= ran     # (one whose stream was not idle at once goes behind its block)
     assert behind.beside_blocks()[1] == 0
     beside.close()
     behind.close()
@@ -57,11 +59,15 @@ def test_large_blocks_go_first(pkg):
     if not beside.beside_blocks()[0]:
         pytest.skip("no stream here runs beside the context's own")
     tok = np.random.default_rng(6).integers(0, cfg.vocab_size, 1700).astype(np.uint32)
-    for block, ran in ((1536, 1), (1537, 1), (1600, 1), (700, 2)):
-        beside.reset()
+    for block, goes in ((1536, True), (1537, False), (1600, False), (700, True)):
+        for attempt in range(5):                  # (one whose stream was not idle at once goes behind its block)
+            beside.reset()
+            before = beside.beside_blocks()[1]
+            got = beside.eval(tok[:block + 1], [block])[0]
+            if beside.beside_blocks()[1] > before:
+                break
+        assert (beside.beside_blocks()[1] > before) == goes, block
         behind.reset()
-        got = beside.eval(tok[:block + 1], [block])[0]
-        assert beside.beside_blocks()[1] == ran, block
         behind.forward_batch(tok[:block])
         assert np.array_equal(got.view(np.uint32), behind.forward(int(tok[block])).view(np.uint32)), block
         assert np.array_equal(beside.forward(4).view(np.uint32), behind.forward(4).view(np.uint32)), block
@@ -80,3 +86,42 @@ def test_the_step_behind_a_first_prompt_is_there(pkg):
     eng.forward(3)
     assert eng.stats()["graph_nodes"] == nodes
     eng.close()
+
+
+def test_contexts_at_work_share_one_stream(pkg):
+    """The device has one stream for such steps, taken by one prompt at a time and only while no other is at work: contexts in threads give what each gives alone, and contexts come and go around it."""
+    m = pkg.SynthModel(pkg.make_config("test-dense-d128", max_seq_len=400), mix="Q4_K_M")
+    tok = np.random.default_rng(7).integers(0, m.config.vocab_size, 400).astype(np.uint32)
+    lengths = (3, 40, 129, 300)
+    first = pkg.HipGpuInference.from_model(m, 400)
+    want = {}
+    for n in lengths:
+        first.reset()
+        want[n] = first.eval(tok[:n], [n - 1])[0].copy()
+    at_work = [first] + [pkg.HipGpuInference.from_model(m, 400) for _ in range(3)]
+    before = [e.beside_blocks()[1] for e in at_work]
+    wrong = []
+
+    def prompts(e, k):
+        for i in range(24):
+            n = lengths[(i + k) % 4]
+            e.reset()
+            if not np.array_equal(e.eval(tok[:n], [n - 1])[0].view(np.uint32), want[n].view(np.uint32)):
+                wrong.append((k, i, n))
+    for _ in range(2):
+        threads = [threading.Thread(target=prompts, args=(e, k)) for k, e in enumerate(at_work)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong
+        ran = [e.beside_blocks()[1] - b for e, b in zip(at_work, before)]
+        assert sum(ran) < 24 * len(at_work), "every prompt had the device to itself"
+        at_work.pop(0).close()                    # the context that made the stream goes first
+        before.pop(0)
+        before = [e.beside_blocks()[1] for e in at_work]
+    for e in at_work:
+        e.close()
+    again = pkg.HipGpuInference.from_model(m, 400)
+    assert np.array_equal(again.eval(tok[:40], [39])[0].view(np.uint32), want[40].view(np.uint32))
+    again.close()
