@@ -1034,7 +1034,8 @@ static bool side_by_side(hipStream_t a, hipStream_t b, int* w, bool& ok) {
   return ok && seen;
 }
 
-// c->side_stream: the device's side stream, if it runs beside the context's; the first context to ask makes it (1 ms: six streams or so are tried).  Without it a prompt's last token follows its block
+// c->side_stream: the device's side stream, if it runs beside the context's; the first context to ask makes it (1 ms: six streams or so are tried).  Without it a prompt's last token follows its block.
+// In front of the weights: the device allocations behind a stream that was destroyed are slower, by 0.7 ms after one and 2 ms after five (a first long prompt's took 2 ms of its 6.6, behind the weights)
 static void side_make(lgh_ctx* c) {
   SideStream* S = side_of(c);
   int* w = nullptr;
@@ -1483,6 +1484,7 @@ int lgh_create(const lgh_model_desc* desc, lgh_ctx** out) {
     return LGH_INITIALIZATION_FAILED;
   }
   c->stream = c->own_stream;
+  if (c->first && c->last && !(d.flags & (LGH_FLAG_NO_GRAPH | LGH_FLAG_EXACT_PREFILL | LGH_FLAG_KV_INT8))) side_make(c);
   uint32_t splits = (d.flags >> LGH_FLAG_ATTN_SPLITS_SHIFT) & 0xFFu;
   if (!splits) {  // one attention workgroup per CU (measured: 605 vs 596 tokens/s at kv 272 and 470 vs 383 at kv 4000 against 128 workgroups)
     splits = 256 / d.num_kv_heads;
@@ -1802,7 +1804,6 @@ int lgh_finalize(lgh_ctx* c) {
   c->pos = 0;
   if ((rc = warm_kernels(c))) return rc;
   if (c->last) (void)out_ensure(c);   // (0.4 ms that the first result would wait for)
-  if (c->first && c->last && !(d.flags & LGH_FLAG_NO_GRAPH) && pf_eligible(c)) side_make(c);
   return LGH_OK;
 }
 
