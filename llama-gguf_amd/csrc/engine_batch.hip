@@ -397,20 +397,31 @@ int stage_control(lgh_ctx* c, const uint32_t* slots, const uint32_t* tokens, uin
   return LGH_OK;
 }
 
-// Rows of the longest sequence up to which a step's attention over f32 slots is one launch (attn_multi_direct_kernel: a workgroup per query head and sequence, 4096 values of rows a step of its waves).  The line
-// goes by how many of them there are: few leave the chip to one head's rows each.  us a step of 4 layers, split and merge against one launch, 32/8 heads of 128:
-//   sequences        1              2              4              8              16
-//   30 rows      256  245      305  289      343  322      407  384      537  516
-//   120          256  252      306  300      347  337      413  395      559  535
-//   250          259  268      312  324      356  355      435  411      593  559
-//   500          262  283      316  342      363  367      451  421      627  592
-//   1000         263  314      321  364      372  388      464  461      653  678
-// (32/4 heads of 64, 8 layers, 2 / 8 / 16 sequences: 30 rows 448 406, 568 478, 677 592; 500 rows 461 504, 587 561, 779 713; 1000 rows 466 519, 600 567, 806 769.  Capacities from 2048 rows on, whose splits
-// have eight waves, 4 layers of 32/8 heads of 128, 2 / 8 / 16 sequences: 30 rows 311 290, 457 386, 585 516; 500 rows 322 366, 467 449, 667 628; 1000 rows 328 381, 486 467, 714 676.)
+// Rows of the longest sequence up to which a step's attention over f32 slots is one launch (attn_multi_direct_kernel: a workgroup per query head and sequence, 4096 values of rows a step of its waves).  us that it
+// saves a step of 4 layers against split and merge, heads of 128, capacities below 2048:
+//   workgroups, heads, sequences    64 rows   96  128  192  256  384  512  640
+//     64   32/8    2                   10      5   -1   -8  -13
+//     64   32/32   2                    2     -2   -1   -6   -9
+//     64   16/2    4                   12      6    2   -8  -17
+//    128   32/8    4                   15      8    4   -6  -10
+//    128   16/16   8                    7      3    4    3                  -1
+//    128   32/32   4                    4      4    4   -2   -1    0   -6
+//    256   32/8    8                   14      7   18   13   12   14   12   15
+//    256   32/16   8                   13     10   12   13   13    9    8   15
+//    256   32/32   8                   11      9    9    6    8   -2  -11
+//    512   32/8   16                   23     18   33   37   32   33   30   28
+//    512   32/16  16                   19     22   24   22   18    3   -4   -1
+//    512   32/32  16                   22     23   17   -7  -13  -17
+//   1024   64/8   16                   38     27   47   57   36   36   23   26   (-10 at 768)
+//   1024   64/64  16                    5     -1   -9  -29
+// Few workgroups leave the chip to one head's rows each: two or three steps.  With one for every CU it pays until the rows are read from memory at its full rate, which split and merge reads once per kv head, that is up
+// to some 2048 steps of all kv heads.  (Heads of 64 the same with twice the rows: 32/4 heads, 8 sequences, 1280 rows 3; 32/32, 16 sequences, 256 rows 6, 384 -7; 32/8, 2, 128 rows 14, 256 4, 384 -8.  From 2048 rows of
+// capacity on, whose splits have eight waves, it saves more: 32/8 heads, 4 / 8 sequences, 96 rows 31 / 57.)
 size_t short_attn_rows(const lgh_ctx* c, uint32_t n_seq) {
   const lgh_model_desc& d = c->d;
   if (kv_is_tq(d.kv_cache_type)) return 0;
-  const uint32_t wgs = d.num_heads * n_seq, steps = wgs >= (uint32_t)kNumCU ? 24 : wgs >= (uint32_t)kNumCU / 2 ? 8 : 4;
+  const uint32_t wgs = d.num_heads * n_seq, group = d.num_heads / d.num_kv_heads, cus = (uint32_t)kNumCU;
+  const uint32_t steps = wgs >= cus ? std::min(20u, 2048 * group / wgs) : wgs >= cus / 2 ? (group == 1 ? 5 : 3) : group >= 4 ? 3 : 2;
   return (size_t)steps * 4096 / d.head_dim;
 }
 

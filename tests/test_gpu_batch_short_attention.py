@@ -39,11 +39,11 @@ def test_one_launch_equals_split_and_merge(pkg, heads, kv_heads, head_dim, max_s
 
 
 def test_a_greedy_loop_across_the_line(pkg):
-    """decode_greedy_multi walks past the line (128 rows here): the launches change between two steps, the tokens are the single steps'."""
+    """decode_greedy_multi walks past the line (96 rows here): the launches change between two steps, the tokens are the single steps'."""
     cfg = pkg.make_config("test-dense-d128", max_seq_len=300, num_layers=2)
     eng = pkg.HipGpuInference.from_model(pkg.SynthModel(cfg, mix="Q4_K_M"), 300)
     eng.batch_create(2)
-    tok = np.random.default_rng(3).integers(0, cfg.vocab_size, (2, 124))
+    tok = np.random.default_rng(3).integers(0, cfg.vocab_size, (2, 92))
     for s in range(2):
         eng.batch_prefill(s, tok[s])
     loop = eng.decode_greedy_multi([0, 1], [5, 9], 8)
