@@ -1005,7 +1005,8 @@ hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc
 
 
 // ---- the same in one launch, bit for bit: a workgroup of 16 waves per (query head, sequence) works through the head's splits, 16 / NW at a time with NW waves each, every split's rows, waves
-// and merges exactly as in attn_partial_kernel, and then merges the splits as attn_combine_kernel does.  Rows are requested four steps ahead, across splits.
+// and merges exactly as in attn_partial_kernel, and then merges the splits as attn_combine_kernel does.  Rows are requested three steps ahead (two with eight
+// waves a split), across splits.
 // What the two launches cost is the dispatch of their workgroups, the partial sums' way through memory and the splits that a workgroup walks one after the other; what this costs is that a query head's rows pass
 // through one CU and are read once per query head (from the L2 that the heads of a kv head share: attn_direct_kernel).
 template <int D, int NW>

@@ -110,8 +110,8 @@ __device__ __forceinline__ h16x8 pf_fin4(uint32_t b0, uint32_t b1, uint32_t b2, 
 }
 
 // eight nibbles (word byte t = w[t] | w[t+4] << 4) -> f16.  A byte up to 16 is, as an 8-bit float, 2^-9 of itself: two whole numbers a conversion, 11 instructions for eight weights
-// (with masks and an exponent, (x & m) | 0x6400 - 1024, 15).  The products' loops are bound by the sum of their matrix and vector instructions, about two of the latter a matrix
-// instruction hidden: 127 tokens of an 8B model in Q4_K_M, gate | up @PFA@ us
+// (with masks and an exponent, (x & m) | 0x6400 - 1024, 15).  The products' loops are bound by the sum of their matrix and vector instructions, about two of the latter a 16 x 16 matrix
+// instruction hidden: 2047 tokens of 16 layers of an 8B model in Q4_K_M 17.2 -> 16.9 ms, 128 of 32 layers 6.00 -> 5.91
 __device__ __forceinline__ h16x8 pf_frag_nib(uint32_t N, h16x2 S, h16x2 O) {
   const uint32_t m = 0x0F0F0F0Fu, lo = N & m, hi = (N >> 4) & m;
   auto two = [](uint32_t b, auto up) { return __builtin_bit_cast(h16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.0f, up.value)); };
