@@ -109,6 +109,7 @@ struct lgh_ctx {
   hipStream_t own_stream = nullptr, stream = nullptr;
   hipStream_t side_stream = nullptr;                  // the token behind a prompt block (engine.hip: tail_layer); the device's, not this context's own
   hipEvent_t side_go = nullptr, side_done = nullptr;
+  uint32_t *side_word = nullptr, *side_word_dev = nullptr, side_asked = 0;   // what the side stream answered last (pinned; as the device sees it), and the last question
   uint64_t beside_blocks = 0;                         // tokens that ran beside their block
   std::vector<lgh::LayerW> layers;
   // embedding table in native GGUF layout (row-dequantized per token) and the output projection

@@ -1040,7 +1040,9 @@ static void side_make(lgh_ctx* c) {
   SideStream* S = side_of(c);
   int* w = nullptr;
   bool ok = S && hipEventCreateWithFlags(&c->side_go, hipEventDisableTiming) == hipSuccess && hipEventCreateWithFlags(&c->side_done, hipEventDisableTiming) == hipSuccess &&
+            hipHostMalloc((void**)&c->side_word, 64, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess && hipHostGetDevicePointer((void**)&c->side_word_dev, c->side_word, 0) == hipSuccess &&
             hipMalloc((void**)&w, 8) == hipSuccess;
+  if (ok) *c->side_word = 0;
   if (ok) {
     std::lock_guard<std::mutex> lock(S->mu);
     if (!S->stream) {
@@ -1074,11 +1076,13 @@ static void side_leave(lgh_ctx* c) {
   if (c->side_stream) {
     SideStream* S = side_of(c);
     std::lock_guard<std::mutex> lock(S->mu);
+    (void)hipStreamSynchronize(S->stream);   // (a question that no prompt waited for)
     if (--S->users == 0) {
       (void)hipStreamDestroy(S->stream);
       S->stream = nullptr;
     }
   }
+  if (c->side_word) (void)hipHostFree(c->side_word);
   if (c->side_go) (void)hipEventDestroy(c->side_go);
   if (c->side_done) (void)hipEventDestroy(c->side_done);
 }
@@ -1086,19 +1090,19 @@ static void side_leave(lgh_ctx* c) {
 // (no stream of the caller's, no recording of launch times, no context that wants its launches one after the other, no model whose steps are not built layer by layer here)
 static bool tail_eligible(const lgh_ctx* c) { return c->side_stream && c->stream == c->own_stream && !c->lm && c->first && c->last && !c->profiling && !(c->d.flags & LGH_FLAG_NO_GRAPH) && pf_eligible(c); }
 
-// Has the side stream's queue nothing else to do?  Work on the null stream, which need not be this library's, would hold every layer of the step up.  An event is recorded when the prompt begins and has to be
-// there when the first layer's rows are under way, or some microseconds later, which the device does not notice: it has those launches in front of it
+// Has the side stream's queue nothing else to do?  Work on the null stream, which need not be this library's, would hold every layer of the step up.  A kernel that is launched there when the prompt begins has
+// to have answered when the first layer's rows are under way, or some microseconds later, which the device does not notice: it has those launches in front of it.  (An event's state is no measure: the runtime may
+// leave it to a thread of its own, and then it took longer than that from one prompt to the next.)
+__global__ void side_answer_kernel(uint32_t* w, uint32_t v) { __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 static hipError_t side_ask(lgh_ctx* c) {
-  const hipError_t e = hipEventRecord(c->side_done, c->side_stream);
-  if (e == hipSuccess && hipEventQuery(c->side_done) != hipSuccess) (void)hipGetLastError();   // (the runtime sends the event on its way with the first question)
-  return e;
+  hipLaunchKernelGGL(side_answer_kernel, dim3(1), dim3(1), 0, c->side_stream, c->side_word_dev, ++c->side_asked);
+  return hipGetLastError();
 }
 static bool side_idle(lgh_ctx* c) {
   const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(30);
   for (;;) {
-    const bool idle = hipEventQuery(c->side_done) == hipSuccess;
-    if (!idle) (void)hipGetLastError();   // (the next launch's check would find it)
-    if (idle || std::chrono::steady_clock::now() >= until) return idle;
+    if (__atomic_load_n(c->side_word, __ATOMIC_RELAXED) == c->side_asked) return true;
+    if (std::chrono::steady_clock::now() >= until) return false;
   }
 }
 
