@@ -394,7 +394,7 @@ int lgh_decode_greedy_multi(lgh_ctx* ctx, const uint32_t* slots, const uint32_t*
 const char* lgh_last_error(const lgh_ctx* ctx);
 int lgh_get_stats(lgh_ctx* ctx, lgh_stats* out);
 /* The token that lgh_eval wants logits of behind a stretch of others runs beside the last of their blocks where the context has a stream for
- * it, the block is not too large and no other prompt is at work on the device (the logits have the same bits either way).  possible: 1 if
+ * it, the work is neither too little nor too much for that and no other call is at work on the device (the logits have the same bits either way).  possible: 1 if
  * it has one; count: the tokens that ran so, up to now.  Either may be NULL. */
 int lgh_beside_blocks(lgh_ctx* ctx, int* possible, uint64_t* count);
 /* on: run eagerly with hipEvent pairs around every launch and accumulate lgh_stats.k_* */

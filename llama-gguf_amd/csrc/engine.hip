@@ -1391,6 +1391,11 @@ static int prefill_wide(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail* 
 // TinyLlama, 600: 4.79 and 4.35, 2047: 10.0 and 9.5; Mixtral widths, 2 layers, 600: 1.22 and 1.17, 2047: 2.58 and 2.53.  In blocks of 128, 8B widths, 10 tokens 0.99 and 0.83, 65: 1.18 and 1.06,
 // 129: 1.44 and 1.34.
 static bool tail_pays(const lgh_ctx* c, uint32_t m) { return (uint64_t)m * c->d.hidden_size <= 1536u * 4096u; }
+// And from this much on: its launches, kernel by kernel instead of a graph, take the host as long as a narrow model's block takes the device.  The block and then the step, us, and what both side by side take more or
+// less: 512 x 1536, 16 layers, 3 tokens 914 +19%, 33: 966 +10%, 50: 1057 0, 97: 1287 -9%; 1024 x 2816, 16 layers, 3: 1030 +9%, 33: 1068 +4%, 50: 1170 -5%, 97: 1442 -10%; 2048 x 5632, 22 layers, 3: 1628 -12%;
+// 2560 x 6912, 16 layers, 3: 1413 -17%; 4096 x 11008, 8 layers, 3: 930 -14%.  All tokens of the stretch count: behind earlier blocks the host is ahead of the device (512 x 1536, 200 tokens 2202 -5%).
+// (One layer: the step has nothing to go beside.)
+static bool tail_reaches(const lgh_ctx* c, size_t n) { return c->l1 - c->l0 >= 2 && (c->d.hidden_size >= 2048 || n * c->d.hidden_size >= 48u * 1024u); }
 
 // n prompt tokens on the batched path; `tail`: the token behind them, beside the last of their blocks
 static int prefill_tokens(lgh_ctx* c, const uint32_t* tokens, size_t n, PfTail* tail = nullptr) {
@@ -1912,14 +1917,15 @@ static int eval_stretch(lgh_ctx* c, const uint32_t* tokens, size_t n, uint32_t t
   const AtWork call(c);
   PfTail t{token, c->pos + n};
   c->attn_direct = t.pos + 1 <= direct_attn_rows(c);
-  if (call.alone) HIP_TRY(c, LGH_OPERATION_FAILED, side_ask(c));
-  int rc = prefill_tokens(c, tokens, n, call.alone ? &t : nullptr);
+  const bool beside = call.alone && tail_reaches(c, n);
+  if (beside) HIP_TRY(c, LGH_OPERATION_FAILED, side_ask(c));
+  int rc = prefill_tokens(c, tokens, n, beside ? &t : nullptr);
   if (!rc && !t.taken && !(rc = set_token(c, token))) rc = step(c, MODE_FORWARD);
   // the step that the next token takes, captured while the device works where it is not there yet: a first token behind a first prompt would wait for it (8B model 2.6 ms
   // instead of 1.57, its prompt of 128 tokens 6.0 either way)
   if (!rc) rc = ensure_graph(c, MODE_FORWARD);
   if (rc) {
-    if (call.alone) (void)hipStreamSynchronize(c->side_stream);   // nothing of the call goes on behind its error, and the next token's position is the one behind what is there
+    if (beside) (void)hipStreamSynchronize(c->side_stream);   // nothing of the call goes on behind its error, and the next token's position is the one behind what is there
     (void)hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, c->stream);
     (void)hipStreamSynchronize(c->stream);
     return rc;

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
     ("test-moe", "Q5_K_M", 700, 0),
 ])
 def test_a_step_beside_its_block(pkg, model, mix, max_seq, slots):
-    cfg = pkg.make_config(model, max_seq_len=max_seq)
+    cfg = pkg.make_config(model, max_seq_len=max_seq, hidden_size=2048, num_layers=2)   # (narrower models take it from more tokens on)
     m = pkg.SynthModel(cfg, mix=mix)
     beside, behind = (pkg.HipGpuInference.from_model(m, max_seq) for _ in range(2))
     assert beside.prefill_is_batched()
@@ -75,9 +75,32 @@ def test_large_blocks_go_first(pkg):
     behind.close()
 
 
+def test_narrow_models_from_more_tokens_on(pkg):
+    """A model of width 1024: stretches of 48 tokens and more have the step beside their block, shorter ones in front of it."""
+    cfg = pkg.make_config("test-dense", max_seq_len=300, hidden_size=1024, num_layers=2)
+    m = pkg.SynthModel(cfg, mix="Q4_K_M")
+    beside, behind = (pkg.HipGpuInference.from_model(m, 300) for _ in range(2))
+    if not beside.beside_blocks()[0]:
+        pytest.skip("no stream here runs beside the context's own")
+    tok = np.random.default_rng(8).integers(0, cfg.vocab_size, 300).astype(np.uint32)
+    for block, goes in ((2, False), (47, False), (48, True), (128, True), (131, True)):
+        for attempt in range(5):
+            beside.reset()
+            before = beside.beside_blocks()[1]
+            got = beside.eval(tok[:block + 1], [block])[0]
+            if beside.beside_blocks()[1] > before:
+                break
+        assert (beside.beside_blocks()[1] > before) == goes, block
+        behind.reset()
+        behind.forward_batch(tok[:block])
+        assert np.array_equal(got.view(np.uint32), behind.forward(int(tok[block])).view(np.uint32)), block
+    beside.close()
+    behind.close()
+
+
 def test_the_step_behind_a_first_prompt_is_there(pkg):
     """A prompt's last token is launched kernel by kernel where it runs beside its block; the graph that the tokens after it take is captured in the same call, not in theirs."""
-    m = pkg.SynthModel(pkg.make_config("test-dense", max_seq_len=300), mix="Q4_K_M")
+    m = pkg.SynthModel(pkg.make_config("test-dense", max_seq_len=300, hidden_size=2048, num_layers=2), mix="Q4_K_M")
     eng = pkg.HipGpuInference.from_model(m, 300)
     assert eng.stats()["graph_nodes"] == 0
     eng.eval(np.arange(40) % m.config.vocab_size, [39])
@@ -90,7 +113,7 @@ def test_the_step_behind_a_first_prompt_is_there(pkg):
 
 def test_contexts_at_work_share_one_stream(pkg):
     """The device has one stream for such steps, taken by one prompt at a time and only while no other is at work: contexts in threads give what each gives alone, and contexts come and go around it."""
-    m = pkg.SynthModel(pkg.make_config("test-dense-d128", max_seq_len=400), mix="Q4_K_M")
+    m = pkg.SynthModel(pkg.make_config("test-dense-d128", max_seq_len=400, hidden_size=2048, num_layers=2), mix="Q4_K_M")
     tok = np.random.default_rng(7).integers(0, m.config.vocab_size, 400).astype(np.uint32)
     lengths = (3, 40, 129, 300)
     first = pkg.HipGpuInference.from_model(m, 400)
