@@ -1,5 +1,6 @@
 """The token behind a prompt block, whose step runs beside the block (engine.hip, tail_layer), against the block and then the step: all bits equal, its own logits and those of the tokens after it.  Portions
 around one block (128 tokens) and a remainder of one token, from nothing and behind earlier tokens, several wanted places, short and long contexts (the two forms of attention), mixtures, a context with slots."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -108,6 +109,29 @@ def test_the_step_behind_a_first_prompt_is_there(pkg):
     assert nodes > 0
     eng.forward(3)
     assert eng.stats()["graph_nodes"] == nodes
+    eng.close()
+
+
+def test_work_on_the_null_stream_sends_the_step_behind(pkg):
+    """The stream shares the null stream's queue: while others' work is in it, a step goes behind its block and waits for none of that."""
+    m = pkg.SynthModel(pkg.make_config("test-dense", max_seq_len=200, hidden_size=2048, num_layers=2), mix="Q4_K_M")
+    eng = pkg.HipGpuInference.from_model(m, 200)
+    if not eng.beside_blocks()[0]:
+        pytest.skip("no stream here runs beside the context's own")
+    tok = np.arange(150) * 7 % m.config.vocab_size
+    want = eng.eval(tok, [149])[0]
+    hip, big, words = C.CDLL(pkg.hip_backend.load_library()._name), C.c_void_p(), 1 << 28   # (the same library: its runtime's functions are found through it)
+    assert hip.hipMalloc(C.byref(big), C.c_size_t(words * 4)) == 0
+    for _ in range(3):
+        eng.reset()
+        before = eng.beside_blocks()[1]
+        for k in range(50):                       # some 0.2 ms each
+            assert hip.hipMemsetD32Async(big, k, C.c_size_t(words), None) == 0
+        got = eng.eval(tok, [149])[0]
+        assert eng.beside_blocks()[1] == before
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        assert hip.hipStreamSynchronize(None) == 0
+    assert hip.hipFree(big) == 0
     eng.close()
 
 
