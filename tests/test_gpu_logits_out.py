@@ -51,7 +51,7 @@ def test_the_callers_pages_keep_what_they_hold_until_the_result(pkg):
     lib, n = pkg.hip_backend.load_library(), 16
     slots = np.arange(n, dtype=np.uint32)
     buf = np.empty(n * cfg.vocab_size * 4, np.uint8)
-    heads = buf[::4096]
+    heads, looks = buf[::4096], 0
     for step in range(20):
         tokens = (slots * 31 + step).astype(np.uint32)
         buf[:] = 0xA5
@@ -61,7 +61,9 @@ def test_the_callers_pages_keep_what_they_hold_until_the_result(pkg):
         while t.is_alive():
             seen.append(heads.copy())
         t.join()
-        assert rc == [0] and seen
+        assert rc == [0]
+        looks += len(seen)
         odd = [int(((s != 0xA5) & (s != heads)).sum()) for s in seen]
         assert not any(odd), (step, odd)
+    assert looks > 0
     eng.close()
