@@ -78,6 +78,7 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
   constexpr uint32_t tb = pf_tile_bytes(F), NB = pw_bufs<F>(), DIST = NB - 1;
   constexpr int NX = TT;   // NX: activation DMA operations per wave and step
   constexpr int UN = 4 * TT, AHEAD = 3;                                                     // units (phase, token tile) of a step
+  constexpr int RPP = TT > 4 ? 2 : 1, RU = TT / RPP;                                        // regions of a phase, units of a region
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t n = lane & 15, g = lane >> 5, tk = lane & 31, sub = lane >> 4 & 1;
   const uint32_t per = (G.nblk + G.S - 1) / G.S, b0 = ks * per, b1 = b0 + per < G.nblk ? b0 + per : G.nblk;
@@ -119,19 +120,20 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(at) : "memory", "m0");
     }
   };
-  // activations: an operation covers 8 tokens x 128 bytes; chunk q of token t lies at position q ^ (t & 7)
+  // activations: an operation covers 8 tokens x 128 bytes; chunk q of token t lies at position q ^ (t >> 1 & 7): 16 tokens' places
+  // differ in their banks, two of a parity included (with t & 7 every second read waited for another; two thirds fewer LDS cycles, experts' gate | up of 600 tokens 464 -> 460 us)
   uint32_t xoff[NX];
 #pragma unroll
   for (int i = 0; i < (int)NX; i++) {
     const uint32_t row = (wave * NX + i) * 8 + (lane >> 3);
     uint32_t m = m0 + row < m_end ? m0 + row : m_end - 1;
     if (GRP && G.src) m = (uint32_t)G.src[m];
-    xoff[i] = m * (G.nblk * 512u) + (((lane & 7) ^ (row & 7)) << 4);
+    xoff[i] = m * (G.nblk * 512u) + (((lane & 7) ^ (row >> 1 & 7)) << 4);
   }
   const uint32_t s0 = b0 * 4, s1 = b1 * 4;   // steps of 64 elements
   // regions of a step; raw operations per region, spread over a block's first two steps, and how many of them each of the two makes
-  constexpr int RS = UN / 4, RP = (R + 2 * RS - 1) / (2 * RS), R0 = R < RS * RP ? R : RS * RP, R1 = R - R0;
-  static_assert((int)NX == RS, "one activation operation per region");
+  constexpr int RS = 4 * RPP, RP = (R + 2 * RS - 1) / (2 * RS), R0 = R < RS * RP ? R : RS * RP, R1 = R - R0;
+  static_assert(TT % RPP == 0 && NX <= RS && RU >= AHEAD, "an activation operation a region at most; the last one holds what is awaited");
   auto x_dma = [&](int i, uint32_t s, uint32_t buf) {   // operation i of a step's activations
     const uint8_t* base = G.x + (size_t)(s < s1 ? s : s1 - 1) * 128;   // past the end: requested again, never read
     pw_dma(base, xoff[i], lds0 + buf * kWStepBytes + (wave * NX + i) * 1024);
@@ -157,7 +159,7 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
 
   uint32_t bo[4];   // this lane's place in a token tile, per phase
 #pragma unroll
-  for (int p = 0; p < 4; p++) bo[p] = tk * 128 + (((4 * g + p) ^ (tk & 7)) << 4);
+  for (int p = 0; p < 4; p++) bo[p] = tk * 128 + (((4 * g + p) ^ (tk >> 1 & 7)) << 4);
   PfRaw w[2][2];    // [v][j]
   h16x2 S[2], O[2];
   h16x8 af[2][2], bf[4];
@@ -189,17 +191,17 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
         for (int i = 0; i < NX; i++) x_dma(i, s + DIST, far);
       }
 #pragma unroll
-      for (int r = 0; r < RS; r++) {   // regions of 4 units: 8 MFMAs, 4 operand reads, one or both of the next phase's A operands, and the DMA piece by piece
-        if (NB == 3) x_dma(r, s + DIST, far);
+      for (int r = 0; r < RS; r++) {   // regions of 3 or 4 units: two MFMAs and an operand read each, one or both of the next phase's A operands, and the DMA piece by piece
+        if (NB == 3 && r < NX) x_dma(r, s + DIST, far);
         if (pp < 2) {
 #pragma unroll
           for (int k = (pp * RS + r) * RP; k < (pp * RS + r + 1) * RP; k++)
             if (k < R) raw_dma(k, b + 1 < b1 ? b + 1 : b);
         }
-        const int p = r / (TT / 4);
+        const int p = r / RPP;
 #pragma unroll
-        for (int v4 = 0; v4 < 4; v4++) {
-          const int u = r * 4 + v4;
+        for (int ru = 0; ru < RU; ru++) {
+          const int u = r * RU + ru;
           if (u == UN - AHEAD) {   // the last reads of this buffer were issued by the unit before
             __builtin_amdgcn_sched_barrier(0);
             constexpr uint32_t XW = NB == 3 ? NX : 0;   // what this step has requested for later ones may be under way
@@ -213,20 +215,20 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
 #pragma unroll
           for (int v = 0; v < 2; v++) pw_mma(acc[v][u % TT], af[p & 1][v], bf[u & 3]);
         }
-        const int p2 = (p + 1) & 3, pp2 = p == 3 ? (pp + 1) & 3 : pp, ri = r % (TT / 4);
-        if (TT == 8) {
+        const int p2 = (p + 1) & 3, pp2 = p == 3 ? (pp + 1) & 3 : pp, ri = r % RPP;
+        if (RPP == 2) {
           operand(ri, pp2, p2, af[p2 & 1][ri]);
         } else {
           operand(0, pp2, p2, af[p2 & 1][0]);
           operand(1, pp2, p2, af[p2 & 1][1]);
         }
-        if (pp == 3 && p == 2 && ri == TT / 4 - 1) raw_read();   // the block's last operands are made: the next block's weights
+        if (pp == 3 && p == 2 && ri == RPP - 1) raw_read();   // the block's last operands are made: the next block's weights
         // one MFMA keeps the matrix pipe busy for 32 cycles, in which this wave can issue a few other instructions: a quarter of the region's between any two
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < 2 * RU; i++) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // MFMA
           if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // LDS read
-          __builtin_amdgcn_sched_group_barrier(0x002, TT == 8 ? 3 : 6, 0);      // vector
+          __builtin_amdgcn_sched_group_barrier(0x002, 24 * (3 - RPP) / (2 * RU), 0);   // vector
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -286,9 +288,9 @@ template <uint32_t MASK, bool GRP, int EPI>
 __global__ void __launch_bounds__(kWWaves * 64) pw_gemm_kernel(const PfWide G, uint32_t n_rg, uint32_t tiles_m) {
   extern __shared__ __attribute__((aligned(16))) uint8_t pw_smem[];
   // token tiles of one weight panel side by side on one XCD (workgroups go round-robin over the 8 XCDs): the panel comes from HBM once per XCD.  A last
-  // token tile that is at most half full takes half the time: its workgroups are the last ones, to fill up the last round.
+  // token tile that is at most three quarters or half full takes so much of the time: its workgroups are the last ones, to fill up the last round.
   uint32_t t = blockIdx.x, total = gridDim.x, wide = tiles_m, tm0 = 0;
-  if (!GRP && tiles_m > 1 && (G.m - 1) % kPfwTile < kPfwTile / 2) {
+  if (!GRP && tiles_m > 1 && (G.m - 1) % kPfwTile < kPfwTile * 3 / 4) {
     const uint32_t first = n_rg * G.S * (tiles_m - 1);
     wide = t < first ? tiles_m - 1 : 1;
     tm0 = t < first ? 0 : tiles_m - 1;
@@ -320,10 +322,13 @@ __global__ void __launch_bounds__(kWWaves * 64) pw_gemm_kernel(const PfWide G, u
   const PfwSeg& sg = G.seg[si];
   const uint32_t rg = rgid - sg.rg_begin;
   auto is = [&](int f) { return (MASK & (1u << f)) && (MASK == (1u << f) || sg.fmt == f); };
+  // Tiles of 256, 192 and 128 tokens: a product takes time with the tokens computed (experts of some 100 to 190 rows, 401 tokens of Mixtral widths: gate | up 364 -> 323 us with the middle one;
+  // a last tile of 1200 and 1700 tokens, 4 layers of an 8B model: 2.55 -> 2.46 and 3.43 -> 3.34 ms)
 #define LGH_PW_RUN(F)                                                                                       \
   do {                                                                                                      \
-    if (m_end - m0 > (uint32_t)kPfwTile / 2) pw_body<F, 8, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); \
-    else pw_body<F, 4, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);                                      \
+    if (m_end - m0 > (uint32_t)kPfwTile * 3 / 4) pw_body<F, 8, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);  \
+    else if (m_end - m0 > (uint32_t)kPfwTile / 2) pw_body<F, 6, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); \
+    else pw_body<F, 4, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);                                          \
   } while (0)
   if (is(PF_Q4K)) LGH_PW_RUN(PF_Q4K);
   else if (is(PF_Q6K)) LGH_PW_RUN(PF_Q6K);

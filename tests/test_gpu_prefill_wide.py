@@ -113,6 +113,23 @@ def test_long_prompts_without_their_own_memory_take_the_short_blocks(pkg):
         e.close()
 
 
+@pytest.mark.parametrize("name,mix,n", [("test-dense", "Q4_K_M", 385), ("test-dense", "Q8_0", 448), ("test-dense", "Q6_K", 449), ("test-dense", "Q4_0", 704), ("test-dense", "Q5_K_M", 420),
+                                        ("test-moe", "Q5_K_M", 290), ("test-moe", "Q6_K", 350), ("test-moe", "Q4_0", 330), ("test-moe", "Q4_K_M", 384)])
+def test_last_tiles_of_up_to_192_tokens(pkg, name, mix, n):
+    """The body for 129 to 192 tokens: a last tile's first, last and first beyond its range, experts whose rows fall into it (four of them, two a token).  A token's sums are the same in a tile of any
+    size, so the cache is, bit for bit, what the same tokens leave as part of a prompt whose last tile is full."""
+    full = (n + 255) // 256 * 256
+    cfg = pkg.make_config(name, max_seq_len=full + 16)
+    model = pkg.SynthModel(cfg, mix=mix)
+    a, b = (pkg.HipGpuInference.from_model(model, full + 16) for _ in range(2))
+    prompt = [(7 * i + 3) % cfg.vocab_size for i in range(full)]
+    a.forward_batch(prompt[:n])
+    b.forward_batch(prompt)
+    b.kv_truncate(n)
+    for t in (5, 77, 9):
+        assert np.array_equal(a.forward(t), b.forward(t))
+
+
 @pytest.mark.parametrize("n", [200, 300])
 def test_stages_against_one_context(pkg, n):
     """Stages hand blocks of 128 tokens over: below 256 tokens the bits of a single context, which takes the long path from there on, behind it its rounding."""
