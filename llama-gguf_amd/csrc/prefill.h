@@ -30,12 +30,12 @@ struct PfGemm {
   float* part;           // [S][part_rows][ncols]
   uint32_t part_rows;    // rows per split: 128, or kPfMoeRows when the experts of a MoE layer share one buffer
   const int* row_base;   // optional (MoE): device word, first row of this expert's batch in the buffer
-  uint32_t m_tiles;      // token tiles that hold real tokens
-  const int* m_count;    // optional (MoE): device word with the number of real rows; overrides m_tiles, 0 rows = nothing to do
-  // gate | up with SwiGLU: the activations (XH), the input's sums of squares and the norm they stand for, the tokens
+  uint32_t m_tokens;
+  const int* m_count;    // optional (MoE): device word with the number of real rows; overrides m_tokens, 0 rows = nothing to do
+  // gate | up with SwiGLU: the activations (XH), the input's sums of squares and the norm they stand for
   uint8_t* act;
   const float* ssq;
-  uint32_t n_ssq, norm_cols, m_tokens;
+  uint32_t n_ssq, norm_cols;
   float eps;
 };
 
@@ -45,7 +45,7 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
                           uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t expert = 0, const int* m_count = nullptr,
                           uint32_t part_rows = kPfTokens, const int* row_base = nullptr);
 // silu(gate) * up of one launch -> XH
-bool pf_pairs(const DevWeight* gate, const DevWeight* up, uint32_t m_tokens);
+bool pf_pairs(const DevWeight* gate, const DevWeight* up);
 hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint8_t* xh, uint8_t* act, const float* ssq, uint32_t norm_cols, float eps, uint32_t m_tokens, hipStream_t st);
 hipError_t pf_row_epi_launch(const float* part, uint32_t S, uint32_t ncols, uint32_t col0, const float* bias, float* hidden, uint32_t H,
                              const float* nw, uint8_t* xh, float* ssq, uint32_t m_tokens, hipStream_t st, const float* moe_w = nullptr);

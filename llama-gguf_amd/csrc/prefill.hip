@@ -25,11 +25,10 @@
 // elements of K (copied verbatim into LDS by LDS-DMA), inside a slab token t owns 512 B = 32 chunks of 8 elements, chunk
 // q stored at position q ^ (t & 15) (so that the 16 tokens of an MFMA operand read 16 different LDS banks groups).
 //
-// GEMM: a workgroup = 4 waves = 256 weight rows x one k-range x all 128 tokens; a wave = 4 row tiles (64 rows): weights
-// go HBM -> registers -> f16 (never through LDS: the dequantized lane layout IS the A operand), an activation fragment
-// read from LDS feeds 4 MFMAs (LDS at 50 % of its bandwidth), 128 f32 accumulators per lane.  K is split over
-// gridDim.y workgroups to fill the chip; the f32 partial sums [split][token][column] are added up by the row-wise
-// kernel that consumes them (together with bias, RoPE, residual, RMSNorm, SwiGLU).
+// GEMM: weights go HBM -> registers -> f16 (never through LDS: the dequantized lane layout IS the A operand), activations by LDS-DMA.  Dense layers: a workgroup = 8 waves = 128 weight
+// rows x one k-range x all tokens in tiles of 32, in two teams that halve every block of k (pf_team).  A mixture's experts: 4 waves = 256 weight rows, a wave 4 row tiles (64 rows), an
+// activation fragment feeds 4 MFMAs (pf_body).  K is split over gridDim.y workgroups to fill the chip; the f32 partial sums [split][token][column] are added up by the row-wise kernel that
+// consumes them (together with bias, RoPE, residual, RMSNorm, SwiGLU).
 #include <type_traits>
 
 #include "device_utils.h"
@@ -218,11 +217,10 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
   LGH_PF_STAMP(14);
 }
 
-// MT: token tiles, known at launch but for a mixture's experts (0: chosen in the kernel).  One kernel with all three bodies has the registers and the
-// LDS of the largest and is scheduled as one: 8 layers of an 8B model, 33 / 64 / 100 / 128 tokens 756 / 825 / 1059 / 1126 us, a kernel each 738 / 800 / 1022 / 1085.
-// (Up to 32 tokens no difference; more k-splits with two workgroups a CU there: 625 -> 684 us, the partial sums.)
-template <uint32_t MASK, int MT>
-__device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem) {
+// A mixture's experts: the token tiles are chosen in the kernel
+template <uint32_t MASK>
+__global__ void __launch_bounds__(kPfWaves * 64) pf_experts_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
   const uint32_t rgid = blockIdx.x;
   int si = 0;
   if (G.nseg > 1 && rgid >= G.seg[1].rg_begin) si = 1;
@@ -230,17 +228,13 @@ __device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem
   const PfSeg& sg = G.seg[si];
   const uint32_t rg = rgid - sg.rg_begin;
   auto is = [&](int f) { return (MASK & (1u << f)) && (MASK == (1u << f) || sg.fmt == f); };
-  uint32_t m_tiles = G.m_tiles;
-  if (G.m_count) {   // MoE: this expert's row count lives on the device (no host round trip per layer)
-    uint32_t cnt;
-    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cnt) : "s"(G.m_count) : "memory");
-    if (cnt == 0) return;
-    m_tiles = (cnt + 15) / 16;
-  }
+  uint32_t cnt;   // this expert's row count lives on the device (no host round trip per layer)
+  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cnt) : "s"(G.m_count) : "memory");
+  if (cnt == 0) return;
+  const uint32_t m_tiles = (cnt + 15) / 16;
 #define LGH_PF_RUN(F)                                                                    \
   do {                                                                                   \
-    if constexpr (MT != 0) pf_body<F, MT>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);      \
-    else if (m_tiles <= 2) pf_body<F, 2>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);       \
+    if (m_tiles <= 2) pf_body<F, 2>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);            \
     else if (m_tiles <= 4) pf_body<F, 4>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);       \
     else pf_body<F, kPfMT>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);                     \
   } while (0)
@@ -251,38 +245,223 @@ __device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem
   else if (is(PF_Q40)) LGH_PF_RUN(PF_Q40);
 #undef LGH_PF_RUN
 }
-template <uint32_t MASK>
-__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) {   // blocks of more than 64 tokens
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-  pf_gemm_device<MASK, kPfMT>(G, pf_smem);
-}
-template <uint32_t MASK, int MT>
-__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_few_kernel(const PfGemm G) {   // of up to 32 / 64, and a mixture's experts
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-  pf_gemm_device<MASK, MT>(G, pf_smem);
-}
 
 // 1 / rms of token t from the per-chunk sums of squares its producer left (simd.rs:847-878); 1 when there is no norm
 __device__ __forceinline__ float pf_inv_rms(const float* ssq, uint32_t n_ssq, uint32_t t, uint32_t H, float eps) {
   if (!ssq) return 1.0f;
+  // all that a token may have at once: a loop over those there are waits for each (64 tokens of gate | up: 4.5 us of the launch)
+  const f32x4 a = *reinterpret_cast<const f32x4*>(ssq + t * kPfSsqChunks), b = *reinterpret_cast<const f32x4*>(ssq + t * kPfSsqChunks + 4);
   float tot = 0.0f;
-  for (uint32_t j = 0; j < n_ssq; j++) tot += ssq[t * kPfSsqChunks + j];
+#pragma unroll
+  for (uint32_t j = 0; j < (uint32_t)kPfSsqChunks; j++) {
+    const float v = j < 4 ? a[j & 3] : b[j & 3];
+    tot = j < n_ssq ? tot + v : tot;
+  }
   return 1.0f / __builtin_sqrtf(tot / (float)H + eps);
 }
 
-// silu(gate) * up without partial sums: a wave has the 16 gate rows and the 16 up rows of the same columns as one tile of 32 over all of k, and up to 32 TT tokens, on
-// v_mfma_f32_32x32x16_f16 (less power per product than the 16 x 16 shape, and power is what bounds these loops).  Lane 32g + 16s + n holds row n of gate (s = 0) or up (1), and of every 64 elements
-// the two 16-element chunks 2g + j that the tile16 layout keeps for lanes 16(2g + j) + n; a block has 16 phases (pp, j, h), each the contraction of elements 64pp + 16(2g + j) + 8h .. + 7 of both g.
-// 127 / 64 / 32 tokens of an 8B model in Q4_K_M (28672 rows of 4096): 44 / 26 / 19.5 us a layer, products in two k-ranges and SwiGLU behind them 52 / 36 / 29.  On the 16 x 16 shape 127 tokens took 46.5;
-// three blocks requested ahead instead of one changed nothing at 64 tokens and saved 1.6 us at 32 (two teams save 3).  The weights alone take 13 us.
-// KH 2: two teams of waves, each over half of k, the second's sums through LDS.  With up to 64 tokens a block is mostly dequantization, and two waves a SIMD issue it twice as fast as one.
-template <int F, int TT, int KH>
-__global__ void __launch_bounds__(KH * kPfWaves * 64) pf_pair_kernel(const PfGemm G) {
+// Blocks of a dense model: a wave has 32 weight rows and up to 32 TT tokens on v_mfma_f32_32x32x16_f16 (less power per product than the 16 x 16 shape, and power is what bounds these loops).  Lane
+// 32g + 16s + n holds row n of 16-row tile s, and of every 64 elements the two 16-element chunks 2g + j that the tile16 layout keeps for lanes 16(2g + j) + n; 256 elements have 16 phases (pp, j, h), each
+// the contraction of elements 64pp + 16(2g + j) + 8h .. + 7 of both g.
+//   PAIR   the tiles are the 16 gate rows and the 16 up rows of the same columns, over all of k: SwiGLU in registers, no partial sums
+//   else   32 rows of one matrix over the blocks of a k-range (blockIdx.y), partial sums as pf_body
+// Eight waves in two teams: both walk all blocks, team 0 with the first 128 elements of each and their weights, team 1 with the others; their sums meet through LDS.  So two waves a SIMD hide what one waits for (with
+// one, 42 % of the cycles issued, 29 % waited for memory or the barrier and 29 % for the matrix cores), and a wave needs half of a block's raw weights, which leaves registers to ask for them two blocks ahead.
+// 128 weight rows a workgroup instead of 256: half as many k-ranges fill the chip, and half the partial sums.  8B model, Q4_K_M, us a layer, four waves of 64 rows (gate | up: of 32) and here:
+//   127 tokens  gate | up 44 and 38, SwiGLU included; wo, QKV, down 16.5, 18.7, 26.5 and 14.8, 18.2, 25.2; the residual's fold 7.1 and 5.2
+//    96 tokens  (three tiles; four before) gate | up 43.7 and 30.7; wo, QKV, down 15.0, 18.3, 25.6 and 12.1, 15.0, 21.6; fold 6.2 and 5.4
+//    49 tokens  gate | up 25.5 and 26.5; wo, QKV, down 11.6, 14.1, 18.1 and 10.3, 10.4, 17.6; fold 5.0 and 4.8
+//    19 tokens  (gate | up: pf_pair_few_kernel) wo, QKV, down 7.9, 11.2, 14.0 and 7.3, 8.9, 13.5; fold 4.9 and 4.7
+constexpr uint32_t pf_half_lds(int tt) { return (uint32_t)tt * 2 * 32 * 512; }
+template <int F> constexpr uint32_t pf_half_loads() { return F == PF_Q6K ? 6 : F == PF_Q5K || F == PF_Q80 ? 5 : 3; }   // vector-memory operations of a load below
+// the raw weights of 128 elements (TEAM) of one block: chunks 2g and 2g + 1 of row n.  pf_scale and pf_frag read what belongs to their step only
+template <int F, int TEAM>
+__device__ __forceinline__ void pf_half_load(PfRaw (&to)[2], const uint8_t* tile, uint32_t g, uint32_t n) {
+  const u32x4 hd = ldg_nt128(tile + (F == PF_Q6K ? 3072 : F == PF_Q80 ? 4096 : 2048) + n * 16);
+  uint32_t dh = 0;
+  if (F == PF_Q6K) dh = ldg_nt32(tile + 3328 + (n >> 1) * 4);
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const uint32_t l16 = 16 * (2 * g + j) + n;
+    to[j].hd = hd;
+    if (F == PF_Q80) {
+      to[j].q[2 * TEAM] = ldg_nt128(tile + 2 * TEAM * 1024 + l16 * 16);
+      to[j].q[2 * TEAM + 1] = ldg_nt128(tile + (2 * TEAM + 1) * 1024 + l16 * 16);
+    } else {
+      to[j].q[TEAM] = ldg_nt128(tile + TEAM * 1024 + l16 * 16);
+      if (F == PF_Q6K) {
+        const u32x2 h = ldg_nt64(tile + 2048 + l16 * 16 + TEAM * 8);
+        if (TEAM == 0) { to[j].q[2].x = h.x; to[j].q[2].y = h.y; }
+        else { to[j].q[2].z = h.x; to[j].q[2].w = h.y; }
+        to[j].q[3].x = dh;
+      }
+      if (F == PF_Q5K) {
+        const uint32_t h = ldg_nt32(tile + 2304 + l16 * 8 + TEAM * 4);
+        if (TEAM == 0) to[j].q[2].x = h;
+        else to[j].q[2].y = h;
+      }
+    }
+  }
+}
+
+// one team's sums over the blocks [b0, b1); wrow: its lanes' 16-row tiles
+template <int F, int TT, int TEAM, typename M>
+__device__ __forceinline__ void pf_team(const PfGemm& G, const uint8_t* wrow, uint32_t b0, uint32_t b1, uint8_t* smem, f32x16 (&acc)[TT], M meanwhile) {
+  constexpr uint32_t kBuf = (uint32_t)TT * 32 * 512, kDma = kBuf / (2 * kPfWaves), tb = pf_tile_bytes(F), LOADS = pf_half_loads<F>();
+  constexpr int AHEAD = 2;                                            // phases the activations are read ahead
+  const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t n = lane & 15, g = lane >> 5, tk = lane & 31;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  auto x_dma = [&](uint32_t b) {   // an eighth of a block's activations
+    const uint8_t* src = G.xh + (size_t)b * kPfSlabBytes + wave * kDma;
+    const uint32_t dst = lds_base + (b & 1) * kBuf + wave * kDma;
+#pragma unroll
+    for (int i = 0; i < (int)(kDma / 1024); i++)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane * 16), "s"(src + i * 1024), "s"(dst + i * 1024) : "memory", "m0");
+  };
+  PfRaw w[3][2];   // [block in turn][j]
+  x_dma(b0);
+  if (b0 + 1 < b1) x_dma(b0 + 1);
+  const uint8_t* from = wrow + (size_t)b0 * tb;
+  auto load = [&](uint32_t b, PfRaw (&to)[2]) {   // (past the end the last ones again: the waits below count them)
+    pf_half_load<F, TEAM>(to, from, g, n);
+    from += b + 1 < b1 ? tb : 0u;
+  };
+  load(b0, w[0]);
+  load(b0 + 1, w[1]);
+#pragma unroll
+  for (int t = 0; t < TT; t++) acc[t] = (f32x16)(0.0f);
+  meanwhile();
+  // all but the newest weights (asked for behind everything that is awaited) have arrived, and every wave has read what it will of the buffer in turn
+  auto landed = [&](auto more) {
+    __builtin_amdgcn_s_waitcnt(more.value ? 0x0070 | LOADS : 0x0070);   // vmcnt(LOADS or 0) lgkmcnt(0); the builtin: see pf_body
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  landed(std::true_type{});
+  h16x8 af[2], bf[4][TT];
+  h16x2 S, O;
+  auto read_bf = [&](uint32_t b, int p) {   // p = 4 (pp - 2 TEAM) + 2 j + h
+    const uint32_t q = (uint32_t)(16 * TEAM + 8 * (p >> 2) + (p & 3)) + 4 * g;
+#pragma unroll
+    for (int t = 0; t < TT; t++) bf[p & 3][t] = *reinterpret_cast<const h16x8*>(smem + (b & 1) * kBuf + (t * 32 + tk) * 512 + ((q ^ n) << 4));
+  };
+  auto frag = [&](const PfRaw (&cw)[2], int p) {
+    const int pp = 2 * TEAM + (p >> 2), j = p >> 1 & 1;
+    if ((p & 3) == 0 || (F == PF_Q6K && (p & 1) == 0)) pf_scale<F>(cw[j], pp, n, 2 * g + j, S, O);
+    af[p & 1] = pf_frag<F>(cw[j], pp, p & 1, S, O);
+  };
+  // more: it asks for weights.  (What the last one reads of the buffer and the registers beyond the end is not used)
+  auto block = [&](auto more, uint32_t b, PfRaw (&cw)[2], PfRaw (&nw)[2], PfRaw (&ow)[2]) {
+    if constexpr (more.value) load(b + 2, ow);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < 8; p++) {
+      if (p == 8 - AHEAD) {
+        landed(more);
+        if (more.value && b + 2 < b1) x_dma(b + 2);
+      }
+      if (p + AHEAD < 8) read_bf(b, p + AHEAD);
+      else read_bf(b + 1, p + AHEAD - 8);
+      if (p < 7) frag(cw, p + 1);
+      else frag(nw, 0);
+#pragma unroll
+      for (int t = 0; t < TT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[p & 1], bf[p & 3][t], acc[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < AHEAD; p++) read_bf(b0, p);
+  frag(w[0], 0);
+  uint32_t b = b0;   // (whole turns, then what is left: with a test inside the loop the compiler sees a way round on which a block's weights are still under way, and waits for them)
+  for (; b + 3 <= b1; b += 3) {
+    block(std::true_type{}, b, w[0], w[1], w[2]);
+    block(std::true_type{}, b + 1, w[1], w[2], w[0]);
+    block(std::true_type{}, b + 2, w[2], w[0], w[1]);
+  }
+  if (b < b1) block(std::false_type{}, b, w[0], w[1], w[2]);
+  if (b + 1 < b1) block(std::false_type{}, b + 1, w[1], w[2], w[0]);
+}
+
+template <int F, int TT, bool PAIR>
+__device__ __forceinline__ void pf_half_device(const PfGemm& G, const PfSeg& sg, uint32_t rg, uint32_t ks, uint8_t* smem) {
+  constexpr int OWN = (TT + 1) / 2;   // token tiles whose sums team 0 puts together; team 1 has the others
+  const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6 & 3)), team = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+  const uint32_t s = lane >> 4 & 1, g = lane >> 5, tk = lane & 31;
+  const uint32_t unit = rg * kPfWaves + wave;                                   // PAIR: a tile of each matrix, else two tiles
+  const uint32_t want = PAIR ? unit : 2 * unit + s, tl = want < sg.ntiles ? want : sg.ntiles - 1;   // clamped: loads are unconditional
+  const uint8_t* const wrow = (PAIR && s ? G.seg[1].w : sg.w) + (size_t)tl * G.nblk * pf_tile_bytes(F);
+  const uint32_t per = (G.nblk + G.S - 1) / G.S, b0 = ks * per, b1 = b0 + per < G.nblk ? b0 + per : G.nblk;
+  f32x16 acc[TT];
+  float inv[TT];   // 1 / rms of this lane's tokens
+  auto norms = [&] {
+    if (PAIR) {
+#pragma unroll
+      for (int t = 0; t < TT; t++) inv[t] = pf_inv_rms(G.ssq, G.n_ssq, t * 32 + tk, G.norm_cols, G.eps) * (1.0f / kPfScale);
+    }
+  };
+  if (team == 0) pf_team<F, TT, 0>(G, wrow, b0, b1, smem, acc, norms);
+  else pf_team<F, TT, 1>(G, wrow, b0, b1, smem, acc, norms);
+  // lane (tk, g) has of token 32 t + tk rows 8i + 4g .. + 3, i = 0 .. 3.  A team leaves the tiles that the other one owns in LDS (36 floats a token: banks) and adds what it finds there to its own
+  float* const place = reinterpret_cast<float*>(smem) + wave * (TT * 32 * 36) + tk * 36 + 4 * g;
+  __syncthreads();   // (every read of the slabs has returned)
+#pragma unroll
+  for (int t = 0; t < TT; t++)
+    if ((t < OWN) != (team == 0)) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) *reinterpret_cast<f32x4*>(place + t * 32 * 36 + 8 * i) = f32x4{acc[t][4 * i], acc[t][4 * i + 1], acc[t][4 * i + 2], acc[t][4 * i + 3]};
+    }
+  __syncthreads();
+  if (PAIR && unit >= sg.ntiles) return;
+#pragma unroll
+  for (int t = 0; t < TT; t++) {
+    if ((t < OWN) != (team == 0)) continue;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(place + t * 32 * 36 + 8 * i);
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[t][4 * i + e] += v[e];
+    }
+    if constexpr (PAIR) {   // gate with i = 0, 1, up with i + 2
+      const uint32_t tok = t * 32 + tk;
+      if (tok >= G.m_tokens) continue;
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        h16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = (_Float16)(silu_act_f(acc[t][4 * i + e] * inv[t]) * (acc[t][4 * i + 8 + e] * inv[t]));
+        *reinterpret_cast<h16x4*>(G.act + xh_offset(tok, unit * 16 + 8 * i + 4 * g)) = o;
+      }
+    } else {   // turned round in the same place, so that a token's 32 sums leave side by side
+#pragma unroll
+      for (int i = 0; i < 4; i++) *reinterpret_cast<f32x4*>(place + t * 32 * 36 + 8 * i) = f32x4{acc[t][4 * i], acc[t][4 * i + 1], acc[t][4 * i + 2], acc[t][4 * i + 3]} * (1.0f / kPfScale);
+      const uint32_t row = unit * 32 + (lane & 7) * 4;
+      float* const part = G.part + (size_t)ks * G.part_rows * G.ncols + sg.col0 + row;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const uint32_t tok = i * 8 + (lane >> 3);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(smem) + wave * (TT * 32 * 36) + (t * 32 + tok) * 36 + (lane & 7) * 4);
+        if (t * 32 + tok < G.m_tokens && row < sg.ntiles * 16) *reinterpret_cast<f32x4*>(part + (size_t)(t * 32 + tok) * G.ncols) = v;
+      }
+    }
+  }
+}
+
+template <int F, int TT>
+__global__ void __launch_bounds__(2 * kPfWaves * 64) pf_pair_kernel(const PfGemm G) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr uint32_t kBuf = (uint32_t)TT * 32 * 512, kDma = kBuf / kPfWaves, tb = pf_tile_bytes(F);
+  pf_half_device<F, TT, true>(G, G.seg[0], blockIdx.x, 0, smem);
+}
+
+// gate | up for up to 32 tokens and whole pairs of blocks a team: each team has half of k, a block between two barriers is twice as long and the weights' addresses and scales are made once for two phases' more products.
+// 28672 rows of 4096 in Q4_K: 20.5 us against 23.4 in halves of blocks, where a block is over before what was asked for has come.
+template <int F>
+__global__ void __launch_bounds__(2 * kPfWaves * 64) pf_pair_few_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr uint32_t kBuf = 32 * 512, kDma = kBuf / kPfWaves, tb = pf_tile_bytes(F);
   constexpr int AHEAD = 2;                                            // phases the activations are read ahead
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6 & 3)), team = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
-  const uint32_t n = lane & 15, s = lane >> 4 & 1, g = lane >> 5, tk = lane & 31, nblk = G.nblk / KH;   // this team's blocks
+  const uint32_t n = lane & 15, s = lane >> 4 & 1, g = lane >> 5, tk = lane & 31, nblk = G.nblk / 2;   // this team's blocks
   const uint32_t tile = blockIdx.x * kPfWaves + wave, tl = tile < G.seg[0].ntiles ? tile : G.seg[0].ntiles - 1;   // clamped: loads are unconditional
   const uint8_t* const wrow = (s ? G.seg[1].w : G.seg[0].w) + ((size_t)tl * G.nblk + team * nblk) * tb;
   uint8_t* const slab = smem + team * 2 * kBuf;
@@ -298,27 +477,22 @@ __global__ void __launch_bounds__(KH * kPfWaves * 64) pf_pair_kernel(const PfGem
 #pragma unroll
     for (int j = 0; j < 2; j++) pf_load<F>(to[j], wrow + (size_t)b * tb, 16 * (2 * g + j) + n, n);   // (the row's scales once: the compiler sees that they are the same)
   };
-  f32x16 acc[TT];
-#pragma unroll
-  for (int t = 0; t < TT; t++) acc[t] = (f32x16)(0.0f);
+  f32x16 acc = (f32x16)(0.0f);
   PfRaw w[2][2];   // [block parity][j]
   x_dma(0);
   load(0, w[0]);
-  float inv[TT];   // 1 / rms of this lane's tokens
-#pragma unroll
-  for (int t = 0; t < TT; t++) inv[t] = pf_inv_rms(G.ssq, G.n_ssq, t * 32 + tk, G.norm_cols, G.eps) * (1.0f / kPfScale);
+  const float inv = pf_inv_rms(G.ssq, G.n_ssq, tk, G.norm_cols, G.eps) * (1.0f / kPfScale);   // of this lane's token
   auto landed = [&] {
     __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): see pf_body
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
   landed();
-  h16x8 af[2], bf[4][TT];
+  h16x8 af[2], bf[4];
   h16x2 S, O;
   auto read_bf = [&](uint32_t b, int p) {   // p = 4 pp + 2 j + h
     const uint32_t q = (uint32_t)(8 * (p >> 2) + (p & 3)) + 4 * g;
-#pragma unroll
-    for (int t = 0; t < TT; t++) bf[p & 3][t] = *reinterpret_cast<const h16x8*>(slab + (b & 1) * kBuf + (t * 32 + tk) * 512 + ((q ^ n) << 4));
+    bf[p & 3] = *reinterpret_cast<const h16x8*>(slab + (b & 1) * kBuf + tk * 512 + ((q ^ n) << 4));
   };
   auto frag = [&](const PfRaw (&cw)[2], int p) {
     const int pp = p >> 2, j = p >> 1 & 1;
@@ -338,88 +512,95 @@ __global__ void __launch_bounds__(KH * kPfWaves * 64) pf_pair_kernel(const PfGem
       else read_bf(b + 1, p + AHEAD - 16);
       if (p < 15) frag(cw, p + 1);
       else frag(nw, 0);
-#pragma unroll
-      for (int t = 0; t < TT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[p & 1], bf[p & 3][t], acc[t], 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[p & 1], bf[p & 3], acc, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 #pragma unroll
   for (int p = 0; p < AHEAD; p++) read_bf(0, p);
   frag(w[0], 0);
-  for (uint32_t b = 0; b < nblk; b += 2) {   // (whole pairs of blocks: pf_pair_go)
+  for (uint32_t b = 0; b < nblk; b += 2) {
     block(b, w[0], w[1]);
     block(b + 1, w[1], w[0]);
   }
-  if constexpr (KH == 2) {
-    f32x4* const sums = reinterpret_cast<f32x4*>(smem) + wave * (TT * 4 * 64) + lane;
-    __syncthreads();   // (every read of the slabs has returned)
-    if (team == 1) {
+  f32x4* const sums = reinterpret_cast<f32x4*>(smem) + wave * (4 * 64) + lane;
+  __syncthreads();   // (every read of the slabs has returned)
+  if (team == 1) {
 #pragma unroll
-      for (int t = 0; t < TT; t++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) sums[(t * 4 + i) * 64] = f32x4{acc[t][4 * i], acc[t][4 * i + 1], acc[t][4 * i + 2], acc[t][4 * i + 3]};
-    }
-    __syncthreads();
-    if (team == 1) return;
-#pragma unroll
-    for (int t = 0; t < TT; t++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const f32x4 v = sums[(t * 4 + i) * 64];
-#pragma unroll
-        for (int e = 0; e < 4; e++) acc[t][4 * i + e] += v[e];
-      }
+    for (int i = 0; i < 4; i++) sums[i * 64] = f32x4{acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
   }
-  // a lane has, per token, rows 8i + 4g .. + 3: gate with i = 0, 1, up with i + 2
-  if (tile >= G.seg[0].ntiles) return;
+  __syncthreads();
+  if (team == 1 || tile >= G.seg[0].ntiles || tk >= G.m_tokens) return;
 #pragma unroll
-  for (int t = 0; t < TT; t++) {
-    const uint32_t tok = t * 32 + tk;
-    if (tok >= G.m_tokens) continue;
+  for (int i = 0; i < 4; i++) {
+    const f32x4 v = sums[i * 64];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      h16x4 o;
+    for (int e = 0; e < 4; e++) acc[4 * i + e] += v[e];
+  }
+  // a lane has rows 8i + 4g .. + 3: gate with i = 0, 1, up with i + 2
 #pragma unroll
-      for (int e = 0; e < 4; e++) o[e] = (_Float16)(silu_act_f(acc[t][4 * i + e] * inv[t]) * (acc[t][4 * i + 8 + e] * inv[t]));
-      *reinterpret_cast<h16x4*>(G.act + xh_offset(tok, tile * 16 + 8 * i + 4 * g)) = o;
-    }
+  for (int i = 0; i < 2; i++) {
+    h16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = (_Float16)(silu_act_f(acc[4 * i + e] * inv) * (acc[4 * i + 8 + e] * inv));
+    *reinterpret_cast<h16x4*>(G.act + xh_offset(tk, tile * 16 + 8 * i + 4 * g)) = o;
   }
 }
 
-template <auto* Kernel, int MT, int TEAMS = 1>
+template <uint32_t MASK, int TT>
+__global__ void __launch_bounds__(2 * kPfWaves * 64) pf_rows_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  int si = 0;
+  if (G.nseg > 1 && blockIdx.x >= G.seg[1].rg_begin) si = 1;
+  if (G.nseg > 2 && blockIdx.x >= G.seg[2].rg_begin) si = 2;
+  const PfSeg& sg = G.seg[si];
+  auto is = [&](int f) { return (MASK & (1u << f)) && (MASK == (1u << f) || sg.fmt == f); };
+  const uint32_t rg = blockIdx.x - sg.rg_begin;
+  if (is(PF_Q4K)) pf_half_device<PF_Q4K, TT, false>(G, sg, rg, blockIdx.y, smem);
+  else if (is(PF_Q6K)) pf_half_device<PF_Q6K, TT, false>(G, sg, rg, blockIdx.y, smem);
+  else if (is(PF_Q5K)) pf_half_device<PF_Q5K, TT, false>(G, sg, rg, blockIdx.y, smem);
+  else if (is(PF_Q80)) pf_half_device<PF_Q80, TT, false>(G, sg, rg, blockIdx.y, smem);
+  else if (is(PF_Q40)) pf_half_device<PF_Q40, TT, false>(G, sg, rg, blockIdx.y, smem);
+}
+
+template <auto* Kernel, size_t LDS, int WAVES>
 static hipError_t pf_gemm_run(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
   static bool attr_set[64] = {};
-  constexpr size_t lds = TEAMS * 2 * (MT ? (size_t)MT * 16 * 512 : kPfSlabBytes);
-  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(Kernel), (int)lds, attr_set); e != hipSuccess) return e;
-  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S), dim3(TEAMS * kPfWaves * 64), lds, st, G);
+  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(Kernel), (int)LDS, attr_set); e != hipSuccess) return e;
+  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S), dim3(WAVES * 64), LDS, st, G);
   return hipGetLastError();
 }
 template <uint32_t MASK>
 static hipError_t pf_gemm_go(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
-  if (G.m_count) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 0>, 0>(G, n_rg, st);
-  if (G.m_tiles <= 2) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 2>, 2>(G, n_rg, st);
-  if (G.m_tiles <= 4) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 4>, 4>(G, n_rg, st);
-  return pf_gemm_run<&pf_gemm_kernel<MASK>, kPfMT>(G, n_rg, st);
+  if (G.m_count) return pf_gemm_run<&pf_experts_kernel<MASK>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
+  switch ((G.m_tokens + 31) / 32) {
+    case 1: return pf_gemm_run<&pf_rows_kernel<MASK, 1>, pf_half_lds(1), 2 * kPfWaves>(G, n_rg, st);
+    case 2: return pf_gemm_run<&pf_rows_kernel<MASK, 2>, pf_half_lds(2), 2 * kPfWaves>(G, n_rg, st);
+    case 3: return pf_gemm_run<&pf_rows_kernel<MASK, 3>, pf_half_lds(3), 2 * kPfWaves>(G, n_rg, st);
+    default: return pf_gemm_run<&pf_rows_kernel<MASK, 4>, pf_half_lds(4), 2 * kPfWaves>(G, n_rg, st);
+  }
 }
 
 bool pf_supported_type(int dev_type) { return pf_fmt_of(dev_type) >= 0; }
 
+// 16-row tiles of a workgroup
+static uint32_t pf_wg_tiles(bool experts) { return experts ? kPfWaves * kPfRT : kPfWaves * 2; }
+
 // k-splits of a GEMM over matrices with n_rows[i] rows and k columns: as many as keep the launch within one workgroup per CU
-static void pf_plan(const uint32_t* n_rows, int nw, uint32_t k, uint32_t* rg_out, uint32_t* S_out) {
-  const uint32_t nblk = k / 256;
+static void pf_plan(const uint32_t* n_rows, int nw, uint32_t k, bool experts, uint32_t* S_out) {
+  const uint32_t nblk = k / 256, wt = pf_wg_tiles(experts);
   uint32_t rg = 0;
-  for (int i = 0; i < nw; i++) rg += (n_rows[i] / 16 + kPfWaves * kPfRT - 1) / (kPfWaves * kPfRT);
+  for (int i = 0; i < nw; i++) rg += (n_rows[i] / 16 + wt - 1) / wt;
   uint32_t S = rg >= (uint32_t)kNumCU ? 1 : kNumCU / rg;
   if (S > nblk) S = nblk;
   const uint32_t per = (nblk + S - 1) / S;
   *S_out = (nblk + per - 1) / per;
-  *rg_out = rg;
 }
 
 // bytes of partial sums such a GEMM writes
 size_t pf_part_bytes(const uint32_t* n_rows, int nw, uint32_t k, uint32_t part_rows) {
-  uint32_t rg, S, cols = 0;
-  pf_plan(n_rows, nw, k, &rg, &S);
+  uint32_t S, cols = 0;
+  pf_plan(n_rows, nw, k, part_rows != (uint32_t)kPfTokens, &S);
   for (int i = 0; i < nw; i++) cols += n_rows[i];
   return (size_t)S * part_rows * cols * 4;
 }
@@ -435,6 +616,7 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
   if (k % 256) return hipErrorInvalidValue;
   G.nseg = nw;
   G.nblk = k / 256;
+  const uint32_t wt = pf_wg_tiles(m_count != nullptr);
   uint32_t rg = 0, col = 0, mask = 0, n_rows[3] = {0, 0, 0};
   for (int i = 0; i < nw; i++) {
     const int f = pf_fmt_of(W[i]->type);
@@ -445,16 +627,15 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
     G.seg[i].rg_begin = rg;
     G.seg[i].fmt = f;
     mask |= 1u << f;
-    rg += (G.seg[i].ntiles + kPfWaves * kPfRT - 1) / (kPfWaves * kPfRT);
+    rg += (G.seg[i].ntiles + wt - 1) / wt;
     col += W[i]->n;
     n_rows[i] = W[i]->n;
   }
-  uint32_t rg2;
-  pf_plan(n_rows, nw, k, &rg2, &G.S);
+  pf_plan(n_rows, nw, k, m_count != nullptr, &G.S);
   G.ncols = col;
   G.xh = xh;
   G.part = part;
-  G.m_tiles = (m_tokens + 15) / 16;
+  G.m_tokens = m_tokens;
   G.m_count = m_count;
   G.part_rows = part_rows;
   G.row_base = row_base;
@@ -476,25 +657,30 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
 // chunks of per-token sums of squares a row of H elements is reduced to (pf_inv_rms adds them up)
 uint32_t pf_ssq_chunks(uint32_t H) { return (H + 2047) / 2048; }
 
-// gate | up as one product without partial sums.  Its workgroups are half as wide as those of a product in k-ranges and not split; with up to 64 tokens that is the faster one for any width (8B widths,
-// 4 layers, 10 / 33 / 50 tokens 526 / 549 / 602 us in ranges, 503 / 523 / 578 here; TinyLlama's, 8 layers, 24 / 50 tokens 706 / 777 and 671 / 744), with more only while the ranges are one or two
-// (8B, two, 128 tokens: 741 -> 722; TinyLlama, five: 100 tokens 920 -> 941, 200 tokens 1539 -> 1565).
-bool pf_pairs(const DevWeight* gate, const DevWeight* up, uint32_t m_tokens) {
-  if (!pf_supported_type(gate->type) || gate->type != up->type || gate->k != up->k || gate->n != up->n || gate->k % 512 || gate->n % 256) return false;
-  return m_tokens <= 64 || 3 * (2 * gate->n / 256) > (uint32_t)kNumCU;
+// gate | up as one product without partial sums while walking all of k costs its workgroups no more than the fold and its launch: a block is 0.8 us, the fold about 5.  In ranges and here, six layers, us:
+// 4096 x 4096 (ranges of 4 of 16 blocks), 50 / 90 / 128 tokens 372 / 446 / 539 and 403 / 479 / 548; 2048 x 5632 (4 of 8) 335 / 390 / 445 and 329 / 378 / 431; 1024 x 2816 (1 of 4) 268 / 308 / 344 and 257 / 294 / 328.
+bool pf_pairs(const DevWeight* gate, const DevWeight* up) {
+  if (!pf_supported_type(gate->type) || gate->type != up->type || gate->k != up->k || gate->n != up->n || gate->k % 256 || gate->n % 256) return false;
+  const uint32_t n_rows[2] = {gate->n, up->n}, nblk = gate->k / 256;
+  uint32_t S;
+  pf_plan(n_rows, 2, gate->k, false, &S);
+  return nblk - (nblk + S - 1) / S <= 6;
 }
 
 template <int F>
 static hipError_t pf_pair_go(const PfGemm& G, hipStream_t st) {
   const uint32_t wgs = (G.seg[0].ntiles + kPfWaves - 1) / kPfWaves;
-  const bool halves = G.nblk % 4 == 0;
-  if (G.m_tiles <= 2) return halves ? pf_gemm_run<&pf_pair_kernel<F, 1, 2>, 2, 2>(G, wgs, st) : pf_gemm_run<&pf_pair_kernel<F, 1, 1>, 2>(G, wgs, st);
-  if (G.m_tiles <= 4) return halves ? pf_gemm_run<&pf_pair_kernel<F, 2, 2>, 4, 2>(G, wgs, st) : pf_gemm_run<&pf_pair_kernel<F, 2, 1>, 4>(G, wgs, st);
-  return pf_gemm_run<&pf_pair_kernel<F, 4, 1>, kPfMT>(G, wgs, st);
+  switch ((G.m_tokens + 31) / 32) {
+    case 1: if (G.nblk % 4 == 0) return pf_gemm_run<&pf_pair_few_kernel<F>, 2 * pf_half_lds(1), 2 * kPfWaves>(G, wgs, st);
+            return pf_gemm_run<&pf_pair_kernel<F, 1>, pf_half_lds(1), 2 * kPfWaves>(G, wgs, st);
+    case 2: return pf_gemm_run<&pf_pair_kernel<F, 2>, pf_half_lds(2), 2 * kPfWaves>(G, wgs, st);
+    case 3: return pf_gemm_run<&pf_pair_kernel<F, 3>, pf_half_lds(3), 2 * kPfWaves>(G, wgs, st);
+    default: return pf_gemm_run<&pf_pair_kernel<F, 4>, pf_half_lds(4), 2 * kPfWaves>(G, wgs, st);
+  }
 }
 
 hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint8_t* xh, uint8_t* act, const float* ssq, uint32_t norm_cols, float eps, uint32_t m_tokens, hipStream_t st) {
-  if (m_tokens == 0 || !pf_pairs(gate, up, m_tokens) || m_tokens > (uint32_t)kPfTokens || !act || !ssq) return hipErrorInvalidValue;
+  if (m_tokens == 0 || !pf_pairs(gate, up) || m_tokens > (uint32_t)kPfTokens || !act || !ssq) return hipErrorInvalidValue;
   PfGemm G{};
   for (int i = 0; i < 2; i++) {
     const DevWeight* W = i ? up : gate;
@@ -511,7 +697,6 @@ hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint
   G.norm_cols = norm_cols;
   G.eps = eps;
   G.m_tokens = m_tokens;
-  G.m_tiles = (m_tokens + 15) / 16;
   switch (pf_fmt_of(gate->type)) {
     case PF_Q4K: return pf_pair_go<PF_Q4K>(G, st);
     case PF_Q6K: return pf_pair_go<PF_Q6K>(G, st);
