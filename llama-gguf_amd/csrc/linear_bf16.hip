@@ -736,13 +736,21 @@ static hipError_t lin_gemm_pick(const LinGemm& a, hipStream_t st) {
   // More tiles of 32 rows than CUs, and tiles of 64 to 128 that give every CU one at most: two teams, with all of the CU's LDS for steps under way (tiles of 128 only where few CUs go without).
   // Two small workgroups a CU against these, us, bf16: 5632 -> 2048 columns, 768 tokens 37.0 and 33.4, 1501: 54.8 and 44.8; 2048 -> 2048, 1501: 22.3 and 21.1; 4096 -> 4096, 300: 28.3 and 25.7,
   // 1000: 46.2 and 44.0; 14336 -> 4096, 300: 104.6 and 95.9, 768: 168 and 120, 1000: 191 and 139.  With 192 tiles of 128 23.0 and 23.7 (2048 -> 3072, 1000), with up to 256 of 32 26.7 and 26.1 (5632 -> 2048, 300).
+  // (Two teams on tiles of 160 and 192 where those of 128 are a few more than the CUs, 2048 -> 3072 and 3456 columns, 1501 tokens: 26 and 28 us against 33 by themselves, in a model, where the weights come from
+  // memory, 37 and 39 against 37 and 38.)
+  auto tiles = [&](uint32_t bm) { return tn * ((a.M + bm - 1) / bm); };
   if constexpr (EPI == LE_F32 && sizeof(T) == 2) {
-    auto tiles = [&](uint32_t bm) { return tn * ((a.M + bm - 1) / bm); };
     if (a.kp >= 1024 && tiles(32) > kNumCU) {
       if (tiles(64) <= kNumCU) return lin_gemm_go<T, 64, 128, 2, EPI, false, 2>(a, st);
       if (tiles(96) <= kNumCU) return lin_gemm_go<T, 96, 128, 2, EPI, false, 2>(a, st);
       if (tiles(128) <= kNumCU && tiles(128) >= 224) return lin_gemm_go<T, 128, 128, 2, EPI, false, 2>(a, st);
     }
+  }
+  // Two workgroups a CU take tiles of 128 or 160 in rounds: the larger ones where a round less is worth a quarter more work in each (2048 -> 5632 / 6272 columns, 1501 tokens, 528 / 588 tiles of 128 and 440 / 490 of
+  // 160, in a model: 59.2 / 66.2 and 45.7 / 47.3 us; by themselves 2048 -> 14336, 600 tokens: 52.8 and 42.5; three rounds of either, 1501: 106.3 and 105.8; two of either, 1000: 68.7 and 79.4)
+  if constexpr (sizeof(T) == 2) {
+    auto rounds = [&](uint32_t bm) { return (tiles(bm) + 2 * kNumCU - 1) / (2 * kNumCU); };
+    if (a.M > 128 && 5 * rounds(160) < 4 * rounds(128)) return lin_gemm_go<T, 160, 128, 2, EPI>(a, st);
   }
   if (a.M > 64 && tn * ((a.M + 127) / 128) >= 224) return lin_gemm_go<T, 128, 128, 2, EPI>(a, st);
   if (a.M > 32 && tn * ((a.M + 63) / 64) >= 160) return lin_gemm_go<T, 64, 128, 4, EPI>(a, st);

@@ -22,3 +22,16 @@ def test_one_tile_a_cu(pkg, gpu, width, vocab, tokens):
         eng.reset()
         lc.check(eng.eval(toks[:n], range(n)), want[:n], "bf16", f"{n} tokens")
     eng.close()
+
+
+def test_tiles_of_160(pkg, gpu):
+    """Where two workgroups a CU would take two rounds of tiles of 128 and take one of 160: the joint input product (32 896 columns, 257 panels) and the gated feed-forward's first (33 200 columns,
+    260 panels); whole and ragged ends, and one token beyond a tile."""
+    cfg = lc.config([lc.mem(heads=64, dim=128, vdim=128, ff=16600)], width=1024, vocab=300)
+    eng, W = lc.make(pkg, cfg, "bf16", max_seq=200)
+    toks = lc.tokens(161, cfg["vocab"])
+    want = lo.forward(cfg, W, toks)
+    for n in (129, 145, 160, 161):
+        eng.reset()
+        lc.check(eng.eval(toks[:n], range(n)), want[:n], "bf16", f"{n} tokens")
+    eng.close()
