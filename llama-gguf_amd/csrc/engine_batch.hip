@@ -6,7 +6,7 @@
 // SLOTS — a slot = one sequence's KV caches + position — and lgh_forward_multi feeds one token to each listed slot in ONE pass
 // over the weights: every quantized mat-vec launch reads its tiles once and multiplies them with all n_seq input vectors
 // (matvec_batch.hip), attention / its merge / embedding / arg-max run with the sequence as the grid's second dimension (over f32 or
-// TurboQuant slots); MoE layers route every sequence to its own experts: from 3 sequences on (moe_group_min) the step's (sequence,
+// TurboQuant slots); MoE layers route every sequence to its own experts: from 2 sequences on (moe_group_min) the step's (sequence,
 // slot) pairs are grouped by expert and each selected expert is read once — all experts of a layer in one gate | up and one down
 // launch, the expert as the grid's third dimension — below that the FFN runs sequence by sequence.  Every sequence's logits are
 // bit-identical to what lgh_forward of the same context computes for the same tokens (tests/test_gpu_batch.py, test_gpu_batch_same_context.py): same
@@ -87,11 +87,11 @@ struct MvIndirect { const int* cnt = nullptr; const int* idx = nullptr; uint32_t
 
 // MoE layers: from how many sequences on a step reads every selected expert ONCE (one router launch, a grouping launch, gate | up
 // and down over all experts with the expert as the grid's third dimension + their epilogue launches, one combine: 7 per layer
-// whatever the step's size) instead of running the FFN sequence by sequence (3 launches per sequence).  Measured on Mixtral-8x7B
-// Q5_K_M, tokens/s grouped vs sequence by sequence: 2 sequences 363 vs 392, 3: 447 vs 421, 4: 520 vs 436, 8: 764 vs 468,
-// 16: 1 030 vs 480 (profiles/r03e_batched_decode.md).
+// whatever the step's size) instead of running the FFN sequence by sequence (3 launches per sequence).  Measured on Mixtral-8x7B's
+// widths, a step of two layers, us, sequence by sequence vs grouped: 2 sequences Q4_K_M 326 / 302, Q5_K_M 351 / 324, Q6_K 364 / 339,
+// Q8_0 410 / 381, Q4_0 305 / 269; the whole model in Q5_K_M, tokens/s, 8: 468 / 764, 16: 480 / 1 030 (profiles/r03e_batched_decode.md).
 uint32_t moe_group_min() {
-  static const uint32_t v = [] { const char* e = std::getenv("LGH_MOE_GROUP_MIN"); return e ? (uint32_t)std::max(2, std::atoi(e)) : 3u; }();
+  static const uint32_t v = [] { const char* e = std::getenv("LGH_MOE_GROUP_MIN"); return e ? (uint32_t)std::max(2, std::atoi(e)) : 2u; }();
   return v;
 }
 

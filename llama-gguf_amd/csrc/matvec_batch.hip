@@ -18,9 +18,10 @@
 // Epilogues: store, +residual, SwiGLU pair, RoPE (every sequence at its own position) and the K / V rows into the sequence's
 // own cache slot; optional XQ image of the output for the next launch.  MoE layers: an expert launch works on an INDIRECT
 // entry list (MvBatch::ind_*: the (sequence, top-k slot) pairs that chose the expert, their number read from device memory), so
-// that an expert's matrices are read once per step; below 7 sequences engine_batch.hip runs the FFN sequence by sequence instead.
+// that an expert's matrices are read once per step: gate | up of few entries an expert by mvqb_few, the others by mvqb2.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "device_utils.h"
 #include "xq.h"
@@ -1020,6 +1021,190 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t w
 }
 
 // ------------------------------------------------------------------------------------------------
+// gate | up of a mixture's experts in a step of few sequences: an expert has one entry or two, so the launch is a stream of weights.  mvqb2 keeps one tile a wave under way behind a barrier per chunk (22 KB a CU);
+// here a workgroup is the single-sequence kernel's (mvq_body): four waves = k-slices x unit groups, every wave with its slices' records of up to two entries in LDS of its own and a few tiles under way, no barrier
+// before the sums meet, and SwiGLU in place; three workgroups a CU.  More entries than two: another turn over the same weights.  Slices, operations and sums are the single-sequence kernel's.
+// Bound by the weights' stream; one layer of 8 experts of 14336 x 4096, two a sequence, mvqb2 -> this: Q5_K 5 sequences 137 -> 104 us (3.6 -> 4.8 TB/s), Q6_K 4: 122 -> 96, 8: 176 -> 165, Q8_0 4: 128 -> 112, 8: 176 -> 194
+// (an expert's third entry reads the weights again).  Q4_0 stays with mvqb2 (60 us of 4 sequences against 69: nothing to convert, and a tile is too small a request).
+// down stays with mvqb2 too: its slices are a grid dimension, so that it has bytes enough under way (Q6_K 51 us as the same stream 50, Q8_0 57 and 58).
+// ------------------------------------------------------------------------------------------------
+constexpr int few_depth(int f) { return f == F_Q4K ? 4 : f == F_Q6K ? 2 : 3; }   // tiles a wave has under way: what the registers of three waves a SIMD hold
+constexpr uint32_t kFewWaves = 4;
+struct MvqbFew { uint32_t T, nbw, nblk, max_sq, red_at, ssq_at; };
+
+template <int F, int SQ>
+__device__ __forceinline__ void mvqb_few_turn(const MvqbFew& Gm, const MvLaunch& L, const MvBatch& B, uint8_t* smem8, uint32_t ez, const int* ind_idx, uint32_t s0, uint32_t n_seq) {
+  constexpr uint32_t tb = fmt_tile_bytes(F), MASK = 1u << F, W = kFewWaves;
+  constexpr int LPT = fmt_loads_per_tile(F), D = few_depth(F);
+  const MvSeg& S = L.seg[0];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, mq = lane >> 4;
+  // T is 1, 2, 4 or 8.  The waves share the slices, SL consecutive ones from ks0 on, and with fewer slices than waves the units
+  const uint32_t SL = Gm.T > W ? Gm.T / W : 1, tw = Gm.T > W ? W : Gm.T, ks0 = (wave & (tw - 1)) * SL;
+  const uint32_t units_w = kBWaves * tw / W, unit0 = Gm.T < W ? (wave >> __builtin_ctz(Gm.T)) * units_w : 0;   // units of this wave
+  const uint32_t blk0 = ks0 * Gm.nbw, blk1 = min(Gm.nblk, blk0 + SL * Gm.nbw);
+  const uint32_t nblk_w = blk0 < blk1 ? blk1 - blk0 : 0;
+  const uint32_t ntiles = (S.n_rows + 15) >> 4, rows = kFuseRed / 2;
+  const uint8_t* const plane0 = S.pass[0].plane[0] + (uint64_t)ez * S.pass[0].sel_stride[0];
+  const uint8_t* const plane1 = S.pass[1].plane[0] + (uint64_t)ez * S.pass[1].sel_stride[0];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem8;
+  const uint32_t wrecs = SL * Gm.nbw, wreg = wave * wrecs * SQ * (uint32_t)kXqRecord;
+  float* const red = reinterpret_cast<float*>(smem8 + Gm.red_at);
+  const uint32_t red_floats = kFuseRed * Gm.T;             // a sequence's, [pass][slice][row]
+  auto store = [&](uint32_t i, uint32_t ks, int s, float t) __attribute__((always_inline)) {
+    const uint32_t w = unit0 + i;
+    if (mq == 0 && (uint32_t)s < n_seq) red[(size_t)s * red_floats + ((w & 1) * Gm.T + ks) * rows + (w >> 1) * 16 + n] = t;
+  };
+  const uint32_t nitems = units_w * nblk_w;
+  // slices beyond the last block: their sums read as zero
+  for (uint32_t ks = ks0 + (nblk_w + Gm.nbw - 1) / Gm.nbw; ks < ks0 + SL; ks++)
+    for (uint32_t i = 0; i < units_w; i++)
+#pragma unroll
+      for (int s = 0; s < SQ; s++) store(i, ks, s, 0.0f);
+  if (nitems == 0) return;
+  // the records of the slices, first of all that is asked for
+#pragma unroll
+  for (int s = 0; s < SQ; s++) {
+    uint32_t v;
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(s0 + s, s0 + n_seq - 1));
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(ind_idx + at) : "memory");
+    const uint8_t* src = S.pass[0].xq + (size_t)(v / B.ind_div) * B.xq_stride + (size_t)blk0 * kXqRecord;
+    for (uint32_t b = 0; b < nblk_w; b++, src += kXqRecord)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                   : : "v"(src + lane * 16), "v"(src + 1024 + lane * 4), "s"(__builtin_amdgcn_readfirstlane((int)(lds0 + wreg + (s * wrecs + b) * (uint32_t)kXqRecord))) : "memory", "m0");
+  }
+  // items in order: unit, then block
+  uint32_t ni = 0, nb = 0;   // the next to request
+  const uint8_t* src = nullptr;
+  auto locate = [&]() __attribute__((always_inline)) {   // a unit is a tile of gate, or of up; beyond the last tile its rows again, never stored
+    const uint32_t w = unit0 + ni, tl = min(blockIdx.x * (kBWaves / 2) + (w >> 1), ntiles - 1);
+    src = (w & 1 ? plane1 : plane0) + ((size_t)tl * Gm.nblk + blk0) * tb;
+  };
+  locate();
+  auto issue = [&](RawT16& r) __attribute__((always_inline)) {
+    mvq_issue_tile<MASK>(F, src, lane, r);
+    src += tb;
+    if (++nb == nblk_w) {
+      nb = 0;
+      if (++ni < units_w) locate();
+    }
+  };
+  uint32_t ci = 0, cb = 0, cs = 0, ck = ks0;   // the item at hand: unit, block, block of the slice, slice
+  float acc[SQ];
+#pragma unroll
+  for (int s = 0; s < SQ; s++) acc[s] = 0.0f;
+  auto consume = [&](const RawT16& r) __attribute__((always_inline)) {
+    const uint8_t* rec = smem8 + wreg + cb * (uint32_t)kXqRecord;
+    if constexpr (SQ == 1) {
+      mvq_consume_tile<MASK>(F, r, rec, lane, acc[0]);
+    } else {
+      TileOps t;
+      mvq_unpack_tile<MASK>(F, r, lane, t);
+#pragma unroll
+      for (int s = 0; s < SQ; s++) {
+        XqOps o;
+        xq_load_ops(rec + s * wrecs * (uint32_t)kXqRecord, lane, o);
+        mvq_mac_tile<MASK>(F, t, o, acc[s]);
+      }
+    }
+    cb++;
+    if (++cs == Gm.nbw || cb == nblk_w) {   // the four lane groups: the slice's sum
+#pragma unroll
+      for (int s = 0; s < SQ; s++) {
+        float t = acc[s] + __shfl_xor(acc[s], 16, 64);
+        t += __shfl_xor(t, 32, 64);
+        store(ci, ck, s, t);
+        acc[s] = 0.0f;
+      }
+      cs = 0;
+      ck++;
+      if (cb == nblk_w) {
+        cb = 0;
+        ck = ks0;
+        ci++;
+      }
+    }
+  };
+  RawT16 buf[D];
+  auto run = [&](auto first) __attribute__((always_inline)) {
+    constexpr int NF = decltype(first)::value;
+#pragma unroll
+    for (int j = 0; j < NF; j++) issue(buf[j]);
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NF * LPT) : "memory");   // the records alone
+    if constexpr (NF < D) {
+#pragma unroll
+      for (int j = 0; j < NF; j++) consume(buf[j]);
+    } else {
+      uint32_t rem = nitems;   // not yet consumed, D of them under way
+      while (rem >= 2 * D) {
+#pragma unroll
+        for (int j = 0; j < D; j++) { consume(buf[j]); issue(buf[j]); }
+        rem -= D;
+      }
+      const uint32_t more = rem - D;
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        consume(buf[j]);
+        if ((uint32_t)j < more) issue(buf[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < D - 1; j++)
+        if ((uint32_t)j < more) consume(buf[j]);
+    }
+  };
+  if (nitems == 1) run(std::integral_constant<int, 1>{});
+  else if (nitems == 2) run(std::integral_constant<int, 2>{});
+  else if (nitems == 3 && D > 3) run(std::integral_constant<int, 3>{});
+  else run(std::integral_constant<int, D>{});
+}
+
+template <int F>
+__global__ void __launch_bounds__(kFewWaves * 64, 3) mvqb_few_kernel(const MvqbFew Gm, const MvLaunch L, const MvBatch B) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  const uint32_t ez = blockIdx.z;
+  uint32_t n_seq;
+  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(n_seq) : "s"(B.ind_cnt + ez) : "memory");
+  n_seq = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(n_seq, B.n_seq));
+  if (n_seq == 0) return;
+  const int* ind_idx = B.ind_idx + (size_t)ez * B.ind_stride;
+  float* const ssq = reinterpret_cast<float*>(smem8 + Gm.ssq_at);
+  if (L.do_norm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
+  for (uint32_t s0 = 0; s0 < n_seq; s0 += Gm.max_sq) {
+    const uint32_t left = n_seq - s0, now = left < Gm.max_sq ? left : Gm.max_sq;
+    if (now == 1) mvqb_few_turn<F, 1>(Gm, L, B, smem8, ez, ind_idx, s0, now);
+    else mvqb_few_turn<F, 2>(Gm, L, B, smem8, ez, ind_idx, s0, now);
+    // SwiGLU as mv_epilogue_view has it: a thread a row and entry
+    constexpr uint32_t rows = kFuseRed / 2;
+    const MvSeg& S = L.seg[0];
+    const float* red = reinterpret_cast<const float*>(smem8 + Gm.red_at);
+    const uint32_t s = threadIdx.x / rows, rl = threadIdx.x % rows, row = blockIdx.x * rows + rl;
+    __syncthreads();
+    if (s < now && row < S.n_rows) {
+      float inv = 1.0f;
+      if (L.do_norm) {
+        float tot = 0.0f;
+        for (uint32_t w = 0; w < (uint32_t)kBWaves; w++) tot += ssq[(s0 + s) * 8 + w];
+        inv = 1.0f / __builtin_sqrtf(tot / (float)L.k + L.eps);
+      }
+      float v[2];
+#pragma unroll
+      for (uint32_t p = 0; p < 2; p++) {
+        float t = 0.0f;
+        for (uint32_t ks = 0; ks < Gm.T; ks++) t += red[(size_t)s * kFuseRed * Gm.T + (p * Gm.T + ks) * rows + rl];
+        v[p] = t * inv;
+      }
+      const float a = silu_f(v[0]) * v[1];
+      const uint32_t so = (uint32_t)ind_idx[s0 + s];
+      S.out[(size_t)so * B.out_stride[0] + row] = a;
+      if (S.xq_out) {
+        const float w = S.xq_nw ? S.xq_nw[row] : 1.0f;
+        xq_store_chunk(S.xq_out + (size_t)so * B.xq_out_stride[0], row >> 4, a * w, S.xq_ssq ? S.xq_ssq + (size_t)so * B.ssq_out_stride[0] : nullptr, a, rl);
+      }
+    }
+    __syncthreads();   // (the next turn's sums go where these were)
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
 // host
 // ------------------------------------------------------------------------------------------------
 size_t mvqb_lds_bytes(uint32_t n_seq, uint32_t red_floats) { return ((size_t)n_seq * red_floats + (size_t)n_seq * 8) * 4 + 64; }
@@ -1034,7 +1219,7 @@ static hipError_t mvqb_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, 
 
 // Sequences from which the groups of four are the faster ones (a step, 4 layers of an 8B model in Q4_K_M / Q8_0, us: 2 sequences 366 / 411 with mvqb2,
 // 388 / 398 in groups; 3: 416 / 439 against 390 / 419; 5: 495 / 494 against 504 / 488; 8: 579 / 567 against 529 / 520; 16: 905 / 867 against 786 / 751).
-// Indirect launches (a mixture's experts) have one or two sequences per expert: they stay with mvqb2.
+// Indirect launches (a mixture's experts) have one or two sequences per expert: they go to mvqb_few or mvqb2.
 constexpr uint32_t kMvqb4MinSeq = 3;
 
 // Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers of an 8B model in Q4_K_M / Q4_0, us, groups of four against
@@ -1081,6 +1266,28 @@ static bool mvqb2_epilogue_few(const MvLaunch& L, const MvBatch& B, const Mvqb2G
   return true;
 }
 
+// gate | up of a layer's experts with few entries each: two on average at most; of Q8_0, where the second read costs most, 1.25 (steps of two layers, us, mvqb2 / mvqb_few, 8 experts, two a sequence: Q4_K_M 4 sequences
+// 482 / 410, 8: 676 / 622; Q5_K_M 5: 609 / 535, 8: 715 / 688, 10: 825 / 808, 12: 851 / 894; Q6_K 7: 681 / 663, 10: 800 / 867; Q8_0 5: 644 / 617, 6: 671 / 689).  mvqb2 where the format is Q4_0.
+static bool mvqb_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, int f, bool seq, MvqbFew* few, size_t* lds) {
+  if (f == F_Q40 || !seq || Gm.fuse != 2 || !B.ind_cnt || B.ind_nz < 2 || L.nseg != 1 || L.seg[0].epi != EPI_SWIGLU || L.seg[0].bias || Gm.T > kBWaves || kBWaves % Gm.T) return false;
+  if (4 * B.n_seq * B.ind_div > (f == F_Q80 ? 5 : 8) * B.ind_nz) return false;
+  for (uint32_t sq = 2; sq >= 1; sq--) {
+    *few = MvqbFew{Gm.T, Gm.nbw, Gm.nblk, sq, std::max(Gm.T, kFewWaves) * Gm.nbw * sq * (uint32_t)kXqRecord, 0};
+    few->ssq_at = few->red_at + sq * kFuseRed * Gm.T * 4;
+    *lds = few->ssq_at + mvqb_fuse_lds(B.n_seq);
+    if (*lds <= 160 * 1024) return true;
+  }
+  return false;
+}
+
+template <int F>
+static hipError_t mvqb_few_go(const MvLaunch& L, const MvBatch& B, const MvqbFew& few, size_t lds, uint32_t groups, hipStream_t st) {
+  static bool attr_set[64] = {};
+  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb_few_kernel<F>), 160 * 1024, attr_set); e != hipSuccess) return e;
+  hipLaunchKernelGGL(mvqb_few_kernel<F>, dim3(groups, 1, B.ind_nz), dim3(kFewWaves * 64), lds, st, few, L, B);
+  return hipGetLastError();
+}
+
 template <uint32_t MASK, int NB>
 static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, Mvqb2Geom Gm, bool seq, uint32_t groups, size_t lds_x,
                            size_t lds_e, uint32_t threads, hipStream_t st) {
@@ -1088,6 +1295,11 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
   Gm.ssq_at = (uint32_t)lds_x;
   lds_x += mvqb_fuse_lds(B.n_seq);
+  if constexpr ((MASK & (MASK - 1)) == 0 && MASK != 1u << F_Q40) {
+    MvqbFew few;
+    size_t lds_few;
+    if (mvqb_few(L, B, Gm, __builtin_ctz(MASK), seq, &few, &lds_few)) return mvqb_few_go<__builtin_ctz(MASK)>(L, B, few, lds_few, groups, st);
+  }
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
     if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);

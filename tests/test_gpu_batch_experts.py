@@ -1,0 +1,38 @@
+"""gate | up of a mixture's experts in a batched step of few sequences (matvec_batch.hip: mvqb_few_kernel): every format it takes, plans of one to eight k-slices (one with blocks for seven of the eight), a last
+workgroup with half its tiles, experts of one entry, two, and more (another turn), and the sequences from which mvqb2 takes over.
+
+Per (row, entry) the kernel does the single-sequence kernel's operations in its order, so the bound is equality of all bits with a single-sequence engine that runs the split attention too (attn_direct=255)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mix,hidden,kw", [
+    ("Q4_K_M", 512, {}), ("Q5_K_M", 1024, {}), ("Q6_K", 2048, {}), ("Q8_0", 512, {}), ("Q8_0", 2048, {}), ("Q4_0", 1024, {}),
+    ("Q5_K_M", 3328, dict(expert_intermediate_size=10496)), ("Q4_K_M", 4096, {}),
+    ("Q6_K", 1024, dict(num_experts=8, num_experts_per_token=1)), ("Q4_K_M", 2048, dict(num_experts=12, num_experts_per_token=4)),
+])
+def test_experts_of_few_entries_are_bitwise_the_single_sequence(pkg, mix, hidden, kw):
+    over = dict(hidden_size=hidden, num_heads=hidden // 64, num_kv_heads=hidden // 128, num_layers=1, num_experts=8, expert_intermediate_size=10240)
+    over.update(kw)
+    cfg = pkg.make_config("test-moe", max_seq_len=32, **over)
+    model = pkg.SynthModel(cfg, mix=mix)
+    multi = pkg.HipGpuInference.from_model(model, 32)
+    single = pkg.HipGpuInference.from_model(model, 32, attn_direct=255)
+    multi.batch_create(12)
+    tok = np.random.default_rng(7).integers(0, cfg.vocab_size, (12, 2))
+    tok[5:9] = tok[5]                                  # four sequences alike: their experts have four entries
+    want = []
+    for s in range(12):
+        single.reset()
+        want.append([single.forward(int(t)).copy() for t in tok[s]])
+    for n in (2, 3, 5, 8, 12):
+        for s in range(12):
+            multi.batch_reset(s)
+        for step in range(2):
+            got, _ = multi.forward_multi(list(range(n)), tok[:n, step])
+            for s in range(n):
+                assert np.array_equal(got[s].view(np.uint32), want[s][step].view(np.uint32)), (n, s, step)
+    multi.close()
+    single.close()
