@@ -484,7 +484,7 @@ hipError_t kv_roundtrip_launch(int fmt, const float* x, uint32_t n, uint8_t* byt
 template <bool MULTI>
 __global__ void __launch_bounds__(128) attn_combine_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_acc,
                                                            uint32_t g_per_kv, uint32_t head_dim, uint32_t n_splits,
-                                                           float* __restrict__ out, uint8_t* __restrict__ xq_out, const int* pos_ptr, uint32_t split_rows) {
+                                                           float* __restrict__ out, uint8_t* __restrict__ xq_out, const int* pos_ptr, uint32_t split_rows, uint8_t* __restrict__ xw, uint32_t xw_block) {
   __shared__ float s_f[64];
   __shared__ float s_linv;
   LGH_TL_BEGIN(attn, lgh::TL_COMBINE, n_splits);
@@ -495,6 +495,7 @@ __global__ void __launch_bounds__(128) attn_combine_kernel(const float* __restri
     part_acc += (size_t)sq * n_heads * n_splits * head_dim;
     out += (size_t)sq * n_heads * head_dim;
     if (xq_out) xq_out += (size_t)sq * xq_bytes((size_t)n_heads * head_dim);
+    if (xw) xw += (size_t)sq * kXwRecord;
     uint32_t pw;
     asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pw) : "s"(pos_ptr + sq) : "memory");
     used = min(n_splits, pw / split_rows + 1);
@@ -526,7 +527,7 @@ __global__ void __launch_bounds__(128) attn_combine_kernel(const float* __restri
     for (uint32_t sidx = 0; sidx < 32; sidx++) a += pa[sidx] * s_f[sidx];   // s_f of absent and empty splits is exp(-1e30 - m) = 0
     const float o = a * s_linv;
     out[(size_t)h * head_dim + dim] = o;
-    if (xq_out) xq_store_chunk(xq_out, (h * head_dim + dim) >> 4, o);   // wo's input as XQ records (head_dim % 16 == 0)
+    if (xq_out) xq_store_chunk(xq_out, (h * head_dim + dim) >> 4, o, nullptr, 0.0f, dim, MULTI ? xw : nullptr, xw_block);   // wo's input as XQ records (head_dim % 16 == 0)
   }
   LGH_TL_END();
 }
@@ -956,7 +957,7 @@ hipError_t attn_combine_launch(const float* part_ml, const float* part_acc, uint
                                uint32_t head_dim, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st) {
   if (n_kv == 0 || n_heads % n_kv || head_dim % 16 || head_dim > 128 || n_splits > 32) return hipErrorInvalidValue;
   hipLaunchKernelGGL(attn_combine_kernel<false>, dim3(n_heads), dim3(head_dim > 64 ? 128 : 64), 0, st, part_ml, part_acc,
-                     n_heads / n_kv, head_dim, n_splits, out, xq_out, (const int*)nullptr, 0u);
+                     n_heads / n_kv, head_dim, n_splits, out, xq_out, (const int*)nullptr, 0u, (uint8_t*)nullptr, 0u);
   return hipGetLastError();
 }
 
@@ -996,10 +997,10 @@ hipError_t attn_multi_launch(const float* q, const float* kcache, const float* v
 }
 
 hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq,
-                                     const int* pos, uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st) {
+                                     const int* pos, uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st, uint8_t* xw, uint32_t xw_block) {
   if (n_kv == 0 || n_heads % n_kv || head_dim % 16 || head_dim > 128 || n_splits > 32 || n_seq == 0 || !pos) return hipErrorInvalidValue;
   hipLaunchKernelGGL(attn_combine_kernel<true>, dim3(n_heads, n_seq), dim3(head_dim > 64 ? 128 : 64), 0, st, part_ml, part_acc,
-                     n_heads / n_kv, head_dim, n_splits, out, xq_out, pos, attn_multi_waves(max_seq) * (256 / head_dim));   // (rows a split takes first)
+                     n_heads / n_kv, head_dim, n_splits, out, xq_out, pos, attn_multi_waves(max_seq) * (256 / head_dim), xw, xw_block);   // (rows a split takes first)
   return hipGetLastError();
 }
 
@@ -1012,7 +1013,7 @@ hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc
 template <int D, int NW>
 __global__ void __launch_bounds__(1024, 8) attn_multi_direct_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, uint32_t n_kv, uint32_t g_per_kv,
                                                                  uint32_t max_seq, float scale, const int* pos_ptr, const int* slot, uint64_t slot_stride, uint32_t n_splits,
-                                                                 float* __restrict__ out, uint8_t* __restrict__ xq_out) {
+                                                                 float* __restrict__ out, uint8_t* __restrict__ xq_out, uint8_t* __restrict__ xw, uint32_t xw_block) {
   constexpr int LPR = D / 4, RPW = 64 / LPR, QS = 16 / NW, B = NW == 4 ? 3 : 2;   // lanes of a row, rows of a load, splits of a round, steps requested ahead
   __shared__ float s_ml[2][16][2];
   __shared__ __attribute__((aligned(16))) float s_acc[2][16][D];
@@ -1130,17 +1131,17 @@ __global__ void __launch_bounds__(1024, 8) attn_multi_direct_kernel(const float*
     for (uint32_t sp = 0; sp < used; sp++) a += p_acc[sp][tid] * s_f[sp];
     const float o = a * s_linv;
     out[((size_t)sq * n_heads + head) * D + tid] = o;
-    if (xq_out) xq_store_chunk(xq_out + (size_t)sq * xq_bytes((size_t)n_heads * D), (head * D + tid) >> 4, o);
+    if (xq_out) xq_store_chunk(xq_out + (size_t)sq * xq_bytes((size_t)n_heads * D), (head * D + tid) >> 4, o, nullptr, 0.0f, tid, xw ? xw + (size_t)sq * kXwRecord : nullptr, xw_block);
   }
 }
 
 hipError_t attn_multi_direct_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos,
-                                    const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st) {
+                                    const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st, uint8_t* xw, uint32_t xw_block) {
   if (n_kv == 0 || n_heads % n_kv || !pos || !slot || n_seq == 0 || n_splits == 0 || n_splits > 32 || !attn_shape_has_fast_kernel(head_dim, n_heads / n_kv)) return hipErrorInvalidValue;
 #define LGH_AMD(DD, WW)                                                                                                                                                          \
   if (head_dim == DD && attn_multi_waves(max_seq) == WW) {                                                                                                                       \
     hipLaunchKernelGGL((attn_multi_direct_kernel<DD, WW>), dim3(n_heads, n_seq), dim3(1024), 0, st, q, kcache, vcache, n_kv, n_heads / n_kv, max_seq, scale, pos, slot, slot_stride, \
-                       n_splits, out, xq_out);                                                                                                                                   \
+                       n_splits, out, xq_out, xw, xw_block);                                                                                                                                        \
     return hipGetLastError();                                                                                                                                                    \
   }
   LGH_AMD(128, 4) LGH_AMD(128, 8) LGH_AMD(64, 4) LGH_AMD(64, 8)

@@ -426,13 +426,14 @@ template <int D, bool MULTI>
 __global__ void __launch_bounds__(D) attn_tq_combine_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_acc,
                                                             const float* __restrict__ signs, const TqTables T, uint32_t g_per_kv,
                                                             uint32_t n_splits, float* __restrict__ out, uint8_t* __restrict__ xq_out,
-                                                            uint32_t xq_stride) {
+                                                            uint32_t xq_stride, uint8_t* __restrict__ xw, uint32_t xw_block) {
   if (MULTI) {
     const size_t per_seq = (size_t)gridDim.x * n_splits;   // (head, split) partials of one sequence
     part_ml += (size_t)blockIdx.y * per_seq * 2;
     part_acc += (size_t)blockIdx.y * per_seq * D;
     out += (size_t)blockIdx.y * gridDim.x * D;
     if (xq_out) xq_out += (size_t)blockIdx.y * xq_stride;
+    if (xw) xw += (size_t)blockIdx.y * kXwRecord;
   }
   __shared__ float s_f[64];
   __shared__ float s_linv;
@@ -462,7 +463,7 @@ __global__ void __launch_bounds__(D) attn_tq_combine_kernel(const float* __restr
   tq_fwht_rows<D>(buf, 1);
   const float o = buf[dim] * T.inv_d * signs[(size_t)(kvh * 2 + 1) * D + dim];
   out[(size_t)h * D + dim] = o;
-  if (xq_out) xq_store_chunk(xq_out, (h * D + dim) >> 4, o);
+  if (xq_out) xq_store_chunk(xq_out, (h * D + dim) >> 4, o, nullptr, 0.0f, dim, MULTI ? xw : nullptr, xw_block);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -476,7 +477,8 @@ template <int D, int BITS, bool MULTI>
 __global__ void __launch_bounds__(1024) attn_tq_direct_kernel(const float* __restrict__ q, uint8_t* __restrict__ kq, uint8_t* __restrict__ vq,
                                                               const float* __restrict__ k_new, const float* __restrict__ v_new,
                                                               const float* __restrict__ signs, const TqTables T, uint32_t g_per_kv, uint32_t max_seq, float scale,
-                                                              const int* pos_ptr, float* __restrict__ out, uint8_t* __restrict__ xq_out, const TqMulti ms, uint32_t xq_stride) {
+                                                              const int* pos_ptr, float* __restrict__ out, uint8_t* __restrict__ xq_out, const TqMulti ms, uint32_t xq_stride, uint8_t* __restrict__ xw,
+                                                              uint32_t xw_block) {
   constexpr uint32_t RB = tq_row_bytes<BITS>(D);
   constexpr int LPR = D / 16, RPW = 64 / LPR, NW = 16;               // lanes per row, rows per wave and round, waves
   __shared__ float rot[3][D];
@@ -498,6 +500,7 @@ __global__ void __launch_bounds__(1024) attn_tq_direct_kernel(const float* __res
     vq += (size_t)sl * ms.code_stride;
     out += (size_t)sq * gridDim.x * D;
     if (xq_out) xq_out += (size_t)sq * xq_stride;
+    if (xw) xw += (size_t)sq * kXwRecord;
   }
   const float* sk = signs + (size_t)(kvh * 2) * D;
   const float* sv = sk + D;
@@ -617,7 +620,7 @@ __global__ void __launch_bounds__(1024) attn_tq_direct_kernel(const float* __res
     const uint32_t dim = lane + e * 64;
     const float o = (e ? a1 : a0) * T.inv_d * sv[dim];
     out[(size_t)h * D + dim] = o;
-    if (xq_out) xq_store_chunk(xq_out, (h * D + dim) >> 4, o);
+    if (xq_out) xq_store_chunk(xq_out, (h * D + dim) >> 4, o, nullptr, 0.0f, dim, MULTI ? xw : nullptr, xw_block);
   }
 }
 
@@ -717,12 +720,12 @@ hipError_t attn_tq_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, co
 // sequences as in attn_tq_multi_launch
 hipError_t attn_tq_direct_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, const float* k_new, const float* v_new, const float* signs,
                                  uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos, float* out, uint8_t* xq_out,
-                                 hipStream_t st, uint32_t n_seq, const int* slot, uint64_t code_stride, uint32_t kv_stride, uint32_t xq_stride) {
+                                 hipStream_t st, uint32_t n_seq, const int* slot, uint64_t code_stride, uint32_t kv_stride, uint32_t xq_stride, uint8_t* xw, uint32_t xw_block) {
   if (n_kv == 0 || n_heads % n_kv || !pos || max_seq == 0 || (n_seq && !slot)) return hipErrorInvalidValue;
   const TqMulti ms{slot, code_stride, 0, kv_stride};
 #define LGH_TQ_GO(DD, BB, MU)                                                                                                                               \
   hipLaunchKernelGGL((attn_tq_direct_kernel<DD, BB, MU>), dim3(n_heads, MU ? n_seq : 1), dim3(1024), 0, st, q, kq, vq, k_new, v_new, signs, tq_tables(DD, BB), \
-                     n_heads / n_kv, max_seq, scale, pos, out, xq_out, ms, xq_stride)
+                     n_heads / n_kv, max_seq, scale, pos, out, xq_out, ms, xq_stride, xw, xw_block)
 #define LGH_TQ_CASE(DD, BB)                   \
   if (head_dim == DD && bits == BB) {         \
     if (n_seq) LGH_TQ_GO(DD, BB, true);       \
@@ -752,16 +755,16 @@ hipError_t attn_tq_multi_launch(int bits, const float* q, uint8_t* kq, uint8_t* 
 // n_seq 0: single sequence; otherwise grid y = sequences, XQ images xq_stride bytes apart
 hipError_t attn_tq_combine_launch(int bits, const float* part_ml, const float* part_acc, const float* signs, uint32_t n_heads, uint32_t n_kv,
                                   uint32_t head_dim, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st, uint32_t n_seq,
-                                  uint32_t xq_stride) {
+                                  uint32_t xq_stride, uint8_t* xw, uint32_t xw_block) {
   if (n_kv == 0 || n_heads % n_kv || n_splits > 32 || (head_dim != 64 && head_dim != 128)) return hipErrorInvalidValue;
   const TqTables T = tq_tables(head_dim, bits);
   const uint32_t gk = n_heads / n_kv;
   if (n_seq) {
-    if (head_dim == 128) hipLaunchKernelGGL((attn_tq_combine_kernel<128, true>), dim3(n_heads, n_seq), dim3(128), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, xq_stride);
-    else hipLaunchKernelGGL((attn_tq_combine_kernel<64, true>), dim3(n_heads, n_seq), dim3(64), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, xq_stride);
+    if (head_dim == 128) hipLaunchKernelGGL((attn_tq_combine_kernel<128, true>), dim3(n_heads, n_seq), dim3(128), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, xq_stride, xw, xw_block);
+    else hipLaunchKernelGGL((attn_tq_combine_kernel<64, true>), dim3(n_heads, n_seq), dim3(64), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, xq_stride, xw, xw_block);
   } else {
-    if (head_dim == 128) hipLaunchKernelGGL((attn_tq_combine_kernel<128, false>), dim3(n_heads), dim3(128), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, 0u);
-    else hipLaunchKernelGGL((attn_tq_combine_kernel<64, false>), dim3(n_heads), dim3(64), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, 0u);
+    if (head_dim == 128) hipLaunchKernelGGL((attn_tq_combine_kernel<128, false>), dim3(n_heads), dim3(128), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, 0u, nullptr, 0u);
+    else hipLaunchKernelGGL((attn_tq_combine_kernel<64, false>), dim3(n_heads), dim3(64), 0, st, part_ml, part_acc, signs, T, gk, n_splits, out, xq_out, 0u, nullptr, 0u);
   }
   return hipGetLastError();
 }

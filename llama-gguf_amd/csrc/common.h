@@ -172,7 +172,14 @@ struct MvBatch {
   uint32_t ind_stride;
   uint32_t ind_nz;            // experts in the launch (grid z); 0 / 1: a single entry list
   uint64_t part_z_floats;     // (set by the launcher)
+  // wide images (xq.h): the input's (NULL: none; mvqb8 needs it), each segment's output's (NULL: not wanted), the bytes between two blocks of either
+  const uint8_t* xw;
+  uint8_t* xw_out[3];
+  uint32_t xw_block;
 };
+// Whether a batched launch over matrices of this tile layout alone takes its input as a wide image
+bool mvqb_wide_input(int dev_type, uint32_t n_seq);
+hipError_t xw_from_xq_launch(const uint8_t* xq, uint32_t xq_stride, uint8_t* xw, uint32_t xw_block, uint32_t k, uint32_t n_seq, hipStream_t st);
 
 // launch-uniform geometry of one int8-MFMA launch as the kernel takes it (mvq_pack)
 struct MvGeom { uint32_t wbpack, geom, geom2, red_floats, lds_red_off, n_wg; };
@@ -221,15 +228,15 @@ hipError_t rope_launch(float* q, float* k, uint32_t n_heads, uint32_t n_kv, uint
                        const float* rope_cs, int neox, hipStream_t st);
 // multi-sequence decode (engine_batch.hip): one launch each for the n_seq sequences of a step
 hipError_t embed_multi_launch(int src_type, const uint8_t* table, const int* tokens, float* dst, uint32_t hidden, uint32_t n_seq, uint8_t* xq,
-                              const float* xq_nw, float* xq_ssq, uint32_t xq_stride, uint32_t ssq_stride, hipStream_t st);
+                              const float* xq_nw, float* xq_ssq, uint32_t xq_stride, uint32_t ssq_stride, hipStream_t st, uint8_t* xw = nullptr, uint32_t xw_block = 0);
 hipError_t argmax_multi_launch(const float* logits, uint32_t n, uint32_t n_seq, float* part_val, int* part_idx, int* next, hipStream_t st);
 hipError_t attn_multi_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                              uint32_t max_seq, float scale, const int* pos, const int* slot, uint64_t slot_stride, uint32_t n_seq,
                              uint32_t n_splits, float* part_ml, float* part_acc, hipStream_t st);
 hipError_t attn_multi_direct_launch(const float* q, const float* kcache, const float* vcache, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos,
-                                    const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st);
+                                    const int* slot, uint64_t slot_stride, uint32_t n_seq, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st, uint8_t* xw = nullptr, uint32_t xw_block = 0);
 hipError_t attn_combine_multi_launch(const float* part_ml, const float* part_acc, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq,
-                                     const int* pos, uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st);
+                                     const int* pos, uint32_t n_splits, uint32_t n_seq, float* out, uint8_t* xq_out, hipStream_t st, uint8_t* xw = nullptr, uint32_t xw_block = 0);
 // the rest of the per-op Backend surface (misc.hip): op = 0 add, 1 mul, 2 scale, 3 silu, 4 gelu
 hipError_t ewise_launch(int op, const float* a, const float* b, float s, float* out, uint64_t n, hipStream_t st);
 hipError_t softmax_rows_launch(const float* x, float* out, uint32_t rows, uint32_t last_dim, hipStream_t st);
@@ -241,7 +248,7 @@ hipError_t advance_launch(int* state, hipStream_t st);
 hipError_t copy_words_launch(void* dst, const void* src, uint32_t n_words, hipStream_t st);
 hipError_t moe_group_launch(const int* sel, uint32_t n_seq, uint32_t top_k, uint32_t n_experts, int* cnt, int* idx, uint32_t idx_stride, hipStream_t st);
 hipError_t moe_combine_launch(const float* tmp, const float* moe_w, uint32_t top_k, float* hidden, uint32_t H, uint32_t n_seq, const float* nw,
-                              uint8_t* xq, uint32_t xq_stride, float* ssq, uint32_t ssq_stride, hipStream_t st);
+                              uint8_t* xq, uint32_t xq_stride, float* ssq, uint32_t ssq_stride, hipStream_t st, uint8_t* xw = nullptr, uint32_t xw_block = 0);
 hipError_t moe_router_launch(const float* x, const float* norm_w, float eps, const float* w, uint32_t hidden,
                              uint32_t n_experts, uint32_t top_k, int* sel, float* sel_w, hipStream_t st, uint32_t n_tokens = 1);
 
@@ -265,10 +272,10 @@ hipError_t attn_tq_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, co
 hipError_t attn_tq_direct_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, const float* k_new, const float* v_new, const float* signs,
                                  uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos, float* out, uint8_t* xq_out,
                                  hipStream_t st, uint32_t n_seq = 0, const int* slot = nullptr, uint64_t code_stride = 0, uint32_t kv_stride = 0,
-                                 uint32_t xq_stride = 0);
+                                 uint32_t xq_stride = 0, uint8_t* xw = nullptr, uint32_t xw_block = 0);
 hipError_t attn_tq_combine_launch(int bits, const float* part_ml, const float* part_acc, const float* signs, uint32_t n_heads, uint32_t n_kv,
                                   uint32_t head_dim, uint32_t n_splits, float* out, uint8_t* xq_out, hipStream_t st, uint32_t n_seq = 0,
-                                  uint32_t xq_stride = 0);
+                                  uint32_t xq_stride = 0, uint8_t* xw = nullptr, uint32_t xw_block = 0);
 hipError_t attn_tq_multi_launch(int bits, const float* q, uint8_t* kq, uint8_t* vq, const float* k_new, const float* v_new, const float* signs,
                                 uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t max_seq, float scale, const int* pos, const int* slot,
                                 uint64_t code_stride, uint64_t x_stride, uint32_t kv_stride, uint32_t n_seq, uint32_t n_splits, float* part_ml,

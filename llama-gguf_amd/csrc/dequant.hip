@@ -187,22 +187,22 @@ hipError_t embed_launch(int src_type, const uint8_t* table, const int* token, fl
 __global__ void __launch_bounds__(256) embed_multi_kernel(int type, const uint8_t* __restrict__ table, const int* __restrict__ tokens,
                                                           float* __restrict__ dst, uint32_t hidden, uint8_t* __restrict__ xq,
                                                           const float* __restrict__ xq_nw, float* __restrict__ xq_ssq, uint32_t xq_stride,
-                                                          uint32_t ssq_stride) {
+                                                          uint32_t ssq_stride, uint8_t* __restrict__ xw, uint32_t xw_block) {
   const uint32_t sq = blockIdx.y;
   const uint64_t row = (uint64_t)(uint32_t)tokens[sq];
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i < hidden) {
     const float v = deq_any(type, table, row * hidden + i);
     dst[(size_t)sq * hidden + i] = v;
-    if (xq) xq_store_chunk(xq + (size_t)sq * xq_stride, i >> 4, xq_nw ? v * xq_nw[i] : v, xq_ssq ? xq_ssq + (size_t)sq * ssq_stride : nullptr, v);
+    if (xq) xq_store_chunk(xq + (size_t)sq * xq_stride, i >> 4, xq_nw ? v * xq_nw[i] : v, xq_ssq ? xq_ssq + (size_t)sq * ssq_stride : nullptr, v, i, xw ? xw + (size_t)sq * kXwRecord : nullptr, xw_block);
   }
 }
 
 hipError_t embed_multi_launch(int src_type, const uint8_t* table, const int* tokens, float* dst, uint32_t hidden, uint32_t n_seq, uint8_t* xq,
-                              const float* xq_nw, float* xq_ssq, uint32_t xq_stride, uint32_t ssq_stride, hipStream_t st) {
+                              const float* xq_nw, float* xq_ssq, uint32_t xq_stride, uint32_t ssq_stride, hipStream_t st, uint8_t* xw, uint32_t xw_block) {
   if (!blk_elems(src_type) || (xq && hidden % 256) || n_seq == 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(embed_multi_kernel, dim3((hidden + 255) / 256, n_seq), dim3(256), 0, st, src_type, table, tokens, dst, hidden, xq, xq_nw,
-                     xq_ssq, xq_stride, ssq_stride);
+                     xq_ssq, xq_stride, ssq_stride, xw, xw_block);
   return hipGetLastError();
 }
 

@@ -30,7 +30,10 @@ enum TokenMode { MODE_PREFILL = 0, MODE_FORWARD = 1, MODE_GREEDY = 2, MODE_COUNT
 
 // The XQ image (xq.h) of an f32 activation buffer, for int8-MFMA consumers.  `fresh` = the image matches the buffer's
 // current contents; `tag` = the RMSNorm weights it was multiplied with (nullptr: none).
-struct XqBuf { const float* f32 = nullptr; uint8_t* xq = nullptr; float* ssq = nullptr; uint32_t k = 0; bool fresh = false; const float* tag = nullptr; };
+struct XqBuf {
+  const float* f32 = nullptr; uint8_t* xq = nullptr; float* ssq = nullptr; uint32_t k = 0; bool fresh = false; const float* tag = nullptr;
+  uint8_t* xw = nullptr; bool wide = false;   // a batched step's vectors, sequence 0's view: all sequences' wide image (xq.h), and whether it holds what the XQ images hold
+};
 
 // scratch of the batched prompt path (prefill.hip), allocated at the first lgh_prefill_batch that uses it
 struct PfScratch {
@@ -78,6 +81,7 @@ struct BatchScratch {
   float *hidden = nullptr, *xnorm = nullptr, *q = nullptr, *attn_out = nullptr, *act = nullptr, *act2 = nullptr, *logits = nullptr,
         *part_ml = nullptr, *part_acc = nullptr, *amax_v = nullptr, *moe_w = nullptr, *mv_part = nullptr;
   uint64_t mv_part_floats = 0;
+  uint32_t xw_block = 0;                              // bytes between two blocks of the wide images (xq.h): max_batch records
   int *amax_i = nullptr, *moe_sel = nullptr;
   int *d_tokens = nullptr, *d_pos = nullptr, *d_slot = nullptr, *d_log = nullptr;   // the step's control words (device), the greedy token log
   std::vector<float*> kcache, vcache;                 // per layer: [slot][kv_head][max_seq][head_dim]

@@ -354,6 +354,7 @@ int build_mv_group(lgh_ctx* c, const SegSpec* specs, int nseg, const float* norm
           });
           if (rq) return rq;
           q->fresh = true;
+          q->wide = false;
           q->tag = norm_w;
         }
         S.pass[p].xq = q->xq;
@@ -372,11 +373,12 @@ int build_mv_group(lgh_ctx* c, const SegSpec* specs, int nseg, const float* norm
         S.xq_nw = sp.xq_next == 2 ? sp.xq_next_nw : nullptr;
         S.xq_ssq = sp.xq_next == 2 ? qo->ssq : nullptr;
         qo->fresh = true;
+        qo->wide = false;
         qo->tag = S.xq_nw;
       } else if (sp.xq_next && qo && sp.epi == EPI_MOE_SWIGLU && W0.n % 16 == 0 && W0.n <= qo->k && plan.rows_per_wg % 16 == 0) {
         XqBuf* q2 = sp.out2 ? xq_find(c, sp.out2) : nullptr;
         S.xq_out = qo->xq;
-        qo->fresh = true; qo->tag = nullptr;
+        qo->fresh = true; qo->wide = false; qo->tag = nullptr;
         if (q2 && sp.npass > 2) { S.xq_out2 = q2->xq; q2->fresh = true; q2->tag = nullptr; }
       } else if (qo && sp.epi != EPI_ROPE_K && sp.epi != EPI_V_CACHE) {
         qo->fresh = false;

@@ -56,13 +56,14 @@ uint32_t ssq_stride_of(uint32_t k) { return k / 16 + 64; }
 
 // sequence-0 view of a batch vector is registered in the context's XQ registry under its f32 address (engine.hip: xq_get), the
 // other sequences' views follow at the strides above: build_mv_group finds the images it needs there
-int register_views(lgh_ctx* c, float* f32, uint8_t* xq, float* ssq, uint32_t k, uint32_t n) {
+int register_views(lgh_ctx* c, float* f32, uint8_t* xq, float* ssq, uint32_t k, uint32_t n, uint8_t* xw = nullptr) {
   for (uint32_t s = 0; s < n; s++) {
     XqBuf q;
     q.f32 = f32 + (size_t)s * k;
     q.k = k;
     q.xq = xq + (size_t)s * xq_stride_of(k);
     q.ssq = ssq + (size_t)s * ssq_stride_of(k);
+    if (s == 0) q.xw = xw;
     c->xqs.push_back(q);
   }
   return LGH_OK;
@@ -96,7 +97,7 @@ uint32_t moe_group_min() {
 }
 
 int launch_mvb(lgh_ctx* c, int cls, const SegSpec* specs, int nseg, const float* norm_w, uint32_t k, uint32_t n_seq, const uint32_t* out_stride,
-               const uint32_t* resid_stride, const uint32_t* xq_out_k, const MvIndirect ind = MvIndirect{}) {
+               const uint32_t* resid_stride, const uint32_t* xq_out_k, const MvIndirect ind = MvIndirect{}, bool wide_out = false) {
   BatchScratch& Bs = c->batch;
   MvLaunch L;
   uint32_t wg = 0, threads = 0;
@@ -136,6 +137,19 @@ int launch_mvb(lgh_ctx* c, int cls, const SegSpec* specs, int nseg, const float*
     B.xq_out_stride[s] = xq_out_k[s] ? xq_stride_of(xq_out_k[s]) : 0;
     B.ssq_out_stride[s] = xq_out_k[s] ? ssq_stride_of(xq_out_k[s]) : 0;
   }
+  // wide images (xq.h): the input's, made here where its writer left none; the output's, where its reader takes one
+  B.xw_block = Bs.xw_block;
+  bool wide = !ind.cnt;
+  for (int s = 0; s < nseg; s++) wide = wide && specs[s].W[0]->type == specs[0].W[0]->type && mvqb_wide_input(specs[s].W[0]->type, n_seq);
+  if (XqBuf* q = wide ? view_of(c, specs[0].x[0]) : nullptr; q && q->xw) {
+    if (!q->wide && (rc = run_k(c, LGH_K_MISC, LGH_SYM_OTHER, 0, [&] { return xw_from_xq_launch(q->xq, B.xq_stride, q->xw, Bs.xw_block, k, n_seq, c->stream); }))) return rc;
+    q->wide = true;
+    B.xw = q->xw;
+  }
+  if (XqBuf* q = wide_out && L.seg[0].xq_out ? view_of(c, specs[0].out) : nullptr; q && q->xw) {
+    B.xw_out[0] = q->xw;
+    q->wide = true;
+  }
   return run_k(c, cls, LGH_SYM_OTHER, alg, [&] { return mvqb_launch(L, B, wg, threads, c->stream); });
 }
 
@@ -170,15 +184,28 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
   const lgh_model_desc& d = c->d;
   const uint32_t H = d.hidden_size, QD = d.num_heads * d.head_dim;
   int rc;
-  auto stale_all = [&] { for (auto& q : c->xqs) q.fresh = false; };
+  auto stale_all = [&] { for (auto& q : c->xqs) q.fresh = q.wide = false; };
+  // whose wide image (xq.h) the launch that reads it takes: attention's output for wo, the activations for down, the residual stream for Q, K, V (one launch, or one each: below), gate | up and the output head
+  auto wide_qkv = [&](uint32_t li) {
+    const int q = c->layers[li].wq.type, k = c->layers[li].wk.type, v = c->layers[li].wv.type;
+    return mvqb_wide_input(q, n_seq) && ((q == k && q == v) || q == kDevQ40_T16);
+  };
+  auto wide_hidden = [&](uint32_t li) { return li < c->l1 ? wide_qkv(li) : mvqb_wide_input(c->output.type, n_seq); };
+  auto wide_of = [&](float* f32, bool want) -> uint8_t* {   // the image for a launch that writes vector f32, marked as written
+    XqBuf* q = want ? view_of(c, f32) : nullptr;
+    if (!q || !q->xw) return nullptr;
+    q->wide = true;
+    return q->xw;
+  };
   stale_all();
   // ---- embedding rows + the first layer's XQ image (embed_kernel's arithmetic)
   {
     LayerW& L0 = c->layers[c->l0];
     XqBuf* qh = view_of(c, Bs.hidden);
+    uint8_t* const xw = wide_of(Bs.hidden, wide_qkv(c->l0));
     if ((rc = run_k(c, LGH_K_EMBED, LGH_SYM_EMBED, (uint64_t)n_seq * H * blk_bytes(c->embd_type) / blk_elems(c->embd_type), [&] {
            return embed_multi_launch(c->embd_type, c->embd_raw, Bs.d_tokens, Bs.hidden, H, n_seq, qh->xq, L0.attn_norm, qh->ssq, xq_stride_of(H),
-                                     ssq_stride_of(H), c->stream);
+                                     ssq_stride_of(H), c->stream, xw, Bs.xw_block);
          })))
       return rc;
     for (uint32_t s = 0; s < n_seq; s++)
@@ -213,6 +240,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       }
     }
     // ---- attention_cached per sequence (ops.rs:1479-1537): split + merge, the sequence as the grid's second dimension
+    uint8_t* const xw_attn = wide_of(Bs.attn_out, mvqb_wide_input(Lw.wo.type, n_seq));
     if (kv_is_tq(d.kv_cache_type)) {
       // TurboQuantKVCache (kv_turboquant.rs) per sequence: write_kv + attention over the slot's codes; the merge inverts the V rotation
       const int bits = kv_tq_bits(d.kv_cache_type);
@@ -225,7 +253,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
         if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
                return attn_tq_direct_launch(bits, Bs.q, Bs.kq[li], Bs.vq[li], Bs.kv_tmp, Bs.kv_tmp + KD, signs, d.num_heads, d.num_kv_heads, d.head_dim,
                                             d.max_seq_len, scale, Bs.d_pos, Bs.attn_out, qa->xq, c->stream, n_seq, Bs.d_slot, Bs.code_stride, 2 * KD,
-                                            (uint32_t)xq_stride_of(QD));
+                                            (uint32_t)xq_stride_of(QD), xw_attn, Bs.xw_block);
              })))
           return rc;
       } else {
@@ -237,7 +265,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
           return rc;
         if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
                return attn_tq_combine_launch(bits, Bs.part_ml, Bs.part_acc, signs, d.num_heads, d.num_kv_heads, d.head_dim, c->n_splits, Bs.attn_out, qa->xq,
-                                             c->stream, n_seq, (uint32_t)xq_stride_of(QD));
+                                             c->stream, n_seq, (uint32_t)xq_stride_of(QD), xw_attn, Bs.xw_block);
              })))
           return rc;
       }
@@ -247,7 +275,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       XqBuf* qa = view_of(c, Bs.attn_out);
       if ((rc = run_k(c, LGH_K_ATTN, LGH_SYM_ATTN, 0, [&] {
              return attn_multi_direct_launch(Bs.q, Bs.kcache[li], Bs.vcache[li], d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, scale, Bs.d_pos, Bs.d_slot, Bs.cache_stride, n_seq,
-                                             c->n_splits, Bs.attn_out, qa->xq, c->stream);
+                                             c->n_splits, Bs.attn_out, qa->xq, c->stream, xw_attn, Bs.xw_block);
            })))
         return rc;
       for (uint32_t s = 0; s < n_seq; s++)
@@ -262,7 +290,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       XqBuf* qa = view_of(c, Bs.attn_out);
       if ((rc = run_k(c, LGH_K_ATTN_COMBINE, LGH_SYM_ATTN_COMBINE, 0, [&] {
              return attn_combine_multi_launch(Bs.part_ml, Bs.part_acc, d.num_heads, d.num_kv_heads, d.head_dim, d.max_seq_len, Bs.d_pos, c->n_splits, n_seq, Bs.attn_out, qa->xq,
-                                              c->stream);
+                                              c->stream, xw_attn, Bs.xw_block);
            })))
         return rc;
       for (uint32_t s = 0; s < n_seq; s++)
@@ -275,7 +303,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       sp.W[0] = &Lw.wo; sp.x[0] = Bs.attn_out; sp.epi = EPI_RESID; sp.out = Bs.hidden; sp.resid = Bs.hidden; sp.bias = Lw.bo;
       sp.xq_next = 2; sp.xq_next_nw = Lw.ffn_norm;
       const uint32_t os[1] = {H}, rs[1] = {H}, xk[1] = {H};
-      if ((rc = launch_mvb(c, LGH_K_WO, &sp, 1, nullptr, Lw.wo.k, n_seq, os, rs, xk))) return rc;
+      if ((rc = launch_mvb(c, LGH_K_WO, &sp, 1, nullptr, Lw.wo.k, n_seq, os, rs, xk, MvIndirect{}, !Lw.moe() && mvqb_wide_input(Lw.gate.type, n_seq)))) return rc;
       spread_state(c, Bs.hidden, H, n_seq);
     }
     // ---- FFN
@@ -289,7 +317,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
         sp.out = Bs.act;
         sp.xq_next = 1;
         const uint32_t os[1] = {Bs.ffn}, rs[1] = {0}, xk[1] = {Bs.ffn};
-        if ((rc = launch_mvb(c, LGH_K_GATEUP, &sp, 1, Lw.ffn_norm, H, n_seq, os, rs, xk))) return rc;
+        if ((rc = launch_mvb(c, LGH_K_GATEUP, &sp, 1, Lw.ffn_norm, H, n_seq, os, rs, xk, MvIndirect{}, mvqb_wide_input(Lw.down.type, n_seq)))) return rc;
         spread_state(c, Bs.act, Bs.ffn, n_seq);
       }
       {
@@ -297,7 +325,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
         sp.W[0] = &Lw.down; sp.x[0] = Bs.act; sp.epi = EPI_RESID; sp.out = Bs.hidden; sp.resid = Bs.hidden;
         sp.xq_next = 2; sp.xq_next_nw = next_nw;
         const uint32_t os[1] = {H}, rs[1] = {H}, xk[1] = {H};
-        if ((rc = launch_mvb(c, LGH_K_DOWN, &sp, 1, nullptr, Lw.down.k, n_seq, os, rs, xk))) return rc;
+        if ((rc = launch_mvb(c, LGH_K_DOWN, &sp, 1, nullptr, Lw.down.k, n_seq, os, rs, xk, MvIndirect{}, wide_hidden(li + 1)))) return rc;
         spread_state(c, Bs.hidden, H, n_seq);
       }
     } else if (Bs.moe_act && n_seq >= moe_group_min()) {
@@ -335,8 +363,9 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
       }
       {
         XqBuf* qh = view_of(c, Bs.hidden);
+        uint8_t* const xw = wide_of(Bs.hidden, wide_hidden(li + 1));
         if ((rc = run_k(c, LGH_K_MISC, LGH_SYM_OTHER, 0, [&] {
-               return moe_combine_launch(Bs.moe_tmp, Bs.moe_w, topk, Bs.hidden, H, n_seq, next_nw, qh->xq, xq_stride_of(H), qh->ssq, ssq_stride_of(H), c->stream);
+               return moe_combine_launch(Bs.moe_tmp, Bs.moe_w, topk, Bs.hidden, H, n_seq, next_nw, qh->xq, xq_stride_of(H), qh->ssq, ssq_stride_of(H), c->stream, xw, Bs.xw_block);
              })))
           return rc;
         for (uint32_t s = 0; s < n_seq; s++)
@@ -487,7 +516,10 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
   // launch row (any matrix) or 8 slices x the rows of a matrix with fewer than 1600 row tiles
   const uint64_t moe_part = d.num_experts ? (uint64_t)d.num_experts * std::max<uint64_t>((uint64_t)2 * EI, (uint64_t)8 * H) : 0;   // every expert's region
   Bs.mv_part_floats = B * std::max<uint64_t>({moe_part, (uint64_t)8 * 1600 * 16, (uint64_t)d.vocab_size + 16, (uint64_t)2 * ffn, (uint64_t)QD + 2 * d.num_kv_heads * d.head_dim, (uint64_t)H});
-  uint8_t *xq_h = nullptr, *xq_a = nullptr, *xq_f = nullptr, *xq_f2 = nullptr;
+  uint8_t *xq_h = nullptr, *xq_a = nullptr, *xq_f = nullptr, *xq_f2 = nullptr, *xw_h = nullptr, *xw_a = nullptr, *xw_f = nullptr;
+  const bool wide = mvqb_wide_input(kDevQ4K_T16, max_batch);
+  Bs.xw_block = (uint32_t)B * kXwRecord;
+  auto xw_bytes = [&](uint32_t k) { return wide ? (size_t)k / 256 * Bs.xw_block + 1024 : 16; };   // (the last block's transfers are whole kilobytes)
   float *ssq_h = nullptr, *ssq_a = nullptr, *ssq_f = nullptr, *ssq_f2 = nullptr;
   struct { void** p; size_t n; } bufs[] = {
       {(void**)&Bs.hidden, B * H * 4},   {(void**)&Bs.xnorm, B * H * 4},   {(void**)&Bs.q, B * QD * 4},   {(void**)&Bs.attn_out, B * QD * 4},
@@ -501,6 +533,7 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
       {(void**)&xq_a, B * xq_stride_of(QD)},  {(void**)&ssq_a, B * ssq_stride_of(QD) * 4},
       {(void**)&xq_f, B * xq_stride_of(ffn)}, {(void**)&ssq_f, B * ssq_stride_of(ffn) * 4},
       {(void**)&xq_f2, B * xq_stride_of(ffn)}, {(void**)&ssq_f2, B * ssq_stride_of(ffn) * 4},
+      {(void**)&xw_h, xw_bytes(H)}, {(void**)&xw_a, xw_bytes(QD)}, {(void**)&xw_f, xw_bytes(ffn)},
   };
   for (auto& b : bufs) {
     if ((rc = dev_alloc(c, b.p, b.n))) return rc;
@@ -559,9 +592,9 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
       register_views(c, Bs.moe_act, xq_m, ssq_m, EI, (uint32_t)np);
     }
   }
-  register_views(c, Bs.hidden, xq_h, ssq_h, H, max_batch);
-  register_views(c, Bs.attn_out, xq_a, ssq_a, QD, max_batch);
-  register_views(c, Bs.act, xq_f, ssq_f, ffn, max_batch);
+  register_views(c, Bs.hidden, xq_h, ssq_h, H, max_batch, wide ? xw_h : nullptr);
+  register_views(c, Bs.attn_out, xq_a, ssq_a, QD, max_batch, wide ? xw_a : nullptr);
+  register_views(c, Bs.act, xq_f, ssq_f, ffn, max_batch, wide ? xw_f : nullptr);
   register_views(c, Bs.act2, xq_f2, ssq_f2, ffn, max_batch);
   Bs.pos.assign(max_batch, 0);
   Bs.ready = true;

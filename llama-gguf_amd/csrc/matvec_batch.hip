@@ -71,6 +71,8 @@ __device__ __forceinline__ void mvqb_tail(const MvLaunch& L, const MvSeg& S, con
     V.xq_out = S.xq_out ? S.xq_out + (size_t)so * B.xq_out_stride[sg] : nullptr;
     V.xq_ssq = S.xq_ssq ? S.xq_ssq + (size_t)so * B.ssq_out_stride[sg] : nullptr;
     V.pos = B.pos + s;
+    V.xw_out = B.xw_out[sg] ? B.xw_out[sg] + (size_t)so * kXwRecord : nullptr;
+    V.xw_block = B.xw_block;
     mv_epilogue_view(L, S, V, wg, rows_per_wg, red + (size_t)s * red_floats, ssq + s * 8, nslots, MvEpiPre{0.0f, 0.0f, false}, tl);
   }
 }
@@ -687,19 +689,18 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
 //   A: row 4 m + 2 q + half of sequence m + 4 q of eight (a lane of group m gets both halves of sequences m and m + 4), K = lane group's four elements of the half's first digit, then of its second
 //   B: the lane group's four weights twice; a lane unpacks one chunk of 64 elements, so the chunks' words are exchanged between the lane groups (4 x 4, four swaps)
 // (Inputs beyond 2^117 in magnitude may overflow a half where a zero scale would have hidden it.)
-// The records are rewritten to this form as they are staged: 80 instructions per 32 digits (without them 2 % less time: not worth a second form of the
-// records in memory).  gate | up of an 8B model (28672 rows of 4096, Q4_K), 16 sequences: 58 us with mvqb4, 44 here, vector instructions three quarters of it.
+// Who writes the input leaves it in this form (xq.h: the wide image), and a chunk's records of all sequences come as they lie in memory, a chunk ahead, by LDS-DMA.  Rewritten from the digits by every workgroup as they
+// were staged, they took a quarter of the vector instructions.  gate | up of an 8B model (28672 rows of 4096, Q4_K): 16 sequences 47.4 -> 42.7 us (58 with mvqb4), 8 33.7 -> 30.5; wo 13.6 -> 12.4; a step of 4 layers, 16
+// sequences, Q4_K_M 639 -> 617 us, Q4_0 599 -> 554.  Bound by the vector instructions: 343 a tile and block of 16 sequences, 192 of them the sums' own, two thirds of the waves' time (two waves a SIMD).
 // ------------------------------------------------------------------------------------------------
-constexpr uint32_t kX8Group = 512;                   // a lane group's part of a record: [chunk 16][half 2][digit 2][element 4] bf16
-constexpr uint32_t kX8Record = 4 * kX8Group + 32;    // an odd multiple of 32: the halves of eight sequences fall into different banks, whichever lane groups read at once
-constexpr uint32_t kX8Sums = 80;                     // a record's 16 sums ([class][step]), behind all records; 16 sequences' in different banks
-constexpr uint32_t kX8Records = 32;                  // a chunk's records: two per 32 threads
+constexpr uint32_t kX8Records = 32;                  // records of a chunk at most
+constexpr uint32_t mvqb8_block_bytes(uint32_t n_seq) { return (n_seq * kXwRecord + 1023) & ~1023u; }   // a block's records in LDS: whole transfers of a wave
 typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
 
 template <uint32_t MASK, int NB, bool SEQ>
 __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
-  static_assert((MASK & (1u << F_Q80 | 1u << F_Q6K)) == 0, "weights of more than 5 bits do not fit the exact range");
+  static_assert((MASK & (MASK - 1)) == 0 && (MASK & (1u << F_Q80 | 1u << F_Q6K)) == 0, "weights of more than 5 bits do not fit the exact range");
   constexpr int NG = (NB + 7) / 8;
   auto nq = [](int g) { return NB - 8 * g > 4 ? 2 : 1; };          // a last group of up to four sequences: one per lane
   const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
@@ -731,83 +732,54 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
       for (int c = 0; c < 4; c++) acc[g][c][q] = 0.0f;
     }
 
-  RawT16 nxt;
-  {
-    const uint32_t bfirst = ks0 * Gm.nbw;
-    if (active && bfirst < Gm.nblk) mvq_issue_tile<MASK>(fmt, wbase + (size_t)bfirst * tb, lane, nxt);
-  }
-  // a chunk of records (cb blocks x sequences): a thread has a chunk of 16 and a half of two records, fetched a chunk ahead and rewritten into a two-deep LDS buffer
-  const uint32_t sj = (tid >> 1) & 15, sh = tid & 1;
-  const uint32_t s_dig = (sj >> 1) * 128 + sh * 64 + (sj & 1) * 16, s_sum = kXqXs16 + (sj & 3) * 16 + (sj >> 2) * 4;
-  const uint32_t buf_recs = Gm.cb * n_seq, buf_bytes = buf_recs * (kX8Record + kX8Sums);
-  struct { u32x4 d[2]; float sx, xs; } stg[2];
+  // a chunk of records (cb blocks x sequences), requested a chunk ahead into a two-deep LDS buffer
+  const uint32_t blk_bytes = mvqb8_block_bytes(n_seq), buf_bytes = Gm.cb * blk_bytes;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem8;
   auto chunk_len = [&](uint32_t ks, uint32_t b0) { return min(Gm.cb, min(ks * Gm.nbw + Gm.nbw, Gm.nblk) - b0); };
-  auto fetch = [&](uint32_t b0, uint32_t cn) {
-#pragma unroll
-    for (uint32_t k = 0; k < 2; k++) {
-      const uint32_t rec = (tid >> 5) + k * 16;
-      if (rec < cn * n_seq) {
-        const uint32_t bi = rec / n_seq, s = rec - bi * n_seq;
-        const uint8_t* p = L.seg[0].pass[0].xq + (size_t)s * B.xq_stride + (size_t)(b0 + bi) * kXqRecord;   // (all segments and passes share the input)
-        stg[k].d[0] = *reinterpret_cast<const u32x4*>(p + s_dig);
-        stg[k].d[1] = *reinterpret_cast<const u32x4*>(p + s_dig + 32);
-        stg[k].xs = *reinterpret_cast<const float*>(p + s_sum);
-        stg[k].sx = *reinterpret_cast<const float*>(p + s_sum + (kXqSx16 - kXqXs16));
-      }
-    }
-  };
-  auto stash = [&](uint32_t cn, uint32_t buf) {
-    auto pack = [](uint32_t w, float s) {
-      const float a = (float)(int)(int8_t)w * s, b = (float)(int)(int8_t)(w >> 8) * s, c = (float)(int)(int8_t)(w >> 16) * s, d = (float)((int)w >> 24) * s;
-      return make_uint2(__builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u), __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x07060302u));
-    };
-#pragma unroll
-    for (uint32_t k = 0; k < 2; k++) {
-      const uint32_t rec = (tid >> 5) + k * 16;
-      if (rec < cn * n_seq) {
-        uint8_t* to = smem8 + buf * buf_bytes;
-        const float s0 = stg[k].sx * (sh ? 256.0f : 16777216.0f), s1 = stg[k].sx * (sh ? 1.0f : 65536.0f);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const uint2 a = pack(stg[k].d[0][e], s0), b = pack(stg[k].d[1][e], s1);
-          *reinterpret_cast<u32x4*>(to + rec * kX8Record + e * kX8Group + sj * 32 + sh * 16) = u32x4{a.x, a.y, b.x, b.y};
-        }
-        if (sh == 0) *reinterpret_cast<float*>(to + buf_recs * kX8Record + rec * kX8Sums + (sj & 3) * 16 + (sj >> 2) * 4) = stg[k].xs;
-      }
+  auto fetch = [&](uint32_t b0, uint32_t cn, uint32_t buf) {
+    const uint32_t np = blk_bytes >> 10;
+    for (uint32_t i = 0; i < cn; i++) {
+      const uint8_t* src = B.xw + (size_t)(b0 + i) * B.xw_block + lane * 16;
+      for (uint32_t p = wave; p < np; p += kBWaves)
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                     : : "v"(src + p * 1024), "s"(__builtin_amdgcn_readfirstlane((int)(lds0 + buf * buf_bytes + i * blk_bytes + p * 1024))) : "memory", "m0");
     }
   };
   uint32_t ks = ks0, b0 = ks0 * Gm.nbw;
   while (ks < ks1 && b0 >= min(ks * Gm.nbw + Gm.nbw, Gm.nblk)) { ks++; b0 = ks * Gm.nbw; }
   uint32_t buf = 0;
-  if (ks < ks1) fetch(b0, chunk_len(ks, b0));
+  if (ks < ks1) fetch(b0, chunk_len(ks, b0), 0);
+  RawT16 nxt;
+  if (active && ks < ks1) mvq_issue_tile<MASK>(fmt, wbase + (size_t)b0 * tb, lane, nxt);
   while (ks < ks1) {
     const uint32_t sb1 = min(ks * Gm.nbw + Gm.nbw, Gm.nblk);
     const uint32_t cn = chunk_len(ks, b0);
-    stash(cn, buf);
+    // this wave's transfers have arrived: behind them only the next tile's loads
+    if (active) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fmt_loads_per_tile(__builtin_ctz(MASK))) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
     __syncthreads();
     uint32_t nks = ks, nb0 = b0 + cn;   // the chunk after this one
     if (nb0 >= sb1) {
       nks = ks + 1; nb0 = nks * Gm.nbw;
       while (nks < ks1 && nb0 >= min(nks * Gm.nbw + Gm.nbw, Gm.nblk)) { nks++; nb0 = nks * Gm.nbw; }
     }
-    if (nks < ks1) fetch(nb0, chunk_len(nks, nb0));
+    if (!active && nks < ks1) fetch(nb0, chunk_len(nks, nb0), buf ^ 1u);   // (every wave has read the chunk that lay there)
     if (active) {
       for (uint32_t bi = 0; bi < cn; bi++) {
         const uint32_t b = b0 + bi;
         // sequences past the last one repeat it: computed, never stored
-        const uint8_t* rec0 = smem8 + buf * buf_bytes + bi * n_seq * kX8Record;
-        const uint8_t* sum0 = smem8 + buf * buf_bytes + buf_recs * kX8Record + bi * n_seq * kX8Sums;
+        const uint8_t* rec0 = smem8 + buf * buf_bytes + bi * blk_bytes;
         const uint8_t *pa[NG], *px[NG][2];
 #pragma unroll
         for (int g = 0; g < NG; g++) {
-          pa[g] = rec0 + min(8 * g + (n >> 2) + (n & 2) * 2, n_seq - 1) * kX8Record + mq * kX8Group + (n & 1) * 16;
+          pa[g] = rec0 + min(8 * g + (n >> 2) + (n & 2) * 2, n_seq - 1) * kXwRecord + mq * 512 + (n & 1) * 16;
 #pragma unroll
-          for (int q = 0; q < 2; q++) px[g][q] = sum0 + min(8 * g + mq + 4 * q, n_seq - 1) * kX8Sums;
+          for (int q = 0; q < 2; q++) px[g][q] = rec0 + min(8 * g + mq + 4 * q, n_seq - 1) * kXwRecord + kXwSums;
         }
         const bool mins = is(F_Q4K) || is(F_Q5K);
         float xm[4];   // the minima's operand: row 4 m + 2 g + q = sequence 8 g + m + 4 q, K = step
         if (mins) {
-          const uint8_t* p = sum0 + min((n & 2) * 4 + (n >> 2) + (n & 1) * 4, n_seq - 1) * kX8Sums + mq * 4;
+          const uint8_t* p = rec0 + min((n & 2) * 4 + (n >> 2) + (n & 1) * 4, n_seq - 1) * kXwRecord + kXwSums + mq * 4;
 #pragma unroll
           for (int c = 0; c < 4; c++) xm[c] = *reinterpret_cast<const float*>(p + c * 16);
         }
@@ -836,6 +808,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
             tw[pp][0] = r02[0]; tw[pp][1] = r13[0]; tw[pp][2] = r02[1]; tw[pp][3] = r13[1];
           }
         }
+        asm volatile("" : : "v"(tw[3][0]));   // (of the tile's last load)
+        if (bi == 0 && nks < ks1) fetch(nb0, chunk_len(nks, nb0), buf ^ 1u);   // the chunk after this one: behind this tile's wait, which would wait for it too, and in front of the next tile's loads
         {   // the unit's next tile (its next block — of this slice, or of the next one this workgroup walks)
           uint32_t bn = b + 1;
           if (bn == sb1) bn = nks < ks1 ? nb0 : Gm.nblk;
@@ -1228,11 +1202,33 @@ constexpr uint32_t kMvqb4MinSeq = 3;
 // sake of exact sums, they take a step of 16 sequences from 548 to 565)
 constexpr uint32_t kMvqb8MinSeq = 5;
 
+bool mvqb_wide_input(int dev_type, uint32_t n_seq) {
+  const int f = fmt_of_dev_type(dev_type);
+  return n_seq >= kMvqb8MinSeq && (f == F_Q4K || f == F_Q5K || f == F_Q40);
+}
+
+// a wide image where the input's writer left none: a workgroup per record, a thread per word of digits
+__global__ void __launch_bounds__(256) xw_from_xq_kernel(const uint8_t* __restrict__ xq, uint32_t xq_stride, uint8_t* __restrict__ xw, uint32_t xw_block) {
+  const uint8_t* rec = xq + (size_t)blockIdx.y * xq_stride + (size_t)blockIdx.x * kXqRecord;
+  uint8_t* wide = xw + (size_t)blockIdx.x * xw_block + (size_t)blockIdx.y * kXwRecord;
+  const uint32_t t = threadIdx.x, i = (t >> 3) & 3, j = (t >> 5) * 2 + ((t >> 2) & 1), Q = t & 3, slot = (j & 3) * 4 + (j >> 2);   // digit 3 - i of elements 4 Q .. of chunk j
+  const float sx = *reinterpret_cast<const float*>(rec + kXqSx16 + slot * 4) * (float)(1u << (8 * (3 - i)));
+  *reinterpret_cast<uint2*>(wide + Q * 512 + j * 32 + (i >> 1) * 16 + (i & 1) * 8) = xw_digits(*reinterpret_cast<const uint32_t*>(rec + t * 4), sx);
+  if (t < 16) *reinterpret_cast<float*>(wide + kXwSums + t * 4) = *reinterpret_cast<const float*>(rec + kXqXs16 + t * 4);
+}
+
+hipError_t xw_from_xq_launch(const uint8_t* xq, uint32_t xq_stride, uint8_t* xw, uint32_t xw_block, uint32_t k, uint32_t n_seq, hipStream_t st) {
+  if (k == 0 || k % 256 || n_seq == 0 || (uint64_t)n_seq * kXwRecord > xw_block) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(xw_from_xq_kernel, dim3(k / 256, n_seq), dim3(256), 0, st, xq, xq_stride, xw, xw_block);
+  return hipGetLastError();
+}
+
 template <uint32_t MASK, int NB>
 static hipError_t mvqb8_go(const MvLaunch& L, const MvBatch& B, Mvqb2Geom Gm, bool seq, uint32_t groups, hipStream_t st) {
   static bool attr_set[2][64] = {};
+  if (!B.xw || (uint64_t)B.n_seq * kXwRecord > B.xw_block) return hipErrorInvalidValue;
   Gm.cb = std::max(1u, std::min(Gm.nbw, kX8Records / B.n_seq));
-  Gm.ssq_at = 2 * Gm.cb * B.n_seq * (kX8Record + kX8Sums);
+  Gm.ssq_at = 2 * Gm.cb * mvqb8_block_bytes(B.n_seq);
   const size_t lds = Gm.ssq_at + mvqb_fuse_lds(B.n_seq);
   if (seq) {
     if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb8_kernel<MASK, NB, true>), 160 * 1024, attr_set[0]); e != hipSuccess) return e;
@@ -1302,7 +1298,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   }
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
-    if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
+    if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);   // (masks of two formats hold Q6_K)
     else if (B.n_seq < kMvqb8MinSeq) e = mvqb4_go<MASK, 4>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 8) e = mvqb8_go<MASK, 8>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 12) e = mvqb8_go<MASK, 12>(L, B, Gm, seq, groups, st);

@@ -321,20 +321,21 @@ hipError_t moe_group_launch(const int* sel, uint32_t n_seq, uint32_t top_k, uint
 // consumer's norm weights and the per-chunk sums of squares.  tmp: [n_seq * top_k][H] expert outputs; grid (H / 256, n_seq).
 __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restrict__ tmp, const float* __restrict__ moe_w, uint32_t top_k, float* __restrict__ hidden,
                                                           uint32_t H, const float* __restrict__ nw, uint8_t* __restrict__ xq, uint32_t xq_stride,
-                                                          float* __restrict__ ssq, uint32_t ssq_stride) {
+                                                          float* __restrict__ ssq, uint32_t ssq_stride, uint8_t* __restrict__ xw, uint32_t xw_block) {
   const uint32_t s = blockIdx.y, row = blockIdx.x * 256 + threadIdx.x;
   if (row >= H) return;
   float acc = 0.0f;
   for (uint32_t p = 0; p < top_k; p++) acc += moe_w[s * top_k + p] * tmp[((size_t)s * top_k + p) * H + row];
   const float outv = acc + hidden[(size_t)s * H + row];
   hidden[(size_t)s * H + row] = outv;
-  if (xq) xq_store_chunk(xq + (size_t)s * xq_stride, row >> 4, outv * (nw ? nw[row] : 1.0f), ssq ? ssq + (size_t)s * ssq_stride : nullptr, outv);
+  if (xq) xq_store_chunk(xq + (size_t)s * xq_stride, row >> 4, outv * (nw ? nw[row] : 1.0f), ssq ? ssq + (size_t)s * ssq_stride : nullptr, outv, row,
+                         xw ? xw + (size_t)s * kXwRecord : nullptr, xw_block);
 }
 
 hipError_t moe_combine_launch(const float* tmp, const float* moe_w, uint32_t top_k, float* hidden, uint32_t H, uint32_t n_seq, const float* nw,
-                              uint8_t* xq, uint32_t xq_stride, float* ssq, uint32_t ssq_stride, hipStream_t st) {
+                              uint8_t* xq, uint32_t xq_stride, float* ssq, uint32_t ssq_stride, hipStream_t st, uint8_t* xw, uint32_t xw_block) {
   if (H % 256 || n_seq == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(moe_combine_kernel, dim3(H / 256, n_seq), dim3(256), 0, st, tmp, moe_w, top_k, hidden, H, nw, xq, xq_stride, ssq, ssq_stride);
+  hipLaunchKernelGGL(moe_combine_kernel, dim3(H / 256, n_seq), dim3(256), 0, st, tmp, moe_w, top_k, hidden, H, nw, xq, xq_stride, ssq, ssq_stride, xw, xw_block);
   return hipGetLastError();
 }
 

@@ -45,7 +45,7 @@ __device__ __forceinline__ void mv_epilogue_prefetch_rope(int epi, uint32_t pos,
 
 // The vectors an epilogue writes and reads: the segment's own (single-sequence launches) or one sequence's slice of them
 // (matvec_batch.hip: every sequence has its own output, residual, XQ image, position and KV cache slot).
-struct MvEpiView { float* out; const float* resid; uint8_t* xq_out; float* xq_ssq; const int* pos; };
+struct MvEpiView { float* out; const float* resid; uint8_t* xq_out; float* xq_ssq; const int* pos; uint8_t* xw_out = nullptr; uint32_t xw_block = 0; };
 
 // Per-row epilogue, one thread per row (or per row pair for RoPE)
 // `nslots` = partial sums per (pass, row) in `red`, laid out red[(p * nslots + slot) * rows_per_wg + row]
@@ -138,7 +138,7 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
   if (xq && has_out) {
     const float* nw = S.xq_nw;
     const float w = !nw ? 1.0f : (pre.valid && (S.epi == EPI_RESID || S.epi == EPI_MOE_DOWN)) ? pre.b : nw[row];
-    xq_store_chunk(xq, row >> 4, outv * w, V.xq_ssq, outv, tid);
+    xq_store_chunk(xq, row >> 4, outv * w, V.xq_ssq, outv, tid, V.xw_out, V.xw_block);
   }
 }
 

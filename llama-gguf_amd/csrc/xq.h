@@ -30,12 +30,23 @@ constexpr uint32_t kXqXs16 = 1024, kXqSx16 = 1088;
 
 __host__ __device__ inline size_t xq_bytes(size_t k) { return (k + 255) / 256 * kXqRecord; }
 
+// The wide image of a batched step's input (matvec_batch.hip, mvqb8: its matrix cores take the digits as bf16 numbers).  A record is [element group 4][chunk 16][half 2][digit 2][element 4] bf16 (element 4 g + e of a chunk
+// of 16; the high half's digits first), a digit times its power of 256 times the chunk's scale, which is a power of two: exact;  then the 16 sums of XQ.  Records lie [block][sequence], blocks `xw_block` bytes apart.
+// An odd multiple of 32 bytes: the halves of eight sequences fall into different LDS banks, whichever lane groups read at once.
+constexpr uint32_t kXwSums = 2048, kXwRecord = kXwSums + 64 + 32;
+
+// four digits (a word of limb bytes) times their scale
+__device__ __forceinline__ uint2 xw_digits(uint32_t w, float s) {
+  const float a = (float)(int)(int8_t)w * s, b = (float)(int)(int8_t)(w >> 8) * s, c = (float)(int)(int8_t)(w >> 16) * s, d = (float)((int)w >> 24) * s;
+  return make_uint2(__builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u), __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x07060302u));
+}
+
 // Called by the 16 consecutive lanes (a DPP row: lane % 16 == element % 16) that hold the 16 elements of chunk
 // `chunk` (global index, element / 16) of a vector; `v` is this lane's element (already multiplied by the norm weight
 // when the consumer normalises).  Writes the chunk's 64 limb bytes, its sum and its scale.
-// With `ssq_part` the chunk's sum of `raw`^2 (the un-normalised values) goes to ssq_part[chunk].
+// With `ssq_part` the chunk's sum of `raw`^2 (the un-normalised values) goes to ssq_part[chunk]; with `xw` the chunk goes to that wide image, too.
 __device__ __forceinline__ void xq_store_chunk(uint8_t* xq, uint32_t chunk, float v, float* ssq_part = nullptr, float raw = 0.0f,
-                                               uint32_t tid = threadIdx.x) {
+                                               uint32_t tid = threadIdx.x, uint8_t* xw = nullptr, uint32_t xw_block = 0) {
   const uint32_t l16 = tid & 15;
   // max |v| and sum over the 16 lanes, in every lane (quad_perm x2, row_half_mirror, row_mirror)
   float amax = fabsf(v), sum = v;
@@ -65,6 +76,11 @@ __device__ __forceinline__ void xq_store_chunk(uint8_t* xq, uint32_t chunk, floa
     *reinterpret_cast<float*>(rec + kXqXs16 + slot * 4) = sum;
     *reinterpret_cast<float*>(rec + kXqSx16 + slot * 4) = __uint_as_float((e + 1u - 30u) << 23);   // s * 2^-30, s = 2^(e-126)
     if (ssq_part) ssq_part[chunk] = sq;
+  }
+  if (xw) {
+    uint8_t* wide = xw + (size_t)blk * xw_block;
+    *reinterpret_cast<uint2*>(wide + Q * 512 + j * 32 + (i >> 1) * 16 + (i & 1) * 8) = xw_digits(word, __uint_as_float((e + 1u - 30u + 8u * q) << 23));
+    if (l16 == 0) *reinterpret_cast<float*>(wide + kXwSums + ((j & 3) * 4 + (j >> 2)) * 4) = sum;
   }
 }
 
