@@ -18,6 +18,7 @@ struct PfSeg {
   uint32_t col0;         // first column in the partial-sum rows
   uint32_t rg_begin;     // first row group (workgroup x index) of this matrix
   int fmt;
+  uint64_t w_z = 0;      // bytes between the weights of consecutive experts
 };
 
 struct PfGemm {
@@ -27,11 +28,13 @@ struct PfGemm {
   uint32_t S;            // k-splits (gridDim.y)
   uint32_t ncols;        // floats per partial-sum row
   const uint8_t* xh;     // input activations [128][k] f16, XH layout
+  size_t xh_z;           // bytes between the inputs of consecutive experts
+  uint32_t n_experts;    // experts of the launch (gridDim.z; MoE), 0: a dense product
   float* part;           // [S][part_rows][ncols]
   uint32_t part_rows;    // rows per split: 128, or kPfMoeRows when the experts of a MoE layer share one buffer
-  const int* row_base;   // optional (MoE): device word, first row of this expert's batch in the buffer
-  uint32_t m_tokens;
-  const int* m_count;    // optional (MoE): device word with the number of real rows; overrides m_tokens, 0 rows = nothing to do
+  const int* row_base;   // MoE: device words, the first row of each expert's batch in the buffer
+  uint32_t m_tokens;     // (MoE: of an expert, on average)
+  const int* m_count;    // MoE: device words, the number of each expert's real rows; 0 rows = nothing to do
   // gate | up with SwiGLU: the activations (XH), the input's sums of squares and the norm they stand for
   uint8_t* act;
   const float* ssq;
@@ -40,9 +43,9 @@ struct PfGemm {
 };
 
 bool pf_supported_type(int dev_type);
-size_t pf_part_bytes(const uint32_t* n_rows, int nw, uint32_t k, uint32_t part_rows = kPfTokens);
+size_t pf_part_bytes(const uint32_t* n_rows, int nw, uint32_t k, uint32_t n_experts = 0);
 hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, float* part, size_t part_bytes, uint32_t m_tokens,
-                          uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t expert = 0, const int* m_count = nullptr,
+                          uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t n_experts = 0, size_t xh_z = 0, const int* m_count = nullptr,
                           uint32_t part_rows = kPfTokens, const int* row_base = nullptr);
 // silu(gate) * up of one launch -> XH
 bool pf_pairs(const DevWeight* gate, const DevWeight* up);

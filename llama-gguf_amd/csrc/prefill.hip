@@ -73,7 +73,7 @@ hipError_t pf_read_stamps(unsigned long long* host, size_t n) {
 // MT = token tiles computed: 8 for a full block, 4 / 2 when at most 64 / 32 rows are real (short prompts, and the rows routed
 // to one MoE expert — about 32 of 128 with 2-of-8 routing): the MFMAs, the LDS reads and the activation DMA shrink with it.
 template <int F, int MT>
-__device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32_t rg, uint32_t ks, uint32_t m_tiles, uint8_t* smem) {
+__device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32_t z, uint32_t rg, uint32_t ks, uint32_t m_tiles, uint8_t* smem) {
   constexpr uint32_t kBuf = (uint32_t)MT * 16 * 512;                // a slab's rows that are copied
   constexpr uint32_t kDma = kBuf / kPfWaves;   // a wave's share of the MT * 16 rows of a slab that are copied
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -87,7 +87,7 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
 #pragma unroll
   for (int r = 0; r < kPfRT; r++) {
     const uint32_t tl = tile0 + r < sg.ntiles ? tile0 + r : sg.ntiles - 1;   // clamped: loads are unconditional
-    wt[r] = sg.w + (size_t)tl * G.nblk * tb;
+    wt[r] = sg.w + (size_t)z * sg.w_z + (size_t)tl * G.nblk * tb;
   }
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
 
@@ -99,7 +99,7 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
 
   // one 64 KB slab -> LDS buffer `buf`: this wave's quarter, 16 x 1 KB by LDS-DMA (no registers)
   auto x_dma = [&](uint32_t b, uint32_t buf) {
-    const uint8_t* src = G.xh + (size_t)b * kPfSlabBytes + wave * kDma + lane * 16;
+    const uint8_t* src = G.xh + (size_t)z * G.xh_z + (size_t)b * kPfSlabBytes + wave * kDma + lane * 16;
     const uint32_t dst = lds_base + buf * kBuf + wave * kDma;
 #pragma unroll
     for (int i = 0; i < (int)(kDma / 1024); i++) {
@@ -198,7 +198,7 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
   if (b < b1) block(std::false_type{}, b);
   // partial sums: lane holds, per (row tile, token tile), rows 4c .. 4c+3 of token n
   uint32_t row0 = 0;
-  if (G.row_base) asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(row0) : "s"(G.row_base) : "memory");
+  if (G.row_base) asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(row0) : "s"(G.row_base + z) : "memory");
   float* part = G.part + ((size_t)ks * G.part_rows + row0) * G.ncols;
 #pragma unroll
   for (int r = 0; r < kPfRT; r++) {
@@ -217,11 +217,11 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
   LGH_PF_STAMP(14);
 }
 
-// A mixture's experts: the token tiles are chosen in the kernel
-template <uint32_t MASK>
-__global__ void __launch_bounds__(kPfWaves * 64) pf_experts_kernel(const PfGemm G) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-  const uint32_t rgid = blockIdx.x;
+// A mixture's experts, all of a layer in one launch (blockIdx.z; a launch each, gate | up and down, was 16 launches of a third of the chip's rate: 8 experts of 14336 x 4096 in Q5_K, 64 tokens, 370 -> 288 us with the sums'
+// fold; one block of weights under way a wave, 3.5 TB/s).  The token tiles are chosen here;  FIXED: experts of full blocks
+template <uint32_t MASK, bool FIXED>
+__device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem) {
+  const uint32_t rgid = blockIdx.x, z = blockIdx.z;
   int si = 0;
   if (G.nseg > 1 && rgid >= G.seg[1].rg_begin) si = 1;
   if (G.nseg > 2 && rgid >= G.seg[2].rg_begin) si = 2;
@@ -229,14 +229,14 @@ __global__ void __launch_bounds__(kPfWaves * 64) pf_experts_kernel(const PfGemm 
   const uint32_t rg = rgid - sg.rg_begin;
   auto is = [&](int f) { return (MASK & (1u << f)) && (MASK == (1u << f) || sg.fmt == f); };
   uint32_t cnt;   // this expert's row count lives on the device (no host round trip per layer)
-  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cnt) : "s"(G.m_count) : "memory");
+  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cnt) : "s"(G.m_count + z) : "memory");
   if (cnt == 0) return;
   const uint32_t m_tiles = (cnt + 15) / 16;
-#define LGH_PF_RUN(F)                                                                    \
-  do {                                                                                   \
-    if (m_tiles <= 2) pf_body<F, 2>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);            \
-    else if (m_tiles <= 4) pf_body<F, 4>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);       \
-    else pf_body<F, kPfMT>(G, sg, rg, blockIdx.y, m_tiles, pf_smem);                     \
+#define LGH_PF_RUN(F)                                                                              \
+  do {                                                                                             \
+    if (!FIXED && m_tiles <= 2) pf_body<F, 2>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);         \
+    else if (!FIXED && m_tiles <= 4) pf_body<F, 4>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);    \
+    else pf_body<F, kPfMT>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);                            \
   } while (0)
   if (is(PF_Q4K)) LGH_PF_RUN(PF_Q4K);
   else if (is(PF_Q6K)) LGH_PF_RUN(PF_Q6K);
@@ -244,6 +244,16 @@ __global__ void __launch_bounds__(kPfWaves * 64) pf_experts_kernel(const PfGemm 
   else if (is(PF_Q80)) LGH_PF_RUN(PF_Q80);
   else if (is(PF_Q40)) LGH_PF_RUN(PF_Q40);
 #undef LGH_PF_RUN
+}
+template <uint32_t MASK>
+__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+  pf_gemm_device<MASK, true>(G, pf_smem);
+}
+template <uint32_t MASK, int MT>
+__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_few_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
+  pf_gemm_device<MASK, MT != 0>(G, pf_smem);
 }
 
 // 1 / rms of token t from the per-chunk sums of squares its producer left (simd.rs:847-878); 1 when there is no norm
@@ -567,12 +577,13 @@ template <auto* Kernel, size_t LDS, int WAVES>
 static hipError_t pf_gemm_run(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
   static bool attr_set[64] = {};
   if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(Kernel), (int)LDS, attr_set); e != hipSuccess) return e;
-  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S), dim3(WAVES * 64), LDS, st, G);
+  hipLaunchKernelGGL(Kernel, dim3(n_rg, G.S, G.n_experts ? G.n_experts : 1), dim3(WAVES * 64), LDS, st, G);
   return hipGetLastError();
 }
 template <uint32_t MASK>
 static hipError_t pf_gemm_go(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
-  if (G.m_count) return pf_gemm_run<&pf_experts_kernel<MASK>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
+  if (G.m_count && G.m_tokens > (uint32_t)kPfTokens * 3 / 4) return pf_gemm_run<&pf_gemm_kernel<MASK>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
+  if (G.m_count) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 0>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
   switch ((G.m_tokens + 31) / 32) {
     case 1: return pf_gemm_run<&pf_rows_kernel<MASK, 1>, pf_half_lds(1), 2 * kPfWaves>(G, n_rg, st);
     case 2: return pf_gemm_run<&pf_rows_kernel<MASK, 2>, pf_half_lds(2), 2 * kPfWaves>(G, n_rg, st);
@@ -586,31 +597,33 @@ bool pf_supported_type(int dev_type) { return pf_fmt_of(dev_type) >= 0; }
 // 16-row tiles of a workgroup
 static uint32_t pf_wg_tiles(bool experts) { return experts ? kPfWaves * kPfRT : kPfWaves * 2; }
 
-// k-splits of a GEMM over matrices with n_rows[i] rows and k columns: as many as keep the launch within one workgroup per CU
-static void pf_plan(const uint32_t* n_rows, int nw, uint32_t k, bool experts, uint32_t* S_out) {
-  const uint32_t nblk = k / 256, wt = pf_wg_tiles(experts);
-  uint32_t rg = 0;
-  for (int i = 0; i < nw; i++) rg += (n_rows[i] / 16 + wt - 1) / wt;
-  uint32_t S = rg >= (uint32_t)kNumCU ? 1 : kNumCU / rg;
+// k-splits of a GEMM over matrices with n_rows[i] rows and k columns: as many as keep the launch within one workgroup per CU;  of a layer's experts, whose workgroups have unequal work, as many as make two per CU
+// (a layer of 8 experts of 14336 x 4096 in Q5_K, us, products and fold, 16 / 64 / 128 tokens: gate | up unsplit 148 / 198 / 231, in two 156 / 196 / 229; down, 128 workgroups unsplit, in two 88 / 106 / 140, in four 89 / 102 / 122)
+static void pf_plan(const uint32_t* n_rows, int nw, uint32_t k, uint32_t n_experts, uint32_t* S_out) {
+  const uint32_t nblk = k / 256, wt = pf_wg_tiles(n_experts != 0), fill = n_experts ? 2 * kNumCU : kNumCU;
+  uint32_t wgs = 0;
+  for (int i = 0; i < nw; i++) wgs += (n_rows[i] / 16 + wt - 1) / wt;
+  if (n_experts) wgs *= n_experts;
+  uint32_t S = wgs >= fill ? 1 : fill / wgs;
   if (S > nblk) S = nblk;
   const uint32_t per = (nblk + S - 1) / S;
   *S_out = (nblk + per - 1) / per;
 }
 
 // bytes of partial sums such a GEMM writes
-size_t pf_part_bytes(const uint32_t* n_rows, int nw, uint32_t k, uint32_t part_rows) {
+size_t pf_part_bytes(const uint32_t* n_rows, int nw, uint32_t k, uint32_t n_experts) {
   uint32_t S, cols = 0;
-  pf_plan(n_rows, nw, k, part_rows != (uint32_t)kPfTokens, &S);
+  pf_plan(n_rows, nw, k, n_experts, &S);
   for (int i = 0; i < nw; i++) cols += n_rows[i];
-  return (size_t)S * part_rows * cols * 4;
+  return (size_t)S * (n_experts ? kPfMoeRows : kPfTokens) * cols * 4;
 }
 
 // Plans and launches one GEMM: up to 3 weight matrices that share the input XH (k elements per token), outputs side by
 // side in the partial-sum buffer.  Returns the split count through *S_out (the consumer adds that many partials).
 hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, float* part, size_t part_bytes, uint32_t m_tokens,
-                          uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t expert, const int* m_count, uint32_t part_rows,
+                          uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t n_experts, size_t xh_z, const int* m_count, uint32_t part_rows,
                           const int* row_base) {
-  if (nw < 1 || nw > 3 || m_tokens == 0 || m_tokens > (uint32_t)kPfTokens) return hipErrorInvalidValue;
+  if (nw < 1 || nw > 3 || m_tokens == 0 || m_tokens > (uint32_t)kPfTokens || (n_experts != 0) != (m_count != nullptr)) return hipErrorInvalidValue;
   PfGemm G{};
   const uint32_t k = W[0]->k;
   if (k % 256) return hipErrorInvalidValue;
@@ -620,8 +633,9 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
   uint32_t rg = 0, col = 0, mask = 0, n_rows[3] = {0, 0, 0};
   for (int i = 0; i < nw; i++) {
     const int f = pf_fmt_of(W[i]->type);
-    if (f < 0 || W[i]->k != k || W[i]->n % 16 || expert >= W[i]->n_stack) return hipErrorInvalidValue;
-    G.seg[i].w = W[i]->plane[0] + (uint64_t)expert * W[i]->stack_stride[0];   // expert stacks: [expert][tiles]
+    if (f < 0 || W[i]->k != k || W[i]->n % 16 || std::max(n_experts, 1u) > W[i]->n_stack) return hipErrorInvalidValue;
+    G.seg[i].w = W[i]->plane[0];
+    G.seg[i].w_z = W[i]->stack_stride[0];   // expert stacks: [expert][tiles]
     G.seg[i].ntiles = W[i]->n / 16;
     G.seg[i].col0 = col;
     G.seg[i].rg_begin = rg;
@@ -631,9 +645,11 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
     col += W[i]->n;
     n_rows[i] = W[i]->n;
   }
-  pf_plan(n_rows, nw, k, m_count != nullptr, &G.S);
+  pf_plan(n_rows, nw, k, n_experts, &G.S);
   G.ncols = col;
   G.xh = xh;
+  G.xh_z = xh_z;
+  G.n_experts = n_experts;
   G.part = part;
   G.m_tokens = m_tokens;
   G.m_count = m_count;
