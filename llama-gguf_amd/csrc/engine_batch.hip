@@ -598,12 +598,14 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
   register_views(c, Bs.act2, xq_f2, ssq_f2, ffn, max_batch);
   Bs.pos.assign(max_batch, 0);
   Bs.ready = true;
-  // a step of every size that launches kernels of its own (matvec_batch.hip: groups of four and eight, of up to 4, 8, 12 and 16 sequences; up to four the epilogue's form goes by the rows), eagerly, before any of them is first
+  // a step of every size that launches kernels of its own (matvec_batch.hip: groups of four and eight, of up to 4, 8, 12 and 16 sequences; up to four the epilogue's form goes by the rows; a mixture's gate | up takes, up to a size that
+  // goes by its experts, a kernel of its own, so there the largest of each group too), eagerly, before any of them is first
   // launched inside a capture (engine.hip: warm_kernels explains the ROCm trap); they write row 0 of the slots' caches, which a slot's first real token overwrites
   uint32_t slots0[kMaxBatch], toks0[kMaxBatch] = {};
   for (uint32_t i = 0; i < (uint32_t)kMaxBatch; i++) slots0[i] = i;
-  for (uint32_t n : {1u, 2u, 3u, 4u, 5u, 9u, 13u}) {
-    if (n > max_batch) break;
+  for (uint32_t n = 1; n <= max_batch; n++) {
+    const bool group = n <= 5 || n == 9 || n == 13, last = n == 8 || n == 16 || n == max_batch;
+    if (!group && !(last && Bs.moe_act)) continue;
     Bs.attn_short = false;
     if ((rc = stage_control(c, slots0, toks0, n))) return rc;
     if (n == 1 && short_attn_rows(c, 1))   // (the single-launch attention's kernel is the same for every size; attn_out is scratch here.  In front of the step, which moves the positions on: a context may hold one row)

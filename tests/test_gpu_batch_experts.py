@@ -36,3 +36,36 @@ def test_experts_of_few_entries_are_bitwise_the_single_sequence(pkg, mix, hidden
                 assert np.array_equal(got[s].view(np.uint32), want[s][step].view(np.uint32)), (n, s, step)
     multi.close()
     single.close()
+
+
+_FRESH = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+import __graft_entry__ as graft
+pkg = graft.load_package()
+cfg = pkg.make_config("test-moe", max_seq_len=32, num_layers=1, num_experts=int(sys.argv[3]), expert_intermediate_size=10240)
+multi = pkg.HipGpuInference.from_model(pkg.SynthModel(cfg, mix=sys.argv[2]), 32)
+slots, n = int(sys.argv[4]), int(sys.argv[5])
+multi.batch_create(slots)
+tok = np.random.default_rng(7).integers(0, cfg.vocab_size, (n, 4))
+got = [multi.forward_multi(list(range(n)), tok[:, i])[0].copy() for i in range(4)]
+for s in range(n):
+    multi.reset()
+    for i in range(4):
+        want = multi.forward(int(tok[s, i]))
+        assert np.array_equal(got[i][s].view(np.uint32), want.view(np.uint32)), (s, i)
+print("equal")
+"""
+
+
+@pytest.mark.parametrize("mix,experts,slots,n", [("Q8_0", 8, 8, 7), ("Q5_K_M", 5, 7, 7)])
+def test_first_step_of_a_size_in_a_fresh_process(mix, experts, slots, n):
+    """A kernel whose first launch in the process happens during a capture is not replayed with the graph: the sizes from which mvqb2 takes over lie inside its groups of up to 4, 8 and 16, so lgh_batch_create launches
+    the largest of each group as well."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", _FRESH, root, mix, str(experts), str(slots), str(n)], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.strip().endswith("equal"), out.stdout + out.stderr
