@@ -15,8 +15,8 @@
 //   XH(attn) --GEMM wo--> partials --pf_resid (+bias, +residual)--> h, XH(h * ffn_norm), sums of squares per token
 //   XH --GEMM gate|up--> partials --pf_swiglu (x 1/rms)--> XH(act), or both in pf_pair_kernel; --GEMM down--> partials --pf_resid--> h, XH(h * attn_norm')
 // MoE layers (moe.rs:321-413): the f32 decode router runs once per token of the block, the (token, slot) pairs are grouped
-// by expert into one row space (prefill.h), and every expert runs ONCE over its rows: one gather launch, a gate|up GEMM per
-// expert, one SwiGLU launch, a down GEMM per expert, one combine launch (routing weight * expert output in selection order,
+// by expert into one row space (prefill.h), and every expert runs ONCE over its rows: one gather launch, one gate|up GEMM
+// of all experts, one SwiGLU launch, one down GEMM, one combine launch (routing weight * expert output in selection order,
 // then the residual).
 // The RMSNorm's 1/rms is a per-token scalar and the GEMM is linear: XH holds h * norm_weight and the kernel that adds
 // up the GEMM's partial sums multiplies by 1/rms (from the sums of squares the producer of h left) — as in the decode path.
