@@ -512,9 +512,15 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
   Bs.ffn = ffn;
   Bs.cache_stride = (uint64_t)d.num_kv_heads * d.max_seq_len * d.head_dim;
   const size_t B = max_batch;
+  // a mixture's layers with every expert's matrices read once a step (the multi-sequence kernels run 8-wave workgroups: both expert shapes must plan to T x G = 8, as Mixtral's do)
+  bool any_moe = false;
+  for (uint32_t i = c->l0; i < c->l1; i++) any_moe = any_moe || c->layers[i].moe();
+  MvPlan pg{}, pd{};
+  const bool plans = mvq_plan(H, EI, 2, &pg, EI) == hipSuccess && mvq_plan(EI, H, 1, &pd, H) == hipSuccess && pg.threads == 512 && pd.threads == 512;
+  const bool by_expert = any_moe && plans && d.num_experts_per_token <= 8 && d.num_experts <= 64 && EI % 256 == 0;
   // partial sums between the two launches of a multi-sequence mat-vec (matvec_batch.hip, mvqb2): per sequence either one value per
-  // launch row (any matrix) or 8 slices x the rows of a matrix with fewer than 1600 row tiles
-  const uint64_t moe_part = d.num_experts ? (uint64_t)d.num_experts * std::max<uint64_t>((uint64_t)2 * EI, (uint64_t)8 * H) : 0;   // every expert's region
+  // launch row (any matrix) or 8 slices x the rows of a matrix with fewer than 1600 row tiles; of a mixture a region an expert
+  const uint64_t moe_part = by_expert ? d.num_experts * std::max(mvqb_expert_part_floats(2 * ((EI + 15) / 16), pg.T, 1), mvqb_expert_part_floats((H + 15) / 16, pd.T, 1)) : 0;
   Bs.mv_part_floats = B * std::max<uint64_t>({moe_part, (uint64_t)8 * 1600 * 16, (uint64_t)d.vocab_size + 16, (uint64_t)2 * ffn, (uint64_t)QD + 2 * d.num_kv_heads * d.head_dim, (uint64_t)H});
   uint8_t *xq_h = nullptr, *xq_a = nullptr, *xq_f = nullptr, *xq_f2 = nullptr, *xw_h = nullptr, *xw_a = nullptr, *xw_f = nullptr;
   const bool wide = mvqb_wide_input(kDevQ4K_T16, max_batch);
@@ -572,12 +578,7 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
     c->stats.kv_bytes += 2 * n;
   }
   {   // MoE layers: the expert-grouped step's buffers ((sequence, slot) pairs)
-    bool any_moe = false;
-    for (uint32_t i = c->l0; i < c->l1; i++) any_moe = any_moe || c->layers[i].moe();
-    // (the multi-sequence kernels run 8-wave workgroups: both expert shapes must plan to T x G = 8, as Mixtral's do)
-    MvPlan pg{}, pd{};
-    const bool plans = mvq_plan(H, EI, 2, &pg, EI) == hipSuccess && mvq_plan(EI, H, 1, &pd, H) == hipSuccess && pg.threads == 512 && pd.threads == 512;
-    if (any_moe && plans && d.num_experts_per_token <= 8 && d.num_experts <= 64 && EI % 256 == 0) {
+    if (by_expert) {
       const size_t np = B * d.num_experts_per_token;
       uint8_t* xq_m = nullptr;
       float* ssq_m = nullptr;

@@ -1329,6 +1329,15 @@ static uint32_t mvqb2_min_seq() {
   return v;
 }
 
+// enough units to fill the chip with whole rows per workgroup; with fewer the k-slices are a grid dimension
+static bool mvqb2_whole_rows(uint32_t n_units, uint32_t T) {
+  static const uint32_t min_groups = [] { const char* e = std::getenv("LGH_MVQB2_SEQ_GROUPS"); return e ? (uint32_t)std::atoi(e) : 160u; }();
+  return (n_units + kBWaves - 1) / kBWaves >= min_groups || T == 1;
+}
+
+// partial sums of one expert in a launch over a layer's experts: matrices of n_units row tiles in T k-slices
+uint64_t mvqb_expert_part_floats(uint32_t n_units, uint32_t T, uint32_t n_seq) { return (uint64_t)(mvqb2_whole_rows(n_units, T) ? 1 : T) * n_seq * n_units * 16; }
+
 // `L` built like a single-sequence launch (engine.hip: build_mv_group, with the batch cap on tiles per workgroup); sequences'
 // vectors at the strides in `B`
 hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uint32_t threads, hipStream_t st) {
@@ -1355,8 +1364,7 @@ hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uin
     Gm.ub1 = L.nseg > 1 ? ub[1] : Gm.n_units;
     Gm.ub2 = L.nseg > 2 ? ub[2] : Gm.n_units;
     uint32_t groups = (Gm.n_units + kBWaves - 1) / kBWaves;
-    static const uint32_t seq_min_groups = [] { const char* e = std::getenv("LGH_MVQB2_SEQ_GROUPS"); return e ? (uint32_t)std::atoi(e) : 160u; }();
-    const bool seq = groups >= seq_min_groups || Gm.T == 1;  // enough units to fill the chip with whole rows per workgroup
+    const bool seq = mvqb2_whole_rows(Gm.n_units, Gm.T);
     Gm.nslots = seq ? 1 : Gm.T;
     if (seq && L.nseg == 1 && (S0.epi == EPI_STORE || S0.epi == EPI_RESID || S0.epi == EPI_SWIGLU)) {
       Gm.fuse = S0.npass == 2 ? 2 : 1;
@@ -1366,7 +1374,7 @@ hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uin
     const int nb_inst = B.n_seq <= 4 ? 4 : B.n_seq <= 8 ? 8 : 16;
     Gm.cb = std::max(1u, std::min(Gm.nbw, mvqb2_stage_bytes((mask & (mask - 1)) == 0, nb_inst) / (B.n_seq * (uint32_t)kXqRecord)));
     const size_t lds_x = (size_t)2 * Gm.cb * B.n_seq * kXqRecord + kXZeroBytes + kXSelBytes;
-    B.part_z_floats = (uint64_t)Gm.nslots * B.n_seq * Gm.n_units * 16;
+    B.part_z_floats = mvqb_expert_part_floats(Gm.n_units, Gm.T, B.n_seq);
     if (B.part_z_floats * (B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1) <= B.part_floats) {
 #define LGH_MVQB2_CASE(M)                                                                         \
   case M:                                                                                         \

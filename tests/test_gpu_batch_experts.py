@@ -38,6 +38,22 @@ def test_experts_of_few_entries_are_bitwise_the_single_sequence(pkg, mix, hidden
     single.close()
 
 
+@pytest.mark.parametrize("mix,hidden,ff,slots", [("Q4_K_M", 2048, 2048, 2), ("Q8_0", 2048, 5632, 2), ("Q5_K_M", 2048, 5632, 7)])
+def test_experts_in_eight_slices_have_room_for_their_sums(pkg, mix, hidden, ff, slots):
+    """Experts whose gate | up is split into eight k-slices, and wider than half the hidden size: their partial sums are the most that a step holds (lgh_batch_create sizes the buffer, and launches its steps)."""
+    cfg = pkg.make_config("test-moe", max_seq_len=32, hidden_size=hidden, num_heads=hidden // 64, num_kv_heads=hidden // 128, num_layers=1, num_experts=8, expert_intermediate_size=ff)
+    multi = pkg.HipGpuInference.from_model(pkg.SynthModel(cfg, mix=mix), 32)
+    multi.batch_create(slots)
+    tok = np.random.default_rng(11).integers(0, cfg.vocab_size, (slots, 2))
+    got = [multi.forward_multi(list(range(slots)), tok[:, step])[0].copy() for step in range(2)]
+    for s in range(slots):
+        multi.reset()
+        for step in range(2):
+            want = multi.forward(int(tok[s, step]))
+            assert np.array_equal(got[step][s].view(np.uint32), want.view(np.uint32)), (s, step)
+    multi.close()
+
+
 _FRESH = """
 import sys
 sys.path.insert(0, sys.argv[1])
