@@ -1,0 +1,25 @@
+// Which kernels a mixture's experts take in a batched step: rules on sizes and formats alone, on the host (matvec_batch.hip, engine_batch.hip).
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace lgh {
+
+constexpr uint32_t kFewWaves = 4, kFewEntries = 2;   // mvqb_few's waves, and the entries of a turn over the weights
+// its LDS: the records of a turn's entries for T k-slices of nbw blocks (an own copy for each wave that shares a slice), their sums, the norms of n_seq sequences
+constexpr uint32_t few_red_at(uint32_t T, uint32_t nbw) { return (T > kFewWaves ? T : kFewWaves) * nbw * kFewEntries * 1280; }
+constexpr uint32_t few_ssq_at(uint32_t T, uint32_t nbw) { return few_red_at(T, nbw) + kFewEntries * 128 * T * 4; }
+constexpr size_t few_lds(uint32_t T, uint32_t nbw, uint32_t n_seq) { return few_ssq_at(T, nbw) + n_seq * 8 * 4; }
+
+// Quarters of an entry that an expert may have on average for gate | up to go to mvqb_few, by how many of its workgroups a CU holds.  Steps of two layers of 8 experts, two a sequence (so n sequences are n quarters), what mvqb2
+// takes over what mvqb_few takes, 4 / 6 / 8 sequences:
+//   three (hidden up to 4096; 4096 x 14336)  Q4_K 1.16 1.15 1.08, Q5_K 1.12 1.13 1.06, Q6_K 1.10 1.08 1.02, Q8_0 1.04 1.01 0.94 (2048 x 10240: 1.14 1.09 1.02)
+//   two (6144 x 16384)                       Q4_K 1.10 1.08 1.04, Q5_K 1.08 1.05 1.03, Q6_K 1.05 1.03 0.98, Q8_0 0.98 0.95 0.91 (3: 1.04)
+//   one (8192 x 14336)                       Q4_K 0.98 0.97 0.91, Q6_K 0.98 0.96 0.90; 6656 x 10240 (26 blocks in slices of four: the last has none): Q4_K 0.94 0.91 0.85, Q6_K 0.93 0.90 0.83, 2 sequences 0.98 0.97
+constexpr uint32_t few_quarters(bool q6k, bool q80, size_t lds) {
+  const size_t wgs = 160 * 1024 / lds;
+  return wgs >= 3 ? (q80 ? 5 : 8) : wgs == 2 ? (q80 ? 3 : q6k ? 6 : 8) : 0;
+}
+
+}  // namespace lgh

@@ -23,6 +23,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "batch_rules.h"
 #include "device_utils.h"
 #include "xq.h"
 #include "mvq_core.h"
@@ -1003,8 +1004,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t w
 // down stays with mvqb2 too: its slices are a grid dimension, so that it has bytes enough under way (Q6_K 51 us as the same stream 50, Q8_0 57 and 58).
 // ------------------------------------------------------------------------------------------------
 constexpr int few_depth(int f) { return f == F_Q4K ? 4 : f == F_Q6K ? 2 : 3; }   // tiles a wave has under way: what the registers of three waves a SIMD hold
-constexpr uint32_t kFewWaves = 4;
-struct MvqbFew { uint32_t T, nbw, nblk, max_sq, red_at, ssq_at; };
+struct MvqbFew { uint32_t T, nbw, nblk; };
 
 template <int F, int SQ>
 __device__ __forceinline__ void mvqb_few_turn(const MvqbFew& Gm, const MvLaunch& L, const MvBatch& B, uint8_t* smem8, uint32_t ez, const int* ind_idx, uint32_t s0, uint32_t n_seq) {
@@ -1022,7 +1022,7 @@ __device__ __forceinline__ void mvqb_few_turn(const MvqbFew& Gm, const MvLaunch&
   const uint8_t* const plane1 = S.pass[1].plane[0] + (uint64_t)ez * S.pass[1].sel_stride[0];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem8;
   const uint32_t wrecs = SL * Gm.nbw, wreg = wave * wrecs * SQ * (uint32_t)kXqRecord;
-  float* const red = reinterpret_cast<float*>(smem8 + Gm.red_at);
+  float* const red = reinterpret_cast<float*>(smem8 + few_red_at(Gm.T, Gm.nbw));
   const uint32_t red_floats = kFuseRed * Gm.T;             // a sequence's, [pass][slice][row]
   auto store = [&](uint32_t i, uint32_t ks, int s, float t) __attribute__((always_inline)) {
     const uint32_t w = unit0 + i;
@@ -1140,16 +1140,16 @@ __global__ void __launch_bounds__(kFewWaves * 64, 3) mvqb_few_kernel(const MvqbF
   n_seq = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(n_seq, B.n_seq));
   if (n_seq == 0) return;
   const int* ind_idx = B.ind_idx + (size_t)ez * B.ind_stride;
-  float* const ssq = reinterpret_cast<float*>(smem8 + Gm.ssq_at);
+  float* const ssq = reinterpret_cast<float*>(smem8 + few_ssq_at(Gm.T, Gm.nbw));
   if (L.do_norm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
-  for (uint32_t s0 = 0; s0 < n_seq; s0 += Gm.max_sq) {
-    const uint32_t left = n_seq - s0, now = left < Gm.max_sq ? left : Gm.max_sq;
+  for (uint32_t s0 = 0; s0 < n_seq; s0 += kFewEntries) {
+    const uint32_t left = n_seq - s0, now = left < kFewEntries ? left : kFewEntries;
     if (now == 1) mvqb_few_turn<F, 1>(Gm, L, B, smem8, ez, ind_idx, s0, now);
     else mvqb_few_turn<F, 2>(Gm, L, B, smem8, ez, ind_idx, s0, now);
     // SwiGLU as mv_epilogue_view has it: a thread a row and entry
     constexpr uint32_t rows = kFuseRed / 2;
     const MvSeg& S = L.seg[0];
-    const float* red = reinterpret_cast<const float*>(smem8 + Gm.red_at);
+    const float* red = reinterpret_cast<const float*>(smem8 + few_red_at(Gm.T, Gm.nbw));
     const uint32_t s = threadIdx.x / rows, rl = threadIdx.x % rows, row = blockIdx.x * rows + rl;
     __syncthreads();
     if (s < now && row < S.n_rows) {
@@ -1262,25 +1262,19 @@ static bool mvqb2_epilogue_few(const MvLaunch& L, const MvBatch& B, const Mvqb2G
   return true;
 }
 
-// gate | up of a layer's experts with few entries each: two on average at most; of Q8_0, where the second read costs most, 1.25 (steps of two layers, us, mvqb2 / mvqb_few, 8 experts, two a sequence: Q4_K_M 4 sequences
-// 482 / 410, 8: 676 / 622; Q5_K_M 5: 609 / 535, 8: 715 / 688, 10: 825 / 808, 12: 851 / 894; Q6_K 7: 681 / 663, 10: 800 / 867; Q8_0 5: 644 / 617, 6: 671 / 689).  mvqb2 where the format is Q4_0.
-static bool mvqb_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, int f, bool seq, MvqbFew* few, size_t* lds) {
+// gate | up of a layer's experts with few entries each (few_quarters).  mvqb2 where the format is Q4_0.
+static bool mvqb_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, int f, bool seq) {
   if (f == F_Q40 || !seq || Gm.fuse != 2 || !B.ind_cnt || B.ind_nz < 2 || L.nseg != 1 || L.seg[0].epi != EPI_SWIGLU || L.seg[0].bias || Gm.T > kBWaves || kBWaves % Gm.T) return false;
-  if (4 * B.n_seq * B.ind_div > (f == F_Q80 ? 5 : 8) * B.ind_nz) return false;
-  for (uint32_t sq = 2; sq >= 1; sq--) {
-    *few = MvqbFew{Gm.T, Gm.nbw, Gm.nblk, sq, std::max(Gm.T, kFewWaves) * Gm.nbw * sq * (uint32_t)kXqRecord, 0};
-    few->ssq_at = few->red_at + sq * kFuseRed * Gm.T * 4;
-    *lds = few->ssq_at + mvqb_fuse_lds(B.n_seq);
-    if (*lds <= 160 * 1024) return true;
-  }
-  return false;
+  return 4 * B.n_seq * B.ind_div <= few_quarters(f == F_Q6K, f == F_Q80, few_lds(Gm.T, Gm.nbw, B.n_seq)) * B.ind_nz;
 }
 
 template <int F>
-static hipError_t mvqb_few_go(const MvLaunch& L, const MvBatch& B, const MvqbFew& few, size_t lds, uint32_t groups, hipStream_t st) {
+static hipError_t mvqb_few_go(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, uint32_t groups, hipStream_t st) {
+  static_assert(kXqRecord == 1280 && kFuseRed == 128 && mvqb_fuse_lds(1) == 32, "as few_lds counts");
   static bool attr_set[64] = {};
+  const MvqbFew few{Gm.T, Gm.nbw, Gm.nblk};
   if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvqb_few_kernel<F>), 160 * 1024, attr_set); e != hipSuccess) return e;
-  hipLaunchKernelGGL(mvqb_few_kernel<F>, dim3(groups, 1, B.ind_nz), dim3(kFewWaves * 64), lds, st, few, L, B);
+  hipLaunchKernelGGL(mvqb_few_kernel<F>, dim3(groups, 1, B.ind_nz), dim3(kFewWaves * 64), few_lds(Gm.T, Gm.nbw, B.n_seq), st, few, L, B);
   return hipGetLastError();
 }
 
@@ -1292,9 +1286,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   Gm.ssq_at = (uint32_t)lds_x;
   lds_x += mvqb_fuse_lds(B.n_seq);
   if constexpr ((MASK & (MASK - 1)) == 0 && MASK != 1u << F_Q40) {
-    MvqbFew few;
-    size_t lds_few;
-    if (mvqb_few(L, B, Gm, __builtin_ctz(MASK), seq, &few, &lds_few)) return mvqb_few_go<__builtin_ctz(MASK)>(L, B, few, lds_few, groups, st);
+    if (mvqb_few(L, B, Gm, __builtin_ctz(MASK), seq)) return mvqb_few_go<__builtin_ctz(MASK)>(L, B, Gm, groups, st);
   }
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
