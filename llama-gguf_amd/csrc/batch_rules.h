@@ -22,4 +22,11 @@ constexpr uint32_t few_quarters(bool q6k, bool q80, size_t lds) {
   return wgs >= 3 ? (q80 ? 5 : 8) : wgs == 2 ? (q80 ? 3 : q6k ? 6 : 8) : 0;
 }
 
+// Two sequences by expert (seven launches a layer, every selected expert read once) or one after the other (three launches each).  A step of two layers, us, one after the other / by expert, Q4_K_M (Q8_0):
+//   where mvqb_few takes gate | up  4096 x 14336 324 / 298 (408 / 370), 4096 x 10240 281 / 269, 2048 x 10240 222 / 199, 6144 x 16384 459 / 431
+//   in Q4_0                         4096 x 14336 306 / 258, 8192 x 14336 477 / 409, 6656 x 10240 368 / 342, 4096 x 8192 246 / 249
+//   small experts                   2048 x 1024 179 / 160 (183 / 163), 1024 x 2048 171 / 152, 512 x 1024 162 / 138, 2048 x 2048 180 / 176 (185 / 184)
+//   the others                      2048 x 4096 189 / 204 (199 / 215), 2048 x 5632 200 / 221, 4096 x 4096 222 / 250, 4096 x 8192 262 / 304, 6656 x 10240 395 / 408, 8192 x 14336 509 / 545
+constexpr bool two_by_expert(bool few, bool q40, uint32_t hidden, uint32_t ff) { return few || q40 || (uint64_t)hidden * ff <= 2048u * 2048u; }
+
 }  // namespace lgh

@@ -6,7 +6,7 @@
 // SLOTS — a slot = one sequence's KV caches + position — and lgh_forward_multi feeds one token to each listed slot in ONE pass
 // over the weights: every quantized mat-vec launch reads its tiles once and multiplies them with all n_seq input vectors
 // (matvec_batch.hip), attention / its merge / embedding / arg-max run with the sequence as the grid's second dimension (over f32 or
-// TurboQuant slots); MoE layers route every sequence to its own experts: from 2 sequences on (moe_group_min) the step's (sequence,
+// TurboQuant slots); MoE layers route every sequence to its own experts: from 2 or 3 sequences on (moe_by_expert) the step's (sequence,
 // slot) pairs are grouped by expert and each selected expert is read once — all experts of a layer in one gate | up and one down
 // launch, the expert as the grid's third dimension — below that the FFN runs sequence by sequence.  Every sequence's logits are
 // bit-identical to what lgh_forward of the same context computes for the same tokens (tests/test_gpu_batch.py, test_gpu_batch_same_context.py): same
@@ -15,6 +15,7 @@
 // A step is a constant hipGraph per n_seq: tokens, positions and slot numbers live in device words (d_tokens / d_pos /
 // d_slot), the arg-max feeds the next token back on the device and `batch_advance` moves the positions, so
 // lgh_decode_greedy_multi replays the graph with no host work in between.
+#include "batch_rules.h"
 #include "engine.h"
 #include "xq.h"
 
@@ -86,14 +87,20 @@ void spread_state(lgh_ctx* c, const float* f32, uint32_t k, uint32_t n) {
 // one batched quantized mat-vec launch: `specs` name sequence 0's vectors
 struct MvIndirect { const int* cnt = nullptr; const int* idx = nullptr; uint32_t div = 0, nz = 0, stride = 0; };
 
-// MoE layers: from how many sequences on a step reads every selected expert ONCE (one router launch, a grouping launch, gate | up
-// and down over all experts with the expert as the grid's third dimension + their epilogue launches, one combine: 7 per layer
-// whatever the step's size) instead of running the FFN sequence by sequence (3 launches per sequence).  Measured on Mixtral-8x7B's
-// widths, a step of two layers, us, sequence by sequence vs grouped: 2 sequences Q4_K_M 326 / 302, Q5_K_M 351 / 324, Q6_K 364 / 339,
-// Q8_0 410 / 381, Q4_0 305 / 269; the whole model in Q5_K_M, tokens/s, 8: 468 / 764, 16: 480 / 1 030 (profiles/r03e_batched_decode.md).
-uint32_t moe_group_min() {
-  static const uint32_t v = [] { const char* e = std::getenv("LGH_MOE_GROUP_MIN"); return e ? (uint32_t)std::max(2, std::atoi(e)) : 2u; }();
-  return v;
+// MoE layers: whether a step reads every selected expert ONCE (one router launch, a grouping launch, gate | up and down over all
+// experts with the expert as the grid's third dimension + their epilogue launches, one combine: 7 per layer whatever the step's
+// size) instead of running the FFN sequence by sequence (3 launches per sequence).  From three sequences on (the whole Mixtral-8x7B
+// in Q5_K_M, tokens/s, sequence by sequence vs grouped, 8: 468 / 764, 16: 480 / 1 030: profiles/r03e_batched_decode.md), or from
+// LGH_MOE_GROUP_MIN on where that is set; two sequences by two_by_expert.
+bool moe_by_expert(const lgh_ctx* c, const LayerW& L, uint32_t n_seq) {
+  static const uint32_t set = [] { const char* e = std::getenv("LGH_MOE_GROUP_MIN"); return e ? (uint32_t)std::max(2, std::atoi(e)) : 0u; }();
+  if (!c->batch.moe_act || n_seq < 2) return false;
+  if (set || n_seq > 2) return n_seq >= (set ? set : 3u);
+  const lgh_model_desc& d = c->d;
+  const uint32_t H = L.gate_exps.k, F = L.gate_exps.n;
+  MvPlan p;
+  if (mvq_plan(H, F, 2, &p, F) != hipSuccess) return false;
+  return two_by_expert(mvqb_few_takes(L.gate_exps.type, p.T, p.units, 2 * ((F + 15) / 16), n_seq, d.num_experts_per_token, d.num_experts), L.gate_exps.type == kDevQ40_T16, H, F);
 }
 
 int launch_mvb(lgh_ctx* c, int cls, const SegSpec* specs, int nseg, const float* norm_w, uint32_t k, uint32_t n_seq, const uint32_t* out_stride,
@@ -328,7 +335,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
         if ((rc = launch_mvb(c, LGH_K_DOWN, &sp, 1, nullptr, Lw.down.k, n_seq, os, rs, xk, MvIndirect{}, wide_hidden(li + 1)))) return rc;
         spread_state(c, Bs.hidden, H, n_seq);
       }
-    } else if (Bs.moe_act && n_seq >= moe_group_min()) {
+    } else if (moe_by_expert(c, Lw, n_seq)) {
       // ---- MoE, every selected expert's matrices read ONCE for the step (MoeLayer::forward per sequence, moe.rs:321-413, regrouped):
       // router -> the (sequence, slot) pairs grouped by expert -> a gate|up launch, every expert over its pairs (SwiGLU, activation
       // + XQ image per pair), and a down launch (output per pair) -> h += sum_p w_p * down_p in selection order

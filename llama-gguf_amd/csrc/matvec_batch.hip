@@ -1262,10 +1262,23 @@ static bool mvqb2_epilogue_few(const MvLaunch& L, const MvBatch& B, const Mvqb2G
   return true;
 }
 
+// enough units to fill the chip with whole rows per workgroup; with fewer the k-slices are a grid dimension
+static bool mvqb2_whole_rows(uint32_t n_units, uint32_t T) {
+  static const uint32_t min_groups = [] { const char* e = std::getenv("LGH_MVQB2_SEQ_GROUPS"); return e ? (uint32_t)std::atoi(e) : 160u; }();
+  return (n_units + kBWaves - 1) / kBWaves >= min_groups || T == 1;
+}
+
+// partial sums of one expert in a launch over a layer's experts: matrices of n_units row tiles in T k-slices
+uint64_t mvqb_expert_part_floats(uint32_t n_units, uint32_t T, uint32_t n_seq) { return (uint64_t)(mvqb2_whole_rows(n_units, T) ? 1 : T) * n_seq * n_units * 16; }
+
 // gate | up of a layer's experts with few entries each (few_quarters).  mvqb2 where the format is Q4_0.
-static bool mvqb_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, int f, bool seq) {
-  if (f == F_Q40 || !seq || Gm.fuse != 2 || !B.ind_cnt || B.ind_nz < 2 || L.nseg != 1 || L.seg[0].epi != EPI_SWIGLU || L.seg[0].bias || Gm.T > kBWaves || kBWaves % Gm.T) return false;
-  return 4 * B.n_seq * B.ind_div <= few_quarters(f == F_Q6K, f == F_Q80, few_lds(Gm.T, Gm.nbw, B.n_seq)) * B.ind_nz;
+bool mvqb_few_takes(int dev_type, uint32_t T, uint32_t nbw, uint32_t n_units, uint32_t n_seq, uint32_t top_k, uint32_t n_experts) {
+  const int f = fmt_of_dev_type(dev_type);
+  if (f < 0 || f == F_Q40 || !mvqb2_whole_rows(n_units, T) || n_experts < 2 || T > kBWaves || kBWaves % T) return false;
+  return 4 * n_seq * top_k <= few_quarters(f == F_Q6K, f == F_Q80, few_lds(T, nbw, n_seq)) * n_experts;
+}
+static bool mvqb_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm) {
+  return Gm.fuse == 2 && B.ind_cnt && B.ind_nz >= 2 && L.nseg == 1 && L.seg[0].epi == EPI_SWIGLU && !L.seg[0].bias && mvqb_few_takes(L.seg[0].type, Gm.T, Gm.nbw, Gm.n_units, B.n_seq, B.ind_div, B.ind_nz);
 }
 
 template <int F>
@@ -1286,7 +1299,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   Gm.ssq_at = (uint32_t)lds_x;
   lds_x += mvqb_fuse_lds(B.n_seq);
   if constexpr ((MASK & (MASK - 1)) == 0 && MASK != 1u << F_Q40) {
-    if (mvqb_few(L, B, Gm, __builtin_ctz(MASK), seq)) return mvqb_few_go<__builtin_ctz(MASK)>(L, B, Gm, groups, st);
+    if (mvqb_few(L, B, Gm)) return mvqb_few_go<__builtin_ctz(MASK)>(L, B, Gm, groups, st);
   }
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
@@ -1320,15 +1333,6 @@ static uint32_t mvqb2_min_seq() {
   }();
   return v;
 }
-
-// enough units to fill the chip with whole rows per workgroup; with fewer the k-slices are a grid dimension
-static bool mvqb2_whole_rows(uint32_t n_units, uint32_t T) {
-  static const uint32_t min_groups = [] { const char* e = std::getenv("LGH_MVQB2_SEQ_GROUPS"); return e ? (uint32_t)std::atoi(e) : 160u; }();
-  return (n_units + kBWaves - 1) / kBWaves >= min_groups || T == 1;
-}
-
-// partial sums of one expert in a launch over a layer's experts: matrices of n_units row tiles in T k-slices
-uint64_t mvqb_expert_part_floats(uint32_t n_units, uint32_t T, uint32_t n_seq) { return (uint64_t)(mvqb2_whole_rows(n_units, T) ? 1 : T) * n_seq * n_units * 16; }
 
 // `L` built like a single-sequence launch (engine.hip: build_mv_group, with the batch cap on tiles per workgroup); sequences'
 // vectors at the strides in `B`

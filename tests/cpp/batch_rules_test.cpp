@@ -18,5 +18,10 @@ int main() {
       CHECK(few_quarters(false, true, lds) == w.k8);
       CHECK(w.k45 == 0 || lds <= 160 * 1024);
     }
+  // two sequences: where mvqb_few takes gate | up, in Q4_0, and small experts; the others one after the other
+  CHECK(two_by_expert(true, false, 4096, 14336) && two_by_expert(false, true, 8192, 14336));
+  CHECK(two_by_expert(false, false, 2048, 1024) && two_by_expert(false, false, 2048, 2048));
+  const struct { uint32_t hidden, ff; } others[] = {{2048, 4096}, {2048, 5632}, {4096, 4096}, {8192, 14336}, {6656, 10240}};
+  for (const auto& o : others) CHECK(!two_by_expert(false, false, o.hidden, o.ff));
   return bad != 0;
 }
