@@ -207,6 +207,7 @@ uint32_t mvq_pack(const MvLaunch& L, uint32_t n_wg, uint32_t threads, MvGeom* g,
 uint32_t mvq_format_mask(const MvLaunch& L);
 uint32_t mvq_tile_bytes(int dev_type);   // bytes of one 16-row x 256-element tile in the device layout of this type (0: not a tile16 type)
 bool mvqb_few_takes(int dev_type, uint32_t T, uint32_t nbw, uint32_t n_units, uint32_t n_seq, uint32_t top_k, uint32_t n_experts);
+uint32_t mvqb2_min_seq();
 uint64_t mvqb_expert_part_floats(uint32_t n_units, uint32_t T, uint32_t n_seq);
 hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& B, uint32_t n_wg, uint32_t threads, hipStream_t st);   // matvec_batch.hip
 size_t mvqb_lds_bytes(uint32_t n_seq, uint32_t red_floats);

@@ -94,7 +94,7 @@ struct MvIndirect { const int* cnt = nullptr; const int* idx = nullptr; uint32_t
 // LGH_MOE_GROUP_MIN on where that is set; two sequences by two_by_expert.
 bool moe_by_expert(const lgh_ctx* c, const LayerW& L, uint32_t n_seq) {
   static const uint32_t set = [] { const char* e = std::getenv("LGH_MOE_GROUP_MIN"); return e ? (uint32_t)std::max(2, std::atoi(e)) : 0u; }();
-  if (!c->batch.moe_act || n_seq < 2) return false;
+  if (!c->batch.moe_act || n_seq < std::max(2u, mvqb2_min_seq())) return false;   // (entry lists exist in the kernels behind LGH_MVQB2_MIN only)
   if (set || n_seq > 2) return n_seq >= (set ? set : 3u);
   const lgh_model_desc& d = c->d;
   const uint32_t H = L.gate_exps.k, F = L.gate_exps.n;

@@ -1325,8 +1325,8 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   return mvqb2_epilogue_few(L, B, Gm) ? epilogue(&mvqb2_epilogue_kernel<true>, attr_set[2]) : epilogue(&mvqb2_epilogue_kernel<false>, attr_set[3]);
 }
 
-// 0: the records-through-LDS structure (mvqb2) from LGH_MVQB2_MIN sequences on (default: measured crossover), 1: never, 2: always
-static uint32_t mvqb2_min_seq() {
+// from how many sequences on the records go through LDS (mvqb2 and the kernels beside it)
+uint32_t mvqb2_min_seq() {
   static const uint32_t v = [] {
     const char* e = std::getenv("LGH_MVQB2_MIN");
     return e ? (uint32_t)std::atoi(e) : 2u;

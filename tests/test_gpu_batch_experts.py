@@ -2,6 +2,10 @@
 workgroup with half its tiles, experts of one entry, two, and more (another turn), and the sequences from which mvqb2 takes over.
 
 Per (row, entry) the kernel does the single-sequence kernel's operations in its order, so the bound is equality of all bits with a single-sequence engine that runs the split attention too (attn_direct=255)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -60,7 +64,7 @@ sys.path.insert(0, sys.argv[1])
 import numpy as np
 import __graft_entry__ as graft
 pkg = graft.load_package()
-cfg = pkg.make_config("test-moe", max_seq_len=32, num_layers=1, num_experts=int(sys.argv[3]), expert_intermediate_size=10240)
+cfg = pkg.make_config("test-moe", max_seq_len=32, num_layers=1, num_experts=int(sys.argv[3]), expert_intermediate_size=int(sys.argv[6]))
 multi = pkg.HipGpuInference.from_model(pkg.SynthModel(cfg, mix=sys.argv[2]), 32)
 slots, n = int(sys.argv[4]), int(sys.argv[5])
 multi.batch_create(slots)
@@ -75,13 +79,20 @@ print("equal")
 """
 
 
+def _in_fresh_process(mix, experts, slots, n, ff, **env):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", _FRESH, root, mix, str(experts), str(slots), str(n), str(ff)], capture_output=True, text=True, timeout=100, env=dict(os.environ, **env))
+    assert out.returncode == 0 and out.stdout.strip().endswith("equal"), out.stdout + out.stderr
+
+
 @pytest.mark.parametrize("mix,experts,slots,n", [("Q8_0", 8, 8, 7), ("Q5_K_M", 5, 7, 7)])
 def test_first_step_of_a_size_in_a_fresh_process(mix, experts, slots, n):
     """A kernel whose first launch in the process happens during a capture is not replayed with the graph: the sizes from which mvqb2 takes over lie inside its groups of up to 4, 8 and 16, so lgh_batch_create launches
     the largest of each group as well."""
-    import os
-    import subprocess
-    import sys
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    out = subprocess.run([sys.executable, "-c", _FRESH, root, mix, str(experts), str(slots), str(n)], capture_output=True, text=True, timeout=100)
-    assert out.returncode == 0 and out.stdout.strip().endswith("equal"), out.stdout + out.stderr
+    _in_fresh_process(mix, experts, slots, n, 10240)
+
+
+@pytest.mark.parametrize("least,slots,n", [(3, 2, 2), (5, 4, 4)])
+def test_fewer_sequences_than_the_kernels_with_entry_lists_take(least, slots, n):
+    """LGH_MVQB2_MIN keeps smaller steps from the kernels that take entry lists: a mixture's sequences go one after the other there."""
+    _in_fresh_process("Q5_K_M", 4, slots, n, 1024, LGH_MVQB2_MIN=str(least))
