@@ -1044,7 +1044,7 @@ __device__ __forceinline__ void mvqb_few_turn(const MvqbFew& Gm, const MvLaunch&
     const uint8_t* src = S.pass[0].xq + (size_t)(v / B.ind_div) * B.xq_stride + (size_t)blk0 * kXqRecord;
     for (uint32_t b = 0; b < nblk_w; b++, src += kXqRecord)
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-                   : : "v"(src + lane * 16), "v"(src + 1024 + lane * 4), "s"(__builtin_amdgcn_readfirstlane((int)(lds0 + wreg + (s * wrecs + b) * (uint32_t)kXqRecord))) : "memory", "m0");
+                   : : "v"(src + lane * 16), "v"(src + 1024 + lane * 4), "s"(__builtin_amdgcn_readfirstlane((int)(lds0 + wreg + (s * wrecs + b) * (uint32_t)kXqRecord))) : "memory", "m0", "scc");
   }
   // items in order: unit, then block
   uint32_t ni = 0, nb = 0;   // the next to request
