@@ -1,4 +1,4 @@
-// Which kernels a mixture's experts take in a batched step: rules on sizes and formats alone, on the host (matvec_batch.hip, engine_batch.hip).
+// Which kernels take a call: rules on sizes and formats alone, on the host.
 #pragma once
 
 #include <cstddef>
@@ -6,6 +6,21 @@
 
 namespace lgh {
 
+// ---- prompt blocks of up to 128 tokens (prefill.hip)
+// k-ranges of a product of `wgs` workgroups over nblk blocks of 256 columns: as many as keep the launch within `fill` workgroups, none of them empty
+constexpr uint32_t pf_ranges(uint32_t wgs, uint32_t fill, uint32_t nblk) {
+  uint32_t S = wgs >= fill ? 1 : fill / wgs;
+  if (S > nblk) S = nblk;
+  const uint32_t per = (nblk + S - 1) / S;
+  return (nblk + per - 1) / per;
+}
+// gate | up of S k-ranges as one product without partial sums: while walking all of k costs its workgroups no more than the fold and its launch.  A block is 0.8 us, the fold about 5.  In ranges and in one, six layers, us:
+// 4096 x 4096 (ranges of 4 of 16 blocks), 50 / 90 / 128 tokens 372 / 446 / 539 and 403 / 479 / 548; 2048 x 5632 (4 of 8) 335 / 390 / 445 and 329 / 378 / 431; 1024 x 2816 (1 of 4) 268 / 308 / 344 and 257 / 294 / 328.
+// Seven blocks more (2048 columns, up to 2048 x 2048) are even on the device with up to 64 tokens and lose with more (2048 x 768, 20 / 64 / 96 / 128 tokens 253 / 292 / 329 / 364 and 240 / 300 / 342 / 384).  But there
+// the host's launches are what a prompt with its last token's step beside it waits for, so one launch a layer less is the faster way up to 64.
+constexpr bool pf_pair_pays(uint32_t nblk, uint32_t S, uint32_t m_tokens) { return nblk - (nblk + S - 1) / S <= (m_tokens <= 64 ? 7u : 6u); }
+
+// ---- a mixture's experts in a batched step (matvec_batch.hip, engine_batch.hip)
 constexpr uint32_t kFewWaves = 4, kFewEntries = 2;   // mvqb_few's waves, and the entries of a turn over the weights
 // its LDS: the records of a turn's entries for T k-slices of nbw blocks (an own copy for each wave that shares a slice), their sums, the norms of n_seq sequences
 constexpr uint32_t few_red_at(uint32_t T, uint32_t nbw) { return (T > kFewWaves ? T : kFewWaves) * nbw * kFewEntries * 1280; }

@@ -1175,7 +1175,7 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail*
     uint8_t* next_xh = next_nw ? P.xh_h : nullptr;
     if (!L.moe()) {
       const DevWeight* gu[2] = {&L.gate, &L.up};
-      if (pf_pairs(&L.gate, &L.up)) {
+      if (pf_pairs(&L.gate, &L.up, m)) {
         if ((rc = K(pf_pair_launch(&L.gate, &L.up, P.xh_h, P.xh_act, P.ssq, H, d.norm_eps, m, st), "gate | up product"))) return rc;
       } else {
         if ((rc = K(pf_gemm_launch(gu, 2, P.xh_h, P.part, P.part_bytes, m, &S, &nc, st), "gate/up GEMM"))) return rc;

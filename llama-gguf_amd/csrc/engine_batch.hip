@@ -15,7 +15,7 @@
 // A step is a constant hipGraph per n_seq: tokens, positions and slot numbers live in device words (d_tokens / d_pos /
 // d_slot), the arg-max feeds the next token back on the device and `batch_advance` moves the positions, so
 // lgh_decode_greedy_multi replays the graph with no host work in between.
-#include "batch_rules.h"
+#include "dispatch_rules.h"
 #include "engine.h"
 #include "xq.h"
 

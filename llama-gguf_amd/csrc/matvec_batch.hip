@@ -23,7 +23,7 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "batch_rules.h"
+#include "dispatch_rules.h"
 #include "device_utils.h"
 #include "xq.h"
 #include "mvq_core.h"

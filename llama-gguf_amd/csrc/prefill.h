@@ -48,7 +48,7 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
                           uint32_t* S_out, uint32_t* ncols_out, hipStream_t st, uint32_t n_experts = 0, size_t xh_z = 0, const int* m_count = nullptr,
                           uint32_t part_rows = kPfTokens, const int* row_base = nullptr);
 // silu(gate) * up of one launch -> XH
-bool pf_pairs(const DevWeight* gate, const DevWeight* up);
+bool pf_pairs(const DevWeight* gate, const DevWeight* up, uint32_t m_tokens);
 hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint8_t* xh, uint8_t* act, const float* ssq, uint32_t norm_cols, float eps, uint32_t m_tokens, hipStream_t st);
 hipError_t pf_row_epi_launch(const float* part, uint32_t S, uint32_t ncols, uint32_t col0, const float* bias, float* hidden, uint32_t H,
                              const float* nw, uint8_t* xh, float* ssq, uint32_t m_tokens, hipStream_t st, const float* moe_w = nullptr);

@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "device_utils.h"
+#include "dispatch_rules.h"
 #include "mv_epilogue.h"
 #include "prefill.h"
 #include "prefill_dequant.h"
@@ -604,10 +605,7 @@ static void pf_plan(const uint32_t* n_rows, int nw, uint32_t k, uint32_t n_exper
   uint32_t wgs = 0;
   for (int i = 0; i < nw; i++) wgs += (n_rows[i] / 16 + wt - 1) / wt;
   if (n_experts) wgs *= n_experts;
-  uint32_t S = wgs >= fill ? 1 : fill / wgs;
-  if (S > nblk) S = nblk;
-  const uint32_t per = (nblk + S - 1) / S;
-  *S_out = (nblk + per - 1) / per;
+  *S_out = pf_ranges(wgs, fill, nblk);
 }
 
 // bytes of partial sums such a GEMM writes
@@ -673,14 +671,13 @@ hipError_t pf_gemm_launch(const DevWeight* const* W, int nw, const uint8_t* xh, 
 // chunks of per-token sums of squares a row of H elements is reduced to (pf_inv_rms adds them up)
 uint32_t pf_ssq_chunks(uint32_t H) { return (H + 2047) / 2048; }
 
-// gate | up as one product without partial sums while walking all of k costs its workgroups no more than the fold and its launch: a block is 0.8 us, the fold about 5.  In ranges and here, six layers, us:
-// 4096 x 4096 (ranges of 4 of 16 blocks), 50 / 90 / 128 tokens 372 / 446 / 539 and 403 / 479 / 548; 2048 x 5632 (4 of 8) 335 / 390 / 445 and 329 / 378 / 431; 1024 x 2816 (1 of 4) 268 / 308 / 344 and 257 / 294 / 328.
-bool pf_pairs(const DevWeight* gate, const DevWeight* up) {
+// gate | up as one product without partial sums (pf_pair_pays)
+bool pf_pairs(const DevWeight* gate, const DevWeight* up, uint32_t m_tokens) {
   if (!pf_supported_type(gate->type) || gate->type != up->type || gate->k != up->k || gate->n != up->n || gate->k % 256 || gate->n % 256) return false;
-  const uint32_t n_rows[2] = {gate->n, up->n}, nblk = gate->k / 256;
+  const uint32_t n_rows[2] = {gate->n, up->n};
   uint32_t S;
-  pf_plan(n_rows, 2, gate->k, false, &S);
-  return nblk - (nblk + S - 1) / S <= 6;
+  pf_plan(n_rows, 2, gate->k, 0, &S);
+  return pf_pair_pays(gate->k / 256, S, m_tokens);
 }
 
 template <int F>
@@ -696,7 +693,7 @@ static hipError_t pf_pair_go(const PfGemm& G, hipStream_t st) {
 }
 
 hipError_t pf_pair_launch(const DevWeight* gate, const DevWeight* up, const uint8_t* xh, uint8_t* act, const float* ssq, uint32_t norm_cols, float eps, uint32_t m_tokens, hipStream_t st) {
-  if (m_tokens == 0 || !pf_pairs(gate, up) || m_tokens > (uint32_t)kPfTokens || !act || !ssq) return hipErrorInvalidValue;
+  if (m_tokens == 0 || !pf_pairs(gate, up, m_tokens) || m_tokens > (uint32_t)kPfTokens || !act || !ssq) return hipErrorInvalidValue;
   PfGemm G{};
   for (int i = 0; i < 2; i++) {
     const DevWeight* W = i ? up : gate;
