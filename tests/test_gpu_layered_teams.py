@@ -24,14 +24,18 @@ def test_one_tile_a_cu(pkg, gpu, width, vocab, tokens):
     eng.close()
 
 
-def test_tiles_of_160(pkg, gpu):
-    """Where two workgroups a CU would take two rounds of tiles of 128 and take one of 160: the joint input product (32 896 columns, 257 panels) and the gated feed-forward's first (33 200 columns,
-    260 panels); whole and ragged ends, and one token beyond a tile."""
-    cfg = lc.config([lc.mem(heads=64, dim=128, vdim=128, ff=16600)], width=1024, vocab=300)
-    eng, W = lc.make(pkg, cfg, "bf16", max_seq=200)
-    toks = lc.tokens(161, cfg["vocab"])
+@pytest.mark.parametrize("heads,ff,tokens", [
+    (64, 16600, (129, 145, 160)),          # 257 and 260 panels, two tiles of 128 and one of 160
+    (50, 12800, (257, 289, 301, 319, 320)),   # 201 and 200 panels, three of 128 and two of 160
+])
+def test_tiles_of_160(pkg, gpu, heads, ff, tokens):
+    """Where two workgroups a CU would take two rounds of tiles of 128 and take one of 160: the joint input product (4 x 128 columns a head and the gates) and the gated feed-forward's first (two columns a unit);
+    whole and ragged last tiles, alone and behind a full one."""
+    cfg = lc.config([lc.mem(heads=heads, dim=128, vdim=128, ff=ff)], width=1024, vocab=300)
+    eng, W = lc.make(pkg, cfg, "bf16", max_seq=360)
+    toks = lc.tokens(tokens[-1], cfg["vocab"])
     want = lo.forward(cfg, W, toks)
-    for n in (129, 145, 160, 161):
+    for n in tokens:
         eng.reset()
         lc.check(eng.eval(toks[:n], range(n)), want[:n], "bf16", f"{n} tokens")
     eng.close()

@@ -1,7 +1,9 @@
-"""A mixture's experts in a prompt block of up to 128 tokens, all of a layer in one launch (prefill.hip): experts of one token tile, of several and of full blocks (pf_gemm_kernel: two experts, both of every token), experts
-nobody chose, one expert a token, k in one range and in several, against the exact token-by-token path.
+"""A mixture's experts in a prompt block of up to 128 tokens, all of a layer in one launch (prefill.hip): experts of one token tile, of several and of full blocks (two experts, both of every token), experts
+nobody chose, one expert a token, k in ranges of one block, of several (gate | up of eight experts 8192 wide and of two 10240 wide, down in ranges of two and four) and with a last range that is shorter, in every format,
+against the exact token-by-token path.
 
 Tolerance as in test_gpu_prefill.py: operands of the blocks are rounded to f16."""
+import block_rows
 import numpy as np
 import pytest
 
@@ -32,3 +34,16 @@ def test_block_of_a_mixture_matches_token_by_token(pkg, mix, kw, sizes):
         assert np.abs(got - want).max() <= 1e-2 * np.abs(want).max() + 1e-2, (m, np.abs(got - want).max())
     exact.close()
     block.close()
+
+
+@pytest.mark.parametrize("mix,experts,top_k,hidden,ff,tokens", [
+    ("Q4_K_M", 2, 2, 2048, 10240, (33, 64, 97, 128)),     # gate | up in ranges of three, three and two blocks, full experts
+    ("Q8_0", 2, 2, 2048, 10240, (65, 128)),
+    ("Q5_K_M", 8, 2, 2048, 8192, (20, 100, 128)),         # in one of eight blocks; some experts of two token tiles, some of more
+    ("Q6_K", 8, 2, 2048, 8192, (128,)),
+    ("Q4_0", 8, 2, 2048, 8192, (128,)),
+    ("Q5_K_M", 8, 2, 512, 2048, (16, 128)),               # one block a range
+])
+def test_rows_behind_a_block(pkg, mix, experts, top_k, hidden, ff, tokens):
+    kw = dict(num_experts=experts, num_experts_per_token=top_k, hidden_size=hidden, expert_intermediate_size=ff, num_layers=2)
+    block_rows.check(pkg, pkg.SynthModel(pkg.make_config("test-moe", max_seq_len=160, **kw), mix=mix), tokens)
