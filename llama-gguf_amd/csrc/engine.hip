@@ -1188,19 +1188,19 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail*
     }
     // ---- MoE (moe.rs:321-413): route every token of the block (f32, the decode router), group the (token, slot) pairs by
     // expert, and run each expert once over its rows: gather -> gate|up GEMM -> SwiGLU -> down GEMM -> rows back to tokens
-    const uint32_t topk = d.num_experts_per_token, EI = L.gate_exps.n, rows_e = std::max(1u, m * topk / d.num_experts);   // (an expert's rows on average)
+    const uint32_t topk = d.num_experts_per_token, EI = L.gate_exps.n;
     if ((rc = K(moe_router_launch(P.hidden, L.ffn_norm, d.norm_eps, L.router, H, d.num_experts, topk, P.moe_sel, P.moe_w, st, m), "router"))) return rc;
     if ((rc = K(pf_moe_group_launch(P.moe_sel, m, topk, d.num_experts, P.moe_cnt, P.moe_base, P.moe_list, P.moe_rowmap, P.moe_tokmap, st), "expert grouping")))
       return rc;
     if ((rc = K(pf_moe_gather_launch(P.xh_h, H, P.moe_list, P.moe_cnt, P.xh_gather, d.num_experts, st), "expert gather"))) return rc;
     {   // every expert's gate|up over its rows, partial sums side by side in one row space
       const DevWeight* gu[2] = {&L.gate_exps, &L.up_exps};
-      if ((rc = K(pf_gemm_launch(gu, 2, P.xh_gather, P.part, P.part_bytes, rows_e, &S, &nc, st, d.num_experts, xh_bytes(H), P.moe_cnt, kPfMoeRows, P.moe_base), "experts' gate/up GEMM"))) return rc;
+      if ((rc = K(pf_gemm_launch(gu, 2, P.xh_gather, P.part, P.part_bytes, m, &S, &nc, st, d.num_experts, xh_bytes(H), P.moe_cnt, kPfMoeRows, P.moe_base), "experts' gate/up GEMM"))) return rc;
     }
     if ((rc = K(pf_moe_swiglu_launch(P.part, S, EI, P.xh_act_e, P.moe_rowmap, P.moe_list, P.ssq, H, d.norm_eps, st), "expert SwiGLU"))) return rc;
     {
       const DevWeight* dn[1] = {&L.down_exps};
-      if ((rc = K(pf_gemm_launch(dn, 1, P.xh_act_e, P.part, P.part_bytes, rows_e, &S, &nc, st, d.num_experts, xh_bytes(EI), P.moe_cnt, kPfMoeRows, P.moe_base), "experts' down GEMM"))) return rc;
+      if ((rc = K(pf_gemm_launch(dn, 1, P.xh_act_e, P.part, P.part_bytes, m, &S, &nc, st, d.num_experts, xh_bytes(EI), P.moe_cnt, kPfMoeRows, P.moe_base), "experts' down GEMM"))) return rc;
     }
     // h += sum over the selected experts, in selection order, of routing weight * expert output (moe.rs:363-368), then the
     // next layer's input

@@ -710,10 +710,9 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
   bool active = u < Gm.n_units;
   const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
   const MvSeg& S = L.seg[active ? sg : 0];
-  constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
-  const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
-  auto is = [&](int f) { return ((MASK >> f) & 1u) != 0 && (kSingle || fmt == f); };
-  const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K) : fmt_tile_bytes(F_Q40);
+  constexpr int fmt = __builtin_ctz(MASK);
+  auto is = [](int f) { return f == fmt; };
+  constexpr uint32_t tb = fmt_tile_bytes(fmt);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
   const uint32_t ul = u - (sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2);
   uint32_t pass, tl;

@@ -33,7 +33,7 @@ struct PfGemm {
   float* part;           // [S][part_rows][ncols]
   uint32_t part_rows;    // rows per split: 128, or kPfMoeRows when the experts of a MoE layer share one buffer
   const int* row_base;   // MoE: device words, the first row of each expert's batch in the buffer
-  uint32_t m_tokens;     // (MoE: of an expert, on average)
+  uint32_t m_tokens;     // (MoE: of the block; an expert's own: m_count)
   const int* m_count;    // MoE: device words, the number of each expert's real rows; 0 rows = nothing to do
   // gate | up with SwiGLU: the activations (XH), the input's sums of squares and the norm they stand for
   uint8_t* act;

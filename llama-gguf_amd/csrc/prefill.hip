@@ -71,8 +71,8 @@ hipError_t pf_read_stamps(unsigned long long* host, size_t n) {
 #define LGH_PF_STAMP(i)
 #endif
 
-// MT = token tiles computed: 8 for a full block, 4 / 2 when at most 64 / 32 rows are real (short prompts, and the rows routed
-// to one MoE expert — about 32 of 128 with 2-of-8 routing): the MFMAs, the LDS reads and the activation DMA shrink with it.
+// A mixture's experts.  MT = token tiles computed: 8 for a full block, 4 / 2 when at most 64 / 32 rows are routed to the expert
+// (about 32 of 128 with 2-of-8 routing): the MFMAs, the LDS reads and the activation DMA shrink with it.
 template <int F, int MT>
 __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32_t z, uint32_t rg, uint32_t ks, uint32_t m_tiles, uint8_t* smem) {
   constexpr uint32_t kBuf = (uint32_t)MT * 16 * 512;                // a slab's rows that are copied
@@ -218,10 +218,12 @@ __device__ __forceinline__ void pf_body(const PfGemm& G, const PfSeg& sg, uint32
   LGH_PF_STAMP(14);
 }
 
-// A mixture's experts, all of a layer in one launch (blockIdx.z; a launch each, gate | up and down, was 16 launches of a third of the chip's rate: 8 experts of 14336 x 4096 in Q5_K, 64 tokens, 370 -> 288 us with the sums'
-// fold; one block of weights under way a wave, 3.5 TB/s).  The token tiles are chosen here;  FIXED: experts of full blocks
-template <uint32_t MASK, bool FIXED>
-__device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem) {
+// All experts of a layer in one launch (blockIdx.z; a launch each, gate | up and down, was 16 launches of a third of the chip's rate: 8 experts of 14336 x 4096 in Q5_K, 64 tokens, 370 -> 288 us with the sums' fold; one block
+// of weights under way a wave, 3.5 TB/s).  The token tiles are chosen here: experts of full blocks alone, a kernel with eight tiles fixed and this one, two of two, two layers, 97 / 112 / 128 tokens: 4096 x 14336 in
+// Q4_K 254 / 253 / 263 and 253 / 254 / 264 us, in Q8_0 273 / 273 / 284 and 273 / 274 / 284.
+template <uint32_t MASK>
+__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
   const uint32_t rgid = blockIdx.x, z = blockIdx.z;
   int si = 0;
   if (G.nseg > 1 && rgid >= G.seg[1].rg_begin) si = 1;
@@ -233,11 +235,11 @@ __device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem
   asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cnt) : "s"(G.m_count + z) : "memory");
   if (cnt == 0) return;
   const uint32_t m_tiles = (cnt + 15) / 16;
-#define LGH_PF_RUN(F)                                                                              \
-  do {                                                                                             \
-    if (!FIXED && m_tiles <= 2) pf_body<F, 2>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);         \
-    else if (!FIXED && m_tiles <= 4) pf_body<F, 4>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);    \
-    else pf_body<F, kPfMT>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);                            \
+#define LGH_PF_RUN(F)                                                                    \
+  do {                                                                                   \
+    if (m_tiles <= 2) pf_body<F, 2>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);         \
+    else if (m_tiles <= 4) pf_body<F, 4>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);    \
+    else pf_body<F, kPfMT>(G, sg, z, rg, blockIdx.y, m_tiles, pf_smem);                  \
   } while (0)
   if (is(PF_Q4K)) LGH_PF_RUN(PF_Q4K);
   else if (is(PF_Q6K)) LGH_PF_RUN(PF_Q6K);
@@ -245,16 +247,6 @@ __device__ __forceinline__ void pf_gemm_device(const PfGemm& G, uint8_t* pf_smem
   else if (is(PF_Q80)) LGH_PF_RUN(PF_Q80);
   else if (is(PF_Q40)) LGH_PF_RUN(PF_Q40);
 #undef LGH_PF_RUN
-}
-template <uint32_t MASK>
-__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_kernel(const PfGemm G) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-  pf_gemm_device<MASK, true>(G, pf_smem);
-}
-template <uint32_t MASK, int MT>
-__global__ void __launch_bounds__(kPfWaves * 64) pf_gemm_few_kernel(const PfGemm G) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-  pf_gemm_device<MASK, MT != 0>(G, pf_smem);
 }
 
 // 1 / rms of token t from the per-chunk sums of squares its producer left (simd.rs:847-878); 1 when there is no norm
@@ -583,8 +575,7 @@ static hipError_t pf_gemm_run(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
 }
 template <uint32_t MASK>
 static hipError_t pf_gemm_go(const PfGemm& G, uint32_t n_rg, hipStream_t st) {
-  if (G.m_count && G.m_tokens > (uint32_t)kPfTokens * 3 / 4) return pf_gemm_run<&pf_gemm_kernel<MASK>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
-  if (G.m_count) return pf_gemm_run<&pf_gemm_few_kernel<MASK, 0>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
+  if (G.m_count) return pf_gemm_run<&pf_gemm_kernel<MASK>, 2 * (size_t)kPfSlabBytes, kPfWaves>(G, n_rg, st);
   switch ((G.m_tokens + 31) / 32) {
     case 1: return pf_gemm_run<&pf_rows_kernel<MASK, 1>, pf_half_lds(1), 2 * kPfWaves>(G, n_rg, st);
     case 2: return pf_gemm_run<&pf_rows_kernel<MASK, 2>, pf_half_lds(2), 2 * kPfWaves>(G, n_rg, st);

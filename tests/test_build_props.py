@@ -73,9 +73,13 @@ def test_long_prompt_kernels_use_no_scratch_and_keep_their_sums_in_registers():
                 assert u["VGPRs"] + u.get("AGPRs", 0) <= 256 and u.get("Occupancy", 2) >= 2, (fn, u)
 
 
-def test_prefill_gemm_of_a_mixtures_experts_keeps_its_accumulators_in_registers():
-    """The experts' kernels (pf_gemm_few_kernel<..., 0>) choose the number of token tiles on the device: up to the 128 accumulators of a full block."""
-    gemm = {fn: u for fn, u in _usage("prefill.hip").items() if "pf_gemm_few_kernel" in fn and "ELi0E" in fn}
-    assert len(gemm) == 8
-    for fn, u in gemm.items():
-        assert u.get("AGPRs", 0) >= 128 and u["VGPRs"] <= 256, (fn, u)
+def test_dense_block_products_keep_their_accumulators_in_registers():
+    """Dense layers' products of a prompt block (pf_rows_kernel, pf_pair_kernel, pf_pair_few_kernel): 16 f32 accumulators a lane and tile of 32 tokens, two waves a SIMD."""
+    usage = _usage("prefill.hip")
+    for pattern, count in ((r"pf_rows_kernelILj\d+ELi(\d)E", 8 * 4), (r"pf_pair_kernelILi\d+ELi(\d)E", 5 * 4), (r"pf_pair_few_kernelILi(\d)E", 5)):
+        found = {fn: (re.search(pattern, fn), u) for fn, u in usage.items() if re.search(pattern, fn)}
+        assert len(found) == count, (pattern, len(found))
+        for fn, (m, u) in found.items():
+            tiles = 1 if "few" in fn else int(m.group(1))
+            assert u["VGPRs"] + u.get("AGPRs", 0) <= 256 and u.get("Occupancy", 2) >= 2, (fn, u)
+            assert u["VGPRs"] + u.get("AGPRs", 0) >= 16 * tiles, (fn, u)
