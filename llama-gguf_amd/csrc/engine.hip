@@ -1214,11 +1214,13 @@ static int prefill_block(lgh_ctx* c, const uint32_t* tokens, uint32_t m, PfTail*
 }
 
 // ---- long prompts: blocks of up to kPfwTokens tokens (prefill_wide.hip) ----
-// From this many tokens on a prompt takes the wide path.  A dense model's products fill a workgroup's 256 tokens there: at Llama-3-8B widths, 8 layers,
-// 255 tokens take 2.12 ms as two blocks and 2.08 ms wide, 192 tokens 1.86 and 1.93, 257 tokens 2.75 and 2.21, 512 tokens 4.33 and 2.67.  A mixture's
-// tokens spread over its experts, so its rows fill no tile either way (Mixtral widths, 2 layers: 160 tokens 1.05 and 0.59 ms, 600 tokens 2.65 and 1.01).
-// The lines hold for narrow models too, whose products leave CUs idle either way: 256 / 257 / 600 tokens in blocks and wide, TinyLlama 4.19 and 3.58, 5.41 and 3.57, 10.5 and
-// 4.18 ms; hidden 512 x 1024, 8 layers, 0.98 and 0.80, 1.28 and 0.79, 2.50 and 0.96; four experts of 768, 160 tokens 1.67 and 0.75.
+// From this many tokens on a prompt takes the wide path: a dense model's where its products fill a workgroup's 256 tokens, a mixture's earlier, for its rows fill no tile either way.  In blocks / wide, ms, Q4_K_M (Q8_0):
+//   4096 x 14336, 8 layers    129: 1.42 / 1.40 (1.57 / 1.44), 192: 1.61 / 1.53 (1.72 / 1.54), 224: 1.73 / 1.78 (1.85 / 1.79), 255: 1.86 / 1.85 (1.99 / 1.86), 257: 2.38 / 1.90, 512: 3.80 / 2.46
+//   2048 x 5632, 8 layers     129: 0.88 / 0.91 (0.92 / 0.97), 192: 0.99 / 0.98 (1.02 / 1.04), 224: 1.05 / 1.16 (1.08 / 1.22), 255: 1.11 / 1.19 (1.14 / 1.25), 257: 1.45 / 1.18, 512: 2.25 / 1.34
+//   512 x 1024, 8 layers      129: 0.62 / 0.60, 192: 0.66 / 0.64, 255: 0.70 / 0.78, 257: 0.96 / 0.77
+//   8 experts of 14336, two a token, 2 layers, Q5_K_M  96: 0.41 / 0.53, 128: 0.42 / 0.52, 129: 0.59 / 0.54, 160: 0.77 / 0.55, 255: 0.82 / 0.61, 600: 2.05 / 0.96
+//   of 768, four, hidden 512                           128: 0.10 / 0.13, 160: 0.17 / 0.15, 255: 0.19 / 0.18
+// (A mixture's 129 to 159 tokens would be faster wide as well, 0.55 instead of 0.59 to 0.77.)
 // Shorter ones keep the blocks that pipeline stages hand over, with their bits.
 static size_t pfw_min_tokens(const lgh_ctx* c) { return c->d.num_experts ? 160 : 256; }
 

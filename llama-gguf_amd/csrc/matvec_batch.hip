@@ -1195,10 +1195,9 @@ static hipError_t mvqb_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, 
 // Indirect launches (a mixture's experts) have one or two sequences per expert: they go to mvqb_few or mvqb2.
 constexpr uint32_t kMvqb4MinSeq = 3;
 
-// Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers of an 8B model in Q4_K_M / Q4_0, us, groups of four against
-// groups of eight: 3 sequences 391 / 378 against 440 / 414, 4: 406 / 381 against 447 / 423; 5: 503 / 484 against 479 / 455, 8: 531 / 512 against 502 / 480,
-// 9: 648 / 624 against 581 / 564, 16: 786 / 761 against 683 / 679; measured with the Q6_K matrices of Q4_K_M in groups of eight as well: in groups of four, as they are for the
-// sake of exact sums, they take a step of 16 sequences from 548 to 565)
+// Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers, us, groups of four against groups of eight over wide images, 3 / 4 sequences: an 8B model in Q4_K_M 342 / 354 against
+// 357 / 370, Q5_K_M 362 / 373 against 389 / 400, Q4_0 323 / 334 against 335 / 347; 2048 x 5632, Q4_K_M, 239 / 249 against 242 / 253; 8192 x 28672 Q4_K_M 775 / 816 against 780 / 808.  Before the wide images, with Q6_K in
+// groups of eight too, 5: 503 / 484 (Q4_K_M / Q4_0) against 479 / 455, 8: 531 / 512 against 502 / 480, 16: 786 / 761 against 683 / 679)
 constexpr uint32_t kMvqb8MinSeq = 5;
 
 bool mvqb_wide_input(int dev_type, uint32_t n_seq) {
