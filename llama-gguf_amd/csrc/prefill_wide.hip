@@ -121,7 +121,7 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
     }
   };
   // activations: an operation covers 8 tokens x 128 bytes; chunk q of token t lies at position q ^ (t >> 1 & 7): 16 tokens' places
-  // differ in their banks, two of a parity included (with t & 7 every second read waited for another; two thirds fewer LDS cycles, experts' gate | up of 600 tokens 464 -> 460 us)
+  // differ in their banks, two of a parity included (with t & 7 every second read waited for another: half of the LDS' cycles, 62.8 -> 33.4 M a launch of gate | up of 2047 tokens; the launch 435.8 and 435.7 us, experts' of 600 tokens 464 -> 460)
   uint32_t xoff[NX];
 #pragma unroll
   for (int i = 0; i < (int)NX; i++) {
