@@ -182,7 +182,7 @@ bool mvqb_wide_input(int dev_type, uint32_t n_seq);
 hipError_t xw_from_xq_launch(const uint8_t* xq, uint32_t xq_stride, uint8_t* xw, uint32_t xw_block, uint32_t k, uint32_t n_seq, hipStream_t st);
 
 // launch-uniform geometry of one int8-MFMA launch as the kernel takes it (mvq_pack)
-struct MvGeom { uint32_t wbpack, geom, geom2, red_floats, lds_red_off, n_wg; };
+struct MvGeom { uint32_t wbpack, geom, geom2, red_floats, lds_red_off, n_wg, flags; };   // flags: 1 the rotation's row lies in LDS
 
 // ---------------------------------------------------------------------------------------------
 // host-side launchers (defined in the .hip files)
@@ -205,6 +205,7 @@ hipError_t hbm_read_launch(const uint8_t* buf, size_t bytes, float* sink, int nt
 // launch-uniform geometry of one int8-MFMA op, packed as the kernel takes it; returns the format mask (0 = not launchable)
 uint32_t mvq_pack(const MvLaunch& L, uint32_t n_wg, uint32_t threads, MvGeom* g, size_t* lds_out);
 uint32_t mvq_format_mask(const MvLaunch& L);
+bool mvq_two_inputs(uint32_t k);   // whether two experts' inputs of k elements fit a launch's LDS side by side
 uint32_t mvq_tile_bytes(int dev_type);   // bytes of one 16-row x 256-element tile in the device layout of this type (0: not a tile16 type)
 bool mvqb_few_takes(int dev_type, uint32_t T, uint32_t nbw, uint32_t n_units, uint32_t n_seq, uint32_t top_k, uint32_t n_experts);
 uint32_t mvqb2_min_seq();

@@ -503,8 +503,9 @@ int ffn_forward(lgh_ctx* c, LayerW& Lw, const FfnView& v, const float* next_nw, 
   // reads the SAME normalised h, so the running sum lives in a scratch vector until the last group writes the residual
   // stream: tmp = 0 + w0 e0 + w1 e1; tmp = tmp + w2 e2 + w3 e3; ...; h = (tmp + ...) + h — moe.rs:363-368's order exactly:
   // one sum over the weighted expert outputs in selection order, then the residual.
-  for (uint32_t g0 = 0; g0 < topk; g0 += 2) {
-    const uint32_t ng = std::min(2u, topk - g0);
+  const uint32_t per = !mfma_type(Lw.down_exps.type) || mvq_two_inputs(Lw.down_exps.k) ? 2 : 1;
+  for (uint32_t g0 = 0; g0 < topk; g0 += per) {
+    const uint32_t ng = std::min(per, topk - g0);
     const bool first_g = g0 == 0, last_g = g0 + ng >= topk;
     {
       SegSpec sp;

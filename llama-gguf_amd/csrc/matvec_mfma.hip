@@ -22,6 +22,7 @@
 // dwords are N0 & 0x0F.., N0 >> 4 & 0x0F.., N1 & 0x0F.., N1 >> 4 & 0x0F.. and every lane loads only its own nibbles:
 //   [0, 1024) lane-major 16 B: N0,N1 of steps 0,1    [1024, 2048) steps 2,3    [2048, 2304) the 16 native 16-byte headers
 #include <algorithm>
+#include <cstring>
 #include <type_traits>
 
 #include "device_utils.h"
@@ -61,8 +62,8 @@ hipError_t mvq_spans(unsigned long long* host, int reset) {
 #define LGH_SPAN(i)                                                                              \
   do {                                                                                           \
     if (threadIdx.x == 0) {                                                                      \
-      if ((i) == 0) atomicMin(&g_span[L.dbg_slot * 2], (unsigned long long)__builtin_amdgcn_s_memrealtime()); \
-      else atomicMax(&g_span[L.dbg_slot * 2 + 1], (unsigned long long)__builtin_amdgcn_s_memrealtime()); \
+      if ((i) == 0) atomicMin(&g_span[A.dbg_slot * 2], (unsigned long long)__builtin_amdgcn_s_memrealtime()); \
+      else atomicMax(&g_span[A.dbg_slot * 2 + 1], (unsigned long long)__builtin_amdgcn_s_memrealtime()); \
     }                                                                                            \
   } while (0)
 #define LGH_WSTAMP(i)                                                                            \
@@ -316,167 +317,238 @@ constexpr int kDepth = 4;   // weight tiles a wave keeps in flight (4 x 2304 B x
 
 // Geometry: ONE workgroup per CU.  Its waves are T k-slices x G row-groups; wave (ks, rg) owns blocks
 // [ks*nbw, (ks+1)*nbw) of k for the Rg tiles of its row-group, i.e. a private stream of npass x Rg x nbw items
-// (item = one 16-row tile x one 256-element block = 2304 B).  Nothing is shared between waves until the final
-// reduction, so there is NO barrier on the way in: a wave requests its slice of x, puts up to kDepth weight tiles in
-// flight right behind it, converts x to limbs in its private LDS region while the tiles travel, and streams.  Few,
-// fat waves on purpose: the dispatcher starts the waves of a grid over ~1 us (measured: the 16 waves of a 1024-thread
-// workgroup began 0.25 / 0.33 / 0.67 / 1.05 us after launch, 4 at a time), which a barrier turns into idle time.
-// A wave issues at most one instruction every ~4 cycles, so a latency-bound prologue costs 1.7 ns PER INSTRUCTION
-// (measured: the first, general version spent 590 instructions = 1.0 us before its first vector load).  Hence:
-//   * everything launch-uniform is computed on the host, packed into eight scalars and delivered by KERNARG PRELOAD
-//     (SGPRs filled at wave launch, no load: -mllvm -amdgpu-kernarg-preload-count=8);
-//   * per-segment fields come from `L` in one batch of scalar loads, per-pass fields only for passes that exist.
+// (item = one 16-row tile x one 256-element block = 2304 B).  Few, fat waves on purpose: the dispatcher starts the waves of a
+// grid over ~1 us (measured: the 16 waves of a 1024-thread workgroup began 0.25 / 0.33 / 0.67 / 1.05 us after launch, 4 at a time).
+// (The second wave of a SIMD streams slower: done at 11.1 us of a gate | up launch, the first at 9.4.  Shares of 9 : 7 end both at 11.2, and the launch no earlier: the CU's loads are what is full, 28 bytes a ns.)
+// A launch is a chain of latencies, and a wave issues one instruction every ~4 cycles (2 ns each where nothing overlaps), so:
+//   * what the kernel does with its results is compiled in (KIND), what is launch-uniform is computed on the host and packed into
+//     scalars delivered by KERNARG PRELOAD (SGPRs filled at wave launch: -mllvm -amdgpu-kernarg-preload-count=8) or read in two batches of
+//     scalar loads: what the first requests need in front of them, what the end needs while the tiles travel.  Read where they are used, behind the last
+//     barrier, the end's were a chain of ten waits.
+//   * x comes first, for the whole workgroup, one copy in LDS: a CU's loads return in the order they went out, and where every wave asks for its own slice of x in front of its tiles, the second four waves' slices
+//     come behind the first four's tiles, from HBM (stamps: 2.3 us after the start, the first four's 1.4).  The barrier between the two costs the 0.15 us that the second four start later.
+// Together (all epilogues in one kernel, every wave's own slice of x, scalars where they are used: before; now), logits to the host after every token: TinyLlama-1.1B Q4_K_M 40 rows 612 -> 535 us a token, Llama-3-8B
+// Q4_K_M 130 rows 1559 -> 1410, Q5_K_M over 3-bit codes (8 layers) 489 -> 450, Q8_0 3000 rows (8 layers) 570 -> 540, Mixtral Q5_K_M (3 layers) 284 -> 266; a launch of 4096 x 4096 ends 3.8 us after its start instead of 4.0 (median
+// workgroup; end behind the last barrier 0.22 us instead of 0.45), gate | up of the 8B model 11.6 instead of 12.3 (0.43 instead of 1.0).
 // geom  = T | G << 8 | nbw << 16 | do_norm << 31         geom2 = nblk | Rg << 16        wbpack = wg_begin[1] | wg_begin[2] << 16
-// offA/B/C = byte strides of a workgroup / a row-group / a k-slice inside one pass's tile array
 // MASK: the formats (1 << F_*) the instantiation handles; with more than one the segment's type decides at run time
-template <uint32_t MASK>
-__device__ __forceinline__ void mvq_body(const uint32_t bid, uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t L_red_floats,
-                                         uint32_t lds_red_off, const MvLaunch& L, uint8_t* smem8) {
-  // the position word (RoPE epilogues): its scalar load goes out with the very first kernarg loads, no wait here
-  const int* L_pos = L.pos;
-  uint32_t pos_now;
-  asm volatile("s_load_dword %0, %1, 0x0" : "=s"(pos_now) : "s"(L_pos) : "memory");
-  const int s = (int)(bid >= (wbpack & 0xFFFFu)) + (int)(bid >= (wbpack >> 16));   // 0xFFFF = no such segment
-  const MvSeg& S = L.seg[s];
-  const uint32_t S_nrows = S.n_rows, S_wgb = S.wg_begin, S_head_dim = S.head_dim;
-  const int S_npass = S.npass, S_epi = S.epi;
-  const float* S_resid = S.resid;
-  const float* S_xq_nw = S.xq_nw;
-  const float* L_rope_cs = L.rope_cs;
+
+// what a launch does with the rows (the epilogues of MvEpilogue that share one instantiation)
+enum : int { MK_OUT = 0, MK_PAIR = 1, MK_QKV = 2, MK_MOE_PAIR = 3, MK_MOE_DOWN = 4 };   // store / + residual; SwiGLU; RoPE and the caches; the selected experts'
+constexpr int mk_passes(int kind) { return kind == MK_PAIR || kind == MK_MOE_DOWN ? 2 : kind == MK_MOE_PAIR ? 4 : 1; }
+
+struct MvqSeg {
+  const uint8_t *w0, *w1;      // tiles of the pass, of the second pass (experts: of the stacks)
+  const float *resid, *xq_nw;
+  uint32_t n_rows, wg_begin, Rg, type;
+  float* out;
+  const float* bias;
+  uint8_t* xq_out;
+  float* xq_ssq;
+  uint32_t epi, head_dim, max_seq, pad;
+};
+struct MvqArgs {
+  const uint8_t *xq, *xq1;     // input (second expert's input of a down launch)
+  const float* ssq_part;
+  const int *sel0, *sel1;      // experts: whose matrices (first two passes or first pass, the rest)
+  uint64_t stride0, stride1;
+  uint32_t n_ssq, npass, k;
+  float eps;
+  const int* pos;
+  const float* rope_cs;
+  const float* moe_w;
+  float* out2;
+  uint8_t* xq_out2;
+  uint64_t dbg_slot;
+  MvqSeg seg[3];
+};
+
+// a pointer that is in scalar registers from here on (global: behind an asm statement the compiler would take it for any address)
+template <class T>
+__device__ __forceinline__ T* mvq_here(T* p) {
+  auto g = (__attribute__((address_space(1))) T*)p;
+  asm volatile("" : "+s"(g));
+  return (T*)g;
+}
+__device__ __forceinline__ void mvq_scalar(uint32_t& v, const int* p) { asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(p) : "memory"); }
+
+template <uint32_t MASK, int KIND>
+__device__ __forceinline__ void mvq_body(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_off, uint32_t flags, const MvqArgs& A, uint8_t* smem8) {
+  constexpr int NP = mk_passes(KIND);
+  const uint32_t bid = blockIdx.x;
+  const int sg = KIND == MK_QKV ? (int)(bid >= (wbpack & 0xFFFFu)) + (int)(bid >= (wbpack >> 16)) : 0;   // 0xFFFF = no such segment
+  const MvqSeg& S = A.seg[sg];
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // ---- the first batch of scalar loads
+  const uint8_t *xq = A.xq, *xq1 = KIND == MK_MOE_DOWN ? A.xq1 : nullptr, *w0 = S.w0, *w1 = NP > 1 ? S.w1 : nullptr;
+  uint32_t S_nrows = S.n_rows, S_wgb = KIND == MK_QKV ? S.wg_begin : 0u, Rg = KIND == MK_QKV ? S.Rg : geom2 >> 16, L_n_ssq = A.n_ssq, S_type = S.type;
+  const float *S_resid = KIND == MK_OUT || KIND == MK_MOE_DOWN ? S.resid : nullptr, *S_nw = KIND == MK_OUT || KIND == MK_MOE_DOWN ? S.xq_nw : nullptr, *L_ssq_part = A.ssq_part;
+  asm volatile("" : "+s"(S_nrows), "+s"(S_wgb), "+s"(Rg), "+s"(L_n_ssq), "+s"(S_type));
+  xq = mvq_here(xq); w0 = mvq_here(w0); L_ssq_part = mvq_here(L_ssq_part);
+  if (KIND == MK_MOE_DOWN) xq1 = mvq_here(xq1);
+  if (NP > 1) w1 = mvq_here(w1);
+  if (KIND == MK_OUT || KIND == MK_MOE_DOWN) { S_resid = mvq_here(S_resid); S_nw = mvq_here(S_nw); }
   constexpr bool kSingle = (MASK & (MASK - 1)) == 0;
   constexpr int kDp = kDepth;   // weight tiles in flight per wave
-  const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type(S.type);
+  const int fmt = kSingle ? __builtin_ctz(MASK) : fmt_of_dev_type((int)S_type);
   auto is = [&](int f) { return ((MASK >> f) & 1u) != 0 && (kSingle || fmt == f); };   // compile-time false for absent formats
   const uint32_t tb = is(F_Q4K) ? fmt_tile_bytes(F_Q4K) : is(F_Q6K) ? fmt_tile_bytes(F_Q6K) : is(F_Q5K) ? fmt_tile_bytes(F_Q5K)
                       : is(F_Q80) ? fmt_tile_bytes(F_Q80) : fmt_tile_bytes(F_Q40);
-  const uint32_t S_T = geom & 0xFFu, S_G = (geom >> 8) & 0xFFu, nbw = (geom >> 16) & 0x3FFFu;
-  const bool nrm = (geom >> 31) != 0;
-  const uint32_t S_nblk = geom2 & 0xFFFFu;
-  // tiles per workgroup and row group: launch-uniform for a single matrix, per segment in a fused launch (S_G is a power of two)
-  const uint32_t Rg = L.nseg > 1 ? S.rows_per_wg >> (4 + __builtin_ctz(S_G)) : geom2 >> 16;
+  const uint32_t S_T = geom & 0xFFu, S_G = (geom >> 8) & 0xFFu, nbw = (geom >> 16) & 0x3FFFu, S_nblk = geom2 & 0xFFFFu;
+  const bool nrm = KIND != MK_MOE_DOWN && (geom >> 31) != 0;
   const uint32_t S_rpw = 16u * Rg * S_G;
   const uint32_t wg = bid - S_wgb;
-
-  const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int S_npass = KIND == MK_MOE_PAIR || KIND == MK_MOE_DOWN ? (int)A.npass : NP;
+  const uint32_t nw = S_T * S_G;                                  // waves
   LGH_WSTAMP(0);
   LGH_SPAN(0);
   uint32_t ks = wave, rg = 0;                                     // wave = rg * T + ks (at most G - 1 subtractions)
   while (ks >= S_T) { ks -= S_T; rg++; }
   const bool active = rg < S_G;
   const uint32_t blk0 = ks * nbw;
-  uint32_t nblk_w = active && blk0 < S_nblk ? min(nbw, S_nblk - blk0) : 0;   // (not const: see the phase loop)
+  uint32_t nblk_w = active && blk0 < S_nblk ? min(nbw, S_nblk - blk0) : 0;   // (not const: see below)
   const uint32_t ntiles = (S_nrows + 15) >> 4;
   const uint32_t tile0 = (wg * S_G + rg) * Rg;
   uint32_t ntile_w = active && tile0 < ntiles ? min(Rg, ntiles - tile0) : 0;
-  // LDS: per-wave private copies of the XQ records of its k-slice (1280 B per block, xq.h), then the partial-sum slots
-  // and the total sum(x^2)
+  // LDS: the XQ records of x (1280 B per block, xq.h; a down launch of two experts: of both inputs), the partial-sum slots [pass][slice][row], 1 / rms, the rotation's cosines and sines
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem8;   // LDS byte address
-  const uint32_t wreg = wave * nbw * kXqRecord;
-  const uint8_t* xrec = smem8 + wreg;
-  const uint32_t xrec_lds = lds_base + wreg;
-  float* red = reinterpret_cast<float*>(smem8 + lds_red_off);
-  float* ssq = red + L_red_floats;
+  const uint32_t xbytes = S_nblk * kXqRecord;
+  float* red = reinterpret_cast<float*>(smem8 + red_off);
+  float* inv_at = red + (size_t)S_npass * S_T * S_rpw;
   // lane roles inside an MFMA: B operand = weight row n, k-chunk c (16 elements); the A operand is block-diagonal over the
   // four k-chunks — rows 4c'..4c'+3 = the four limbs of chunk c' — because XQ scales every 16 elements; so lane group
   // mq = c of D holds the limb sums of chunk c of weight row n
-  const uint32_t n = lane & 15, c = lane >> 4;
-  const uint32_t mq = c;
+  const uint32_t n = lane & 15, mq = lane >> 4;
 
-  // per-pass base of this wave's tiles and input vector.  The MoE expert index is a SCALAR load — a vector load would
-  // sit in the same in-order queue as the weight tiles.
-  const uint64_t woff = ((uint64_t)tile0 * S_nblk + blk0) * tb;
-  // (four named scalars each, not arrays: an array indexed by the pass number ends up in scratch memory, and a kernel
-  // that touches scratch pays for it at every launch)
-  const uint8_t *pb0 = nullptr, *pb1 = nullptr, *pb2 = nullptr, *pb3 = nullptr;
-  const uint8_t *px0 = nullptr, *px1 = nullptr, *px2 = nullptr, *px3 = nullptr;
-  auto pass_setup = [&](int p, const uint8_t*& pb, const uint8_t*& px) {
-    if (p < S_npass) {
-      const MvPass& P = S.pass[p];
-      const uint8_t* plane = P.plane[0];
-      const int* sel = P.sel;
-      px = P.xq;
-      if (sel) {
-        uint32_t e32;
-        asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(e32) : "s"(sel) : "memory");
-        plane += (uint64_t)e32 * P.sel_stride[0];
-      }
-      pb = plane + woff;
-    }
-  };
-  pass_setup(0, pb0, px0);
-  pass_setup(1, pb1, px1);
-  pass_setup(2, pb2, px2);
-  pass_setup(3, pb3, px3);
   // RMSNorm: the producer of x left partial sums of x^2; wave 0 gathers up to 256 of them now (oldest loads of the wave,
   // first used after the last tile) and the rest, if any, at the end
-  const float* L_ssq_part = L.ssq_part;
-  const uint32_t L_n_ssq = L.n_ssq_part;
-  float ssp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto load_ssp = [&]() {
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      if (lane + 64 * j < L_n_ssq) ssp[j] = L_ssq_part[lane + 64 * j];
-  };
-  if (nrm && wave == 0) load_ssp();
-  MvEpiPre epi_pre = {0.0f, 0.0f, false};
-  mv_epilogue_prefetch_resid(S_epi, S_resid, S_xq_nw, S_nrows, wg, S_rpw, epi_pre);
-  asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(pos_now));   // long since there: the kernarg batch above was waited for
-  mv_epilogue_prefetch_rope(S_epi, pos_now, L_rope_cs, S_head_dim, S_nrows, wg, S_rpw, epi_pre);
+  // (four names, not an array: as one value of four registers the second load would wait for the first)
+  float ss0 = 0.0f, ss1 = 0.0f, ss2 = 0.0f, ss3 = 0.0f;
+  if (nrm && wave == 0) {
+    if (lane < L_n_ssq) ss0 = L_ssq_part[lane];
+    if (lane + 64 < L_n_ssq) ss1 = L_ssq_part[lane + 64];
+    if (lane + 128 < L_n_ssq) ss2 = L_ssq_part[lane + 128];
+    if (lane + 192 < L_n_ssq) ss3 = L_ssq_part[lane + 192];
+  }
+  // the residual element and the next consumer's norm weight of this thread's row
+  float pre_res = 0.0f, pre_nw = 1.0f;
+  const uint32_t row = wg * S_rpw + tid;
+  const bool live = tid < S_rpw && row < S_nrows;
+  if ((KIND == MK_OUT || KIND == MK_MOE_DOWN) && live) {
+    if (S_resid) pre_res = S_resid[row];
+    if (S_nw) pre_nw = S_nw[row];
+  }
   LGH_WSTAMP(1);
+  LGH_STAMP(0);
+
+  // ---- x into LDS by LDS-DMA (no registers, no vector ALU), 1 KB a transfer.  Inline asm: with the builtin hipcc drains vmcnt to 0 at the next load it issues.
+  auto x_request = [&](const uint8_t* src, uint32_t at) {
+    for (uint32_t p = wave; p * 1024u < xbytes; p += nw) {
+      const uint32_t off = p * 1024u + lane * 16u;
+      if (off < xbytes) {
+        uint32_t keep;
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                     : "=&s"(keep) : "v"(src + off), "s"(lds_base + at + p * 1024u) : "memory");
+      }
+    }
+  };
+  auto meet = [&]() { asm volatile("s_barrier" : : : "memory"); };
+
+  // the passes' tiles; experts are chosen on the device, by SCALAR loads — vector loads would sit in the same in-order queue as the weight tiles
+  const uint64_t woff = ((uint64_t)tile0 * S_nblk + blk0) * tb;
+  const uint8_t *pb0 = w0 + woff, *pb1 = w1 + woff, *pb2 = nullptr, *pb3 = nullptr;
+  if (KIND == MK_MOE_PAIR) {
+    uint32_t e0, e1 = 0;
+    mvq_scalar(e0, A.sel0);
+    if (S_npass > 2) mvq_scalar(e1, A.sel1);
+    pb2 = pb0 + (uint64_t)e1 * A.stride0;
+    pb3 = pb1 + (uint64_t)e1 * A.stride1;
+    pb0 += (uint64_t)e0 * A.stride0;
+    pb1 += (uint64_t)e0 * A.stride1;
+  } else if (KIND == MK_MOE_DOWN) {
+    uint32_t e0, e1 = 0;
+    mvq_scalar(e0, A.sel0);
+    if (S_npass > 1) mvq_scalar(e1, A.sel1);
+    pb0 += (uint64_t)e0 * A.stride0;
+    pb1 += (uint64_t)e1 * A.stride1;
+  }
   struct Pos { uint32_t p, tl, b; };
-  auto issue = [&](const Pos& q, RawT16& r) {   // fmt_loads_per_tile(format) loads (x_finish counts on it)
-    const uint8_t* base = q.p == 0 ? pb0 : q.p == 1 ? pb1 : q.p == 2 ? pb2 : pb3;
+  auto issue = [&](const Pos& q, RawT16& r) {   // fmt_loads_per_tile(format) loads (the wait for x counts on it)
+    const uint8_t* base = NP == 1 || q.p == 0 ? pb0 : NP == 2 || q.p == 1 ? pb1 : q.p == 2 ? pb2 : pb3;
     mvq_issue_tile<MASK>(fmt, base + ((size_t)q.tl * S_nblk + q.b) * tb, lane, r);
   };
-
-  LGH_STAMP(0);
   // item order: pass-major, then tile, then block (innermost: one accumulator per (pass, tile))
   Pos nx = {0, 0, 0};
   auto advance = [&]() {
     if (++nx.b == nblk_w) { nx.b = 0; if (++nx.tl == ntile_w) { nx.tl = 0; ++nx.p; } }
   };
   float acc = 0.0f;
-
-  auto finish_tile = [&](const Pos& q) {   // last block of a (pass, tile): the four lane groups -> one partial sum per row
-    float t = acc + __shfl_xor(acc, 16, 64);
-    t += __shfl_xor(t, 32, 64);
-    if (mq == 0) red[(size_t)(q.p * S_T + ks) * S_rpw + (rg * Rg + q.tl) * 16 + n] = t;
-    acc = 0.0f;
-  };
-  // one item = 16 weight rows x 256 elements.  Both formats: four MFMAs (one per 64 elements); lane group c then holds,
+  auto slot = [&](uint32_t p, uint32_t tl) -> float& { return red[(size_t)(p * S_T + ks) * S_rpw + (rg * Rg + tl) * 16 + n]; };
+  // one item = 16 weight rows x 256 elements: four MFMAs (one per 64 elements); lane group c then holds,
   // for weight row n, the four limb sums of chunk 4pp + c, recombined to V = sum_k q_k * I_k (exact int, rounded once to f32).
   auto consume = [&](const Pos& q, const RawT16& r) {
-    mvq_consume_tile<MASK>(fmt, r, xrec + q.b * kXqRecord, lane, acc);
-    if (q.b + 1 == nblk_w) finish_tile(q);
+    const uint32_t xat = KIND == MK_MOE_DOWN && q.p == 1 ? xbytes : 0u;
+    mvq_consume_tile<MASK>(fmt, r, smem8 + xat + (blk0 + q.b) * kXqRecord, lane, acc);
+    if (q.b + 1 == nblk_w) {   // last block of a (pass, tile): the four lane groups -> one partial sum per row
+      const float t = swap32_add(swap16_add(acc));
+      if (mq == 0) slot(q.p, q.tl) = t;
+      acc = 0.0f;
+    }
   };
 
-  auto x_of = [&](int p) -> const uint8_t* { return p == 0 ? px0 : p == 1 ? px1 : p == 2 ? px2 : px3; };
-  for (int p0 = 0; p0 < S_npass;) {   // phases: runs of passes that share one input vector
-    int p1 = p0 + 1;
-    while (p1 < S_npass && x_of(p1) == x_of(p0)) p1++;
-    const uint32_t npp = (uint32_t)(p1 - p0);
-    const uint8_t* xg = x_of(p0) + (size_t)blk0 * kXqRecord;   // this wave's k-slice of XQ records
-    nx.p = (uint32_t)p0; nx.tl = 0; nx.b = 0;
-    // Opaque to the optimizer (the values do not change): otherwise every shape's loop-invariant bookkeeping — ~300
-    // scalar instructions, most of them for paths not taken — is hoisted in front of the first load, at 1.7 ns each.
-    asm volatile("" : "+s"(nblk_w), "+s"(ntile_w));
-    const uint32_t nitems = npp * ntile_w * nblk_w;
+  // ---- the second batch of scalar loads and what hangs on it: while the tiles travel
+  float *S_out = nullptr, *S_ssq = nullptr, *L_out2 = nullptr;
+  const float *S_bias = nullptr, *L_moe_w = nullptr, *L_cs = nullptr;
+  uint8_t *S_xq = nullptr, *S_xq2 = nullptr;
+  uint32_t S_epi = 0, S_hd = 0, S_maxseq = 0, L_k = 0, pos = 0;
+  float L_eps = 0.0f;
+  const uint32_t cs_at = (red_off + (uint32_t)S_npass * S_T * S_rpw * 4u + 16u + 15u) & ~15u;
+  bool cs_lds = false;
+  auto end_scalars = [&]() {
+    S_out = S.out;
+    if (KIND != MK_MOE_DOWN) { L_k = A.k; L_eps = A.eps; }
+    if (KIND != MK_QKV) S_xq = S.xq_out;
+    if (KIND == MK_OUT || KIND == MK_MOE_DOWN) S_ssq = S.xq_ssq;
+    if (KIND == MK_OUT || KIND == MK_QKV) S_bias = S.bias;
+    if (KIND == MK_QKV) { S_epi = S.epi; S_hd = S.head_dim; S_maxseq = S.max_seq; L_cs = A.rope_cs; }
+    if (KIND == MK_MOE_PAIR) { L_out2 = A.out2; S_xq2 = A.xq_out2; }
+    if (KIND == MK_MOE_DOWN) { L_out2 = A.out2; L_moe_w = A.moe_w; }
+    if (KIND != MK_MOE_DOWN) asm volatile("" : "+s"(L_k), "+s"(L_eps));
+    S_out = mvq_here(S_out);
+    if (KIND != MK_QKV) S_xq = mvq_here(S_xq);
+    if (KIND == MK_OUT || KIND == MK_MOE_DOWN) S_ssq = mvq_here(S_ssq);
+    if (KIND == MK_OUT || KIND == MK_QKV) S_bias = mvq_here(S_bias);
+    if (KIND == MK_QKV) {
+      asm volatile("" : "+s"(S_epi), "+s"(S_hd), "+s"(S_maxseq));
+      L_cs = mvq_here(L_cs);
+    }
+    if (KIND == MK_MOE_PAIR) S_xq2 = mvq_here(S_xq2);
+    if (KIND == MK_MOE_PAIR || KIND == MK_MOE_DOWN) L_out2 = mvq_here(L_out2);
+    if (KIND == MK_MOE_DOWN) L_moe_w = mvq_here(L_moe_w);
+    if (KIND == MK_QKV) {
+      mvq_scalar(pos, A.pos);
+      cs_lds = (S_epi == EPI_ROPE_Q || S_epi == EPI_ROPE_K) && (flags & 1u) != 0;
+    }
+  };
+  // the position's cosines and sines into LDS (behind the tiles: the compiler's waits for those do not know of it and wait for one load more than they have to)
+  auto rotation = [&]() {
+    if (KIND == MK_QKV && cs_lds && wave == 0 && lane * 4 < S_hd) {
+      const uint8_t* src = reinterpret_cast<const uint8_t*>(L_cs) + (uint64_t)pos * S_hd * 4;
+      uint32_t keep;
+      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                   : "=&s"(keep) : "v"(src + lane * 16), "s"(lds_base + cs_at) : "memory");
+    }
+  };
 
-    // ---- x staging: the wave's XQ records go straight into its LDS region by LDS-DMA (1024 B + 256 B per record, no
-    // registers, no vector ALU), requested FIRST; the caller's tile issues follow, loads return in order, so x_finish
-    // waits for x alone (vmcnt = the weight loads behind it).  Inline asm: with the builtin hipcc drains vmcnt to 0 at
-    // the next load it issues.
-    auto x_request = [&]() {
-      for (uint32_t b = 0; b < nblk_w; b++) {
-        const uint8_t* src = xg + b * kXqRecord;
-        const uint32_t dst = xrec_lds + b * kXqRecord;
-        uint32_t keep;
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_add_u32 m0, m0, 0x400\n\t"
-                     "s_nop 0\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0"
-                     : "=&s"(keep) : "v"(src + lane * 16), "v"(src + 1024 + lane * 4), "s"(dst) : "memory", "scc");
-      }
-    };
+  x_request(xq, 0);
+  if (KIND == MK_MOE_DOWN && S_npass > 1) x_request(xq1, xbytes);
+  meet();                                      // all of x is on its way: now the tiles
+  {
+    // Opaque to the optimizer (the values do not change): otherwise every shape's loop-invariant bookkeeping — ~300
+    // scalar instructions, most of them for paths not taken — is hoisted in front of the first load.
+    asm volatile("" : "+s"(nblk_w), "+s"(ntile_w));
+    const uint32_t nitems = (uint32_t)S_npass * ntile_w * nblk_w;
     auto x_finish = [&](auto n_tiles) {
       constexpr int NT = decltype(n_tiles)::value;
       // n_tiles x fmt_loads_per_tile loads were issued behind the x requests
@@ -492,57 +564,63 @@ __device__ __forceinline__ void mvq_body(const uint32_t bid, uint32_t wbpack, ui
     else if constexpr (NT * (LPT) == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");          \
     else if constexpr (NT * (LPT) == 5) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");          \
     else if constexpr (NT * (LPT) == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          \
-    else asm volatile("s_waitcnt vmcnt(3)" ::: "memory");                                         \
+    else if constexpr (NT * (LPT) == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");          \
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                         \
   } while (0)
       if (is(F_Q6K) || is(F_Q80)) LGH_WAIT_BEHIND(5);
       else if (is(F_Q5K)) LGH_WAIT_BEHIND(4);
       else LGH_WAIT_BEHIND(3);
 #undef LGH_WAIT_BEHIND
+      meet();
       LGH_WSTAMP(4);
     };
 
     RawT16 buf[kDp];
-    Pos pos[kDp];
+    Pos at[kDp];
     // `run` for a static number of tiles put in flight up front; every path ends with nothing in flight
     auto run = [&](auto n_first) {
       constexpr int NF = decltype(n_first)::value;
-      LGH_WSTAMP(2);
-      x_request();
 #pragma unroll
-      for (int j = 0; j < NF; j++) { pos[j] = nx; issue(nx, buf[j]); advance(); }
+      for (int j = 0; j < NF; j++) { at[j] = nx; issue(nx, buf[j]); advance(); }
+      LGH_WSTAMP(2);
+      end_scalars();
       x_finish(n_first);
+      rotation();
       LGH_WSTAMP(5);
       if constexpr (NF < kDp) {   // that was everything
 #pragma unroll
-        for (int j = 0; j < NF; j++) consume(pos[j], buf[j]);
+        for (int j = 0; j < NF; j++) consume(at[j], buf[j]);
       } else {
         uint32_t rem = nitems;       // not yet consumed; kDp of them in flight
         while (rem >= 2 * kDp) {
 #pragma unroll
           for (int j = 0; j < kDp; j++) {
-            consume(pos[j], buf[j]);
-            pos[j] = nx; issue(nx, buf[j]); advance();
+            consume(at[j], buf[j]);
+            at[j] = nx; issue(nx, buf[j]); advance();
           }
           rem -= kDp;
         }
         const uint32_t unissued = rem - kDp;   // 0 .. kDp-1
 #pragma unroll
         for (int j = 0; j < kDp; j++) {
-          consume(pos[j], buf[j]);
-          if ((uint32_t)j < unissued) { pos[j] = nx; issue(nx, buf[j]); advance(); }
+          consume(at[j], buf[j]);
+          if ((uint32_t)j < unissued) { at[j] = nx; issue(nx, buf[j]); advance(); }
         }
 #pragma unroll
         for (int j = 0; j < kDp - 1; j++)
-          if ((uint32_t)j < unissued) consume(pos[j], buf[j]);
+          if ((uint32_t)j < unissued) consume(at[j], buf[j]);
       }
     };
     if (nitems == 0) {
       if (nblk_w == 0 && ntile_w > 0) {
         // a k-slice beyond the last block (T does not divide the block count): its partial-sum slots must read as zero
-        for (uint32_t p = (uint32_t)p0; p < (uint32_t)p1; p++)
+        for (uint32_t p = 0; p < (uint32_t)S_npass; p++)
           for (uint32_t tl = 0; tl < ntile_w; tl++)
-            if (mq == 0) red[(size_t)(p * S_T + ks) * S_rpw + (rg * Rg + tl) * 16 + n] = 0.0f;
+            if (mq == 0) slot(p, tl) = 0.0f;
       }
+      end_scalars();
+      x_finish(std::integral_constant<int, 0>{});
+      rotation();
     } else if (nitems == 1) {
       run(std::integral_constant<int, 1>{});
     } else if (nitems == 2) {
@@ -552,32 +630,113 @@ __device__ __forceinline__ void mvq_body(const uint32_t bid, uint32_t wbpack, ui
     } else {
       run(std::integral_constant<int, kDp>{});
     }
-    p0 = p1;
     LGH_STAMP(3);
     LGH_WSTAMP(6);
   }
-  if (nrm && wave == 0) {   // the producer's partial sums of x^2 -> ssq[0]; the other waves contribute nothing
-    float ss = (ssp[0] + ssp[1]) + (ssp[2] + ssp[3]);
+  if (nrm && wave == 0) {   // the producer's partial sums of x^2 -> 1 / rms (simd.rs:853-855)
+    float ss = (ss0 + ss1) + (ss2 + ss3);
     for (uint32_t i = 256 + lane; i < L_n_ssq; i += 64) ss += L_ssq_part[i];
     ss = wave_sum_to_lane63(ss);
-    if (lane == 63) ssq[0] = ss;
-  } else if (nrm && lane == 0) {
-    ssq[wave] = 0.0f;
+    if (lane == 63) inv_at[0] = mv_inv_rms(ss, L_k, L_eps);
   }
+  if (KIND == MK_QKV) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the rotation's row, long since there)
   __syncthreads();
   LGH_STAMP(4);
-  mv_epilogue(L, S, wg, red, ssq, S_T, epi_pre);
+
+  // ---- the end: one thread per row (or per row pair for RoPE)
+  const float inv = nrm ? inv_at[0] : 1.0f;
+  auto rowval = [&](int p, uint32_t rl) {
+    const float* r = red + (size_t)p * S_T * S_rpw + rl;
+    float v = 0.0f;
+    if (S_T == 8) {
+      float t[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) t[j] = r[j * S_rpw];
+#pragma unroll
+      for (int j = 0; j < 8; j++) v += t[j];
+    } else {
+#pragma nounroll
+      for (uint32_t j = 0; j < S_T; j++) v += r[j * S_rpw];
+    }
+    return v * inv;
+  };
+  if (KIND == MK_QKV && (S_epi == EPI_ROPE_Q || S_epi == EPI_ROPE_K)) {
+    const uint32_t rl = 2 * tid, r0 = wg * S_rpw + rl;
+    if (rl < S_rpw && r0 < S_nrows) {
+      float x0 = rowval(0, rl), x1 = rowval(0, rl + 1);
+      if (S_bias) { x0 += S_bias[r0]; x1 += S_bias[r0 + 1]; }
+      const uint32_t head = (S_hd & (S_hd - 1)) == 0 ? r0 >> __builtin_ctz(S_hd) : r0 / S_hd, e = r0 - head * S_hd;   // e even: the pair's first element
+      float c, s;
+      if (cs_lds) {
+        const float* cs = reinterpret_cast<const float*>(smem8 + cs_at) + e;
+        c = cs[0]; s = cs[1];
+      } else {
+        const float* cs = L_cs + (size_t)pos * S_hd + e;
+        c = cs[0]; s = cs[1];
+      }
+      const float y0 = x0 * c - x1 * s, y1 = x0 * s + x1 * c;  // ops.rs:1326-1331
+      float* dst = S_epi == EPI_ROPE_Q ? S_out + r0 : S_out + ((size_t)head * S_maxseq + pos) * S_hd + e;
+      dst[0] = y0;
+      dst[1] = y1;
+    }
+  } else if (live) {
+    float v0 = rowval(0, tid);
+    if ((KIND == MK_OUT || KIND == MK_QKV) && S_bias) v0 += S_bias[row];
+    if (KIND == MK_QKV) {
+      if (S_epi == EPI_V_CACHE) {
+        const uint32_t head = (S_hd & (S_hd - 1)) == 0 ? row >> __builtin_ctz(S_hd) : row / S_hd;
+        S_out[((size_t)head * S_maxseq + pos) * S_hd + (row - head * S_hd)] = v0;
+      } else {
+        S_out[row] = v0;
+      }
+    } else if (KIND == MK_MOE_PAIR) {
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        if (2 * e + 1 >= S_npass) break;
+        const float g = e == 0 ? v0 : rowval(2, tid), a = silu_f(g) * rowval(2 * e + 1, tid);
+        (e == 0 ? S_out : L_out2)[row] = a;
+        uint8_t* xo = e == 0 ? S_xq : S_xq2;   // each expert's activation feeds its own down projection
+        if (xo) xq_store_chunk(xo, row >> 4, a, nullptr, 0.0f, tid);
+      }
+    } else {
+      float outv;
+      if (KIND == MK_PAIR) outv = silu_f(v0) * rowval(1, tid);
+      else if (KIND == MK_OUT) outv = S_resid ? v0 + pre_res : v0;
+      else {
+        // moe.rs:363-368: ONE zero-initialised sum, += weight * expert_out over all selected experts in selection order, then the
+        // residual.  The experts run two per launch: a launch continues the running sum the earlier ones left (out2; none: it
+        // starts from zero) and only the last one adds the residual (resid; none: the output is the running sum).
+        float sum = L_out2 ? L_out2[row] : 0.0f;
+        sum += L_moe_w[0] * v0;
+        if (S_npass > 1) sum += L_moe_w[1] * rowval(1, tid);
+        outv = S_resid ? sum + pre_res : sum;
+      }
+      S_out[row] = outv;
+      // XQ image of the output for a matrix-core consumer (xq.h).  n_rows is a multiple of 16 here (host-checked), so the
+      // 16 threads of a chunk are all live; with a norm in front of the consumer the record holds out * norm_weight and each
+      // chunk leaves its sum of out^2.
+      if (S_xq) xq_store_chunk(S_xq, row >> 4, outv * pre_nw, S_ssq, outv, tid);
+    }
+  }
   LGH_STAMP(5);
   LGH_WSTAMP(7);
   LGH_SPAN(1);
 }
 
+// Q, K and V of a layer (all of the mixes' launches are)
 template <uint32_t MASK>
-__global__ void __launch_bounds__(kWaves * 64) mvq_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t L_red_floats,
-                                                          uint32_t lds_red_off, const MvLaunch L) {
+__global__ void __launch_bounds__(kWaves * 64) mvq_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_off, uint32_t flags, const MvqArgs A) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
   LGH_TL_BEGIN(mvq, lgh::TL_MVQ, geom2);
-  mvq_body<MASK>(blockIdx.x, wbpack, geom, geom2, L_red_floats, lds_red_off, L, smem8);
+  mvq_body<MASK, MK_QKV>(wbpack, geom, geom2, red_off, flags, A, smem8);
+  LGH_TL_END();
+}
+// everything else
+template <uint32_t MASK, int KIND>
+__global__ void __launch_bounds__(kWaves * 64) mvq_rows_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_off, uint32_t flags, const MvqArgs A) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  LGH_TL_BEGIN(mvq, lgh::TL_MVQ, geom2);
+  mvq_body<MASK, KIND>(wbpack, geom, geom2, red_off, flags, A, smem8);
   LGH_TL_END();
 }
 
@@ -613,25 +772,22 @@ hipError_t mvq_plan(uint32_t k, uint32_t n_rows, int npass, MvPlan* plan, uint32
   return hipSuccess;
 }
 
-static uint32_t mvq_red_offset(uint32_t nwaves, uint32_t nbw) { return nwaves * nbw * kXqRecord; }
-size_t mvq_lds_bytes(uint32_t nwaves, uint32_t nbw, uint32_t red_floats) {
-  return (size_t)mvq_red_offset(nwaves, nbw) + (size_t)red_floats * 4 + 64;
-}
+// LDS of a launch: x (of `n_x` inputs), the partial sums, 1 / rms (and the rotation's row where there is room)
+static uint32_t mvq_red_offset(uint32_t nblk, uint32_t n_x) { return nblk * kXqRecord * n_x; }
+static size_t mvq_lds_bytes(uint32_t nblk, uint32_t n_x, uint32_t red_floats) { return (size_t)mvq_red_offset(nblk, n_x) + (size_t)red_floats * 4 + 16; }
 
-template <uint32_t MASK>
-static hipError_t mvq_go(const MvLaunch& L, uint32_t n_wg, uint32_t threads, size_t lds, hipStream_t st, uint32_t wbpack, uint32_t geom,
-                         uint32_t geom2, uint32_t red_off) {
-  static bool attr_set[64] = {};
-  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(&mvq_kernel<MASK>), 160 * 1024, attr_set); e != hipSuccess) return e;
-  hipLaunchKernelGGL((mvq_kernel<MASK>), dim3(n_wg), dim3(threads), lds, st, wbpack, geom, geom2, L.red_floats, red_off, L);
-  return hipGetLastError();
-}
+bool mvq_two_inputs(uint32_t k) { return mvq_lds_bytes((k + 255) / 256, 2, 2 * 8 * kWaves * 16) <= 160 * 1024; }   // (with the partial sums of up to eight tiles a workgroup)
 
 // launch-uniform geometry of one op, packed for the kernel; returns the format mask (0 = not launchable)
 uint32_t mvq_pack(const MvLaunch& L, uint32_t n_wg, uint32_t threads, MvGeom* g, size_t* lds_out) {
   const MvSeg& S0 = L.seg[0];
-  const size_t lds = mvq_lds_bytes(threads / 64, S0.units, L.red_floats);
-  if (lds > 160 * 1024 || threads == 0 || threads > kWaves * 64 || n_wg == 0 || L.nseg < 1 || L.nseg > 3) return 0;
+  if (threads == 0 || threads > kWaves * 64 || n_wg == 0 || L.nseg < 1 || L.nseg > 3) return 0;
+  const uint32_t n_x = S0.epi == EPI_MOE_DOWN && S0.npass > 1 ? 2 : 1, row = S0.head_dim * 4;
+  size_t lds = mvq_lds_bytes(S0.nblk, n_x, L.red_floats);
+  if (lds > 160 * 1024) return 0;
+  const bool rotation = (S0.epi == EPI_ROPE_Q || S0.epi == EPI_ROPE_K) && row % 16 == 0 && row <= 1024 && lds + 16 + row <= 160 * 1024;   // a transfer of 64 lanes
+  if (rotation) lds += 16 + row;
+  g->flags = rotation ? 1u : 0u;
   uint32_t mask = 0;
   for (int i = 0; i < L.nseg; i++) {   // the launch-uniform geometry travels as scalars
     const MvSeg& Si = L.seg[i];
@@ -650,18 +806,110 @@ uint32_t mvq_pack(const MvLaunch& L, uint32_t n_wg, uint32_t threads, MvGeom* g,
   g->geom = S0.T | S0.G << 8 | S0.units << 16 | (L.do_norm ? 1u << 31 : 0u);
   g->geom2 = S0.nblk | Rg << 16;
   g->red_floats = L.red_floats;
-  g->lds_red_off = mvq_red_offset(threads / 64, S0.units);
+  g->lds_red_off = mvq_red_offset(S0.nblk, n_x);
   g->n_wg = n_wg;
   *lds_out = lds;
   return mask;
 }
 
+// the launch as the kernel takes it; the instantiation (MK_*), or -1 where there is none
+static int mvq_args(const MvLaunch& L, MvqArgs* A) {
+  std::memset(A, 0, sizeof(*A));
+  const MvSeg& S0 = L.seg[0];
+  int kind = -1;
+  switch (S0.epi) {
+    case EPI_STORE: case EPI_RESID: kind = L.nseg == 1 && S0.npass == 1 ? MK_OUT : -1; break;
+    case EPI_SWIGLU: kind = L.nseg == 1 && S0.npass == 2 ? MK_PAIR : -1; break;
+    case EPI_ROPE_Q: case EPI_ROPE_K: case EPI_V_CACHE: kind = MK_QKV; break;
+    case EPI_MOE_SWIGLU: kind = L.nseg == 1 && (S0.npass == 2 || S0.npass == 4) ? MK_MOE_PAIR : -1; break;
+    case EPI_MOE_DOWN: kind = L.nseg == 1 && (S0.npass == 1 || S0.npass == 2) ? MK_MOE_DOWN : -1; break;
+    default: break;
+  }
+  if (kind < 0 || (kind == MK_MOE_DOWN && L.do_norm)) return -1;
+  const MvPass* P = S0.pass;
+  const bool moe = kind == MK_MOE_PAIR || kind == MK_MOE_DOWN;
+  const int second = kind == MK_MOE_PAIR ? 2 : 1;   // the second expert's first pass
+  for (int p = 0; p < S0.npass; p++) {
+    if ((P[p].sel != nullptr) != moe) return -1;
+    if (kind != MK_MOE_DOWN && P[p].xq != P[0].xq) return -1;
+    if (moe && (P[p].plane[0] != P[p % second].plane[0] || P[p].sel_stride[0] != P[p % second].sel_stride[0] || P[p].sel != P[p / second * second].sel)) return -1;
+  }
+  A->xq = P[0].xq;
+  A->xq1 = S0.npass > 1 ? P[1].xq : P[0].xq;
+  A->ssq_part = L.ssq_part;
+  A->n_ssq = L.n_ssq_part;
+  A->npass = (uint32_t)S0.npass;
+  A->k = L.k;
+  A->eps = L.eps;
+  A->pos = L.pos;
+  A->rope_cs = L.rope_cs;
+  A->moe_w = S0.moe_w;
+  A->out2 = S0.out2;
+  A->xq_out2 = S0.xq_out2;
+  A->dbg_slot = L.dbg_slot;
+  if (moe) {
+    A->sel0 = P[0].sel;
+    A->sel1 = S0.npass > second ? P[second].sel : P[0].sel;
+    A->stride0 = P[0].sel_stride[0];
+    A->stride1 = P[S0.npass > 1 ? 1 : 0].sel_stride[0];
+  }
+  for (int i = 0; i < L.nseg; i++) {
+    const MvSeg& S = L.seg[i];
+    if (i > 0 && (S.npass != 1 || S.pass[0].sel || S.pass[0].xq != P[0].xq)) return -1;
+    if (i > 0 && S.epi != EPI_ROPE_Q && S.epi != EPI_ROPE_K && S.epi != EPI_V_CACHE && S.epi != EPI_STORE) return -1;
+    if ((kind == MK_QKV && S.xq_out) || (kind == MK_PAIR && S.xq_nw) || ((moe || kind == MK_PAIR) && S.bias)) return -1;
+    MvqSeg& D = A->seg[i];
+    D.w0 = S.pass[0].plane[0];
+    D.w1 = S.npass > 1 ? S.pass[1].plane[0] : S.pass[0].plane[0];
+    D.resid = kind == MK_MOE_DOWN || S.epi == EPI_RESID ? S.resid : nullptr;
+    D.xq_nw = S.xq_out ? S.xq_nw : nullptr;
+    D.n_rows = S.n_rows;
+    D.wg_begin = S.wg_begin;
+    D.Rg = S.rows_per_wg / 16 / S.G;
+    D.type = (uint32_t)S.type;
+    D.out = S.out;
+    D.bias = S.bias;
+    D.xq_out = S.xq_out;
+    D.xq_ssq = S.xq_ssq;
+    D.epi = (uint32_t)S.epi;
+    D.head_dim = S.head_dim;
+    D.max_seq = S.max_seq;
+  }
+  return kind;
+}
+
+typedef void (*MvqKernel)(uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, const MvqArgs);
+template <MvqKernel FN>
+static hipError_t mvq_go(const MvqArgs& A, const MvGeom& g, uint32_t threads, size_t lds, hipStream_t st) {
+  static bool attr_set[64] = {};
+  if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(FN), 160 * 1024, attr_set); e != hipSuccess) return e;
+  hipLaunchKernelGGL(FN, dim3(g.n_wg), dim3(threads), lds, st, g.wbpack, g.geom, g.geom2, g.lds_red_off, g.flags, A);
+  return hipGetLastError();
+}
+
+template <uint32_t MASK>
+static hipError_t mvq_kind(int kind, const MvqArgs& A, const MvGeom& g, uint32_t threads, size_t lds, hipStream_t st) {
+  if (kind == MK_QKV) return mvq_go<&mvq_kernel<MASK>>(A, g, threads, lds, st);
+  if constexpr ((MASK & (MASK - 1)) == 0) {   // (only the fused QKV launch mixes formats)
+    switch (kind) {
+      case MK_OUT: return mvq_go<&mvq_rows_kernel<MASK, MK_OUT>>(A, g, threads, lds, st);
+      case MK_PAIR: return mvq_go<&mvq_rows_kernel<MASK, MK_PAIR>>(A, g, threads, lds, st);
+      case MK_MOE_PAIR: return mvq_go<&mvq_rows_kernel<MASK, MK_MOE_PAIR>>(A, g, threads, lds, st);
+      case MK_MOE_DOWN: return mvq_go<&mvq_rows_kernel<MASK, MK_MOE_DOWN>>(A, g, threads, lds, st);
+      default: break;
+    }
+  }
+  return hipErrorInvalidValue;
+}
+
 hipError_t mvq_launch(const MvLaunch& L, uint32_t n_wg, uint32_t threads, hipStream_t st) {
   MvGeom g;
+  MvqArgs A;
   size_t lds = 0;
   const uint32_t mask = mvq_pack(L, n_wg, threads, &g, &lds);
-  const uint32_t wbpack = g.wbpack, geom = g.geom, geom2 = g.geom2, red_off = g.lds_red_off;
-#define LGH_MVQ_CASE(M) case M: return mvq_go<M>(L, n_wg, threads, lds, st, wbpack, geom, geom2, red_off)
+  const int kind = mask ? mvq_args(L, &A) : -1;
+  if (kind < 0) return hipErrorInvalidValue;
+#define LGH_MVQ_CASE(M) case M: return mvq_kind<M>(kind, A, g, threads, lds, st)
   switch (mask) {   // single formats and the two mixes of the "_M" quantisations (fused QKV: V in Q6_K)
     LGH_MVQ_CASE(1u << F_Q4K); LGH_MVQ_CASE(1u << F_Q6K); LGH_MVQ_CASE(1u << F_Q5K); LGH_MVQ_CASE(1u << F_Q80); LGH_MVQ_CASE(1u << F_Q40);
     LGH_MVQ_CASE((1u << F_Q4K) | (1u << F_Q6K)); LGH_MVQ_CASE((1u << F_Q5K) | (1u << F_Q6K));

@@ -47,6 +47,8 @@ __device__ __forceinline__ void mv_epilogue_prefetch_rope(int epi, uint32_t pos,
 // (matvec_batch.hip: every sequence has its own output, residual, XQ image, position and KV cache slot).
 struct MvEpiView { float* out; const float* resid; uint8_t* xq_out; float* xq_ssq; const int* pos; uint8_t* xw_out = nullptr; uint32_t xw_block = 0; };
 
+__device__ __forceinline__ float mv_inv_rms(float ss, uint32_t k, float eps) { return 1.0f / __builtin_sqrtf(ss / (float)k + eps); }
+
 // Per-row epilogue, one thread per row (or per row pair for RoPE)
 // `nslots` = partial sums per (pass, row) in `red`, laid out red[(p * nslots + slot) * rows_per_wg + row]
 __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg& S, const MvEpiView V, uint32_t wg, uint32_t rows_per_wg, const float* red,
@@ -58,7 +60,7 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
   if (L.do_norm) {  // simd.rs:853-855: rms = sqrt(ss/n + eps); inv = 1/rms
     float tot = 0.0f;
     for (uint32_t w = 0; w < (blockDim.x >> 6); w++) tot += ssq[w];
-    inv = 1.0f / __builtin_sqrtf(tot / (float)L.k + L.eps);
+    inv = mv_inv_rms(tot, L.k, L.eps);
   }
   auto rowval = [&](int p, uint32_t rl) {
     float v = 0.0f;

@@ -1,6 +1,6 @@
 // mvq_core.h — the tile-level core of the int8 matrix-core mat-vec (internal, device side): how one 16-row x 256-element
 // weight tile is requested from HBM and how it is multiplied with the XQ record of its 256 input elements.  Shared by
-// the launch-per-op kernel (matvec_mfma.hip: mvq_kernel) and the persistent token kernel (decode_persistent.hip), so both
+// the single-sequence kernels (matvec_mfma.hip) and the batched ones (matvec_batch.hip), so that both
 // produce the same bits for the same tile.  Formats, tile layouts and the arithmetic are described in matvec_mfma.hip.
 #pragma once
 
