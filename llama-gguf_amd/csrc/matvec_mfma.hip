@@ -325,7 +325,7 @@ constexpr int kDepth = 4;   // weight tiles a wave keeps in flight (4 x 2304 B x
 //     scalars delivered by KERNARG PRELOAD (SGPRs filled at wave launch: -mllvm -amdgpu-kernarg-preload-count=8) or read in two batches of
 //     scalar loads: what the first requests need in front of them, what the end needs while the tiles travel.  Read where they are used, behind the last
 //     barrier, the end's were a chain of ten waits.
-//   * x comes first, for the whole workgroup, one copy in LDS: a CU's loads return in the order they went out, and where every wave asks for its own slice of x in front of its tiles, the second four waves' slices
+//   * x comes first (behind one tile a wave), for the whole workgroup, one copy in LDS: a CU's loads return in the order they went out, and where every wave asks for its own slice of x in front of its tiles, the second four waves' slices
 //     come behind the first four's tiles, from HBM (stamps: 2.3 us after the start, the first four's 1.4).  The barrier between the two costs the 0.15 us that the second four start later.
 // Together (all epilogues in one kernel, every wave's own slice of x, scalars where they are used: before; now), logits to the host after every token: TinyLlama-1.1B Q4_K_M 40 rows 612 -> 535 us a token, Llama-3-8B
 // Q4_K_M 130 rows 1559 -> 1410, Q5_K_M over 3-bit codes (8 layers) 489 -> 450, Q8_0 3000 rows (8 layers) 570 -> 540, Mixtral Q5_K_M (3 layers) 284 -> 266; a launch of 4096 x 4096 ends 3.8 us after its start instead of 4.0 (median
@@ -541,9 +541,11 @@ __device__ __forceinline__ void mvq_body(uint32_t wbpack, uint32_t geom, uint32_
     }
   };
 
-  x_request(xq, 0);
-  if (KIND == MK_MOE_DOWN && S_npass > 1) x_request(xq1, xbytes);
-  meet();                                      // all of x is on its way: now the tiles
+  auto x_all = [&]() {
+    x_request(xq, 0);
+    if (KIND == MK_MOE_DOWN && S_npass > 1) x_request(xq1, xbytes);
+    meet();                                    // all of x is on its way: now the tiles
+  };
   {
     // Opaque to the optimizer (the values do not change): otherwise every shape's loop-invariant bookkeeping — ~300
     // scalar instructions, most of them for paths not taken — is hoisted in front of the first load.
@@ -580,11 +582,13 @@ __device__ __forceinline__ void mvq_body(uint32_t wbpack, uint32_t geom, uint32_
     // `run` for a static number of tiles put in flight up front; every path ends with nothing in flight
     auto run = [&](auto n_first) {
       constexpr int NF = decltype(n_first)::value;
+      at[0] = nx; issue(nx, buf[0]); advance();   // one tile in front of x: HBM is at work while x comes (8 layers of an 8B model 374.5 -> 371 us a token; two tiles 374, x is late then)
+      x_all();
 #pragma unroll
-      for (int j = 0; j < NF; j++) { at[j] = nx; issue(nx, buf[j]); advance(); }
+      for (int j = 1; j < NF; j++) { at[j] = nx; issue(nx, buf[j]); advance(); }
       LGH_WSTAMP(2);
       end_scalars();
-      x_finish(n_first);
+      x_finish(std::integral_constant<int, NF - 1>{});
       rotation();
       LGH_WSTAMP(5);
       if constexpr (NF < kDp) {   // that was everything
@@ -618,6 +622,7 @@ __device__ __forceinline__ void mvq_body(uint32_t wbpack, uint32_t geom, uint32_
           for (uint32_t tl = 0; tl < ntile_w; tl++)
             if (mq == 0) slot(p, tl) = 0.0f;
       }
+      x_all();
       end_scalars();
       x_finish(std::integral_constant<int, 0>{});
       rotation();
