@@ -223,7 +223,7 @@ hipError_t repack_launch(int src_type, const uint8_t* raw, uint8_t* dst, const u
                          hipStream_t st);
 hipError_t dequant_launch(int src_type, const uint8_t* raw, float* dst, uint64_t n_elems, hipStream_t st);
 // dequantize row `*token` of a [vocab][hidden] table in its NATIVE GGUF layout into dst (embedding lookup)
-hipError_t embed_launch(int src_type, const uint8_t* table, const int* token, float* dst, uint32_t hidden, int* state,
+hipError_t embed_launch(int src_type, const uint8_t* table, const int* token, int given, float* dst, uint32_t hidden, int* state,
                         uint8_t* xq, const float* xq_nw, float* xq_ssq, hipStream_t st);
 
 // misc kernels
@@ -250,6 +250,10 @@ hipError_t argmax_launch(const float* logits, uint32_t n, float* part_val, int* 
                          hipStream_t st);
 hipError_t advance_launch(int* state, hipStream_t st);
 hipError_t copy_words_launch(void* dst, const void* src, uint32_t n_words, hipStream_t st);
+// results on their way to the host (misc.hip): rows x cols floats, ld apart, to pinned memory, whose parts of kOutPart floats answer one by one
+constexpr uint32_t kOutPart = 16384;
+struct OutDev { uint32_t serial, parts_done, blocks_done[32]; };   // of a context, all zero at first; up to 32 parts a launch
+hipError_t results_out_launch(float* dst, const float* src, uint32_t cols, uint32_t ld, uint32_t rows, OutDev* dev, uint32_t* answer, hipStream_t st);
 hipError_t moe_group_launch(const int* sel, uint32_t n_seq, uint32_t top_k, uint32_t n_experts, int* cnt, int* idx, uint32_t idx_stride, hipStream_t st);
 hipError_t moe_combine_launch(const float* tmp, const float* moe_w, uint32_t top_k, float* hidden, uint32_t H, uint32_t n_seq, const float* nw,
                               uint8_t* xq, uint32_t xq_stride, float* ssq, uint32_t ssq_stride, hipStream_t st, uint8_t* xw = nullptr, uint32_t xw_block = 0);

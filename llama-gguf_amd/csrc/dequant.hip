@@ -153,7 +153,7 @@ hipError_t dequant_launch(int src_type, const uint8_t* raw, float* dst, uint64_t
 // Embedding lookup (llama.rs:293-307; gpu_only.rs:849-858): dst = dequantize(table row *token).
 // Thread 0 of block 0 also opens the token: state[POS] = state[NEXT]++ (every later kernel of this
 // token reads state[POS]; stream order makes the store visible).
-__global__ void __launch_bounds__(256) embed_kernel(int type, const uint8_t* __restrict__ table, const int* token,
+__global__ void __launch_bounds__(256) embed_kernel(int type, const uint8_t* __restrict__ table, const int* token, int given,
                                                     float* __restrict__ dst, uint32_t hidden, int* state,
                                                     uint8_t* __restrict__ xq, const float* __restrict__ xq_nw, float* __restrict__ xq_ssq) {
   LGH_TL_BEGIN(deq, lgh::TL_EMBED, hidden);
@@ -161,8 +161,9 @@ __global__ void __launch_bounds__(256) embed_kernel(int type, const uint8_t* __r
     int p = state[ST_NEXT];
     state[ST_POS] = p;
     state[ST_NEXT] = p + 1;
+    if (given >= 0) state[ST_TOKEN] = given;
   }
-  const uint64_t row = (uint64_t)(uint32_t)*token;
+  const uint64_t row = (uint64_t)(uint32_t)(given >= 0 ? given : *token);
   uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i < hidden) {
     const float v = deq_any(type, table, row * hidden + i);
@@ -173,10 +174,11 @@ __global__ void __launch_bounds__(256) embed_kernel(int type, const uint8_t* __r
   LGH_TL_END();
 }
 
-hipError_t embed_launch(int src_type, const uint8_t* table, const int* token, float* dst, uint32_t hidden, int* state,
+// given >= 0: that token (the host's), which goes to the state word, too
+hipError_t embed_launch(int src_type, const uint8_t* table, const int* token, int given, float* dst, uint32_t hidden, int* state,
                         uint8_t* xq, const float* xq_nw, float* xq_ssq, hipStream_t st) {
   if (!blk_elems(src_type) || (xq && hidden % 256)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(embed_kernel, dim3((hidden + 255) / 256), dim3(256), 0, st, src_type, table, token, dst, hidden,
+  hipLaunchKernelGGL(embed_kernel, dim3((hidden + 255) / 256), dim3(256), 0, st, src_type, table, token, given, dst, hidden,
                      state, xq, xq_nw, xq_ssq);
   return hipGetLastError();
 }

@@ -63,11 +63,16 @@ struct PfwScratch {
 };
 
 // pinned memory through which results reach the caller (engine.hip: floats_to_host)
-constexpr int kOutSlots = 4;
+constexpr size_t kOutFloats = 32 * lgh::kOutPart;
 struct HostOut {
-  float *pin = nullptr, *dev = nullptr;   // the same memory, as the host and as the device sees it
-  hipEvent_t ready[kOutSlots] = {};
-  bool refused = false;                   // there is none: the runtime's own copies
+  float *pin = nullptr, *dev = nullptr;   // the same memory, as the host and as the device sees it: the floats, then a word a part in which the device answers
+  lgh::OutDev* sync = nullptr;            // the device's own words
+  uint32_t number = 0;                    // launches so far
+  bool in_step = false;                   // the step that was launched last has one for its logits
+  bool in_graph[2] = {};                  // whether the graph of a step that the host feeds has one (by the attention variant)
+  bool refused = false;                   // there is no such memory: the runtime's own copies
+  const volatile uint32_t* answers() const { return reinterpret_cast<const volatile uint32_t*>(pin + kOutFloats); }
+  uint32_t* answers_dev() const { return reinterpret_cast<uint32_t*>(dev + kOutFloats); }
 };
 
 struct ProfRec { int cls; int sym; uint64_t bytes; hipEvent_t a, b; };
@@ -98,7 +103,8 @@ struct BatchScratch {
   int *moe_cnt = nullptr, *moe_idx = nullptr;
   std::vector<size_t> pos;                            // per slot: tokens in its cache
   bool attn_short = false;                            // attention of the step being enqueued: one launch (chosen by the longest sequence's position), or split and merge; the same bits
-  hipGraphExec_t graph[kMaxBatch + 1][2][2] = {};     // [n_seq][0 logits only, 1 + arg-max fed back][attn_short]
+  hipGraphExec_t graph[kMaxBatch + 1][2][2] = {};     // [n_seq][0 logits, which it brings to pinned memory where they fit, 1 + arg-max fed back][attn_short]
+  bool brings[kMaxBatch + 1][2] = {};                 // of the former: whether it does
 };
 
 struct LayeredModel;   // layered.hip: models described layer by layer
@@ -137,7 +143,7 @@ struct lgh_ctx {
   bool profiling = false;
   std::string err;
   uint32_t fail_alloc = 0;                         // lgh_debug_fail_alloc
-  hipGraphExec_t graph[lgh::MODE_COUNT][2] = {};   // [mode][attention variant: 0 split + combine, 1 single launch (short context)]
+  hipGraphExec_t graph[lgh::MODE_COUNT][2][2] = {};   // [mode][attention variant: 0 split + combine, 1 single launch (short context)][1: a step that the host feeds, see step()]
   bool attn_direct = false;                        // variant of the token being enqueued (chosen by the host-side position)
   uint32_t direct_attn_max_kv = 0;                 // contexts up to this many rows take the single-launch attention
   uint64_t graph_nodes = 0;
@@ -218,6 +224,9 @@ struct AtWork {
   AtWork& operator=(const AtWork&) = delete;
 };
 int floats_to_host(lgh_ctx* c, float* dst, const float* src, size_t cols, size_t ld, size_t rows);
+bool results_fit(const lgh_ctx* c, size_t n);                            // whether a step may bring n floats of results itself: ...
+int results_enqueue(lgh_ctx* c, const float* src, size_t n);             // ... its last launch (not counted yet: HostOut::number)
+int results_of_step(lgh_ctx* c, float* dst, const float* src, size_t n); // what the step that was launched last has at src
 // layered.hip, behind the entry points of engine.hip when c->lm is set
 int layered_upload(lgh_ctx* c, const char* name, uint32_t type, const uint64_t ne[4], const void* host, size_t nbytes);
 int layered_finalize(lgh_ctx* c);

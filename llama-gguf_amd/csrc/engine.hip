@@ -669,7 +669,8 @@ static int layer_forward(lgh_ctx* c, uint32_t li, const float* next_nw, bool nex
 }
 
 // the token's embedding row (or the hidden vector that the stage before left) and its position
-static int token_begin(lgh_ctx* c) {
+// `given`: the token, where the host has it (else it is the state word's).  launch = false: what the launch leaves is there already
+static int token_begin(lgh_ctx* c, int given = -1, bool launch = true) {
   const lgh_model_desc& d = c->d;
   int rc;
   for (auto& q : c->xqs) q.fresh = false;   // the residual stream is (re)written in f32 now (embedding / previous stage)
@@ -681,8 +682,8 @@ static int token_begin(lgh_ctx* c) {
       qh = xq_get(c, c->hidden, d.hidden_size);
       nw0 = c->layers[c->l0].attn_norm;
     }
-    if ((rc = run_k(c, LGH_K_EMBED, LGH_SYM_EMBED, (uint64_t)d.hidden_size * blk_bytes(c->embd_type) / blk_elems(c->embd_type), [&] {
-           return embed_launch(c->embd_type, c->embd_raw, c->state + ST_TOKEN, c->hidden, d.hidden_size, c->state,
+    if (launch && (rc = run_k(c, LGH_K_EMBED, LGH_SYM_EMBED, (uint64_t)d.hidden_size * blk_bytes(c->embd_type) / blk_elems(c->embd_type), [&] {
+           return embed_launch(c->embd_type, c->embd_raw, c->state + ST_TOKEN, given, c->hidden, d.hidden_size, c->state,
                                qh ? qh->xq : nullptr, nw0, qh ? qh->ssq : nullptr, c->stream);
          })))
       return rc;
@@ -732,14 +733,42 @@ static int token_end(lgh_ctx* c, int mode) {
   return LGH_OK;
 }
 
-// Everything one token needs, in stream order.  Used eagerly and under graph capture.
-static int enqueue_token(lgh_ctx* c, int mode) {
+// Everything one token needs, in stream order.  Used eagerly and under graph capture.  begun: its first launch is there already
+static int enqueue_token(lgh_ctx* c, int mode, bool begun = false) {
   if (c->lm) return layered_enqueue_token(c, mode);
   int rc;
-  if ((rc = token_begin(c))) return rc;
+  if ((rc = token_begin(c, -1, !begun))) return rc;
   for (uint32_t li = c->l0; li < c->l1; li++)
     if ((rc = token_layer(c, li, mode))) return rc;
   return token_end(c, mode);
+}
+
+// Results' way to the caller (see floats_to_host): the context's pinned memory
+static bool out_ensure(lgh_ctx* c) {
+  HostOut& O = c->out;
+  if (O.pin) return true;
+  if (O.refused) return false;
+  if (hipHostMalloc((void**)&O.pin, kOutFloats * 4 + 32 * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) { O.pin = nullptr; O.refused = true; }
+  if (!O.refused && hipHostGetDevicePointer((void**)&O.dev, O.pin, 0) != hipSuccess) O.refused = true;
+  if (!O.refused && hipMalloc((void**)&O.sync, sizeof(OutDev)) != hipSuccess) { O.sync = nullptr; O.refused = true; }
+  if (!O.refused && (hipMemsetAsync(O.sync, 0, sizeof(OutDev), c->stream) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)) O.refused = true;
+  if (O.refused) {
+    if (O.sync) (void)hipFree(O.sync);
+    if (O.pin) (void)hipHostFree(O.pin);
+    O.sync = nullptr; O.pin = nullptr;
+    (void)hipGetLastError();   // (the next launch's check would find it)
+    return false;
+  }
+  std::memset(O.pin + kOutFloats, 0, 32 * 4);
+  return true;
+}
+// whether a step that the host feeds takes its token as a launch's argument, and brings its logits itself
+static bool given_tokens(const lgh_ctx* c) { return c->first && !c->lm; }
+bool results_fit(const lgh_ctx* c, size_t n) { return c->out.pin && n && n <= kOutFloats; }
+static bool step_brings_logits(const lgh_ctx* c) { return c->last && results_fit(c, c->d.vocab_size); }
+int results_enqueue(lgh_ctx* c, const float* src, size_t n) {
+  HIP_TRY(c, LGH_OPERATION_FAILED, results_out_launch(c->out.dev, src, (uint32_t)n, (uint32_t)n, 1, c->out.sync, c->out.answers_dev(), c->stream));
+  return LGH_OK;
 }
 
 // One token through the context's kernels, launched eagerly, before any of them is first launched inside a stream
@@ -763,24 +792,31 @@ static int warm_kernels(lgh_ctx* c) {
   c->attn_direct = keep_direct;
   for (auto& q : c->xqs) q.fresh = false;
   if (rc) return rc;
+  if (step_brings_logits(c)) {
+    if ((rc = results_enqueue(c, c->logits, c->d.vocab_size))) return rc;
+    c->out.number++;
+  }
   HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetAsync(c->state, 0, ST_WORDS * 4, c->stream));
   HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
   return LGH_OK;
 }
 
-static int ensure_graph(lgh_ctx* c, int mode) {
-  const int var = c->attn_direct ? 1 : 0;
-  if (c->graph[mode][var]) return LGH_OK;
+static int ensure_graph(lgh_ctx* c, int mode, bool fed = false) {
+  hipGraphExec_t& ge = c->graph[mode][c->attn_direct ? 1 : 0][fed ? 1 : 0];
+  if (ge) return LGH_OK;
   hipGraph_t g = nullptr;
   HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  int rc = enqueue_token(c, mode);
+  int rc = enqueue_token(c, mode, fed && given_tokens(c));
+  const bool brings = fed && mode == MODE_FORWARD && step_brings_logits(c);
+  if (!rc && brings) rc = results_enqueue(c, c->logits, c->d.vocab_size);
+  if (fed && mode == MODE_FORWARD) c->out.in_graph[c->attn_direct ? 1 : 0] = brings;
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
   if (e != hipSuccess) return fail(c, LGH_OPERATION_FAILED, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
   size_t n_nodes = 0;
   (void)hipGraphGetNodes(g, nullptr, &n_nodes);
   if (mode == MODE_GREEDY || c->graph_nodes == 0) c->graph_nodes = n_nodes;
-  e = hipGraphInstantiate(&c->graph[mode][var], g, nullptr, nullptr, 0);
+  e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e != hipSuccess) return fail(c, LGH_OPERATION_FAILED, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   return LGH_OK;
@@ -793,18 +829,32 @@ static uint32_t direct_attn_rows(const lgh_ctx* c) {
   return kv_is_tq(c->d.kv_cache_type) && c->d.max_seq_len <= c->direct_attn_max_kv ? c->direct_attn_max_kv : 0;
 }
 
-// run one token in `mode` (token id already in the device state)
-static int step(lgh_ctx* c, int mode) {
+static int set_token(lgh_ctx* c, uint32_t token) {
+  if (c->first && token >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");  // llama.rs:296-302
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_TOKEN), (int)token, 1, c->stream));
+  return LGH_OK;
+}
+
+// run one token in `mode`: the state word's, or the host's (`token`).  A step that the host feeds has the token in the arguments of its first launch, which is not part of the graph then (a fill in front of the graph was
+// 3 us, and 4 until the graph began), and its logits go to the pinned memory with its last one (a launch behind a graph begins 9 to 12 us after it, one inside 1.5).
+static int step(lgh_ctx* c, int mode, const uint32_t* token = nullptr) {
+  c->out.in_step = false;
+  const bool graphs = !c->profiling && !(c->d.flags & LGH_FLAG_NO_GRAPH);
+  if (token && c->first && *token >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");  // llama.rs:296-302
   if (c->pos >= c->d.max_seq_len)  // the reference has no such check: OOB write past the KV capacity
     return fail(c, LGH_INVALID_ARGUMENT, "position " + std::to_string(c->pos) + " >= max_seq_len " + std::to_string(c->d.max_seq_len));
   int rc;
   c->attn_direct = c->pos + 1 <= direct_attn_rows(c);   // the token at position pos attends to pos + 1 rows
-  if (c->profiling || (c->d.flags & LGH_FLAG_NO_GRAPH)) {
+  if (!graphs) {
+    if (token && (rc = set_token(c, *token))) return rc;
     if ((rc = enqueue_token(c, mode))) return rc;
     if (c->profiling && (rc = drain_prof(c))) return rc;
   } else {
-    if ((rc = ensure_graph(c, mode))) return rc;
-    HIP_TRY(c, LGH_OPERATION_FAILED, hipGraphLaunch(c->graph[mode][c->attn_direct ? 1 : 0], c->stream));
+    const bool fed = token != nullptr;
+    if ((rc = ensure_graph(c, mode, fed))) return rc;
+    if (fed && (rc = given_tokens(c) ? token_begin(c, (int)*token) : set_token(c, *token))) return rc;
+    HIP_TRY(c, LGH_OPERATION_FAILED, hipGraphLaunch(c->graph[mode][c->attn_direct ? 1 : 0][fed ? 1 : 0], c->stream));
+    if (fed && mode == MODE_FORWARD && c->out.in_graph[c->attn_direct ? 1 : 0]) { c->out.in_step = true; c->out.number++; }
   }
   c->pos += 1;
   c->stats.tokens_processed += 1;
@@ -813,8 +863,9 @@ static int step(lgh_ctx* c, int mode) {
 
 static void drop_graphs(lgh_ctx* c) {
   for (int m = 0; m < MODE_COUNT; m++)
-    for (int v = 0; v < 2; v++)
-      if (c->graph[m][v]) { (void)hipGraphExecDestroy(c->graph[m][v]); c->graph[m][v] = nullptr; }
+    for (auto& gv : c->graph[m])
+      for (auto& ge : gv)
+        if (ge) { (void)hipGraphExecDestroy(ge); ge = nullptr; }
   for (auto& gg : c->batch.graph)
     for (auto& gs : gg)
       for (auto& ge : gs)
@@ -823,75 +874,97 @@ static void drop_graphs(lgh_ctx* c) {
 
 static int bind(const lgh_ctx* c) { return hipSetDevice(c->device) == hipSuccess ? LGH_OK : LGH_NOT_AVAILABLE; }
 
-static int set_token(lgh_ctx* c, uint32_t token) {
-  if (c->first && token >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");  // llama.rs:296-302
-  HIP_TRY(c, LGH_OPERATION_FAILED, hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_TOKEN), (int)token, 1, c->stream));
-  return LGH_OK;
-}
-
 // ------------------------------------------------------------------------------------------------
 // results to the caller's memory
 // ------------------------------------------------------------------------------------------------
 // A copy to ordinary host memory through the runtime starts when the work before it has ended, moves a MiB at a time to a buffer of the runtime's and waits for each.  Here a kernel behind that
-// work, in the same queue, writes pieces to pinned memory of the context, and the host takes each to the caller while the next ones are on their way.  Behind a kernel of 88 us, until the caller has
-// them, us, the runtime's copy and this one: 32000 floats 154 and 94, 128 256: 309 and 111, 512 000: 212 and 169 (179 in pieces of half the size, 226 in quarters: an event between two kernels is some 8 us).
-constexpr size_t kOutPiece = 128 * 1024;   // floats
-static bool out_ensure(lgh_ctx* c) {
+// work, in the same queue, writes to pinned memory of the context, and the host takes each part to the caller as its answer arrives, while the next ones are on their way.  A step that the host feeds has that kernel as its
+// last one, and is over for the host when the last part has answered: no launch and no event of its own, no wait for the stream.  From the head's end to the next token's first kernel 70 us -> 35 (32000 floats); logits to the
+// host after every token, before; now: TinyLlama-1.1B 40 rows 530 -> 515 us, Llama-3-8B (8 layers) 371 -> 360, Mixtral (3 layers) 265 -> 252; five sequences of Mixtral (2 layers) 541 -> 523 a step; 16 sequences of the 8B model (8 layers,
+// 2 MB a step) as before: there the host's copy is what takes the time, 16 GB/s.
+// n floats to the caller's memory that launch number `number` brought to the parts from `first` on
+static int results_take(lgh_ctx* c, float* dst, size_t n, uint32_t number, uint32_t first) {
   HostOut& O = c->out;
-  if (O.pin) return true;
-  if (O.refused) return false;
-  for (auto& e : O.ready)
-    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) O.refused = true;
-  if (!O.refused && hipHostMalloc((void**)&O.pin, kOutPiece * kOutSlots * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) { O.pin = nullptr; O.refused = true; }
-  if (!O.refused && hipHostGetDevicePointer((void**)&O.dev, O.pin, 0) != hipSuccess) { (void)hipHostFree(O.pin); O.pin = nullptr; O.refused = true; }
-  if (O.refused) (void)hipGetLastError();   // (the next launch's check would find it)
-  return !O.refused;
+  // A result of many parts in pieces of 512 KB: the device is ahead of the host's copy from the second on, and a large copy runs at 20 GB/s, parts of 64 KB at 16.
+  const size_t last = first + (n + kOutPart - 1) / kOutPart, group = n > 16 * (size_t)kOutPart ? 8 : 1;
+  for (size_t part = first; part < last; part += group) {
+    const size_t end = std::min(part + group, last);
+    for (size_t i = part; i < end; i++) {
+      for (uint32_t turn = 1; O.answers()[i] != number; turn++) {
+        __builtin_ia32_pause();
+        if (turn % 4096) continue;
+        // now and then: whether the work is still going on (a launch that was lost leaves no answer)
+        const hipError_t e = hipStreamQuery(c->stream);
+        if (e == hipErrorNotReady) continue;
+        HIP_TRY(c, LGH_OPERATION_FAILED, e);
+        if (O.answers()[i] != number) return fail(c, LGH_OPERATION_FAILED, "results did not arrive");
+      }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    const size_t at = (part - first) * kOutPart;
+    std::memcpy(dst + at, O.pin + part * kOutPart, std::min((end - part) * (size_t)kOutPart, n - at) * 4);
+  }
+  return LGH_OK;
+}
+
+// The caller's pages, while the device works: a caller that keeps its results has the next one on fresh pages, whose faults would come between the parts (steps of 16 sequences, 4 layers of an 8B model,
+// all 40 results kept: 1008 us a step without this, 683 with it, 634 on used pages).
+// Adding nothing leaves them as they are until the result is there, also where there will be none.
+static void results_touch(float* dst, size_t n) {
+  const volatile uint8_t nothing = 0;   // (the compiler makes a fence and a read of an addition of a 0 that it knows)
+  for (size_t at_byte = 0; at_byte < n * 4; at_byte += 4096) __atomic_fetch_add(reinterpret_cast<uint8_t*>(dst) + at_byte, nothing, __ATOMIC_RELAXED);
+}
+
+static bool results_ordinary(const float* dst) {   // not memory that the device reaches itself
+  hipPointerAttribute_t at;
+  const bool ordinary = hipPointerGetAttributes(&at, dst) != hipSuccess || at.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();   // (what the question about ordinary memory may leave)
+  return ordinary;
 }
 
 // `rows` rows of `cols` floats, `ld` apart, to dst, behind what c->stream holds; returns when they and all of that are there
 int floats_to_host(lgh_ctx* c, float* dst, const float* src, size_t cols, size_t ld, size_t rows) {
-  hipPointerAttribute_t at;
-  const bool ordinary = hipPointerGetAttributes(&at, dst) != hipSuccess || at.type == hipMemoryTypeUnregistered;
-  (void)hipGetLastError();   // (what the question about ordinary memory may leave)
-  if (!ordinary || !out_ensure(c)) {   // memory that the device reaches itself
+  if (!results_ordinary(dst) || !out_ensure(c)) {
     HIP_TRY(c, LGH_OPERATION_FAILED, hipMemcpy2DAsync(dst, cols * 4, src, ld * 4, cols * 4, rows, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
     return LGH_OK;
   }
   HostOut& O = c->out;
-  if (ld == cols) { cols *= rows; ld = cols; rows = 1; }
-  const size_t per_row = (cols + kOutPiece - 1) / kOutPiece, n = per_row * rows;
-  auto piece = [&](size_t i, size_t& from, size_t& to, size_t& len) {
-    const size_t r = i / per_row, at0 = (i - r * per_row) * kOutPiece;
-    from = r * ld + at0;
-    to = r * cols + at0;
-    len = std::min(kOutPiece, cols - at0);
+  if (ld == cols) { cols *= rows; ld = cols; rows = cols ? 1 : 0; }
+  // launches of what fits: all of the memory for one, halves in turn for more
+  const size_t cap = cols * rows <= kOutFloats ? kOutFloats : kOutFloats / 2;
+  const size_t in_row = cols ? (cols + cap - 1) / cap : 0, per = in_row == 1 ? std::min(rows, cap / cols) : 1;   // launches of a row, rows of a launch
+  const size_t n = per ? (rows + per - 1) / per * in_row : 0;
+  struct Piece { size_t from, to, cols, rows; };
+  auto piece = [&](size_t i) {
+    const size_t r = i / in_row * per, at0 = i % in_row * cap;
+    return Piece{r * ld + at0, r * cols + at0, std::min(cap, cols - at0), std::min(per, rows - r)};
   };
+  const uint32_t base = O.number;
   auto request = [&](size_t i) -> int {
-    size_t from, to, len;
-    piece(i, from, to, len);
-    HIP_TRY(c, LGH_OPERATION_FAILED, copy_words_launch(O.dev + i % kOutSlots * kOutPiece, src + from, (uint32_t)len, c->stream));
-    if (i + 1 < n) HIP_TRY(c, LGH_OPERATION_FAILED, hipEventRecord(O.ready[i % kOutSlots], c->stream));
+    const Piece p = piece(i);
+    const uint32_t first = (uint32_t)(i % 2 * cap / kOutPart) * (n > 1);
+    HIP_TRY(c, LGH_OPERATION_FAILED, results_out_launch(O.dev + first * kOutPart, src + p.from, (uint32_t)p.cols, p.rows > 1 ? (uint32_t)ld : (uint32_t)p.cols, (uint32_t)p.rows, O.sync, O.answers_dev() + first, c->stream));
+    O.number++;
     return LGH_OK;
   };
   int rc;
-  for (size_t i = 0; i < std::min<size_t>(n, kOutSlots); i++)
+  for (size_t i = 0; i < std::min<size_t>(n, 2); i++)
     if ((rc = request(i))) return rc;
-  // the caller's pages, while the device works: a caller that keeps its results has the next one on fresh pages, whose faults would come between the pieces (steps of 16 sequences, 4 layers of an 8B model,
-  // all 40 results kept: 1008 us a step without this, 683 with it, 634 on used pages)
-  // Adding nothing leaves them as they are until the result is there, also where there will be none.
-  const volatile uint8_t nothing = 0;   // (the compiler makes a fence and a read of an addition of a 0 that it knows)
-  for (size_t at_byte = 0; at_byte < cols * rows * 4; at_byte += 4096) __atomic_fetch_add(reinterpret_cast<uint8_t*>(dst) + at_byte, nothing, __ATOMIC_RELAXED);
+  results_touch(dst, cols * rows);
   for (size_t i = 0; i < n; i++) {
-    size_t from, to, len;
-    piece(i, from, to, len);
-    if (i + 1 < n) HIP_TRY(c, LGH_OPERATION_FAILED, hipEventSynchronize(O.ready[i % kOutSlots]));
-    else HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
-    std::memcpy(dst + to, O.pin + i % kOutSlots * kOutPiece, len * 4);
-    if (i + kOutSlots < n && (rc = request(i + kOutSlots))) return rc;   // (its slot has been read)
+    const Piece p = piece(i);
+    if ((rc = results_take(c, dst + p.to, p.cols * p.rows, base + 1 + (uint32_t)i, (uint32_t)(i % 2 * cap / kOutPart) * (n > 1)))) return rc;
+    if (i + 2 < n && (rc = request(i + 2))) return rc;   // (its half has been read)
   }
-  if (!n) HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
+  if (!n) HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));   // (else the last answer came from behind everything else)
   return LGH_OK;
+}
+
+int results_of_step(lgh_ctx* c, float* dst, const float* src, size_t n) {
+  if (!c->out.in_step || !results_ordinary(dst)) return floats_to_host(c, dst, src, n, n, 1);
+  results_touch(dst, n);
+  return results_take(c, dst, n, c->out.number, 0);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1652,7 +1725,7 @@ int lgh_finalize(lgh_ctx* c) {
     if ((rc = layered_finalize(c))) return rc;
     c->finalized = true;
     c->pos = 0;
-    (void)out_ensure(c);
+    (void)out_ensure(c);   // (0.4 ms that the first result would wait for)
     return warm_kernels(c);
   }
   if (c->first && !c->embd_raw) return fail(c, LGH_INITIALIZATION_FAILED, "missing token_embd.weight");
@@ -1810,18 +1883,18 @@ int lgh_finalize(lgh_ctx* c) {
   HIP_TRY(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
   c->finalized = true;
   c->pos = 0;
-  if ((rc = warm_kernels(c))) return rc;
   if (c->last) (void)out_ensure(c);   // (0.4 ms that the first result would wait for)
-  return LGH_OK;
+  return warm_kernels(c);
 }
 
 void lgh_destroy(lgh_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  for (int m = 0; m < MODE_COUNT; m++)
-    for (int v = 0; v < 2; v++)
-      if (c->graph[m][v]) (void)hipGraphExecDestroy(c->graph[m][v]);
+  for (auto& gm : c->graph)
+    for (auto& gv : gm)
+      for (auto& ge : gv)
+        if (ge) (void)hipGraphExecDestroy(ge);
   for (auto& r : c->prof) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
   for (void* p : c->allocs) (void)hipFree(p);
   for (auto& gg : c->batch.graph)
@@ -1831,8 +1904,7 @@ void lgh_destroy(lgh_ctx* c) {
   if (c->pf.tok_pinned) (void)hipHostFree(c->pf.tok_pinned);
   if (c->pf.tok_copied) (void)hipEventDestroy(c->pf.tok_copied);
   if (c->out.pin) (void)hipHostFree(c->out.pin);
-  for (auto& e : c->out.ready)
-    if (e) (void)hipEventDestroy(e);
+  if (c->out.sync) (void)hipFree(c->out.sync);
   side_leave(c);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   layered_destroy(c);
@@ -1852,17 +1924,15 @@ int lgh_forward(lgh_ctx* c, uint32_t token, float* logits_out) {
   if (!logits_out) return fail(c, LGH_INVALID_ARGUMENT, "logits_out is NULL");
   if (!c->first || !c->last) return fail(c, LGH_INVALID_ARGUMENT, "lgh_forward needs a single-stage context; use lgh_stage_forward");
   const AtWork call(c);
-  if ((rc = set_token(c, token))) return rc;
-  if ((rc = step(c, MODE_FORWARD))) return rc;
-  return floats_to_host(c, logits_out, c->logits, c->d.vocab_size, c->d.vocab_size, 1);
+  if ((rc = step(c, MODE_FORWARD, &token))) return rc;
+  return results_of_step(c, logits_out, c->logits, c->d.vocab_size);
 }
 
 int lgh_prefill_token(lgh_ctx* c, uint32_t token) {
   int rc = check_ready(c);
   if (rc) return rc;
   if (!c->first || !c->last) return fail(c, LGH_INVALID_ARGUMENT, "lgh_prefill_token needs a single-stage context");
-  if ((rc = set_token(c, token))) return rc;
-  return step(c, MODE_PREFILL);
+  return step(c, MODE_PREFILL, &token);
 }
 
 int lgh_prefill_is_batched(lgh_ctx* c) { return c && c->finalized && (c->lm ? layered_has_blocks(c) : pf_eligible(c)) ? 1 : 0; }
@@ -1919,17 +1989,18 @@ static int eval_stretch(lgh_ctx* c, const uint32_t* tokens, size_t n, uint32_t t
   const bool beside = call.alone && tail_reaches(c, n);
   if (beside) HIP_TRY(c, LGH_OPERATION_FAILED, side_ask(c));
   int rc = prefill_tokens(c, tokens, n, beside ? &t : nullptr);
-  if (!rc && !t.taken && !(rc = set_token(c, token))) rc = step(c, MODE_FORWARD);
+  c->out.in_step = false;
+  if (!rc && !t.taken) rc = step(c, MODE_FORWARD, &token);
   // the step that the next token takes, captured while the device works where it is not there yet: a first token behind a first prompt would wait for it (8B model 2.6 ms
   // instead of 1.57, its prompt of 128 tokens 6.0 either way)
-  if (!rc) rc = ensure_graph(c, MODE_FORWARD);
+  if (!rc) rc = ensure_graph(c, MODE_FORWARD, true);
   if (rc) {
     if (beside) (void)hipStreamSynchronize(c->side_stream);   // nothing of the call goes on behind its error, and the next token's position is the one behind what is there
     (void)hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, c->stream);
     (void)hipStreamSynchronize(c->stream);
     return rc;
   }
-  return floats_to_host(c, logits_out, c->logits, c->d.vocab_size, c->d.vocab_size, 1);
+  return results_of_step(c, logits_out, c->logits, c->d.vocab_size);
 }
 
 int lgh_beside_blocks(lgh_ctx* c, int* possible, uint64_t* count) {

@@ -465,6 +465,7 @@ size_t short_attn_rows(const lgh_ctx* c, uint32_t n_seq) {
 int run_multi(lgh_ctx* c, uint32_t n_seq, bool greedy, size_t longest) {
   BatchScratch& Bs = c->batch;
   Bs.attn_short = longest + 1 <= short_attn_rows(c, n_seq);
+  c->out.in_step = false;
   if (c->profiling || (c->d.flags & LGH_FLAG_NO_GRAPH)) {
     int rc = enqueue_multi(c, n_seq, greedy);
     if (rc) return rc;
@@ -475,6 +476,10 @@ int run_multi(lgh_ctx* c, uint32_t n_seq, bool greedy, size_t longest) {
     hipGraph_t g = nullptr;
     HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_multi(c, n_seq, greedy);
+    const size_t n_out = (size_t)n_seq * c->d.vocab_size;
+    const bool brings = !greedy && results_fit(c, n_out);   // (behind the graph it would begin 9 us later)
+    if (!rc && brings) rc = results_enqueue(c, Bs.logits, n_out);
+    if (!greedy) Bs.brings[n_seq][Bs.attn_short ? 1 : 0] = brings;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
     if (e != hipSuccess) return fail(c, LGH_OPERATION_FAILED, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
@@ -483,6 +488,7 @@ int run_multi(lgh_ctx* c, uint32_t n_seq, bool greedy, size_t longest) {
     if (e != hipSuccess) return fail(c, LGH_OPERATION_FAILED, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   }
   HIP_TRYB(c, LGH_OPERATION_FAILED, hipGraphLaunch(ge, c->stream));
+  if (!greedy && Bs.brings[n_seq][Bs.attn_short ? 1 : 0]) { c->out.in_step = true; c->out.number++; }
   return LGH_OK;
 }
 
@@ -647,9 +653,9 @@ int lgh_forward_multi(lgh_ctx* c, const uint32_t* slots, const uint32_t* tokens,
   if ((rc = stage_control(c, slots, tokens, n_seq))) return rc;
   if ((rc = run_multi(c, n_seq, next_tokens != nullptr, longest_of(c, slots, n_seq)))) return rc;
   BatchScratch& Bs = c->batch;
-  if (logits_out && (rc = floats_to_host(c, logits_out, Bs.logits, (size_t)n_seq * c->d.vocab_size, (size_t)n_seq * c->d.vocab_size, 1))) return rc;
+  if (logits_out && (rc = results_of_step(c, logits_out, Bs.logits, (size_t)n_seq * c->d.vocab_size))) return rc;
   if (next_tokens) HIP_TRYB(c, LGH_OPERATION_FAILED, hipMemcpyAsync(next_tokens, Bs.d_tokens, (size_t)n_seq * 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));
+  if (next_tokens || !logits_out) HIP_TRYB(c, LGH_OPERATION_FAILED, hipStreamSynchronize(c->stream));   // (the logits came from behind everything else)
   for (uint32_t i = 0; i < n_seq; i++) Bs.pos[slots[i]] += 1;
   c->stats.tokens_processed += n_seq;
   return LGH_OK;

@@ -339,8 +339,7 @@ hipError_t moe_combine_launch(const float* tmp, const float* moe_w, uint32_t top
   return hipGetLastError();
 }
 
-// same-device pipeline hop (hidden vector / token word) as a graph node of the producing stage; results on their way to pinned host memory.  (One word a lane: a wave's store is
-// 256 bytes either way, and neither side need be aligned to more.)
+// same-device pipeline hop (hidden vector / token word) as a graph node of the producing stage
 __global__ void copy_words_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
@@ -348,6 +347,55 @@ __global__ void copy_words_kernel(uint32_t* __restrict__ dst, const uint32_t* __
 
 hipError_t copy_words_launch(void* dst, const void* src, uint32_t n, hipStream_t st) {
   hipLaunchKernelGGL(copy_words_kernel, dim3((n + 255) / 256), dim3(256), 0, st, (uint32_t*)dst, (const uint32_t*)src, n);
+  return hipGetLastError();
+}
+
+// A word to memory that the host looks at: written through, so that it is there when the store has been acknowledged.
+__device__ __forceinline__ void store_out(float* p, float v) { __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+
+// Results to pinned host memory, in parts of kOutPart floats: the last workgroup of a part writes the launch's number behind it, so that the host takes the part while the next ones are on their way, without an event
+// and a launch of its own for each (an event between two kernels is some 8 us).  Bound by the host's side of the link, 55 GB/s.  One word a lane: a wave's store is 256 bytes either way, and neither side need be
+// aligned to more.
+constexpr uint32_t kOutBlock = 1024;    // floats of a workgroup's turn
+constexpr uint32_t kOutGroups = 128;    // workgroups at most: eight parts under way at a time, so that the first ones are there first (all 512 of 2 MB at once share the link, and every part answers at the end)
+static_assert(kOutPart % kOutBlock == 0, "");
+__global__ void __launch_bounds__(256) results_out_kernel(float* __restrict__ dst, const float* __restrict__ src, uint32_t cols, uint32_t ld, uint32_t n, OutDev* dev, uint32_t* answer) {
+  const uint32_t number = __hip_atomic_load(&dev->serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;   // (raised by the launch's last workgroup, behind everybody's look)
+  const uint32_t parts = (n + kOutPart - 1) / kOutPart;
+  for (uint64_t at = (uint64_t)blockIdx.x * kOutBlock; at < n; at += (uint64_t)gridDim.x * kOutBlock) {
+    const uint32_t b0 = (uint32_t)at;
+    if (ld == cols) {
+#pragma unroll
+      for (uint32_t j = 0; j < kOutBlock / 256; j++) {
+        const uint32_t i = b0 + j * 256 + threadIdx.x;
+        if (i < n) store_out(dst + i, src[i]);
+      }
+    } else {
+      for (uint32_t j = 0; j < kOutBlock / 256; j++) {
+        const uint32_t i = b0 + j * 256 + threadIdx.x;
+        if (i < n) { const uint32_t r = i / cols; store_out(dst + i, src[(size_t)r * ld + (i - r * cols)]); }
+      }
+    }
+    // Every store has been acknowledged.  (A fence for the whole system would write back all that is dirty in the XCD's L2, for each of the workgroups.)
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    __syncthreads();
+    if (threadIdx.x) continue;
+    const uint32_t part = b0 / kOutPart, blocks = (min(n - part * kOutPart, kOutPart) + kOutBlock - 1) / kOutBlock;
+    if (__hip_atomic_fetch_add(&dev->blocks_done[part], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != blocks) continue;
+    __hip_atomic_store(&dev->blocks_done[part], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_fetch_add(&dev->parts_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == parts) {   // the last answer says, too, that the device's words are the next launch's, on whichever stream
+      __hip_atomic_store(&dev->parts_done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&dev->serial, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    __hip_atomic_store(&answer[part], number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+hipError_t results_out_launch(float* dst, const float* src, uint32_t cols, uint32_t ld, uint32_t rows, OutDev* dev, uint32_t* answer, hipStream_t st) {
+  const uint64_t n = (uint64_t)cols * rows;
+  if (n == 0 || n > 32ull * kOutPart || ld < cols) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(results_out_kernel, dim3(std::min<uint32_t>(kOutGroups, (uint32_t)((n + kOutBlock - 1) / kOutBlock))), dim3(256), 0, st, dst, src, cols, ld, (uint32_t)n, dev, answer);
   return hipGetLastError();
 }
 
