@@ -233,8 +233,8 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb_kernel(uint32_t wbpack, uin
 //                 (Mvqb2Geom::fuse), else through the partial buffer;
 //   SEQ  = false  (matrices with too few units to fill the chip that way: wo, down, QKV) blockIdx.y = the slice; p_ks goes to
 //                 the partial buffer (nslots = T) and the epilogue adds them in slice order.
-// Otherwise a second, small launch (mvqb2_epilogue_kernel) loads the partial sums into LDS in the layout the single-sequence
-// epilogue reads and runs exactly that epilogue per sequence — every sequence's result is bit-identical to matvec_mfma.hip's.
+// Otherwise a second, small launch (mvqb_rows_kernel) adds the partial sums up in that order and does what the single-sequence
+// epilogue does — every sequence's result is bit-identical to matvec_mfma.hip's.
 // ================================================================================================
 struct Mvqb2Geom {
   uint32_t T, nbw, nblk;      // the single-sequence kernel's k-slices
@@ -912,86 +912,140 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
   }
 }
 
-// grid / block = the single-sequence geometry of `L` (segments' wg_begin, rows_per_wg).  dynamic LDS: mvqb_lds_bytes(n_seq, L.red_floats)
-// FEW: up to four sequences whose rows in a workgroup are one a thread at most (mvqb2_epilogue_few): loaded as they are, divided into quads they take longer than they save
-// (a step, 32 layers of an 8B model, 2 / 4 sequences: 2.545 / 2.850 ms in quads, 2.486 / 2.822 here)
-template <bool FEW>
-__global__ void __launch_bounds__(kBWaves * 64) mvqb2_epilogue_kernel(uint32_t wbpack, uint32_t geom, uint32_t geom2, uint32_t red_floats,
-                                                                      const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B,
-                                                                      const float* __restrict__ part) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
-  const uint32_t bid = blockIdx.x;
-  const int sg = (int)(bid >= (wbpack & 0xFFFFu)) + (int)(bid >= (wbpack >> 16));
-  const MvSeg& S = L.seg[sg];
-  const uint32_t S_G = (geom >> 8) & 0xFFu;
-  const bool nrm = (geom >> 31) != 0;
-  const uint32_t Rg = L.nseg > 1 ? S.rows_per_wg >> (4 + __builtin_ctz(S_G)) : geom2 >> 16;
-  const uint32_t S_rpw = 16u * Rg * S_G;
-  const uint32_t wg = bid - S.wg_begin;
-  uint32_t n_seq = B.n_seq;
+// ------------------------------------------------------------------------------------------------
+// The epilogue of a launch whose partial sums went through memory: per row and sequence the sum over the slices, then what mv_epilogue_view does with it.  Workgroups are the single-sequence geometry's.
+// A launch of this size is nothing but latency, so it is one chain: a thread has one (sequence, row), everything it will need (partial sums, residual, the next norm's weight, position and slot, the rotation) is
+// requested at once, the sum is made in registers, and what a launch does with its rows is compiled in.  No LDS, and no barrier but for the norm's factors.  (Before, the partial sums went through LDS and everything
+// else was asked for behind their barrier: 5.7 to 6.2 us a launch at 16 sequences of an 8B model, now 5.0, of which an empty launch is 1.5 to 2; prompts and 24 steps of 8 layers 37.9 -> 36.8 ms, five sequences of
+// Mixtral, two layers, 24 steps 12.30 -> 12.15.)
+// ------------------------------------------------------------------------------------------------
+enum : int { ER_OUT = 0, ER_PAIR = 1, ER_QKV = 2 };   // store / + residual; SwiGLU; RoPE, caches and what is stored beside them
+struct MvqbRowsSeg {
+  float* out;
+  const float *resid, *nw, *bias;
+  uint8_t* xq;
+  float* ssq;
+  uint8_t* xw;
+  uint32_t n_rows, wg_begin, rows, unit_begin;   // rows: of a workgroup
+  uint32_t out_stride, resid_stride, xq_stride, ssq_stride;
+  uint32_t epi, head_dim, max_seq, pad;
+};
+struct MvqbRows {
+  const float *part, *ssq_part, *rope_cs;
+  const int *pos, *slot, *ind_cnt, *ind_idx;
+  uint64_t cache_stride, part_z_floats;
+  uint32_t n_seq, nslots, rows16, wb1, wb2;      // rows16: of all units; wb: first workgroups of segments 1 and 2
+  uint32_t n_ssq, ssq_stride, k;
+  uint32_t ind_div, ind_stride, xw_block;
+  float eps;
+  MvqbRowsSeg seg[3];
+};
+
+template <int KIND, bool NORM>
+__global__ void __launch_bounds__(kBWaves * 64) mvqb_rows_kernel(const MvqbRows A) {
+  constexpr int NP = KIND == ER_PAIR ? 2 : 1, kSlots = 8;
+  __shared__ float s_inv[kMaxBatch];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), bid = blockIdx.x;
+  const int sg = KIND == ER_QKV ? (int)(bid >= A.wb1) + (int)(bid >= A.wb2) : 0;
+  const MvqbRowsSeg& S = A.seg[sg];
+  const float* part = A.part;
+  uint32_t n_seq = A.n_seq;
+  const uint32_t n_part = n_seq;
   const int* ind_idx = nullptr;
-  if (B.ind_cnt) {
+  if (KIND != ER_QKV && A.ind_cnt) {
     uint32_t cw;
-    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cw) : "s"(B.ind_cnt + blockIdx.z) : "memory");
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(cw) : "s"(A.ind_cnt + blockIdx.z) : "memory");
     n_seq = min(cw, n_seq);
     if (n_seq == 0) return;
-    ind_idx = B.ind_idx + (size_t)blockIdx.z * B.ind_stride;
-    part += (size_t)blockIdx.z * B.part_z_floats;
+    ind_idx = A.ind_idx + (size_t)blockIdx.z * A.ind_stride;
+    part += (size_t)blockIdx.z * A.part_z_floats;
   }
-  const uint32_t nslots = Gm.nslots;
-  const uint32_t npass = (uint32_t)S.npass;
-  float* red = reinterpret_cast<float*>(smem8);           // [n_seq][red_floats]: red[(p * nslots + slot) * S_rpw + rl]
-  float* ssq = red + (size_t)n_seq * red_floats;          // [n_seq][8]
-  const uint32_t ntiles = (S.n_rows + 15) >> 4;
-  const uint32_t ub = sg == 0 ? 0u : sg == 1 ? Gm.ub1 : Gm.ub2;
-  const size_t rows16 = (size_t)Gm.n_units * 16;
-  if constexpr (FEW) {
-    const uint32_t per_seq = npass * nslots * S_rpw, s = threadIdx.x / per_seq, j = threadIdx.x - s * per_seq;
-    const uint32_t ps = j / S_rpw, p = ps / nslots, row = wg * S_rpw + j - ps * S_rpw;                 // ps = p * nslots + slot
-    float v = 0.0f;
-    if (s < n_seq && row < ntiles * 16) v = part[((size_t)(ps - p * nslots) * B.n_seq + s) * rows16 + (size_t)(ub + p * ntiles) * 16 + row];
-    if (nrm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
-    if (s < n_seq) red[(size_t)s * red_floats + j] = v;
-  } else {
-    // four rows a load, four loads of a thread under way at once, the norms' behind the first of them: 6.0 us at 16 sequences of an 8B model (one row a load, each awaited: 7.2)
-    const uint32_t quads = S_rpw / 4, items = n_seq * npass * nslots * quads;
-    constexpr uint32_t kAtOnce = 4;
-    f32x4 v[kAtOnce];
-    auto place = [&](uint32_t i, uint32_t& s, uint32_t& ps, uint32_t& rl) {   // item -> sequence, p * nslots + slot, first row
-      const uint32_t j = i / quads;
-      rl = (i - j * quads) * 4;
-      s = j / (npass * nslots);
-      ps = j - s * npass * nslots;
-    };
-    auto load = [&](uint32_t i0) {
+  const uint32_t rows = S.rows, chunks = rows >> 4, items = n_seq * rows, row0 = (bid - S.wg_begin) * rows;
+  const uint32_t n_rows = S.n_rows, padded = (n_rows + 15) & ~15u, nslots = A.nslots;
+  const bool rope = KIND == ER_QKV && (S.epi == EPI_ROPE_Q || S.epi == EPI_ROPE_K), cache = KIND == ER_QKV && (S.epi == EPI_ROPE_K || S.epi == EPI_V_CACHE);
+  // the norm's partial sums: wave w has sequences w and w + 8 (as wave 0 of the single-sequence kernel has its own)
+  float nsum[2][4];
+  auto norm_part = [&](uint32_t s) { return A.ssq_part + (size_t)(ind_idx ? (uint32_t)ind_idx[s] / A.ind_div : s) * A.ssq_stride; };
+  if (NORM) {
 #pragma unroll
-      for (uint32_t k = 0; k < kAtOnce; k++) {
-        const uint32_t i = i0 + k * (kBWaves * 64);
-        uint32_t s, ps, rl;
-        place(i < items ? i : 0, s, ps, rl);
-        const uint32_t p = ps / nslots, slot = ps - p * nslots, row = wg * S_rpw + rl;
-        v[k] = (f32x4)(0.0f);
-        if (i < items && row < ntiles * 16)
-          v[k] = *reinterpret_cast<const f32x4*>(part + ((size_t)slot * B.n_seq + s) * rows16 + (size_t)(ub + p * ntiles) * 16 + row);
+    for (uint32_t h = 0; h < 2; h++) {
+      const uint32_t s = wave + h * kBWaves;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        nsum[h][j] = 0.0f;
+        if (s < n_seq && lane + 64 * j < A.n_ssq) nsum[h][j] = norm_part(s)[lane + 64 * j];
       }
-    };
-    load(threadIdx.x);
-    if (nrm) mvqb_norms(L, B, n_seq, ssq, ind_idx);
-    for (uint32_t i0 = threadIdx.x; i0 < items; i0 += kAtOnce * kBWaves * 64) {
-#pragma unroll
-      for (uint32_t k = 0; k < kAtOnce; k++) {
-        const uint32_t i = i0 + k * (kBWaves * 64);
-        if (i < items) {
-          uint32_t s, ps, rl;
-          place(i, s, ps, rl);
-#pragma unroll
-          for (int e = 0; e < 4; e++) red[(size_t)s * red_floats + ps * S_rpw + rl + e] = v[k][e];
-        }
-      }
-      if (i0 + kAtOnce * kBWaves * 64 < items) load(i0 + kAtOnce * kBWaves * 64);
     }
   }
-  mvqb_tail(L, S, B, sg, wg, S.rows_per_wg, n_seq, red_floats, red, ssq, nslots, ind_idx);
+  for (uint32_t i0 = 0; i0 < items; i0 += kBWaves * 64) {
+    const uint32_t c = (i0 + tid) >> 4, sc = c / chunks;
+    const bool in = sc < n_seq;
+    const uint32_t s = in ? sc : 0, rl = in ? (c - sc * chunks) * 16 + (tid & 15) : tid & 15, row = row0 + rl;
+    const bool live = in && row < n_rows;
+    const uint32_t rc = row < padded ? row : 0, rl_ = row < n_rows ? row : 0;   // (loads are unconditional)
+    uint32_t so = s;                                   // whose output vectors (an indirect entry's (sequence, slot) pair)
+    if (KIND != ER_QKV && ind_idx) so = (uint32_t)ind_idx[s];
+    uint32_t pos = 0, slot = 0;
+    if (KIND == ER_QKV) { pos = (uint32_t)A.pos[s]; slot = (uint32_t)A.slot[s]; }
+    float v[NP][kSlots];
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (uint32_t j = 0; j < kSlots; j++)
+        v[p][j] = part[((size_t)(j < nslots ? j : 0) * n_part + s) * A.rows16 + (size_t)S.unit_begin * 16 + p * padded + rc];
+    const float res = KIND == ER_OUT && S.resid ? S.resid[(size_t)so * S.resid_stride + rl_] : 0.0f;
+    const float nw = KIND != ER_QKV && S.nw ? S.nw[rl_] : 1.0f;
+    const float bias = S.bias ? S.bias[rl_] : 0.0f;
+    const uint32_t d = KIND == ER_QKV ? S.head_dim : 0, head = d == 0 ? 0 : (d & (d - 1)) == 0 ? row >> __builtin_ctz(d) : row / d, e = row - head * d;
+    float cs = 0.0f, sn = 0.0f;
+    if (rope) {
+      const float* at = A.rope_cs + ((size_t)pos * (d / 2) + e / 2) * 2;
+      cs = at[0];
+      sn = at[1];
+    }
+    if (NORM && i0 == 0) {
+#pragma unroll
+      for (uint32_t h = 0; h < 2; h++) {
+        const uint32_t q = wave + h * kBWaves;
+        if (q < n_seq) {
+          float ss = (nsum[h][0] + nsum[h][1]) + (nsum[h][2] + nsum[h][3]);
+          const float* np = norm_part(q);
+          for (uint32_t i = 256 + lane; i < A.n_ssq; i += 64) ss += np[i];
+          ss = wave_sum_to_lane63(ss);
+          if (lane == 63) s_inv[q] = mv_inv_rms(ss, A.k, A.eps);
+        }
+      }
+      __syncthreads();
+    }
+    const float inv = NORM ? s_inv[s] : 1.0f;
+    float t[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      t[p] = 0.0f;
+#pragma unroll
+      for (uint32_t j = 0; j < kSlots; j++)
+        if (j < nslots) t[p] += v[p][j];
+      t[p] *= inv;
+    }
+    if (S.bias) t[0] += bias;
+    if (KIND == ER_QKV) {
+      const float other = dpp_f<0xB1>(t[0]);           // the pair's other element
+      if (rope) {
+        const float x0 = (tid & 1) ? other : t[0], x1 = (tid & 1) ? t[0] : other;
+        const float y0 = x0 * cs - x1 * sn, y1 = x0 * sn + x1 * cs;  // ops.rs:1326-1331
+        t[0] = (tid & 1) ? y1 : y0;
+      }
+      if (live) {
+        float* dst = cache ? S.out + (size_t)slot * A.cache_stride + ((size_t)head * S.max_seq + pos) * d + e : S.out + (size_t)s * S.out_stride + row;
+        *dst = t[0];
+      }
+    } else if (live) {
+      const float outv = KIND == ER_PAIR ? silu_f(t[0]) * t[1] : S.resid ? t[0] + res : t[0];
+      S.out[(size_t)so * S.out_stride + row] = outv;
+      if (S.xq)                                        // (n_rows is a multiple of 16 here: a chunk's 16 threads are all live)
+        xq_store_chunk(S.xq + (size_t)so * S.xq_stride, row >> 4, outv * nw, S.ssq ? S.ssq + (size_t)so * S.ssq_stride : nullptr, outv, tid, S.xw ? S.xw + (size_t)so * kXwRecord : nullptr, A.xw_block);
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1253,11 +1307,51 @@ static hipError_t mvqb4_go(const MvLaunch& L, const MvBatch& B, Mvqb2Geom Gm, bo
   return hipGetLastError();
 }
 
-static bool mvqb2_epilogue_few(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm) {
-  if (B.ind_cnt || B.n_seq > 4) return false;
-  for (int i = 0; i < L.nseg; i++)
-    if (B.n_seq * (uint32_t)L.seg[i].npass * Gm.nslots * L.seg[i].rows_per_wg > (uint32_t)kBWaves * 64) return false;
-  return true;
+template <int KIND, bool NORM>
+static hipError_t mvqb_rows_go(const MvqbRows& A, uint32_t n_wg, uint32_t nz, hipStream_t st) {
+  hipLaunchKernelGGL((mvqb_rows_kernel<KIND, NORM>), dim3(n_wg, 1, nz), dim3(kBWaves * 64), 0, st, A);
+  return hipGetLastError();
+}
+
+// what mvqb_rows_kernel does with the rows of a launch, or -1
+static int mvqb_rows_kind(const MvLaunch& L) {
+  const MvSeg& S0 = L.seg[0];
+  if (L.nseg == 1 && S0.npass == 1 && (S0.epi == EPI_STORE || S0.epi == EPI_RESID)) return ER_OUT;
+  if (L.nseg == 1 && S0.npass == 2 && S0.epi == EPI_SWIGLU) return ER_PAIR;
+  for (int i = 0; i < L.nseg; i++) {
+    const MvSeg& S = L.seg[i];
+    const bool turned = S.epi == EPI_ROPE_Q || S.epi == EPI_ROPE_K;
+    if (S.npass != 1 || S.xq_out || !(turned || S.epi == EPI_V_CACHE || S.epi == EPI_STORE) || (S.epi != EPI_STORE && S.head_dim == 0) || (turned && S.head_dim % 2)) return -1;
+  }
+  return ER_QKV;
+}
+
+static hipError_t mvqb_rows_launch(const MvLaunch& L, const MvBatch& B, const Mvqb2Geom& Gm, uint32_t n_wg, uint32_t nz, hipStream_t st) {
+  const int kind = mvqb_rows_kind(L);
+  if (kind < 0 || (kind == ER_QKV && B.ind_cnt) || Gm.nslots > 8) return hipErrorInvalidValue;
+  MvqbRows A{};
+  A.part = B.part; A.ssq_part = L.ssq_part; A.rope_cs = L.rope_cs;
+  A.pos = B.pos; A.slot = B.slot; A.ind_cnt = B.ind_cnt; A.ind_idx = B.ind_idx;
+  A.cache_stride = B.cache_stride; A.part_z_floats = B.part_z_floats;
+  A.n_seq = B.n_seq; A.nslots = Gm.nslots; A.rows16 = Gm.n_units * 16;
+  A.wb1 = L.nseg > 1 ? L.seg[1].wg_begin : 0xFFFFFFFFu; A.wb2 = L.nseg > 2 ? L.seg[2].wg_begin : 0xFFFFFFFFu;
+  A.n_ssq = L.n_ssq_part; A.ssq_stride = B.ssq_stride; A.k = L.k; A.eps = L.eps;
+  A.ind_div = B.ind_div; A.ind_stride = B.ind_stride; A.xw_block = B.xw_block;
+  for (int i = 0; i < L.nseg; i++) {
+    const MvSeg& S = L.seg[i];
+    MvqbRowsSeg& D = A.seg[i];
+    D.out = S.out; D.resid = S.epi == EPI_RESID ? S.resid : nullptr; D.nw = S.xq_out ? S.xq_nw : nullptr; D.bias = S.bias;
+    D.xq = S.xq_out; D.ssq = S.xq_ssq; D.xw = B.xw_out[i];
+    D.n_rows = S.n_rows; D.wg_begin = S.wg_begin; D.rows = S.rows_per_wg;
+    D.unit_begin = i == 0 ? 0u : i == 1 ? Gm.ub1 : Gm.ub2;
+    D.out_stride = B.out_stride[i]; D.resid_stride = B.resid_stride[i]; D.xq_stride = B.xq_out_stride[i]; D.ssq_stride = B.ssq_out_stride[i];
+    D.epi = (uint32_t)S.epi; D.head_dim = S.head_dim; D.max_seq = S.max_seq;
+  }
+  switch (kind) {
+    case ER_OUT: return L.do_norm ? mvqb_rows_go<ER_OUT, true>(A, n_wg, nz, st) : mvqb_rows_go<ER_OUT, false>(A, n_wg, nz, st);
+    case ER_PAIR: return L.do_norm ? mvqb_rows_go<ER_PAIR, true>(A, n_wg, nz, st) : mvqb_rows_go<ER_PAIR, false>(A, n_wg, nz, st);
+    default: return L.do_norm ? mvqb_rows_go<ER_QKV, true>(A, n_wg, nz, st) : mvqb_rows_go<ER_QKV, false>(A, n_wg, nz, st);
+  }
 }
 
 // enough units to fill the chip with whole rows per workgroup; with fewer the k-slices are a grid dimension
@@ -1290,9 +1384,8 @@ static hipError_t mvqb_few_go(const MvLaunch& L, const MvBatch& B, const Mvqb2Ge
 }
 
 template <uint32_t MASK, int NB>
-static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, Mvqb2Geom Gm, bool seq, uint32_t groups, size_t lds_x,
-                           size_t lds_e, uint32_t threads, hipStream_t st) {
-  static bool attr_set[4][64] = {};
+static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, Mvqb2Geom Gm, bool seq, uint32_t groups, size_t lds_x, hipStream_t st) {
+  static bool attr_set[2][64] = {};
   const uint32_t nz = B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1;   // a layer's experts as the grid's third dimension
   Gm.ssq_at = (uint32_t)lds_x;
   lds_x += mvqb_fuse_lds(B.n_seq);
@@ -1315,12 +1408,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
     hipLaunchKernelGGL((mvqb2_kernel<MASK, NB, false>), dim3(groups, Gm.T, nz), dim3(kBWaves * 64), lds_x, st, Gm, L, B, B.part);
   }
   if (hipError_t e = hipGetLastError(); e != hipSuccess || Gm.fuse) return e;
-  auto epilogue = [&](auto* kernel, bool (&opted)[64]) -> hipError_t {
-    if (hipError_t e = lds_opt_in(reinterpret_cast<const void*>(kernel), 160 * 1024, opted); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, dim3(g.n_wg, 1, nz), dim3(threads), lds_e, st, g.wbpack, g.geom, g.geom2, L.red_floats, Gm, L, B, (const float*)B.part);
-    return hipGetLastError();
-  };
-  return mvqb2_epilogue_few(L, B, Gm) ? epilogue(&mvqb2_epilogue_kernel<true>, attr_set[2]) : epilogue(&mvqb2_epilogue_kernel<false>, attr_set[3]);
+  return mvqb_rows_launch(L, B, Gm, g.n_wg, nz, st);
 }
 
 // from how many sequences on the records go through LDS (mvqb2 and the kernels beside it)
@@ -1372,9 +1460,9 @@ hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uin
     if (B.part_z_floats * (B.ind_cnt && B.ind_nz > 1 ? B.ind_nz : 1) <= B.part_floats) {
 #define LGH_MVQB2_CASE(M)                                                                         \
   case M:                                                                                         \
-    if (B.n_seq <= 4) return mvqb2_go<M, 4>(L, B, g, Gm, seq, groups, lds_x, lds, threads, st);  \
-    if (B.n_seq <= 8) return mvqb2_go<M, 8>(L, B, g, Gm, seq, groups, lds_x, lds, threads, st);  \
-    return mvqb2_go<M, 16>(L, B, g, Gm, seq, groups, lds_x, lds, threads, st)
+    if (B.n_seq <= 4) return mvqb2_go<M, 4>(L, B, g, Gm, seq, groups, lds_x, st);  \
+    if (B.n_seq <= 8) return mvqb2_go<M, 8>(L, B, g, Gm, seq, groups, lds_x, st);  \
+    return mvqb2_go<M, 16>(L, B, g, Gm, seq, groups, lds_x, st)
       switch (mask) {
         LGH_MVQB2_CASE(1u << F_Q4K); LGH_MVQB2_CASE(1u << F_Q6K); LGH_MVQB2_CASE(1u << F_Q5K); LGH_MVQB2_CASE(1u << F_Q80); LGH_MVQB2_CASE(1u << F_Q40);
         LGH_MVQB2_CASE((1u << F_Q4K) | (1u << F_Q6K)); LGH_MVQB2_CASE((1u << F_Q5K) | (1u << F_Q6K));
