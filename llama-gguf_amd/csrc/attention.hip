@@ -158,8 +158,8 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
       float m0, m1, l0, l1, a0, a1;
       both(m[g], m0, m1);
       both(l[g], l0, l1);
-      const float mn = fmaxf(m0, m1);
-      const float a = expf(m0 - mn), b = expf(m1 - mn);
+      float mn, a, b;
+      merge_two(m0, m1, mn, a, b);
       l[g] = l0 * a + l1 * b;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -183,16 +183,10 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_kernel(const float* __re
   const size_t pbase = ((size_t)kvh * n_splits + sp) * G;
   for (uint32_t e = threadIdx.x; e < (uint32_t)(G * D); e += NW * 64) {
     const uint32_t g = e / D, dim = e % D;
-    float mn = s_ml[0][g][0];
+    float mn, lsum, a = 0.0f, f[NW];
+    merge_factors<NW>(&s_ml[0][g][0], 2 * G, f, mn, lsum);
 #pragma unroll
-    for (int w = 1; w < NW; w++) mn = fmaxf(mn, s_ml[w][g][0]);
-    float lsum = 0.0f, a = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-      const float f = expf(s_ml[w][g][0] - mn);
-      lsum += s_ml[w][g][1] * f;
-      a += s_acc[w][g][dim] * f;
-    }
+    for (int w = 0; w < NW; w++) a += s_acc[w][g][dim] * f[w];
     if (PF) {
       const _Float16 o = (_Float16)(a * (1.0f / lsum));   // simd.rs:718-720: multiply by 1/sum
       *reinterpret_cast<_Float16*>(reinterpret_cast<uint8_t*>(part_acc) + xh_offset(blockIdx.y, (uint32_t)(pbase + g) * D + dim)) = o;
@@ -381,8 +375,8 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_q8_kernel(const float* _
       f32x4 oa;
       oa.x = __shfl_xor(acc[g].x, off, 64); oa.y = __shfl_xor(acc[g].y, off, 64);
       oa.z = __shfl_xor(acc[g].z, off, 64); oa.w = __shfl_xor(acc[g].w, off, 64);
-      const float mn = fmaxf(m[g], om);
-      const float a = expf(m[g] - mn), b = expf(om - mn);
+      float mn, a, b;
+      merge_two(m[g], om, mn, a, b);
       l[g] = l[g] * a + ol * b;
       acc[g] = acc[g] * a + oa * b;
       m[g] = mn;
@@ -399,16 +393,10 @@ __global__ void __launch_bounds__(NW * 64) attn_partial_q8_kernel(const float* _
   const size_t pbase = ((size_t)kvh * n_splits + sp) * G;
   for (uint32_t e = threadIdx.x; e < (uint32_t)(G * D); e += NW * 64) {
     const uint32_t g = e / D, dim = e % D;
-    float mn = s_ml[0][g][0];
+    float mn, lsum, a = 0.0f, f[NW];
+    merge_factors<NW>(&s_ml[0][g][0], 2 * G, f, mn, lsum);
 #pragma unroll
-    for (int w = 1; w < NW; w++) mn = fmaxf(mn, s_ml[w][g][0]);
-    float lsum = 0.0f, a = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-      const float f = expf(s_ml[w][g][0] - mn);
-      lsum += s_ml[w][g][1] * f;
-      a += s_acc[w][g][dim] * f;
-    }
+    for (int w = 0; w < NW; w++) a += s_acc[w][g][dim] * f[w];
     part_acc[(pbase + g) * D + dim] = a;
     if (dim == 0) { part_ml[(pbase + g) * 2] = mn; part_ml[(pbase + g) * 2 + 1] = lsum; }
   }
@@ -1081,7 +1069,8 @@ __global__ void __launch_bounds__(1024, 8) attn_multi_direct_kernel(const float*
         float m0, m1, l0, l1, a0, a1;
         both(m, m0, m1);
         both(l, l0, l1);
-        const float mn = fmaxf(m0, m1), a = expf(m0 - mn), b = expf(m1 - mn);
+        float mn, a, b;
+        merge_two(m0, m1, mn, a, b);
         l = l0 * a + l1 * b;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -1100,18 +1089,11 @@ __global__ void __launch_bounds__(1024, 8) attn_multi_direct_kernel(const float*
       __syncthreads();   // (two sets: the next round's waves may write while this one is merged)
       const uint32_t qs = tid / D, dim = tid % D, sp = r * QS + qs;
       if (tid < (uint32_t)(QS * D) && sp < used) {
-        const float(*ml)[2] = &s_ml[r & 1][qs * NW];
         const float(*ac)[D] = &s_acc[r & 1][qs * NW];
-        float mn = ml[0][0];
+        float mn, lsum, a = 0.0f, f[NW];
+        merge_factors<NW>(&s_ml[r & 1][qs * NW][0], 2, f, mn, lsum);
 #pragma unroll
-        for (int w = 1; w < NW; w++) mn = fmaxf(mn, ml[w][0]);
-        float lsum = 0.0f, a = 0.0f;
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-          const float f = expf(ml[w][0] - mn);
-          lsum += ml[w][1] * f;
-          a += ac[w][dim] * f;
-        }
+        for (int w = 0; w < NW; w++) a += ac[w][dim] * f[w];
         p_acc[sp][dim] = a;
         if (dim == 0) { p_ml[sp][0] = mn; p_ml[sp][1] = lsum; }
       }

@@ -384,8 +384,8 @@ __global__ void __launch_bounds__(256) attn_tq_partial_kernel(const float* __res
 #pragma unroll
     for (int g = 0; g < G; g++) {
       const float om = __shfl_xor(m[g], off, 64), ol = __shfl_xor(l[g], off, 64);
-      const float mn = fmaxf(m[g], om);
-      const float a = expf(m[g] - mn), b = expf(om - mn);
+      float mn, a, b;
+      merge_two(m[g], om, mn, a, b);
       l[g] = l[g] * a + ol * b;
 #pragma unroll
       for (int c = 0; c < 16; c++) acc[g][c] = acc[g][c] * a + __shfl_xor(acc[g][c], off, 64) * b;
@@ -405,16 +405,10 @@ __global__ void __launch_bounds__(256) attn_tq_partial_kernel(const float* __res
   const size_t pbase = ((size_t)kvh * n_splits + sp) * G;
   for (uint32_t e = tid; e < (uint32_t)(G * D); e += 256) {
     const uint32_t g = e / D, dim = e % D;
-    float mn = s_ml[g * 2];
+    float mn, lsum, a = 0.0f, f[NW];
+    merge_factors<NW>(&s_ml[g * 2], 2 * G, f, mn, lsum);
 #pragma unroll
-    for (int w = 1; w < NW; w++) mn = fmaxf(mn, s_ml[(w * G + g) * 2]);
-    float lsum = 0.0f, a = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-      const float f = expf(s_ml[(w * G + g) * 2] - mn);
-      lsum += s_ml[(w * G + g) * 2 + 1] * f;
-      a += s_acc[((size_t)w * G + g) * D + dim] * f;
-    }
+    for (int w = 0; w < NW; w++) a += s_acc[((size_t)w * G + g) * D + dim] * f[w];
     part_acc[(pbase + g) * D + dim] = a;
     if (dim == 0) { part_ml[(pbase + g) * 2] = mn; part_ml[(pbase + g) * 2 + 1] = lsum; }
   }
@@ -599,15 +593,20 @@ __global__ void __launch_bounds__(1024) attn_tq_direct_kernel(const float* __res
   }
   __syncthreads();
   if (wave > 0) return;
-  // the first wave: the waves' parts, then out = signs * (1 / d) * H (sqrt(d) * o), as attn_tq_combine_kernel
-  float mn = s_m[0];
-#pragma unroll
-  for (int w = 1; w < NW; w++) mn = fmaxf(mn, s_m[w]);
+  // the first wave: the waves' parts, then out = signs * (1 / d) * H (sqrt(d) * o), as attn_tq_combine_kernel.  A lane has one wave's factor (expf is a dozen instructions, and one wave issues them all); they go round as scalars.
+  static_assert(NW == 16, "a wave for each lane of a row");
+  const float wmax = s_m[lane & 15];
+  float mn = fmaxf(wmax, dpp_f<0xB1>(wmax));
+  mn = fmaxf(mn, dpp_f<0x4E>(mn));
+  mn = fmaxf(mn, dpp_f<0x141>(mn));
+  mn = fmaxf(mn, dpp_f<0x140>(mn));
+  const float fl = expf(wmax - mn), pl = s_l[lane & 15] * fl;
+  auto of_lane = [](float v, int w) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), w)); };
   float lsum = 0.0f, a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
   for (int w = 0; w < NW; w++) {
-    const float fw = expf(s_m[w] - mn);
-    lsum += s_l[w] * fw;
+    const float fw = of_lane(fl, w);
+    lsum += of_lane(pl, w);
     a0 += s_acc[w][lane] * fw;
     if (D == 128) a1 += s_acc[w][lane + (D == 128 ? 64 : 0)] * fw;
   }

@@ -114,4 +114,32 @@ __device__ __forceinline__ float silu_act_f(float x) {
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, y), r, q), d, y);
 }
 
+// Factors with which NW waves' partial results (their m, l: ml[w * stride], behind it) become one, and the merged m and l.  A quad's four lanes merge the same waves: each lane has one factor (two of eight) and takes the
+// others from its neighbours, for expf is a dozen instructions.  Sums in the waves' order.
+template <int NW>
+__device__ __forceinline__ void merge_factors(const float* ml, uint32_t stride, float (&f)[NW], float& m, float& l) {
+  static_assert(NW == 4 || NW == 8, "");
+  const uint32_t q = threadIdx.x & 3;
+  float mw[NW / 4], lw[NW / 4];
+#pragma unroll
+  for (int h = 0; h < NW / 4; h++) { mw[h] = ml[(q + 4 * h) * stride]; lw[h] = ml[(q + 4 * h) * stride + 1]; }
+  m = NW == 8 ? fmaxf(mw[0], mw[NW / 8]) : mw[0];
+  m = fmaxf(m, dpp_f<0xB1>(m));
+  m = fmaxf(m, dpp_f<0x4E>(m));
+  l = 0.0f;
+#pragma unroll
+  for (int h = 0; h < NW / 4; h++) {
+    const float e = expf(mw[h] - m), p = lw[h] * e;
+    f[4 * h] = dpp_f<0x00>(e); f[4 * h + 1] = dpp_f<0x55>(e); f[4 * h + 2] = dpp_f<0xAA>(e); f[4 * h + 3] = dpp_f<0xFF>(e);
+    l += dpp_f<0x00>(p); l += dpp_f<0x55>(p); l += dpp_f<0xAA>(p); l += dpp_f<0xFF>(p);
+  }
+}
+// exp(m0 - max) and exp(m1 - max): the larger one's is 1
+__device__ __forceinline__ void merge_two(float m0, float m1, float& m, float& a, float& b) {
+  m = fmaxf(m0, m1);
+  const float e = expf(fminf(m0, m1) - m);
+  a = m0 >= m1 ? 1.0f : e;
+  b = m1 >= m0 ? 1.0f : e;
+}
+
 }  // namespace lgh
