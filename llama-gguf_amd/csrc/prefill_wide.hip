@@ -78,7 +78,7 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
   constexpr uint32_t tb = pf_tile_bytes(F), NB = pw_bufs<F>(), DIST = NB - 1;
   constexpr int NX = TT;   // NX: activation DMA operations per wave and step
   constexpr int UN = 4 * TT, AHEAD = 3;                                                     // units (phase, token tile) of a step
-  constexpr int RPP = TT > 4 ? 2 : 1, RU = TT / RPP;                                        // regions of a phase, units of a region
+  constexpr int RPP = TT > 4 && TT % 2 == 0 ? 2 : 1, RU = TT / RPP;                         // regions of a phase, units of a region
   const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t n = lane & 15, g = lane >> 5, tk = lane & 31, sub = lane >> 4 & 1;
   const uint32_t per = (G.nblk + G.S - 1) / G.S, b0 = ks * per, b1 = b0 + per < G.nblk ? b0 + per : G.nblk;
@@ -133,7 +133,8 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
   const uint32_t s0 = b0 * 4, s1 = b1 * 4;   // steps of 64 elements
   // regions of a step; raw operations per region, spread over a block's first two steps, and how many of them each of the two makes
   constexpr int RS = 4 * RPP, RP = (R + 2 * RS - 1) / (2 * RS), R0 = R < RS * RP ? R : RS * RP, R1 = R - R0;
-  static_assert(TT % RPP == 0 && NX <= RS && RU >= AHEAD, "an activation operation a region at most; the last one holds what is awaited");
+  constexpr int XP = (NX + RS - 1) / RS;   // activation operations per region
+  static_assert(TT % RPP == 0 && RU >= AHEAD, "the last region holds what is awaited");
   auto x_dma = [&](int i, uint32_t s, uint32_t buf) {   // operation i of a step's activations
     const uint8_t* base = G.x + (size_t)(s < s1 ? s : s1 - 1) * 128;   // past the end: requested again, never read
     pw_dma(base, xoff[i], lds0 + buf * kWStepBytes + (wave * NX + i) * 1024);
@@ -191,8 +192,12 @@ __device__ __forceinline__ void pw_body(const PfWide& G, const PfwSeg& sg, uint3
         for (int i = 0; i < NX; i++) x_dma(i, s + DIST, far);
       }
 #pragma unroll
-      for (int r = 0; r < RS; r++) {   // regions of 3 or 4 units: two MFMAs and an operand read each, one or both of the next phase's A operands, and the DMA piece by piece
-        if (NB == 3 && r < NX) x_dma(r, s + DIST, far);
+      for (int r = 0; r < RS; r++) {   // regions of 3 to 7 units: two MFMAs and an operand read each, one or both of the next phase's A operands, and the DMA piece by piece
+        if (NB == 3) {
+#pragma unroll
+          for (int i = r * XP; i < (r + 1) * XP; i++)
+            if (i < NX) x_dma(i, s + DIST, far);
+        }
         if (pp < 2) {
 #pragma unroll
           for (int k = (pp * RS + r) * RP; k < (pp * RS + r + 1) * RP; k++)
@@ -322,13 +327,19 @@ __global__ void __launch_bounds__(kWWaves * 64) pw_gemm_kernel(const PfWide G, u
   const PfwSeg& sg = G.seg[si];
   const uint32_t rg = rgid - sg.rg_begin;
   auto is = [&](int f) { return (MASK & (1u << f)) && (MASK == (1u << f) || sg.fmt == f); };
-  // Tiles of 256, 192 and 128 tokens: a product takes time with the tokens computed (experts of some 100 to 190 rows, 401 tokens of Mixtral widths: gate | up 364 -> 323 us with the middle one;
-  // a last tile of 1200 and 1700 tokens, 4 layers of an 8B model: 2.55 -> 2.46 and 3.43 -> 3.34 ms)
+  // Tiles of 256 tokens down to 96 in steps of 32: a product takes time with the tokens computed, and below 96 with the weights' dequantization.  256, 192 and 128 alone, then these: two layers of Mixtral Q5_K_M, 200 / 330 /
+  // 600 tokens (experts of some 50, 80, 150 rows) 816 / 830 / 1196 -> 767 / 786 / 1167 us; 4 layers of an 8B model, last tiles of 148, 217 and 160 tokens (660, 729, 416): 1610 / 1706 / 1187 -> 1590 / 1685 / 1181.
+  // (Before, 256 and 128 alone: experts of some 100 to 190 rows, 401 tokens of Mixtral widths: gate | up 364 -> 323 us with 192.)
 #define LGH_PW_RUN(F)                                                                                       \
   do {                                                                                                      \
-    if (m_end - m0 > (uint32_t)kPfwTile * 3 / 4) pw_body<F, 8, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);  \
-    else if (m_end - m0 > (uint32_t)kPfwTile / 2) pw_body<F, 6, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); \
-    else pw_body<F, 4, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem);                                          \
+    switch ((m_end - m0 + 31) / 32) {                                                                       \
+      case 8: pw_body<F, 8, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); break;                    \
+      case 7: pw_body<F, 7, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); break;                    \
+      case 6: pw_body<F, 6, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); break;                    \
+      case 5: pw_body<F, 5, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); break;                    \
+      case 4: pw_body<F, 4, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); break;                    \
+      default: pw_body<F, 3, GRP, EPI>(G, sg, rg, ks, m0, m_end, expert, pw_smem); break;   /* (up to 96) */  \
+    }                                                                                                       \
   } while (0)
   if (is(PF_Q4K)) LGH_PW_RUN(PF_Q4K);
   else if (is(PF_Q6K)) LGH_PW_RUN(PF_Q6K);
