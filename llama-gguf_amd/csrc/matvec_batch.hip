@@ -687,14 +687,15 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
 // addition (the halves: the rounding that the fused multiply-add of the other kernels does, shifted by a power of two) and the fused multiply-add with the weights' scale: the same
 // bits.  The sum over the minima, a chain of four fused multiply-adds, is a 16x16x4 f32 matrix instruction, which rounds as that chain does.
 //   A: row 4 m + 2 q + half of sequence m + 4 q of eight (a lane of group m gets both halves of sequences m and m + 4), K = lane group's four elements of the half's first digit, then of its second
-//   B: the lane group's four weights twice; a lane unpacks one chunk of 64 elements, so the chunks' words are exchanged between the lane groups (4 x 4, four swaps)
+//   B: the lane group's four weights twice; a lane unpacks one chunk of 64 elements, so the chunks' words are exchanged between the lane groups (4 x 4, four swaps, of packed words three)
 // (Inputs beyond 2^117 in magnitude may overflow a half where a zero scale would have hidden it.)
 // Q6_K's weights are signed (0 .. 63 would reach 2^25; as nibble and upper bits in two products they took 64 matrix instructions a tile and spilled), and a half is cut so that 16 weights of -32 stay in range: with halves
 // of 2^14 and 2^16 units the low one passed 2^24 by 0.4 %.  Against the integer cores (mvqb4), 16 sequences of an 8B model: down 29.4 -> 20.3 us, Q, K and V with one Q6_K matrix 20.9 -> 15.0, the head (32000 rows) 65 -> 38;
 // a step of 4 layers, us, 5 / 8 / 16 sequences: Q4_K_M 389 / 416 / 588 -> 370 / 396 / 539, Q6_K 445 / 477 / 710 -> 384 / 415 / 551, Q5_K_M 417 / 444 / 612 -> 397 / 427 / 568; Mixtral Q5_K_M, one layer, 297 / 378 / 563 -> 282 / 360 / 526.
 // Who writes the input leaves it in this form (xq.h: the wide image), and a chunk's records of all sequences come as they lie in memory, a chunk ahead, by LDS-DMA.  Rewritten from the digits by every workgroup as they
 // were staged, they took a quarter of the vector instructions.  gate | up of an 8B model (28672 rows of 4096, Q4_K): 16 sequences 47.4 -> 42.7 us (58 with mvqb4), 8 33.7 -> 30.5; wo 13.6 -> 12.4; a step of 4 layers, 16
-// sequences, Q4_K_M 639 -> 617 us, Q4_0 599 -> 554.  Bound by the vector instructions: 343 a tile and block of 16 sequences, 192 of them the sums' own, two thirds of the waves' time (two waves a SIMD).
+// sequences, Q4_K_M 639 -> 617 us, Q4_0 599 -> 554.  Bound by the vector instructions: 339 a tile and block of 16 sequences, 192 of them the sums' own, 65 % of the SIMDs' cycles (the matrix cores 23 %; two waves a SIMD).
+// (Two workgroups a CU with half the records a chunk, where registers allow, 5 to 8 sequences: no difference.  In 128 registers 16 sequences spill.  Without the priorities 41.1 us.)
 // (Matrix and vector instructions dealt out one to six by the scheduler instead of a step's products in front of the sums of the one before: 40.2 -> 41.8 us.)
 // ------------------------------------------------------------------------------------------------
 constexpr uint32_t kX8Records = 32;                  // records of a chunk at most
@@ -795,16 +796,29 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
         TileScales ts;
         uint32_t tw[4][4];   // [step pp][class c]: the lane group's four weights of chunk 4 pp + c
         {
-          TileOps t;
-          mvq_unpack_tile<MASK>(fmt, nxt, lane, t);
           mvq_row_scales<MASK>(fmt, nxt, lane, ts);
+          if constexpr (F == F_Q4K || F == F_Q40) {
+            // a word holds the nibbles of two elements' fours: whole words change halves first, then the unpacked ones rows (three swaps a step instead of four:
+            // 16 sequences, gate | up 39.7 -> 39.4 us, the products split over k 12.45 -> 12.2)
 #pragma unroll
-          for (int pp = 0; pp < 4; pp++) {
-            const auto r01 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][0], (uint32_t)t.bw[pp][1], false, false);
-            const auto r23 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][2], (uint32_t)t.bw[pp][3], false, false);
-            const auto r02 = __builtin_amdgcn_permlane32_swap(r01[0], r23[0], false, false);
-            const auto r13 = __builtin_amdgcn_permlane32_swap(r01[1], r23[1], false, false);
-            tw[pp][0] = r02[0]; tw[pp][1] = r13[0]; tw[pp][2] = r02[1]; tw[pp][3] = r13[1];
+            for (int pp = 0; pp < 4; pp++) {
+              const uint32_t N0 = (pp & 1) ? nxt.q[pp >> 1].z : nxt.q[pp >> 1].x, N1 = (pp & 1) ? nxt.q[pp >> 1].w : nxt.q[pp >> 1].y;
+              const auto h = __builtin_amdgcn_permlane32_swap(N0, N1, false, false);
+              const auto r01 = __builtin_amdgcn_permlane16_swap(h[0] & 0x0F0F0F0Fu, (h[0] >> 4) & 0x0F0F0F0Fu, false, false);
+              const auto r23 = __builtin_amdgcn_permlane16_swap(h[1] & 0x0F0F0F0Fu, (h[1] >> 4) & 0x0F0F0F0Fu, false, false);
+              tw[pp][0] = r01[0]; tw[pp][1] = r01[1]; tw[pp][2] = r23[0]; tw[pp][3] = r23[1];
+            }
+          } else {
+            TileOps t;
+            mvq_unpack_tile<MASK>(fmt, nxt, lane, t);
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) {
+              const auto r01 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][0], (uint32_t)t.bw[pp][1], false, false);
+              const auto r23 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][2], (uint32_t)t.bw[pp][3], false, false);
+              const auto r02 = __builtin_amdgcn_permlane32_swap(r01[0], r23[0], false, false);
+              const auto r13 = __builtin_amdgcn_permlane32_swap(r01[1], r23[1], false, false);
+              tw[pp][0] = r02[0]; tw[pp][1] = r13[0]; tw[pp][2] = r02[1]; tw[pp][3] = r13[1];
+            }
           }
         }
         asm volatile("" : : "v"(tw[3][0]), "v"(ts.dd));   // (of the tile's last load)
