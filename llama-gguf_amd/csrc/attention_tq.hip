@@ -384,8 +384,8 @@ __global__ void __launch_bounds__(256) attn_tq_partial_kernel(const float* __res
 #pragma unroll
     for (int g = 0; g < G; g++) {
       const float om = __shfl_xor(m[g], off, 64), ol = __shfl_xor(l[g], off, 64);
-      float mn, a, b;
-      merge_two(m[g], om, mn, a, b);
+      const float mn = fmaxf(m[g], om);
+      const float a = expf(m[g] - mn), b = expf(om - mn);
       l[g] = l[g] * a + ol * b;
 #pragma unroll
       for (int c = 0; c < 16; c++) acc[g][c] = acc[g][c] * a + __shfl_xor(acc[g][c], off, 64) * b;
@@ -405,10 +405,16 @@ __global__ void __launch_bounds__(256) attn_tq_partial_kernel(const float* __res
   const size_t pbase = ((size_t)kvh * n_splits + sp) * G;
   for (uint32_t e = tid; e < (uint32_t)(G * D); e += 256) {
     const uint32_t g = e / D, dim = e % D;
-    float mn, lsum, a = 0.0f, f[NW];
-    merge_factors<NW>(&s_ml[g * 2], 2 * G, f, mn, lsum);
+    float mn = s_ml[g * 2];
 #pragma unroll
-    for (int w = 0; w < NW; w++) a += s_acc[((size_t)w * G + g) * D + dim] * f[w];
+    for (int w = 1; w < NW; w++) mn = fmaxf(mn, s_ml[(w * G + g) * 2]);
+    float lsum = 0.0f, a = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = expf(s_ml[(w * G + g) * 2] - mn);
+      lsum += s_ml[(w * G + g) * 2 + 1] * f;
+      a += s_acc[((size_t)w * G + g) * D + dim] * f;
+    }
     part_acc[(pbase + g) * D + dim] = a;
     if (dim == 0) { part_ml[(pbase + g) * 2] = mn; part_ml[(pbase + g) * 2 + 1] = lsum; }
   }

@@ -12,7 +12,7 @@
 // the sequences' records staged ONCE per workgroup in LDS and shared by its 8 waves, sequences two at a time (the pair's 8 MFMAs,
 // then the vector work while the next pair's operands load), the epilogue as a second small launch — what bounded the first
 // structure and what each change bought: profiles/r03e_batched_decode.md.  From three sequences on its products take the sequences in
-// groups of four (mvqb4) or, from five on and for weights of up to 6 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
+// groups of four (mvqb4) or, from five on and for weights below 6 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
 // workgroup = the 8 k-slices of a few row tiles) with a loop over the sequences inside it and their records from L2 into a
 // register ring; kept for one sequence and for launches whose segments do not share their input vector.
 // Epilogues: store, +residual, SwiGLU pair, RoPE (every sequence at its own position) and the K / V rows into the sequence's
@@ -492,7 +492,7 @@ __device__ __forceinline__ void mvq_row_scales(int fmt, const RawT16& r, uint32_
     for (int pp = 0; pp < 4; pp++)
 #pragma unroll
       for (int c = 0; c < 4; c++) t.f[pp][c] = (float)(int)__builtin_amdgcn_sbfe((int)hdw[pp], c * 8, 8);
-    t.dd = mvq_q6_scale(r, n);
+    t.dd = h2f((n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu);
     t.dmin = 0.0f;
   } else if (is(F_Q80) || is(F_Q40)) {
 #pragma unroll
@@ -679,38 +679,43 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
 }
 
 // ------------------------------------------------------------------------------------------------
-// The same for formats whose weights are whole numbers of at most 32 (all but Q8_0), on the bf16 matrix cores: what a digit needs beside its product moves into the
+// The same for formats whose weights are whole numbers below 32 (all but Q6_K and Q8_0), on the bf16 matrix cores: what a digit needs beside its product moves into the
 // operands.  mvqb4 spends eight vector instructions per (row, sequence, 16 elements): two shifts and additions of digit sums, two conversions, a fused
-// multiply-add, and the scales.  Here a digit is a bf16 number, the digit times its power of two times the chunk's scale, itself a power of two (both exact),
+// multiply-add, and the scales.  Here a digit is a bf16 number, the digit times its power of 256 times the chunk's scale, itself a power of two (both exact),
 // and the high two and the low two digits of 16 elements lie along one K of 32: the product IS the scaled high or low half, in f32.  Every partial sum is a whole
-// multiple of the scale of at most 2^24 of it (xq.h, the wide image: 16 elements, |weight| <= 32, halves of at most 2^15), so nothing rounds in it.  What is left is one
+// multiple of the scale below 2^24 of it (16 elements, weights <= 31; high half |I| >> 16 <= 2^14: 31 * 2^18; low half, two balanced digits, up to 128 * 256 + 128: 16 * 31 * 32896 = 16 316 416),
+// so nothing rounds in it.  (Weights of six bits would reach 33 158 336 in the low half, and beyond 2^24 the matrix instruction rounds where the integer sum does not.)  What is left is one
 // addition (the halves: the rounding that the fused multiply-add of the other kernels does, shifted by a power of two) and the fused multiply-add with the weights' scale: the same
 // bits.  The sum over the minima, a chain of four fused multiply-adds, is a 16x16x4 f32 matrix instruction, which rounds as that chain does.
 //   A: row 4 m + 2 q + half of sequence m + 4 q of eight (a lane of group m gets both halves of sequences m and m + 4), K = lane group's four elements of the half's first digit, then of its second
 //   B: the lane group's four weights twice; a lane unpacks one chunk of 64 elements, so the chunks' words are exchanged between the lane groups (4 x 4, four swaps, of packed words three)
 // (Inputs beyond 2^117 in magnitude may overflow a half where a zero scale would have hidden it.)
-// Q6_K's weights are signed (0 .. 63 would reach 2^25; as nibble and upper bits in two products they took 64 matrix instructions a tile and spilled), and a half is cut so that 16 weights of -32 stay in range: with halves
-// of 2^14 and 2^16 units the low one passed 2^24 by 0.4 %.  Against the integer cores (mvqb4), 16 sequences of an 8B model: down 29.4 -> 20.3 us, Q, K and V with one Q6_K matrix 20.9 -> 15.0, the head (32000 rows) 65 -> 38;
-// a step of 4 layers, us, 5 / 8 / 16 sequences: Q4_K_M 389 / 416 / 588 -> 370 / 396 / 539, Q6_K 445 / 477 / 710 -> 384 / 415 / 551, Q5_K_M 417 / 444 / 612 -> 397 / 427 / 568; Mixtral Q5_K_M, one layer, 297 / 378 / 563 -> 282 / 360 / 526.
 // Who writes the input leaves it in this form (xq.h: the wide image), and a chunk's records of all sequences come as they lie in memory, a chunk ahead, by LDS-DMA.  Rewritten from the digits by every workgroup as they
 // were staged, they took a quarter of the vector instructions.  gate | up of an 8B model (28672 rows of 4096, Q4_K): 16 sequences 47.4 -> 42.7 us (58 with mvqb4), 8 33.7 -> 30.5; wo 13.6 -> 12.4; a step of 4 layers, 16
 // sequences, Q4_K_M 639 -> 617 us, Q4_0 599 -> 554.  Bound by the vector instructions: 339 a tile and block of 16 sequences, 192 of them the sums' own, 65 % of the SIMDs' cycles (the matrix cores 23 %; two waves a SIMD).
-// (Two workgroups a CU with half the records a chunk, where registers allow, 5 to 8 sequences: no difference.  In 128 registers 16 sequences spill.  Without the priorities 41.1 us.)
-// (Matrix and vector instructions dealt out one to six by the scheduler instead of a step's products in front of the sums of the one before: 40.2 -> 41.8 us.)
+// (Matrix and vector instructions dealt out one to six by the scheduler instead of a step's products in front of the sums of the one before: 40.2 -> 41.8 us; without the priorities 41.1.  Two workgroups a CU with half the
+// records a chunk, where registers allow, 5 to 8 sequences: no difference.  In 128 registers 16 sequences spill.)
+// (Q6_K's signed weights, -32 .. 31, and halves cut at 15 bits would stay in range, too: down 29.4 -> 20.3 us, the head 65 -> 38.  But they are another rounding than ql | qh << 4 less 32 times the sum of x, in the
+// single-sequence kernel as well then, and a compressed cache's codes turn on such a rounding.  With ql | qh << 4 in halves of 16 bits the low half passes 2^24, and the matrix core rounds 0.07 % of such sums otherwise than
+// to the nearest.)
 // ------------------------------------------------------------------------------------------------
 constexpr uint32_t kX8Records = 32;                  // records of a chunk at most
 constexpr uint32_t mvqb8_block_bytes(uint32_t n_seq) { return (n_seq * kXwRecord + 1023) & ~1023u; }   // a block's records in LDS: whole transfers of a wave
 typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
 
-template <int F, int NB, bool SEQ>
-__device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& L, const MvBatch& B, float* __restrict__ part, const MvSeg& S, int sg, bool active, uint8_t* smem8) {
-  static_assert(F != F_Q80, "weights of eight bits do not fit the exact range");
-  constexpr uint32_t MASK = 1u << F;
-  constexpr int NG = (NB + 7) / 8, fmt = F;
+template <uint32_t MASK, int NB, bool SEQ>
+__global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  static_assert((MASK & (MASK - 1)) == 0 && (MASK & (1u << F_Q80 | 1u << F_Q6K)) == 0, "weights of more than 5 bits do not fit the exact range");
+  constexpr int NG = (NB + 7) / 8;
   auto nq = [](int g) { return NB - 8 * g > 4 ? 2 : 1; };          // a last group of up to four sequences: one per lane
   const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
+  bool active = u < Gm.n_units;
+  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  const MvSeg& S = L.seg[active ? sg : 0];
+  constexpr int fmt = __builtin_ctz(MASK);
   auto is = [](int f) { return f == fmt; };
   constexpr uint32_t tb = fmt_tile_bytes(fmt);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
@@ -755,7 +760,7 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
     const uint32_t sb1 = min(ks * Gm.nbw + Gm.nbw, Gm.nblk);
     const uint32_t cn = chunk_len(ks, b0);
     // this wave's transfers have arrived: behind them only the next tile's loads
-    if (active) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fmt_loads_per_tile(fmt)) : "memory");
+    if (active) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fmt_loads_per_tile(__builtin_ctz(MASK))) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
     __syncthreads();
     uint32_t nks = ks, nb0 = b0 + cn;   // the chunk after this one
@@ -797,7 +802,7 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
         uint32_t tw[4][4];   // [step pp][class c]: the lane group's four weights of chunk 4 pp + c
         {
           mvq_row_scales<MASK>(fmt, nxt, lane, ts);
-          if constexpr (F == F_Q4K || F == F_Q40) {
+          if constexpr (fmt == F_Q4K || fmt == F_Q40) {
             // a word holds the nibbles of two elements' fours: whole words change halves first, then the unpacked ones rows (three swaps a step instead of four:
             // 16 sequences, gate | up 39.7 -> 39.4 us, the products split over k 12.45 -> 12.2)
 #pragma unroll
@@ -821,7 +826,7 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
             }
           }
         }
-        asm volatile("" : : "v"(tw[3][0]), "v"(ts.dd));   // (of the tile's last load)
+        asm volatile("" : : "v"(tw[3][0]));   // (of the tile's last load)
         if (bi == 0 && nks < ks1) fetch(nb0, chunk_len(nks, nb0), buf ^ 1u);   // the chunk after this one: behind this tile's wait, which would wait for it too, and in front of the next tile's loads
         {   // the unit's next tile (its next block — of this slice, or of the next one this workgroup walks)
           uint32_t bn = b + 1;
@@ -839,9 +844,6 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
               if (is(F_Q5K)) {
                 lo = __builtin_amdgcn_perm(__float_as_uint(ub1(v)), __float_as_uint(ub0(v)), 0x07060302u);
                 hi = __builtin_amdgcn_perm(__float_as_uint(ub3(v)), __float_as_uint(ub2(v)), 0x07060302u);
-              } else if (is(F_Q6K)) {
-                lo = __builtin_amdgcn_perm(__float_as_uint((float)(int8_t)(v >> 8)), __float_as_uint((float)(int8_t)v), 0x07060302u);
-                hi = __builtin_amdgcn_perm(__float_as_uint((float)((int)v >> 24)), __float_as_uint((float)(int8_t)(v >> 16)), 0x07060302u);
               } else {   // a byte up to 16 is, as an 8-bit float, 2^-9 of itself: two a conversion (gate | up as above 42.7 -> 40.3 us)
                 lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, false));
                 hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, true));
@@ -852,7 +854,7 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
           }
 #pragma unroll
           for (int pp = 0; pp < 4; pp++) d[st & 1][pp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[st & 1][pp], w[pp], zero, 0, 0, 0);
-          if (is(F_Q40)) {
+          if (!mins) {
 #pragma unroll
             for (int q = 0; q < nq(g); q++) xs[st & 1][q] = *reinterpret_cast<const f32x4*>(px[g][q] + c * 16);
           }
@@ -876,10 +878,6 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
 #pragma unroll
               for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], V[pp], s1);
               acc[g][c][q] += ts.dd * s1 - ts.dmin * s2[c & 1][2 * g + q];
-            } else if (is(F_Q6K)) {
-#pragma unroll
-              for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], V[pp], s1);
-              acc[g][c][q] = __builtin_fmaf(ts.dd, s1, acc[g][c][q]);
             } else {
 #pragma unroll
               for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], __builtin_fmaf(-8.0f, xs[st & 1][q][pp], V[pp]), s1);
@@ -929,22 +927,6 @@ __device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& 
         const uint32_t s = 8 * g + mq + 4 * q;
         if (q < nq(g) && s < n_seq) part[((size_t)slot * n_seq + s) * rows16 + (size_t)u * 16 + n] = tot[g][q];
       }
-  }
-}
-
-// (a launch of two formats: a wave takes its unit's path; both meet at the same barriers, which the launch's geometry alone decides)
-template <uint32_t MASK, int NB, bool SEQ>
-__global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
-  const uint32_t u = blockIdx.x * kBWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool active = u < Gm.n_units;
-  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
-  const MvSeg& S = L.seg[active ? sg : 0];
-  if constexpr ((MASK & (MASK - 1)) == 0) {
-    mvqb8_body<__builtin_ctz(MASK), NB, SEQ>(Gm, L, B, part, S, sg, active, smem8);
-  } else {
-    if (fmt_of_dev_type(S.type) == F_Q6K) mvqb8_body<F_Q6K, NB, SEQ>(Gm, L, B, part, S, sg, active, smem8);
-    else mvqb8_body<__builtin_ctz(MASK & ~(1u << F_Q6K)), NB, SEQ>(Gm, L, B, part, S, sg, active, smem8);
   }
 }
 
@@ -1287,12 +1269,12 @@ constexpr uint32_t kMvqb4MinSeq = 3;
 
 // Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers, us, groups of four against groups of eight over wide images, 3 / 4 sequences: an 8B model in Q4_K_M 342 / 354 against
 // 357 / 370, Q5_K_M 362 / 373 against 389 / 400, Q4_0 323 / 334 against 335 / 347; 2048 x 5632, Q4_K_M, 239 / 249 against 242 / 253; 8192 x 28672 Q4_K_M 775 / 816 against 780 / 808.  Before the wide images, with Q6_K in
-// groups of eight as two products, 5: 503 / 484 (Q4_K_M / Q4_0) against 479 / 455, 8: 531 / 512 against 502 / 480, 16: 786 / 761 against 683 / 679)
+// groups of eight too, 5: 503 / 484 (Q4_K_M / Q4_0) against 479 / 455, 8: 531 / 512 against 502 / 480, 16: 786 / 761 against 683 / 679)
 constexpr uint32_t kMvqb8MinSeq = 5;
 
 bool mvqb_wide_input(int dev_type, uint32_t n_seq) {
   const int f = fmt_of_dev_type(dev_type);
-  return n_seq >= kMvqb8MinSeq && f >= 0 && f != F_Q80;
+  return n_seq >= kMvqb8MinSeq && (f == F_Q4K || f == F_Q5K || f == F_Q40);
 }
 
 // a wide image where the input's writer left none: a workgroup per record, a thread per word of digits
@@ -1300,17 +1282,8 @@ __global__ void __launch_bounds__(256) xw_from_xq_kernel(const uint8_t* __restri
   const uint8_t* rec = xq + (size_t)blockIdx.y * xq_stride + (size_t)blockIdx.x * kXqRecord;
   uint8_t* wide = xw + (size_t)blockIdx.x * xw_block + (size_t)blockIdx.y * kXwRecord;
   const uint32_t t = threadIdx.x, i = (t >> 3) & 3, j = (t >> 5) * 2 + ((t >> 2) & 1), Q = t & 3, slot = (j & 3) * 4 + (j >> 2);   // digit 3 - i of elements 4 Q .. of chunk j
-  uint32_t limb[4], word = 0;
-#pragma unroll
-  for (uint32_t d = 0; d < 4; d++) limb[d] = *reinterpret_cast<const uint32_t*>(rec + ((t & ~0x18u) | (3 - d) << 3) * 4);   // digits d of the four elements
-#pragma unroll
-  for (uint32_t e = 0; e < 4; e++) {
-    uint32_t I = 0;
-#pragma unroll
-    for (uint32_t d = 0; d < 4; d++) I += (uint32_t)(int)(int8_t)(limb[d] >> (8 * e)) << (8 * d);
-    word |= ((xw_word((int)I) >> (8 * (3 - i))) & 0xFFu) << (8 * e);
-  }
-  *reinterpret_cast<uint2*>(wide + Q * 512 + j * 32 + (i >> 1) * 16 + (i & 1) * 8) = xw_digits(word, 3 - i, *reinterpret_cast<const float*>(rec + kXqSx16 + slot * 4));
+  const float sx = *reinterpret_cast<const float*>(rec + kXqSx16 + slot * 4) * (float)(1u << (8 * (3 - i)));
+  *reinterpret_cast<uint2*>(wide + Q * 512 + j * 32 + (i >> 1) * 16 + (i & 1) * 8) = xw_digits(*reinterpret_cast<const uint32_t*>(rec + t * 4), sx);
   if (t < 16) *reinterpret_cast<float*>(wide + kXwSums + t * 4) = *reinterpret_cast<const float*>(rec + kXqXs16 + t * 4);
 }
 
@@ -1439,7 +1412,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   }
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
-    if constexpr ((MASK & (1u << F_Q80)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
+    if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);   // (masks of two formats hold Q6_K)
     else if (B.n_seq < kMvqb8MinSeq) e = mvqb4_go<MASK, 4>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 8) e = mvqb8_go<MASK, 8>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 12) e = mvqb8_go<MASK, 12>(L, B, Gm, seq, groups, st);

@@ -59,21 +59,6 @@ __device__ __forceinline__ void mvq_issue_tile(int fmt, const uint8_t* tile, uin
     }
 }
 
-// Q6_K's sums are those of the signed weights q = (ql | qh << 4) - 32 (dequant.rs:343-350), not of ql | qh << 4 less 32 times the sum of x: two roundings fewer, and half the range.
-// Several sequences (mvq_mac_tile, mvqb8) take the weights of step pp as four times q, -128 .. 124: the six bits at the upper end of a byte, their first inverted, are that number as it stands; the row's scale takes the
-// four back, so that the bits are mvq_consume_tile's.
-__device__ __forceinline__ i32x4 mvq_q6_bytes(const RawT16& r, int pp) {
-  const uint32_t N0 = (pp & 1) ? r.q[pp >> 1].z : r.q[pp >> 1].x, N1 = (pp & 1) ? r.q[pp >> 1].w : r.q[pp >> 1].y;
-  const uint32_t H = (pp == 0 ? r.q[2].x : pp == 1 ? r.q[2].y : pp == 2 ? r.q[2].z : r.q[2].w) ^ 0xAAAAAAAAu;
-  i32x4 bw;
-  bw.x = (int)(((N0 << 2) & 0x3C3C3C3Cu) | ((H << 6) & 0xC0C0C0C0u));
-  bw.y = (int)(((N0 >> 2) & 0x3C3C3C3Cu) | ((H << 4) & 0xC0C0C0C0u));
-  bw.z = (int)(((N1 << 2) & 0x3C3C3C3Cu) | ((H << 2) & 0xC0C0C0C0u));
-  bw.w = (int)(((N1 >> 2) & 0x3C3C3C3Cu) | (H & 0xC0C0C0C0u));
-  return bw;
-}
-__device__ __forceinline__ float mvq_q6_scale(const RawT16& r, uint32_t n) { return 0.25f * h2f((n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu); }
-
 // acc += (weight rows n of the tile) . (the 256 elements of XQ record `rec`, in LDS), this lane's k-chunk c = lane >> 4 only:
 // four MFMAs (one per 64 elements); lane group c then holds, for weight row n, the four limb sums of chunk 4pp + c,
 // recombined to V = sum_k q_k * I_k (exact int, rounded once to f32).
@@ -95,26 +80,23 @@ __device__ __forceinline__ void mvq_consume_tile(int fmt, const RawT16& r, const
     if (is(F_Q6K)) {
       const uint32_t s8 = c * 8;
       const uint32_t hdw[4] = {r.hd.x, r.hd.y, r.hd.z, r.hd.w};   // int8 scales 4pp .. 4pp+3 of row n (dequant.rs:343-350)
-      const i32x4 zero = {0, 0, 0, 0}, less = (i32x4)((int)0xE0E0E0E0u);   // sixteen times -32
-      i32x4 d[4];
-#pragma unroll
-      for (int pp = 0; pp < 4; pp++) d[pp] = __builtin_amdgcn_mfma_i32_16x16x64_i8(areg[pp], less, zero, 0, 0, 0);
       float s1 = 0.0f;
 #pragma unroll
       for (int pp = 0; pp < 4; pp++) {
         const uint32_t N0 = (pp & 1) ? r.q[pp >> 1].z : r.q[pp >> 1].x, N1 = (pp & 1) ? r.q[pp >> 1].w : r.q[pp >> 1].y;
         const uint32_t H = pp == 0 ? r.q[2].x : pp == 1 ? r.q[2].y : pp == 2 ? r.q[2].z : r.q[2].w;
-        i32x4 bw;   // ql | qh << 4, 0..63; the reference's "- 32" is in the sum already (the matrix core has time, the vector ALU none)
+        i32x4 bw;   // q' = ql | qh << 4, 0..63; the reference's "- 32" is applied through the chunk's sum of x below
         bw.x = (int)((N0 & 0x0F0F0F0Fu) | ((H & 0x03030303u) << 4));
         bw.y = (int)(((N0 >> 4) & 0x0F0F0F0Fu) | (((H >> 2) & 0x03030303u) << 4));
         bw.z = (int)((N1 & 0x0F0F0F0Fu) | (((H >> 4) & 0x03030303u) << 4));
         bw.w = (int)(((N1 >> 4) & 0x0F0F0F0Fu) | (((H >> 6) & 0x03030303u) << 4));
-        d[pp] = __builtin_amdgcn_mfma_i32_16x16x64_i8(areg[pp], bw, d[pp], 0, 0, 0);
-        // both halves exact in f32 (but for a low half of 16 weights of -32 whose elements' low digits all lie within 0.4 % of their end)
-        const float hi = (float)((d[pp].x << 8) + d[pp].y), lo = (float)((d[pp].z << 8) + d[pp].w);
+        const i32x4 zero = {0, 0, 0, 0};
+        const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(areg[pp], bw, zero, 0, 0, 0);
+        // |D0| <= 64*63*16, so the high half is exact in f32; the low half may round at 2^-24 of a term that is 2^-16 of the sum
+        const float hi = (float)((d.x << 8) + d.y), lo = (float)((d.z << 8) + d.w);
         const float V = __builtin_fmaf(hi, 65536.0f, lo);
         const float scf = (float)(int)__builtin_amdgcn_sbfe((int)hdw[pp], s8, 8);
-        s1 = __builtin_fmaf(scf * sx[pp], V, s1);
+        s1 = __builtin_fmaf(scf, __builtin_fmaf(sx[pp], V, -32.0f * xs[pp]), s1);
       }
       const uint32_t dh = (n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu;
       acc = __builtin_fmaf(h2f(dh), s1, acc);
@@ -223,11 +205,17 @@ __device__ __forceinline__ void mvq_unpack_tile(int fmt, const RawT16& r, uint32
     const uint32_t hdw[4] = {r.hd.x, r.hd.y, r.hd.z, r.hd.w};
 #pragma unroll
     for (int pp = 0; pp < 4; pp++) {
-      t.bw[pp] = mvq_q6_bytes(r, pp);
+      const uint32_t N0 = (pp & 1) ? r.q[pp >> 1].z : r.q[pp >> 1].x, N1 = (pp & 1) ? r.q[pp >> 1].w : r.q[pp >> 1].y;
+      const uint32_t H = pp == 0 ? r.q[2].x : pp == 1 ? r.q[2].y : pp == 2 ? r.q[2].z : r.q[2].w;
+      t.bw[pp].x = (int)((N0 & 0x0F0F0F0Fu) | ((H & 0x03030303u) << 4));
+      t.bw[pp].y = (int)(((N0 >> 4) & 0x0F0F0F0Fu) | (((H >> 2) & 0x03030303u) << 4));
+      t.bw[pp].z = (int)((N1 & 0x0F0F0F0Fu) | (((H >> 4) & 0x03030303u) << 4));
+      t.bw[pp].w = (int)(((N1 >> 4) & 0x0F0F0F0Fu) | (((H >> 6) & 0x03030303u) << 4));
       t.f[pp] = (float)(int)__builtin_amdgcn_sbfe((int)hdw[pp], s8, 8);
       t.g[pp] = 0.0f;
     }
-    t.dd = mvq_q6_scale(r, n);
+    const uint32_t dh = (n & 1) ? r.q[3].x >> 16 : r.q[3].x & 0xFFFFu;
+    t.dd = h2f(dh);
     t.dmin = 0.0f;
   } else if (is(F_Q80) || is(F_Q40)) {
     const uint32_t hdw[4] = {r.hd.x, r.hd.y, r.hd.z, r.hd.w};
@@ -308,7 +296,7 @@ __device__ __forceinline__ void mvq_mac_finish(int fmt, const TileOps& t, const 
   if (is(F_Q6K)) {
     float s1 = 0.0f;
 #pragma unroll
-    for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(t.f[pp] * o.sx[pp], V[pp], s1);
+    for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(t.f[pp], __builtin_fmaf(o.sx[pp], V[pp], -32.0f * o.xs[pp]), s1);
     acc = __builtin_fmaf(t.dd, s1, acc);
   } else if (is(F_Q80) || is(F_Q40)) {
     float s1 = 0.0f;

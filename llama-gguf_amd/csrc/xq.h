@@ -31,35 +31,14 @@ constexpr uint32_t kXqXs16 = 1024, kXqSx16 = 1088;
 __host__ __device__ inline size_t xq_bytes(size_t k) { return (k + 255) / 256 * kXqRecord; }
 
 // The wide image of a batched step's input (matvec_batch.hip, mvqb8: its matrix cores take the digits as bf16 numbers).  A record is [element group 4][chunk 16][half 2][digit 2][element 4] bf16 (element 4 g + e of a chunk
-// of 16; the high half's digits first), a digit times its power of two times the chunk's scale, which is a power of two: exact;  then the 16 sums of XQ.  Records lie [block][sequence], blocks `xw_block` bytes apart.
-// The halves: I = hi * 2^15 + lo, |hi| <= 2^15, |lo| <= 2^14 (of a hi that would be 2^15: 2^15 - 64, hi one less), so that 16 of either, times weights up to 32, add up to 2^24 at most.  Their digits of 8 bits: the first
-// signed, the second not.
+// of 16; the high half's digits first), a digit times its power of 256 times the chunk's scale, which is a power of two: exact;  then the 16 sums of XQ.  Records lie [block][sequence], blocks `xw_block` bytes apart.
 // An odd multiple of 32 bytes: the halves of eight sequences fall into different LDS banks, whichever lane groups read at once.
 constexpr uint32_t kXwSums = 2048, kXwRecord = kXwSums + 64 + 32;
 
-// I as the bytes of its digits: high half's first, second, low half's first, second (most significant byte first)
-__device__ __forceinline__ uint32_t xw_word(int I) {
-  const int r = (I >> 15) + ((I >> 14) & 1), hi = r < 32767 ? r : 32767, lo = (int)((uint32_t)I - ((uint32_t)hi << 15));
-  return (uint32_t)hi << 16 | ((uint32_t)lo & 0xFFFFu);
-}
-// four elements' digits q (0: a word's least significant byte) times their weights; sx: the chunk's scale * 2^-30
-__device__ __forceinline__ uint2 xw_digits(uint32_t w, uint32_t q, float sx) {
-  const float s = sx * __uint_as_float((127u + (q & 1) * 8 + (q >> 1) * 15) << 23);
-  const uint32_t u = (q & 1) ? w ^ 0x80808080u : w;                              // a signed digit as itself + 128
-  const float o = (q & 1) ? -128.0f * s : 0.0f;
-  const float a = __builtin_fmaf((float)(u & 0xFFu), s, o), b = __builtin_fmaf((float)((u >> 8) & 0xFFu), s, o), c = __builtin_fmaf((float)((u >> 16) & 0xFFu), s, o),
-              d = __builtin_fmaf((float)(u >> 24), s, o);
+// four digits (a word of limb bytes) times their scale
+__device__ __forceinline__ uint2 xw_digits(uint32_t w, float s) {
+  const float a = (float)(int)(int8_t)w * s, b = (float)(int)(int8_t)(w >> 8) * s, c = (float)(int)(int8_t)(w >> 16) * s, d = (float)((int)w >> 24) * s;
   return make_uint2(__builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u), __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x07060302u));
-}
-
-// byte q of the quad's four words as one word, the quad's first lane's first (a lane's q its own)
-__device__ __forceinline__ uint32_t xq_quad_bytes(uint32_t w, uint32_t q) {
-  const uint32_t w0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x00, 0xF, 0xF, true);   // quad_perm [0,0,0,0]
-  const uint32_t w1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x55, 0xF, 0xF, true);   // [1,1,1,1]
-  const uint32_t w2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xAA, 0xF, 0xF, true);   // [2,2,2,2]
-  const uint32_t w3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xFF, 0xF, 0xF, true);   // [3,3,3,3]
-  const uint32_t sel2 = q | (q + 4) << 8;                    // byte q of the low word, byte q of the high word
-  return __builtin_amdgcn_perm(__builtin_amdgcn_perm(w3, w2, sel2), __builtin_amdgcn_perm(w1, w0, sel2), 0x05040100u);
 }
 
 // Called by the 16 consecutive lanes (a DPP row: lane % 16 == element % 16) that hold the 16 elements of chunk
@@ -80,8 +59,15 @@ __device__ __forceinline__ void xq_store_chunk(uint8_t* xq, uint32_t chunk, floa
   e = e < 30u ? 30u : (e > 250u ? 250u : e);                 // vanishing / overflowing chunks: clamp (|x'| stays < 1)
   const int I = (int)__builtin_rintf(v * __uint_as_float((283u - e) << 23));   // x' * 2^30, |I| <= 2^30
   const uint32_t w = ((uint32_t)I + 0x00808080u) ^ 0x00808080u;               // bytes = balanced digits d0..d3
+  // the quad's four words -> this lane's limb word: lane q of the quad builds digit q of elements 4Q..4Q+3
+  const uint32_t w0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x00, 0xF, 0xF, true);   // quad_perm [0,0,0,0]
+  const uint32_t w1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x55, 0xF, 0xF, true);   // [1,1,1,1]
+  const uint32_t w2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xAA, 0xF, 0xF, true);   // [2,2,2,2]
+  const uint32_t w3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xFF, 0xF, 0xF, true);   // [3,3,3,3]
   const uint32_t q = l16 & 3, Q = l16 >> 2;
-  const uint32_t word = xq_quad_bytes(w, q);                 // lane q of the quad: digit q of elements 4Q..4Q+3
+  const uint32_t sel2 = q | (q + 4) << 8;                    // byte q of the low word, byte q of the high word
+  const uint32_t lo = __builtin_amdgcn_perm(w1, w0, sel2), hi = __builtin_amdgcn_perm(w3, w2, sel2);
+  const uint32_t word = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
   const uint32_t blk = chunk >> 4, j = chunk & 15, g = j >> 1, i = 3 - q;
   uint8_t* rec = xq + (size_t)blk * kXqRecord;
   *reinterpret_cast<uint32_t*>(rec + (g * 4 + i) * 32 + (j & 1) * 16 + Q * 4) = word;
@@ -93,7 +79,7 @@ __device__ __forceinline__ void xq_store_chunk(uint8_t* xq, uint32_t chunk, floa
   }
   if (xw) {
     uint8_t* wide = xw + (size_t)blk * xw_block;
-    *reinterpret_cast<uint2*>(wide + Q * 512 + j * 32 + (i >> 1) * 16 + (i & 1) * 8) = xw_digits(xq_quad_bytes(xw_word(I), q), q, __uint_as_float((e + 1u - 30u) << 23));
+    *reinterpret_cast<uint2*>(wide + Q * 512 + j * 32 + (i >> 1) * 16 + (i & 1) * 8) = xw_digits(word, __uint_as_float((e + 1u - 30u + 8u * q) << 23));
     if (l16 == 0) *reinterpret_cast<float*>(wide + kXwSums + ((j & 3) * 4 + (j >> 2)) * 4) = sum;
   }
 }

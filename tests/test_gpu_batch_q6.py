@@ -1,7 +1,7 @@
-"""Six-bit weights in groups of eight sequences on the bf16 matrix cores (matvec_batch.hip, mvqb8): alone with whole rows per workgroup and with k-slices, and beside four- and five-bit ones in one launch, whose workgroups
-walk all of k there too (24576 rows of Q, K and V).  Group sizes of every instantiation.
+"""Six-bit weights in a batched step: alone with whole rows per workgroup and with k-slices, and beside four- and five-bit ones in one launch, whose workgroups walk all of k there too (24576 rows of Q, K and V).  Group sizes
+of every instantiation.
 
-The sums are exact and rounded once, as the single-sequence kernel's: equality of all bits."""
+The sums and their roundings are the single-sequence kernel's: equality of all bits."""
 import numpy as np
 import pytest
 
