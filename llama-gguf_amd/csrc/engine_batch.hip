@@ -147,7 +147,7 @@ int launch_mvb(lgh_ctx* c, int cls, const SegSpec* specs, int nseg, const float*
   // wide images (xq.h): the input's, made here where its writer left none; the output's, where its reader takes one
   B.xw_block = Bs.xw_block;
   bool wide = !ind.cnt;
-  for (int s = 0; s < nseg; s++) wide = wide && specs[s].W[0]->type == specs[0].W[0]->type && mvqb_wide_input(specs[s].W[0]->type, n_seq);
+  for (int s = 0; s < nseg; s++) wide = wide && mvqb_wide_input(specs[s].W[0]->type, n_seq);
   if (XqBuf* q = wide ? view_of(c, specs[0].x[0]) : nullptr; q && q->xw) {
     if (!q->wide && (rc = run_k(c, LGH_K_MISC, LGH_SYM_OTHER, 0, [&] { return xw_from_xq_launch(q->xq, B.xq_stride, q->xw, Bs.xw_block, k, n_seq, c->stream); }))) return rc;
     q->wide = true;
@@ -193,10 +193,7 @@ int enqueue_multi(lgh_ctx* c, uint32_t n_seq, bool greedy) {
   int rc;
   auto stale_all = [&] { for (auto& q : c->xqs) q.fresh = q.wide = false; };
   // whose wide image (xq.h) the launch that reads it takes: attention's output for wo, the activations for down, the residual stream for Q, K, V (one launch, or one each: below), gate | up and the output head
-  auto wide_qkv = [&](uint32_t li) {
-    const int q = c->layers[li].wq.type, k = c->layers[li].wk.type, v = c->layers[li].wv.type;
-    return mvqb_wide_input(q, n_seq) && ((q == k && q == v) || q == kDevQ40_T16);
-  };
+  auto wide_qkv = [&](uint32_t li) { return mvqb_wide_input(c->layers[li].wq.type, n_seq); };   // (in one launch with K and V the formats are wide ones all, and alone it is Q's)
   auto wide_hidden = [&](uint32_t li) { return li < c->l1 ? wide_qkv(li) : mvqb_wide_input(c->output.type, n_seq); };
   auto wide_of = [&](float* f32, bool want) -> uint8_t* {   // the image for a launch that writes vector f32, marked as written
     XqBuf* q = want ? view_of(c, f32) : nullptr;

@@ -12,7 +12,7 @@
 // the sequences' records staged ONCE per workgroup in LDS and shared by its 8 waves, sequences two at a time (the pair's 8 MFMAs,
 // then the vector work while the next pair's operands load), the epilogue as a second small launch — what bounded the first
 // structure and what each change bought: profiles/r03e_batched_decode.md.  From three sequences on its products take the sequences in
-// groups of four (mvqb4) or, from five on and for weights below 6 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
+// groups of four (mvqb4) or, from five on and for weights of up to 6 bits, of eight (mvqb8).  mvqb (first): the single-sequence decomposition (a
 // workgroup = the 8 k-slices of a few row tiles) with a loop over the sequences inside it and their records from L2 into a
 // register ring; kept for one sequence and for launches whose segments do not share their input vector.
 // Epilogues: store, +residual, SwiGLU pair, RoPE (every sequence at its own position) and the K / V rows into the sequence's
@@ -679,43 +679,44 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb4_kernel(const Mvqb2Geom Gm,
 }
 
 // ------------------------------------------------------------------------------------------------
-// The same for formats whose weights are whole numbers below 32 (all but Q6_K and Q8_0), on the bf16 matrix cores: what a digit needs beside its product moves into the
+// The same for formats whose weights are whole numbers below 32 (Q6_K: below), on the bf16 matrix cores: what a digit needs beside its product moves into the
 // operands.  mvqb4 spends eight vector instructions per (row, sequence, 16 elements): two shifts and additions of digit sums, two conversions, a fused
 // multiply-add, and the scales.  Here a digit is a bf16 number, the digit times its power of 256 times the chunk's scale, itself a power of two (both exact),
 // and the high two and the low two digits of 16 elements lie along one K of 32: the product IS the scaled high or low half, in f32.  Every partial sum is a whole
 // multiple of the scale below 2^24 of it (16 elements, weights <= 31; high half |I| >> 16 <= 2^14: 31 * 2^18; low half, two balanced digits, up to 128 * 256 + 128: 16 * 31 * 32896 = 16 316 416),
-// so nothing rounds in it.  (Weights of six bits would reach 33 158 336 in the low half, and beyond 2^24 the matrix instruction rounds where the integer sum does not.)  What is left is one
+// so nothing rounds in it.  What is left is one
 // addition (the halves: the rounding that the fused multiply-add of the other kernels does, shifted by a power of two) and the fused multiply-add with the weights' scale: the same
 // bits.  The sum over the minima, a chain of four fused multiply-adds, is a 16x16x4 f32 matrix instruction, which rounds as that chain does.
 //   A: row 4 m + 2 q + half of sequence m + 4 q of eight (a lane of group m gets both halves of sequences m and m + 4), K = lane group's four elements of the half's first digit, then of its second
 //   B: the lane group's four weights twice; a lane unpacks one chunk of 64 elements, so the chunks' words are exchanged between the lane groups (4 x 4, four swaps, of packed words three)
 // (Inputs beyond 2^117 in magnitude may overflow a half where a zero scale would have hidden it.)
+// Q6_K: 0 .. 63 would reach 33 158 336 in the low half, and of sums beyond 2^24 the matrix instruction rounds some (0.07 % of those made so on purpose) otherwise than to the nearest.  So a row of A is ONE digit of one of four
+// sequences, K the chunk's 16 elements: a digit's sum is exact whatever its weights, the high half's addition is exact (63 * 2^18), the low half's rounds as the integer's conversion does, and the third is the one above:
+// twice the matrix instructions (which have the time) and two additions more a sum.  Against the integer cores (mvqb4: 843 vector instructions a tile and block of 16 sequences), 16 sequences of an 8B model: down
+// 29.5 -> 24.2 us, Q, K and V with one Q6_K matrix 21.0 -> 16.0, the head (32000 rows) 65 -> 51; a step of 4 layers, us, 5 / 8 / 16 sequences: Q4_K_M 382 / 410 / 588 -> 371 / 403 / 556, Q6_K 440 / 472 / 709 -> 405 / 447 / 628,
+// Q5_K_M 411 / 440 / 614 -> 398 / 430 / 578; Mixtral Q5_K_M, one layer, 297 / 374 / 554 -> 288 / 365 / 530.
+// (Signed weights, -32 .. 31, and halves cut at 15 bits need no second product, 20.3, 15.0 and 38 us for the three.  But they are another rounding than ql | qh << 4 less 32 times the sum of x, in the single-sequence kernel
+// as well then, and a compressed cache's codes turn on such a rounding.)
 // Who writes the input leaves it in this form (xq.h: the wide image), and a chunk's records of all sequences come as they lie in memory, a chunk ahead, by LDS-DMA.  Rewritten from the digits by every workgroup as they
 // were staged, they took a quarter of the vector instructions.  gate | up of an 8B model (28672 rows of 4096, Q4_K): 16 sequences 47.4 -> 42.7 us (58 with mvqb4), 8 33.7 -> 30.5; wo 13.6 -> 12.4; a step of 4 layers, 16
 // sequences, Q4_K_M 639 -> 617 us, Q4_0 599 -> 554.  Bound by the vector instructions: 339 a tile and block of 16 sequences, 192 of them the sums' own, 65 % of the SIMDs' cycles (the matrix cores 23 %; two waves a SIMD).
 // (Matrix and vector instructions dealt out one to six by the scheduler instead of a step's products in front of the sums of the one before: 40.2 -> 41.8 us; without the priorities 41.1.  Two workgroups a CU with half the
 // records a chunk, where registers allow, 5 to 8 sequences: no difference.  In 128 registers 16 sequences spill.)
-// (Q6_K's signed weights, -32 .. 31, and halves cut at 15 bits would stay in range, too: down 29.4 -> 20.3 us, the head 65 -> 38.  But they are another rounding than ql | qh << 4 less 32 times the sum of x, in the
-// single-sequence kernel as well then, and a compressed cache's codes turn on such a rounding.  With ql | qh << 4 in halves of 16 bits the low half passes 2^24, and the matrix core rounds 0.07 % of such sums otherwise than
-// to the nearest.)
 // ------------------------------------------------------------------------------------------------
 constexpr uint32_t kX8Records = 32;                  // records of a chunk at most
 constexpr uint32_t mvqb8_block_bytes(uint32_t n_seq) { return (n_seq * kXwRecord + 1023) & ~1023u; }   // a block's records in LDS: whole transfers of a wave
 typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-template <uint32_t MASK, int NB, bool SEQ>
-__global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
-  static_assert((MASK & (MASK - 1)) == 0 && (MASK & (1u << F_Q80 | 1u << F_Q6K)) == 0, "weights of more than 5 bits do not fit the exact range");
-  constexpr int NG = (NB + 7) / 8;
+template <int F, int NB, bool SEQ>
+__device__ __forceinline__ void mvqb8_body(const Mvqb2Geom& Gm, const MvLaunch& L, const MvBatch& B, float* __restrict__ part, const MvSeg& S, int sg, bool active, uint8_t* smem8) {
+  static_assert(F != F_Q80, "weights of eight bits do not fit the exact range");
+  constexpr uint32_t MASK = 1u << F;
+  constexpr int NG = (NB + 7) / 8, fmt = F;
   auto nq = [](int g) { return NB - 8 * g > 4 ? 2 : 1; };          // a last group of up to four sequences: one per lane
   const uint32_t tid = threadIdx.x, lane = tid & 63, n_seq = B.n_seq;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t u = blockIdx.x * kBWaves + wave;                 // this wave's unit
-  bool active = u < Gm.n_units;
-  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
-  const MvSeg& S = L.seg[active ? sg : 0];
-  constexpr int fmt = __builtin_ctz(MASK);
   auto is = [](int f) { return f == fmt; };
   constexpr uint32_t tb = fmt_tile_bytes(fmt);
   const uint32_t ntiles = (S.n_rows + 15) >> 4;
@@ -760,7 +761,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
     const uint32_t sb1 = min(ks * Gm.nbw + Gm.nbw, Gm.nblk);
     const uint32_t cn = chunk_len(ks, b0);
     // this wave's transfers have arrived: behind them only the next tile's loads
-    if (active) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fmt_loads_per_tile(__builtin_ctz(MASK))) : "memory");
+    if (active) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fmt_loads_per_tile(fmt)) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
     __syncthreads();
     uint32_t nks = ks, nb0 = b0 + cn;   // the chunk after this one
@@ -774,6 +775,83 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
         const uint32_t b = b0 + bi;
         // sequences past the last one repeat it: computed, never stored
         const uint8_t* rec0 = smem8 + buf * buf_bytes + bi * blk_bytes;
+        if constexpr (F == F_Q6K) {   // one digit of one sequence a row: sequence 4 g + mq is the (g & 1)-th of group g >> 1
+          constexpr int N4 = NB / 4, kSteps = 4 * N4;
+          const uint8_t *pa[N4], *px[N4];
+#pragma unroll
+          for (int g = 0; g < N4; g++) {
+            pa[g] = rec0 + min(4 * g + (n >> 2), n_seq - 1) * kXwRecord + mq * 512 + (n & 3) * 8;
+            px[g] = rec0 + min(4 * g + mq, n_seq - 1) * kXwRecord + kXwSums;
+          }
+          s16x4 a[2][4], w[4];
+          f32x4 d[2][4], xs[2];
+          auto load_a = [&](int st) {
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) a[st & 1][pp] = *reinterpret_cast<const s16x4*>(pa[st % N4] + (pp * 4 + st / N4) * 32);
+          };
+          load_a(0);
+          load_a(1);
+          TileScales ts;
+          uint32_t tw[4][4];
+          {
+            TileOps t;
+            mvq_unpack_tile<MASK>(fmt, nxt, lane, t);
+            mvq_row_scales<MASK>(fmt, nxt, lane, ts);
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) {
+              const auto r01 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][0], (uint32_t)t.bw[pp][1], false, false);
+              const auto r23 = __builtin_amdgcn_permlane16_swap((uint32_t)t.bw[pp][2], (uint32_t)t.bw[pp][3], false, false);
+              const auto r02 = __builtin_amdgcn_permlane32_swap(r01[0], r23[0], false, false);
+              const auto r13 = __builtin_amdgcn_permlane32_swap(r01[1], r23[1], false, false);
+              tw[pp][0] = r02[0]; tw[pp][1] = r13[0]; tw[pp][2] = r02[1]; tw[pp][3] = r13[1];
+            }
+          }
+          asm volatile("" : : "v"(tw[3][0]), "v"(ts.dd));   // (of the tile's last loads)
+          if (bi == 0 && nks < ks1) fetch(nb0, chunk_len(nks, nb0), buf ^ 1u);
+          {
+            uint32_t bn = b + 1;
+            if (bn == sb1) bn = nks < ks1 ? nb0 : Gm.nblk;
+            if (bn < Gm.nblk) mvq_issue_tile<MASK>(fmt, wbase + (size_t)bn * tb, lane, nxt);
+          }
+          const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+          auto products = [&](int st) {
+            const int c = st / N4, g = st % N4;
+            if (g == 0) {
+#pragma unroll
+              for (int pp = 0; pp < 4; pp++) {
+                const uint32_t v = tw[pp][c];
+                w[pp] = __builtin_bit_cast(s16x4, make_uint2(__builtin_amdgcn_perm(__float_as_uint(ub1(v)), __float_as_uint(ub0(v)), 0x07060302u),
+                                                             __builtin_amdgcn_perm(__float_as_uint(ub3(v)), __float_as_uint(ub2(v)), 0x07060302u)));
+              }
+            }
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) d[st & 1][pp] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[st & 1][pp], w[pp], zero, 0, 0, 0);
+            xs[st & 1] = *reinterpret_cast<const f32x4*>(px[g] + c * 16);
+          };
+          products(0);
+#pragma unroll
+          for (int st = 0; st < kSteps; st++) {
+            const int c = st / N4, g = st % N4;
+            if (st + 1 < kSteps) {
+              __builtin_amdgcn_s_setprio(1);
+              products(st + 1);
+              __builtin_amdgcn_s_setprio(0);
+            }
+            if (st + 2 < kSteps) load_a(st + 2);
+            float s1 = 0.0f, V[4];
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) {   // high half exact; low half, where it passes 2^24, rounded as the integer's conversion rounds it
+              const f32x4 e = d[st & 1][pp];
+              V[pp] = (e[0] + e[1]) + (e[2] + e[3]);
+            }
+#pragma unroll
+            for (int pp = 0; pp < 4; pp++) s1 = __builtin_fmaf(ts.f[pp][c], __builtin_fmaf(-32.0f, xs[st & 1][pp], V[pp]), s1);
+            acc[g >> 1][c][g & 1] = __builtin_fmaf(ts.dd, s1, acc[g >> 1][c][g & 1]);
+            asm volatile("" : "+v"(acc[g >> 1][c][g & 1]));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          continue;
+        }
         const uint8_t *pa[NG], *px[NG][2];
 #pragma unroll
         for (int g = 0; g < NG; g++) {
@@ -802,7 +880,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
         uint32_t tw[4][4];   // [step pp][class c]: the lane group's four weights of chunk 4 pp + c
         {
           mvq_row_scales<MASK>(fmt, nxt, lane, ts);
-          if constexpr (fmt == F_Q4K || fmt == F_Q40) {
+          if constexpr (F == F_Q4K || F == F_Q40) {
             // a word holds the nibbles of two elements' fours: whole words change halves first, then the unpacked ones rows (three swaps a step instead of four:
             // 16 sequences, gate | up 39.7 -> 39.4 us, the products split over k 12.45 -> 12.2)
 #pragma unroll
@@ -826,7 +904,7 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
             }
           }
         }
-        asm volatile("" : : "v"(tw[3][0]));   // (of the tile's last load)
+        asm volatile("" : : "v"(tw[3][0]), "v"(ts.dd));   // (of the tile's last load)
         if (bi == 0 && nks < ks1) fetch(nb0, chunk_len(nks, nb0), buf ^ 1u);   // the chunk after this one: behind this tile's wait, which would wait for it too, and in front of the next tile's loads
         {   // the unit's next tile (its next block — of this slice, or of the next one this workgroup walks)
           uint32_t bn = b + 1;
@@ -927,6 +1005,22 @@ __global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm,
         const uint32_t s = 8 * g + mq + 4 * q;
         if (q < nq(g) && s < n_seq) part[((size_t)slot * n_seq + s) * rows16 + (size_t)u * 16 + n] = tot[g][q];
       }
+  }
+}
+
+// (a launch of two formats: a wave takes its unit's path; both meet at the same barriers, which the launch's geometry alone decides)
+template <uint32_t MASK, int NB, bool SEQ>
+__global__ void __launch_bounds__(kBWaves * 64) mvqb8_kernel(const Mvqb2Geom Gm, const MvLaunch L, const MvBatch B, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem8[];
+  const uint32_t u = blockIdx.x * kBWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool active = u < Gm.n_units;
+  const int sg = SEQ && Gm.fuse ? 0 : (int)(u >= Gm.ub1) + (int)(u >= Gm.ub2);
+  const MvSeg& S = L.seg[active ? sg : 0];
+  if constexpr ((MASK & (MASK - 1)) == 0) {
+    mvqb8_body<__builtin_ctz(MASK), NB, SEQ>(Gm, L, B, part, S, sg, active, smem8);
+  } else {
+    if (fmt_of_dev_type(S.type) == F_Q6K) mvqb8_body<F_Q6K, NB, SEQ>(Gm, L, B, part, S, sg, active, smem8);
+    else mvqb8_body<__builtin_ctz(MASK & ~(1u << F_Q6K)), NB, SEQ>(Gm, L, B, part, S, sg, active, smem8);
   }
 }
 
@@ -1269,12 +1363,12 @@ constexpr uint32_t kMvqb4MinSeq = 3;
 
 // Sequences from which groups of eight on the bf16 matrix cores are the faster ones (a step, 4 layers, us, groups of four against groups of eight over wide images, 3 / 4 sequences: an 8B model in Q4_K_M 342 / 354 against
 // 357 / 370, Q5_K_M 362 / 373 against 389 / 400, Q4_0 323 / 334 against 335 / 347; 2048 x 5632, Q4_K_M, 239 / 249 against 242 / 253; 8192 x 28672 Q4_K_M 775 / 816 against 780 / 808.  Before the wide images, with Q6_K in
-// groups of eight too, 5: 503 / 484 (Q4_K_M / Q4_0) against 479 / 455, 8: 531 / 512 against 502 / 480, 16: 786 / 761 against 683 / 679)
+// groups of eight as two products, 5: 503 / 484 (Q4_K_M / Q4_0) against 479 / 455, 8: 531 / 512 against 502 / 480, 16: 786 / 761 against 683 / 679)
 constexpr uint32_t kMvqb8MinSeq = 5;
 
 bool mvqb_wide_input(int dev_type, uint32_t n_seq) {
   const int f = fmt_of_dev_type(dev_type);
-  return n_seq >= kMvqb8MinSeq && (f == F_Q4K || f == F_Q5K || f == F_Q40);
+  return n_seq >= kMvqb8MinSeq && f >= 0 && f != F_Q80;
 }
 
 // a wide image where the input's writer left none: a workgroup per record, a thread per word of digits
@@ -1412,7 +1506,7 @@ static hipError_t mvqb2_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g,
   }
   if (!B.ind_cnt && B.n_seq >= kMvqb4MinSeq) {
     hipError_t e;
-    if constexpr ((MASK & (1u << F_Q80 | 1u << F_Q6K)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);   // (masks of two formats hold Q6_K)
+    if constexpr ((MASK & (1u << F_Q80)) != 0) e = mvqb4_go<MASK, NB>(L, B, Gm, seq, groups, st);
     else if (B.n_seq < kMvqb8MinSeq) e = mvqb4_go<MASK, 4>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 8) e = mvqb8_go<MASK, 8>(L, B, Gm, seq, groups, st);
     else if (B.n_seq <= 12) e = mvqb8_go<MASK, 12>(L, B, Gm, seq, groups, st);

@@ -1,4 +1,4 @@
-"""Six-bit weights in a batched step: alone with whole rows per workgroup and with k-slices, and beside four- and five-bit ones in one launch, whose workgroups walk all of k there too (24576 rows of Q, K and V).  Group sizes
+"""Six-bit weights in a batched step, from five sequences on one digit a row on the bf16 matrix cores (matvec_batch.hip, mvqb8): alone with whole rows per workgroup and with k-slices, and beside four- and five-bit ones in one launch, whose workgroups walk all of k there too (24576 rows of Q, K and V).  Group sizes
 of every instantiation.
 
 The sums and their roundings are the single-sequence kernel's: equality of all bits."""
