@@ -410,6 +410,8 @@ int lgh_synchronize(lgh_ctx* ctx);
 int lgh_read_hidden(lgh_ctx* ctx, float* out);
 /* debug: the nth device allocation of this context from now on fails as if the memory were gone, the ones after it succeed (0: none fails) */
 int lgh_debug_fail_alloc(lgh_ctx* ctx, uint32_t nth);
+/* debug: the nth launch of this context from now on is reported as failed, the ones after it not (0: none).  A kernel's launch is queued all the same; a step's graph is not. */
+int lgh_debug_fail_launch(lgh_ctx* ctx, uint32_t nth);
 
 /* ---- pipeline stages over xGMI (replaces ShardServer::forward, src/distributed/shard.rs:377-445) ----
  * The hop between stages is one f32[hidden_size] vector; the host side moves it with RCCL

@@ -143,6 +143,7 @@ struct lgh_ctx {
   bool profiling = false;
   std::string err;
   uint32_t fail_alloc = 0;                         // lgh_debug_fail_alloc
+  uint32_t fail_launch = 0;                        // lgh_debug_fail_launch
   hipGraphExec_t graph[lgh::MODE_COUNT][2][2] = {};   // [mode][attention variant: 0 split + combine, 1 single launch (short context)][1: a step that the host feeds, see step()]
   bool attn_direct = false;                        // variant of the token being enqueued (chosen by the host-side position)
   uint32_t direct_attn_max_kv = 0;                 // contexts up to this many rows take the single-launch attention
@@ -248,6 +249,7 @@ inline int run_k(lgh_ctx* c, int cls, int sym, uint64_t alg_bytes, F&& f) {
     (void)hipEventRecord(rec.a, c->stream);
   }
   hipError_t e = f();
+  if (c->fail_launch && --c->fail_launch == 0 && e == hipSuccess) e = hipErrorUnknown;   // (queued all the same)
   if (e != hipSuccess) return fail(c, LGH_OPERATION_FAILED, std::string("kernel launch (class ") + std::to_string(cls) + "): " + hipGetErrorString(e));
   if (c->profiling) {
     (void)hipEventRecord(rec.b, c->stream);

@@ -835,6 +835,12 @@ static int set_token(lgh_ctx* c, uint32_t token) {
   return LGH_OK;
 }
 
+static int graph_go(lgh_ctx* c, hipGraphExec_t ge) {
+  if (c->fail_launch && --c->fail_launch == 0) return fail(c, LGH_OPERATION_FAILED, "hipGraphLaunch: refused on request (lgh_debug_fail_launch)");
+  HIP_TRY(c, LGH_OPERATION_FAILED, hipGraphLaunch(ge, c->stream));
+  return LGH_OK;
+}
+
 // run one token in `mode`: the state word's, or the host's (`token`).  A step that the host feeds has the token in the arguments of its first launch, which is not part of the graph then (a fill in front of the graph was
 // 3 us, and 4 until the graph began), and its logits go to the pinned memory with its last one (a launch behind a graph begins 9 to 12 us after it, one inside 1.5).
 static int step(lgh_ctx* c, int mode, const uint32_t* token = nullptr) {
@@ -843,18 +849,24 @@ static int step(lgh_ctx* c, int mode, const uint32_t* token = nullptr) {
   if (token && c->first && *token >= c->d.vocab_size) return fail(c, LGH_INVALID_ARGUMENT, "token id exceeds vocab size");  // llama.rs:296-302
   if (c->pos >= c->d.max_seq_len)  // the reference has no such check: OOB write past the KV capacity
     return fail(c, LGH_INVALID_ARGUMENT, "position " + std::to_string(c->pos) + " >= max_seq_len " + std::to_string(c->d.max_seq_len));
-  int rc;
+  int rc = LGH_OK;
+  (void)hipGetLastError();   // (an error that another library's call left in this thread: a launch's check would find it)
   c->attn_direct = c->pos + 1 <= direct_attn_rows(c);   // the token at position pos attends to pos + 1 rows
+  const bool fed = token != nullptr;
+  if (graphs && (rc = ensure_graph(c, mode, fed))) return rc;   // (captures: nothing has been launched yet)
+  if (token && !(graphs && given_tokens(c))) rc = set_token(c, *token);
   if (!graphs) {
-    if (token && (rc = set_token(c, *token))) return rc;
-    if ((rc = enqueue_token(c, mode))) return rc;
-    if (c->profiling && (rc = drain_prof(c))) return rc;
+    if (!rc) rc = enqueue_token(c, mode);
+    if (!rc && c->profiling) rc = drain_prof(c);
   } else {
-    const bool fed = token != nullptr;
-    if ((rc = ensure_graph(c, mode, fed))) return rc;
-    if (fed && (rc = given_tokens(c) ? token_begin(c, (int)*token) : set_token(c, *token))) return rc;
-    HIP_TRY(c, LGH_OPERATION_FAILED, hipGraphLaunch(c->graph[mode][c->attn_direct ? 1 : 0][fed ? 1 : 0], c->stream));
-    if (fed && mode == MODE_FORWARD && c->out.in_graph[c->attn_direct ? 1 : 0]) { c->out.in_step = true; c->out.number++; }
+    if (fed && given_tokens(c)) rc = token_begin(c, (int)*token);
+    if (!rc) rc = graph_go(c, c->graph[mode][c->attn_direct ? 1 : 0][fed ? 1 : 0]);
+    if (!rc && fed && mode == MODE_FORWARD && c->out.in_graph[c->attn_direct ? 1 : 0]) { c->out.in_step = true; c->out.number++; }
+  }
+  if (rc) {
+    // The step's first launch has raised the device's word for the next position where it was queued: back to what the host counts, or the next token would be a row too far.
+    (void)hipMemsetD32Async((hipDeviceptr_t)(c->state + ST_NEXT), (int)c->pos, 1, c->stream);
+    return rc;
   }
   c->pos += 1;
   c->stats.tokens_processed += 1;
@@ -2259,6 +2271,12 @@ int lgh_synchronize(lgh_ctx* c) {
 int lgh_debug_fail_alloc(lgh_ctx* c, uint32_t nth) {
   if (!c) return LGH_INVALID_ARGUMENT;
   c->fail_alloc = nth;
+  return LGH_OK;
+}
+
+int lgh_debug_fail_launch(lgh_ctx* c, uint32_t nth) {
+  if (!c) return LGH_INVALID_ARGUMENT;
+  c->fail_launch = nth;
   return LGH_OK;
 }
 

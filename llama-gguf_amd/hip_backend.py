@@ -29,7 +29,7 @@ ABI_SYMBOLS = (
     "lgh_op_matvec_q", "lgh_op_attention", "lgh_op_attention_prompt", "lgh_backend_create", "lgh_backend_destroy", "lgh_backend_load_weight",
     "lgh_backend_has_weight", "lgh_backend_vec_mat_q", "lgh_backend_last_error", "lgh_reset", "lgh_position", "lgh_kv_truncate", "lgh_kv_shift_left", "lgh_stage_prefill_batch", "lgh_stage_hidden_block_buffer", "lgh_forward_argmax", "lgh_decode_greedy",
     "lgh_last_error", "lgh_get_stats", "lgh_beside_blocks", "lgh_set_profiling", "lgh_set_stream", "lgh_get_stream", "lgh_synchronize",
-    "lgh_read_hidden", "lgh_debug_fail_alloc", "lgh_stage_hidden_buffer", "lgh_stage_forward", "lgh_op_dequantize", "lgh_op_vec_mat",
+    "lgh_read_hidden", "lgh_debug_fail_alloc", "lgh_debug_fail_launch", "lgh_stage_hidden_buffer", "lgh_stage_forward", "lgh_op_dequantize", "lgh_op_vec_mat",
     "lgh_op_rms_norm", "lgh_op_rope", "lgh_op_attention_cached", "lgh_op_silu_mul", "lgh_op_norm_vec_mat",
     "lgh_op_swiglu_vec_mat", "lgh_bench_vec_mat", "lgh_bench_hbm_read", "lgh_gguf_inspect", "lgh_load_gguf",
     "lgh_stage_io_buffers", "lgh_stage_set_forward_targets", "lgh_stage_step", "lgh_stage_read_tokens", "lgh_gguf_get", "lgh_stage_read_logits",
@@ -159,7 +159,7 @@ def load_library() -> C.CDLL:
         "lgh_beside_blocks": (C.c_int, [vp, C.POINTER(C.c_int), C.POINTER(C.c_uint64)]),
         "lgh_set_profiling": (C.c_int, [vp, C.c_int]), "lgh_set_stream": (C.c_int, [vp, vp]),
         "lgh_get_stream": (vp, [vp]), "lgh_synchronize": (C.c_int, [vp]), "lgh_read_hidden": (C.c_int, [vp, vp]),
-        "lgh_debug_fail_alloc": (C.c_int, [vp, u32]),
+        "lgh_debug_fail_alloc": (C.c_int, [vp, u32]), "lgh_debug_fail_launch": (C.c_int, [vp, u32]),
         "lgh_stage_hidden_buffer": (C.c_int, [vp, C.POINTER(vp)]),
         "lgh_stage_forward": (C.c_int, [vp, u32, C.c_int, vp, C.POINTER(u32)]),
         "lgh_op_dequantize": (C.c_int, [C.c_int, u32, vp, sz, vp]),
@@ -511,6 +511,9 @@ class HipGpuInference:
 
     def debug_fail_alloc(self, nth: int) -> None:
         self._call(load_library().lgh_debug_fail_alloc(self._h, nth))
+
+    def debug_fail_launch(self, nth: int) -> None:
+        self._call(load_library().lgh_debug_fail_launch(self._h, nth))
 
     def read_hidden(self) -> np.ndarray:
         out = np.empty(self.hidden_size, dtype=np.float32)
