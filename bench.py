@@ -32,14 +32,16 @@ import __graft_entry__ as graft  # noqa: E402
 # guides/MI355X_MICROARCH.md "HBM traffic"), which cannot be collected from inside this process: tools/gpu_measure.sh
 # runs them on the same command and tools/summarize_profiles.py commits the per-kernel table under profiles/.  The
 # newest committed table is what `roofline.traffic` reports (with its file name), null when there is none.
-def committed_traffic(kernel):
+def committed_traffic(kernel, tables=None):
     import csv
-    tables = sorted((Path(__file__).resolve().parent / "profiles").glob("*_pmc_traffic.csv"))
+    tables = sorted((Path(__file__).resolve().parent / "profiles").glob("*_pmc_traffic.csv")) if tables is None else tables
     for t in reversed(tables):
         with open(t, newline="") as f:
-            for row in csv.DictReader(f):
-                if row["kernel"] == kernel and int(row["launches_fetch_pass"]) > 0:
-                    return int(float(row["hbm_bytes_per_launch_corrected"])), t.name
+            rows = {row["kernel"]: row for row in csv.DictReader(f) if int(row["launches_fetch_pass"]) > 0}
+        found = graft.load_package().hip_backend.symbol_rows(kernel, list(rows))
+        if found:   # (a symbol of several kernels: the mean over their launches)
+            n = {k: int(rows[k]["launches_fetch_pass"]) for k in found}
+            return int(sum(float(rows[k]["hbm_bytes_per_launch_corrected"]) * n[k] for k in found) / sum(n.values())), t.name
     return None, None
 
 

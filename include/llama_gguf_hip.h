@@ -140,9 +140,9 @@ enum {
 
 /* kernel SYMBOLS reported by lgh_get_stats (profiling mode): what `rocprofv3 --kernel-trace --stats` groups by.
  * LGH_SYM_MV_* are the instantiations of lgh::mv_kernel<MASK, MAXT> (the VALU dequant mat-vec, csrc/matvec.hip; MASK bits:
- * Q4_K 1, Q5_K 2, Q6_K 4, Q8_0 8, Q4_0 16; MAXT = the instantiation's thread cap).  LGH_SYM_MVQ_* are the instantiations of
- * lgh::mvq_kernel<MASK>, lgh::mvq_rows_kernel<MASK, ..> (the int8 matrix-core mat-vec, csrc/matvec_mfma.hip; ITS mask bits: Q4_K 1, Q6_K 2, Q5_K 4, Q8_0 8,
- * Q4_0 16). */
+ * Q4_K 1, Q5_K 2, Q6_K 4, Q8_0 8, Q4_0 16; MAXT = the instantiation's thread cap).  LGH_SYM_MVQ_* are the int8 matrix-core mat-vec
+ * (csrc/matvec_mfma.hip; ITS mask bits: Q4_K 1, Q6_K 2, Q5_K 4, Q8_0 8, Q4_0 16), one symbol a format: lgh::mvq_kernel<MASK> (Q, K and V of a layer, the only
+ * launches of two formats) and lgh::mvq_rows_kernel<MASK, KIND> (everything else) together. */
 enum {
   LGH_SYM_MV_Q4K = 0,      /* lgh::mv_kernel<1u, 1024>  : every matrix of the launch Q4_K */
   LGH_SYM_MV_Q80 = 1,      /* lgh::mv_kernel<8u, 1024>  : Q8_0 */
@@ -159,11 +159,11 @@ enum {
   LGH_SYM_ARGMAX = 12,     /* argmax_stage1 + argmax_stage2 (two launches, timed together) */
   LGH_SYM_ROUTER = 13,
   LGH_SYM_OTHER = 14,
-  LGH_SYM_MVQ_Q4K = 15,    /* lgh::mvq_kernel<1u> : int8 matrix-core mat-vec, every matrix of the launch Q4_K */
-  LGH_SYM_MVQ_Q6K = 16,    /* lgh::mvq_kernel<2u> : ... every matrix Q6_K */
+  LGH_SYM_MVQ_Q4K = 15,    /* lgh::mvq_kernel<1u>, lgh::mvq_rows_kernel<1u, ..> : int8 matrix-core mat-vec, every matrix of the launch Q4_K */
+  LGH_SYM_MVQ_Q6K = 16,    /* lgh::mvq_kernel<2u>, lgh::mvq_rows_kernel<2u, ..> : ... every matrix Q6_K */
   LGH_SYM_MVQ_MIXED = 17,  /* lgh::mvq_kernel<3u> : ... Q4_K and Q6_K matrices in one launch (fused QKV of Q4_K_M) */
-  LGH_SYM_MVQ_Q5K = 18,    /* lgh::mvq_kernel<4u> / <6u> : Q5_K (and Q5_K + Q6_K) */
-  LGH_SYM_MVQ_Q80_Q40 = 19, /* lgh::mvq_kernel<8u> / <16u> : Q8_0 / Q4_0 */
+  LGH_SYM_MVQ_Q5K = 18,    /* lgh::mvq_kernel<4u> / <6u>, lgh::mvq_rows_kernel<4u, ..> : Q5_K (and Q5_K + Q6_K) */
+  LGH_SYM_MVQ_Q80_Q40 = 19, /* lgh::mvq_kernel<8u> / <16u>, lgh::mvq_rows_kernel<8u / 16u, ..> : Q8_0 / Q4_0 */
   LGH_SYM_PTOK = 20,       /* (unused) */
   LGH_SYM_LINEAR = 21,     /* lgh::lin_mv_kernel / lgh::lin_gemm_kernel : products over weights kept in bf16 (lgh_create_layered) */
   LGH_SYM_LATENT = 22,     /* lgh::latent_* : attention over a shared latent */

@@ -11,6 +11,7 @@ call goes through ``lib/libllama_gguf_hip.so`` and FAILS LOUDLY if that library 
 from __future__ import annotations
 
 import ctypes as C
+import fnmatch
 import os
 import threading
 from typing import Iterable, Optional, Sequence, Tuple
@@ -44,13 +45,24 @@ ABI_SYMBOLS = (
 K_NAMES = ("embed", "qkv", "attn", "attn_combine", "wo", "gate_up", "down", "router", "output", "argmax", "misc", "token", "expand", "experts")
 K_COUNT = 16
 SYM_COUNT = 29
-# kernel symbols as rocprofv3 prints them (LGH_SYM_* order)
+# kernel symbols as rocprofv3 prints them (LGH_SYM_* order); several kernels whose launches are counted together: joined by " + ", "*" for any template argument
 SYM_NAMES = ("lgh::mv_kernel<1u, 1024>", "lgh::mv_kernel<8u, 1024>", "lgh::mv_kernel<16u, 1024>",
              "lgh::mv_kernel<2u, 768>", "lgh::mv_kernel<4u, 512>", "lgh::mv_kernel<5u, 512>", "lgh::mv_kernel<6u, 512>",
              "lgh::mv_kernel<31u, 512>", "lgh::f32_matvec_kernel", "lgh::attn_partial_kernel", "lgh::attn_combine_kernel",
-             "lgh::embed_kernel", "lgh::argmax_stage1+2", "lgh::moe_router_kernel", "other", "lgh::mvq_kernel<1u>", "lgh::mvq_kernel<2u>", "lgh::mvq_kernel<3u>", "lgh::mvq_kernel<4u>",
-             "lgh::mvq_kernel<8u>", "unused", "lgh::lin_mv / lin_gemm", "lgh::latent_*", "lgh::mlstm_*", "lgh::tied_*", "lgh::gattn_*", "lgh::gla_*",
+             "lgh::embed_kernel", "lgh::argmax_stage1+2", "lgh::moe_router_kernel", "other",
+             "lgh::mvq_kernel<1u> + lgh::mvq_rows_kernel<1u, *>", "lgh::mvq_kernel<2u> + lgh::mvq_rows_kernel<2u, *>", "lgh::mvq_kernel<3u>",
+             "lgh::mvq_kernel<4u> + lgh::mvq_kernel<6u> + lgh::mvq_rows_kernel<4u, *>",
+             "lgh::mvq_kernel<8u> + lgh::mvq_kernel<16u> + lgh::mvq_rows_kernel<8u, *> + lgh::mvq_rows_kernel<16u, *>", "unused", "lgh::lin_mv / lin_gemm", "lgh::latent_*", "lgh::mlstm_*", "lgh::tied_*", "lgh::gattn_*", "lgh::gla_*",
              "lgh::glru_*", "lgh::delta_*")
+
+
+def symbol_rows(symbol: str, names: Sequence[str]) -> list:
+    """Which of the kernel names (a profiler's) a reported symbol stands for.  Empty unless a kernel of every kind (the name in front of the template's arguments) is among them: a table without one of them is another tree's."""
+    parts = symbol.split(" + ")
+    found = [n for n in names if any(fnmatch.fnmatchcase(n, p) for p in parts)]
+    return found if {p.split("<")[0] for p in parts} <= {n.split("<")[0] for n in found} else []
+
+
 FLAG_NO_GRAPH = 1
 FLAG_EXACT_PREFILL = 4   # forward_batch feeds tokens one by one (f32 throughout) instead of the batched f16 GEMM path
 KV_F32, KV_INT8, KV_FP8_E4M3, KV_FP8_E5M2 = 0, 1, 2, 3   # lgh_model_desc.kv_cache_type: f32, or QuantizedKVCache's formats (kv_quantized.rs; no CLI flag reaches them)

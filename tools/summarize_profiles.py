@@ -18,6 +18,10 @@ from collections import defaultdict
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent.parent
+sys.path.insert(0, str(ROOT))
+import __graft_entry__ as graft  # noqa: E402
+
+symbol_rows = graft.load_package().hip_backend.symbol_rows
 
 
 def short(name: str) -> str:
@@ -78,45 +82,42 @@ def main():
 
     rl = bench["roofline"]
     kname = rl["kernel"]
-    if kname.endswith(">") and kname not in {short(k) for k in []}:
-        pass
-    if rl.get("traffic") is None:   # the bench line ran before this session's PMC table existed: fill it from the same session
-        for r in rows:
-            if r[0] == kname and r[1] > 0:
-                rl["traffic"], rl["traffic_source"] = int(r[5]), f"{tag}_pmc_traffic.csv"
-        (dst / f"{tag}_bench.json").write_text(json.dumps(bench) + "\n")
+    traffic = {r[0]: r for r in rows}
+    in_traffic = symbol_rows(kname, [k for k in traffic if traffic[k][1] > 0])
+    if in_traffic:   # (a symbol of several kernels: the mean over their launches)
+        launch_bytes = sum(traffic[k][5] * traffic[k][1] for k in in_traffic) / sum(traffic[k][1] for k in in_traffic)
+        if rl.get("traffic") is None:   # the bench line ran before this session's PMC table existed: fill it from the same session
+            rl["traffic"], rl["traffic_source"] = int(launch_bytes), f"{tag}_pmc_traffic.csv"
+            (dst / f"{tag}_bench.json").write_text(json.dumps(bench) + "\n")
     with open(stats, newline="") as f:
         st = {short(r["Name"]): r for r in csv.DictReader(f)}
-    if kname not in st:   # a bench line written with the symbol name of an earlier template signature (mvq_kernel<1u> -> <1u, false>)
-        alt = kname[:-1] + ", false>"
-        if alt in st:
-            for d in (bench.get("kernels", {}),):
-                for k in list(d):
-                    if k.endswith(">") and k[:-1] + ", false>" in st:
-                        d[k[:-1] + ", false>"] = d.pop(k)
-            kname = rl["kernel"] = alt
+    in_stats = symbol_rows(kname, list(st))
+
+    def bench_avg(k):
+        b = bench.get("kernels", {}).get(k)
+        return f"{b['avg_us'] - rl.get('event_bracket_us', 0.0) + rl.get('dispatch_gap_us', 0.0):.2f}" if b else ""
+
     lines = [f"# {tag}: measurement summary", "",
              f"bench: {bench['value']} {bench['unit']}, {bench['ms_per_step']} ms/token, n_gpus={bench['n_gpus']}", "",
              "| kernel | rocprof calls | rocprof avg us | share % | bench avg us (hipEvent, bracket removed, + dispatch gap) | FETCH raw KB | WRITE raw KB | HBM bytes/launch (corrected) |",
              "|---|---|---|---|---|---|---|---|"]
-    traffic = {r[0]: r for r in rows}
     for k, r in st.items():
         if not k.startswith("lgh::"):
             continue
-        b = bench.get("kernels", {}).get(k, {})
-        bavg = ""
-        if b:
-            bavg = f"{b['avg_us'] - rl.get('event_bracket_us', 0.0) + rl.get('dispatch_gap_us', 0.0):.2f}"
         t = traffic.get(k)
-        lines.append(f"| `{k}` | {r['Calls']} | {float(r['AverageNs']) / 1e3:.2f} | {r['Percentage']} | {bavg} | "
-                     f"{t[2]:.0f} | {t[4]:.0f} | {t[5] / 1e6:.2f} MB |" if t else
-                     f"| `{k}` | {r['Calls']} | {float(r['AverageNs']) / 1e3:.2f} | {r['Percentage']} | {bavg} | | | |")
+        lines.append(f"| `{k}` | {r['Calls']} | {float(r['AverageNs']) / 1e3:.2f} | {r['Percentage']} | {bench_avg(k)} | "
+                     + (f"{t[2]:.0f} | {t[4]:.0f} | {t[5] / 1e6:.2f} MB |" if t else "| | |"))
+    for k in bench.get("kernels", {}):   # symbols of several kernels: what the bench times is their mean
+        found = symbol_rows(k, list(st)) if k not in st else []
+        if found:
+            calls = sum(int(st[f]["Calls"]) for f in found)
+            lines.append(f"| `{k}` | {calls} | {sum(float(st[f]['TotalDurationNs']) for f in found) / calls / 1e3:.2f} | {sum(float(st[f]['Percentage']) for f in found):.2f} | {bench_avg(k)} | | | |")
     lines += ["",
               f"dominant kernel `{kname}`: algorithmic {rl['alg_bytes_per_launch'] / 1e6:.2f} MB/launch, "
               f"bench avg {rl['avg_launch_us']} us -> {rl['achieved']} GB/s = {rl['frac']:.3f} of {rl['peak']} GB/s; "
-              f"rocprof avg {float(st[kname]['AverageNs']) / 1e3:.2f} us."]
-    if kname in traffic:
-        lines.append(f"PMC traffic for it: {traffic[kname][5] / 1e6:.2f} MB/launch "
+              + (f"rocprof avg {sum(float(st[k]['TotalDurationNs']) for k in in_stats) / sum(int(st[k]['Calls']) for k in in_stats) / 1e3:.2f} us." if in_stats else "not in the rocprof table.")]
+    if in_traffic:
+        lines.append(f"PMC traffic for it: {launch_bytes / 1e6:.2f} MB/launch "
                      f"(FETCH_SIZE x2 + WRITE_SIZE; the PMC passes ran `bench.py --steps 8 --warmup 2 --prompt 8`).")
     if bench.get("prefill"):
         pf = bench["prefill"]
