@@ -222,7 +222,8 @@ void lgh_destroy(lgh_ctx* ctx);
 
 /* ---- GpuInference (src/backend/mod.rs:283-296) ---- */
 
-/* GpuInference::forward (gpu_only.rs:728-771): logits_out = vocab_size f32, caller-owned. */
+/* GpuInference::forward (gpu_only.rs:728-771): logits_out = vocab_size f32, caller-owned.
+ * Calls that bring logits poll for them: the thread does not sleep; after some 0.1 ms it yields its core to other threads between polls. */
 int lgh_forward(lgh_ctx* ctx, uint32_t token_id, float* logits_out);
 /* GpuInference::prefill_token (gpu_only.rs:792-806) */
 int lgh_prefill_token(lgh_ctx* ctx, uint32_t token_id);

@@ -215,7 +215,7 @@ void xq_stale(lgh_ctx* c, const float* f32);
 int linear_any(lgh_ctx* c, int cls, const lgh::DevWeight& W, const float* x, float* out, const float* norm_w,
                const float* resid, const float* bias, int xq_next = 0, const float* xq_next_nw = nullptr);
 int drain_prof(lgh_ctx* c);
-// a call at work on the context's device, until everything it launched has ended (engine.hip: the side stream); alone: no other was when it began
+// a call at work on the context's device, until its results are there: behind everything it launched, whose last kernel may still be ending (engine.hip: the side stream); alone: no other was when it began
 struct AtWork {
   std::atomic<int>* const calls;
   const bool alone;

@@ -894,6 +894,7 @@ static int bind(const lgh_ctx* c) { return hipSetDevice(c->device) == hipSuccess
 // last one, and is over for the host when the last part has answered: no launch and no event of its own, no wait for the stream.  From the head's end to the next token's first kernel 70 us -> 35 (32000 floats); logits to the
 // host after every token, before; now: TinyLlama-1.1B 40 rows 530 -> 515 us, Llama-3-8B (8 layers) 371 -> 360, Mixtral (3 layers) 265 -> 252; five sequences of Mixtral (2 layers) 541 -> 523 a step; 16 sequences of the 8B model (8 layers,
 // 2 MB a step) as before: there the host's copy is what takes the time, 16 GB/s.
+constexpr uint32_t kSpinTurns = 4096;   // some 0.1 ms: between the parts of a result the answers are closer than that
 // n floats to the caller's memory that launch number `number` brought to the parts from `first` on
 static int results_take(lgh_ctx* c, float* dst, size_t n, uint32_t number, uint32_t first) {
   HostOut& O = c->out;
@@ -903,8 +904,9 @@ static int results_take(lgh_ctx* c, float* dst, size_t n, uint32_t number, uint3
     const size_t end = std::min(part + group, last);
     for (size_t i = part; i < end; i++) {
       for (uint32_t turn = 1; O.answers()[i] != number; turn++) {
-        __builtin_ia32_pause();
-        if (turn % 4096) continue;
+        if (turn < kSpinTurns) __builtin_ia32_pause();
+        else std::this_thread::yield();   // a step or a prompt: others may have the core
+        if (turn % kSpinTurns) continue;
         // now and then: whether the work is still going on (a launch that was lost leaves no answer)
         const hipError_t e = hipStreamQuery(c->stream);
         if (e == hipErrorNotReady) continue;
