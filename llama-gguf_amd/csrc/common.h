@@ -182,7 +182,7 @@ bool mvqb_wide_input(int dev_type, uint32_t n_seq);
 hipError_t xw_from_xq_launch(const uint8_t* xq, uint32_t xq_stride, uint8_t* xw, uint32_t xw_block, uint32_t k, uint32_t n_seq, hipStream_t st);
 
 // launch-uniform geometry of one int8-MFMA launch as the kernel takes it (mvq_pack)
-struct MvGeom { uint32_t wbpack, geom, geom2, red_floats, lds_red_off, n_wg, flags; };   // flags: 1 the rotation's row lies in LDS
+struct MvGeom { uint32_t wbpack, geom, geom2, lds_red_off, n_wg, flags; };   // flags: 1 the rotation's row lies in LDS
 
 // ---------------------------------------------------------------------------------------------
 // host-side launchers (defined in the .hip files)

@@ -74,7 +74,7 @@ __device__ __forceinline__ void mvqb_tail(const MvLaunch& L, const MvSeg& S, con
     V.pos = B.pos + s;
     V.xw_out = B.xw_out[sg] ? B.xw_out[sg] + (size_t)so * kXwRecord : nullptr;
     V.xw_block = B.xw_block;
-    mv_epilogue_view(L, S, V, wg, rows_per_wg, red + (size_t)s * red_floats, ssq + s * 8, nslots, MvEpiPre{0.0f, 0.0f, false}, tl);
+    mv_epilogue_view(L, S, V, wg, rows_per_wg, red + (size_t)s * red_floats, ssq + s * 8, nslots, tl);
   }
 }
 

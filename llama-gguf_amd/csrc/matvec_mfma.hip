@@ -810,7 +810,6 @@ uint32_t mvq_pack(const MvLaunch& L, uint32_t n_wg, uint32_t threads, MvGeom* g,
   g->wbpack = (L.nseg > 1 ? L.seg[1].wg_begin : 0xFFFFu) | (L.nseg > 2 ? L.seg[2].wg_begin : 0xFFFFu) << 16;
   g->geom = S0.T | S0.G << 8 | S0.units << 16 | (L.do_norm ? 1u << 31 : 0u);
   g->geom2 = S0.nblk | Rg << 16;
-  g->red_floats = L.red_floats;
   g->lds_red_off = mvq_red_offset(S0.nblk, n_x);
   g->n_wg = n_wg;
   *lds_out = lds;

@@ -1,4 +1,4 @@
-// mv_epilogue.h — per-row epilogues shared by the VALU and the int8-MFMA mat-vec kernels (internal).
+// mv_epilogue.h — per-row epilogues shared by the VALU mat-vec and the batched int8-MFMA kernels (internal).
 #pragma once
 
 #include "device_utils.h"
@@ -7,41 +7,6 @@
 namespace lgh {
 
 __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + expf(-g)); }
-
-// Operands of the epilogue that do not depend on the mat-vec — the residual element, or RoPE's cos/sin at the current
-// position — can be fetched at kernel START and carried in two registers: loaded after the final barrier they are a
-// dependent chain of global loads (position -> table index -> cos/sin) of ~1.5 us on the critical path.
-struct MvEpiPre { float a, b; bool valid; };
-
-// The residual element: issued first thing (one load, older than everything else in the wave's queue).  `epi` and
-// `resid` come from the caller's first batch of scalar loads — fetched here they would be two more dependent round trips.
-__device__ __forceinline__ void mv_epilogue_prefetch_resid(int epi, const float* resid, const float* xq_nw, uint32_t n_rows, uint32_t wg,
-                                                           uint32_t rows_per_wg, MvEpiPre& pre, uint32_t tid = threadIdx.x) {
-  if (resid && (epi == EPI_RESID || epi == EPI_MOE_DOWN)) {
-    const uint32_t t = tid, row = wg * rows_per_wg + t;
-    if (t < rows_per_wg && row < n_rows) {
-      pre.a = resid[row];
-      pre.b = xq_nw ? xq_nw[row] : 1.0f;   // the next consumer's norm weight, for the XQ image of the output
-      pre.valid = true;
-    }
-  }
-}
-// RoPE's cos/sin at the current position (`pos` already in a scalar register).  Like the residual it must be issued
-// BEFORE the input vector and the weight tiles: a conditional load issued after them makes the compiler's wait for the
-// input vector conservative (it then also waits for the first tile to arrive from HBM).
-__device__ __forceinline__ void mv_epilogue_prefetch_rope(int epi, uint32_t pos, const float* rope_cs, uint32_t head_dim,
-                                                          uint32_t n_rows, uint32_t wg, uint32_t rows_per_wg, MvEpiPre& pre,
-                                                          uint32_t tid = threadIdx.x) {
-  if (epi == EPI_ROPE_Q || epi == EPI_ROPE_K) {
-    const uint32_t rl = 2 * tid, row = wg * rows_per_wg + rl;
-    if (rl < rows_per_wg && row < n_rows) {
-      const uint32_t half = head_dim / 2, i = (row % head_dim) / 2;
-      pre.a = rope_cs[((size_t)pos * half + i) * 2];
-      pre.b = rope_cs[((size_t)pos * half + i) * 2 + 1];
-      pre.valid = true;
-    }
-  }
-}
 
 // The vectors an epilogue writes and reads: the segment's own (single-sequence launches) or one sequence's slice of them
 // (matvec_batch.hip: every sequence has its own output, residual, XQ image, position and KV cache slot).
@@ -52,8 +17,7 @@ __device__ __forceinline__ float mv_inv_rms(float ss, uint32_t k, float eps) { r
 // Per-row epilogue, one thread per row (or per row pair for RoPE)
 // `nslots` = partial sums per (pass, row) in `red`, laid out red[(p * nslots + slot) * rows_per_wg + row]
 __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg& S, const MvEpiView V, uint32_t wg, uint32_t rows_per_wg, const float* red,
-                                                 const float* ssq, uint32_t nslots, const MvEpiPre pre = MvEpiPre{0.0f, 0.0f, false},
-                                                 uint32_t tid = threadIdx.x) {
+                                                 const float* ssq, uint32_t nslots, uint32_t tid = threadIdx.x) {
   const uint32_t t = tid;
   const uint32_t rbase = wg * rows_per_wg;
   float inv = 1.0f;
@@ -74,8 +38,8 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
     if (S.bias) { x0 += S.bias[row]; x1 += S.bias[row + 1]; }
     const uint32_t pos = (uint32_t)*V.pos, d = S.head_dim, half = d / 2;
     const uint32_t head = row / d, i = (row % d) / 2;
-    const float c = pre.valid ? pre.a : L.rope_cs[((size_t)pos * half + i) * 2];
-    const float s = pre.valid ? pre.b : L.rope_cs[((size_t)pos * half + i) * 2 + 1];
+    const float c = L.rope_cs[((size_t)pos * half + i) * 2];
+    const float s = L.rope_cs[((size_t)pos * half + i) * 2 + 1];
     float y0 = x0 * c - x1 * s, y1 = x0 * s + x1 * c;  // ops.rs:1326-1331
     if (S.epi == EPI_ROPE_Q) {
       V.out[row] = y0;
@@ -96,7 +60,7 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
   bool has_out = false;
   switch (S.epi) {
     case EPI_STORE: outv = v0; V.out[row] = outv; has_out = true; break;
-    case EPI_RESID: outv = v0 + (pre.valid ? pre.a : V.resid[row]); V.out[row] = outv; has_out = true; break;
+    case EPI_RESID: outv = v0 + V.resid[row]; V.out[row] = outv; has_out = true; break;
     case EPI_SWIGLU: {
       float up = rowval(1, t);
       outv = silu_f(v0) * up;
@@ -126,7 +90,7 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
       // starts from zero) and only the last one adds the residual (resid; none: the output is the running sum).
       float acc = S.out2 ? S.out2[row] : 0.0f;
       for (int p = 0; p < S.npass; p++) acc += S.moe_w[p] * rowval(p, t);
-      outv = V.resid ? acc + (pre.valid ? pre.a : V.resid[row]) : acc;
+      outv = V.resid ? acc + V.resid[row] : acc;
       V.out[row] = outv;
       has_out = true;
       break;
@@ -138,15 +102,14 @@ __device__ __forceinline__ void mv_epilogue_view(const MvLaunch& L, const MvSeg&
   // chunk leaves its sum of out^2.
   uint8_t* xq = V.xq_out;
   if (xq && has_out) {
-    const float* nw = S.xq_nw;
-    const float w = !nw ? 1.0f : (pre.valid && (S.epi == EPI_RESID || S.epi == EPI_MOE_DOWN)) ? pre.b : nw[row];
+    const float w = S.xq_nw ? S.xq_nw[row] : 1.0f;
     xq_store_chunk(xq, row >> 4, outv * w, V.xq_ssq, outv, tid, V.xw_out, V.xw_block);
   }
 }
 
 __device__ __forceinline__ void mv_epilogue(const MvLaunch& L, const MvSeg& S, uint32_t wg, const float* red, const float* ssq,
-                                            uint32_t nslots, const MvEpiPre pre = MvEpiPre{0.0f, 0.0f, false}, uint32_t tid = threadIdx.x) {
-  mv_epilogue_view(L, S, MvEpiView{S.out, S.resid, S.xq_out, S.xq_ssq, L.pos}, wg, S.rows_per_wg, red, ssq, nslots, pre, tid);
+                                            uint32_t nslots) {
+  mv_epilogue_view(L, S, MvEpiView{S.out, S.resid, S.xq_out, S.xq_ssq, L.pos}, wg, S.rows_per_wg, red, ssq, nslots);
 }
 
 }  // namespace lgh
