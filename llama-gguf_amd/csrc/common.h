@@ -211,7 +211,6 @@ bool mvqb_few_takes(int dev_type, uint32_t T, uint32_t nbw, uint32_t n_units, ui
 uint32_t mvqb2_min_seq();
 uint64_t mvqb_expert_part_floats(uint32_t n_units, uint32_t T, uint32_t n_seq);
 hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& B, uint32_t n_wg, uint32_t threads, hipStream_t st);   // matvec_batch.hip
-size_t mvqb_lds_bytes(uint32_t n_seq, uint32_t red_floats);
 hipError_t xq_quantize_launch(const float* x, const float* nw, uint8_t* xq, float* ssq_part, uint32_t k, hipStream_t st);
 hipError_t repack_t16_launch(int dev_type, const uint8_t* raw, uint8_t* dst, uint32_t n_rows, uint32_t nblk, hipStream_t st);
 hipError_t repack_q6k_t16_launch(const uint8_t* raw, uint8_t* dst, uint32_t n_rows, uint32_t nblk, hipStream_t st);  // LGH_SYM_MV_* of the instantiation mv_launch will pick

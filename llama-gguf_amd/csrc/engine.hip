@@ -260,8 +260,8 @@ void xq_stale(lgh_ctx* c, const float* f32) {
 static uint32_t g_launch_seq = 0;   // diagnostic builds: consecutive launches get consecutive span slots
 // Assembles the launch descriptor of one group of segments (and keeps the XQ bookkeeping: images this launch consumes are
 // converted here if their producer did not leave them; images it produces are marked fresh).
-// `tile_cap` (multi-sequence launches, engine_batch.hip): at most that many 16-row tiles per workgroup — the partial sums of
-// every sequence of the step must fit LDS.  It changes which workgroup computes a row, never the row's arithmetic.
+// `tile_cap` (multi-sequence launches, engine_batch.hip): at most that many 16-row tiles per workgroup — where one kernel does
+// all of the launch, the partial sums of every sequence of the step must fit LDS.  It changes which workgroup computes a row, never the row's arithmetic.
 int build_mv_group(lgh_ctx* c, const SegSpec* specs, int nseg, const float* norm_w, uint32_t k, bool mfma, MvLaunch& L,
                    uint32_t& wg, uint32_t& threads, uint64_t& alg, uint32_t tile_cap) {
   std::memset(&L, 0, sizeof(L));

@@ -109,7 +109,7 @@ int launch_mvb(lgh_ctx* c, int cls, const SegSpec* specs, int nseg, const float*
   MvLaunch L;
   uint32_t wg = 0, threads = 0;
   uint64_t alg = 0;
-  // partial sums of all sequences in LDS: n_seq * npass * T * 16 * R floats <= ~120 KB
+  // partial sums of all sequences in LDS, where one kernel does all (mvqb_kernel): n_seq * npass * T * 16 * R floats <= ~120 KB
   uint32_t cap = 32;
   {
     int npass_max = 1;
@@ -119,7 +119,6 @@ int launch_mvb(lgh_ctx* c, int cls, const SegSpec* specs, int nseg, const float*
   }
   int rc = build_mv_group(c, specs, nseg, norm_w, k, true, L, wg, threads, alg, cap);
   if (rc) return rc;
-  if (mvqb_lds_bytes(n_seq, L.red_floats) > 160 * 1024) return fail(c, LGH_UNSUPPORTED, "multi-sequence mat-vec: partial sums do not fit LDS");
   MvBatch B{};
   B.n_seq = n_seq;
   B.pos = Bs.d_pos;

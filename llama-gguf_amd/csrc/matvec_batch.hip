@@ -1346,7 +1346,7 @@ __global__ void __launch_bounds__(kFewWaves * 64, 3) mvqb_few_kernel(const MvqbF
 // ------------------------------------------------------------------------------------------------
 // host
 // ------------------------------------------------------------------------------------------------
-size_t mvqb_lds_bytes(uint32_t n_seq, uint32_t red_floats) { return ((size_t)n_seq * red_floats + (size_t)n_seq * 8) * 4 + 64; }
+static size_t mvqb_lds_bytes(uint32_t n_seq, uint32_t red_floats) { return ((size_t)n_seq * red_floats + (size_t)n_seq * 8) * 4 + 64; }
 
 template <uint32_t MASK, int NB>
 static hipError_t mvqb_go(const MvLaunch& L, const MvBatch& B, const MvGeom& g, uint32_t threads, size_t lds, hipStream_t st) {
@@ -1543,8 +1543,6 @@ hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uin
   if (!mask) return hipErrorInvalidValue;
   for (int i = 0; i < L.nseg; i++)
     if (L.seg[i].npass > 2 || L.seg[i].pass[0].sel || (L.seg[i].npass == 2 && L.seg[i].pass[1].xq != L.seg[i].pass[0].xq)) return hipErrorInvalidValue;
-  const size_t lds = mvqb_lds_bytes(B.n_seq, L.red_floats);
-  if (lds > 160 * 1024) return hipErrorInvalidValue;
   if (B.ind_cnt && (B.part == nullptr || B.n_seq < mvqb2_min_seq() || !B.ind_idx || B.ind_div == 0)) return hipErrorInvalidValue;   // indirect entries: mvqb2 only
   bool shared_x = B.part != nullptr;
   for (int i = 0; i < L.nseg; i++) shared_x = shared_x && L.seg[i].pass[0].xq == L.seg[0].pass[0].xq;
@@ -1584,6 +1582,8 @@ hipError_t mvqb_launch(const MvLaunch& L, const MvBatch& Bin, uint32_t n_wg, uin
     }
   }
   if (B.ind_cnt) return hipErrorInvalidValue;   // (indirect entries exist in the mvqb2 structure only)
+  const size_t lds = mvqb_lds_bytes(B.n_seq, L.red_floats);
+  if (lds > 160 * 1024) return hipErrorInvalidValue;
 #define LGH_MVQB_NB(M, NBV) return mvqb_go<M, NBV>(L, B, g, threads, lds, st)
 #define LGH_MVQB_CASE(M)                                         \
   case M:                                                        \
