@@ -608,7 +608,7 @@ int lgh_batch_create(lgh_ctx* c, uint32_t max_batch) {
   register_views(c, Bs.act2, xq_f2, ssq_f2, ffn, max_batch);
   Bs.pos.assign(max_batch, 0);
   Bs.ready = true;
-  // a step of every size that launches kernels of its own (matvec_batch.hip: groups of four and eight, of up to 4, 8, 12 and 16 sequences; up to four the epilogue's form goes by the rows; a mixture's gate | up takes, up to a size that
+  // a step of every size that launches kernels of its own (matvec_batch.hip: groups of four and eight, of up to 4, 8, 12 and 16 sequences; a mixture's gate | up takes, up to a size that
   // goes by its experts, a kernel of its own, so there the largest of each group too), eagerly, before any of them is first
   // launched inside a capture (engine.hip: warm_kernels explains the ROCm trap); they write row 0 of the slots' caches, which a slot's first real token overwrites
   uint32_t slots0[kMaxBatch], toks0[kMaxBatch] = {};
